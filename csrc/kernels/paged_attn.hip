@@ -118,7 +118,8 @@ struct Args {
   int64_t out_tok_stride;
   float* part_o;   // [splits, T, nq, D]
   float* part_ml;  // [splits, T, nq, 2]
-  int T;
+  int T;           // rows of a split's partials
+  const int* seqs; // [n][2]: sequence, row of its first partial; null: all sequences, partials by token row
   int window;      // sliding window (Mistral / Qwen2): keys older than `window` positions are masked; 0 = off
   int* counters;   // [S * nkv] zeroed split-arrival counters: the last split of a (seq, kv head) merges; or null
 };
@@ -165,7 +166,7 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(Args a) {
   __shared__ int64_t koff_lds[kWaves][KC];
   __shared__ float mrg_ml[kWaves][PR][2];
 
-  const int seq = blockIdx.x / a.nkv, kvh = blockIdx.x - (blockIdx.x / a.nkv) * a.nkv;
+  const int item = blockIdx.x / a.nkv, kvh = blockIdx.x - item * a.nkv, seq = a.seqs ? a.seqs[2 * item] : item;
   const int split = blockIdx.y;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int g = lane >> 4, i = lane & 15;
@@ -340,7 +341,7 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(Args a) {
       if (a.splits == 1) {
         a.out[(int64_t)t * a.out_tok_stride + (int64_t)h * D + d] = f32_to_bf16(L > 0.f ? sum / L : 0.f);
       } else {
-        const int64_t pidx = ((int64_t)split * a.T + t) * a.nq + h;
+        const int64_t pidx = ((int64_t)split * a.T + (a.seqs ? a.seqs[2 * item + 1] + tok : t)) * a.nq + h;
         a.part_o[pidx * D + d] = sum;
         if (d == 0) {
           a.part_ml[pidx * 2 + 0] = M;
@@ -404,28 +405,30 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(Args a) {
   }
 }
 
-// Combine the splits' fp32 partials of one (token, head): every load of a group of up to 16 splits is
-// issued before the first use (a loop that consumes each partial before loading the next makes a
-// chain of dependent ~1 us memory round trips: 10 us at 16 splits).
-template <int D>
-__global__ __launch_bounds__(D) void merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
-                                                  int splits, int T, int nq, unsigned short* __restrict__ out,
-                                                  int64_t out_tok_stride) {
-  constexpr int U = 16;
-  const int th = blockIdx.x;  // t * nq + h
-  const int t = th / nq, h = th - t * nq;
-  const int d = threadIdx.x;
-  const int64_t sstride = (int64_t)T * nq;
-  float M = -INFINITY, acc = 0.f, L = 0.f;
+// Combine the splits' fp32 partials: D / 4 threads a (token, head) row, 16 bytes a load, every load of a group of up to U
+// splits issued before the first use (a loop that consumes each partial before loading the next makes a chain of
+// dependent ~1 us memory round trips: 10 us at 16 splits).
+template <int D, int U>
+__global__ __launch_bounds__(256) void merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
+                                                    int splits, int64_t T, int nq, unsigned short* __restrict__ out,
+                                                    int64_t out_tok_stride, const int* __restrict__ rows) {
+  constexpr int TPR = D / 4, RPB = 256 / TPR;
+  const int64_t sstride = T * nq, th = (int64_t)blockIdx.x * RPB + threadIdx.x / TPR;  // partial row * nq + h
+  const int d = threadIdx.x % TPR * 4;
+  if (th >= sstride) return;
+  const int64_t pt = th / nq, t = rows ? rows[pt] : pt;  // rows: token row of every partial row
+  const int h = th - pt * nq;
+  float M = -INFINITY, L = 0.f;
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int s0 = 0; s0 < splits; s0 += U) {
-    float ms[U], ls[U], os[U];
+    float ms[U], ls[U];
+    f32x4 os[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int s = min(s0 + u, splits - 1);
-      const int64_t idx = s * sstride + th;
+      const int64_t idx = (int64_t)min(s0 + u, splits - 1) * sstride + th;
       ms[u] = part_ml[idx * 2];
       ls[u] = part_ml[idx * 2 + 1];
-      os[u] = part_o[idx * D + d];
+      os[u] = *reinterpret_cast<const f32x4*>(part_o + idx * D + d);
     }
     float Mc = M;
 #pragma unroll
@@ -444,7 +447,10 @@ __global__ __launch_bounds__(D) void merge_kernel(const float* __restrict__ part
     }
     M = Mc;
   }
-  out[(int64_t)t * out_tok_stride + (int64_t)h * D + d] = f32_to_bf16(L > 0.f ? acc / L : 0.f);
+  u16x4 y;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) y[e] = f32_to_bf16(L > 0.f ? acc[e] / L : 0.f);
+  *reinterpret_cast<u16x4*>(out + t * out_tok_stride + (int64_t)h * D + d) = y;
 }
 
 }  // namespace pa
@@ -509,13 +515,34 @@ void kv_cache_append(const at::Tensor& qkv, at::Tensor cache, const at::Tensor& 
   SXE_LAUNCH_CHECK();
 }
 
+// part_o [splits, R, nq, D], part_ml [splits, R, nq, 2] -> out [T, nq, D]; rows: token row of each of the R (null: itself)
+static void launch_merge(const at::Tensor& part_o, const at::Tensor& part_ml, const int* rows, at::Tensor& out) {
+  const int splits = part_o.size(0), R = part_o.size(1), nq = part_o.size(2), D = part_o.size(3);
+  auto* op = reinterpret_cast<unsigned short*>(out.data_ptr());
+  auto launch = [&](auto kern) {
+    const int64_t rpb = 1024 / D;
+    hipLaunchKernelGGL(kern, dim3(((int64_t)R * nq + rpb - 1) / rpb), dim3(256), 0, cur_stream(), part_o.data_ptr<float>(),
+                       part_ml.data_ptr<float>(), splits, (int64_t)R, nq, op, out.stride(0), rows);
+  };
+  if (D == 128) launch(splits <= 4 ? pa::merge_kernel<128, 4> : pa::merge_kernel<128, 16>);
+  else if (D == 256) launch(splits <= 4 ? pa::merge_kernel<256, 4> : pa::merge_kernel<256, 16>);
+  else launch(splits <= 4 ? pa::merge_kernel<64, 4> : pa::merge_kernel<64, 16>);
+  SXE_LAUNCH_CHECK();
+}
+
+void paged_merge(const at::Tensor& part_o, const at::Tensor& part_ml, const at::Tensor& rows, at::Tensor& out) {
+  launch_merge(part_o, part_ml, rows.data_ptr<int>(), out);
+}
+
 // q: [T, nq, D] (token stride free); returns out [T, nq, D] bf16. parts != nullptr (and splits > 1):
 // no merge launch -- the fp32 partials go to (*parts)[0] = part_o [splits, T, nq, D] and
 // (*parts)[1] = part_ml [splits, T, nq, 2] for a consumer that merges them itself (skinny_gemm_merge)
 static at::Tensor paged_attention_impl(const at::Tensor& q, const at::Tensor& cache, const at::Tensor& block_table,
                                        const at::Tensor& q_start, const at::Tensor& q_len, const at::Tensor& kv_len,
                                        double scale, int64_t max_kv_len, int64_t splits, int64_t window,
-                                       std::vector<at::Tensor>* parts, const c10::optional<at::Tensor>& counters = {}) {
+                                       std::vector<at::Tensor>* parts, const c10::optional<at::Tensor>& counters = {},
+                                       const at::Tensor* seqs = nullptr, const at::Tensor* rows = nullptr,
+                                       const at::Tensor* into = nullptr) {
   SXE_CHECK_CUDA(q);
   SXE_CHECK(q.scalar_type() == at::kBFloat16 && cache.scalar_type() == at::kBFloat16, "bf16 only");
   SXE_CHECK(q.dim() == 3 && q.stride(2) == 1 && q.stride(1) == q.size(2), "q must be [T, nq, D] with head stride D");
@@ -528,8 +555,8 @@ static at::Tensor paged_attention_impl(const at::Tensor& q, const at::Tensor& ca
   const int T = q.size(0), nq = q.size(1), D = q.size(2);
   const int nkv = cache.size(2), bs = cache.size(3);
   SXE_CHECK(cache.size(4) == D && nq % nkv == 0, "head layout mismatch");
-  const int S = block_table.size(0);
-  auto out = at::empty({T, nq, D}, q.options());
+  const int S = seqs ? seqs->size(0) : block_table.size(0);
+  auto out = into ? *into : at::empty({T, nq, D}, q.options());
   if (T == 0 || S == 0) return out;
   c10::DeviceGuard g(q.device());
   splits = std::max<int64_t>(1, splits);
@@ -554,7 +581,8 @@ static at::Tensor paged_attention_impl(const at::Tensor& q, const at::Tensor& ca
   a.keys_per_split = (int)kps;
   a.out = reinterpret_cast<unsigned short*>(out.data_ptr());
   a.out_tok_stride = out.stride(0);
-  a.T = T;
+  a.T = rows ? rows->numel() : T;
+  a.seqs = seqs ? seqs->data_ptr<int>() : nullptr;
   a.part_o = nullptr;
   a.part_ml = nullptr;
   a.window = (int)std::max<int64_t>(0, window);
@@ -566,8 +594,8 @@ static at::Tensor paged_attention_impl(const at::Tensor& q, const at::Tensor& ca
     a.counters = counters->data_ptr<int>();
   }
   if (splits > 1) {
-    part_o = at::empty({splits, T, nq, D}, q.options().dtype(at::kFloat));
-    part_ml = at::empty({splits, T, nq, 2}, q.options().dtype(at::kFloat));
+    part_o = at::empty({splits, a.T, nq, D}, q.options().dtype(at::kFloat));
+    part_ml = at::empty({splits, a.T, nq, 2}, q.options().dtype(at::kFloat));
     a.part_o = part_o.data_ptr<float>();
     a.part_ml = part_ml.data_ptr<float>();
   }
@@ -590,18 +618,7 @@ static at::Tensor paged_attention_impl(const at::Tensor& q, const at::Tensor& ca
     *parts = {part_o, part_ml};
     return out;
   }
-  if (splits > 1 && a.counters == nullptr) {
-    if (D == 128)
-      hipLaunchKernelGGL(pa::merge_kernel<128>, dim3(T * nq), dim3(128), 0, cur_stream(), a.part_o, a.part_ml,
-                         (int)splits, T, nq, a.out, a.out_tok_stride);
-    else if (D == 256)
-      hipLaunchKernelGGL(pa::merge_kernel<256>, dim3(T * nq), dim3(256), 0, cur_stream(), a.part_o, a.part_ml,
-                         (int)splits, T, nq, a.out, a.out_tok_stride);
-    else
-      hipLaunchKernelGGL(pa::merge_kernel<64>, dim3(T * nq), dim3(64), 0, cur_stream(), a.part_o, a.part_ml,
-                         (int)splits, T, nq, a.out, a.out_tok_stride);
-    SXE_LAUNCH_CHECK();
-  }
+  if (splits > 1 && a.counters == nullptr) launch_merge(part_o, part_ml, rows ? rows->data_ptr<int>() : nullptr, out);
   return out;
 }
 
@@ -610,6 +627,21 @@ at::Tensor paged_attention(const at::Tensor& q, const at::Tensor& cache, const a
                            int64_t max_kv_len, int64_t splits, int64_t window, const c10::optional<at::Tensor>& counters) {
   return paged_attention_impl(q, cache, block_table, q_start, q_len, kv_len, scale, max_kv_len, splits, window, nullptr,
                               counters);
+}
+
+// The sequences of `seqs` only (int32 [n, 2]: sequence, row of its first partial; rows int32 [R]: token row of every
+// partial row), written into `out`.
+void paged_attention_some(const at::Tensor& q, const at::Tensor& cache, const at::Tensor& block_table,
+                          const at::Tensor& q_start, const at::Tensor& q_len, const at::Tensor& kv_len,
+                          const at::Tensor& seqs, const at::Tensor& rows, double scale, int64_t max_kv_len, int64_t splits,
+                          int64_t window, at::Tensor out) {
+  SXE_CHECK(seqs.is_cuda() && seqs.scalar_type() == at::kInt && seqs.is_contiguous() && seqs.dim() == 2 && seqs.size(1) == 2,
+            "paged_attention_some: seqs int32 [n, 2]");
+  SXE_CHECK(rows.is_cuda() && rows.scalar_type() == at::kInt && rows.is_contiguous(), "paged_attention_some: rows int32 [R]");
+  SXE_CHECK(out.sizes() == q.sizes() && out.is_contiguous() && out.scalar_type() == at::kBFloat16,
+            "paged_attention_some: out contiguous bf16 like q");
+  paged_attention_impl(q, cache, block_table, q_start, q_len, kv_len, scale, max_kv_len, splits, window, nullptr, {}, &seqs,
+                       &rows, &out);
 }
 
 // [out, part_o, part_ml]: with one split `out` is the attention output and the partials are empty;
@@ -636,6 +668,8 @@ TORCH_LIBRARY_FRAGMENT(sxe, m) {
         "int nq, int nkv) -> ()");
   m.def("paged_attention(Tensor q, Tensor cache, Tensor block_table, Tensor q_start, Tensor q_len, Tensor kv_len, "
         "float scale, int max_kv_len, int splits, int window=0, Tensor(a!)? counters=None) -> Tensor");
+  m.def("paged_attention_some(Tensor q, Tensor cache, Tensor block_table, Tensor q_start, Tensor q_len, Tensor kv_len, "
+        "Tensor seqs, Tensor rows, float scale, int max_kv_len, int splits, int window, Tensor(a!) out) -> ()");
   m.def("paged_attention_parts(Tensor q, Tensor cache, Tensor block_table, Tensor q_start, Tensor q_len, "
         "Tensor kv_len, float scale, int max_kv_len, int splits, int window=0) -> Tensor[]");
 }
@@ -643,5 +677,6 @@ TORCH_LIBRARY_IMPL(sxe, CUDA, m) {
   m.impl("kv_cache_append", &sxe::kv_cache_append);
   m.impl("rope_kv_cache_append", &sxe::rope_kv_cache_append);
   m.impl("paged_attention", &sxe::paged_attention);
+  m.impl("paged_attention_some", &sxe::paged_attention_some);
   m.impl("paged_attention_parts", &sxe::paged_attention_parts);
 }

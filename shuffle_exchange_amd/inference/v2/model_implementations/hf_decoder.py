@@ -34,11 +34,11 @@ from ....ops import native
 from ....ops.activation import ACT, bias_act, gated_act
 from ....ops.linear import linear
 from ....ops.norm import layer_norm, rms_norm
-from ....ops.paged_attention import kv_cache_append, paged_attention
+from ....ops.paged_attention import kv_cache_append
+from ....ops.paged_attention import ragged_attention as _ragged_attention
 from ....ops.rope import RopeCache, apply_rope_tokens_
 from ....ops.rows import embed, gather_last
 
-FLASH_PREFILL_MIN = 128
 
 
 @dataclass
@@ -340,40 +340,8 @@ def convert_hf_weights(spec, sd, hf_cfg=None):
 
 # ---------------------------------------------------------------------------- shared attention
 def ragged_attention(qkv, kv_layer, batch, nq, nkv, D, scale, window=None):
-    """Attention of a ragged batch's new tokens over their paged KV: pure prefills of >= 128 tokens
-    run the training flash kernel (MFMA, causal), the rest the paged-attention kernel."""
-    q = qkv[:, :nq]
-    use_flash = (native.use_hip(qkv) and D == 128 and qkv.dtype == torch.bfloat16 and
-                 (window is None or batch.max_kv_len <= window))
-    flash_ids = [i for i in range(batch.num_seqs)
-                 if use_flash and batch.host_seen[i] == 0 and batch.host_q_len[i] >= FLASH_PREFILL_MIN] \
-        if use_flash else []
-    if not flash_ids:
-        return paged_attention(q, kv_layer, batch.block_table, batch.q_start, batch.q_len, batch.kv_len, scale,
-                               batch.max_kv_len, window=window)
-    out = torch.empty(qkv.shape[0], nq, D, dtype=qkv.dtype, device=qkv.device)
-    fset = set(flash_ids)
-    rest = [i for i in range(batch.num_seqs) if i not in fset]
-    for i in flash_ids:
-        s, n = batch.host_q_start[i], batch.host_q_len[i]
-        pad = (-n) % 128
-        x = qkv[s:s + n]
-        if pad:
-            x = torch.cat([x, x.new_zeros(pad, *x.shape[1:])])
-        x = x.unsqueeze(0)
-        o, _ = torch.ops.sxe.flash_attn_fwd(x[:, :, :nq], x[:, :, nq:nq + nkv], x[:, :, nq + nkv:], True, float(scale))
-        out[s:s + n] = o[0, :n]
-    if rest:
-        idx = torch.tensor(rest, device=qkv.device)
-        o = paged_attention(q, kv_layer, batch.block_table.index_select(0, idx).contiguous(),
-                            batch.q_start.index_select(0, idx).contiguous(),
-                            batch.q_len.index_select(0, idx).contiguous(),
-                            batch.kv_len.index_select(0, idx).contiguous(), scale,
-                            max(batch.host_kv_len[i] for i in rest), window=window)
-        for i in rest:
-            s, n = batch.host_q_start[i], batch.host_q_len[i]
-            out[s:s + n] = o[s:s + n]
-    return out
+    """Attention of a ragged batch's new tokens over their paged KV (ops/paged_attention.py)."""
+    return _ragged_attention(qkv[:, :nq], kv_layer, batch, scale, window)
 
 
 # Measured on MI355X (tools/grouped_gemm_bench.py, profiles/grouped_gemm_bench.log): the grouped

@@ -7,8 +7,8 @@ BLAS linear, cutlass MoE GEMM) replaced by this framework's gfx950 kernels:
 
   * RMSNorm with fused residual add (norm.hip), projections through hipBLASLt,
   * RoPE in place on the packed QKV (rope.hip), KV scatter into the blocked cache and paged
-    attention (paged_attn.hip); sequences in pure prefill (no history, >= 128 new tokens) run the
-    training flash-attention kernel instead (MFMA, causal; their padding rows are discarded),
+    attention (paged_attn.hip; sequences with many new tokens, with or without earlier ones, in one
+    launch of the tile kernel, paged_prefill.hip),
   * SwiGLU (act.hip); Mixtral experts via the grouped MoE path of moe/,
   * only the last token of every sequence goes through the final norm + LM head.
 The weights are the training modules' own parameters (no copy): a trained LlamaForCausalLM /
@@ -30,10 +30,8 @@ import torch.nn.functional as F
 from ....ops import native
 from ....ops.activation import swiglu
 from ....ops.linear import linear
-from ....ops.paged_attention import paged_attention, paged_attention_parts, rope_kv_cache_append
+from ....ops.paged_attention import paged_attention_parts, paged_batch_attention, ragged_attention, rope_kv_cache_append
 from ....ops.rows import embed, gather_rows
-
-FLASH_PREFILL_MIN = 128
 
 
 class _TPShards:
@@ -165,40 +163,9 @@ class RaggedLlama:
         return next(self.model.parameters()).dtype
 
     def _attention(self, qkv, kv_layer, batch):
-        nq, D = self.nq, self.head_dim
-        scale = D ** -0.5
-        q = qkv[:, :nq]
-        use_flash = native.use_hip(qkv) and self.attn_impl.flash_prefill and D == 128 and qkv.dtype == torch.bfloat16
-        flash_ids = [i for i in range(batch.num_seqs)
-                     if use_flash and batch.host_seen[i] == 0 and batch.host_q_len[i] >= FLASH_PREFILL_MIN] \
-            if use_flash else []
-        if not flash_ids:
-            return paged_attention(q, kv_layer, batch.block_table, batch.q_start, batch.q_len, batch.kv_len, scale,
-                                   batch.max_kv_len)
-        out = torch.empty(qkv.shape[0], nq, D, dtype=qkv.dtype, device=qkv.device)
-        fset = set(flash_ids)
-        rest = [i for i in range(batch.num_seqs) if i not in fset]
-        for i in flash_ids:
-            s, n = batch.host_q_start[i], batch.host_q_len[i]
-            pad = (-n) % 128
-            x = qkv[s:s + n]
-            if pad:
-                x = torch.cat([x, x.new_zeros(pad, *x.shape[1:])])
-            x = x.unsqueeze(0)
-            o, _ = torch.ops.sxe.flash_attn_fwd(x[:, :, :nq], x[:, :, nq:nq + self.nkv], x[:, :, nq + self.nkv:],
-                                                True, float(scale))
-            out[s:s + n] = o[0, :n]
-        if rest:
-            idx = torch.tensor(rest, device=qkv.device)
-            o = paged_attention(q, kv_layer, batch.block_table.index_select(0, idx).contiguous(),
-                                batch.q_start.index_select(0, idx).contiguous(),
-                                batch.q_len.index_select(0, idx).contiguous(),
-                                batch.kv_len.index_select(0, idx).contiguous(), scale,
-                                max(batch.host_kv_len[i] for i in rest))
-            for i in rest:
-                s, n = batch.host_q_start[i], batch.host_q_len[i]
-                out[s:s + n] = o[s:s + n]
-        return out
+        pinned = (self._pins or {}).get("attention") == "dense_blocked_attention"
+        attend = paged_batch_attention if pinned else ragged_attention
+        return attend(qkv[:, :self.nq], kv_layer, batch, self.head_dim ** -0.5)
 
     def _proj(self, mod, x, li, key):
         if self.tps is not None:

@@ -98,8 +98,8 @@ class BlasLinear:
 # ----------------------------------------------------------------------------------- attention
 @register("attention", "dense_blocked_attention_flash_prefill", priority=10)
 class PagedAttentionFlashPrefill:
-    """Paged decode kernel (paged_attn.hip) for decode / continuation chunks; long fresh prompts
-    take the flash-attention kernel (flash_attn.hip) on the contiguous prompt."""
+    """Paged decode kernel (paged_attn.hip) for sequences with few new tokens; prompts and chunks of
+    prompts take the tile kernel over the same cache (paged_prefill.hip)."""
     flash_prefill = True
     flash_min_tokens = 256
 
@@ -113,7 +113,8 @@ class PagedAttentionFlashPrefill:
 
 @register("attention", "dense_blocked_attention", priority=0)
 class PagedAttention:
-    """Paged attention for every token (HIP kernel for head dims 64 / 128 / 256 with optional
+    """Paged attention, also what the heuristics give other head dims (their prompts take the tile
+    kernel, too); pinned by name, the decode kernel runs every token (HIP kernel for head dims 64 / 128 / 256 with optional
     sliding window; the PyTorch gather path elsewhere -- ops/paged_attention.py)."""
     flash_prefill = False
     flash_min_tokens = 1 << 30

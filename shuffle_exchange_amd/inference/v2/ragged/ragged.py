@@ -12,7 +12,7 @@ in one copy per dtype.
 """
 import math
 from dataclasses import dataclass, field
-from typing import List
+from typing import List, Optional
 
 import torch
 
@@ -209,6 +209,19 @@ class DSStateManager:
             self.kv.states.free(s.state_slot)
 
 
+@dataclass
+class AttentionLists:
+    """int32 device lists of one attention over a ragged batch: ``tiles`` [n, 4] (sequence, first token row, tokens, row among
+    ``tile_rows``), ``tile_rows`` the token rows they hold by sequence, ``tile_keys`` the longest key range; ``seqs`` [m, 2]
+    (sequence, row among ``seq_rows``), ``seq_rows``, ``seq_keys`` the same for the sequences outside the tiles (None: none)."""
+    tiles: torch.Tensor
+    tile_rows: torch.Tensor
+    tile_keys: int
+    seqs: Optional[torch.Tensor]
+    seq_rows: Optional[torch.Tensor]
+    seq_keys: int
+
+
 class RaggedBatch:
     """Device metadata of one forward over a ragged set of sequences (all int tensors on device).
 
@@ -307,6 +320,31 @@ class RaggedBatch:
             self._tables[key] = self._upload(rows, 2)
         return self._tables[key]
 
+    def attention_lists(self, tile, least):
+        """What ops/paged_attention.ragged_attention launches, or None if no sequence has ``least`` new tokens: tiles of
+        up to ``tile`` tokens of the sequences that have, longest key range first, and the other sequences."""
+        key = ("attention", tile, least)
+        if key not in self._tables:
+            tiles, seqs, tile_rows, seq_rows, a, b = [], [], [], [], 0, 0
+            for i, (q, n, seen) in enumerate(zip(self.host_q_start, self.host_q_len, self.host_seen)):
+                if n >= least:
+                    tiles += [(seen + min(j + tile, n), i, q + j, min(tile, n - j), a + j) for j in range(0, n, tile)]
+                    tile_rows.append(torch.arange(q, q + n, dtype=torch.int32))
+                    a += n
+                elif n:
+                    seqs.append((i, b))
+                    seq_rows.append(torch.arange(q, q + n, dtype=torch.int32))
+                    b += n
+            if tiles:
+                tiles.sort(reverse=True)
+                self._tables[key] = AttentionLists(
+                    self._upload([t[1:] for t in tiles], 4), self._upload(torch.cat(tile_rows), 1).view(-1), tiles[0][0],
+                    self._upload(seqs, 2) if seqs else None, self._upload(torch.cat(seq_rows), 1).view(-1) if seqs else None,
+                    max((self.host_kv_len[i] for i, _ in seqs), default=0))
+            else:
+                self._tables[key] = None
+        return self._tables[key]
+
     def _upload(self, rows, n):
-        t = torch.tensor(rows, dtype=torch.int32).reshape(-1, n)
+        t = torch.as_tensor(rows, dtype=torch.int32).reshape(-1, n)
         return t.pin_memory().to(self.slots.device, non_blocking=True) if self.slots.is_cuda else t

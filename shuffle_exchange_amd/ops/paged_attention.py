@@ -163,3 +163,57 @@ def paged_attention(q, cache, block_table, q_start, q_len, kv_len, scale, max_kv
         warning_once(f"paged_attention: head_dim={q.shape[-1]} window={window} not covered by the HIP kernel; "
                      f"using the PyTorch reference")
     return paged_attention_reference(q, cache, block_table, q_start, q_len, kv_len, scale, window)
+
+
+# A sequence takes the tile kernel from this many rows (new tokens x query heads of a kv head): up to 16 rows the decode
+# kernel reads the keys once, beyond it once for every 16 rows. Heads 32 / 8 of 128, us in the decode / the tile kernel:
+# 16 rows: 8 sequences behind 3000 keys 29 / 26, one behind 3000 15 / 19, 32 fresh 9.7 / 12; 20 rows: 44 / 25, 20 / 20,
+# 13.5 / 12.6; 128 rows: 159 / 40, 73 / 24, 60 / 12.5.
+TILE_MIN_ROWS = 17
+TILE_ROWS = 128  # rows of a workgroup of the tile kernel
+
+
+def choose_tile_splits(num_tiles, nkv, max_keys, target_wgs=None):
+    """(splits, keys of a split) of the tile kernel: the fewest splits that give every CU two workgroups, none under
+    512 keys (a split's partials cost as much traffic as ~64 keys of its tile)."""
+    target_wgs = PA_TARGET_WGS if target_wgs is None else target_wgs
+    want = math.ceil(target_wgs / max(1, num_tiles * nkv))
+    splits = max(1, min(want, math.ceil(max_keys / 512)))
+    keys = -(-math.ceil(max(max_keys, 1) / splits) // 64) * 64
+    return -(-max(max_keys, 1) // keys), keys
+
+
+def _tileable(q, cache, scale):
+    return (native.use_hip(q) and q.dtype == torch.bfloat16 and cache.dtype == torch.bfloat16 and q.shape[-1] in (64, 128, 256)
+            and q.shape[1] % cache.shape[2] == 0 and q.shape[1] // cache.shape[2] <= TILE_ROWS and scale > 0
+            and q.stride(2) == 1 and q.stride(1) == q.shape[2] and q.stride(0) % 8 == 0 and q.data_ptr() % 16 == 0)
+
+
+def paged_batch_attention(q, cache, batch, scale, window=None):
+    """``paged_attention`` of a whole ragged batch."""
+    return paged_attention(q, cache, batch.block_table, batch.q_start, batch.q_len, batch.kv_len, scale, batch.max_kv_len,
+                           window=window)
+
+
+def ragged_attention(q, cache, batch, scale, window=None):
+    """Causal attention of a ragged batch's new tokens q [T, nq, D] over their paged keys (the new ones among them).
+    Sequences with many new tokens -- prompts, and chunks of prompts behind earlier tokens -- run the tile kernel, the
+    others the decode kernel."""
+    nkv = cache.shape[2]
+    if window is not None and batch.max_kv_len <= window:
+        window = None
+    lists = None
+    if hasattr(batch, "attention_lists") and _tileable(q, cache, scale):
+        G = q.shape[1] // nkv
+        lists = batch.attention_lists(TILE_ROWS // G, -(-TILE_MIN_ROWS // G))
+    if lists is None:
+        return paged_batch_attention(q, cache, batch, scale, window)
+    out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+    meta = (q, cache, batch.block_table, batch.q_start, batch.q_len, batch.kv_len)
+    splits, keys = choose_tile_splits(lists.tiles.shape[0], nkv, lists.tile_keys)
+    torch.ops.sxe.paged_prefill(*meta, lists.tiles, lists.tile_rows, float(scale), int(window or 0), splits, keys, out)
+    if lists.seqs is not None:
+        splits = choose_splits(lists.seqs.shape[0], nkv, lists.seq_keys)
+        torch.ops.sxe.paged_attention_some(*meta, lists.seqs, lists.seq_rows, float(scale), int(lists.seq_keys), int(splits),
+                                           int(window or 0), out)
+    return out

@@ -1,0 +1,73 @@
+"""Attention of ragged batches over the paged cache: the tile kernel (csrc/kernels/paged_prefill.hip) and the lists that
+route sequences to it, against the fp32 reference."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from shuffle_exchange_amd.inference.v2.ragged.ragged import DSSequenceDescriptor, RaggedBatch
+from shuffle_exchange_amd.ops import paged_attention as PA
+
+
+def _batch(seqs, bs, device, seed=0):
+    """A ragged batch of (earlier, new) token counts over shuffled cache blocks."""
+    g = torch.Generator().manual_seed(seed)
+    need = [(c + n + bs - 1) // bs for c, n in seqs]
+    ids = torch.randperm(sum(need) + 2, generator=g).tolist()
+    desc = []
+    for i, ((c, n), k) in enumerate(zip(seqs, need)):
+        d = DSSequenceDescriptor(i, 1 << 20)
+        d.blocks, ids = ids[:k], ids[k:]
+        d.seen_tokens = c
+        desc.append(d)
+    return RaggedBatch(desc, [torch.zeros(n, dtype=torch.int64) for _, n in seqs], bs, torch.device(device)), sum(need) + 2
+
+
+def test_lists_hold_every_token_once():
+    seqs = [(0, 70), (500, 1), (33, 200), (0, 8), (9, 9)]
+    b, _ = _batch(seqs, 16, "cpu")
+    x = b.attention_lists(32, 9)
+    tiles = x.tiles.tolist()
+    keys = [seqs[s][0] + (q - b.host_q_start[s]) + n for s, q, n, _ in tiles]
+    assert keys == sorted(keys, reverse=True) and x.tile_keys == keys[0] and max(t[2] for t in tiles) <= 32
+    got = sorted(t for _, q, n, _ in tiles for t in range(q, q + n))
+    assert got == sorted(x.tile_rows.tolist()) and sorted(got + x.seq_rows.tolist()) == list(range(b.num_tokens))
+    for _, q, n, at in tiles:
+        assert x.tile_rows[at:at + n].tolist() == list(range(q, q + n))
+    for s, at in x.seqs.tolist():
+        assert x.seq_rows[at:at + seqs[s][1]].tolist() == list(range(b.host_q_start[s], b.host_q_start[s] + seqs[s][1]))
+    assert x.seq_keys == 501 and b.attention_lists(32, 201) is None
+
+
+def test_tile_splits_cover_the_keys():
+    for tiles in (1, 3, 40, 1000):
+        for nkv in (1, 8):
+            for keys in (1, 64, 500, 513, 4097, 100000):
+                n, k = PA.choose_tile_splits(tiles, nkv, keys)
+                assert k % 64 == 0 and n * k >= keys > (n - 1) * k
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("seqs", [[(0, 33)], [(0, 1), (63, 65), (64, 64), (0, 129)], [(4000, 300), (700, 1), (31, 2), (5, 40)],
+                                  [(1, 127), (127, 1), (0, 700), (2500, 9)]])
+@pytest.mark.parametrize("nq,nkv,D,bs,window", [(32, 8, 128, 64, None), (4, 4, 64, 16, None), (7, 1, 128, 128, 100),
+                                                (6, 2, 64, 48, 1), (8, 4, 256, 32, 300), (16, 1, 128, 64, None)])
+def test_ragged_attention(seqs, nq, nkv, D, bs, window):
+    b, blocks = _batch(seqs, bs, "cuda", seed=1)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    cache = torch.randn(blocks, 2, nkv, bs, D, device="cuda", generator=g).to(torch.bfloat16)
+    # slots that no sequence has written hold anything
+    used = torch.zeros(blocks * bs, dtype=torch.bool, device="cuda")
+    for i, (c, n) in enumerate(seqs):
+        p = torch.arange(c + n, device="cuda")
+        used[b.block_table[i].long()[p // bs] * bs + p % bs] = True
+    cache.view(blocks, 2, nkv, bs, D).permute(0, 3, 1, 2, 4)[~used.view(blocks, bs)] = float("nan")
+    qkv = torch.randn(b.num_tokens, nq + 2 * nkv, D, device="cuda", generator=g).to(torch.bfloat16)
+    q, scale = qkv[:, :nq], D ** -0.5
+    ref = PA.paged_attention_reference(q.float(), cache.float(), b.block_table, b.q_start, b.q_len, b.kv_len, scale, window)
+    got = PA.ragged_attention(q, cache, b, scale, window)
+    # p and the output are rounded to 8 bits each, the rest is fp32: 2 x 2^-9 and slack for the rows' spread
+    assert ((got.float() - ref).norm() / ref.norm()).item() < 6e-3
+    for i in range(b.num_seqs):  # every sequence for itself: a short one cannot hide behind a long one
+        s, n = b.host_q_start[i], b.host_q_len[i]
+        assert ((got[s:s + n].float() - ref[s:s + n]).norm() / ref[s:s + n].norm()).item() < 8e-3, seqs[i]
