@@ -5,471 +5,676 @@
 // Reference: ops/deepspeed4science/evoformer_attn.py (CUTLASS kernels of csrc/deepspeed4science,
 // not in the snapshot; kMax = 64 there too).
 //
-// The flash-attention structure of flash_attn.hip, generalised to narrow heads and additive biases:
-//  * swapped products (S^T = K Q^T: one lane = one query's scores, lane-local softmax) on
-//    v_mfma_f32_32x32x16_bf16, the score accumulator reused as the B operand of O^T += V^T P^T;
-//  * K/V (or Q/dO) tiles staged through registers into XOR-swizzled 256-byte LDS rows (a D-wide
-//    row uses its first D/8 chunks), row reads + ds_read_b64_tr_b16 transposed reads;
-//  * biases are added in the log2 domain inside the online softmax, so no [L, L] matrix is ever
-//    materialised; rows past L are zero-staged and masked (any L > 0);
-//  * workgroups of the N MSA rows that share one (b, h, query block) are adjacent in the grid, so
-//    their pair-bias tile is read from L2 once per row group rather than from HBM per row;
-//  * dbias2 = sum over the N rows of dS: fp32 global atomics (vector memory) from the dK/dV
-//    kernel; dbias1 = sum over heads and queries: per-lane register sums, one atomic per key.
+// What bounds it: with D = 32 a score costs 4 matrix-core cycles and ~11 VALU ones (bias, exponent, sums, rounding), so
+// every access and instruction a score has to pay for counts. Structure:
+//  * swapped products (S^T = K Q^T: one lane = one query's scores, lane-local softmax) on v_mfma_f32_32x32x16_bf16, the
+//    score accumulator reused as the B operand of O^T += V^T P^T; 128 queries (or keys) a workgroup, K / V (Q / dO) tiles
+//    of 64 rows direct to LDS in rows of D elements, two slots;
+//  * the pair bias is brought into the accumulator's order once a call (pack_pair: 2 x [H, L, L]), in the type it came in:
+//    a lane then reads its 16 scores' biases as 16-byte vectors (lane = query for the forward and dQ, lane = key for
+//    dK / dV and dbias2) one tile ahead. Read in place they are 16 loads of one value, each over 32 rows of the matrix;
+//  * the row mask is packed to fp32 in the log2 domain with -inf behind the last key, which is all the tail masking there
+//    is; rows behind L are read from a row of zeros;
+//  * dbias2 = sum of dS over the N rows has a kernel of its own that keeps a 64 x 128 tile of it in registers while it
+//    walks the rows (a third recomputation of dS costs less than L x L atomics a row and is deterministic); where that
+//    gives too few workgroups the rows are split and the parts added up by a last pass. dbias1: per-lane sums, one atomic
+//    a key;
+//  * delta = rowsum(dO O) is formed in the dQ kernel, which leaves it and the log2-domain LSE to the other two.
+// MSA row attention 1 x 128 x 384, 8 heads of 32, bf16 biases, MI355X, forward + backward: 1595 us with biases read in
+// place, dbias2 by atomics and delta by torch; see the kernels below for what each takes now.
 #include "sxe_common.h"
-#include "sxe_mfma.h"
+#include "sxe_tile.h"
 #include <torch/library.h>
+#include <type_traits>
 
 namespace sxe {
 namespace evo {
+using namespace tl;
 
-using namespace mf;
+constexpr int NW = 4, QB = 32 * NW, KT = 64;  // waves, rows of a workgroup, rows of a streamed tile
+constexpr int TAIL = 2 * KT * 4;              // bytes of a slot's two fp32 rows
 
-constexpr int QW = 32, NWV = 4, QB = QW * NWV, KT = 64, QT = 32;
+__device__ const __attribute__((aligned(128))) unsigned short kZeroRow[64] = {0};
 
 struct Args {
   const unsigned short *q, *k, *v, *dout, *o;
-  const float *lse, *delta;   // [BN, H, Lp]
-  const float *b1, *b2;       // [BN, L], [B, H, L, L] fp32 or null
+  const float* b1;        // packed row mask [B N, Lp]
+  const void *pq, *pk;    // packed pair bias, lane = query / lane = key; null: none
+  float *lse, *lse2, *ndelta;  // [B N, H, Lp]: natural log; log2 domain, -delta
   int B, N, L, H, Lp;
-  float scale;
+  float c;                // log2(e) / sqrt(D)
 };
 
-__device__ __forceinline__ void map_q(const Args& a, int nblk, int& b, int& n, int& h, int& blk) {
-  int idx = blockIdx.x;
-  n = idx % a.N;
-  idx /= a.N;
-  blk = idx % nblk;
-  idx /= nblk;
-  h = idx % a.H;
-  b = idx / a.H;
+// ------------------------------------------------------------------------------------ bias packing
+// One launch for both. bias1 (null: none) [B N, L] -> [B N, Lp] fp32 * log2(e), -inf behind L: the blocks of the last grid row.
+// bias2 [B H, L, L] -> 32 x 32 tiles in accumulator order: element (tile (a, b), half i / 8, lane, i % 8) is the value of
+// register i of that lane. pq: lane = query of tile row a, registers = keys of b; pk (may be null): lane = key of tile row
+// a, registers = queries of b. Grid: (nt * nt, B H + 1), nt = Lp / 32; without bias2 (64, 1).
+template <typename T>
+__global__ void __launch_bounds__(256) pack_kernel(const void* __restrict__ b1, int b1_bf16, float* __restrict__ mask, int64_t n1,
+                                                   const T* __restrict__ b2, T* __restrict__ pq, T* __restrict__ pk, int L, int nt) {
+  if (blockIdx.y == gridDim.y - 1) {
+    const int Lp = 32 * nt;
+    for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < n1; i += gridDim.x * 256ll) {
+      const int key = i % Lp;
+      const int64_t at = i / Lp * L + key;
+      float x = 0.f;
+      if (b1 != nullptr && key < L)
+        x = b1_bf16 ? bf16_to_f32(reinterpret_cast<const unsigned short*>(b1)[at]) : reinterpret_cast<const float*>(b1)[at];
+      mask[i] = key < L ? x * LOG2E : -INFINITY;
+    }
+    return;
+  }
+  __shared__ T t[32][33];
+  const int a = blockIdx.x / nt, b = blockIdx.x - a * nt;
+  const T* src = b2 + (int64_t)blockIdx.y * L * L;
+  for (int i = threadIdx.x; i < 1024; i += 256) {
+    const int q = 32 * a + i / 32, k = 32 * b + i % 32;
+    t[i / 32][i % 32] = q < L && k < L ? src[(int64_t)q * L + k] : (T)0;
+  }
+  __syncthreads();
+  const int64_t tiles = (int64_t)blockIdx.y * nt * nt;
+  for (int i = threadIdx.x; i < 1024; i += 256) {
+    const int reg = (i >> 9) * 8 + (i & 7), lane = (i >> 3) & 63, r = acc_row(reg, lane >> 5);
+    pq[(tiles + (int64_t)a * nt + b) * 1024 + i] = t[lane & 31][r];
+    if (pk != nullptr) pk[(tiles + (int64_t)b * nt + a) * 1024 + i] = t[r][lane & 31];
+  }
 }
 
-// (bias1[key] + bias2[query][key]) * log2(e) for the lane's 16 scores of key-half j
-__device__ __forceinline__ float bias_term(const Args& a, int bn, int b, int h, int q, int key) {
-  key = key < a.L ? key : a.L - 1;  // callers mask keys past L; the clamp keeps every load in bounds
-  q = q < a.L ? q : a.L - 1;
-  float t = 0.f;
-  if (a.b1) t += a.b1[(int64_t)bn * a.L + key];
-  if (a.b2) t += a.b2[(((int64_t)b * a.H + h) * a.L + q) * a.L + key];
-  return t * LOG2E;
+struct NoBias {};
+// waves a SIMD: what the registers allow without spills
+template <int D, typename BT>
+constexpr int min_waves() { return D == 32 && !std::is_same<BT, float>::value ? 3 : 2; }
+// a lane's 16 biases of one 32 x 32 tile
+template <typename BT>
+struct Bias {
+  u32x4 v[sizeof(BT)];
+  __device__ __forceinline__ void load(const void* packed, int64_t tile, int lane) {
+    const char* p = reinterpret_cast<const char*>(packed) + (tile * 1024 + lane * 8) * sizeof(BT);
+#pragma unroll
+    for (int i = 0; i < (int)sizeof(BT); ++i)  // halves are 512 elements apart, a half is sizeof(BT) / 2 vectors
+      v[i] = *reinterpret_cast<const u32x4*>(p + (sizeof(BT) == 2 ? i * 1024 : (i >> 1) * 2048 + (i & 1) * 16));
+  }
+  __device__ __forceinline__ float at(int i) const {
+    if constexpr (sizeof(BT) == 2) {
+      const unsigned x = v[i >> 3][(i & 7) >> 1];
+      return __uint_as_float(i & 1 ? x & 0xffff0000u : x << 16);
+    } else {
+      return __uint_as_float(v[i >> 2][i & 3]);
+    }
+  }
+};
+template <>
+struct Bias<NoBias> {
+  __device__ __forceinline__ void load(const void*, int64_t, int) {}
+};
+// (bias1 + bias2) * log2(e); m: the packed bias1
+template <typename BT>
+__device__ __forceinline__ float bias_term(const Bias<BT>& b, int i, float m) {
+  if constexpr (std::is_same<BT, NoBias>::value) return m;
+  else return __builtin_fmaf(b.at(i), LOG2E, m);
+}
+
+__device__ __forceinline__ void glds4(const void* src, char* dst) {
+  const unsigned a = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)lds +
+                                                    (unsigned)(dst - lds));
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(a), "v"(src) : "memory", "m0");
+}
+
+// rows row0 .. of x (rows of one (b, n), head h) to LDS; rows behind L are zeros
+template <int D>
+__device__ __forceinline__ void load_rows(char* dst, const unsigned short* x, int64_t rs, int row0, int L) {
+  load_tile<KT, D, NW>(dst, D / 8, [&](int r) { return row0 + r < L ? x + (int64_t)(row0 + r) * rs : kZeroRow; });
+}
+template <int D>
+__device__ __forceinline__ void frags(bf16x8 (&f)[D / 16], const unsigned short* x, int64_t rs, int row, int L, int hf) {
+#pragma unroll
+  for (int t = 0; t < D / 16; ++t)
+    f[t] = *reinterpret_cast<const bf16x8*>((row < L ? x + (int64_t)row * rs : kZeroRow) + 16 * t + 8 * hf);
+}
+// four floats of each register group of a lane half: rows 8 g + 4 hf .. of an LDS row of floats
+struct Rows16 {
+  f32x4 x[4];
+  __device__ __forceinline__ void load(const char* p, int first, int hf) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) x[g] = *reinterpret_cast<const f32x4*>(p + 4 * (first + 8 * g + 4 * hf));
+  }
+  __device__ __forceinline__ float at(int i) const { return x[i >> 2][i & 3]; }
+};
+
+struct Place {
+  int b, n, h, blk, bn;
+  int64_t rs, base, row;  // row stride; element of (b, n, 0, h, 0); row of the [B N, H, Lp] arrays
+};
+// The N rows that share a pair-bias tile are neighbours in the grid. (A row's blocks and heads on one XCD instead measured
+// the same: K / V traffic does not bound these kernels.)
+template <int D>
+__device__ __forceinline__ Place place(const Args& a) {
+  Place p;
+  int idx = blockIdx.x;
+  p.n = idx % a.N;
+  idx /= a.N;
+  const int nblk = a.Lp / QB;
+  p.blk = idx % nblk;
+  idx /= nblk;
+  p.h = idx % a.H;
+  p.b = idx / a.H;
+  p.bn = p.b * a.N + p.n;
+  p.rs = (int64_t)a.H * D;
+  p.base = (int64_t)p.bn * a.L * p.rs + (int64_t)p.h * D;
+  p.row = ((int64_t)p.bn * a.H + p.h) * a.Lp;
+  return p;
+}
+
+template <int D>
+__device__ __forceinline__ void store_rows(const f32x16 (&acc)[D / 32], unsigned short* out, float s, int hf) {
+#pragma unroll
+  for (int t = 0; t < D / 32; ++t) store_acc_t(acc[t], out + 32 * t + 4 * hf, s);
 }
 
 // ------------------------------------------------------------------------------------ forward
-template <int DH>
-__global__ void __launch_bounds__(256, 2) fwd_kernel(Args a, unsigned short* __restrict__ out, float* __restrict__ lse) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  constexpr int BUF = 2 * KT * ROWB;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 31, hf = lane >> 5;
-  const int nqb = (a.L + QB - 1) / QB;
-  int b, n, h, qb;
-  map_q(a, nqb, b, n, h, qb);
-  const int bn = b * a.N + n;
-  const int64_t rs = (int64_t)a.H * DH;  // row stride of [.., L, H, D]
-  const int64_t base = (int64_t)bn * a.L * rs + (int64_t)h * DH;
-  const int q = qb * QB + w * QW + r;
-  const int qc = q < a.L ? q : a.L - 1;
-  const float c = a.scale * LOG2E;
-
-  bf16x8 qf[DH / 16];
+template <int D, typename BT>
+__global__ void __launch_bounds__(256, (min_waves<D, BT>())) fwd_kernel(Args a, unsigned short* __restrict__ out) {
+  constexpr int TILE = KT * 2 * D, SLOT = 2 * TILE + TAIL;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, hf = lane >> 5;
+  const Place p = place<D>(a);
+  const int q0 = p.blk * QB + 32 * w, q = q0 + r, nt32 = a.Lp / 32;
+  const int64_t tiles = (((int64_t)p.b * a.H + p.h) * nt32 + q0 / 32) * nt32;
+  bf16x8 qf[D / 16];
+  frags<D>(qf, a.q + p.base, p.rs, q, a.L, hf);
+  f32x16 o[D / 32];
 #pragma unroll
-  for (int t = 0; t < DH / 16; ++t)
-    qf[t] = q < a.L ? *reinterpret_cast<const bf16x8*>(a.q + base + (int64_t)q * rs + 16 * t + 8 * hf)
-                    : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-  f32x16 oacc[DH / 32];
-#pragma unroll
-  for (int t = 0; t < DH / 32; ++t) oacc[t] = zero16();
+  for (int t = 0; t < D / 32; ++t) o[t] = zero16();
   float m = -INFINITY, l = 0.f;
-
-  const int ntiles = (a.L + KT - 1) / KT;
-  RowStager<KT, DH, 256> sk, sv;
-  sk.load(a.k + base, rs, 0, a.L);
-  sv.load(a.v + base, rs, 0, a.L);
-  sk.store(smem);
-  sv.store(smem + KT * ROWB);
+  const int n = (a.L + KT - 1) / KT;
+  auto load = [&](int t, char* slot) {
+    load_rows<D>(slot, a.k + p.base, p.rs, t * KT, a.L);
+    load_rows<D>(slot + TILE, a.v + p.base, p.rs, t * KT, a.L);
+    if (w == 0) glds4(a.b1 + (int64_t)p.bn * a.Lp + t * KT + lane, slot + 2 * TILE);
+  };
+  Bias<BT> bias[2], next[2];
+  load(0, lds);
+#pragma unroll
+  for (int j = 0; j < 2; ++j) next[j].load(a.pq, tiles + j, lane);
+  wait_loads();
   __syncthreads();
-  int cur = 0;
-  for (int t = 0; t < ntiles; ++t) {
-    const bool more = t + 1 < ntiles;
-    if (more) {
-      sk.load(a.k + base, rs, (t + 1) * KT, a.L);
-      sv.load(a.v + base, rs, (t + 1) * KT, a.L);
+  LaneOffs<D> lo;
+  lo.init(lane);
+  for (int t = 0; t < n; ++t) {
+    const char* kt = lds + (t & 1) * SLOT;
+    const char* vt = kt + TILE;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) bias[j] = next[j];
+    if (t + 1 < n) {
+      load(t + 1, lds + ((t & 1) ^ 1) * SLOT);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) next[j].load(a.pq, tiles + 2 * (t + 1) + j, lane);
     }
-    const int kbase = t * KT;
-    const char* kt = smem + cur * BUF;
-    const char* vt = kt + KT * ROWB;
-    f32x16 s[2];
+    if (q0 < a.L) {
+      f32x16 s[2];
+      float mx = -INFINITY;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      s[j] = zero16();
+      for (int j = 0; j < 2; ++j) {
+        s[j] = zero16();
 #pragma unroll
-      for (int t2 = 0; t2 < DH / 16; ++t2) s[j] = mfma(lds_row16(kt, 32 * j + r, 2 * t2 + hf), qf[t2], s[j]);
-    }
-    float mx = -INFINITY;
+        for (int t2 = 0; t2 < D / 16; ++t2) s[j] = mfma(row_at(kt + 32 * j * 2 * D, lo.row[t2]), qf[t2], s[j]);
+        Rows16 mask;
+        mask.load(vt + TILE, 32 * j, hf);
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int key = kbase + 32 * j + acc_row(i, hf);
-        const float bt = bias_term(a, bn, b, h, qc, key);
-        const float x = key < a.L ? __builtin_fmaf(s[j][i], c, bt) : -INFINITY;
-        s[j][i] = x;
-        mx = fmaxf(mx, x);
+        for (int i = 0; i < 16; ++i) {
+          s[j][i] = __builtin_fmaf(s[j][i], a.c, bias_term(bias[j], i, mask.at(i)));
+          mx = fmaxf(mx, s[j][i]);
+        }
       }
-    mx = fmaxf(mx, xor32(mx));
-    const bool grow = mx > m + 8.f;
-    const float mnew = grow ? mx : m;
-    const float mref = (mnew == -INFINITY) ? 0.f : mnew;
-    const float alpha = fast_exp2(m - mref);
-    float ps = 0.f;
+      mx = fmaxf(mx, xor32(mx));
+      const bool grow = mx > m + 8.f;  // lazy rescale: p <= 2^8
+      const float mnew = grow ? mx : m, mref = mnew == -INFINITY ? 0.f : mnew, alpha = fast_exp2(m - mref);
+      float ps = 0.f;
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float p = fast_exp2(s[j][i] - mref);
-        s[j][i] = p;
-        ps += p;
+        for (int i = 0; i < 16; ++i) {
+          s[j][i] = fast_exp2(s[j][i] - mref);
+          ps += s[j][i];
+        }
+      l = l * alpha + ps;
+      m = mnew;
+      if (__any(grow)) {
+#pragma unroll
+        for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
       }
-    l = l * alpha + ps;
-    m = mnew;
-    if (__any(grow)) {
 #pragma unroll
-      for (int dt = 0; dt < DH / 32; ++dt)
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) oacc[dt][i] *= alpha;
+        for (int s2 = 0; s2 < 2; ++s2) {
+          const bf16x8 pb = acc_to_b(s[j], s2);
+#pragma unroll
+          for (int dt = 0; dt < D / 32; ++dt) o[dt] = mfma(tr_at(vt + (32 * j + 16 * s2) * 2 * D, lo.tr[dt]), pb, o[dt]);
+        }
     }
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) {
-        const bf16x8 pb = acc_to_b(s[j], s2);
-#pragma unroll
-        for (int dt = 0; dt < DH / 32; ++dt) oacc[dt] = mfma(lds_trA(vt, 32 * j + 16 * s2, dt, lane), pb, oacc[dt]);
-      }
-    if (more) {
-      sk.store(smem + (cur ^ 1) * BUF);
-      sv.store(smem + (cur ^ 1) * BUF + KT * ROWB);
-    }
+    wait_loads();
     __syncthreads();
-    cur ^= 1;
   }
-  const float lt = l + xor32(l);
-  const float inv = lt > 0.f ? 1.f / lt : 0.f;
-  if (q < a.L) {
-    unsigned short* op = out + base + (int64_t)q * rs;
-#pragma unroll
-    for (int dt = 0; dt < DH / 32; ++dt)
-#pragma unroll
-      for (int rg = 0; rg < 4; ++rg) {
-        u16x4 pk;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) pk[e] = f32_to_bf16(oacc[dt][4 * rg + e] * inv);
-        *reinterpret_cast<u16x4*>(op + 32 * dt + 8 * rg + 4 * hf) = pk;
-      }
-  }
-  if (hf == 0 && q < a.Lp)
-    lse[((int64_t)bn * a.H + h) * a.Lp + q] = (q < a.L && lt > 0.f) ? (m + log2f(lt)) * LN2 : INFINITY;
+  l += xor32(l);
+  if (q < a.L) store_rows<D>(o, out + p.base + (int64_t)q * p.rs, l > 0.f ? 1.f / l : 0.f, hf);
+  if (hf == 0) a.lse[p.row + q] = q < a.L && l > 0.f ? (m + log2f(l)) * LN2 : INFINITY;
 }
 
 // ----------------------------------------------------------------------------------------- dQ
-template <int DH>
-__global__ void __launch_bounds__(256, 2) dq_kernel(Args a, unsigned short* __restrict__ dq) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  constexpr int BUF = 2 * KT * ROWB;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 31, hf = lane >> 5;
-  const int nqb = (a.L + QB - 1) / QB;
-  int b, n, h, qb;
-  map_q(a, nqb, b, n, h, qb);
-  const int bn = b * a.N + n;
-  const int64_t rs = (int64_t)a.H * DH;
-  const int64_t base = (int64_t)bn * a.L * rs + (int64_t)h * DH;
-  const int q = qb * QB + w * QW + r;
-  const int qc = q < a.L ? q : a.L - 1;
-  const float c = a.scale * LOG2E;
-  const int64_t li = ((int64_t)bn * a.H + h) * a.Lp + q;
-  const float lse2 = a.lse[li] * LOG2E, dlt = a.delta[li];
-  bf16x8 qf[DH / 16], df[DH / 16];
+template <int D, typename BT>
+__global__ void __launch_bounds__(256, (min_waves<D, BT>())) dq_kernel(Args a, unsigned short* __restrict__ dq) {
+  constexpr int TILE = KT * 2 * D, SLOT = 2 * TILE + TAIL;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, hf = lane >> 5;
+  const Place p = place<D>(a);
+  const int q0 = p.blk * QB + 32 * w, q = q0 + r, nt32 = a.Lp / 32;
+  const int64_t tiles = (((int64_t)p.b * a.H + p.h) * nt32 + q0 / 32) * nt32;
+  bf16x8 qf[D / 16], df[D / 16], of[D / 16];
+  frags<D>(qf, a.q + p.base, p.rs, q, a.L, hf);
+  frags<D>(df, a.dout + p.base, p.rs, q, a.L, hf);
+  frags<D>(of, a.o + p.base, p.rs, q, a.L, hf);
+  const int n = (a.L + KT - 1) / KT;
+  auto load = [&](int t, char* slot) {
+    load_rows<D>(slot, a.k + p.base, p.rs, t * KT, a.L);
+    load_rows<D>(slot + TILE, a.v + p.base, p.rs, t * KT, a.L);
+    if (w == 0) glds4(a.b1 + (int64_t)p.bn * a.Lp + t * KT + lane, slot + 2 * TILE);
+  };
+  Bias<BT> bias[2], next[2];
+  load(0, lds);
 #pragma unroll
-  for (int t = 0; t < DH / 16; ++t) {
-    const bool ok = q < a.L;
-    qf[t] = ok ? *reinterpret_cast<const bf16x8*>(a.q + base + (int64_t)q * rs + 16 * t + 8 * hf)
-               : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-    df[t] = ok ? *reinterpret_cast<const bf16x8*>(a.dout + base + (int64_t)q * rs + 16 * t + 8 * hf)
-               : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  for (int j = 0; j < 2; ++j) next[j].load(a.pq, tiles + j, lane);
+  const float lse2 = a.lse[p.row + q] * LOG2E;
+  float delta = 0.f;
+#pragma unroll
+  for (int t = 0; t < D / 16; ++t)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) delta += (float)df[t][e] * (float)of[t][e];
+  delta += xor32(delta);
+  if (hf == 0) {
+    a.lse2[p.row + q] = lse2;
+    a.ndelta[p.row + q] = -delta;
   }
-  f32x16 acc[DH / 32];
+  f32x16 acc[D / 32], nd;
 #pragma unroll
-  for (int t = 0; t < DH / 32; ++t) acc[t] = zero16();
-  const int ntiles = (a.L + KT - 1) / KT;
-  RowStager<KT, DH, 256> sk, sv;
-  sk.load(a.k + base, rs, 0, a.L);
-  sv.load(a.v + base, rs, 0, a.L);
-  sk.store(smem);
-  sv.store(smem + KT * ROWB);
+  for (int t = 0; t < D / 32; ++t) acc[t] = zero16();
+#pragma unroll
+  for (int i = 0; i < 16; ++i) nd[i] = -delta;
+  wait_loads();
   __syncthreads();
-  int cur = 0;
-  for (int t = 0; t < ntiles; ++t) {
-    const bool more = t + 1 < ntiles;
-    if (more) {
-      sk.load(a.k + base, rs, (t + 1) * KT, a.L);
-      sv.load(a.v + base, rs, (t + 1) * KT, a.L);
+  LaneOffs<D> lo;
+  lo.init(lane);
+  for (int t = 0; t < n; ++t) {
+    const char* kt = lds + (t & 1) * SLOT;
+    const char* vt = kt + TILE;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) bias[j] = next[j];
+    if (t + 1 < n) {
+      load(t + 1, lds + ((t & 1) ^ 1) * SLOT);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) next[j].load(a.pq, tiles + 2 * (t + 1) + j, lane);
     }
-    const int kbase = t * KT;
-    const char* kt = smem + cur * BUF;
-    const char* vt = kt + KT * ROWB;
+    if (q0 < a.L) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      f32x16 s = zero16(), dp = zero16();
+      for (int j = 0; j < 2; ++j) {
+        f32x16 s = zero16(), dp = nd;
 #pragma unroll
-      for (int t2 = 0; t2 < DH / 16; ++t2) {
-        s = mfma(lds_row16(kt, 32 * j + r, 2 * t2 + hf), qf[t2], s);
-        dp = mfma(lds_row16(vt, 32 * j + r, 2 * t2 + hf), df[t2], dp);
-      }
+        for (int t2 = 0; t2 < D / 16; ++t2) {
+          s = mfma(row_at(kt + 32 * j * 2 * D, lo.row[t2]), qf[t2], s);
+          dp = mfma(row_at(vt + 32 * j * 2 * D, lo.row[t2]), df[t2], dp);
+        }
+        Rows16 mask;
+        mask.load(vt + TILE, 32 * j, hf);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int key = kbase + 32 * j + acc_row(i, hf);
-        const float bt = bias_term(a, bn, b, h, qc, key);
-        const float p = key < a.L ? fast_exp2(__builtin_fmaf(s[i], c, bt) - lse2) : 0.f;
-        s[i] = p * (dp[i] - dlt);  // dS^T
-      }
+        for (int i = 0; i < 16; ++i)
+          s[i] = fast_exp2(__builtin_fmaf(s[i], a.c, bias_term(bias[j], i, mask.at(i))) - lse2) * dp[i];  // dS^T
 #pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) {
-        const bf16x8 db = acc_to_b(s, s2);
+        for (int s2 = 0; s2 < 2; ++s2) {
+          const bf16x8 db = acc_to_b(s, s2);
 #pragma unroll
-        for (int dt = 0; dt < DH / 32; ++dt) acc[dt] = mfma(lds_trA(kt, 32 * j + 16 * s2, dt, lane), db, acc[dt]);
+          for (int dt = 0; dt < D / 32; ++dt) acc[dt] = mfma(tr_at(kt + (32 * j + 16 * s2) * 2 * D, lo.tr[dt]), db, acc[dt]);
+        }
       }
     }
-    if (more) {
-      sk.store(smem + (cur ^ 1) * BUF);
-      sv.store(smem + (cur ^ 1) * BUF + KT * ROWB);
-    }
+    wait_loads();
     __syncthreads();
-    cur ^= 1;
   }
-  if (q < a.L) {
-    unsigned short* op = dq + base + (int64_t)q * rs;
-#pragma unroll
-    for (int dt = 0; dt < DH / 32; ++dt)
-#pragma unroll
-      for (int rg = 0; rg < 4; ++rg) {
-        u16x4 pk;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) pk[e] = f32_to_bf16(acc[dt][4 * rg + e] * a.scale);
-        *reinterpret_cast<u16x4*>(op + 32 * dt + 8 * rg + 4 * hf) = pk;
-      }
-  }
+  if (q < a.L) store_rows<D>(acc, dq + p.base + (int64_t)q * p.rs, a.c * LN2, hf);
 }
 
 // -------------------------------------------------------------------------------------- dK, dV
-// Keys on the lanes (32 per wave, 128 per workgroup); sweep every 32-query tile; Q / dO tiles and
-// their lse / delta staged through registers into a 2-slot LDS ring.
-constexpr int SLOT = 2 * QT * ROWB + 2 * QT * 4;
+// Keys on the lanes; Q / dO tiles and their LSE / -delta stream by.
+template <int D>
+__device__ __forceinline__ void load_query_tile(const Args& a, const unsigned short* q, const unsigned short* d, int64_t rs,
+                                                int64_t row, int q0, char* slot, int w, int lane) {
+  constexpr int TILE = KT * 2 * D;
+  load_rows<D>(slot, q, rs, q0, a.L);
+  load_rows<D>(slot + TILE, d, rs, q0, a.L);
+  if (w == 0) glds4(a.lse2 + row + q0 + lane, slot + 2 * TILE);
+  if (w == 1) glds4(a.ndelta + row + q0 + lane, slot + 2 * TILE + KT * 4);
+}
 
-template <int DH>
-__global__ void __launch_bounds__(256, 2) dkdv_kernel(Args a, unsigned short* __restrict__ dk,
-                                                      unsigned short* __restrict__ dv, float* __restrict__ db1,
-                                                      float* __restrict__ db2) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 31, hf = lane >> 5;
-  const int nkb = (a.L + QB - 1) / QB;
-  int b, n, h, kb;
-  map_q(a, nkb, b, n, h, kb);
-  const int bn = b * a.N + n;
-  const int64_t rs = (int64_t)a.H * DH;
-  const int64_t base = (int64_t)bn * a.L * rs + (int64_t)h * DH;
-  const int key = kb * QB + w * QW + r;
-  const bool kok = key < a.L;
-  const float c = a.scale * LOG2E;
-  bf16x8 kf[DH / 16], vf[DH / 16];
+// P and dS [query][key] of 32 queries of a slot, keys on the lanes (queries behind L: LSE inf, so P = 0)
+template <int D, typename BT>
+__device__ __forceinline__ void score_grads(f32x16& pr, f32x16& ds, const char* slot, int j, const LaneOffs<D>& lo,
+                                            const bf16x8 (&kf)[D / 16], const bf16x8 (&vf)[D / 16], const Bias<BT>& bias, float mask,
+                                            float c, int hf) {
+  constexpr int TILE = KT * 2 * D;
+  Rows16 ls, nd;
+  ls.load(slot + 2 * TILE, 32 * j, hf);
+  nd.load(slot + 2 * TILE + KT * 4, 32 * j, hf);
+  pr = zero16();
 #pragma unroll
-  for (int t = 0; t < DH / 16; ++t) {
-    kf[t] = kok ? *reinterpret_cast<const bf16x8*>(a.k + base + (int64_t)key * rs + 16 * t + 8 * hf)
-                : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-    vf[t] = kok ? *reinterpret_cast<const bf16x8*>(a.v + base + (int64_t)key * rs + 16 * t + 8 * hf)
-                : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-  }
-  f32x16 dka[DH / 32], dva[DH / 32];
+  for (int i = 0; i < 16; ++i) ds[i] = nd.at(i);
 #pragma unroll
-  for (int t = 0; t < DH / 32; ++t) {
-    dka[t] = zero16();
-    dva[t] = zero16();
+  for (int t = 0; t < D / 16; ++t) {
+    pr = mfma(row_at(slot + 32 * j * 2 * D, lo.row[t]), kf[t], pr);
+    ds = mfma(row_at(slot + TILE + 32 * j * 2 * D, lo.row[t]), vf[t], ds);
   }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    pr[i] = fast_exp2(__builtin_fmaf(pr[i], c, bias_term(bias, i, mask)) - ls.at(i));
+    ds[i] *= pr[i];
+  }
+}
+
+template <int D, typename BT>
+__global__ void __launch_bounds__(256, (min_waves<D, BT>())) dkdv_kernel(Args a, unsigned short* __restrict__ dk,
+                                                                   unsigned short* __restrict__ dv, float* __restrict__ db1) {
+  constexpr int TILE = KT * 2 * D, SLOT = 2 * TILE + TAIL;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, hf = lane >> 5;
+  const Place p = place<D>(a);
+  const int k0 = p.blk * QB + 32 * w, key = k0 + r, nt32 = a.Lp / 32;
+  const int64_t tiles = (((int64_t)p.b * a.H + p.h) * nt32 + k0 / 32) * nt32;
+  bf16x8 kf[D / 16], vf[D / 16];
+  frags<D>(kf, a.k + p.base, p.rs, key, a.L, hf);
+  frags<D>(vf, a.v + p.base, p.rs, key, a.L, hf);
+  const float mask = a.b1[(int64_t)p.bn * a.Lp + key];
+  f32x16 dka[D / 32], dva[D / 32];
+#pragma unroll
+  for (int t = 0; t < D / 32; ++t) dka[t] = dva[t] = zero16();
   float b1acc = 0.f;
-  const int ntq = (a.L + QT - 1) / QT;
-  const int64_t lrow = ((int64_t)bn * a.H + h) * a.Lp;
-  RowStager<QT, DH, 256> sq, sd;
-  float lreg = 0.f;
-  auto load = [&](int it) {
-    sq.load(a.q + base, rs, it * QT, a.L);
-    sd.load(a.dout + base, rs, it * QT, a.L);
-    if (threadIdx.x < 2 * QT) {
-      const int qq = it * QT + (threadIdx.x & (QT - 1));
-      lreg = threadIdx.x < QT ? a.lse[lrow + qq] : a.delta[lrow + qq];
-    }
-  };
-  auto store = [&](char* slot) {
-    sq.store(slot);
-    sd.store(slot + QT * ROWB);
-    if (threadIdx.x < 2 * QT) reinterpret_cast<float*>(slot + 2 * QT * ROWB)[threadIdx.x] = lreg;
-  };
-  load(0);
-  store(smem);
-  __syncthreads();
-  int cur = 0;
-  for (int it = 0; it < ntq; ++it) {
-    const bool more = it + 1 < ntq;
-    if (more) load(it + 1);
-    const char* slot = smem + cur * SLOT;
-    const char* qt = slot;
-    const char* dt_ = slot + QT * ROWB;
-    const float* l2 = reinterpret_cast<const float*>(slot + 2 * QT * ROWB);
-    const float* dl = l2 + QT;
-    const int qt0 = it * QT;
-    f32x16 s = zero16(), dp = zero16();
+  const int n = (a.L + KT - 1) / KT;
+  Bias<BT> bias[2], next[2];
+  load_query_tile<D>(a, a.q + p.base, a.dout + p.base, p.rs, p.row, 0, lds, w, lane);
 #pragma unroll
-    for (int t2 = 0; t2 < DH / 16; ++t2) {
-      s = mfma(lds_row16(qt, r, 2 * t2 + hf), kf[t2], s);    // S  [query][key]
-      dp = mfma(lds_row16(dt_, r, 2 * t2 + hf), vf[t2], dp);  // dP [query][key]
+  for (int j = 0; j < 2; ++j) next[j].load(a.pk, tiles + j, lane);
+  wait_loads();
+  __syncthreads();
+  LaneOffs<D> lo;
+  lo.init(lane);
+  for (int t = 0; t < n; ++t) {
+    const char* slot = lds + (t & 1) * SLOT;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) bias[j] = next[j];
+    if (t + 1 < n) {
+      load_query_tile<D>(a, a.q + p.base, a.dout + p.base, p.rs, p.row, (t + 1) * KT, lds + ((t & 1) ^ 1) * SLOT, w, lane);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) next[j].load(a.pk, tiles + 2 * (t + 1) + j, lane);
     }
+    if (k0 < a.L) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        f32x16 pr, ds;
+        score_grads<D>(pr, ds, slot, j, lo, kf, vf, bias[j], mask, a.c, hf);
+        if (db1 != nullptr) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) b1acc += ds[i];
+        }
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2) {
+          const bf16x8 pb = acc_to_b(pr, s2), db = acc_to_b(ds, s2);
+#pragma unroll
+          for (int dt = 0; dt < D / 32; ++dt) {
+            dva[dt] = mfma(tr_at(slot + TILE + (32 * j + 16 * s2) * 2 * D, lo.tr[dt]), pb, dva[dt]);  // dV^T += dO^T P
+            dka[dt] = mfma(tr_at(slot + (32 * j + 16 * s2) * 2 * D, lo.tr[dt]), db, dka[dt]);         // dK^T += Q^T dS
+          }
+        }
+      }
+    }
+    wait_loads();
+    __syncthreads();
+  }
+  if (key >= a.L) return;
+  if (db1 != nullptr) {
+    b1acc += xor32(b1acc);
+    if (hf == 0) atomicAdd(db1 + (int64_t)p.bn * a.L + key, b1acc);
+  }
+  store_rows<D>(dka, dk + p.base + (int64_t)key * p.rs, a.c * LN2, hf);
+  store_rows<D>(dva, dv + p.base + (int64_t)key * p.rs, 1.f, hf);
+}
+
+// -------------------------------------------------------------------------------------- dbias2
+// A workgroup holds dbias2 of 64 queries x 128 keys of one (b, h) and walks rows_per of the N rows. part: fp32 [parts,
+// B H, L, L]. Grid: (query tiles * key blocks * B H, parts), heads fastest: with 8 heads an XCD walks one head's rows
+// (82 us at 128 x 384 x 8 heads of 32; 103 us with the tiles of a head spread over the XCDs).
+template <int D, typename BT>
+__global__ void __launch_bounds__(256, (min_waves<D, BT>())) dpair_kernel(Args a, float* __restrict__ part, int rows_per) {
+  constexpr int TILE = KT * 2 * D, SLOT = 2 * TILE + TAIL;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, hf = lane >> 5;
+  const int nqt = (a.L + KT - 1) / KT, nkb = a.Lp / QB, nt32 = a.Lp / 32;
+  const int nbh = a.B * a.H, bh = blockIdx.x % nbh, kb = blockIdx.x / nbh % nkb, qt = blockIdx.x / nbh / nkb;
+  const int h = bh % a.H, b = bh / a.H;
+  const int k0 = kb * QB + 32 * w, key = k0 + r, q0 = qt * KT;
+  const int64_t rs = (int64_t)a.H * D;
+  Bias<BT> bias[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) bias[j].load(a.pk, ((int64_t)bh * nt32 + k0 / 32) * nt32 + 2 * qt + j, lane);
+  const int n0 = blockIdx.y * rows_per, n1 = min(a.N, n0 + rows_per);
+  f32x16 acc[2] = {zero16(), zero16()};
+  bf16x8 kf[D / 16], vf[D / 16], kn[D / 16], vn[D / 16];
+  float mask = 0.f, maskn = 0.f;
+  auto load = [&](int n, char* slot) {
+    const int bn = b * a.N + n;
+    const int64_t base = (int64_t)bn * a.L * rs + (int64_t)h * D;
+    load_query_tile<D>(a, a.q + base, a.dout + base, rs, ((int64_t)bn * a.H + h) * a.Lp, q0, slot, w, lane);
+    frags<D>(kn, a.k + base, rs, key, a.L, hf);
+    frags<D>(vn, a.v + base, rs, key, a.L, hf);
+    maskn = a.b1[(int64_t)bn * a.Lp + key];
+  };
+  if (n0 < n1) load(n0, lds);
+  wait_loads();
+  __syncthreads();
+  LaneOffs<D> lo;
+  lo.init(lane);
+  for (int n = n0; n < n1; ++n) {
+    const int cur = (n - n0) & 1;
+#pragma unroll
+    for (int t = 0; t < D / 16; ++t) {
+      kf[t] = kn[t];
+      vf[t] = vn[t];
+    }
+    mask = maskn;
+    if (n + 1 < n1) load(n + 1, lds + (cur ^ 1) * SLOT);
+    if (k0 < a.L) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        f32x16 pr, ds;
+        score_grads<D>(pr, ds, lds + cur * SLOT, j, lo, kf, vf, bias[j], mask, a.c, hf);
+        acc[j] += ds;
+      }
+    }
+    wait_loads();
+    __syncthreads();
+  }
+  if (key >= a.L) return;
+  float* out = part + ((int64_t)blockIdx.y * a.B * a.H + bh) * a.L * a.L + key;
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const int qi = acc_row(i, hf), qq = qt0 + qi;
-      const bool ok = kok && qq < a.L;
-      const float bt = bias_term(a, bn, b, h, qq, key);
-      const float p = ok ? fast_exp2(__builtin_fmaf(s[i], c, bt) - l2[qi] * LOG2E) : 0.f;
-      const float ds = p * (dp[i] - dl[qi]);
-      if (db2 != nullptr && ok) atomicAdd(db2 + (((int64_t)b * a.H + h) * a.L + qq) * a.L + key, ds);
-      b1acc += ds;
-      s[i] = p;
-      dp[i] = ds;
+      const int qq = q0 + 32 * j + acc_row(i, hf);
+      if (qq < a.L) out[(int64_t)qq * a.L] = acc[j][i];
     }
-#pragma unroll
-    for (int s2 = 0; s2 < 2; ++s2) {
-      const bf16x8 pb = acc_to_b(s, s2);
-      const bf16x8 db = acc_to_b(dp, s2);
-#pragma unroll
-      for (int t = 0; t < DH / 32; ++t) {
-        dva[t] = mfma(lds_trA(dt_, 16 * s2, t, lane), pb, dva[t]);  // dV^T += dO^T P
-        dka[t] = mfma(lds_trA(qt, 16 * s2, t, lane), db, dka[t]);   // dK^T += Q^T dS
-      }
-    }
-    if (more) store(smem + (cur ^ 1) * SLOT);
-    __syncthreads();
-    cur ^= 1;
-  }
-  const float b1tot = b1acc + xor32(b1acc);
-  if (db1 != nullptr && kok && hf == 0) atomicAdd(db1 + (int64_t)bn * a.L + key, b1tot);
-  if (kok) {
-    unsigned short* kop = dk + base + (int64_t)key * rs;
-    unsigned short* vop = dv + base + (int64_t)key * rs;
-#pragma unroll
-    for (int t = 0; t < DH / 32; ++t)
-#pragma unroll
-      for (int rg = 0; rg < 4; ++rg) {
-        u16x4 pk, pv;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          pk[e] = f32_to_bf16(dka[t][4 * rg + e] * a.scale);
-          pv[e] = f32_to_bf16(dva[t][4 * rg + e]);
-        }
-        *reinterpret_cast<u16x4*>(kop + 32 * t + 8 * rg + 4 * hf) = pk;
-        *reinterpret_cast<u16x4*>(vop + 32 * t + 8 * rg + 4 * hf) = pv;
-      }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256) dpair_sum_kernel(const float* __restrict__ part, T* __restrict__ out, int64_t n, int parts) {
+  for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < n; i += gridDim.x * 256ll) {
+    float s = 0.f;
+    for (int p = 0; p < parts; ++p) s += part[p * n + i];
+    if constexpr (sizeof(T) == 2) out[i] = f32_to_bf16(s);
+    else out[i] = s;
   }
 }
 
 }  // namespace evo
 
 // ------------------------------------------------------------------------------- host side
-static evo::Args evo_args(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
-                          const c10::optional<at::Tensor>& b1, const c10::optional<at::Tensor>& b2) {
+// 16-byte aligned storage (a view of a larger tensor may start anywhere)
+static at::Tensor evo_aligned(const at::Tensor& t) {
+  return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 ? t.clone() : t;
+}
+static bool evo_has(const c10::optional<at::Tensor>& t) { return t.has_value() && t->defined(); }
+
+struct EvoCall {
+  evo::Args a{};
+  at::Tensor q, k, v, b1, pq, pk;  // keep what the pointers look at
+  at::ScalarType pair = at::ScalarType::Undefined;
+};
+
+static EvoCall evo_call(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const c10::optional<at::Tensor>& b1,
+                        const c10::optional<at::Tensor>& b2, bool backward) {
   SXE_CHECK(q.dim() == 5 && q.sizes() == k.sizes() && q.sizes() == v.sizes(), "evoformer: q/k/v [B, N, L, H, D]");
   for (const at::Tensor* t : {&q, &k, &v})
     SXE_CHECK(t->is_contiguous() && t->scalar_type() == at::kBFloat16, "evoformer: contiguous bf16 q/k/v");
   const int D = q.size(4);
   SXE_CHECK(D == 32 || D == 64, "evoformer: head dim 32 or 64");
-  evo::Args a{};
+  EvoCall c;
+  evo::Args& a = c.a;
   a.B = q.size(0);
   a.N = q.size(1);
   a.L = q.size(2);
   a.H = q.size(3);
   a.Lp = (a.L + evo::QB - 1) / evo::QB * evo::QB;
-  a.scale = 1.f / std::sqrt((float)D);
-  a.q = reinterpret_cast<const unsigned short*>(q.data_ptr());
-  a.k = reinterpret_cast<const unsigned short*>(k.data_ptr());
-  a.v = reinterpret_cast<const unsigned short*>(v.data_ptr());
-  if (b1.has_value() && b1->defined()) {
-    SXE_CHECK(b1->scalar_type() == at::kFloat && b1->is_contiguous() && b1->numel() == (int64_t)a.B * a.N * a.L,
-              "evoformer: bias1 fp32 [B, N, 1, 1, L]");
-    a.b1 = b1->data_ptr<float>();
+  a.c = mf::LOG2E / std::sqrt((float)D);
+  c.q = evo_aligned(q);
+  c.k = evo_aligned(k);
+  c.v = evo_aligned(v);
+  a.q = reinterpret_cast<const unsigned short*>(c.q.data_ptr());
+  a.k = reinterpret_cast<const unsigned short*>(c.k.data_ptr());
+  a.v = reinterpret_cast<const unsigned short*>(c.v.data_ptr());
+  const int64_t rows = (int64_t)a.B * a.N;
+  auto ok = [](const at::Tensor& t) { return t.is_contiguous() && (t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16); };
+  c.b1 = at::empty({rows, a.Lp}, q.options().dtype(at::kFloat));
+  a.b1 = c.b1.data_ptr<float>();
+  if (evo_has(b1)) SXE_CHECK(ok(*b1) && b1->numel() == rows * a.L, "evoformer: bias1 fp32 / bf16 [B, N, 1, 1, L]");
+  const int nt = a.Lp / 32;
+  if (evo_has(b2)) {
+    SXE_CHECK(ok(*b2) && b2->numel() == (int64_t)a.B * a.H * a.L * a.L, "evoformer: bias2 fp32 / bf16 [B, 1, H, L, L]");
+    c.pair = b2->scalar_type();
+    c.pq = at::empty({(int64_t)a.B * a.H, a.Lp, a.Lp}, b2->options());
+    if (backward) c.pk = at::empty_like(c.pq);
+    a.pq = c.pq.data_ptr();
+    a.pk = backward ? c.pk.data_ptr() : nullptr;
   }
-  if (b2.has_value() && b2->defined()) {
-    SXE_CHECK(b2->scalar_type() == at::kFloat && b2->is_contiguous() &&
-                  b2->numel() == (int64_t)a.B * a.H * a.L * a.L, "evoformer: bias2 fp32 [B, 1, H, L, L]");
-    a.b2 = b2->data_ptr<float>();
-  }
-  return a;
+  if (rows * a.Lp == 0) return c;
+  auto pack = [&](auto* t) {
+    using T = std::remove_pointer_t<decltype(t)>;
+    const bool pair = evo_has(b2), has1 = evo_has(b1);
+    hipLaunchKernelGGL(evo::pack_kernel<T>, pair ? dim3(nt * nt, a.B * a.H + 1) : dim3(64, 1), dim3(256), 0, cur_stream(),
+                       has1 ? b1->data_ptr() : nullptr, has1 && b1->scalar_type() == at::kBFloat16, c.b1.data_ptr<float>(),
+                       rows * a.Lp, pair ? reinterpret_cast<const T*>(b2->data_ptr()) : nullptr,
+                       pair ? reinterpret_cast<T*>(c.pq.data_ptr()) : nullptr,
+                       pair && backward ? reinterpret_cast<T*>(c.pk.data_ptr()) : nullptr, a.L, nt);
+  };
+  if (c.pair == at::kBFloat16) pack((unsigned short*)nullptr);
+  else pack((float*)nullptr);
+  SXE_LAUNCH_CHECK();
+  return c;
+}
+
+// f(head dim constant, pair bias type tag)
+template <typename F>
+static void evo_dispatch(int D, at::ScalarType pair, F f) {
+  auto with = [&](auto d) {
+    if (pair == at::kBFloat16) f(d, (unsigned short)0);
+    else if (pair == at::kFloat) f(d, 0.f);
+    else f(d, evo::NoBias{});
+  };
+  if (D == 32) with(std::integral_constant<int, 32>{});
+  else with(std::integral_constant<int, 64>{});
 }
 
 std::vector<at::Tensor> evoformer_fwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
                                       const c10::optional<at::Tensor>& b1, const c10::optional<at::Tensor>& b2) {
   SXE_CHECK_CUDA(q);
-  evo::Args a = evo_args(q, k, v, b1, b2);
   c10::DeviceGuard g(q.device());
+  EvoCall c = evo_call(q, k, v, b1, b2, false);
+  evo::Args& a = c.a;
   auto o = at::empty_like(q);
   auto lse = at::empty({(int64_t)a.B * a.N, a.H, a.Lp}, q.options().dtype(at::kFloat));
   const int grid = a.B * a.N * a.H * (a.Lp / evo::QB);
-  const size_t lds = 4 * evo::KT * mf::ROWB;
-  static bool attr = false;
-  if (!attr) {
-    for (const void* f : {reinterpret_cast<const void*>(&evo::fwd_kernel<32>), reinterpret_cast<const void*>(&evo::fwd_kernel<64>),
-                          reinterpret_cast<const void*>(&evo::dq_kernel<32>), reinterpret_cast<const void*>(&evo::dq_kernel<64>)})
-      SXE_HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    attr = true;
-  }
-  auto* op = reinterpret_cast<unsigned short*>(o.data_ptr());
-  if (q.size(4) == 32)
-    hipLaunchKernelGGL(evo::fwd_kernel<32>, dim3(grid), dim3(256), lds, cur_stream(), a, op, lse.data_ptr<float>());
-  else
-    hipLaunchKernelGGL(evo::fwd_kernel<64>, dim3(grid), dim3(256), lds, cur_stream(), a, op, lse.data_ptr<float>());
+  if (grid == 0) return {o, lse};
+  a.lse = lse.data_ptr<float>();
+  evo_dispatch(q.size(4), c.pair, [&](auto d, auto t) {
+    constexpr int D = decltype(d)::value;
+    hipLaunchKernelGGL((evo::fwd_kernel<D, decltype(t)>), dim3(grid), dim3(256), 2 * (2 * evo::KT * 2 * D + evo::TAIL), cur_stream(),
+                       a, reinterpret_cast<unsigned short*>(o.data_ptr()));
+  });
   SXE_LAUNCH_CHECK();
   return {o, lse};
 }
 
-// delta [BN, H, Lp] = rowsum(dO * O) (padded rows 0) is computed by the caller.
-std::vector<at::Tensor> evoformer_bwd(const at::Tensor& dout, const at::Tensor& q, const at::Tensor& k,
-                                      const at::Tensor& v, const at::Tensor& lse, const at::Tensor& delta,
-                                      const c10::optional<at::Tensor>& b1, const c10::optional<at::Tensor>& b2,
-                                      bool need_db1, bool need_db2) {
+std::vector<at::Tensor> evoformer_bwd(const at::Tensor& dout, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                                      const at::Tensor& o, const at::Tensor& lse, const c10::optional<at::Tensor>& b1,
+                                      const c10::optional<at::Tensor>& b2, bool need_db1, bool need_db2) {
   SXE_CHECK_CUDA(q);
-  evo::Args a = evo_args(q, k, v, b1, b2);
-  SXE_CHECK(dout.sizes() == q.sizes() && dout.is_contiguous() && dout.scalar_type() == at::kBFloat16,
-            "evoformer_bwd: dout like q");
-  SXE_CHECK(lse.numel() == (int64_t)a.B * a.N * a.H * a.Lp && delta.numel() == lse.numel() &&
-                lse.scalar_type() == at::kFloat && delta.scalar_type() == at::kFloat && lse.is_contiguous() &&
-                delta.is_contiguous(), "evoformer_bwd: lse / delta fp32 [B*N, H, Lp]");
   c10::DeviceGuard g(q.device());
-  a.dout = reinterpret_cast<const unsigned short*>(dout.data_ptr());
+  EvoCall c = evo_call(q, k, v, b1, b2, true);
+  evo::Args& a = c.a;
+  for (const at::Tensor* t : {&dout, &o})
+    SXE_CHECK(t->sizes() == q.sizes() && t->is_contiguous() && t->scalar_type() == at::kBFloat16, "evoformer_bwd: dout / o like q");
+  SXE_CHECK(lse.numel() == (int64_t)a.B * a.N * a.H * a.Lp && lse.scalar_type() == at::kFloat && lse.is_contiguous(),
+            "evoformer_bwd: lse fp32 [B*N, H, Lp]");
+  SXE_CHECK(!need_db2 || evo_has(b2), "evoformer_bwd: gradient of a bias2 that is not there");
+  const at::Tensor d = evo_aligned(dout), oo = evo_aligned(o);
+  auto stats = at::empty({2, lse.numel()}, lse.options());
+  a.dout = reinterpret_cast<const unsigned short*>(d.data_ptr());
+  a.o = reinterpret_cast<const unsigned short*>(oo.data_ptr());
   a.lse = lse.data_ptr<float>();
-  a.delta = delta.data_ptr<float>();
+  a.lse2 = stats.data_ptr<float>();
+  a.ndelta = a.lse2 + lse.numel();
   auto dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
   at::Tensor db1, db2;
   if (need_db1) db1 = at::zeros({a.B, a.N, 1, 1, a.L}, q.options().dtype(at::kFloat));
-  if (need_db2) db2 = at::zeros({a.B, 1, a.H, a.L, a.L}, q.options().dtype(at::kFloat));
+  if (need_db2) db2 = at::empty({a.B, 1, a.H, a.L, a.L}, b2->options());
   const int grid = a.B * a.N * a.H * (a.Lp / evo::QB);
-  const size_t lds_q = 4 * evo::KT * mf::ROWB, lds_kv = 2 * evo::SLOT;
+  if (grid == 0) {
+    if (need_db2) db2.zero_();
+    return {dq, dk, dv, need_db1 ? db1 : at::Tensor(), need_db2 ? db2 : at::Tensor()};
+  }
   auto* dqp = reinterpret_cast<unsigned short*>(dq.data_ptr());
   auto* dkp = reinterpret_cast<unsigned short*>(dk.data_ptr());
   auto* dvp = reinterpret_cast<unsigned short*>(dv.data_ptr());
-  float* b1p = need_db1 ? db1.data_ptr<float>() : nullptr;
-  float* b2p = need_db2 ? db2.data_ptr<float>() : nullptr;
-  if (q.size(4) == 32) {
-    hipLaunchKernelGGL(evo::dq_kernel<32>, dim3(grid), dim3(256), lds_q, cur_stream(), a, dqp);
-    hipLaunchKernelGGL(evo::dkdv_kernel<32>, dim3(grid), dim3(256), lds_kv, cur_stream(), a, dkp, dvp, b1p, b2p);
-  } else {
-    hipLaunchKernelGGL(evo::dq_kernel<64>, dim3(grid), dim3(256), lds_q, cur_stream(), a, dqp);
-    hipLaunchKernelGGL(evo::dkdv_kernel<64>, dim3(grid), dim3(256), lds_kv, cur_stream(), a, dkp, dvp, b1p, b2p);
-  }
+  evo_dispatch(q.size(4), c.pair, [&](auto dd, auto t) {
+    constexpr int D = decltype(dd)::value;
+    using BT = decltype(t);
+    const size_t lds = 2 * (2 * evo::KT * 2 * D + evo::TAIL);
+    hipLaunchKernelGGL((evo::dq_kernel<D, BT>), dim3(grid), dim3(256), lds, cur_stream(), a, dqp);
+    hipLaunchKernelGGL((evo::dkdv_kernel<D, BT>), dim3(grid), dim3(256), lds, cur_stream(), a, dkp, dvp,
+                       need_db1 ? db1.data_ptr<float>() : nullptr);
+    if constexpr (!std::is_same<BT, evo::NoBias>::value) if (need_db2) {
+      // as many parts as all run at once (a part of at least 8 rows): a second, part-filled round costs more than the
+      // longer walk
+      const int wgs = (a.L + evo::KT - 1) / evo::KT * (a.Lp / evo::QB) * a.B * a.H;
+      const int most = std::max(1, std::min((a.N + 7) / 8, evo::min_waves<D, BT>() * kNumCUs / wgs));
+      const int rows_per = (a.N + most - 1) / most, parts = (a.N + rows_per - 1) / rows_per;
+      const bool direct = parts == 1 && db2.scalar_type() == at::kFloat;
+      auto part = direct ? db2 : at::empty({parts, db2.numel()}, q.options().dtype(at::kFloat));
+      hipLaunchKernelGGL((evo::dpair_kernel<D, BT>), dim3(wgs, parts), dim3(256), lds, cur_stream(), a, part.template data_ptr<float>(),
+                         rows_per);
+      if (!direct) {
+        const dim3 gs(stream_grid(db2.numel(), 256));
+        if (db2.scalar_type() == at::kFloat)
+          hipLaunchKernelGGL(evo::dpair_sum_kernel<float>, gs, dim3(256), 0, cur_stream(), part.template data_ptr<float>(),
+                             db2.data_ptr<float>(), db2.numel(), parts);
+        else
+          hipLaunchKernelGGL(evo::dpair_sum_kernel<unsigned short>, gs, dim3(256), 0, cur_stream(), part.template data_ptr<float>(),
+                             reinterpret_cast<unsigned short*>(db2.data_ptr()), db2.numel(), parts);
+      }
+    }
+  });
   SXE_LAUNCH_CHECK();
   return {dq, dk, dv, need_db1 ? db1 : at::Tensor(), need_db2 ? db2 : at::Tensor()};
 }
@@ -478,8 +683,8 @@ std::vector<at::Tensor> evoformer_bwd(const at::Tensor& dout, const at::Tensor& 
 
 TORCH_LIBRARY_FRAGMENT(sxe, m) {
   m.def("evoformer_fwd(Tensor q, Tensor k, Tensor v, Tensor? bias1, Tensor? bias2) -> Tensor[]");
-  m.def("evoformer_bwd(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor lse, Tensor delta, Tensor? bias1, "
-        "Tensor? bias2, bool need_db1, bool need_db2) -> Tensor[]");
+  m.def("evoformer_bwd(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, Tensor? bias1, Tensor? bias2, "
+        "bool need_db1, bool need_db2) -> Tensor[]");
 }
 TORCH_LIBRARY_IMPL(sxe, CUDA, m) {
   m.impl("evoformer_fwd", &sxe::evoformer_fwd);

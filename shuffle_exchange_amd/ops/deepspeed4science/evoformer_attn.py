@@ -5,8 +5,8 @@ O = softmax(Q K^T / sqrt(D) + bias1 + bias2) V with Q/K/V [B, N, L, H, D], bias1
 (MSA row mask) and bias2 [B, 1, H, L, L] (pair bias), gradients for Q, K, V and both biases.
 
 GPU (bf16, head dim 32 / 64): the fused gfx950 flash kernels of csrc/kernels/evoformer.hip --
-biases added inside the online softmax, no L x L matrix materialised, dbias1 / dbias2 accumulated
-by the dK/dV kernel. Elsewhere (CPU, other dtypes / head dims): a query-chunked PyTorch computation
+biases added inside the online softmax, no L x L matrix of scores materialised, dbias1 accumulated by
+the dK/dV kernel, dbias2 by one of its own. Elsewhere (CPU, other dtypes / head dims): a query-chunked PyTorch computation
 (each chunk recomputed in the backward, so only one chunk's L x L probabilities are ever live).
 Parity with the CUTLASS kernel is unpinned (not vendored); the tests check the exact formula.
 """
@@ -53,14 +53,18 @@ def _hip_ok(Q, K, V):
             and Q.shape == K.shape == V.shape and Q.shape[-3] > 0)
 
 
+def _bias(b):
+    """A bias as the kernels take it: contiguous, bf16 or fp32."""
+    return None if b is None else (b if b.dtype in (torch.bfloat16, torch.float32) else b.float()).contiguous()
+
+
 class EvoformerFusedAttention(torch.autograd.Function):
     """Fused HIP forward / backward (evoformer.hip); returns dbias1 / dbias2 in the bias dtypes."""
 
     @staticmethod
     def forward(ctx, q, k, v, bias1=None, bias2=None):
         q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
-        b1 = bias1.float().contiguous() if bias1 is not None else None
-        b2 = bias2.float().contiguous() if bias2 is not None else None
+        b1, b2 = _bias(bias1), _bias(bias2)
         o, lse = torch.ops.sxe.evoformer_fwd(q, k, v, b1, b2)
         ctx.save_for_backward(q, k, v, o, lse, b1, b2)
         ctx.bias_dtypes = (bias1.dtype if bias1 is not None else None, bias2.dtype if bias2 is not None else None)
@@ -69,14 +73,9 @@ class EvoformerFusedAttention(torch.autograd.Function):
     @staticmethod
     def backward(ctx, do):
         q, k, v, o, lse, b1, b2 = ctx.saved_tensors
-        B, N, L, H, _ = q.shape
-        Lp = lse.shape[-1]
-        delta = torch.zeros(B * N, H, Lp, dtype=torch.float32, device=q.device)
-        delta[:, :, :L] = (do.float() * o.float()).sum(-1).reshape(B * N, L, H).transpose(1, 2)
         need1 = b1 is not None and ctx.needs_input_grad[3]
         need2 = b2 is not None and ctx.needs_input_grad[4]
-        dq, dk, dv, db1, db2 = torch.ops.sxe.evoformer_bwd(do.contiguous().to(q.dtype), q, k, v, lse, delta, b1, b2,
-                                                           need1, need2)
+        dq, dk, dv, db1, db2 = torch.ops.sxe.evoformer_bwd(do.contiguous().to(q.dtype), q, k, v, o, lse, b1, b2, need1, need2)
         db1 = db1.to(ctx.bias_dtypes[0]) if need1 else None
         db2 = db2.to(ctx.bias_dtypes[1]) if need2 else None
         return dq, dk, dv, db1, db2

@@ -61,3 +61,54 @@ def test_evoformer_hip_kernels_vs_fp32(D, L):
     for name, a, b in zip("QKV12", grads, rgrads):
         err = ((a.float() - b).norm() / b.norm()).item()
         assert err < 2e-2, (name, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,N,L,H,D", [(1, 1, 1, 1, 32), (1, 17, 31, 3, 32), (1, 9, 64, 4, 64), (2, 33, 129, 2, 32), (1, 5, 200, 8, 32),
+                                       (1, 70, 128, 1, 64)])
+@pytest.mark.parametrize("bias", ["bf16", "fp32", "mask", "pair", "none"])
+def test_evoformer_tiles_and_biases(B, N, L, H, D, bias):
+    """Tile edges, a single key, more rows than one part of dbias2, every bias form; masked keys (-inf, the type's lowest
+    value, -1e9) and a row without any key left."""
+    torch.manual_seed(1)
+    mk = lambda *s: torch.randn(*s, device="cuda")
+    Q, K, V, g = (mk(B, N, L, H, D).bfloat16() for _ in range(4))
+    dt = torch.float32 if bias == "fp32" else torch.bfloat16
+    b1 = b2 = None
+    if bias in ("bf16", "fp32", "mask"):
+        b1 = mk(B, N, 1, 1, L)
+        b1[mk(B, N, 1, 1, L) > 1.5] = -1e9
+        b1[mk(B, N, 1, 1, L) > 2] = float("-inf")
+        b1[mk(B, N, 1, 1, L) > 2] = torch.finfo(torch.float32).min
+        b1[..., 0] = 0.5
+        b1[0, N - 1] = float("-inf")
+        b1 = b1.to(dt)
+    if bias in ("bf16", "fp32", "pair"):
+        b2 = (mk(B, 1, H, L, L) * 2).to(dt)
+    base = torch.empty(Q.numel() + 1, dtype=torch.bfloat16, device="cuda")  # a q that starts 2 bytes behind an aligned address
+    q = base[1:].view(Q.shape).copy_(Q)
+    ins = [t.requires_grad_(True) if t is not None else None for t in (q.detach(), K, V, b1, b2)]
+    out = ea.evoformer_attention(*ins)
+    live = [t for t in ins if t is not None]
+    grads = torch.autograd.grad(out, live, g)
+    ref = [t.detach().double().requires_grad_(True) if t is not None else None for t in ins]
+    r = [t.transpose(-2, -3) for t in ref[:3]]
+    s = r[0] @ r[1].transpose(-1, -2) / D ** 0.5
+    for t in ref[3:]:
+        s = s if t is None else s + t
+    p = torch.softmax(s, -1)
+    want = (torch.where(torch.isnan(p), torch.zeros_like(p), p) @ r[2]).transpose(-2, -3)
+    keep = torch.ones(B, N, 1, 1, 1, device="cuda", dtype=torch.bool)
+    if b1 is not None:
+        keep[0, N - 1] = False  # no key left: the output is zero and nothing flows back
+        assert out[0, N - 1].abs().max() == 0 and all(not t[0, N - 1].any() for t in grads[:3])
+    s2 = s.masked_fill(~keep, 0.0)  # the reference's own gradient of that row is nan: leave the row out of it
+    want_live = ((torch.softmax(s2, -1) * keep) @ r[2]).transpose(-2, -3)
+    rg = torch.autograd.grad(want_live, [t for t in ref if t is not None], g.double())
+    # p, ds and the results are rounded to 8 bits (2^-9 each, relative to their largest): 4 x 2^-9. A single key has dS = 0
+    # exactly; what is left of it is the rounding of o in delta, at most 2^-9 sum |do o| a row
+    slack = 2 ** -9 * (g.abs() * out.abs()).double().sum(-1).norm().item() * D ** 0.5 * (L == 1)
+    assert (out.double() - want).norm() <= 8e-3 * want.norm() + 1e-6
+    for a, b in zip(grads, rg):
+        assert a.dtype == (dt if a.shape != Q.shape else torch.bfloat16)
+        assert torch.isfinite(a).all() and (a.double() - b).norm() <= 8e-3 * b.norm() + slack, a.shape
