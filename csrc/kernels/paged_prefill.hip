@@ -211,8 +211,8 @@ void paged_merge(const at::Tensor& part_o, const at::Tensor& part_ml, const at::
 // q [T, nq, D], out [T, nq, D] (only the listed tokens are written); tiles int32 [n, 4] (sequence, first token row,
 // tokens, partial row), tokens * (nq / nkv) <= 128; splits > 1: rows int32 [R] is the token row of every partial row.
 void paged_prefill(const at::Tensor& q, const at::Tensor& cache, const at::Tensor& block_table, const at::Tensor& q_start,
-                   const at::Tensor& q_len, const at::Tensor& kv_len, const at::Tensor& tiles, const at::Tensor& rows,
-                   double scale, int64_t window, int64_t splits, int64_t keys_per_split, at::Tensor out) {
+                   const at::Tensor& q_len, const at::Tensor& kv_len, const at::Tensor& tiles,
+                   const c10::optional<at::Tensor>& rows, double scale, int64_t window, int64_t splits, int64_t keys_per_split, at::Tensor out) {
   SXE_CHECK_CUDA(q);
   SXE_CHECK(q.scalar_type() == at::kBFloat16 && cache.scalar_type() == at::kBFloat16 && out.scalar_type() == at::kBFloat16,
             "paged_prefill: bf16 only");
@@ -255,8 +255,9 @@ void paged_prefill(const at::Tensor& q, const at::Tensor& cache, const at::Tenso
   a.out_tok_stride = out.stride(0);
   at::Tensor part_o, part_ml;
   if (splits > 1) {
-    SXE_CHECK(rows.scalar_type() == at::kInt && rows.is_contiguous() && rows.is_cuda(), "paged_prefill: rows int32 [R]");
-    a.part_rows = rows.numel();
+    SXE_CHECK(rows.has_value() && rows->scalar_type() == at::kInt && rows->is_contiguous() && rows->is_cuda(),
+              "paged_prefill: rows int32 [R]");
+    a.part_rows = rows->numel();
     part_o = at::empty({splits, a.part_rows, nq, D}, q.options().dtype(at::kFloat));
     part_ml = at::empty({splits, a.part_rows, nq, 2}, q.options().dtype(at::kFloat));
     a.part_o = part_o.data_ptr<float>();
@@ -275,13 +276,13 @@ void paged_prefill(const at::Tensor& q, const at::Tensor& cache, const at::Tenso
   else if (D == 256) launch(whole ? pp::prefill_kernel<256, true> : pp::prefill_kernel<256, false>, lds);
   else SXE_CHECK(false, "paged_prefill: head_dim must be 64, 128 or 256");
   SXE_LAUNCH_CHECK();
-  if (splits > 1) paged_merge(part_o, part_ml, rows, out);
+  if (splits > 1) paged_merge(part_o, part_ml, *rows, out);
 }
 
 }  // namespace sxe
 
 TORCH_LIBRARY_FRAGMENT(sxe, m) {
   m.def("paged_prefill(Tensor q, Tensor cache, Tensor block_table, Tensor q_start, Tensor q_len, Tensor kv_len, "
-        "Tensor tiles, Tensor rows, float scale, int window, int splits, int keys_per_split, Tensor(a!) out) -> ()");
+        "Tensor tiles, Tensor? rows, float scale, int window, int splits, int keys_per_split, Tensor(a!) out) -> ()");
 }
 TORCH_LIBRARY_IMPL(sxe, CUDA, m) { m.impl("paged_prefill", &sxe::paged_prefill); }

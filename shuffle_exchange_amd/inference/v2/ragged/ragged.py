@@ -212,10 +212,11 @@ class DSStateManager:
 @dataclass
 class AttentionLists:
     """int32 device lists of one attention over a ragged batch: ``tiles`` [n, 4] (sequence, first token row, tokens, row among
-    ``tile_rows``), ``tile_rows`` the token rows they hold by sequence, ``tile_keys`` the longest key range; ``seqs`` [m, 2]
-    (sequence, row among ``seq_rows``), ``seq_rows``, ``seq_keys`` the same for the sequences outside the tiles (None: none)."""
+    the token rows that the tiles hold by sequence), ``tile_rows`` those rows (first row and count of each sequence until
+    ``RaggedBatch.tile_rows`` is asked for them), ``tile_keys`` the longest key range; ``seqs`` [m, 2] (sequence, row among
+    ``seq_rows``), ``seq_rows``, ``seq_keys`` the same for the sequences outside the tiles (None: none)."""
     tiles: torch.Tensor
-    tile_rows: torch.Tensor
+    tile_rows: object
     tile_keys: int
     seqs: Optional[torch.Tensor]
     seq_rows: Optional[torch.Tensor]
@@ -325,25 +326,31 @@ class RaggedBatch:
         up to ``tile`` tokens of the sequences that have, longest key range first, and the other sequences."""
         key = ("attention", tile, least)
         if key not in self._tables:
-            tiles, seqs, tile_rows, seq_rows, a, b = [], [], [], [], 0, 0
+            tiles, flat, held, rows, a = [], [], [], [], 0
             for i, (q, n, seen) in enumerate(zip(self.host_q_start, self.host_q_len, self.host_seen)):
                 if n >= least:
                     tiles += [(seen + min(j + tile, n), i, q + j, min(tile, n - j), a + j) for j in range(0, n, tile)]
-                    tile_rows.append(torch.arange(q, q + n, dtype=torch.int32))
+                    held.append((q, n))
                     a += n
                 elif n:
-                    seqs.append((i, b))
-                    seq_rows.append(torch.arange(q, q + n, dtype=torch.int32))
-                    b += n
+                    flat += [i, len(rows)]
+                    rows += range(q, q + n)
             if tiles:
                 tiles.sort(reverse=True)
+                nt, ns = len(tiles), len(flat) // 2
+                d = self._upload([x for t in tiles for x in t[1:]] + flat + rows, 1).view(-1)  # one copy to the device
                 self._tables[key] = AttentionLists(
-                    self._upload([t[1:] for t in tiles], 4), self._upload(torch.cat(tile_rows), 1).view(-1), tiles[0][0],
-                    self._upload(seqs, 2) if seqs else None, self._upload(torch.cat(seq_rows), 1).view(-1) if seqs else None,
-                    max((self.host_kv_len[i] for i, _ in seqs), default=0))
+                    d[:4 * nt].view(nt, 4), held, tiles[0][0], d[4 * nt:4 * nt + 2 * ns].view(ns, 2) if ns else None,
+                    d[4 * nt + 2 * ns:] if ns else None, max((self.host_kv_len[i] for i in flat[::2]), default=0))
             else:
                 self._tables[key] = None
         return self._tables[key]
+
+    def tile_rows(self, lists):
+        """int32 device list of the token rows that ``lists.tiles`` hold, sequence by sequence."""
+        if isinstance(lists.tile_rows, list):
+            lists.tile_rows = self._upload(torch.cat([torch.arange(q, q + n, dtype=torch.int32) for q, n in lists.tile_rows]), 1).view(-1)
+        return lists.tile_rows
 
     def _upload(self, rows, n):
         t = torch.as_tensor(rows, dtype=torch.int32).reshape(-1, n)

@@ -211,7 +211,8 @@ def ragged_attention(q, cache, batch, scale, window=None):
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     meta = (q, cache, batch.block_table, batch.q_start, batch.q_len, batch.kv_len)
     splits, keys = choose_tile_splits(lists.tiles.shape[0], nkv, lists.tile_keys)
-    torch.ops.sxe.paged_prefill(*meta, lists.tiles, lists.tile_rows, float(scale), int(window or 0), splits, keys, out)
+    rows = batch.tile_rows(lists) if splits > 1 else None
+    torch.ops.sxe.paged_prefill(*meta, lists.tiles, rows, float(scale), int(window or 0), splits, keys, out)
     if lists.seqs is not None:
         splits = choose_splits(lists.seqs.shape[0], nkv, lists.seq_keys)
         torch.ops.sxe.paged_attention_some(*meta, lists.seqs, lists.seq_rows, float(scale), int(lists.seq_keys), int(splits),

@@ -31,9 +31,10 @@ def test_lists_hold_every_token_once():
     keys = [seqs[s][0] + (q - b.host_q_start[s]) + n for s, q, n, _ in tiles]
     assert keys == sorted(keys, reverse=True) and x.tile_keys == keys[0] and max(t[2] for t in tiles) <= 32
     got = sorted(t for _, q, n, _ in tiles for t in range(q, q + n))
-    assert got == sorted(x.tile_rows.tolist()) and sorted(got + x.seq_rows.tolist()) == list(range(b.num_tokens))
+    rows = b.tile_rows(x)
+    assert got == sorted(rows.tolist()) and b.tile_rows(x) is rows and sorted(got + x.seq_rows.tolist()) == list(range(b.num_tokens))
     for _, q, n, at in tiles:
-        assert x.tile_rows[at:at + n].tolist() == list(range(q, q + n))
+        assert rows[at:at + n].tolist() == list(range(q, q + n))
     for s, at in x.seqs.tolist():
         assert x.seq_rows[at:at + seqs[s][1]].tolist() == list(range(b.host_q_start[s], b.host_q_start[s] + seqs[s][1]))
     assert x.seq_keys == 501 and b.attention_lists(32, 201) is None
