@@ -534,6 +534,17 @@ std::vector<at::Tensor> route_topk(const at::Tensor& h, const at::Tensor& router
   return out;
 }
 
+// logits fp32 [T, E] -> ex::choose
+std::vector<at::Tensor> route_choose(const at::Tensor& logits, int64_t k) {
+  SXE_CHECK_CUDA(logits);
+  SXE_CHECK(logits.dim() == 2 && logits.is_contiguous() && logits.scalar_type() == at::kFloat && logits.size(1) > 0 &&
+                logits.size(1) <= ex::kMaxE, "route_choose: logits fp32 [T, up to ", ex::kMaxE, "]");
+  c10::DeviceGuard g(logits.device());
+  auto out = ex::choose(logits, k);
+  SXE_LAUNCH_CHECK();
+  return out;
+}
+
 // Decode: v = x + rms(y) wp [+ add], h = rms(v) wn, then route_topk(h). Returns [v fp32 [M, K], h bf16 [M, K], route_topk's].
 std::vector<at::Tensor> route_sandwich(const at::Tensor& x, const at::Tensor& y, const at::Tensor& wp, const at::Tensor& wn,
                                        const c10::optional<at::Tensor>& slots, const c10::optional<at::Tensor>& add, double eps,
@@ -617,12 +628,14 @@ at::Tensor expert_gemm(const at::Tensor& x, const at::Tensor& w, const at::Tenso
 
 TORCH_LIBRARY_FRAGMENT(sxe, m) {
   m.def("route_topk(Tensor h, Tensor router, int k) -> Tensor[]");
+  m.def("route_choose(Tensor logits, int k) -> Tensor[]");
   m.def("route_sandwich(Tensor x, Tensor y, Tensor wp, Tensor wn, Tensor? slots, Tensor? add, float eps, Tensor router, int k) -> "
         "Tensor[]");
   m.def("expert_gemm(Tensor x, Tensor w, Tensor offs, Tensor active, Tensor? token, Tensor? ws, int R, int act) -> Tensor");
 }
 TORCH_LIBRARY_IMPL(sxe, CUDA, m) {
   m.impl("route_topk", &sxe::route_topk);
+  m.impl("route_choose", &sxe::route_choose);
   m.impl("route_sandwich", &sxe::route_sandwich);
   m.impl("expert_gemm", &sxe::expert_gemm);
 }

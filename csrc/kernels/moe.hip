@@ -108,9 +108,9 @@ __global__ void __launch_bounds__(NT) dispatch_kernel(const typename dt_traits<T
 }
 
 // out[t] = sum_c coef[t, c] * src[slots[t, c]]  (coef == nullptr: 1). Serves dispatch' and combine.
-template <DT T>
+template <DT T, typename I>
 __global__ void __launch_bounds__(NT) gather_sum_kernel(const typename dt_traits<T>::storage* __restrict__ src,
-                                                        const int64_t* __restrict__ slots,
+                                                        const I* __restrict__ slots,
                                                         const float* __restrict__ coef,
                                                         typename dt_traits<T>::storage* __restrict__ out,
                                                         int64_t S, int H, int k) {
@@ -227,8 +227,8 @@ at::Tensor moe_dispatch(const at::Tensor& x, const at::Tensor& slot_src, int64_t
 // and the combine forward
 at::Tensor moe_gather_sum(const at::Tensor& src, const at::Tensor& slots, const c10::optional<at::Tensor>& coef) {
   check_rows(src, "moe_gather_sum src");
-  SXE_CHECK(slots.scalar_type() == at::kLong && slots.dim() == 2 && slots.is_contiguous() && slots.is_cuda(),
-            "moe_gather_sum: int64 [S, k] slots");
+  SXE_CHECK((slots.scalar_type() == at::kLong || slots.scalar_type() == at::kInt) && slots.dim() == 2 && slots.is_contiguous() &&
+                slots.is_cuda(), "moe_gather_sum: int64 / int32 [S, k] slots");
   const float* cp = nullptr;
   if (coef.has_value()) {
     SXE_CHECK(coef->scalar_type() == at::kFloat && coef->is_contiguous() && coef->numel() == slots.numel(),
@@ -242,9 +242,13 @@ at::Tensor moe_gather_sum(const at::Tensor& src, const at::Tensor& slots, const 
   if (S == 0) return out;
   SXE_DISPATCH_DT(dtype_of(src), T, {
     using st = typename dt_traits<T>::storage;
-    hipLaunchKernelGGL(moe::gather_sum_kernel<T>, dim3(moe::row_grid(S)), dim3(moe::NT), 0, cur_stream(),
-                       reinterpret_cast<const st*>(src.data_ptr()), slots.data_ptr<int64_t>(), cp,
-                       reinterpret_cast<st*>(out.data_ptr()), S, H, k);
+    auto launch = [&](auto* sp) {
+      using I = std::remove_const_t<std::remove_pointer_t<decltype(sp)>>;
+      hipLaunchKernelGGL((moe::gather_sum_kernel<T, I>), dim3(moe::row_grid(S)), dim3(moe::NT), 0, cur_stream(),
+                         reinterpret_cast<const st*>(src.data_ptr()), sp, cp, reinterpret_cast<st*>(out.data_ptr()), S, H, k);
+    };
+    if (slots.scalar_type() == at::kLong) launch(slots.data_ptr<int64_t>());
+    else launch(slots.data_ptr<int>());
   });
   SXE_LAUNCH_CHECK();
   return out;

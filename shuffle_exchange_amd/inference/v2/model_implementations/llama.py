@@ -159,6 +159,17 @@ class RaggedLlama:
         return next(self.model.parameters()).device
 
     @property
+    def device_routing(self):
+        """A MoE model's expert counts stay on the device at decode, so its steps can be captured."""
+        from ....ops.moe import swiglu_experts_ok
+        if not self.is_moe or self.tps is not None or self.device.type != "cuda" or not self.moe_impl.use_hip_gating:
+            return False
+        probe = torch.empty(0, self.cfg.hidden_size, dtype=self.dtype, device=self.device)
+        moes = [(x.block_sparse_moe if hasattr(x, "block_sparse_moe") else x.moe).deepspeed_moe for x in self.model.layers]
+        return all(m.ep_size == 1 and hasattr(m.experts, "w_gate_up") and m.gate.wg.weight.dtype == self.dtype
+                   and swiglu_experts_ok(probe, m.experts.w_gate_up, m.experts.w_down) for m in moes)
+
+    @property
     def dtype(self):
         return next(self.model.parameters()).dtype
 
@@ -250,14 +261,21 @@ class RaggedLlama:
 
     def _moe_dropless(self, moe, m, w_gu=None, w_down=None):
         """Exact top-k routing for inference (no capacity, no dropped tokens): tokens are grouped
-        by expert (one argsort), each expert runs its two GEMMs on its rows, results are scattered
-        back weighted by the renormalised top-k gate probabilities (reference
-        ragged_ops/top_k_gating + moe_scatter + moe_gather)."""
+        by expert, each expert runs its two GEMMs on its rows, results are gathered back weighted by the
+        renormalised top-k gate probabilities (reference ragged_ops/top_k_gating + moe_scatter +
+        moe_gather): on the device where the expert kernels cover the sizes (ops/moe.swiglu_experts),
+        else with an argsort and a loop over the experts."""
         gate, ex = moe.gate, moe.experts
         assert moe.ep_size == 1, "ragged inference runs experts locally (ep_size == 1)"
         w_gu = ex.w_gate_up if w_gu is None else w_gu
         w_down = ex.w_down if w_down is None else w_down
         k = gate.k
+        from ....ops.moe import route_logits, route_topk, swiglu_experts, swiglu_experts_ok
+        if (self.moe_impl is not None and self.moe_impl.use_hip_gating and swiglu_experts_ok(m, w_gu, w_down)):
+            wg = gate.wg.weight
+            routing = (route_topk(m, wg, k) if wg.dtype == m.dtype and wg.is_contiguous()
+                       else route_logits(F.linear(m.float(), wg.float()), k))
+            return swiglu_experts(m, routing, w_gu, w_down)
         logits = F.linear(m.float(), gate.wg.weight.float())
         if self.moe_impl is not None and self.moe_impl.use_hip_gating and logits.is_cuda:
             from ....ops.moe import topk_softmax  # fused softmax + top-k kernel (moe.hip)

@@ -278,6 +278,15 @@ def route_topk(h, router, top):
     return Routing(idx.to(torch.int32), torch.softmax(val, -1))
 
 
+def route_logits(logits, top):
+    """``route_topk`` from fp32 logits [T, E]."""
+    if _hip(logits):
+        idx, wt, *lists = torch.ops.sxe.route_choose(logits.contiguous(), int(top))
+        return Routing(idx, wt, tuple(lists))
+    val, idx = logits.topk(top, dim=-1)
+    return Routing(idx.to(torch.int32), torch.softmax(val, -1))
+
+
 def fused_sandwich_route(x, y, post_weight, next_weight, eps, slots, add, router, top):
     """Decode (<= 4 rows): ``sandwich_norm`` (ops/residual_norm.py) and ``route_topk`` of its result in two
     launches: (x', h, Routing). None when not covered."""
@@ -312,3 +321,43 @@ def expert_mlp(h, routing, up, down, act="relu2"):
         a = f(F.linear(h.index_select(0, r // k).float(), up[e].float())).to(h.dtype)
         y[r] = (F.linear(a.float(), down[e].float()) * routing.weight.reshape(-1, 1)[r]).to(h.dtype)
     return y, torch.arange(R, dtype=torch.int32, device=h.device).view(T, k)
+
+
+# ---------------------------------------------------- routed SwiGLU experts, weights [E, K, N] as trained
+# Mean rows per expert up to which the streaming kernels are used. One layer of 8 experts, top 2, us streaming / library
+# (with its row counts read back): 4096 x 14336: 1 token 153 / 299, 16: 533 / 1051, 128: 599 / 968, 256 (64 rows each):
+# 866 / 1043, 384: 1177 / 1103; 2048 x 8192: 1: 52 / 150, 128: 202 / 487, 512 (128 rows): 448 / 565.
+KN_ROWS = 80
+
+
+def swiglu_experts_ok(x, w_gate_up, w_down):
+    """The kernels of csrc/kernels/experts_kn.hip cover these experts."""
+    return (_hip(x) and x.dtype == torch.bfloat16 and w_gate_up.is_cuda and w_gate_up.dtype == torch.bfloat16
+            and w_down.dtype == torch.bfloat16 and w_gate_up.is_contiguous() and w_down.is_contiguous()
+            and w_gate_up.shape[1] % 32 == 0 and w_gate_up.shape[2] % 128 == 0 and w_down.shape[1] % 32 == 0 and w_down.shape[2] % 128 == 0
+            and w_gate_up.shape[0] <= 1024 and w_gate_up.data_ptr() % 16 == 0 and w_down.data_ptr() % 16 == 0)
+
+
+def swiglu_experts(x, routing, w_gate_up, w_down):
+    """sum_j weight[t, j] * down_e(silu(gate_e x_t) * up_e x_t) over the choices of every token: x [T, K], w_gate_up
+    [E, K, 2 I], w_down [E, I, K] (``swiglu_experts_ok``), ``routing`` from route_topk / route_logits. Few rows per expert
+    stream the weights without a host synchronisation; more take a library product per expert, for which the row counts are
+    read back once."""
+    from .activation import swiglu
+    rows, _, slots, offs, active = routing.lists
+    x = x.contiguous()
+    E, R = w_gate_up.shape[0], rows.numel()
+    if R <= KN_ROWS * E or torch.cuda.is_current_stream_capturing():
+        h = torch.ops.sxe.expert_swiglu_kn(x, w_gate_up, offs, active, rows)
+        return torch.ops.sxe.expert_down_kn(h, w_down, offs, active, slots, routing.weight)
+    xs = x.index_select(0, rows)
+    gu = torch.empty(R, w_gate_up.shape[2], dtype=x.dtype, device=x.device)
+    y = torch.empty(R, w_down.shape[2], dtype=x.dtype, device=x.device)
+    bounds = offs.tolist()
+    spans = [(e, a, b) for e, (a, b) in enumerate(zip(bounds, bounds[1:])) if b > a]
+    for e, a, b in spans:
+        torch.mm(xs[a:b], w_gate_up[e], out=gu[a:b])
+    h = swiglu(gu)
+    for e, a, b in spans:
+        torch.mm(h[a:b], w_down[e], out=y[a:b])
+    return torch.ops.sxe.moe_gather_sum(y, slots, routing.weight)

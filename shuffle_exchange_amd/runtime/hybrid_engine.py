@@ -30,9 +30,12 @@ class SXEHybridEngine(SXEEngine):
         if self._ragged is None:
             from ..inference.v2 import RaggedInferenceEngineConfig, build_engine
             from ..inference.v2.engine_v2 import MemoryConfig, StateManagerConfig
+            from ..moe.utils import is_moe_param
             cfg = RaggedInferenceEngineConfig(state_manager=StateManagerConfig(
                 memory_config=MemoryConfig(fraction=self._he_cfg.kv_cache_fraction)),
                 tensor_parallel={"tp_size": int(self._he_cfg.inference_tp_size)})
+            # expert weights may move between generations (optimizer steps, gathers): their steps run eagerly
+            cfg.decode_graphs = not any(is_moe_param(p) for p in self.module.parameters())
             if not torch.cuda.is_available():
                 cfg.num_kv_blocks = 1024
                 cfg.kv_block_size = 16
