@@ -119,6 +119,7 @@ struct Args {
   float* part_o;   // [splits, T, nq, D]
   float* part_ml;  // [splits, T, nq, 2]
   int T;           // rows of a split's partials
+  int lazy;        // the merge leaves out partials whose maximum is -inf: a split without keys writes nothing else
   const int* seqs; // [n][2]: sequence, row of its first partial; null: all sequences, partials by token row
   int window;      // sliding window (Mistral / Qwen2): keys older than `window` positions are masked; 0 = off
   int* counters;   // [S * nkv] zeroed split-arrival counters: the last split of a (seq, kv head) merges; or null
@@ -149,7 +150,9 @@ constexpr int PR = 16;  // query rows per pass
 
 template <int D>
 struct PaGeo {
-  static constexpr int NT = D >= 256 ? 2 : 4;  // 16-key tiles per wave chunk (register budget at D = 256)
+  // 16-key tiles per wave chunk. D 128: 32 keys keep three workgroups a CU (148 registers, 33 KB) where 64 keep two: 24
+  // sequences of 270 - 5300 keys (heads 32 / 8) 49 against 60 us, 32 of 3000 keys 78 against 82 us
+  static constexpr int NT = D >= 128 ? 2 : 4;
   static constexpr int KC = 16 * NT;           // keys per wave chunk
   static constexpr int KS = D / 32;            // k-steps of the Q K^T product
   static constexpr int DT = D / 16;            // 16-wide d tiles of O^T
@@ -159,7 +162,7 @@ struct PaGeo {
 };
 
 template <int D>
-__global__ __launch_bounds__(256) void paged_attn_kernel(Args a) {
+__global__ __launch_bounds__(256, D == 256 ? 1 : 3) void paged_attn_kernel(Args a) {
   using P = PaGeo<D>;
   constexpr int NT = P::NT, KC = P::KC, KS = P::KS, DT = P::DT;
   extern __shared__ __attribute__((aligned(16))) char smem[];  // V images, then the wave-merge buffer
@@ -182,6 +185,15 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(Args a) {
   char* vimg = smem + wave * P::VIMG;
   float* mrg_o = reinterpret_cast<float*>(smem);  // [kWaves][PR][D] after the key loop
   const int krow = kperm(i >> 2) + (i & 3);        // this lane's key row in a tile (A operand of Q K^T)
+  if (a.lazy && k_begin >= kl) {  // a split behind the sequence's last key
+    for (int row = threadIdx.x; row < nrows_total; row += 256) {
+      const int tok = row / G, h = kvh * G + row - tok * G;
+      const int64_t pidx = ((int64_t)split * a.T + (a.seqs ? a.seqs[2 * item + 1] : qs) + tok) * a.nq + h;
+      a.part_ml[pidx * 2] = -INFINITY;
+      a.part_ml[pidx * 2 + 1] = 0.f;
+    }
+    return;
+  }
 
   for (int row0 = 0; row0 < nrows_total; row0 += PR) {
     const int nrows = min(PR, nrows_total - row0);
@@ -407,7 +419,7 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(Args a) {
 
 // Combine the splits' fp32 partials: D / 4 threads a (token, head) row, 16 bytes a load, every load of a group of up to U
 // splits issued before the first use (a loop that consumes each partial before loading the next makes a chain of
-// dependent ~1 us memory round trips: 10 us at 16 splits).
+// dependent ~1 us memory round trips: 10 us at 16 splits). Splits without keys (maximum -inf) are not read.
 template <int D, int U>
 __global__ __launch_bounds__(256) void merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                                     int splits, int64_t T, int nq, unsigned short* __restrict__ out,
@@ -425,10 +437,14 @@ __global__ __launch_bounds__(256) void merge_kernel(const float* __restrict__ pa
     f32x4 os[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t idx = (int64_t)min(s0 + u, splits - 1) * sstride + th;
-      ms[u] = part_ml[idx * 2];
-      ls[u] = part_ml[idx * 2 + 1];
-      os[u] = *reinterpret_cast<const f32x4*>(part_o + idx * D + d);
+      const float2 ml = *reinterpret_cast<const float2*>(part_ml + ((int64_t)min(s0 + u, splits - 1) * sstride + th) * 2);
+      ms[u] = s0 + u < splits ? ml.x : -INFINITY;
+      ls[u] = ml.y;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      os[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (ms[u] != -INFINITY) os[u] = *reinterpret_cast<const f32x4*>(part_o + ((int64_t)(s0 + u) * sstride + th) * D + d);
     }
     float Mc = M;
 #pragma unroll
@@ -561,7 +577,7 @@ static at::Tensor paged_attention_impl(const at::Tensor& q, const at::Tensor& ca
   c10::DeviceGuard g(q.device());
   splits = std::max<int64_t>(1, splits);
   int64_t kps = (std::max<int64_t>(max_kv_len, 1) + splits - 1) / splits;
-  kps = (kps + 63) / 64 * 64;  // whole wave chunks (64 keys; 32 at head dim 256)
+  kps = (kps + 63) / 64 * 64;  // whole wave chunks (64 keys; 32 from head dim 128)
   splits = (std::max<int64_t>(max_kv_len, 1) + kps - 1) / kps;
   at::Tensor part_o, part_ml;
   pa::Args a;
@@ -583,6 +599,7 @@ static at::Tensor paged_attention_impl(const at::Tensor& q, const at::Tensor& ca
   a.out_tok_stride = out.stride(0);
   a.T = rows ? rows->numel() : T;
   a.seqs = seqs ? seqs->data_ptr<int>() : nullptr;
+  a.lazy = splits > 1 && parts == nullptr && !counters.has_value();
   a.part_o = nullptr;
   a.part_ml = nullptr;
   a.window = (int)std::max<int64_t>(0, window);
