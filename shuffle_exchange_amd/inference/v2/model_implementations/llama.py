@@ -238,6 +238,22 @@ class RaggedLlama:
         a, h = (norm(x), x) if res is None else norm(x, res)
         return self._proj(mod, a, li, key), h
 
+    def _norm_glu(self, layer, x, res, li):
+        """(silu(gate) * up of the normed residual sum, the sum) through the streaming kernel at batched decode; (None, None)
+        when not covered."""
+        mlp, T = layer.mlp, x.shape[0]
+        if (self.tps is not None or not self.FUSE_MAX_T < T <= 32 or self.device.type != "cuda"
+                or getattr(mlp.gate_up_proj, "bias", None) is not None or not native.hip_available()):
+            return None, None
+        from ....ops.linear import glu_linear
+        # quantized layers run more than 16 rows on the module's own weight
+        w = self._wobj(mlp.gate_up_proj, li, "gu") if T <= 16 else mlp.gate_up_proj.weight
+        a, h = layer.post_attention_layernorm(x, res)
+        mid = glu_linear(a, w)
+        if mid is None:
+            mid = swiglu(self._proj(mlp.gate_up_proj, a, li, "gu"))
+        return mid, h
+
     def _mlp(self, layer, m, li=0, gu=None):
         """``gu``: the gate_up projection when the caller already ran it (fused with the norm)."""
         if hasattr(layer, "mlp"):
@@ -333,8 +349,12 @@ class RaggedLlama:
                 rope_kv_cache_append(qkv, rope, batch.positions, kv_layer, batch.slots, self.nq, self.nkv)
                 o = self._attn_o(attn, qkv, kv_layer, batch, li, T)
             if hasattr(layer, "mlp"):
-                gu, h2 = self._norm_proj(layer.post_attention_layernorm, o, h, layer.mlp.gate_up_proj, li, "gu")
-                x, res = self._mlp(layer, None, li, gu=gu), h2
+                mid, h2 = self._norm_glu(layer, o, h, li)
+                if mid is not None:
+                    x, res = self._proj(layer.mlp.down_proj, mid, li, "down"), h2
+                else:
+                    gu, h2 = self._norm_proj(layer.post_attention_layernorm, o, h, layer.mlp.gate_up_proj, li, "gu")
+                    x, res = self._mlp(layer, None, li, gu=gu), h2
             else:
                 m, h2 = layer.post_attention_layernorm(o, h)
                 x, res = self._mlp(layer, m, li), h2

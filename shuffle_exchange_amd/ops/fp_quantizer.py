@@ -239,7 +239,12 @@ class FP8Weight:
                 and x2.stride(-1) == 1 and x2.stride(0) % 8 == 0 and x2.data_ptr() % 16 == 0):
             native.require_hip()
             b = bias.to(torch.bfloat16).contiguous() if bias is not None else None
-            y = torch.ops.sxe.skinny_gemm_fp8w(x2, self.q.view(torch.uint8), self.scale, b)
+            q = self.q.view(torch.uint8)
+            # from 5 rows the streaming kernel: 8 rows, us: 28672 x 4096 36 -> 29, 4096 x 14336 21 -> 16.5, 4096 x 4096 8.0 -> 7.3
+            if x2.shape[0] > 4 and q.shape[0] % 4 == 0 and q.shape[0] > 0 and q.stride(0) % 16 == 0 and q.data_ptr() % 16 == 0:
+                y = torch.ops.sxe.stream_gemm(x2, q, self.scale, b, False)
+            else:
+                y = torch.ops.sxe.skinny_gemm_fp8w(x2, q, self.scale, b)
             return y.view(*x.shape[:-1], self.q.shape[0])
         return fp8_linear(x, self.q, self.scale, bias, out_dtype=x.dtype)
 

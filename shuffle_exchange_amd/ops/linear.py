@@ -54,6 +54,45 @@ def _skinny(x, weight, bias):
     return torch.ops.sxe.skinny_gemm(x2, weight, bias).view(*x.shape[:-1], weight.shape[0])
 
 
+# Batched decode: up to 16 rows, and up to 32 of a small weight, take the weight-streaming kernel (csrc/kernels/stream_gemm.hip).
+# Llama-3-8B shapes, us, hipBLASLt / streaming: 16 rows: QKV 14.2 / 14.8, o 15.5 / 9.7, gate | up 63.0 / 47.4, down 25.6 / 25.0,
+# 32000-row head 58.7 / 50.9; 32 rows: o 13.1 / 12.2, 3072 x 2048 11.1 / 6.9, but QKV 15.1 / 16.5, gate | up 53.6 / 53.4.
+STREAM_ROWS, STREAM_ROWS_SMALL, STREAM_SMALL = 16, 32, 1 << 24
+
+
+def _streamable(x2, weight, bias, unit=8):
+    return (x2.dtype == torch.bfloat16 and x2.stride(1) == 1 and x2.stride(0) % 8 == 0 and x2.data_ptr() % 16 == 0
+            and weight.dim() == 2 and weight.stride(1) == 1 and weight.stride(0) % unit == 0 and weight.data_ptr() % 16 == 0
+            and weight.shape[1] == x2.shape[1] and x2.shape[1] % unit == 0 and weight.shape[0] % 4 == 0 and weight.shape[0] > 0
+            and x2.shape[1] > 0 and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous())))
+
+
+def _stream(x, weight, bias):
+    if torch.compiler.is_compiling() or SKINNY_MAX_M <= 0 or weight.dtype != torch.bfloat16 or not weight.is_cuda:
+        return None
+    rows = x.numel() // max(1, x.shape[-1])
+    if not SKINNY_MAX_M < rows <= (STREAM_ROWS if weight.numel() > STREAM_SMALL else STREAM_ROWS_SMALL):
+        return None
+    x2 = x.reshape(-1, x.shape[-1])
+    if not _streamable(x2, weight, bias):
+        return None
+    from . import native
+    native.require_hip()
+    return torch.ops.sxe.stream_gemm(x2, weight, None, bias, False).view(*x.shape[:-1], weight.shape[0])
+
+
+def glu_linear(x, weight):
+    """silu(gate) * up of ``linear(x, weight)`` with weight = [gate | up], in ONE launch (stream_gemm.hip): 5 to 32 rows (16 of an
+    FP8Weight), no autograd; None when not covered. One rounding, of the result."""
+    wk = _pro_weight(weight)
+    if wk is None or torch.compiler.is_compiling() or not x.is_cuda or x.requires_grad or x.dim() != 2:
+        return None
+    w, sc = wk
+    if not 4 < x.shape[0] <= (32 if sc is None else 16) or w.shape[0] % 32 or not _streamable(x, w, None, 8 if sc is None else 16):
+        return None
+    return torch.ops.sxe.stream_gemm(x, w, sc, None, True)
+
+
 def _pro_weight(weight):
     """(w, scale) for the fused-prologue skinny kernels: a bf16 [N, K] tensor or an FP8Weight."""
     if isinstance(weight, torch.Tensor):
@@ -401,6 +440,8 @@ def linear(x, weight, bias=None):
         return _Linear.apply(x, weight, bias)
     if not grad and SKINNY_MAX_M > 0 and x.is_cuda:
         y = _skinny(x, weight, bias)
+        if y is None:
+            y = _stream(x, weight, bias)
         if y is not None:
             return y
     return F.linear(x, weight, bias)

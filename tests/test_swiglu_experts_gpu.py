@@ -6,6 +6,12 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(scope="module", autouse=True)
+def _native():
+    from shuffle_exchange_amd.ops import native
+    native.require_hip()
+
+
 def _reference(x, logits, k, w_gu, w_down):
     top, idx = logits.double().topk(k, -1)
     wt = torch.softmax(top, -1)
