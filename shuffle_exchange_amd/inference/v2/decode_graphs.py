@@ -18,6 +18,7 @@ while the HBM time of the step is ~2 ms. The reference captures CUDA graphs only
 MoE models whose expert counts go through the host and sliding windows narrower than the KV bucket run
 eagerly.
 """
+import numpy as np
 import torch
 
 MIN_KV_BUCKET = 256
@@ -50,6 +51,7 @@ class _StaticBatch:
         self.host_q_start = list(range(S))
         self.host_kv_len = [kv_bucket] * S
         self.rows = torch.arange(S, dtype=torch.int32, device=device)[:, None].repeat(1, 2)
+        self.order = np.arange(S)
         self.copied = None  # event: last H2D copy out of the pinned buffers
 
     def token_rows(self, below=None):
@@ -109,29 +111,26 @@ class DecodeGraphRunner:
     def _fill(self, sb, seqs, tokens):
         if sb.copied is not None:
             sb.copied.synchronize()  # the previous step's copy has left the pinned buffers
-        S, mb, bs = sb.num_seqs, sb.max_blocks, self.bs
-        h64, h32 = sb.h64.view(4, S), sb.h32
-        ids, pos, slots, last = h64.unbind(0)
-        qs, ql, kl, ss = h32[:4 * S].view(4, S).unbind(0)
-        bt = h32[4 * S:].view(S, mb)
-        scratch_slot = self.scratch_block * bs
-        ids.zero_()
-        pos.zero_()
-        slots.fill_(scratch_slot)
-        last.copy_(torch.arange(S))
-        qs.copy_(torch.arange(S, dtype=torch.int32))
-        ql.fill_(1)
-        kl.fill_(1)
-        ss.fill_(self.scratch_state)
-        bt.fill_(self.scratch_block)
-        for i, (s, t) in enumerate(zip(seqs, tokens)):
-            p = s.seen_tokens
-            ids[i] = int(t.reshape(-1)[0])
-            pos[i] = p
-            slots[i] = s.blocks[p // bs] * bs + p % bs
-            kl[i], ss[i] = p + 1, s.state_slot
+        S, mb, bs, n = sb.num_seqs, sb.max_blocks, self.bs, len(seqs)
+        # numpy views of the pinned buffers: a small numpy operation costs a tenth of a tensor one (24 sequences:
+        # 740 us of host time with tensors, 165 us so)
+        ids, pos, slots, last = sb.h64.numpy().reshape(4, S)
+        qs, ql, kl, ss = sb.h32.numpy()[:4 * S].reshape(4, S)
+        bt = sb.h32.numpy()[4 * S:].reshape(S, mb)
+        p = np.array([s.seen_tokens for s in seqs], dtype=np.int64)
+        ids[:n] = torch.cat([t.reshape(-1)[:1].to("cpu", torch.int64) for t in tokens]).numpy()
+        pos[:n] = p
+        slots[:n] = np.array([s.blocks[s.seen_tokens // bs] for s in seqs], dtype=np.int64) * bs + p % bs
+        last[:] = qs[:] = sb.order
+        ql.fill(1)
+        kl[:n] = p + 1
+        ss[:n] = [s.state_slot for s in seqs]
+        for i, s in enumerate(seqs):
             nb = len(s.blocks)
-            bt[i, :nb] = torch.tensor(s.blocks, dtype=torch.int32)
+            bt[i, :nb] = s.blocks
+            bt[i, nb:] = self.scratch_block
+        ids[n:] = pos[n:] = 0  # rows past the batch: one key in the scratch block
+        slots[n:], kl[n:], ss[n:], bt[n:] = self.scratch_block * bs, 1, self.scratch_state, self.scratch_block
         sb.d64.copy_(sb.h64, non_blocking=True)
         sb.d32.copy_(sb.h32, non_blocking=True)
         ev = torch.cuda.Event()
