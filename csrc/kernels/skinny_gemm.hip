@@ -10,14 +10,16 @@
 //    the 16 bytes at k0 + 32 s + 8 g, so each load instruction reads 64 contiguous bytes of each of
 //    16 rows and two consecutive steps complete the 128-byte lines (a lane-owns-128-bytes map was
 //    2x slower: 64 distinct lines per instruction);
-//  * one workgroup per 16 output columns, K split over its NW = 4/8 waves (NW = 8 for narrow N,
-//    so more waves per CU stream at once; 16 waves would cap VGPRs at 128 and spill), two super-steps of loads in flight per wave, partial
-//    tiles summed through NW KB of LDS.
+//  * one workgroup per 16 output columns (8 for M <= 4 where that measured faster: skinny_gemm_kernel), K split over its NW = 4/8
+//    waves (NW = 8 for narrow N, so more waves per CU stream at once; 16 waves would cap VGPRs at 128 and spill), two
+//    super-steps of loads in flight per wave, partial tiles summed through NW KB of LDS.
 //  * fused prologues (decode, M <= 4): PRO_RMS builds the GEMM input (residual add + RMSNorm) and
 //    PRO_SWIGLU (silu(gate) * up) in LDS inside the GEMM launch -- every workgroup recomputes the
 //    few KB of activations it needs (L2 hits) while its first weight super-step is already in
 //    flight, so the norm / gated-activation launches (4-5 us each at batch 1, latency-bound) are
 //    gone from the decode layer. Workgroup 0 also writes the new residual stream h = x + res.
+//  * SwiGLU in the epilogue of PRO_RMS (w = gate | up, a tile holds 8 (4) gate columns and their up columns): the down
+//    projection then has no prologue. One row, 8192 wide, us: 16384 x 2048 18.7 -> 17.9, 2048 x 8192 14.2 -> 9.4.
 #include "sxe_common.h"
 #include "sxe_sandwich.h"
 #include <torch/library.h>
@@ -38,20 +40,21 @@ struct Frag {
 // guide measures issued -> landed -18 % for a once-read cold weight stream)
 // (a kernel template parameter: with a runtime flag the compiler merges the two loads of one address
 // and drops the non-temporal hint)
-template <bool NT = false>
+template <bool NT, int STEP>
 __device__ __forceinline__ void load_w(Frag& f, const unsigned short* __restrict wrow, bool wok, int kbase, int K) {
 #pragma unroll
   for (int s = 0; s < 8; ++s) {
-    const int k = kbase + s * 32;
+    const int k = kbase + s * STEP;
     const bf16x8* p = reinterpret_cast<const bf16x8*>(wrow + k);
     if (wok && k < K) f.w[s] = NT ? __builtin_nontemporal_load(p) : *p;
     else f.w[s] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
   }
 }
+template <int STEP>
 __device__ __forceinline__ void load_x(Frag& f, const unsigned short* __restrict xrow, bool xok, int kbase, int K) {
 #pragma unroll
   for (int s = 0; s < 8; ++s) {
-    const int k = kbase + s * 32;
+    const int k = kbase + s * STEP;
     f.x[s] = (xok && k < K) ? *reinterpret_cast<const bf16x8*>(xrow + k) : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
   }
 }
@@ -80,6 +83,7 @@ struct ProArgs {
   unsigned short* rcache;
   int rnq, rnkv, rbs;
   int nt;  // non-temporal weight loads (SXE_SKINNY_NT)
+  int half;  // RMS: not 0: w = [gate | up] of `half` rows each, y [M, half] = silu(gate) * up of the fp32 sums
   // ADDNORM: norm AFTER a scaled residual sum over a 32-bit residual stream, v = alpha r + x, input =
   // rms(v) (offset + gw). r is given either as it is (rw == nullptr) or as an earlier such sum still to be
   // normalised: r = res32 rrinv[m] (offset + rw). hout32 = v and rinv_out = 1 / rms(v) are written by
@@ -98,26 +102,29 @@ struct ProArgs {
   // GATENORM: input = rms(x) gw sigmoid(gate)
 };
 
-// output column of lane `col` in tile `tile` (identity unless the RoPE epilogue pairs columns)
+// output column of column `col` of tile `tile` (identity unless the RoPE or SwiGLU epilogue pairs columns, partners CW / 2 apart)
+template <int CW>
 __device__ __forceinline__ int out_col(const ProArgs& p, int tile, int col) {
-  const int h = tile >> 3, j = tile & 7;
-  if (p.rcos == nullptr || h >= p.rnq + p.rnkv) return tile * 16 + col;
-  return h * 128 + (col < 8 ? 8 * j + col : 56 + 8 * j + col);
+  if (p.half) return tile * (CW / 2) + col + (col < CW / 2 ? 0 : p.half - CW / 2);
+  const int h = tile / (128 / CW), j = tile % (128 / CW);
+  if (p.rcos == nullptr || h >= p.rnq + p.rnkv) return tile * CW + col;
+  return h * 128 + j * (CW / 2) + col + (col < CW / 2 ? 0 : 64 - CW / 2);
 }
 
 // Wave-0 epilogue store of output (m, n) = v under the RoPE epilogue; every lane calls it (the pair
 // exchange is a whole-wave shuffle).
+template <int CW>
 __device__ __forceinline__ void rope_store(const ProArgs& p, float v, int m, int M, int n, int tile, int col,
                                            unsigned short* __restrict y, int64_t ldy) {
-  const int h = tile >> 3;
-  const float pv = __shfl_xor(v, 8, 64);
+  const int h = tile / (128 / CW);
+  const float pv = __shfl_xor(v, CW / 2, 64);
   if (m >= M) return;
   const int d = n - h * 128;
   float out = v;
   if (h < p.rnq + p.rnkv) {
     const int64_t ps = p.rpos[m];
     const float c = p.rcos[ps * 64 + (d & 63)], sn = p.rsin[ps * 64 + (d & 63)];
-    out = col < 8 ? v * c - pv * sn : v * c + pv * sn;
+    out = col < CW / 2 ? v * c - pv * sn : v * c + pv * sn;
   }
   const unsigned short ob = f32_to_bf16(out);
   y[(int64_t)m * ldy + n] = ob;
@@ -250,7 +257,7 @@ __device__ __forceinline__ void build_act(const unsigned short* __restrict x, in
   // U chunks of 8 per thread per round, every load of a round issued before the first use: a loop
   // that consumes each chunk before loading the next is a chain of dependent L2 round trips (it made
   // the fused down projection 9 us slower than the separate SwiGLU launch)
-  constexpr int U = MODE == PRO_ADDNORM ? 2 : 4;
+  constexpr int U = MODE == PRO_ADDNORM || MODE == PRO_RMS ? 2 : 4;
   __shared__ float red[NT / 64][kProMaxM];
   const int per = (khi - klo) / 8, n = M * per;
   float ss[kProMaxM] = {0.f, 0.f, 0.f, 0.f};
@@ -344,83 +351,96 @@ __device__ __forceinline__ void build_act(const unsigned short* __restrict x, in
   __syncthreads();
 }
 
-template <int NW, int MODE = PRO_NONE, bool NT = false>
-__global__ __launch_bounds__(NW * 64) void skinny_gemm_kernel(const unsigned short* __restrict x, int64_t ldx,
-                                                          const unsigned short* __restrict w, int64_t ldw,
-                                                          const unsigned short* __restrict bias,
-                                                          unsigned short* __restrict y, int64_t ldy, int M, int N,
-                                                          int K, int ss_per_wave, ProArgs pro) {
+// The sum over the waves (and the K slices of a narrow tile) and the store, by wave 0 of a workgroup. Full tiles: the lane's
+// rows are m = 4 g + r of column col; narrow ones (CW columns, M <= 4): lane = CW m + column, from the slices' diagonal blocks.
+template <int NW, int MODE, int CW, bool FP8>
+__device__ __forceinline__ void finish(const f32x4 (&red)[NW][64], int lane, int tile, const ProArgs& pro, const float* rinv,
+                                       const float* __restrict wscale, const unsigned short* __restrict bias,
+                                       unsigned short* __restrict y, int64_t ldy, int M, int N) {
+  constexpr int KS = 16 / CW;
+  constexpr bool kScaled = MODE == PRO_RMS || MODE == PRO_ADDNORM || MODE == PRO_SANDWICH || MODE == PRO_GATENORM;
+  const int col = lane % CW, n = MODE == PRO_RMS ? out_col<CW>(pro, tile, col) : tile * CW + col;
+  const float ws = FP8 && n < N ? wscale[n] : 1.f, b = bias != nullptr && n < N ? bf16_to_f32(bias[n]) : 0.f;
+  auto put = [&](float v, int m) {
+    v *= ws;
+    if constexpr (kScaled) v *= rinv[m < kProMaxM ? m : 0];
+    if (MODE == PRO_RMS && pro.rcos != nullptr) {  // (no bias: checked on the host)
+      rope_store<CW>(pro, v, m, M, n, tile, col, y, ldy);
+    } else if (MODE == PRO_RMS && pro.half) {  // whole tiles, no bias: checked on the host
+      const float up = __shfl_xor(v, CW / 2, 64);
+      if (m < M && col < CW / 2) y[(int64_t)m * ldy + n] = f32_to_bf16(v / (1.f + __expf(-v)) * up);
+    } else if (m < M && n < N) {
+      y[(int64_t)m * ldy + n] = f32_to_bf16(v + b);
+    }
+  };
+  if constexpr (KS == 1) {
+    f32x4 t = red[0][lane];
+#pragma unroll
+    for (int v = 1; v < NW; ++v) t += red[v][lane];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) put(t[r], 4 * (lane >> 4) + r);
+  } else {
+    const int m = lane / CW;  // from 4 on past the rows
+    float t = 0.f;
+#pragma unroll
+    for (int v = 0; v < NW; ++v)
+#pragma unroll
+      for (int sl = 0; sl < KS; ++sl) t += reinterpret_cast<const float*>(&red[v][16 * sl + CW * sl + col])[m & 3];
+    put(t, m);
+  }
+}
+
+// CW: columns of a tile. 16, or 8 for M <= 4 where 16 leave compute units idle: the matrix tile's 16 columns are then 8 columns
+// at KS = 2 slices of K (the first 32 K values of a step and the next), its rows the M rows at slice 0 and again at slice 1, and
+// the two blocks in which the slices agree are the sums. A load instruction then reads 128 contiguous bytes of 8 rows.
+template <int NW, int MODE, bool NT, int CW>
+__global__ __launch_bounds__(NW * 64, MODE == PRO_RMS ? 4 : 1) void skinny_gemm_kernel(
+    const unsigned short* __restrict x, int64_t ldx, const unsigned short* __restrict w, int64_t ldw,
+    const unsigned short* __restrict bias, unsigned short* __restrict y, int64_t ldy, int M, int N, int K, int ss_per_wave,
+    ProArgs pro) {
   __shared__ f32x4 red[NW][64];
   extern __shared__ __attribute__((aligned(16))) unsigned short act_lds[];  // PRO_*: the M x K input
+  constexpr int KS = 16 / CW, STEP = 32 * KS, SS = kSS * KS;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, g = lane >> 4;
   const int tile = blockIdx.x;
-  const int n = MODE == PRO_RMS ? out_col(pro, tile, col) : tile * 16 + col;
-  const bool wok = n < N, xok = col < M;
+  const int n = MODE == PRO_RMS ? out_col<CW>(pro, tile, col % CW) : tile * CW + col % CW;
+  const int m = KS == 1 ? col : col & 3;
+  const bool wok = n < N, xok = m < M && col < (KS == 1 ? 16 : 4 * KS);
   const unsigned short* wrow = w + (int64_t)(wok ? n : 0) * ldw;
-  const unsigned short* xrow = MODE == PRO_NONE ? x + (int64_t)(xok ? col : 0) * ldx
-                                                : act_lds + (int64_t)(xok ? col : 0) * K;
-  const int ss0 = wave * ss_per_wave;
+  const unsigned short* xrow = MODE == PRO_NONE ? x + (int64_t)(xok ? m : 0) * ldx : act_lds + (int64_t)(xok ? m : 0) * K;
+  const int ss0 = wave * ss_per_wave, kw = g * 8 + 32 * (col / CW), kx = g * 8 + (KS == 1 ? 0 : 32 * (col >> 2));
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   __shared__ float rinv[kProMaxM];
   Frag cur, nxt;
   if constexpr (MODE == PRO_NONE) {
-    load_w<NT>(cur, wrow, wok, ss0 * kSS + g * 8, K);
-    load_x(cur, xrow, xok, ss0 * kSS + g * 8, K);
+    load_w<NT, STEP>(cur, wrow, wok, ss0 * SS + kw, K);
+    load_x<STEP>(cur, xrow, xok, ss0 * SS + kx, K);
     for (int i = 0; i < ss_per_wave; ++i) {
       if (i + 1 < ss_per_wave) {
-        load_w<NT>(nxt, wrow, wok, (ss0 + i + 1) * kSS + g * 8, K);
-        load_x(nxt, xrow, xok, (ss0 + i + 1) * kSS + g * 8, K);
+        load_w<NT, STEP>(nxt, wrow, wok, (ss0 + i + 1) * SS + kw, K);
+        load_x<STEP>(nxt, xrow, xok, (ss0 + i + 1) * SS + kx, K);
       }
 #pragma unroll
       for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.x[s], cur.w[s], acc, 0, 0, 0);
       cur = nxt;
     }
   } else {
-    // the weight stream runs two super-steps ahead of the prologue, which builds the input in LDS
-    Frag nx2;
-    load_w<NT>(cur, wrow, wok, ss0 * kSS + g * 8, K);
-    if (ss_per_wave > 1) load_w<NT>(nxt, wrow, wok, (ss0 + 1) * kSS + g * 8, K);
+    // two super-steps of weights are in flight while the prologue builds the input in LDS
+    load_w<NT, STEP>(cur, wrow, wok, ss0 * SS + kw, K);
+    if (ss_per_wave > 1) load_w<NT, STEP>(nxt, wrow, wok, (ss0 + 1) * SS + kw, K);
     build_act<MODE, NW * 64>(x, ldx, M, K, 0, K, pro, act_lds, rinv);
     for (int i = 0; i < ss_per_wave; ++i) {
-      if (i + 2 < ss_per_wave) load_w<NT>(nx2, wrow, wok, (ss0 + i + 2) * kSS + g * 8, K);
-      load_x(cur, xrow, xok, (ss0 + i) * kSS + g * 8, K);
+      load_x<STEP>(cur, xrow, xok, (ss0 + i) * SS + kx, K);
 #pragma unroll
       for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.x[s], cur.w[s], acc, 0, 0, 0);
       cur = nxt;
-      nxt = nx2;
+      if (i + 2 < ss_per_wave) load_w<NT, STEP>(nxt, wrow, wok, (ss0 + i + 2) * SS + kw, K);
     }
   }
-  // acc: C[row m = 4 g + r][col n] -- sum the 4 waves' K partials
-  red[wave][lane] = acc;
+  red[wave][lane] = acc;  // C[row 4 g + r][col]
   __syncthreads();
-  if (wave == 0) {
-    f32x4 t = red[0][lane];
-#pragma unroll
-    for (int v = 1; v < NW; ++v) {
-      const f32x4 u = red[v][lane];
-      t[0] += u[0];
-      t[1] += u[1];
-      t[2] += u[2];
-      t[3] += u[3];
-    }
-    if (MODE == PRO_RMS && pro.rcos != nullptr) {  // RoPE epilogue (no bias: checked on the host)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = 4 * g + r;
-        rope_store(pro, t[r] * rinv[m < kProMaxM ? m : 0], m, M, n, tile, col, y, ldy);
-      }
-    } else if (n < N) {
-      const float b = bias ? bf16_to_f32(bias[n]) : 0.f;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = 4 * g + r;
-        constexpr bool kScaled = MODE == PRO_RMS || MODE == PRO_ADDNORM || MODE == PRO_SANDWICH || MODE == PRO_GATENORM;
-        const float sc = kScaled ? rinv[m < kProMaxM ? m : 0] : 1.f;
-        if (m < M) y[(int64_t)m * ldy + n] = f32_to_bf16(t[r] * sc + b);
-      }
-    }
-  }
+  if (wave == 0) finish<NW, MODE, CW, false>(red, lane, tile, pro, rinv, nullptr, bias, y, ldy, M, N);
 }
 
 // Waves per workgroup: NW = 8 (more waves streaming per CU) while the tiles still fit on the chip
@@ -464,7 +484,7 @@ __device__ __forceinline__ bf16x8 fp8x8_to_bf16(uint2 w) {
   return r;
 }
 
-template <int NW, int MODE = PRO_NONE>
+template <int NW, int MODE, int CW>
 __global__ __launch_bounds__(NW * 64) void skinny_gemm_fp8w_kernel(const unsigned short* __restrict x, int64_t ldx,
                                                                    const uint8_t* __restrict w, int64_t ldw,
                                                                    const float* __restrict wscale,
@@ -473,37 +493,39 @@ __global__ __launch_bounds__(NW * 64) void skinny_gemm_fp8w_kernel(const unsigne
                                                                    int N, int K, int ss_per_wave, ProArgs pro) {
   __shared__ f32x4 red[NW][64];
   extern __shared__ __attribute__((aligned(16))) unsigned short act_lds[];  // PRO_*: the M x K input
+  constexpr int KS = 16 / CW, STEP = 64 * KS, SS = kSS8 * KS;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, g = lane >> 4;
-  const int n = MODE == PRO_RMS ? out_col(pro, blockIdx.x, col) : blockIdx.x * 16 + col;
-  const bool wok = n < N, xok = col < M;
+  const int n = MODE == PRO_RMS ? out_col<CW>(pro, blockIdx.x, col % CW) : blockIdx.x * CW + col % CW;
+  const int m = KS == 1 ? col : col & 3;
+  const bool wok = n < N, xok = m < M && col < (KS == 1 ? 16 : 4 * KS);
   const uint8_t* wrow = w + (int64_t)(wok ? n : 0) * ldw;
-  const unsigned short* xrow = MODE == PRO_NONE ? x + (int64_t)(xok ? col : 0) * ldx
-                                                : act_lds + (int64_t)(xok ? col : 0) * K;
+  const unsigned short* xrow = MODE == PRO_NONE ? x + (int64_t)(xok ? m : 0) * ldx : act_lds + (int64_t)(xok ? m : 0) * K;
+  const int sw = 64 * (col / CW), sx = KS == 1 ? 0 : 64 * (col >> 2);  // the K slice of this lane's weight, of its input
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   __shared__ float rinv[kProMaxM];
   uint4 wv0[8];  // first super-step's weights: in flight while the prologue builds the input
   if constexpr (MODE != PRO_NONE) {
-    const int k0 = (wave * ss_per_wave) * kSS8 + 16 * g;
+    const int k0 = (wave * ss_per_wave) * SS + 16 * g + sw;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const int k = k0 + 64 * j;
+      const int k = k0 + STEP * j;
       wv0[j] = (wok && k < K && ss_per_wave > 0) ? *reinterpret_cast<const uint4*>(wrow + k) : uint4{0u, 0u, 0u, 0u};
     }
     build_act<MODE, NW * 64>(x, ldx, M, K, 0, K, pro, act_lds, rinv);
   }
   for (int i = 0; i < ss_per_wave; ++i) {
-    const int k0 = (wave * ss_per_wave + i) * kSS8 + 16 * g;
+    const int k0 = (wave * ss_per_wave + i) * SS + 16 * g;
     uint4 wv[8];
     bf16x8 xa[8], xb[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const int k = k0 + 64 * j;
-      const bool in = k < K;
+      const int k = k0 + STEP * j + sw, kx = k0 + STEP * j + sx;
+      const bool in = kx < K;
       if (MODE != PRO_NONE && i == 0) wv[j] = wv0[j];
-      else wv[j] = (wok && in) ? *reinterpret_cast<const uint4*>(wrow + k) : uint4{0u, 0u, 0u, 0u};
-      xa[j] = (xok && in) ? *reinterpret_cast<const bf16x8*>(xrow + k) : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-      xb[j] = (xok && in) ? *reinterpret_cast<const bf16x8*>(xrow + k + 8) : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      else wv[j] = (wok && k < K) ? *reinterpret_cast<const uint4*>(wrow + k) : uint4{0u, 0u, 0u, 0u};
+      xa[j] = (xok && in) ? *reinterpret_cast<const bf16x8*>(xrow + kx) : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      xb[j] = (xok && in) ? *reinterpret_cast<const bf16x8*>(xrow + kx + 8) : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -513,42 +535,92 @@ __global__ __launch_bounds__(NW * 64) void skinny_gemm_fp8w_kernel(const unsigne
   }
   red[wave][lane] = acc;
   __syncthreads();
-  if (wave == 0) {
-    f32x4 t = red[0][lane];
-#pragma unroll
-    for (int v = 1; v < NW; ++v) {
-      const f32x4 u = red[v][lane];
-      t[0] += u[0];
-      t[1] += u[1];
-      t[2] += u[2];
-      t[3] += u[3];
-    }
-    if (MODE == PRO_RMS && pro.rcos != nullptr) {  // RoPE epilogue (no bias: checked on the host)
-      const float sc = wscale[n];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = 4 * g + r;
-        rope_store(pro, t[r] * sc * rinv[m < kProMaxM ? m : 0], m, M, n, blockIdx.x, col, y, ldy);
-      }
-    } else if (n < N) {
-      const float sc = wscale[n];
-      const float b = bias ? bf16_to_f32(bias[n]) : 0.f;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = 4 * g + r;
-        const float rs = MODE == PRO_RMS ? rinv[m < kProMaxM ? m : 0] : 1.f;
-        if (m < M) y[(int64_t)m * ldy + n] = f32_to_bf16(t[r] * sc * rs + b);
-      }
-    }
-  }
+  if (wave == 0) finish<NW, MODE, CW, true>(red, lane, blockIdx.x, pro, rinv, wscale, bias, y, ldy, M, N);
 }
 
-// Waves per workgroup and super-steps per wave of the bf16 kernel. (A split-K variant -- K split
-// over 2-4 workgroups with a last-arrival reduction -- was measured and removed: 5.9 vs 3.7 ms per
-// batch-1 decode step, profiles/r05/decode_splitk_ab.log.)
-inline void plan(int tiles, int ss_total, int& nw, int& spw) {
-  nw = pick_nw(tiles, ss_total, 4, 1);
-  spw = (ss_total + nw - 1) / nw;
+// Tiles and waves of a launch. Narrow tiles read 128 contiguous bytes of a row a load and give small N twice the workgroups;
+// wide ones build the input half as often and leave every wave a super-step where K is small. One row, us, 16 / 8 columns:
+//   bf16 plain 2048 x 2048 4.9 / 4.0, 2048 x 8192 13.7 / 9.4, 4096 x 4096 10.0 / 9.3, 4096 x 14336 28.5 / 26.6, 32000 x 2048
+//   27.1 / 24.9; RMS 6144 x 4096 16.0 / 14.6, 28672 x 4096 48.6 / 46.6, 16384 x 2048 17.9 / 18.3
+//   e4m3 plain 2048 x 8192 9.1 / 6.9, 4096 x 4096 7.1 / 6.9, 32000 x 2048 16.9 / 18.9; RMS 6144 x 4096 13.0 / 11.1, 3072 x 2048
+//   6.5 / 7.0, 28672 x 4096 31.6 / 33.8
+// SwiGLU's and the merge's prologues are long: 2048 x 8192 14.2 / 10.7, but 3072 x 8192 15.2 / 16.5; merge of 16 splits
+// 2048 x 2048 7.9 / 7.1, 3072 x 3072 12.8 / 14.4 (four waves) and 10.5 (eight waves of wide tiles).
+// (A split-K variant -- K split over 2-4 workgroups with a last-arrival reduction -- was measured and removed: 5.9 vs 3.7 ms
+// per batch-1 decode step, profiles/r05/decode_splitk_ab.log.)
+struct Plan {
+  int cw, nw, spw, tiles;
+};
+inline Plan plan(int mode, int M, int N, int K, bool fp8) {
+  const int wide = (N + 15) / 16, ss = fp8 ? kSS8 : kSS;
+  bool narrow = M <= kProMaxM;
+  if (mode == PRO_NONE) narrow = narrow && (!fp8 || wide <= kNumCUs);
+  else if (mode == PRO_RMS) narrow = M == 1 && K >= 8 * ss && (!fp8 || 2 * wide <= 3 * kNumCUs);
+  else if (mode == PRO_SWIGLU) narrow = narrow && 2 * wide <= kNumCUs;
+  else if (mode == PRO_MERGE) narrow = narrow && 2 * wide <= kNumCUs && K <= 2048;
+  else narrow = false;
+  Plan p;
+  p.cw = narrow ? 8 : 16;
+  p.tiles = (N + p.cw - 1) / p.cw;
+  const int total = (K + ss * (16 / p.cw) - 1) / (ss * (16 / p.cw));
+  p.nw = pick_nw(p.tiles, total, fp8 ? 2 : 4, fp8 ? 2 : 1);
+  if (mode == PRO_MERGE ? !narrow && total >= 6 : narrow && p.tiles < 2 * kNumCUs && total >= 16) p.nw = 8;
+  p.spw = (total + p.nw - 1) / p.nw;
+  return p;
+}
+
+// LDS of the prologue past the default limit (once a kernel)
+template <auto KERN>
+void allow_lds() {
+  static const bool done = [] {
+    SXE_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(KERN), hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024));
+    return true;
+  }();
+  (void)done;
+}
+
+struct Operands {
+  const unsigned short* x;
+  int64_t ldx;
+  const at::Tensor* w;
+  const float* wscale;  // or null: bf16 weights
+  const unsigned short* bias;
+  at::Tensor* y;
+  int M, N, K;
+};
+
+template <int MODE, int NW, int CW>
+void launch_as(const Operands& o, const Plan& p, size_t lds, const ProArgs& pro) {
+  auto* yp = reinterpret_cast<unsigned short*>(o.y->data_ptr());
+  const dim3 grid(p.tiles), block(NW * 64);
+  auto bf16 = [&](auto nt) {
+    constexpr auto kern = &skinny_gemm_kernel<NW, MODE, decltype(nt)::value, CW>;
+    if (lds) allow_lds<kern>();
+    hipLaunchKernelGGL(kern, grid, block, lds, cur_stream(), o.x, o.ldx, reinterpret_cast<const unsigned short*>(o.w->data_ptr()),
+                       o.w->stride(0), o.bias, yp, o.y->stride(0), o.M, o.N, o.K, p.spw, pro);
+  };
+  if (o.wscale != nullptr) {
+    if constexpr (MODE <= PRO_MERGE) {
+      constexpr auto kern = &skinny_gemm_fp8w_kernel<NW, MODE, CW>;
+      if (lds) allow_lds<kern>();
+      hipLaunchKernelGGL(kern, grid, block, lds, cur_stream(), o.x, o.ldx, reinterpret_cast<const uint8_t*>(o.w->data_ptr()),
+                         o.w->stride(0), o.wscale, o.bias, yp, o.y->stride(0), o.M, o.N, o.K, p.spw, pro);
+    }
+  } else if (MODE <= PRO_MERGE && pro.nt) {
+    if constexpr (MODE <= PRO_MERGE) bf16(std::true_type{});
+  } else {
+    bf16(std::false_type{});
+  }
+  SXE_LAUNCH_CHECK();
+}
+
+template <int MODE>
+void launch(const Operands& o, const Plan& p, const ProArgs& pro) {
+  const size_t lds = MODE == PRO_NONE ? 0 : (size_t)o.M * o.K * 2;
+  if constexpr (MODE <= PRO_MERGE) {
+    if (p.cw == 8) return p.nw == 4 ? launch_as<MODE, 4, 8>(o, p, lds, pro) : launch_as<MODE, 8, 8>(o, p, lds, pro);
+  }
+  p.nw == 4 ? launch_as<MODE, 4, 16>(o, p, lds, pro) : launch_as<MODE, 8, 16>(o, p, lds, pro);
 }
 
 }  // namespace sg
@@ -573,22 +645,10 @@ at::Tensor skinny_gemm(const at::Tensor& x, const at::Tensor& w, const c10::opti
   auto y = at::empty({M, N}, x.options());
   if (N == 0) return y;
   c10::DeviceGuard gd(x.device());
-  const int ss_total = (K + sg::kSS - 1) / sg::kSS;
-  const int tiles = (N + 15) / 16;
-  int nw = 4, ss_per_wave = 1;
   sg::ProArgs pro{};
   pro.nt = sg::nt_loads();
-  sg::plan(tiles, ss_total, nw, ss_per_wave);
-  auto* xp = reinterpret_cast<const unsigned short*>(x.data_ptr());
-  auto* wp = reinterpret_cast<const unsigned short*>(w.data_ptr());
-  auto* yp = reinterpret_cast<unsigned short*>(y.data_ptr());
-#define SXE_SG_LAUNCH(NW, NT)                                                                              \
-  hipLaunchKernelGGL((sg::skinny_gemm_kernel<NW, sg::PRO_NONE, NT>), dim3(tiles), dim3(NW * 64), 0, cur_stream(), \
-                     xp, x.stride(0), wp, w.stride(0), bp, yp, y.stride(0), M, N, K, ss_per_wave, pro)
-  if (pro.nt) { if (nw == 4) SXE_SG_LAUNCH(4, true); else SXE_SG_LAUNCH(8, true); }
-  else { if (nw == 4) SXE_SG_LAUNCH(4, false); else SXE_SG_LAUNCH(8, false); }
-#undef SXE_SG_LAUNCH
-  SXE_LAUNCH_CHECK();
+  sg::launch<sg::PRO_NONE>({reinterpret_cast<const unsigned short*>(x.data_ptr()), x.stride(0), &w, nullptr, bp, &y, M, N, K},
+                           sg::plan(sg::PRO_NONE, M, N, K, false), pro);
   return y;
 }
 
@@ -615,22 +675,8 @@ at::Tensor skinny_gemm_fp8w(const at::Tensor& x, const at::Tensor& wq, const at:
   auto y = at::empty({M, N}, x.options());
   if (N == 0) return y;
   c10::DeviceGuard gd(x.device());
-  const int ss_total = (K + sg::kSS8 - 1) / sg::kSS8;
-  const int tiles = (N + 15) / 16;
-  const int nw = sg::pick_nw(tiles, ss_total, 2, 2);
-  const int ss_per_wave = (ss_total + nw - 1) / nw;
-  auto* xp = reinterpret_cast<const unsigned short*>(x.data_ptr());
-  auto* wp = reinterpret_cast<const uint8_t*>(wq.data_ptr());
-  auto* yp = reinterpret_cast<unsigned short*>(y.data_ptr());
-  if (nw == 4)
-    hipLaunchKernelGGL(sg::skinny_gemm_fp8w_kernel<4>, dim3(tiles), dim3(256), 0, cur_stream(), xp, x.stride(0), wp,
-                       wq.stride(0), wscale.data_ptr<float>(), bp, yp, y.stride(0), M, N, K, ss_per_wave,
-                       sg::ProArgs{});
-  else
-    hipLaunchKernelGGL(sg::skinny_gemm_fp8w_kernel<8>, dim3(tiles), dim3(512), 0, cur_stream(), xp, x.stride(0), wp,
-                       wq.stride(0), wscale.data_ptr<float>(), bp, yp, y.stride(0), M, N, K, ss_per_wave,
-                       sg::ProArgs{});
-  SXE_LAUNCH_CHECK();
+  sg::launch<sg::PRO_NONE>({reinterpret_cast<const unsigned short*>(x.data_ptr()), x.stride(0), &wq, wscale.data_ptr<float>(), bp, &y,
+                            M, N, K}, sg::plan(sg::PRO_NONE, M, N, K, true), sg::ProArgs{});
   return y;
 }
 
@@ -638,6 +684,8 @@ at::Tensor skinny_gemm_fp8w(const at::Tensor& x, const at::Tensor& wq, const at:
 // mode 1 (rms): x [M, K], res [M, K] or None (same row stride), gw [K], eps -> (y [M, N], h [M, K] = x + res)
 // mode 2 (swiglu): x = gu [M, 2K] (gate | up halves) -> y [M, N]
 // wq: bf16 [N, K] (wscale None) or e4m3 bytes [N, K] with wscale fp32 [N]
+// mode 3: mode 1 with w = gate | up and y [M, N / 2] = silu(gate) * up of the fp32 sums
+constexpr int64_t kRmsGlu = 3;
 struct RopeTensors {
   const at::Tensor *cos, *sin, *pos, *slots, *cache;
   int64_t nq, nkv;
@@ -649,7 +697,9 @@ static std::vector<at::Tensor> skinny_gemm_pro_impl(const at::Tensor& x, const c
                                                     const c10::optional<at::Tensor>& bias, int64_t mode,
                                                     const RopeTensors* rope) {
   SXE_CHECK_CUDA(x);
-  SXE_CHECK(mode == sg::PRO_RMS || mode == sg::PRO_SWIGLU, "skinny_gemm_pro: mode 1 (rms) or 2 (swiglu)");
+  const bool glu = mode == kRmsGlu;
+  if (glu) mode = sg::PRO_RMS;
+  SXE_CHECK(mode == sg::PRO_RMS || mode == sg::PRO_SWIGLU, "skinny_gemm_pro: mode 1 (rms), 2 (swiglu) or 3 (rms, swiglu epilogue)");
   SXE_CHECK(x.scalar_type() == at::kBFloat16 && x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0 &&
                 reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0, "skinny_gemm_pro: x bf16 [M, *], 16-B rows");
   const bool fp8 = wscale.has_value() && wscale->defined();
@@ -703,61 +753,20 @@ static std::vector<at::Tensor> skinny_gemm_pro_impl(const at::Tensor& x, const c
     SXE_CHECK(bias->scalar_type() == at::kBFloat16 && bias->is_contiguous() && bias->numel() == N, "bias: bf16 [N]");
     bp = reinterpret_cast<const unsigned short*>(bias->data_ptr());
   }
-  auto y = at::empty({M, N}, x.options());
+  SXE_CHECK(!glu || (N % 16 == 0 && bp == nullptr), "skinny_gemm_pro: gate and up of a multiple of 8 rows, no bias");
+  pro.half = glu ? N / 2 : 0;
+  auto y = at::empty({M, glu ? N / 2 : N}, x.options());
   if (N == 0) return {y, h.defined() ? h : x};
   c10::DeviceGuard gd(x.device());
   const size_t lds = (size_t)M * K * 2;
   SXE_CHECK(lds <= 144 * 1024, "skinny_gemm_pro: M x K input exceeds the LDS budget");
-  const int tiles = (N + 15) / 16;
-  auto* xp = reinterpret_cast<const unsigned short*>(x.data_ptr());
-  auto* yp = reinterpret_cast<unsigned short*>(y.data_ptr());
-  static bool attr[3][2][2] = {};  // [bf16 / fp8 / bf16 nt][NW == 8][mode]
-  auto set = [&](const void* f, int a, int b, int c) {
-    if (!attr[a][b][c]) {
-      SXE_HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024));
-      attr[a][b][c] = true;
-    }
-  };
-  const int mi = mode == sg::PRO_RMS ? 0 : 1;
-  if (!fp8) {
-    const int ss_total = (K + sg::kSS - 1) / sg::kSS;
-    int nw = 4, spw = 1;
-    sg::plan(tiles, ss_total, nw, spw);
-    auto* wp = reinterpret_cast<const unsigned short*>(w.data_ptr());
-#define SXE_SGP1(NW, MODE, NT)                                                                                       \
-  do {                                                                                                               \
-    set(reinterpret_cast<const void*>(&sg::skinny_gemm_kernel<NW, MODE, NT>), NT ? 2 : 0, NW == 8, mi);              \
-    hipLaunchKernelGGL((sg::skinny_gemm_kernel<NW, MODE, NT>), dim3(tiles), dim3(NW * 64), lds, cur_stream(), xp,     \
-                       x.stride(0), wp, w.stride(0), bp, yp, y.stride(0), M, N, K, spw, pro);                         \
-  } while (0)
-#define SXE_SGP(NW, MODE)                                                                                            \
-  do {                                                                                                               \
-    if (pro.nt) SXE_SGP1(NW, MODE, true);                                                                            \
-    else SXE_SGP1(NW, MODE, false);                                                                                  \
-  } while (0)
-    if (mode == sg::PRO_RMS) { if (nw == 4) SXE_SGP(4, sg::PRO_RMS); else SXE_SGP(8, sg::PRO_RMS); }
-    else { if (nw == 4) SXE_SGP(4, sg::PRO_SWIGLU); else SXE_SGP(8, sg::PRO_SWIGLU); }
-#undef SXE_SGP
-#undef SXE_SGP1
-  } else {
+  if (fp8)
     SXE_CHECK(wscale->scalar_type() == at::kFloat && wscale->is_contiguous() && wscale->numel() == N,
               "skinny_gemm_pro: wscale fp32 [N]");
-    const int ss_total = (K + sg::kSS8 - 1) / sg::kSS8;
-    const int nw = sg::pick_nw(tiles, ss_total, 2, 2);
-    const int spw = (ss_total + nw - 1) / nw;
-    auto* wp = reinterpret_cast<const uint8_t*>(w.data_ptr());
-    const float* sp = wscale->data_ptr<float>();
-#define SXE_SGP8(NW, MODE)                                                                                           \
-  do {                                                                                                               \
-    set(reinterpret_cast<const void*>(&sg::skinny_gemm_fp8w_kernel<NW, MODE>), 1, NW == 8, mi);                      \
-    hipLaunchKernelGGL((sg::skinny_gemm_fp8w_kernel<NW, MODE>), dim3(tiles), dim3(NW * 64), lds, cur_stream(), xp,    \
-                       x.stride(0), wp, w.stride(0), sp, bp, yp, y.stride(0), M, N, K, spw, pro);                     \
-  } while (0)
-    if (mode == sg::PRO_RMS) { if (nw == 4) SXE_SGP8(4, sg::PRO_RMS); else SXE_SGP8(8, sg::PRO_RMS); }
-    else { if (nw == 4) SXE_SGP8(4, sg::PRO_SWIGLU); else SXE_SGP8(8, sg::PRO_SWIGLU); }
-#undef SXE_SGP8
-  }
-  SXE_LAUNCH_CHECK();
+  const sg::Operands o{reinterpret_cast<const unsigned short*>(x.data_ptr()), x.stride(0), &w,
+                       fp8 ? wscale->data_ptr<float>() : nullptr, bp, &y, M, N, K};
+  if (mode == sg::PRO_RMS) sg::launch<sg::PRO_RMS>(o, sg::plan(mode, M, N, K, fp8), pro);
+  else sg::launch<sg::PRO_SWIGLU>(o, sg::plan(mode, M, N, K, fp8), pro);
   return {y, h.defined() ? h : x};
 }
 
@@ -810,53 +819,11 @@ at::Tensor skinny_gemm_merge(const at::Tensor& part_o, const at::Tensor& part_ml
   c10::DeviceGuard gd(part_o.device());
   const size_t lds = (size_t)M * K * 2;
   SXE_CHECK(lds <= 144 * 1024, "skinny_gemm_merge: M x K input exceeds the LDS budget");
-  const int tiles = (N + 15) / 16;
-  auto* yp = reinterpret_cast<unsigned short*>(y.data_ptr());
-  static bool attr[3][2] = {};  // [bf16 / fp8 / bf16 nt][NW == 8]
-  auto set = [&](const void* f, int a, int b) {
-    if (!attr[a][b]) {
-      SXE_HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024));
-      attr[a][b] = true;
-    }
-  };
-  if (!fp8) {
-    const int ss_total = (K + sg::kSS - 1) / sg::kSS;
-    int nw = 4, spw = 1;
-    sg::plan(tiles, ss_total, nw, spw);
-    auto* wp = reinterpret_cast<const unsigned short*>(w.data_ptr());
-#define SXE_SGM1(NW, NT)                                                                                             \
-  do {                                                                                                               \
-    set(reinterpret_cast<const void*>(&sg::skinny_gemm_kernel<NW, sg::PRO_MERGE, NT>), NT ? 2 : 0, NW == 8);         \
-    hipLaunchKernelGGL((sg::skinny_gemm_kernel<NW, sg::PRO_MERGE, NT>), dim3(tiles), dim3(NW * 64), lds,              \
-                       cur_stream(),                                                                                 \
-                       nullptr, K, wp, w.stride(0), bp, yp, y.stride(0), M, N, K, spw, pro);                          \
-  } while (0)
-#define SXE_SGM(NW)                                                                                                  \
-  do {                                                                                                               \
-    if (pro.nt) SXE_SGM1(NW, true);                                                                                  \
-    else SXE_SGM1(NW, false);                                                                                        \
-  } while (0)
-    if (nw == 4) SXE_SGM(4); else SXE_SGM(8);
-#undef SXE_SGM
-#undef SXE_SGM1
-  } else {
+  if (fp8)
     SXE_CHECK(wscale->scalar_type() == at::kFloat && wscale->is_contiguous() && wscale->numel() == N,
               "skinny_gemm_merge: wscale fp32 [N]");
-    const int ss_total = (K + sg::kSS8 - 1) / sg::kSS8;
-    const int nw = sg::pick_nw(tiles, ss_total, 2, 2);
-    const int spw = (ss_total + nw - 1) / nw;
-    auto* wp = reinterpret_cast<const uint8_t*>(w.data_ptr());
-    const float* sp = wscale->data_ptr<float>();
-#define SXE_SGM8(NW)                                                                                                 \
-  do {                                                                                                               \
-    set(reinterpret_cast<const void*>(&sg::skinny_gemm_fp8w_kernel<NW, sg::PRO_MERGE>), 1, NW == 8);                 \
-    hipLaunchKernelGGL((sg::skinny_gemm_fp8w_kernel<NW, sg::PRO_MERGE>), dim3(tiles), dim3(NW * 64), lds,            \
-                       cur_stream(), nullptr, K, wp, w.stride(0), sp, bp, yp, y.stride(0), M, N, K, spw, pro);        \
-  } while (0)
-    if (nw == 4) SXE_SGM8(4); else SXE_SGM8(8);
-#undef SXE_SGM8
-  }
-  SXE_LAUNCH_CHECK();
+  sg::launch<sg::PRO_MERGE>({nullptr, K, &w, fp8 ? wscale->data_ptr<float>() : nullptr, bp, &y, M, N, K},
+                            sg::plan(sg::PRO_MERGE, M, N, K, fp8), pro);
   return y;
 }
 
@@ -871,39 +838,16 @@ static at::Tensor skinny_launch(int mode, const unsigned short* xp, int64_t ldx,
   SXE_CHECK(lds <= 144 * 1024, "skinny gemm: M x K input exceeds the LDS budget");
   auto y = at::empty({M, N}, w.options());
   if (N == 0) return y;
-  const int ss_total = (K + sg::kSS - 1) / sg::kSS, tiles = (N + 15) / 16;
-  int nw = 4, spw = 1;
-  sg::plan(tiles, ss_total, nw, spw);
-  if (mode == sg::PRO_SANDWICH && (int64_t)M * K > 2 * 8 * 256) {  // the prologue keeps its rows in registers
-    nw = 8;
-    spw = (ss_total + nw - 1) / nw;
+  sg::Plan p = sg::plan(mode, M, N, K, false);
+  if (mode == sg::PRO_SANDWICH && (int64_t)M * K > 2 * 8 * 256 && p.nw == 4) {  // the prologue keeps its rows in registers
+    p.nw = 8;
+    p.spw = (p.spw + 1) / 2;
   }
-  pro.nt = sg::nt_loads();
-  static bool attr[8][2] = {};
-  auto go = [&](auto kern, int ni) {
-    bool& done = attr[mode][ni];
-    if (!done) {
-      SXE_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024));
-      done = true;
-    }
-    hipLaunchKernelGGL(kern, dim3(tiles), dim3(nw * 64), lds, cur_stream(), xp, ldx,
-                       reinterpret_cast<const unsigned short*>(w.data_ptr()), w.stride(0), (const unsigned short*)nullptr,
-                       reinterpret_cast<unsigned short*>(y.data_ptr()), y.stride(0), M, N, K, spw, pro);
-  };
-  if (mode == sg::PRO_ADDNORM) {
-    if (nw == 4) go(sg::skinny_gemm_kernel<4, sg::PRO_ADDNORM, false>, 0);
-    else go(sg::skinny_gemm_kernel<8, sg::PRO_ADDNORM, false>, 1);
-  } else if (mode == sg::PRO_SANDWICH) {
-    if (nw == 4) go(sg::skinny_gemm_kernel<4, sg::PRO_SANDWICH, false>, 0);
-    else go(sg::skinny_gemm_kernel<8, sg::PRO_SANDWICH, false>, 1);
-  } else if (mode == sg::PRO_GATENORM) {
-    if (nw == 4) go(sg::skinny_gemm_kernel<4, sg::PRO_GATENORM, false>, 0);
-    else go(sg::skinny_gemm_kernel<8, sg::PRO_GATENORM, false>, 1);
-  } else {
-    if (nw == 4) go(sg::skinny_gemm_kernel<4, sg::PRO_GATESUM, false>, 0);
-    else go(sg::skinny_gemm_kernel<8, sg::PRO_GATESUM, false>, 1);
-  }
-  SXE_LAUNCH_CHECK();
+  const sg::Operands o{xp, ldx, &w, nullptr, nullptr, &y, M, N, K};
+  if (mode == sg::PRO_ADDNORM) sg::launch<sg::PRO_ADDNORM>(o, p, pro);
+  else if (mode == sg::PRO_SANDWICH) sg::launch<sg::PRO_SANDWICH>(o, p, pro);
+  else if (mode == sg::PRO_GATENORM) sg::launch<sg::PRO_GATENORM>(o, p, pro);
+  else sg::launch<sg::PRO_GATESUM>(o, p, pro);
   return y;
 }
 

@@ -82,13 +82,13 @@ def _stream(x, weight, bias):
 
 
 def glu_linear(x, weight):
-    """silu(gate) * up of ``linear(x, weight)`` with weight = [gate | up], in ONE launch (stream_gemm.hip): 5 to 32 rows (16 of an
+    """silu(gate) * up of ``linear(x, weight)`` with weight = [gate | up], in ONE launch (stream_gemm.hip): up to 32 rows (16 of an
     FP8Weight), no autograd; None when not covered. One rounding, of the result."""
     wk = _pro_weight(weight)
     if wk is None or torch.compiler.is_compiling() or not x.is_cuda or x.requires_grad or x.dim() != 2:
         return None
     w, sc = wk
-    if not 4 < x.shape[0] <= (32 if sc is None else 16) or w.shape[0] % 32 or not _streamable(x, w, None, 8 if sc is None else 16):
+    if not 0 < x.shape[0] <= (32 if sc is None else 16) or w.shape[0] % 32 or not _streamable(x, w, None, 8 if sc is None else 16):
         return None
     return torch.ops.sxe.stream_gemm(x, w, sc, None, True)
 
@@ -127,6 +127,27 @@ def fused_rms_linear(x, residual, norm_weight, eps, weight, bias=None):
     if x.shape[1] != w.shape[1]:
         return None
     y, h = torch.ops.sxe.skinny_gemm_pro(x, residual, norm_weight, float(eps), w, sc, bias, 1)
+    return y, (h if residual is not None else x)
+
+
+# Rows x K up to which the GEMM builds its normed input itself; every workgroup does. us, one launch / norm and streaming kernel:
+# bf16, 1 x 4096 47.0 / 55.0, 2 x 4096 51.1 / 54.3, 4 x 2048 20.1 / 21.8, 3 x 3072 27.8 / 27.0, 4 x 4096 59.0 / 54.8;
+# e4m3, 1 x 4096 31.4 / 34.2, 1 x 3072 16.2 / 18.3, 2 x 4096 34.5 / 34.1, 4 x 2048 16.8 / 14.1
+RMS_GLU_BF16, RMS_GLU_FP8 = 8192, 4096
+
+
+def fused_rms_glu(x, residual, norm_weight, eps, weight):
+    """Decode (<= 4 rows): ``silu(gate) * up`` of ``linear(rms_norm(x + residual), [gate | up])`` in ONE launch (skinny_gemm.hip
+    PRO_RMS with the SwiGLU epilogue; one rounding, of the result). Returns (y, h) like ``fused_rms_linear``, or None."""
+    wk = _pro_weight(weight)
+    if (wk is None or not _pro_ok(x) or norm_weight.dtype != torch.bfloat16 or not norm_weight.is_contiguous()
+            or x.shape[1] != wk[0].shape[1] or wk[0].shape[0] % 16
+            or x.numel() > (RMS_GLU_BF16 if wk[1] is None else RMS_GLU_FP8)):
+        return None
+    if residual is not None and (residual.shape != x.shape or residual.stride() != x.stride()
+                                 or residual.dtype != x.dtype):
+        return None
+    y, h = torch.ops.sxe.skinny_gemm_pro(x, residual, norm_weight, float(eps), wk[0], wk[1], None, 3)
     return y, (h if residual is not None else x)
 
 

@@ -277,3 +277,79 @@ def test_fused_rms_rope_epilogue_vs_separate_ops(M, nq, nkv, fp8):
     written[ok // bs, ok % bs] = True
     diff = (c_f != c_ref).any(dim=-1).any(dim=2).any(dim=1)  # [blocks, bs]
     assert not (diff & ~written).any()  # no stray writes outside the appended slots
+
+
+def _weights(N, K, fp8, seed):
+    from shuffle_exchange_amd.ops.fp_quantizer import FP8Weight
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    w = (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).bfloat16()
+    if not fp8:
+        return w, w, None, w.double()
+    q = FP8Weight.__new__(FP8Weight)  # (its quantizer takes multiples of 64 only)
+    q.scale = w.float().abs().amax(1) / 448
+    q.q = (w.float() / q.scale[:, None]).to(torch.float8_e4m3fn)
+    return q, q.q.view(torch.uint8), q.scale, q.q.double() * q.scale.double()[:, None]
+
+
+# what is left against fp64 of the same bf16 operands: fp32 sums and one rounding of the result (2^-9)
+REL = 3e-3
+
+
+@pytest.mark.parametrize("M", [1, 2, 4, 5])
+@pytest.mark.parametrize("N,K", [(8, 16), (13, 528), (2048, 2064), (4084, 4096), (512, 8208), (5000, 1040)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_tile_widths_vs_fp64(M, N, K, fp8):
+    """Tiles of 8 columns (two K slices a matrix step) and of 16: remainders of N and of K, rows 1 to 5."""
+    _, w, s, ref = _weights(N, K, fp8, M + N + K)
+    x = torch.randn(M, K + 8, device="cuda").bfloat16()[:, :K]
+    b = torch.randn(N, device="cuda").bfloat16()
+    y = torch.ops.sxe.skinny_gemm_fp8w(x, w, s, b) if fp8 else torch.ops.sxe.skinny_gemm(x, w, b)
+    want = x.double() @ ref.T + b.double()
+    assert (y.double() - want).norm() < REL * want.norm()
+
+
+@pytest.mark.parametrize("M", [1, 2, 4])
+@pytest.mark.parametrize("N,K", [(16, 64), (48, 2048), (11264, 2048), (14336, 4096)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_rms_glu_epilogue_vs_fp64(M, N, K, fp8):
+    """Mode 3: silu(gate) * up in the epilogue of the RMS prologue; the normed input is rounded to bf16 before its 1 / rms (2^-9)
+    as in mode 1, so the error of the product is twice a rounding's."""
+    from shuffle_exchange_amd.ops.linear import RMS_GLU_BF16, RMS_GLU_FP8, fused_rms_glu
+    wobj, w, s, ref = _weights(N, K, fp8, M + N + K)
+    x, res = torch.randn(2, M, K, device="cuda").bfloat16()
+    g = (1 + 0.1 * torch.randn(K, device="cuda")).bfloat16()
+    y, h = torch.ops.sxe.skinny_gemm_pro(x, res, g, 1e-5, w, s, None, 3)
+    hr = (x.float() + res.float()).bfloat16()
+    a = (hr.double() * g.double()).bfloat16().double() * torch.rsqrt(hr.double().square().mean(-1, keepdim=True) + 1e-5)
+    gate, up = (a @ ref.T).chunk(2, -1)
+    want = torch.nn.functional.silu(gate) * up
+    assert torch.equal(h, hr) and y.shape == (M, N // 2) and (y.double() - want).norm() < 2 * REL * want.norm()
+    r = fused_rms_glu(x, res, g, 1e-5, wobj)
+    assert (r is not None) == (M * K <= (RMS_GLU_FP8 if fp8 else RMS_GLU_BF16))
+    if r is not None:
+        assert torch.equal(r[0], y) and torch.equal(r[1], h)
+
+
+@pytest.mark.parametrize("nq,nkv", [(16, 4), (2, 1)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_rope_epilogue_of_narrow_tiles(nq, nkv, fp8):
+    """One row and K large enough for tiles of 8 columns: rotation pairs four lanes apart, against fp64 of the same operands."""
+    from shuffle_exchange_amd.ops.linear import fused_rms_rope_linear
+    from shuffle_exchange_amd.ops.rope import RopeCache
+    K, D, bs, n = 4096, 128, 16, (nq + 2 * nkv)
+    wobj, _, _, ref = _weights(n * D, K, fp8, nq)
+    x, res = torch.randn(2, 1, K, device="cuda").bfloat16()
+    g = (1 + 0.1 * torch.randn(K, device="cuda")).bfloat16()
+    rope = RopeCache(D, 4096, 500000.0, device="cuda")
+    pos, slots = torch.tensor([3001], device="cuda"), torch.tensor([37], device="cuda")
+    cache = torch.zeros(4, 2, nkv, bs, D, device="cuda", dtype=torch.bfloat16)
+    y, h = fused_rms_rope_linear(x, res, g, 1e-5, wobj, rope, pos, cache, slots, nq, nkv)
+    hr = (x.float() + res.float()).bfloat16().double()
+    a = (hr * g.double()).bfloat16().double() * torch.rsqrt(hr.square().mean(-1, keepdim=True) + 1e-5)
+    want = (a @ ref.T).view(n, 2, D // 2)
+    c, s = rope.cos[3001].double(), rope.sin[3001].double()
+    lo, hi = want[:nq + nkv, 0].clone(), want[:nq + nkv, 1].clone()
+    want[:nq + nkv, 0], want[:nq + nkv, 1] = lo * c - hi * s, hi * c + lo * s
+    want = want.view(n, D)
+    assert (y.view(n, D).double() - want).norm() < 2 * REL * want.norm()
+    assert torch.equal(cache[2, :, :, 5], y.view(n, D)[nq:].view(2, nkv, D)) and cache.count_nonzero() <= 2 * nkv * D
