@@ -11,6 +11,7 @@
 // and dbeta are accumulated per wave in registers across all rows the wave visits, reduced across
 // the block's 4 waves in LDS and written as one fp32 partial row per block; the caller sums the
 // (grid x H) partial matrix (a single small reduction instead of per-row atomics).
+#include "sxe_colsum.h"
 #include "sxe_common.h"
 #include <torch/library.h>
 
@@ -340,8 +341,9 @@ std::vector<at::Tensor> norm_bwd(at::Tensor dy, at::Tensor x, at::Tensor rstd, c
                        layernorm ? db_part.data_ptr<float>() : nullptr, rows, H);
   })))));
   SXE_LAUNCH_CHECK();
-  auto dw = dw_part.sum(0);
-  auto db = layernorm ? db_part.sum(0) : db_part;
+  auto dw = at::empty({H}, dw_part.options()), db = layernorm ? at::empty({H}, dw_part.options()) : db_part;
+  colsum<DT::F32, DT::F32>({dw_part.data_ptr(), db_part.data_ptr()}, {dw.data_ptr(), db.data_ptr()}, grid, H, H, layernorm ? 2 : 1,
+                           dw_part.options());
   return {dx, dw, db};
 }
 

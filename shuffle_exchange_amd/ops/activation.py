@@ -65,7 +65,8 @@ class _BiasAct(torch.autograd.Function):
     def backward(ctx, dy):
         x, bias = ctx.saved_tensors
         dx = torch.ops.sxe.bias_act_bwd(dy.contiguous(), x, bias, ctx.act)
-        db = dx.view(-1, dx.shape[-1]).float().sum(0).to(bias.dtype) if bias is not None else None
+        from .linear import column_sum
+        db = column_sum(dx.view(-1, dx.shape[-1]), bias.dtype) if bias is not None else None
         return dx, db, None
 
 

@@ -418,6 +418,17 @@ def _autocast_dtype(x):
     return None
 
 
+def column_sum(x, dtype):
+    """``x.sum(0)`` of [R, N] in ``dtype``, accumulated in fp32 (csrc/kernels/colsum.hip; fp64 and recorded sums: torch)."""
+    if (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16, torch.float32) and x.stride(1) == 1
+            and dtype in (x.dtype, torch.float32) and not (torch.is_grad_enabled() and x.requires_grad)
+            and not torch.compiler.is_compiling()):
+        from . import native
+        native.require_hip()
+        return torch.ops.sxe.column_sum(x, dtype)
+    return x.sum(0) if dtype == x.dtype else x.float().sum(0).to(dtype)
+
+
 class _Linear(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias):
@@ -449,7 +460,7 @@ class _Linear(torch.autograd.Function):
             if not write_weight_grad(wp, gy2, x2):
                 dw = gy2.t() @ x2
         if ctx.has_bias and ctx.needs_input_grad[2]:
-            db = gy2.sum(0)
+            db = column_sum(gy2, gy2.dtype)
         return dx, dw, db
 
 
