@@ -8,6 +8,9 @@
 // (online softmax), the 4 waves merge through LDS, and the backward sweep re-reads the row
 // (Infinity-Cache resident at these row sizes) and writes bf16 gradients IN PLACE, so the
 // [tokens, vocab] logits tensor is never duplicated (4 GiB at 16K tokens x 128K vocab).
+// The sweeps are memory-bound at 16 bytes a load, so a row that starts off a 16-byte boundary (an odd vocabulary) is swept from its
+// first boundary on, the few elements around that by single lanes: 2048 x 50257 of bf16, us, element by element / so: loss
+// 116 / 42, gradient 153 / 86; 256 rows 89 / 20 and 86 / 22.
 #include "sxe_common.h"
 #include <torch/library.h>
 
@@ -20,24 +23,36 @@ __device__ __forceinline__ void ms_merge(float& m, float& s, float m2, float s2)
   m = mn;
 }
 
-template <DT T, bool VEC>
-__device__ __forceinline__ float row_lse(const typename dt_traits<T>::storage* __restrict__ row, int V, float* red) {
+// elements of a row before its first 16-byte boundary: rows of an odd vocabulary start anywhere
+template <typename S>
+__device__ __forceinline__ int row_head(const S* row, int V) {
+  return min(V, (int)((0 - reinterpret_cast<uintptr_t>(row) / sizeof(S)) & (16 / sizeof(S) - 1)));
+}
+// f8(first, 8 elements) over the 16-byte aligned body of a row, f1(element) over what lies before and behind it (< 8 each)
+template <typename F8, typename F1>
+__device__ __forceinline__ void for_row(int V, int head, F8 f8, F1 f1) {
+  const int body = (V - head) & ~7;
+  for (int c = head + threadIdx.x * 8; c < head + body; c += blockDim.x * 8) f8(c);
+  if ((int)threadIdx.x < head) f1(threadIdx.x);
+  const int c = head + body + threadIdx.x;
+  if (c < V) f1(c);
+}
+
+template <DT T>
+__device__ __forceinline__ float row_lse(const typename dt_traits<T>::storage* __restrict__ row, int V, int head, float* red) {
   float m = -INFINITY, s = 0.f;
-  if constexpr (VEC) {
-    for (int c = threadIdx.x * 8; c < V; c += blockDim.x * 8) {
-      float v[8];
-      load8<T>(row + c, v);
-      float lm = v[0];
+  for_row(V, head, [&](int c) {
+    float v[8];
+    load8<T>(row + c, v);
+    float lm = v[0];
 #pragma unroll
-      for (int j = 1; j < 8; ++j) lm = fmaxf(lm, v[j]);
-      float ls = 0.f;
+    for (int j = 1; j < 8; ++j) lm = fmaxf(lm, v[j]);
+    float ls = 0.f;
+    const float ref = lm == -INFINITY ? 0.f : lm;  // eight masked logits add nothing
 #pragma unroll
-      for (int j = 0; j < 8; ++j) ls += __expf(v[j] - lm);
-      ms_merge(m, s, lm, ls);
-    }
-  } else {
-    for (int c = threadIdx.x; c < V; c += blockDim.x) ms_merge(m, s, to_f32<T>(row[c]), 1.f);
-  }
+    for (int j = 0; j < 8; ++j) ls += __expf(v[j] - ref);
+    ms_merge(m, s, lm, ls);
+  }, [&](int c) { ms_merge(m, s, to_f32<T>(row[c]), 1.f); });
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     float m2 = __shfl_xor(m, o, 64), s2 = __shfl_xor(s, o, 64);
@@ -53,7 +68,7 @@ __device__ __forceinline__ float row_lse(const typename dt_traits<T>::storage* _
 }
 
 // mode: 0 = forward only; 1 = forward + in-place gradient with grad = scale * (softmax - onehot)
-template <DT T, bool VEC>
+template <DT T>
 __global__ void __launch_bounds__(256) xent_kernel(typename dt_traits<T>::storage* __restrict__ logits, int64_t rows, int V,
                                                    const int64_t* __restrict__ target, int64_t ignore_index,
                                                    float* __restrict__ loss, float* __restrict__ lse_out, int mode,
@@ -64,7 +79,8 @@ __global__ void __launch_bounds__(256) xent_kernel(typename dt_traits<T>::storag
     typename dt_traits<T>::storage* row = logits + r * V;
     const int64_t tgt = target[r];
     const bool ign = (tgt == ignore_index);
-    const float lse = row_lse<T, VEC>(row, V, red);
+    const int head = row_head(row, V);
+    const float lse = row_lse<T>(row, V, head, red);
     if (threadIdx.x == 0) {
       const float xt = ign ? 0.f : to_f32<T>(row[tgt]);
       loss[r] = ign ? 0.f : (lse - xt);
@@ -73,25 +89,18 @@ __global__ void __launch_bounds__(256) xent_kernel(typename dt_traits<T>::storag
     __syncthreads();  // the target logit is read above before the gradient overwrites it
     if (mode == 1) {
       const float sc = ign ? 0.f : scale;
-      if constexpr (VEC) {
-        for (int c = threadIdx.x * 8; c < V; c += blockDim.x * 8) {
-          float v[8];
-          load8<T>(row + c, v);
+      for_row(V, head, [&](int c) {
+        float v[8];
+        load8<T>(row + c, v);
 #pragma unroll
-          for (int j = 0; j < 8; ++j) v[j] = sc * (__expf(v[j] - lse) - ((c + j) == tgt ? 1.f : 0.f));
-          store8<T>(row + c, v);
-        }
-      } else {
-        for (int c = threadIdx.x; c < V; c += blockDim.x) {
-          float v = to_f32<T>(row[c]);
-          row[c] = from_f32<T>(sc * (__expf(v - lse) - (c == tgt ? 1.f : 0.f)));
-        }
-      }
+        for (int j = 0; j < 8; ++j) v[j] = sc * (__expf(v[j] - lse) - ((c + j) == tgt ? 1.f : 0.f));
+        store8<T>(row + c, v);
+      }, [&](int c) { row[c] = from_f32<T>(sc * (__expf(to_f32<T>(row[c]) - lse) - (c == tgt ? 1.f : 0.f))); });
     }
   }
 }
 
-// grad = dloss[r] * (softmax - onehot), written into grad_out (may alias logits).
+// grad = dloss[r] * (softmax - onehot), written into grad_out (may alias logits). VEC: both start alike against 16 bytes.
 template <DT T, bool VEC>
 __global__ void __launch_bounds__(256) xent_bwd_kernel(const typename dt_traits<T>::storage* __restrict__ logits,
                                                        typename dt_traits<T>::storage* __restrict__ grad, int64_t rows, int V,
@@ -103,19 +112,17 @@ __global__ void __launch_bounds__(256) xent_bwd_kernel(const typename dt_traits<
     const float l = lse[r];
     const typename dt_traits<T>::storage* in = logits + r * V;
     typename dt_traits<T>::storage* out = grad + r * V;
+    auto one = [&](int c) { out[c] = from_f32<T>(sc * (__expf(to_f32<T>(in[c]) - l) - (c == tgt ? 1.f : 0.f))); };
     if constexpr (VEC) {
-      for (int c = threadIdx.x * 8; c < V; c += blockDim.x * 8) {
+      for_row(V, row_head(in, V), [&](int c) {
         float v[8];
         load8<T>(in + c, v);
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] = sc * (__expf(v[j] - l) - ((c + j) == tgt ? 1.f : 0.f));
         store8<T>(out + c, v);
-      }
+      }, one);
     } else {
-      for (int c = threadIdx.x; c < V; c += blockDim.x) {
-        float v = to_f32<T>(in[c]);
-        out[c] = from_f32<T>(sc * (__expf(v - l) - (c == tgt ? 1.f : 0.f)));
-      }
+      for (int c = threadIdx.x; c < V; c += blockDim.x) one(c);
     }
   }
 }
@@ -231,15 +238,14 @@ std::tuple<at::Tensor, at::Tensor> xent_fwd(at::Tensor logits, at::Tensor target
     SXE_CHECK(scale_t->scalar_type() == at::kFloat && scale_t->is_cuda(), "xent: scale tensor fp32");
     sp = scale_t->data_ptr<float>();
   }
-  const bool vec = (V % 8 == 0);
   const int grid = (int)std::min<int64_t>(rows, 8192);
   DT d = dtype_of(logits);
-  SXE_DISPATCH_DT(d, TT, SXE_DISPATCH_BOOL(vec, VB, {
+  SXE_DISPATCH_DT(d, TT, {
     using S = typename dt_traits<TT>::storage;
-    hipLaunchKernelGGL((xent_kernel<TT, VB>), dim3(grid), dim3(256), 0, cur_stream(), reinterpret_cast<S*>(logits.data_ptr()),
+    hipLaunchKernelGGL((xent_kernel<TT>), dim3(grid), dim3(256), 0, cur_stream(), reinterpret_cast<S*>(logits.data_ptr()),
                        rows, V, target.data_ptr<int64_t>(), ignore_index, loss.data_ptr<float>(), lse.data_ptr<float>(),
                        inplace_grad ? 1 : 0, sp, (float)grad_scale);
-  }));
+  });
   SXE_LAUNCH_CHECK();
   return {loss, lse};
 }
@@ -253,7 +259,7 @@ at::Tensor xent_bwd(at::Tensor logits, at::Tensor target, at::Tensor lse, at::Te
   c10::DeviceGuard guard(logits.device());
   at::Tensor grad = inplace ? logits : at::empty_like(logits);
   if (rows == 0) return grad;
-  const bool vec = (V % 8 == 0);
+  const bool vec = ((reinterpret_cast<uintptr_t>(logits.data_ptr()) ^ reinterpret_cast<uintptr_t>(grad.data_ptr())) & 15) == 0;
   const int grid = (int)std::min<int64_t>(rows, 8192);
   DT d = dtype_of(logits);
   SXE_DISPATCH_DT(d, TT, SXE_DISPATCH_BOOL(vec, VB, {
