@@ -324,10 +324,11 @@ def expert_mlp(h, routing, up, down, act="relu2"):
 
 
 # ---------------------------------------------------- routed SwiGLU experts, weights [E, K, N] as trained
-# Mean rows per expert up to which the streaming kernels are used. One layer of 8 experts, top 2, us streaming / library
-# (with its row counts read back): 4096 x 14336: 1 token 153 / 299, 16: 533 / 1051, 128: 599 / 968, 256 (64 rows each):
-# 866 / 1043, 384: 1177 / 1103; 2048 x 8192: 1: 52 / 150, 128: 202 / 487, 512 (128 rows): 448 / 565.
-KN_ROWS = 80
+# Mean rows per expert up to which the streaming kernels are used. One layer of 8 experts, top 2, us streaming / tiles / a library
+# product per expert (with its row counts read back): 4096 x 14336: 32 rows 619 / 635 / 973, 64: 879 / 683 / 1087, 128: 1458 /
+# 788 / 1232, 775: - / 2205 / 2776, 2048: - / 5563 / 5799; 2048 x 8192: 32: 204 / 243 / 500, 64: 300 / 259 / 519, 775: - / 734 /
+# 1101, 2048: - / 1752 / 2001; 3072 x 8192: 32: 293 / 295 / 555.
+KN_ROWS = 40
 
 
 def swiglu_experts_ok(x, w_gate_up, w_down):
@@ -341,23 +342,13 @@ def swiglu_experts_ok(x, w_gate_up, w_down):
 def swiglu_experts(x, routing, w_gate_up, w_down):
     """sum_j weight[t, j] * down_e(silu(gate_e x_t) * up_e x_t) over the choices of every token: x [T, K], w_gate_up
     [E, K, 2 I], w_down [E, I, K] (``swiglu_experts_ok``), ``routing`` from route_topk / route_logits. Few rows per expert
-    stream the weights without a host synchronisation; more take a library product per expert, for which the row counts are
-    read back once."""
-    from .activation import swiglu
+    stream the weights (csrc/kernels/experts_kn.hip), more run on tiles of 256 rows (experts_kn_tile.hip); no host
+    synchronisation."""
     rows, _, slots, offs, active = routing.lists
     x = x.contiguous()
     E, R = w_gate_up.shape[0], rows.numel()
-    if R <= KN_ROWS * E or torch.cuda.is_current_stream_capturing():
+    if R <= KN_ROWS * E:
         h = torch.ops.sxe.expert_swiglu_kn(x, w_gate_up, offs, active, rows)
         return torch.ops.sxe.expert_down_kn(h, w_down, offs, active, slots, routing.weight)
-    xs = x.index_select(0, rows)
-    gu = torch.empty(R, w_gate_up.shape[2], dtype=x.dtype, device=x.device)
-    y = torch.empty(R, w_down.shape[2], dtype=x.dtype, device=x.device)
-    bounds = offs.tolist()
-    spans = [(e, a, b) for e, (a, b) in enumerate(zip(bounds, bounds[1:])) if b > a]
-    for e, a, b in spans:
-        torch.mm(xs[a:b], w_gate_up[e], out=gu[a:b])
-    h = swiglu(gu)
-    for e, a, b in spans:
-        torch.mm(h[a:b], w_down[e], out=y[a:b])
-    return torch.ops.sxe.moe_gather_sum(y, slots, routing.weight)
+    h = torch.ops.sxe.expert_swiglu_kn_tile(x, w_gate_up, offs, rows)
+    return torch.ops.sxe.moe_gather_sum(torch.ops.sxe.expert_down_kn_tile(h, w_down, offs), slots, routing.weight)

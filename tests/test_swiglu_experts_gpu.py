@@ -1,4 +1,4 @@
-"""Routed SwiGLU experts over [E, K, N] weights (csrc/kernels/experts_kn.hip) against fp64, and Mixtral decode steps replayed
+"""Routed SwiGLU experts over [E, K, N] weights (csrc/kernels/experts_kn.hip, experts_kn_tile.hip) against fp64, and Mixtral decode steps replayed
 from graphs against eager ones."""
 import pytest
 import torch
@@ -41,9 +41,36 @@ def test_streaming_kernels(T, E, k, K, I, N, skew, monkeypatch):
     ref = _reference(x, logits, k, w_gu, w_down)
     # the hidden row and the output are rounded to bf16 (2^-9 each)
     assert ((got.double() - ref).norm() / ref.norm()).item() < 5e-3
-    monkeypatch.setattr(moe, "KN_ROWS", 0)  # the library products behind the same routing
-    lib = moe.swiglu_experts(x, moe.route_logits(logits, k), w_gu, w_down)
-    assert ((lib.double() - ref).norm() / ref.norm()).item() < 8e-3
+    monkeypatch.setattr(moe, "KN_ROWS", 0)  # the tile products behind the same routing
+    tiles = moe.swiglu_experts(x, moe.route_logits(logits, k), w_gu, w_down)
+    assert ((tiles.double() - ref).norm() / ref.norm()).item() < 8e-3
+
+
+@pytest.mark.parametrize("T", [1, 127, 128, 129, 300, 1025])
+@pytest.mark.parametrize("E,k,K,I,N", [(8, 2, 256, 192, 128), (4, 1, 32, 64, 384), (2, 2, 96, 136, 272), (70, 2, 160, 128, 256)])
+@pytest.mark.parametrize("skew", [False, True])
+def test_tile_kernels(T, E, k, K, I, N, skew):
+    """Prefill's products: row tiles and halves of them, column remainders, one to five slabs of K, more experts than lanes."""
+    from shuffle_exchange_amd.ops import moe
+    g = torch.Generator(device="cuda").manual_seed(T + K)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x = rnd(T, K).bfloat16()
+    w_gu, w_down = (rnd(E, K, 2 * I) * K ** -0.5).bfloat16(), (rnd(E, I if I % 32 == 0 else K, N) * I ** -0.5).bfloat16()
+    logits = rnd(T, E)
+    if skew:
+        logits[:, :k] += 100
+    rows, _, _, offs, _ = moe.route_logits(logits, k).lists
+    h = torch.ops.sxe.expert_swiglu_kn_tile(x, w_gu, offs, rows)
+    a = h if I % 32 == 0 else x[rows.long()]
+    y = torch.ops.sxe.expert_down_kn_tile(a, w_down, offs)
+    o = offs.tolist()
+    for e in range(E):
+        r = slice(o[e], o[e + 1])
+        gate, up = (x[rows[r].long()].double() @ w_gu[e].double()).chunk(2, -1)
+        want, wy = torch.nn.functional.silu(gate) * up, a[r].double() @ w_down[e].double()
+        # fp32 sums and one rounding of the result (2^-9)
+        assert (h[r].double() - want).norm() <= 3e-3 * want.norm()
+        assert (y[r].double() - wy).norm() <= 3e-3 * wy.norm()
 
 
 def test_mixtral_decode_graphs_match_eager():
