@@ -38,10 +38,11 @@ class _StaticBatch:
         self.num_tokens = self.num_seqs = S
         self.max_blocks = max_blocks
         self.max_kv_len = kv_bucket
-        self.d64 = torch.zeros(4 * S, dtype=torch.int64, device=device)
-        self.d32 = torch.zeros(4 * S + S * max_blocks, dtype=torch.int32, device=device)
-        self.h64 = torch.zeros(4 * S, dtype=torch.int64, pin_memory=True)
-        self.h32 = torch.zeros(4 * S + S * max_blocks, dtype=torch.int32, pin_memory=True)
+        n64, n32 = 32 * S, 16 * S + 4 * S * max_blocks  # bytes: one copy brings both
+        self.dev = torch.zeros(n64 + n32, dtype=torch.uint8, device=device)
+        self.host = torch.zeros(n64 + n32, dtype=torch.uint8, pin_memory=True)
+        self.d64, self.d32 = self.dev[:n64].view(torch.int64), self.dev[n64:].view(torch.int32)
+        self.h64, self.h32 = self.host[:n64].view(torch.int64), self.host[n64:].view(torch.int32)
         self.input_ids, self.positions, self.slots, self.last_idx = self.d64.view(4, S).unbind(0)
         self.q_start, self.q_len, self.kv_len, self.state_slots = self.d32[:4 * S].view(4, S).unbind(0)
         self.block_table = self.d32[4 * S:].view(S, max_blocks)
@@ -131,8 +132,7 @@ class DecodeGraphRunner:
             bt[i, nb:] = self.scratch_block
         ids[n:] = pos[n:] = 0  # rows past the batch: one key in the scratch block
         slots[n:], kl[n:], ss[n:], bt[n:] = self.scratch_block * bs, 1, self.scratch_state, self.scratch_block
-        sb.d64.copy_(sb.h64, non_blocking=True)
-        sb.d32.copy_(sb.h32, non_blocking=True)
+        sb.dev.copy_(sb.host, non_blocking=True)
         ev = torch.cuda.Event()
         ev.record()
         sb.copied = ev

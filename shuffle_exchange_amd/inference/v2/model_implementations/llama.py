@@ -31,7 +31,7 @@ from ....ops import native
 from ....ops.activation import swiglu
 from ....ops.linear import linear
 from ....ops.paged_attention import paged_attention_parts, paged_batch_attention, ragged_attention, rope_kv_cache_append
-from ....ops.rows import embed, gather_rows
+from ....ops.rows import embed, gather_last
 
 
 class _TPShards:
@@ -226,9 +226,12 @@ class RaggedLlama:
 
     def _wobj(self, mod, li, key):
         if self.qw is not None and key in self.qw[li]:
-            impl = self.qw[li][key]
-            return getattr(impl, "q", None) if getattr(impl, "q", None) is not None else getattr(impl, "weight", None)
+            return self._impl_weight(self.qw[li][key])
         return mod.weight
+
+    @staticmethod
+    def _impl_weight(impl):
+        return getattr(impl, "q", None) if getattr(impl, "q", None) is not None else getattr(impl, "weight", None)
 
     def _norm_proj(self, norm, x, res, mod, li, key):
         """(norm(x + res) @ W^T, h) through the fused kernel, else the separate launches."""
@@ -369,7 +372,17 @@ class RaggedLlama:
                 m, h2 = layer.post_attention_layernorm(o, h)
                 x, res = self._mlp(layer, m, li), h2
         last = batch.last_idx
-        h = model.norm(gather_rows(x, last), gather_rows(res, last))[0]
+        x = gather_last(x, last, res)
+        if self._fusable(x.shape[0]):
+            from ....ops.linear import RMS_GLU_BF16, RMS_GLU_FP8, _pro_weight, fused_rms_linear
+            w = model.lm_head.weight if self.qw is None else self._impl_weight(self.qhead)
+            wk = _pro_weight(w)
+            # one launch for the norm and the head, where building its input in every workgroup costs less than a launch
+            if wk is not None and x.numel() <= (RMS_GLU_BF16 if wk[1] is None else RMS_GLU_FP8):
+                r = fused_rms_linear(x, None, model.norm.weight, model.norm.eps, w)
+                if r is not None:
+                    return r[0].float()
+        h = model.norm(x)
         if self.tps is not None:  # vocab-parallel head: gather every rank's logit columns
             from .... import comm as dist
             part = (self.qhead(h) if self.qw is not None else linear(h, self.tps.head)).float()

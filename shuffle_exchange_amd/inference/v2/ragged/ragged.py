@@ -243,8 +243,9 @@ class RaggedBatch:
         n_want = sum(len(x) for x in want)
         maxb = max(1, max(len(s.blocks) for s in seqs))
         pin = torch.cuda.is_available() and device.type == "cuda"
-        i64 = torch.empty(3 * T + n_want, dtype=torch.int64, pin_memory=pin)
-        i32 = torch.empty(4 * S + S * maxb, dtype=torch.int32, pin_memory=pin)
+        n64 = 8 * (3 * T + n_want)  # bytes: one copy brings both
+        host = torch.empty(n64 + 4 * (4 * S + S * maxb), dtype=torch.uint8, pin_memory=pin)
+        i64, i32 = host[:n64].view(torch.int64), host[n64:].view(torch.int32)
         if T:
             torch.cat([tk.reshape(-1).to("cpu", torch.int64) for tk in tokens], out=i64[:T])
         # numpy views: a small numpy operation costs a tenth of a tensor one (24 sequences of one token:
@@ -270,8 +271,8 @@ class RaggedBatch:
                 nw += 1
             t += n
         meta[0], meta[1], meta[2], meta[3] = starts, lens, self.host_kv_len, [s.state_slot for s in seqs]
-        d64 = i64.to(device, non_blocking=True)
-        d32 = i32.to(device, non_blocking=True)
+        dev = host.to(device, non_blocking=True)
+        d64, d32 = dev[:n64].view(torch.int64), dev[n64:].view(torch.int32)
         self.input_ids, self.positions, self.slots, self.last_idx = d64[:T], d64[T:2 * T], d64[2 * T:3 * T], d64[3 * T:]
         self.q_start, self.q_len, self.kv_len = d32[:S], d32[S:2 * S], d32[2 * S:3 * S]
         self.state_slots = d32[3 * S:4 * S]
