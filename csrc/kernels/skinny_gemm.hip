@@ -233,7 +233,8 @@ __device__ __forceinline__ void build_gatesum(int M, int K, const ProArgs& p, un
 
 // Only columns [klo, khi) of the input are built (a split-K part needs no more), except under
 // PRO_RMS, whose row norm needs the whole row.
-template <int MODE, int NT>
+// LEAN: half the loads of a round, for kernels that keep four waves on a SIMD.
+template <int MODE, int NT, bool LEAN>
 __device__ __forceinline__ void build_act(const unsigned short* __restrict x, int64_t ldx, int M, int K, int klo,
                                           int khi, const ProArgs& p, unsigned short* act, float* rinv) {
   if constexpr (MODE == PRO_MERGE) {
@@ -257,7 +258,7 @@ __device__ __forceinline__ void build_act(const unsigned short* __restrict x, in
   // U chunks of 8 per thread per round, every load of a round issued before the first use: a loop
   // that consumes each chunk before loading the next is a chain of dependent L2 round trips (it made
   // the fused down projection 9 us slower than the separate SwiGLU launch)
-  constexpr int U = MODE == PRO_ADDNORM || MODE == PRO_RMS ? 2 : 4;
+  constexpr int U = MODE == PRO_ADDNORM || LEAN ? 2 : 4;
   __shared__ float red[NT / 64][kProMaxM];
   const int per = (khi - klo) / 8, n = M * per;
   float ss[kProMaxM] = {0.f, 0.f, 0.f, 0.f};
@@ -394,13 +395,14 @@ __device__ __forceinline__ void finish(const f32x4 (&red)[NW][64], int lane, int
 // at KS = 2 slices of K (the first 32 K values of a step and the next), its rows the M rows at slice 0 and again at slice 1, and
 // the two blocks in which the slices agree are the sums. A load instruction then reads 128 contiguous bytes of 8 rows.
 template <int NW, int MODE, bool NT, int CW>
-__global__ __launch_bounds__(NW * 64, MODE == PRO_RMS ? 4 : 1) void skinny_gemm_kernel(
+__global__ __launch_bounds__(NW * 64, MODE == PRO_RMS && CW == 8 ? 4 : 1) void skinny_gemm_kernel(
     const unsigned short* __restrict x, int64_t ldx, const unsigned short* __restrict w, int64_t ldw,
     const unsigned short* __restrict bias, unsigned short* __restrict y, int64_t ldy, int M, int N, int K, int ss_per_wave,
     ProArgs pro) {
   __shared__ f32x4 red[NW][64];
   extern __shared__ __attribute__((aligned(16))) unsigned short act_lds[];  // PRO_*: the M x K input
   constexpr int KS = 16 / CW, STEP = 32 * KS, SS = kSS * KS;
+  constexpr bool LEAN = MODE == PRO_RMS && CW == 8;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, g = lane >> 4;
   const int tile = blockIdx.x;
@@ -426,16 +428,20 @@ __global__ __launch_bounds__(NW * 64, MODE == PRO_RMS ? 4 : 1) void skinny_gemm_
       cur = nxt;
     }
   } else {
-    // two super-steps of weights are in flight while the prologue builds the input in LDS
+    // the weight stream runs two super-steps ahead of the prologue, which builds the input in LDS, and of the products: three sets
+    // of registers; with two (LEAN), a third more workgroups are on a CU, which is faster for one row's narrow tiles alone
+    Frag nx2;
     load_w<NT, STEP>(cur, wrow, wok, ss0 * SS + kw, K);
     if (ss_per_wave > 1) load_w<NT, STEP>(nxt, wrow, wok, (ss0 + 1) * SS + kw, K);
-    build_act<MODE, NW * 64>(x, ldx, M, K, 0, K, pro, act_lds, rinv);
+    build_act<MODE, NW * 64, LEAN>(x, ldx, M, K, 0, K, pro, act_lds, rinv);
     for (int i = 0; i < ss_per_wave; ++i) {
+      if (!LEAN && i + 2 < ss_per_wave) load_w<NT, STEP>(nx2, wrow, wok, (ss0 + i + 2) * SS + kw, K);
       load_x<STEP>(cur, xrow, xok, (ss0 + i) * SS + kx, K);
 #pragma unroll
       for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.x[s], cur.w[s], acc, 0, 0, 0);
       cur = nxt;
-      if (i + 2 < ss_per_wave) load_w<NT, STEP>(nxt, wrow, wok, (ss0 + i + 2) * SS + kw, K);
+      if (!LEAN) nxt = nx2;
+      else if (i + 2 < ss_per_wave) load_w<NT, STEP>(nxt, wrow, wok, (ss0 + i + 2) * SS + kw, K);
     }
   }
   red[wave][lane] = acc;  // C[row 4 g + r][col]
@@ -512,7 +518,7 @@ __global__ __launch_bounds__(NW * 64) void skinny_gemm_fp8w_kernel(const unsigne
       const int k = k0 + STEP * j;
       wv0[j] = (wok && k < K && ss_per_wave > 0) ? *reinterpret_cast<const uint4*>(wrow + k) : uint4{0u, 0u, 0u, 0u};
     }
-    build_act<MODE, NW * 64>(x, ldx, M, K, 0, K, pro, act_lds, rinv);
+    build_act<MODE, NW * 64, false>(x, ldx, M, K, 0, K, pro, act_lds, rinv);
   }
   for (int i = 0; i < ss_per_wave; ++i) {
     const int k0 = (wave * ss_per_wave + i) * SS + 16 * g;

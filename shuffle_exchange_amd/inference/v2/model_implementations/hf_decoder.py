@@ -30,7 +30,6 @@ from typing import Optional
 import torch
 import torch.nn.functional as F
 
-from ....ops import native
 from ....ops.activation import ACT, bias_act, gated_act
 from ....ops.linear import linear
 from ....ops.norm import layer_norm, rms_norm

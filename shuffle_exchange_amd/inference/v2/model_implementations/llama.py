@@ -31,7 +31,7 @@ from ....ops import native
 from ....ops.activation import swiglu
 from ....ops.linear import linear
 from ....ops.paged_attention import paged_attention_parts, paged_batch_attention, ragged_attention, rope_kv_cache_append
-from ....ops.rows import embed, gather_last
+from ....ops.rows import gather_last
 
 
 class _TPShards:
