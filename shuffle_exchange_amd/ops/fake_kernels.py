@@ -118,3 +118,8 @@ def _gather_rows(src, idx, offset=0, add=None):
 @_reg("sxe::scatter_rows_")
 def _scatter_rows(dst, idx, src):
     return None
+
+
+@_reg("sxe::column_sum")
+def _column_sum(x, dtype):
+    return x.new_empty((x.shape[1],), dtype=dtype)

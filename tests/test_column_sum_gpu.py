@@ -56,3 +56,13 @@ def test_users(rows, H):
              grads(lambda x, w, b: torch.nn.functional.gelu(x + b, approximate="tanh"), torch.float64))
     for got, want in (*ln, *ge):
         assert (got - want).norm() < 6e-3 * want.norm()  # roundings of bf16 terms and results: 2^-8 each at most
+
+
+def test_traces():
+    """The op has a shape function like the other kernels of a training step."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    import shuffle_exchange_amd.ops.fake_kernels  # noqa: F401
+    with FakeTensorMode() as mode:
+        x = mode.from_tensor(torch.empty(12, 40, device="cuda", dtype=torch.bfloat16))
+        y = torch.ops.sxe.column_sum(x, torch.float32)
+        assert y.shape == (40,) and y.dtype == torch.float32 and y.device == x.device
