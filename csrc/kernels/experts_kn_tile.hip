@@ -11,9 +11,9 @@
 // 32 k (32 KB) arrive by direct loads in a ring of five, four ahead; x rows are gathered on the way. x is read from LDS as it
 // lies, W transposed (ds_read_b64_tr_b16). The two groups of four waves (rows 0 - 127 and the rest, one wave of each on a SIMD)
 // run one barrier apart, with a barrier behind either of a slab's two steps of eight products a wave, so that one group's waits
-// and reads lie under the other's products: 8 experts of 2048 rows, 4096 x 14336, ms of both products 5.85 in step, 5.49 so;
+// and reads lie under the other's products: 8 experts of 2048 rows, 4096 x 14336, ms of both products 5.9 in step, 5.5 so;
 // ring depth (4 or 5) and the order of loads and reads are within 2 %. The row tiles of an expert and column block run side by
-// side on one XCD, so W comes from memory once. Waves whose 128 rows lie past the expert's rows run no products. 5.49 ms are 1.05
+// side on one XCD, so W comes from memory once. Waves whose 128 rows lie past the expert's rows run no products. 5.5 ms are 1.05
 // PFLOP/s at about 1.9 GHz, matrix cores busy for a good half of the time, no LDS bank conflicts.
 #include "sxe_common.h"
 #include "sxe_tile.h"

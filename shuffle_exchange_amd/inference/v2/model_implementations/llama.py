@@ -194,8 +194,8 @@ class RaggedLlama:
             return self.qw[li][key](x)
         return mod(x)
 
-    # decode (<= 4 tokens): RMSNorm folded into the QKV / gate_up GEMMs and SwiGLU into the down GEMM
-    # (skinny_gemm.hip prologues) -- three latency-bound launches fewer per layer
+    # decode (<= 4 tokens): RMSNorm folded into the QKV / gate_up GEMMs as their prologue, SwiGLU into gate_up's
+    # epilogue (skinny_gemm.hip) -- three latency-bound launches fewer per layer
     FUSE_MAX_T = 4
 
     def _fusable(self, T):

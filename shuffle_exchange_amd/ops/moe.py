@@ -332,7 +332,7 @@ KN_ROWS = 40
 
 
 def swiglu_experts_ok(x, w_gate_up, w_down):
-    """The kernels of csrc/kernels/experts_kn.hip cover these experts."""
+    """The kernels of csrc/kernels/experts_kn.hip and experts_kn_tile.hip cover these experts."""
     return (_hip(x) and x.dtype == torch.bfloat16 and w_gate_up.is_cuda and w_gate_up.dtype == torch.bfloat16
             and w_down.dtype == torch.bfloat16 and w_gate_up.is_contiguous() and w_down.is_contiguous()
             and w_gate_up.shape[1] % 32 == 0 and w_gate_up.shape[2] % 128 == 0 and w_down.shape[1] % 32 == 0 and w_down.shape[2] % 128 == 0
