@@ -17,6 +17,8 @@ import weakref
 import torch
 import torch.nn.functional as F
 
+from . import native
+
 # Large weight-gradient GEMMs (MLP projections, LM head) run faster as two HBM-speed transposes +
 # a forward-layout ("TN") bf16 GEMM + an fp32 accumulate than as one fp32-output GEMM in the
 # token-major "NT" layout: hipBLASLt reaches 1.47-1.61 PF in TN vs 1.06-1.19 PF in NT on MI355X
@@ -37,8 +39,6 @@ SKINNY_MAX_M = int(os.environ.get("SXE_SKINNY_MAX_M", 4))
 
 
 def _skinny(x, weight, bias):
-    if torch.compiler.is_compiling():  # data_ptr() is not traceable; graphs keep the library GEMM
-        return None
     K = x.shape[-1]
     if not (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.dim() == 2
             and weight.is_contiguous() and K % 8 == 0 and weight.data_ptr() % 16 == 0):
@@ -49,7 +49,6 @@ def _skinny(x, weight, bias):
     if not (0 < x2.shape[0] <= SKINNY_MAX_M and x2.stride(1) == 1 and x2.stride(0) % 8 == 0
             and x2.data_ptr() % 16 == 0):
         return None
-    from . import native
     native.require_hip()
     return torch.ops.sxe.skinny_gemm(x2, weight, bias).view(*x.shape[:-1], weight.shape[0])
 
@@ -68,7 +67,7 @@ def _streamable(x2, weight, bias, unit=8):
 
 
 def _stream(x, weight, bias):
-    if torch.compiler.is_compiling() or SKINNY_MAX_M <= 0 or weight.dtype != torch.bfloat16 or not weight.is_cuda:
+    if weight.dtype != torch.bfloat16 or not weight.is_cuda:
         return None
     rows = x.numel() // max(1, x.shape[-1])
     if not SKINNY_MAX_M < rows <= (STREAM_ROWS if weight.numel() > STREAM_SMALL else STREAM_ROWS_SMALL):
@@ -76,7 +75,6 @@ def _stream(x, weight, bias):
     x2 = x.reshape(-1, x.shape[-1])
     if not _streamable(x2, weight, bias):
         return None
-    from . import native
     native.require_hip()
     return torch.ops.sxe.stream_gemm(x2, weight, None, bias, False).view(*x.shape[:-1], weight.shape[0])
 
@@ -85,7 +83,7 @@ def glu_linear(x, weight):
     """silu(gate) * up of ``linear(x, weight)`` with weight = [gate | up], in ONE launch (stream_gemm.hip): up to 32 rows (16 of an
     FP8Weight), no autograd; None when not covered. One rounding, of the result."""
     wk = _pro_weight(weight)
-    if wk is None or torch.compiler.is_compiling() or not x.is_cuda or x.requires_grad or x.dim() != 2:
+    if wk is None or not x.is_cuda or x.requires_grad or x.dim() != 2 or not native.plain(x):
         return None
     w, sc = wk
     if not 0 < x.shape[0] <= (32 if sc is None else 16) or w.shape[0] % 32 or not _streamable(x, w, None, 8 if sc is None else 16):
@@ -421,9 +419,7 @@ def _autocast_dtype(x):
 def column_sum(x, dtype):
     """``x.sum(0)`` of [R, N] in ``dtype``, accumulated in fp32 (csrc/kernels/colsum.hip; fp64 and recorded sums: torch)."""
     if (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16, torch.float32) and x.stride(1) == 1
-            and dtype in (x.dtype, torch.float32) and not (torch.is_grad_enabled() and x.requires_grad)
-            and not torch.compiler.is_compiling()):
-        from . import native
+            and dtype in (x.dtype, torch.float32) and not (torch.is_grad_enabled() and x.requires_grad) and native.plain(x)):
         native.require_hip()
         return torch.ops.sxe.column_sum(x, dtype)
     return x.sum(0) if dtype == x.dtype else x.float().sum(0).to(dtype)
@@ -470,7 +466,8 @@ def linear(x, weight, bias=None):
     grad = torch.is_grad_enabled() and (weight.requires_grad or x.requires_grad)
     if grad and weight.requires_grad and hasattr(weight, "_sxe_grad_target"):
         return _Linear.apply(x, weight, bias)
-    if not grad and SKINNY_MAX_M > 0 and x.is_cuda:
+    if (not grad and SKINNY_MAX_M > 0 and x.is_cuda and x.numel() <= max(SKINNY_MAX_M, STREAM_ROWS_SMALL) * x.shape[-1]
+            and native.plain(x, weight, bias)):
         y = _skinny(x, weight, bias)
         if y is None:
             y = _stream(x, weight, bias)

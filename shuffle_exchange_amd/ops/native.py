@@ -14,6 +14,8 @@ import os
 import threading
 
 import torch
+import torch.autograd.forward_ad as fwAD
+from torch._C import _functorch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 HIP_LIB = os.environ.get("SXE_HIP_LIB") or os.path.join(_HERE, "_sxe_hip.so")  # override: A/B kernel experiments
@@ -94,6 +96,23 @@ def use_hip(t):
         require_hip()
         return True
     return False
+
+
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def plain(*tensors):
+    """A kernel that looks at its operands' memory and has no derivative may take these (None: no operand): no transform's wrapper
+    (vmap, jvp, functionalize), no subclass (fake and distributed tensors), and nobody who follows the call by its operators:
+    compilation, a trace, forward-mode derivatives."""
+    if (torch.compiler.is_compiling() or torch._C._is_tracing() or fwAD._current_level >= 0
+            or _functorch.peek_interpreter_stack() is not None
+            or (torch._C._len_torch_dispatch_stack() and torch._C._get_dispatch_mode(torch._C._TorchDispatchModeKey.PROXY) is not None)):
+        return False
+    for t in tensors:
+        if t is not None and (type(t) not in _PLAIN or _functorch.is_legacy_batchedtensor(t)):
+            return False
+    return True
 
 
 def status():

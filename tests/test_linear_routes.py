@@ -1,0 +1,109 @@
+"""Which calls the kernels behind ops/linear.py take: those that read tensors' memory and differentiate by no operator.
+Everything else -- transformed or fake tensors, traces, forward-mode derivatives -- runs the library's product."""
+import pytest
+import torch
+import torch.autograd.forward_ad as fwAD
+import torch.nn.functional as F
+
+gpu = pytest.mark.gpu
+
+
+def _operands(rows, dtype=torch.bfloat16, device="cuda", N=64, K=128):
+    g = torch.Generator(device).manual_seed(rows)
+    return (torch.randn(rows, K, generator=g, device=device).to(dtype), (torch.randn(N, K, generator=g, device=device) / K ** 0.5).to(dtype),
+            torch.randn(N, generator=g, device=device).to(dtype))
+
+
+def _close(got, want):
+    # both are fp32 sums of exact products, rounded once to bf16 (2^-9 each)
+    assert got.dtype == want.dtype and got.shape == want.shape
+    assert (got.double() - want.double()).norm() <= 6e-3 * want.double().norm()
+
+
+def test_plain_tensors():
+    """What ``native.plain`` lets through, on the CPU."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    from shuffle_exchange_amd.ops.native import plain
+    x, w, b = _operands(5, torch.float32, "cpu")
+    assert plain(x, torch.nn.Parameter(w), None) and plain(x[1:, ::2])
+    seen = []
+
+    def look(t):
+        seen.append(plain(t))
+        return t * 2
+    torch.func.vmap(look)(x)
+    torch.func.jvp(look, (x,), (x,))
+    torch.func.grad(lambda t: look(t).sum())(x)
+    torch.func.functionalize(look)(x)
+    with fwAD.dual_level():
+        look(fwAD.make_dual(x, x))
+        assert not plain(x)  # another operand of the call may be dual
+    with FakeTensorMode() as mode:
+        look(mode.from_tensor(x))
+    make_fx(look)(x)
+    torch.jit.trace(look, (x,), check_trace=False)
+
+    class Twice(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, t):
+            return t * 2
+
+        @staticmethod
+        def backward(ctx, g):
+            return look(g)
+    t = x.clone().requires_grad_()
+    torch.autograd.grad(Twice.apply(t), t, torch.ones(3, *x.shape), is_grads_batched=True)
+    assert len(seen) >= 8 and not any(seen)
+    assert plain(x)
+
+
+@gpu
+@pytest.mark.parametrize("rows", [1, 4, 5, 16, 17, 32, 33])
+def test_forward_mode(rows):
+    from shuffle_exchange_amd.ops.linear import linear
+    x, w, b = _operands(rows)
+    t = _operands(rows + 100)[0][:rows]
+    want = F.linear(t, w)
+    with torch.no_grad(), fwAD.dual_level():
+        y = fwAD.unpack_dual(linear(fwAD.make_dual(x, t), w, b))
+        assert y.tangent is not None
+        _close(y.tangent, want)
+        dw = fwAD.unpack_dual(linear(x, fwAD.make_dual(w, w), b)).tangent
+        _close(dw, F.linear(x, w))
+    _close(torch.func.jvp(lambda a: linear(a, w, b), (x,), (t,))[1], want)
+
+
+@gpu
+@pytest.mark.parametrize("rows", [2, 8, 24])
+def test_vmap(rows):
+    from shuffle_exchange_amd.ops.linear import linear
+    x, w, b = _operands(3 * rows)
+    with torch.no_grad():
+        _close(torch.func.vmap(lambda a: linear(a, w, b))(x.view(3, rows, -1)), F.linear(x, w, b).view(3, rows, -1))
+
+
+@gpu
+@pytest.mark.parametrize("rows", [4, 8, 32])
+def test_traces(rows):
+    """A trace of few rows runs more, and a fake tensor has no memory to look at."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from shuffle_exchange_amd.ops.linear import linear
+    x, w, b = _operands(rows)
+    with torch.no_grad():
+        traced = torch.jit.trace(lambda a: linear(a, w, b), (x,), check_trace=False)
+        many = _operands(100)[0]
+        _close(traced(many), F.linear(many, w, b))
+        with FakeTensorMode(allow_non_fake_inputs=True) as mode:
+            assert linear(mode.from_tensor(x), w, b).shape == (rows, 64)
+
+
+@gpu
+def test_column_sum_transforms():
+    from shuffle_exchange_amd.ops.linear import column_sum
+    x = torch.randn(3, 40, 72, device="cuda")
+    f = lambda a: column_sum(a, a.dtype)  # noqa: E731
+    torch.testing.assert_close(torch.func.vmap(f)(x), x.sum(1), rtol=1e-5, atol=1e-4)
+    torch.testing.assert_close(torch.func.jvp(f, (x[0],), (x[1],))[1], x[1].sum(0), rtol=1e-5, atol=1e-4)
