@@ -463,7 +463,7 @@ class _Linear(torch.autograd.Function):
 def linear(x, weight, bias=None):
     if not isinstance(weight, torch.Tensor):  # quantized inference weight (ops/fp_quantizer.FP8Weight)
         return weight.linear(x, bias)
-    grad = torch.is_grad_enabled() and (weight.requires_grad or x.requires_grad)
+    grad = torch.is_grad_enabled() and (weight.requires_grad or x.requires_grad or (bias is not None and bias.requires_grad))
     if grad and weight.requires_grad and hasattr(weight, "_sxe_grad_target"):
         return _Linear.apply(x, weight, bias)
     if (not grad and SKINNY_MAX_M > 0 and x.is_cuda and x.numel() <= max(SKINNY_MAX_M, STREAM_ROWS_SMALL) * x.shape[-1]

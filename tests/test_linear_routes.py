@@ -1,5 +1,5 @@
 """Which calls the kernels behind ops/linear.py take: those that read tensors' memory and differentiate by no operator.
-Everything else -- transformed or fake tensors, traces, forward-mode derivatives -- runs the library's product."""
+Everything else -- transformed or fake tensors, traces, forward-mode derivatives, trainable biases -- runs the library's product."""
 import pytest
 import torch
 import torch.autograd.forward_ad as fwAD
@@ -107,3 +107,16 @@ def test_column_sum_transforms():
     f = lambda a: column_sum(a, a.dtype)  # noqa: E731
     torch.testing.assert_close(torch.func.vmap(f)(x), x.sum(1), rtol=1e-5, atol=1e-4)
     torch.testing.assert_close(torch.func.jvp(f, (x[0],), (x[1],))[1], x[1].sum(0), rtol=1e-5, atol=1e-4)
+
+
+@gpu
+@pytest.mark.parametrize("rows", [4, 8, 32, 40])
+def test_trainable_bias_alone(rows):
+    """Bias-only training: the first layer's input and weight want no gradient, its bias does."""
+    from shuffle_exchange_amd.ops.linear import linear
+    x, w, b = _operands(rows)
+    b.requires_grad_()
+    y = linear(x, w, b)
+    assert y.requires_grad
+    y.float().sum().backward()
+    assert torch.equal(b.grad, torch.full_like(b, rows))
