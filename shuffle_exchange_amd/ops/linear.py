@@ -38,12 +38,16 @@ TN_FP32_OUT = os.environ.get("SXE_WGRAD_TN_FP32OUT", "1") == "1"
 SKINNY_MAX_M = int(os.environ.get("SXE_SKINNY_MAX_M", 4))
 
 
+def _bias_ok(bias, weight):
+    return bias is None or (bias.dtype == torch.bfloat16 and bias.shape == weight.shape[:1] and bias.is_contiguous())
+
+
 def _skinny(x, weight, bias):
     K = x.shape[-1]
     if not (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.dim() == 2
             and weight.is_contiguous() and K % 8 == 0 and weight.data_ptr() % 16 == 0):
         return None
-    if bias is not None and not (bias.dtype == torch.bfloat16 and bias.is_contiguous()):
+    if not _bias_ok(bias, weight):
         return None
     x2 = x.reshape(-1, K)
     if not (0 < x2.shape[0] <= SKINNY_MAX_M and x2.stride(1) == 1 and x2.stride(0) % 8 == 0
@@ -63,7 +67,7 @@ def _streamable(x2, weight, bias, unit=8):
     return (x2.dtype == torch.bfloat16 and x2.stride(1) == 1 and x2.stride(0) % 8 == 0 and x2.data_ptr() % 16 == 0
             and weight.dim() == 2 and weight.stride(1) == 1 and weight.stride(0) % unit == 0 and weight.data_ptr() % 16 == 0
             and weight.shape[1] == x2.shape[1] and x2.shape[1] % unit == 0 and weight.shape[0] % 4 == 0 and weight.shape[0] > 0
-            and x2.shape[1] > 0 and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous())))
+            and x2.shape[1] > 0 and _bias_ok(bias, weight))
 
 
 def _stream(x, weight, bias):

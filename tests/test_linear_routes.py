@@ -120,3 +120,16 @@ def test_trainable_bias_alone(rows):
     assert y.requires_grad
     y.float().sum().backward()
     assert torch.equal(b.grad, torch.full_like(b, rows))
+
+
+@gpu
+@pytest.mark.parametrize("rows", [4, 8, 32, 40])
+def test_bias_forms(rows):
+    """What the library's product takes as a bias is taken at every row count, and a bias of another length is refused."""
+    from shuffle_exchange_amd.ops.linear import linear
+    x, w, b = _operands(rows)
+    for bias in (b[:1], b.repeat(2)[::2].contiguous(), torch.stack([b, b], 1)[:, 0]):
+        with torch.no_grad():
+            _close(linear(x, w, bias), F.linear(x, w, bias))
+    with pytest.raises(RuntimeError), torch.no_grad():
+        linear(x, w, b[:7])
