@@ -133,3 +133,12 @@ def test_bias_forms(rows):
             _close(linear(x, w, bias), F.linear(x, w, bias))
     with pytest.raises(RuntimeError), torch.no_grad():
         linear(x, w, b[:7])
+
+
+@gpu
+def test_autocast_type():
+    from shuffle_exchange_amd.ops.linear import linear
+    for rows in (4, 8, 32, 40):
+        x, w, b = _operands(rows)
+        with torch.no_grad(), torch.autocast("cuda", torch.float16):
+            assert linear(x, w, b).dtype == F.linear(x, w, b).dtype == torch.float16
