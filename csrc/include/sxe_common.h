@@ -29,6 +29,13 @@ namespace sxe {
 constexpr int kWave = 64;
 constexpr int kNumCUs = 256;
 
+// What a kernel reads or writes beside `t` lies on t's GPU: a pointer into host memory or another GPU's faults in the kernel.
+inline void check_beside(const at::Tensor& t, std::initializer_list<c10::optional<at::Tensor>> others) {
+  SXE_CHECK_CUDA(t);
+  for (const auto& o : others)
+    SXE_CHECK(!o.has_value() || !o->defined() || o->device() == t.device(), "an operand is on ", o->device(), ", the others on ", t.device());
+}
+
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));

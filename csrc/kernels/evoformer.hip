@@ -598,7 +598,7 @@ static void evo_dispatch(int D, at::ScalarType pair, F f) {
 
 std::vector<at::Tensor> evoformer_fwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
                                       const c10::optional<at::Tensor>& b1, const c10::optional<at::Tensor>& b2) {
-  SXE_CHECK_CUDA(q);
+  check_beside(q, {k, v, b1, b2});
   c10::DeviceGuard g(q.device());
   EvoCall c = evo_call(q, k, v, b1, b2, false);
   evo::Args& a = c.a;
@@ -619,7 +619,7 @@ std::vector<at::Tensor> evoformer_fwd(const at::Tensor& q, const at::Tensor& k, 
 std::vector<at::Tensor> evoformer_bwd(const at::Tensor& dout, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
                                       const at::Tensor& o, const at::Tensor& lse, const c10::optional<at::Tensor>& b1,
                                       const c10::optional<at::Tensor>& b2, bool need_db1, bool need_db2) {
-  SXE_CHECK_CUDA(q);
+  check_beside(q, {dout, k, v, o, lse, b1, b2});
   c10::DeviceGuard g(q.device());
   EvoCall c = evo_call(q, k, v, b1, b2, true);
   evo::Args& a = c.a;

@@ -559,7 +559,7 @@ static at::Tensor paged_attention_impl(const at::Tensor& q, const at::Tensor& ca
                                        std::vector<at::Tensor>* parts, const c10::optional<at::Tensor>& counters = {},
                                        const at::Tensor* seqs = nullptr, const at::Tensor* rows = nullptr,
                                        const at::Tensor* into = nullptr) {
-  SXE_CHECK_CUDA(q);
+  check_beside(q, {cache, block_table, q_start, q_len, kv_len, counters});
   SXE_CHECK(q.scalar_type() == at::kBFloat16 && cache.scalar_type() == at::kBFloat16, "bf16 only");
   SXE_CHECK(q.dim() == 3 && q.stride(2) == 1 && q.stride(1) == q.size(2), "q must be [T, nq, D] with head stride D");
   SXE_CHECK(cache.dim() == 5 && cache.is_contiguous(), "cache must be [blocks, 2, nkv, bs, D]");
@@ -652,9 +652,10 @@ void paged_attention_some(const at::Tensor& q, const at::Tensor& cache, const at
                           const at::Tensor& q_start, const at::Tensor& q_len, const at::Tensor& kv_len,
                           const at::Tensor& seqs, const at::Tensor& rows, double scale, int64_t max_kv_len, int64_t splits,
                           int64_t window, at::Tensor out) {
-  SXE_CHECK(seqs.is_cuda() && seqs.scalar_type() == at::kInt && seqs.is_contiguous() && seqs.dim() == 2 && seqs.size(1) == 2,
+  check_beside(q, {seqs, rows, out});
+  SXE_CHECK(seqs.scalar_type() == at::kInt && seqs.is_contiguous() && seqs.dim() == 2 && seqs.size(1) == 2,
             "paged_attention_some: seqs int32 [n, 2]");
-  SXE_CHECK(rows.is_cuda() && rows.scalar_type() == at::kInt && rows.is_contiguous(), "paged_attention_some: rows int32 [R]");
+  SXE_CHECK(rows.scalar_type() == at::kInt && rows.is_contiguous(), "paged_attention_some: rows int32 [R]");
   SXE_CHECK(out.sizes() == q.sizes() && out.is_contiguous() && out.scalar_type() == at::kBFloat16,
             "paged_attention_some: out contiguous bf16 like q");
   paged_attention_impl(q, cache, block_table, q_start, q_len, kv_len, scale, max_kv_len, splits, window, nullptr, {}, &seqs,

@@ -213,7 +213,7 @@ void paged_merge(const at::Tensor& part_o, const at::Tensor& part_ml, const at::
 void paged_prefill(const at::Tensor& q, const at::Tensor& cache, const at::Tensor& block_table, const at::Tensor& q_start,
                    const at::Tensor& q_len, const at::Tensor& kv_len, const at::Tensor& tiles,
                    const c10::optional<at::Tensor>& rows, double scale, int64_t window, int64_t splits, int64_t keys_per_split, at::Tensor out) {
-  SXE_CHECK_CUDA(q);
+  check_beside(q, {cache, block_table, q_start, q_len, kv_len, tiles, rows, out});
   SXE_CHECK(q.scalar_type() == at::kBFloat16 && cache.scalar_type() == at::kBFloat16 && out.scalar_type() == at::kBFloat16,
             "paged_prefill: bf16 only");
   SXE_CHECK(q.dim() == 3 && q.stride(2) == 1 && q.stride(1) == q.size(2) && q.stride(0) % 8 == 0 &&
@@ -255,7 +255,7 @@ void paged_prefill(const at::Tensor& q, const at::Tensor& cache, const at::Tenso
   a.out_tok_stride = out.stride(0);
   at::Tensor part_o, part_ml;
   if (splits > 1) {
-    SXE_CHECK(rows.has_value() && rows->scalar_type() == at::kInt && rows->is_contiguous() && rows->is_cuda(),
+    SXE_CHECK(rows.has_value() && rows->scalar_type() == at::kInt && rows->is_contiguous(),
               "paged_prefill: rows int32 [R]");
     a.part_rows = rows->numel();
     part_o = at::empty({splits, a.part_rows, nq, D}, q.options().dtype(at::kFloat));

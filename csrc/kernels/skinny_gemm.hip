@@ -633,7 +633,7 @@ void launch(const Operands& o, const Plan& p, const ProArgs& pro) {
 
 // x [M, K] (row stride free, unit column stride), w [N, K] contiguous rows, bias [N] or None.
 at::Tensor skinny_gemm(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias) {
-  SXE_CHECK_CUDA(x);
+  check_beside(x, {w, bias});
   SXE_CHECK(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16, "skinny_gemm: bf16 only");
   SXE_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1), "skinny_gemm: x [M, K], w [N, K]");
   SXE_CHECK(x.stride(1) == 1 && w.stride(1) == 1, "skinny_gemm: unit stride along K");
@@ -661,7 +661,7 @@ at::Tensor skinny_gemm(const at::Tensor& x, const at::Tensor& w, const c10::opti
 // x [M, K] bf16, wq [N, K] e4m3 bytes (uint8 or float8_e4m3fn), wscale [N] fp32, bias [N] bf16 or None
 at::Tensor skinny_gemm_fp8w(const at::Tensor& x, const at::Tensor& wq, const at::Tensor& wscale,
                             const c10::optional<at::Tensor>& bias) {
-  SXE_CHECK_CUDA(x);
+  check_beside(x, {wq, wscale, bias});
   SXE_CHECK(x.scalar_type() == at::kBFloat16, "skinny_gemm_fp8w: bf16 activations");
   SXE_CHECK(wq.element_size() == 1 && wq.dim() == 2 && wq.stride(1) == 1, "skinny_gemm_fp8w: wq [N, K] bytes");
   SXE_CHECK(wscale.scalar_type() == at::kFloat && wscale.is_contiguous() && wscale.numel() == wq.size(0),
@@ -702,7 +702,8 @@ static std::vector<at::Tensor> skinny_gemm_pro_impl(const at::Tensor& x, const c
                                                     const at::Tensor& w, const c10::optional<at::Tensor>& wscale,
                                                     const c10::optional<at::Tensor>& bias, int64_t mode,
                                                     const RopeTensors* rope) {
-  SXE_CHECK_CUDA(x);
+  check_beside(x, {res, gw, w, wscale, bias});
+  if (rope != nullptr) check_beside(x, {*rope->cos, *rope->sin, *rope->pos, *rope->slots, *rope->cache});
   const bool glu = mode == kRmsGlu;
   if (glu) mode = sg::PRO_RMS;
   SXE_CHECK(mode == sg::PRO_RMS || mode == sg::PRO_SWIGLU, "skinny_gemm_pro: mode 1 (rms), 2 (swiglu) or 3 (rms, swiglu epilogue)");
@@ -799,7 +800,7 @@ std::vector<at::Tensor> skinny_gemm_pro_rope(const at::Tensor& x, const c10::opt
 // (wscale None) or e4m3 bytes with wscale fp32 [N]; K = nq * D. One launch instead of merge + GEMM.
 at::Tensor skinny_gemm_merge(const at::Tensor& part_o, const at::Tensor& part_ml, const at::Tensor& w,
                              const c10::optional<at::Tensor>& wscale, const c10::optional<at::Tensor>& bias) {
-  SXE_CHECK_CUDA(part_o);
+  check_beside(part_o, {part_ml, w, wscale, bias});
   SXE_CHECK(part_o.scalar_type() == at::kFloat && part_o.dim() == 4 && part_o.is_contiguous() &&
                 part_ml.scalar_type() == at::kFloat && part_ml.is_contiguous() && part_ml.dim() == 4 &&
                 part_ml.size(0) == part_o.size(0) && part_ml.size(1) == part_o.size(1) &&

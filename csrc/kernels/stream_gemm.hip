@@ -206,7 +206,7 @@ __global__ void __launch_bounds__(64 * NW, 2) stream_gemm_kernel(Args a) {
 // x [M, K] bf16, w [N, K] bf16, or e4m3 bytes with wscale fp32 [N]; bias bf16 [N] or None; glu: w = gate | up
 at::Tensor stream_gemm(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& wscale,
                        const c10::optional<at::Tensor>& bias, bool glu) {
-  SXE_CHECK_CUDA(x);
+  check_beside(x, {w, wscale, bias});
   const bool fp8 = wscale.has_value() && wscale->defined();
   SXE_CHECK(x.scalar_type() == at::kBFloat16 && x.dim() == 2 && x.stride(1) == 1 && w.is_cuda() && w.dim() == 2 && w.stride(1) == 1 &&
                 x.size(1) == w.size(1) && (fp8 ? w.element_size() == 1 : w.scalar_type() == at::kBFloat16),

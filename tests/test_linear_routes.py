@@ -142,3 +142,22 @@ def test_autocast_type():
         x, w, b = _operands(rows)
         with torch.no_grad(), torch.autocast("cuda", torch.float16):
             assert linear(x, w, b).dtype == F.linear(x, w, b).dtype == torch.float16
+
+
+@gpu
+@pytest.mark.parametrize("rows", [4, 8, 32, 40])
+def test_operands_on_one_device(rows):
+    """A bias or scale in host memory is refused before any launch."""
+    from shuffle_exchange_amd.ops.fp_quantizer import FP8Weight
+    from shuffle_exchange_amd.ops.linear import linear
+    x, w, b = _operands(rows)
+    q = FP8Weight(w)
+    with torch.no_grad():
+        with pytest.raises(RuntimeError):
+            linear(x, w, b.cpu())
+        if rows <= 16:
+            for scale, bias in ((q.scale.cpu(), b), (q.scale, b.cpu())):
+                q.scale = scale
+                with pytest.raises(RuntimeError, match="operand is on cpu"):
+                    q.linear(x, bias)
+                q.scale = scale.cuda()

@@ -72,3 +72,21 @@ def test_ragged_attention(seqs, nq, nkv, D, bs, window):
     for i in range(b.num_seqs):  # every sequence for itself: a short one cannot hide behind a long one
         s, n = b.host_q_start[i], b.host_q_len[i]
         assert ((got[s:s + n].float() - ref[s:s + n]).norm() / ref[s:s + n].norm()).item() < 8e-3, seqs[i]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("seqs", [[(0, 70)], [(300, 1)], [(0, 70), (300, 1)]])
+def test_metadata_on_one_device(seqs):
+    """Lists left in host memory are refused before any launch."""
+    b, blocks = _batch(seqs, 64, "cuda")
+    cache = torch.zeros(blocks, 2, 2, 64, 128, device="cuda", dtype=torch.bfloat16)
+    q = torch.randn(b.num_tokens, 4, 128, device="cuda").to(torch.bfloat16)
+    for name in ("block_table", "q_start", "q_len", "kv_len"):
+        there = getattr(b, name)
+        setattr(b, name, there.cpu())
+        with pytest.raises(RuntimeError, match="operand is on cpu"):
+            PA.ragged_attention(q, cache, b, 128 ** -0.5)
+        setattr(b, name, there)
+    with pytest.raises(RuntimeError, match="operand is on cpu"):
+        PA.ragged_attention(q, cache.cpu(), b, 128 ** -0.5)
+    PA.ragged_attention(q, cache, b, 128 ** -0.5)
