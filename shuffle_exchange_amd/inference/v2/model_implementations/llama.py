@@ -29,7 +29,8 @@ import torch.nn.functional as F
 
 from ....ops import native
 from ....ops.activation import swiglu
-from ....ops.linear import linear
+from ....ops.linear import Linear, is_own_forward, linear
+from ....ops.norm import RMSNorm
 from ....ops.paged_attention import paged_attention_parts, paged_batch_attention, ragged_attention, rope_kv_cache_append
 from ....ops.rows import gather_last
 
@@ -225,9 +226,10 @@ class RaggedLlama:
         return self._proj(attn.o_proj, o.reshape(T, self.nq * self.head_dim), li, "o")
 
     def _wobj(self, mod, li, key):
+        """The weight that a fused launch reads in place of running ``mod``; None where the module is more than its product."""
         if self.qw is not None and key in self.qw[li]:
             return self._impl_weight(self.qw[li][key])
-        return mod.weight
+        return mod.weight if is_own_forward(mod, Linear, torch.nn.Linear) else None
 
     @staticmethod
     def _impl_weight(impl):
@@ -235,7 +237,7 @@ class RaggedLlama:
 
     def _norm_proj(self, norm, x, res, mod, li, key):
         """(norm(x + res) @ W^T, h) through the fused kernel, else the separate launches."""
-        if self._fusable(x.shape[0]) and getattr(mod, "bias", None) is None:
+        if self._fusable(x.shape[0]) and getattr(mod, "bias", None) is None and is_own_forward(norm, RMSNorm):
             from ....ops.linear import fused_rms_linear
             r = fused_rms_linear(x, res, norm.weight, norm.eps, self._wobj(mod, li, key))
             if r is not None:
@@ -250,18 +252,18 @@ class RaggedLlama:
         if (self.tps is not None or not 0 < T <= 32 or (T <= self.FUSE_MAX_T and not self._fusable(T)) or self.device.type != "cuda"
                 or getattr(mlp.gate_up_proj, "bias", None) is not None or not native.hip_available()):
             return None, None
+        w, norm = self._wobj(mlp.gate_up_proj, li, "gu"), layer.post_attention_layernorm
         if T <= self.FUSE_MAX_T:
             from ....ops.linear import _pro_weight, fused_rms_glu
-            norm, w = layer.post_attention_layernorm, self._wobj(mlp.gate_up_proj, li, "gu")
             if _pro_weight(w) is None:
                 return None, None
-            r = fused_rms_glu(x, res, norm.weight, norm.eps, w)
+            r = fused_rms_glu(x, res, norm.weight, norm.eps, w) if is_own_forward(norm, RMSNorm) else None
             if r is not None:
                 return r
         from ....ops.linear import glu_linear
-        # quantized layers run more than 16 rows on the module's own weight
-        w = self._wobj(mlp.gate_up_proj, li, "gu") if T <= 16 else mlp.gate_up_proj.weight
-        a, h = layer.post_attention_layernorm(x, res)
+        if T > 16 and self.qw is not None:  # quantized layers run more than 16 rows on the weight as it came
+            w = self.qw[li]["gu"].weight
+        a, h = norm(x, res)
         mid = glu_linear(a, w)
         if mid is None:
             mid = swiglu(self._proj(mlp.gate_up_proj, a, li, "gu"))
@@ -345,7 +347,7 @@ class RaggedLlama:
             kv_layer = kv_cache.layer(li)
             r = None
             if (self._fusable(T) and self.head_dim == 128 and getattr(attn.qkv_proj, "bias", None) is None
-                    and os.environ.get("SXE_DECODE_FUSE_ATTN", "1") == "1"):
+                    and is_own_forward(layer.input_layernorm, RMSNorm) and os.environ.get("SXE_DECODE_FUSE_ATTN", "1") == "1"):
                 # decode: RMSNorm prologue + QKV GEMM + RoPE / KV-append epilogue in one launch
                 from ....ops.linear import fused_rms_rope_linear
                 ln = layer.input_layernorm
@@ -373,7 +375,7 @@ class RaggedLlama:
                 x, res = self._mlp(layer, m, li), h2
         last = batch.last_idx
         x = gather_last(x, last, res)
-        if self._fusable(x.shape[0]):
+        if self._fusable(x.shape[0]) and is_own_forward(model.norm, RMSNorm):
             from ....ops.linear import RMS_GLU_BF16, RMS_GLU_FP8, _pro_weight, fused_rms_linear
             w = model.lm_head.weight if self.qw is None else self._impl_weight(self.qhead)
             wk = _pro_weight(w)

@@ -480,6 +480,14 @@ def linear(x, weight, bias=None):
     return F.linear(x, weight, bias)
 
 
+def is_own_forward(mod, *types):
+    """``mod(x)`` runs the forward of one of ``types`` and nothing else, so a caller may read its weight and run another kernel: not a
+    subclass (low-rank, fake-quantized or partitioned layers), no patched forward, no hooks."""
+    every = torch.nn.modules.module
+    return (type(mod) in types and "forward" not in mod.__dict__ and not mod._forward_hooks and not mod._forward_pre_hooks
+            and not every._global_forward_hooks and not every._global_forward_pre_hooks)
+
+
 class Linear(torch.nn.Linear):
     """``nn.Linear`` whose GEMMs go through ``linear`` (fused weight-grad into ZeRO buffers).
     AutoTP swaps it for a column/row-parallel layer with the same call signature.

@@ -1,0 +1,103 @@
+"""Ragged Llama: the launches that read a module's weight themselves against the modules' own forwards, at the token counts where the
+route changes, and modules that do more than a product."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+HIDDEN, FF, VOCAB = 512, 1024, 512
+
+
+def _model(seed=0):
+    from shuffle_exchange_amd.models import LlamaForCausalLM, llama_config
+    torch.manual_seed(seed)
+    cfg = llama_config("llama-tiny", hidden_size=HIDDEN, intermediate_size=FF, num_attention_heads=4, num_key_value_heads=2,
+                       vocab_size=VOCAB, num_hidden_layers=2, max_position_embeddings=4096)
+    return LlamaForCausalLM(cfg).to("cuda", torch.bfloat16).eval()
+
+
+def _engine(model, **kw):
+    from shuffle_exchange_amd.inference.v2 import RaggedInferenceEngineConfig, build_engine
+    return build_engine(model, RaggedInferenceEngineConfig(kv_block_size=64, num_kv_blocks=128, decode_graphs=False, **kw))
+
+
+def _decode(engine, n):
+    """Logits of a prompt of 7 tokens for each of n sequences and of one decode step of all."""
+    g = torch.Generator().manual_seed(n)
+    prompts = [torch.randint(0, VOCAB, (7,), generator=g).tolist() for _ in range(n)]
+    first = torch.cat([engine.put([u], [p]) for u, p in enumerate(prompts)])
+    step = engine.put(list(range(n)), [[int(t)] for t in torch.randint(0, VOCAB, (n,), generator=g)])
+    return torch.cat([first, step])
+
+
+def _rel(a, b):
+    return ((a - b).norm() / b.norm()).item()
+
+
+@pytest.mark.parametrize("tokens", [1, 4, 5, 16, 17, 32, 33])
+@pytest.mark.parametrize("quant", [None, "fp8"])
+def test_gate_up_routes(tokens, quant, monkeypatch):
+    from shuffle_exchange_amd.inference.v2.model_implementations.llama import RaggedLlama
+    from shuffle_exchange_amd.ops.activation import swiglu
+    model = _model()
+    got = _decode(_engine(model, weight_quant=quant), tokens)
+
+    def apart(self, layer, x, res, li):
+        a, h = layer.post_attention_layernorm(x, res)
+        return swiglu(self._proj(layer.mlp.gate_up_proj, a, li, "gu")), h
+    monkeypatch.setattr(RaggedLlama, "_norm_glu", apart)
+    monkeypatch.setenv("SXE_DECODE_FUSE", "0")
+    want = _decode(_engine(model, weight_quant=quant), tokens)
+    # two layers of about six bf16 roundings (2^-9) on a branch of the stream's size; a wrong weight or residual is 1 or more
+    assert _rel(got, want) < 2e-2
+
+
+@pytest.mark.parametrize("tokens", [2, 8, 40])
+@pytest.mark.parametrize("which", ["qkv_proj", "o_proj", "gate_up_proj", "down_proj"])
+def test_lora_modules(tokens, which):
+    """A low-rank module beside its merged weight in a plain one."""
+    from shuffle_exchange_amd.linear import LoRAConfig, OptimizedLinear
+    model, merged = _model(), _model()
+    for layer, other in zip(model.layers, merged.layers):
+        owner, plain = ((layer.self_attn, other.self_attn) if hasattr(layer.self_attn, which) else (layer.mlp, other.mlp))
+        w = getattr(plain, which).weight
+        lora = OptimizedLinear(w.shape[1], w.shape[0], lora_config=LoRAConfig(lora_r=4, lora_alpha=8), device="cuda")
+        lora.load_base_weight(w.detach().clone())
+        with torch.no_grad():
+            lora.lora_weight_2.normal_(std=0.5 / w.shape[1] ** 0.5)
+            w.add_((lora.lora_weight_2.float() @ lora.lora_weight_1.float()).to(w.dtype), alpha=lora.lora_scaling)
+        setattr(owner, which, lora)
+    # as above, and the merged weight is rounded once more
+    assert _rel(_decode(_engine(model), tokens), _decode(_engine(merged), tokens)) < 2e-2
+
+
+@pytest.mark.parametrize("tokens", [2, 8])
+def test_hooks_run(tokens):
+    model = _model()
+    mods = [m for layer in model.layers for m in (layer.self_attn.qkv_proj, layer.self_attn.o_proj, layer.mlp.gate_up_proj,
+                                                  layer.mlp.down_proj, layer.input_layernorm, layer.post_attention_layernorm)]
+    mods.append(model.norm)
+    ran = []
+    for m in mods:
+        m.register_forward_hook(lambda mod, args, out: ran.append(id(mod)))
+    eng = _engine(model)
+    eng.put(list(range(tokens)), [[5]] * tokens)
+    assert set(ran) == {id(m) for m in mods}
+
+
+def test_changed_forward_runs():
+    """Subclasses and patched forwards, as compression and tensor-parallel replacement bring them."""
+    model = _model()
+    calls = []
+    for layer in model.layers:
+        class Counted(type(layer.mlp.gate_up_proj)):
+            def forward(self, x):
+                calls.append("class")
+                return super().forward(x)
+        layer.mlp.gate_up_proj.__class__ = Counted
+        old = layer.mlp.down_proj.forward
+        layer.mlp.down_proj.forward = lambda x, old=old: (calls.append("instance"), old(x))[1]
+    for n in (2, 8, 24):
+        calls.clear()
+        _engine(model).put(list(range(n)), [[5]] * n)
+        assert sorted(calls) == ["class"] * 2 + ["instance"] * 2
