@@ -34,8 +34,9 @@ class SXEHybridEngine(SXEEngine):
             cfg = RaggedInferenceEngineConfig(state_manager=StateManagerConfig(
                 memory_config=MemoryConfig(fraction=self._he_cfg.kv_cache_fraction)),
                 tensor_parallel={"tp_size": int(self._he_cfg.inference_tp_size)})
-            # expert weights may move between generations (optimizer steps, gathers): their steps run eagerly
-            cfg.decode_graphs = not any(is_moe_param(p) for p in self.module.parameters())
+            # weights that move between generations (experts: optimizer steps and gathers; fused low-rank weights are new tensors
+            # each time) are not for captured steps, which would read where they were
+            cfg.decode_graphs = not (self._lora_modules() or any(is_moe_param(p) for p in self.module.parameters()))
             if not torch.cuda.is_available():
                 cfg.num_kv_blocks = 1024
                 cfg.kv_block_size = 16

@@ -82,3 +82,20 @@ def test_lora_fuse_matches_unfused():
     fused = lin(x)
     lin.unfuse_lora()
     assert torch.allclose(fused, ref, atol=1e-5) and torch.allclose(lin(x), ref)
+
+
+def test_lora_generation_is_not_captured(monkeypatch):
+    """Every generation fuses its weights into new tensors: a captured decode step would read the former ones."""
+    from types import SimpleNamespace
+
+    import shuffle_exchange_amd.inference.v2 as v2
+    from shuffle_exchange_amd.linear.optimized_linear import LoRAConfig, OptimizedLinear
+    from shuffle_exchange_amd.runtime.hybrid_engine import SXEHybridEngine
+    monkeypatch.setattr(v2, "build_engine", lambda module, cfg: cfg)
+    for lora, graphs in ((None, True), (LoRAConfig(lora_r=2), False)):
+        eng = SXEHybridEngine.__new__(SXEHybridEngine)
+        torch.nn.Module.__init__(eng) if isinstance(eng, torch.nn.Module) else None
+        eng.module = torch.nn.Sequential(OptimizedLinear(16, 16, lora_config=lora))
+        eng._he_cfg = SimpleNamespace(kv_cache_fraction=0.5, inference_tp_size=1)
+        eng._ragged = None
+        assert eng._inference_engine().decode_graphs is graphs
