@@ -87,7 +87,7 @@ def glu_linear(x, weight):
     """silu(gate) * up of ``linear(x, weight)`` with weight = [gate | up], in ONE launch (stream_gemm.hip): up to 32 rows (16 of an
     FP8Weight), no autograd; None when not covered. One rounding, of the result."""
     wk = _pro_weight(weight)
-    if wk is None or not x.is_cuda or x.requires_grad or x.dim() != 2 or not native.plain(x):
+    if wk is None or SKINNY_MAX_M <= 0 or not x.is_cuda or x.requires_grad or x.dim() != 2 or not native.plain(x):
         return None
     w, sc = wk
     if not 0 < x.shape[0] <= (32 if sc is None else 16) or w.shape[0] % 32 or not _streamable(x, w, None, 8 if sc is None else 16):

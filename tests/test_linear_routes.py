@@ -161,3 +161,14 @@ def test_operands_on_one_device(rows):
                 with pytest.raises(RuntimeError, match="operand is on cpu"):
                     q.linear(x, bias)
                 q.scale = scale.cuda()
+
+
+@gpu
+def test_library_switch(monkeypatch):
+    """SXE_SKINNY_MAX_M = 0: no product of linear() or of the gated form leaves the library."""
+    from shuffle_exchange_amd.ops import linear as L
+    monkeypatch.setattr(L, "SKINNY_MAX_M", 0)
+    for rows in (1, 8, 32):
+        x, w, _ = _operands(rows)
+        with torch.no_grad():
+            assert L.glu_linear(x, w) is None and torch.equal(L.linear(x, w), F.linear(x, w))
