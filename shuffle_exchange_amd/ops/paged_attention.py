@@ -103,12 +103,17 @@ def choose_splits(num_seqs, nkv, max_kv_len, target_wgs=None):
 # Keys of a split at most where the batch has a merge launch anyway. Decode step of 4 Llama-8B layers, us at 1024 / 512 / 256:
 # 24 sequences of 270 - 5300 keys 935 / 920 / 937 (1097 with two splits of 4096), 32 of 3000 keys 1012 / 983 / 1020 (987).
 PA_SPLIT_KEYS = 512
+# Bytes of fp32 partials that such short splits may take: 256 decoding sequences keep splits of 512 keys up to 32k keys (heads of
+# 32 x 128), a call of many tokens has the splits of choose_splits, as its partials grow with tokens x splits.
+PA_SPLIT_BYTES = 1 << 28
 
 
-def choose_balanced_splits(num_seqs, nkv, max_kv_len):
+def choose_balanced_splits(num_seqs, nkv, max_kv_len, split_bytes):
     """``choose_splits``, and no split over PA_SPLIT_KEYS keys: sequences of a batch differ in length, and a workgroup that
-    walks a long one alone outlasts the rest. Splits behind a sequence's end exit at once, the merge does not read them."""
-    return max(choose_splits(num_seqs, nkv, max_kv_len), math.ceil(max_kv_len / PA_SPLIT_KEYS))
+    walks a long one alone outlasts the rest. Splits behind a sequence's end exit at once, the merge does not read them.
+    ``split_bytes``: partials of one split (rows x heads x head dim, fp32)."""
+    short = min(math.ceil(max_kv_len / PA_SPLIT_KEYS), PA_SPLIT_BYTES // max(1, split_bytes))
+    return max(choose_splits(num_seqs, nkv, max_kv_len), short)
 
 
 def paged_attention_parts(q, cache, block_table, q_start, q_len, kv_len, scale, max_kv_len, splits=None):
@@ -163,7 +168,7 @@ def paged_attention(q, cache, block_table, q_start, q_len, kv_len, scale, max_kv
         window = None
     if native.use_hip(q) and q.shape[-1] in (64, 128, 256):
         if splits is None:
-            splits = choose_balanced_splits(block_table.shape[0], cache.shape[2], max_kv_len)
+            splits = choose_balanced_splits(block_table.shape[0], cache.shape[2], max_kv_len, 4 * q.numel())
         S = block_table.shape[0]
         cnt = (_split_counters(q.device, S * cache.shape[2])
                if PA_LAST_MERGE and splits > 1 and q.shape[0] <= 4 * S else None)
@@ -225,7 +230,7 @@ def ragged_attention(q, cache, batch, scale, window=None):
     rows = batch.tile_rows(lists) if splits > 1 else None
     torch.ops.sxe.paged_prefill(*meta, lists.tiles, rows, float(scale), int(window or 0), splits, keys, out)
     if lists.seqs is not None:
-        splits = choose_balanced_splits(lists.seqs.shape[0], nkv, lists.seq_keys)
+        splits = choose_balanced_splits(lists.seqs.shape[0], nkv, lists.seq_keys, 4 * lists.seq_rows.numel() * q.shape[1] * q.shape[2])
         torch.ops.sxe.paged_attention_some(*meta, lists.seqs, lists.seq_rows, float(scale), int(lists.seq_keys), int(splits),
                                            int(window or 0), out)
     return out

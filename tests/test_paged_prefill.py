@@ -48,6 +48,18 @@ def test_tile_splits_cover_the_keys():
                 assert k % 64 == 0 and n * k >= keys > (n - 1) * k
 
 
+@pytest.mark.parametrize("rows,seqs,keys", [(8192, 1, 131072), (16984, 16, 16384), (32768, 64, 16384), (131072, 32, 4096), (256, 256, 131072),
+                                            (64, 64, 8192), (1, 1, 131072), (0, 1, 1)])
+@pytest.mark.parametrize("nq,nkv,D", [(32, 8, 128), (64, 8, 128), (16, 1, 256), (7, 7, 64)])
+def test_decode_splits_bound_their_partials(rows, seqs, keys, nq, nkv, D):
+    """The fp32 partials of a call do not grow with rows x keys: short splits only as far as they fit a fixed size."""
+    row = nq * D * 4
+    plain, n = PA.choose_splits(seqs, nkv, keys), PA.choose_balanced_splits(seqs, nkv, keys, rows * row)
+    assert n >= plain and (n == plain or n * rows * row <= PA.PA_SPLIT_BYTES)
+    if rows <= 64:  # decode-sized calls keep splits of at most 512 keys
+        assert n >= -(-keys // 512)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("seqs", [[(0, 33)], [(0, 1), (63, 65), (64, 64), (0, 129)], [(4000, 300), (700, 1), (31, 2), (5, 40)],
                                   [(1, 127), (127, 1), (0, 700), (2500, 9)]])
