@@ -340,7 +340,7 @@ def convert_hf_weights(spec, sd, hf_cfg=None):
 # ---------------------------------------------------------------------------- shared attention
 def ragged_attention(qkv, kv_layer, batch, nq, nkv, D, scale, window=None):
     """Attention of a ragged batch's new tokens over their paged KV (ops/paged_attention.py)."""
-    return _ragged_attention(qkv[:, :nq], kv_layer, batch, scale, window)
+    return _ragged_attention(qkv[:, :nq], kv_layer, batch, scale, window, kv=qkv[:, nq:])
 
 
 # Measured on MI355X (tools/grouped_gemm_bench.py, profiles/grouped_gemm_bench.log): the grouped

@@ -176,8 +176,8 @@ class RaggedLlama:
 
     def _attention(self, qkv, kv_layer, batch):
         pinned = (self._pins or {}).get("attention") == "dense_blocked_attention"
-        attend = paged_batch_attention if pinned else ragged_attention
-        return attend(qkv[:, :self.nq], kv_layer, batch, self.head_dim ** -0.5)
+        q, scale = qkv[:, :self.nq], self.head_dim ** -0.5
+        return paged_batch_attention(q, kv_layer, batch, scale) if pinned else ragged_attention(q, kv_layer, batch, scale, kv=qkv[:, self.nq:])
 
     def _proj(self, mod, x, li, key):
         if self.tps is not None:

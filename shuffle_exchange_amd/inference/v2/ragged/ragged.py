@@ -213,10 +213,10 @@ class DSStateManager:
 @dataclass
 class AttentionLists:
     """int32 device lists of one attention over a ragged batch: ``tiles`` [n, 4] (sequence, first token row, tokens, row among
-    the token rows that the tiles hold by sequence), ``tile_rows`` those rows (first row and count of each sequence until
+    the token rows that the tiles hold by sequence; None: none), ``tile_rows`` those rows (first row and count of each sequence until
     ``RaggedBatch.tile_rows`` is asked for them), ``tile_keys`` the longest key range; ``seqs`` [m, 2] (sequence, row among
     ``seq_rows``), ``seq_rows``, ``seq_keys`` the same for the sequences outside the tiles (None: none)."""
-    tiles: torch.Tensor
+    tiles: Optional[torch.Tensor]
     tile_rows: object
     tile_keys: int
     seqs: Optional[torch.Tensor]
@@ -327,26 +327,31 @@ class RaggedBatch:
             self._tables[key] = self._upload(rows, 2)
         return self._tables[key]
 
-    def attention_lists(self, tile, least):
+    def attention_lists(self, tile, least, done=(), tails=False):
         """What ops/paged_attention.ragged_attention launches, or None if no sequence has ``least`` new tokens: tiles of
-        up to ``tile`` tokens of the sequences that have, longest key range first, and the other sequences."""
-        key = ("attention", tile, least)
+        up to ``tile`` tokens of the sequences that have, longest key range first, and the other sequences. ``done``: (sequence,
+        its first new tokens that another launch takes) pairs; these sequences are left out, or with ``tails`` what is left of
+        them is all there is."""
+        key = ("attention", tile, least, done, tails)
         if key not in self._tables:
-            tiles, flat, held, rows, a = [], [], [], [], 0
+            tiles, flat, held, rows, a, first = [], [], [], [], 0, dict(done)
             for i, (q, n, seen) in enumerate(zip(self.host_q_start, self.host_q_len, self.host_seen)):
-                if n >= least:
-                    tiles += [(seen + min(j + tile, n), i, q + j, min(tile, n - j), a + j) for j in range(0, n, tile)]
-                    held.append((q, n))
-                    a += n
+                if (i in first) != tails:
+                    continue
+                at = first.get(i, 0)
+                if n >= least or tails:
+                    tiles += [(seen + min(j + tile, n), i, q + j, min(tile, n - j), a + j - at) for j in range(at, n, tile)]
+                    held.append((q + at, n - at))
+                    a += n - at
                 elif n:
                     flat += [i, len(rows)]
                     rows += range(q, q + n)
-            if tiles:
+            if tiles or (done and flat):
                 tiles.sort(reverse=True)
                 nt, ns = len(tiles), len(flat) // 2
                 d = self._upload([x for t in tiles for x in t[1:]] + flat + rows, 1).view(-1)  # one copy to the device
                 self._tables[key] = AttentionLists(
-                    d[:4 * nt].view(nt, 4), held, tiles[0][0], d[4 * nt:4 * nt + 2 * ns].view(ns, 2) if ns else None,
+                    d[:4 * nt].view(nt, 4) if nt else None, held, tiles[0][0] if nt else 0, d[4 * nt:4 * nt + 2 * ns].view(ns, 2) if ns else None,
                     d[4 * nt + 2 * ns:] if ns else None, max((self.host_kv_len[i] for i in flat[::2]), default=0))
             else:
                 self._tables[key] = None

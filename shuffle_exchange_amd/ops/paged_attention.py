@@ -211,25 +211,59 @@ def paged_batch_attention(q, cache, batch, scale, window=None):
                            window=window)
 
 
-def ragged_attention(q, cache, batch, scale, window=None):
+# The longest prompts take the training forward (csrc/kernels/flash_attn.hip) on the new tokens' own keys up to their last multiple of
+# 128 tokens, the tile kernel the tail. It is faster a tile, but starts with few of them and one prompt a launch; a tail costs a
+# launch with its merge. us, training forward (and tail) / tile kernel, heads of 128: 32 / 8 heads: 3072 tokens 114 / 106, 4096
+# 163 / 174, 5120 256 / 249, 6144 345 / 348, 6200 397 / 366, 8192 544 / 618, 8193 589 / 623, 16500 2200 / 2421, 32767 8850 / 9420;
+# 24 / 8: 5120 181 / 199, 9000 554 / 580; 16 / 4: 6144 189 / 191, 8192 280 / 330, 9000 388 / 388, 12300 681 / 694; 8 / 2: 12300
+# 388 / 378, 16384 538 / 640; 4 / 1: 12416 270 / 240, 65500 4440 / 4830.
+# (new tokens, new tokens x query heads) from which, without a tail and with one
+FLASH_WHOLE, FLASH_TAIL = (4096, 1 << 17), (8192, 3 << 16)
+
+
+def _flash_prompts(q, kv, batch, window):
+    """Pairs (sequence, first tokens) that the training forward takes."""
+    if kv is None or window is not None or q.shape[-1] != 128 or not (kv.is_cuda and kv.dtype == q.dtype and kv.stride()[1:] == (128, 1)):
+        return ()
+    took = []
+    for i, (n, seen) in enumerate(zip(batch.host_q_len, batch.host_seen)):
+        tokens, work = FLASH_TAIL if n % 128 else FLASH_WHOLE
+        if seen == 0 and n >= tokens and n * q.shape[1] >= work:
+            took.append((i, n // 128 * 128))
+    return tuple(took)
+
+
+def ragged_attention(q, cache, batch, scale, window=None, kv=None):
     """Causal attention of a ragged batch's new tokens q [T, nq, D] over their paged keys (the new ones among them).
     Sequences with many new tokens -- prompts, and chunks of prompts behind earlier tokens -- run the tile kernel, the
-    others the decode kernel."""
+    others the decode kernel. ``kv`` [T, 2 nkv, D]: the new tokens' keys and values as they are in the cache, for the longest
+    prompts."""
     nkv = cache.shape[2]
     if window is not None and batch.max_kv_len <= window:
         window = None
-    lists = None
-    if hasattr(batch, "attention_lists") and _tileable(q, cache, scale):
-        G = q.shape[1] // nkv
-        lists = batch.attention_lists(TILE_ROWS // G, -(-TILE_MIN_ROWS // G))
-    if lists is None:
+    if not (hasattr(batch, "attention_lists") and _tileable(q, cache, scale)):
         return paged_batch_attention(q, cache, batch, scale, window)
-    out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+    tile, least = TILE_ROWS // (q.shape[1] // nkv), -(-TILE_MIN_ROWS // (q.shape[1] // nkv))
+    flash = _flash_prompts(q, kv, batch, window)
+    lists = batch.attention_lists(tile, least, flash)
+    if lists is None and not flash:
+        return paged_batch_attention(q, cache, batch, scale, window)
+    out = None
+    for i, n in flash:
+        at = slice(batch.host_q_start[i], batch.host_q_start[i] + n)
+        o = torch.ops.sxe.flash_attn_fwd(q[None, at], kv[None, at, :nkv], kv[None, at, nkv:], True, float(scale))[0][0]
+        if n == q.shape[0]:
+            return o
+        out = torch.empty(q.shape, dtype=q.dtype, device=q.device) if out is None else out
+        out[at] = o
+    out = torch.empty(q.shape, dtype=q.dtype, device=q.device) if out is None else out
     meta = (q, cache, batch.block_table, batch.q_start, batch.q_len, batch.kv_len)
-    splits, keys = choose_tile_splits(lists.tiles.shape[0], nkv, lists.tile_keys)
-    rows = batch.tile_rows(lists) if splits > 1 else None
-    torch.ops.sxe.paged_prefill(*meta, lists.tiles, rows, float(scale), int(window or 0), splits, keys, out)
-    if lists.seqs is not None:
+    for x in (batch.attention_lists(tile, least, flash, True) if flash else None, lists):
+        if x is not None and x.tiles is not None:
+            splits, keys = choose_tile_splits(x.tiles.shape[0], nkv, x.tile_keys)
+            rows = batch.tile_rows(x) if splits > 1 else None
+            torch.ops.sxe.paged_prefill(*meta, x.tiles, rows, float(scale), int(window or 0), splits, keys, out)
+    if lists is not None and lists.seqs is not None:
         splits = choose_balanced_splits(lists.seqs.shape[0], nkv, lists.seq_keys, 4 * lists.seq_rows.numel() * q.shape[1] * q.shape[2])
         torch.ops.sxe.paged_attention_some(*meta, lists.seqs, lists.seq_rows, float(scale), int(lists.seq_keys), int(splits),
                                            int(window or 0), out)

@@ -102,3 +102,66 @@ def test_metadata_on_one_device(seqs):
     with pytest.raises(RuntimeError, match="operand is on cpu"):
         PA.ragged_attention(q, cache.cpu(), b, 128 ** -0.5)
     PA.ragged_attention(q, cache, b, 128 ** -0.5)
+
+
+def test_lists_without_long_prompts():
+    """The sequences that another launch takes are in neither list, their last tokens in one of their own."""
+    seqs = [(0, 300), (0, 70), (40, 1), (0, 256)]
+    b, _ = _batch(seqs, 16, "cpu")
+    done = ((0, 256), (3, 256))
+    rest, tails = b.attention_lists(32, 9, done), b.attention_lists(32, 9, done, True)
+    rows = lambda x: sorted(t for _, q, n, _ in x.tiles.tolist() for t in range(q, q + n))  # noqa: E731
+    assert rows(rest) == list(range(300, 370)) and rest.seq_rows.tolist() == [370]
+    assert rows(tails) == list(range(256, 300)) == b.tile_rows(tails).tolist() and tails.seqs is None and tails.tile_keys == 300
+    for x in (rest, tails):
+        for _, q, n, at in x.tiles.tolist():
+            assert b.tile_rows(x)[at:at + n].tolist() == list(range(q, q + n))
+    b, _ = _batch([(0, 256), (40, 1)], 16, "cpu")
+    done = ((0, 256),)
+    assert b.attention_lists(32, 9, done).tiles is None and b.attention_lists(32, 9, done).seq_rows.tolist() == [256]
+    assert b.attention_lists(32, 9, done, True) is None
+    b, _ = _batch([(0, 256)], 16, "cpu")
+    assert b.attention_lists(32, 9, done) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("seqs", [[(0, 256)], [(0, 129)], [(0, 128), (40, 1)], [(0, 300), (0, 70), (200, 1), (0, 256), (130, 260)],
+                                  [(0, 20), (0, 8319)]])
+@pytest.mark.parametrize("nq,nkv", [(8, 2), (6, 2), (16, 16)])
+def test_long_prompts(seqs, nq, nkv, monkeypatch):
+    """The training forward for a prompt's first tokens beside the tile and decode kernels for the rest of the batch."""
+    for name in ("FLASH_WHOLE", "FLASH_TAIL"):
+        monkeypatch.setattr(PA, name, (128, 1))
+    b, blocks = _batch(seqs, 64, "cuda", seed=3)
+    g = torch.Generator(device="cuda").manual_seed(4)
+    cache = torch.randn(blocks, 2, nkv, 64, 128, device="cuda", generator=g).to(torch.bfloat16)
+    qkv = torch.randn(b.num_tokens, nq + 2 * nkv, 128, device="cuda", generator=g).to(torch.bfloat16)
+    PA.kv_cache_append(qkv, cache, b.slots, nq, nkv)
+    took = PA._flash_prompts(qkv[:, :nq], qkv[:, nq:], b, None)
+    assert took == tuple((i, n // 128 * 128) for i, (c, n) in enumerate(seqs) if c == 0 and n >= 128)
+    got = PA.ragged_attention(qkv[:, :nq], cache, b, 128 ** -0.5, kv=qkv[:, nq:])
+    want = PA.ragged_attention(qkv[:, :nq], cache, b, 128 ** -0.5)  # checked against the reference above
+    for i in range(b.num_seqs):
+        s, n = b.host_q_start[i], b.host_q_len[i]
+        # p and the output are rounded to 8 bits on either side: 2 x 2^-9 each
+        assert ((got[s:s + n] - want[s:s + n]).float().norm() / want[s:s + n].float().norm()).item() < 8e-3, seqs[i]
+
+
+def test_long_prompt_rule():
+    """A prompt without history, long enough and with heads enough to fill the chip; never under a window."""
+    class B:
+        def __init__(self, *seqs):
+            self.host_seen, self.host_q_len = [c for c, _ in seqs], [n for _, n in seqs]
+
+    class T:
+        is_cuda, dtype = True, torch.bfloat16
+
+        def __init__(self, heads, D=128):
+            self.shape, self.H = (1, heads, D), heads
+
+        def stride(self):
+            return (self.H * 128, 128, 1)
+    b = B((0, 8192), (0, 8191), (64, 9000), (0, 9000), (0, 40), (0, 4096), (0, 3968))
+    assert PA._flash_prompts(T(32), T(16), b, None) == ((0, 8192), (3, 8960), (5, 4096))
+    assert PA._flash_prompts(T(16), T(8), b, None) == ((0, 8192),) and PA._flash_prompts(T(8), T(4), b, None) == ()
+    assert PA._flash_prompts(T(32), T(16), b, 4096) == () == PA._flash_prompts(T(32), None, b, None) == PA._flash_prompts(T(32, 64), T(16), b, None)
