@@ -46,11 +46,12 @@ __device__ __forceinline__ bf16x8 tr_at(const char* base, const int (&o)[2]) {
 extern __shared__ __attribute__((aligned(16))) char lds[];  // a kernel's dynamic LDS
 
 // 16 bytes per lane from `src` to lane-linear LDS at the wave-uniform `dst`. Inline asm, so that the compiler's
-// wait counts do not tie it to the LDS reads in between: consumers run wait_loads() and a barrier.
+// wait counts do not tie it to the LDS reads in between: consumers run wait_loads() and a barrier. s_nop: the vector memory
+// instruction reads m0 one wait state behind the scalar write at the earliest, and the compiler adds none inside this text.
 __device__ __forceinline__ void glds16(const void* src, char* dst) {
   const unsigned a = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)lds +
                                                     (unsigned)(dst - lds));
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(a), "v"(src) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(a), "v"(src) : "memory", "m0");
 }
 __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 

@@ -118,7 +118,7 @@ __device__ __forceinline__ float bias_term(const Bias<BT>& b, int i, float m) {
 __device__ __forceinline__ void glds4(const void* src, char* dst) {
   const unsigned a = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)lds +
                                                     (unsigned)(dst - lds));
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(a), "v"(src) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(a), "v"(src) : "memory", "m0");
 }
 
 // rows row0 .. of x (rows of one (b, n), head h) to LDS; rows behind L are zeros

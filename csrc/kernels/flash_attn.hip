@@ -244,12 +244,13 @@ __device__ __forceinline__ unsigned lds_addr(const char* p) {
   return __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem +
                                         (unsigned)(p - smem));
 }
+// s_nop: the load reads m0 one wait state behind the scalar write at the earliest
 __device__ __forceinline__ void glds16(const void* gsrc, char* lds_wave_base) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_addr(lds_wave_base)), "v"(gsrc)
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_addr(lds_wave_base)), "v"(gsrc)
                : "memory", "m0");
 }
 __device__ __forceinline__ void glds4(const void* gsrc, char* lds_wave_base) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_addr(lds_wave_base)), "v"(gsrc)
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_addr(lds_wave_base)), "v"(gsrc)
                : "memory", "m0");
 }
 template <int ROWS, int D, int NWV = NW>

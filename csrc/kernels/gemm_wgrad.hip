@@ -73,9 +73,10 @@ __device__ __forceinline__ bf16x8 frag_at(const char* lane_base, int row0) {
 // LDS-DMA issued from inline asm: hipcc's waitcnt pass cannot see it, so it does not put a
 // conservative `s_waitcnt vmcnt(0)` in front of every ds_read of the ring (it did with the
 // builtin: the whole prefetch drained each K-step). Completion is tracked by the explicit counted
-// vmcnt + barrier in the main loop. `lds` is the wave-uniform LDS byte address (M0).
+// vmcnt + barrier in the main loop. `lds` is the wave-uniform LDS byte address (M0), which the load reads
+// one wait state behind the scalar write at the earliest (s_nop).
 __device__ __forceinline__ void glds16(const void* gsrc, unsigned lds) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(gsrc) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(gsrc) : "memory", "m0");
 }
 
 // Per-thread DMA source/destination of one slab. Wave w moves 4 k rows x 256 bytes of A-half

@@ -201,9 +201,9 @@ __device__ __forceinline__ unsigned pack2(float a, float b) {
 __device__ __forceinline__ unsigned lds_at(const char* p) {
   return __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(const __attribute__((address_space(3))) char*)p);
 }
-// the same with a base per lane
+// the same with a base per lane (s_nop: the load reads m0 one wait state behind its write at the earliest)
 __device__ __forceinline__ void dma16(unsigned lds, const void* src) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
 }
 __device__ __forceinline__ const unsigned short* uniform_ptr(const unsigned short* p) {
   const uint64_t v = (uint64_t)p;
@@ -213,7 +213,7 @@ __device__ __forceinline__ const unsigned short* uniform_ptr(const unsigned shor
 // 16 bytes per lane from base + off straight to LDS at lds + 16 lane. Inline asm: the compiler's wait-count
 // pass would put a full wait before every later LDS read that might alias it.
 __device__ __forceinline__ void dma16(unsigned lds, const void* base, unsigned off) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
 }
 // LDS traffic of this wave done, then the workgroup barrier; loads from memory stay in flight across it
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
