@@ -12,6 +12,7 @@
 #include <ATen/hip/HIPContext.h>
 #include <c10/core/DeviceGuard.h>
 #include <stdint.h>
+#include <atomic>
 
 #define SXE_CHECK(cond, ...) TORCH_CHECK(cond, "sxe: ", __VA_ARGS__)
 #define SXE_CHECK_CUDA(t) SXE_CHECK((t).is_cuda(), #t " must be a GPU tensor")
@@ -28,6 +29,18 @@ namespace sxe {
 
 constexpr int kWave = 64;
 constexpr int kNumCUs = 256;
+
+// Dynamic LDS beyond the default limit of 64 KB: a kernel is opted in once on every device.
+template <auto KERN>
+inline void allow_lds(int bytes) {
+  static std::atomic<uint64_t> done[4] = {};
+  int dev = 0;
+  SXE_HIP_CHECK(hipGetDevice(&dev));
+  const uint64_t bit = 1ull << (dev & 63);
+  if (dev < 256 && (done[dev >> 6].load(std::memory_order_relaxed) & bit)) return;
+  SXE_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(KERN), hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+  if (dev < 256) done[dev >> 6].fetch_or(bit, std::memory_order_relaxed);
+}
 
 // What a kernel reads or writes beside `t` lies on t's GPU: a pointer into host memory or another GPU's faults in the kernel.
 inline void check_beside(const at::Tensor& t, std::initializer_list<c10::optional<at::Tensor>> others) {

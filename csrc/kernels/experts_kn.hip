@@ -149,14 +149,15 @@ template <bool GATE>
 void launch(const Args& a, hipStream_t stream) {
   const dim3 grid(a.N / COLS, std::min(a.E, a.R), a.splits);
   const size_t lds = sizeof(float) * NW * 16 * LDP;
-  auto go = [&](auto kern) {
-    SXE_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  auto go = [&](auto mb) {
+    constexpr auto kern = &expert_kn_kernel<decltype(mb)::value, GATE>;
+    allow_lds<kern>((int)lds);
     hipLaunchKernelGGL(kern, grid, dim3(64 * NW), lds, stream, a);
   };
   // blocks of 16 rows that share a pass: twice the mean, so that an uneven routing seldom takes a second pass
-  if (a.R <= 8 * a.E) go(expert_kn_kernel<1, GATE>);
-  else if (a.R <= 16 * a.E) go(expert_kn_kernel<2, GATE>);
-  else go(expert_kn_kernel<4, GATE>);
+  if (a.R <= 8 * a.E) go(std::integral_constant<int, 1>{});
+  else if (a.R <= 16 * a.E) go(std::integral_constant<int, 2>{});
+  else go(std::integral_constant<int, 4>{});
   SXE_LAUNCH_CHECK();
 }
 

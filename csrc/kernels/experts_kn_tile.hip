@@ -226,12 +226,7 @@ static void launch(const Args& a) {
   // every expert may end in a part of a tile
   const int64_t grid = ((int64_t)a.R / BM + std::min(a.E, a.R)) * ((a.cols + CB - 1) / CB);
   SXE_CHECK(grid < (1ll << 31), "expert tile product: too many tiles");
-  static const bool lds = [] {
-    SXE_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&tile_kernel<GLU>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      RING * SLOT));
-    return true;
-  }();
-  (void)lds;
+  allow_lds<&tile_kernel<GLU>>(RING * SLOT);
   hipLaunchKernelGGL(tile_kernel<GLU>, dim3((unsigned)grid), dim3(NTHR), RING * SLOT, cur_stream(), a);
   SXE_LAUNCH_CHECK();
 }

@@ -575,15 +575,7 @@ inline Plan plan(int mode, int M, int N, int K, bool fp8) {
   return p;
 }
 
-// LDS of the prologue past the default limit (once a kernel)
-template <auto KERN>
-void allow_lds() {
-  static const bool done = [] {
-    SXE_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(KERN), hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024));
-    return true;
-  }();
-  (void)done;
-}
+constexpr int kProLds = 144 * 1024;  // most that a prologue's M x K input may take
 
 struct Operands {
   const unsigned short* x;
@@ -601,14 +593,14 @@ void launch_as(const Operands& o, const Plan& p, size_t lds, const ProArgs& pro)
   const dim3 grid(p.tiles), block(NW * 64);
   auto bf16 = [&](auto nt) {
     constexpr auto kern = &skinny_gemm_kernel<NW, MODE, decltype(nt)::value, CW>;
-    if (lds) allow_lds<kern>();
+    if (lds) allow_lds<kern>(kProLds);
     hipLaunchKernelGGL(kern, grid, block, lds, cur_stream(), o.x, o.ldx, reinterpret_cast<const unsigned short*>(o.w->data_ptr()),
                        o.w->stride(0), o.bias, yp, o.y->stride(0), o.M, o.N, o.K, p.spw, pro);
   };
   if (o.wscale != nullptr) {
     if constexpr (MODE <= PRO_MERGE) {
       constexpr auto kern = &skinny_gemm_fp8w_kernel<NW, MODE, CW>;
-      if (lds) allow_lds<kern>();
+      if (lds) allow_lds<kern>(kProLds);
       hipLaunchKernelGGL(kern, grid, block, lds, cur_stream(), o.x, o.ldx, reinterpret_cast<const uint8_t*>(o.w->data_ptr()),
                          o.w->stride(0), o.wscale, o.bias, yp, o.y->stride(0), o.M, o.N, o.K, p.spw, pro);
     }
@@ -766,7 +758,7 @@ static std::vector<at::Tensor> skinny_gemm_pro_impl(const at::Tensor& x, const c
   if (N == 0) return {y, h.defined() ? h : x};
   c10::DeviceGuard gd(x.device());
   const size_t lds = (size_t)M * K * 2;
-  SXE_CHECK(lds <= 144 * 1024, "skinny_gemm_pro: M x K input exceeds the LDS budget");
+  SXE_CHECK(lds <= sg::kProLds, "skinny_gemm_pro: M x K input exceeds the LDS budget");
   if (fp8)
     SXE_CHECK(wscale->scalar_type() == at::kFloat && wscale->is_contiguous() && wscale->numel() == N,
               "skinny_gemm_pro: wscale fp32 [N]");
@@ -825,7 +817,7 @@ at::Tensor skinny_gemm_merge(const at::Tensor& part_o, const at::Tensor& part_ml
   if (N == 0) return y;
   c10::DeviceGuard gd(part_o.device());
   const size_t lds = (size_t)M * K * 2;
-  SXE_CHECK(lds <= 144 * 1024, "skinny_gemm_merge: M x K input exceeds the LDS budget");
+  SXE_CHECK(lds <= sg::kProLds, "skinny_gemm_merge: M x K input exceeds the LDS budget");
   if (fp8)
     SXE_CHECK(wscale->scalar_type() == at::kFloat && wscale->is_contiguous() && wscale->numel() == N,
               "skinny_gemm_merge: wscale fp32 [N]");
@@ -842,7 +834,7 @@ static at::Tensor skinny_launch(int mode, const unsigned short* xp, int64_t ldx,
             "skinny gemm: w bf16 [N, K], 16-B rows");
   SXE_CHECK(M >= 1 && M <= sg::kProMaxM, "skinny gemm: 1 <= M <= 4");
   const size_t lds = (size_t)M * K * 2;
-  SXE_CHECK(lds <= 144 * 1024, "skinny gemm: M x K input exceeds the LDS budget");
+  SXE_CHECK(lds <= sg::kProLds, "skinny gemm: M x K input exceeds the LDS budget");
   auto y = at::empty({M, N}, w.options());
   if (N == 0) return y;
   sg::Plan p = sg::plan(mode, M, N, K, false);
