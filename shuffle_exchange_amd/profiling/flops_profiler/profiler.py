@@ -62,6 +62,25 @@ def _register_sxe_formulas():
         def _skinny8(x, wq, *a, out_shape=None, **kw):
             return 2 * x[0] * wq[0] * wq[1]
 
+        @register_flop_formula(ops.stream_gemm)
+        def _stream(x, w, *a, out_shape=None, **kw):
+            return 2 * x[0] * w[0] * w[1]
+
+        def _routed(rows, w):  # every row meets exactly one expert, w [E, K, N]
+            return 2 * rows * w[1] * w[2]
+
+        @register_flop_formula(ops.expert_swiglu_kn)
+        def _expert_up(x, w, offs, active, token, *a, out_shape=None, **kw):
+            return _routed(token[0], w)
+
+        @register_flop_formula(ops.expert_swiglu_kn_tile)
+        def _expert_up_tile(x, w, offs, token, *a, out_shape=None, **kw):
+            return _routed(token[0], w)
+
+        @register_flop_formula([ops.expert_down_kn, ops.expert_down_kn_tile])
+        def _expert_down(h, w, *a, out_shape=None, **kw):
+            return _routed(h[0], w)
+
         @register_flop_formula(ops.grouped_gemm)
         def _grouped(x, w, *a, out_shape=None, **kw):  # every row meets exactly one expert
             return 2 * x[0] * w[1] * w[2]

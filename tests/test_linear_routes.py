@@ -172,3 +172,39 @@ def test_library_switch(monkeypatch):
         x, w, _ = _operands(rows)
         with torch.no_grad():
             assert L.glu_linear(x, w) is None and torch.equal(L.linear(x, w), F.linear(x, w))
+
+
+@gpu
+@pytest.mark.parametrize("rows", [1, 8, 32, 100])
+def test_flops_are_counted(rows):
+    from torch.utils.flop_counter import FlopCounterMode
+
+    from shuffle_exchange_amd.ops.fp_quantizer import FP8Weight
+    from shuffle_exchange_amd.ops.linear import glu_linear, linear
+    from shuffle_exchange_amd.profiling.flops_profiler.profiler import _register_sxe_formulas
+    _register_sxe_formulas()
+    x, w, b = _operands(rows)
+    for weight in (w, FP8Weight(w)) if rows <= 16 else (w,):
+        with torch.no_grad(), FlopCounterMode(display=False) as c:
+            linear(x, weight, b)
+        assert c.get_total_flops() == 2 * rows * 64 * 128
+    if rows <= 32:
+        with torch.no_grad(), FlopCounterMode(display=False) as c:
+            assert glu_linear(x, w) is not None
+        assert c.get_total_flops() == 2 * rows * 64 * 128
+
+
+@gpu
+@pytest.mark.parametrize("tokens", [3, 200])
+def test_flops_of_routed_experts(tokens):
+    from torch.utils.flop_counter import FlopCounterMode
+
+    from shuffle_exchange_amd.ops.moe import route_logits, swiglu_experts
+    from shuffle_exchange_amd.profiling.flops_profiler.profiler import _register_sxe_formulas
+    _register_sxe_formulas()
+    x = torch.randn(tokens, 128, device="cuda").bfloat16()
+    up, down = (torch.randn(4, *s, device="cuda").bfloat16() / 16 for s in ((128, 256), (128, 128)))
+    routing = route_logits(torch.randn(tokens, 4, device="cuda"), 2)
+    with torch.no_grad(), FlopCounterMode(display=False) as c:
+        swiglu_experts(x, routing, up, down)
+    assert c.get_total_flops() == 2 * 2 * tokens * (128 * 256 + 128 * 128)
