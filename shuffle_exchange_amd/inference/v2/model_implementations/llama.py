@@ -246,41 +246,29 @@ class RaggedLlama:
         return self._proj(mod, a, li, key), h
 
     def _norm_glu(self, layer, x, res, li):
-        """(silu(gate) * up of the normed residual sum, the sum) with the activation in the GEMM's epilogue, at decode; (None, None)
-        when not covered."""
-        mlp, T = layer.mlp, x.shape[0]
-        if (self.tps is not None or not 0 < T <= 32 or (T <= self.FUSE_MAX_T and not self._fusable(T)) or self.device.type != "cuda"
-                or getattr(mlp.gate_up_proj, "bias", None) is not None or not native.hip_available()):
-            return None, None
-        w, norm = self._wobj(mlp.gate_up_proj, li, "gu"), layer.post_attention_layernorm
-        if T <= self.FUSE_MAX_T:
-            from ....ops.linear import _pro_weight, fused_rms_glu
-            if _pro_weight(w) is None:
-                return None, None
-            r = fused_rms_glu(x, res, norm.weight, norm.eps, w) if is_own_forward(norm, RMSNorm) else None
+        """(silu(gate) * up of the normed residual sum, the sum); the activation in the GEMM's epilogue at decode, the norm in its
+        prologue up to 4 tokens."""
+        mlp, norm, T = layer.mlp, layer.post_attention_layernorm, x.shape[0]
+        w = None
+        if (self.tps is None and T <= 32 and (T > self.FUSE_MAX_T or self._fusable(T)) and self.device.type == "cuda"
+                and getattr(mlp.gate_up_proj, "bias", None) is None and native.hip_available()):
+            w = self._wobj(mlp.gate_up_proj, li, "gu")
+            if T > 16 and self.qw is not None:  # quantized layers run more than 16 rows on the weight as it came
+                w = self.qw[li]["gu"].weight
+        if w is not None and T <= self.FUSE_MAX_T and is_own_forward(norm, RMSNorm):
+            from ....ops.linear import fused_rms_glu
+            r = fused_rms_glu(x, res, norm.weight, norm.eps, w)
             if r is not None:
                 return r
-        from ....ops.linear import glu_linear
-        if T > 16 and self.qw is not None:  # quantized layers run more than 16 rows on the weight as it came
-            w = self.qw[li]["gu"].weight
         a, h = norm(x, res)
-        mid = glu_linear(a, w)
-        if mid is None:
-            mid = swiglu(self._proj(mlp.gate_up_proj, a, li, "gu"))
-        return mid, h
+        if w is not None:
+            from ....ops.linear import glu_linear
+            mid = glu_linear(a, w)
+            if mid is not None:
+                return mid, h
+        return swiglu(self._proj(mlp.gate_up_proj, a, li, "gu")), h
 
-    def _mlp(self, layer, m, li=0, gu=None):
-        """``gu``: the gate_up projection when the caller already ran it (fused with the norm)."""
-        if hasattr(layer, "mlp"):
-            mlp = layer.mlp
-            if gu is None:
-                gu = self._proj(mlp.gate_up_proj, m, li, "gu")
-            if self._fusable(gu.shape[0]) and getattr(mlp.down_proj, "bias", None) is None:
-                from ....ops.linear import fused_swiglu_linear
-                y = fused_swiglu_linear(gu, self._wobj(mlp.down_proj, li, "down"))
-                if y is not None:
-                    return y
-            return self._proj(mlp.down_proj, swiglu(gu), li, "down")
+    def _moe(self, layer, m, li):
         moe = layer.block_sparse_moe if hasattr(layer, "block_sparse_moe") else layer.moe
         if self.tps is not None:  # this rank's expert columns -> partial sums -> one all-reduce
             d = self.tps.layers[li]
@@ -364,15 +352,11 @@ class RaggedLlama:
                 rope_kv_cache_append(qkv, rope, batch.positions, kv_layer, batch.slots, self.nq, self.nkv)
                 o = self._attn_o(attn, qkv, kv_layer, batch, li, T)
             if hasattr(layer, "mlp"):
-                mid, h2 = self._norm_glu(layer, o, h, li)
-                if mid is not None:
-                    x, res = self._proj(layer.mlp.down_proj, mid, li, "down"), h2
-                else:
-                    gu, h2 = self._norm_proj(layer.post_attention_layernorm, o, h, layer.mlp.gate_up_proj, li, "gu")
-                    x, res = self._mlp(layer, None, li, gu=gu), h2
+                mid, res = self._norm_glu(layer, o, h, li)
+                x = self._proj(layer.mlp.down_proj, mid, li, "down")
             else:
-                m, h2 = layer.post_attention_layernorm(o, h)
-                x, res = self._mlp(layer, m, li), h2
+                m, res = layer.post_attention_layernorm(o, h)
+                x = self._moe(layer, m, li)
         last = batch.last_idx
         x = gather_last(x, last, res)
         if self._fusable(x.shape[0]) and is_own_forward(model.norm, RMSNorm):
