@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Training benchmarks on N MI355X GPUs (one process per GPU, RCCL over xGMI), one per BASELINE.json config.
+"""Training benchmarks on N MI355X GPUs (one process per GPU, RCCL over xGMI), one per benchmark configuration.
 
 Contract (driver): ``python bench.py --gpus N --steps K --warmup W``; for N > 1 launched by
 ``torch.distributed.run`` (RANK/LOCAL_RANK/WORLD_SIZE/MASTER_* from env). W untimed steps, then
@@ -12,7 +12,7 @@ architecture (no network access for checkpoints/datasets).
 ``--config`` (default ``llama8b-z3``, the headline):
   llama8b-z3          Llama-3-8B, ZeRO-3, bf16, seq 2048, 16 sequences per GPU (8 x 2 micro-steps),
                       MI355X-tuned residency (288 GB HBM: gathered weights kept for the step,
-                      gradient sums reduce-scattered once per step) -- BASELINE.json metric
+                      gradient sums reduce-scattered once per step) -- the headline metric
   llama8b-z3-default  the same model/batch with the REFERENCE's default ZeRO-3 knobs (a gather per
                       micro-step forward, backward re-gathers beyond reuse distance 1e9 / max_live
                       1e9, a reduce-scatter every micro-step, prefetch bucket 5e7)

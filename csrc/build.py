@@ -6,7 +6,7 @@ Outputs (in-tree, next to the Python loaders so they travel with the repo):
   shuffle_exchange_amd/ops/_sxe_cpu.so   host kernels: CPU Adam/Lion/Adagrad (AVX-512/AVX2
                                          runtime dispatch + OpenMP) and the async-IO engine
 
-There is no JIT op_builder (the reference's `op_builder/*` is a per-op JIT; see SURVEY §0):
+There is no JIT op_builder (the reference's `op_builder/*` is a per-op JIT):
 every extension is compiled once with hipcc / g++ and loaded with torch.ops.load_library.
 Incremental: an object is rebuilt only if its source or any header under csrc/include changed.
 

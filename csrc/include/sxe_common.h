@@ -1,8 +1,8 @@
 // Shared device helpers for the gfx950 (CDNA4) kernels of shuffle_exchange_amd.
 //
-// Conventions (MI355X-first, see /opt/skills/guides/cdna_hip_programming.md):
+// Conventions:
 //  * wave = 64 lanes, always; reductions use 64-wide butterflies (__shfl_xor up to 32).
-//  * every memory-bound kernel moves 16 bytes per lane per access (Guideline 13): bf16 as
+//  * every memory-bound kernel moves 16 bytes per lane per access: bf16 as
 //    8-element vectors, fp32 as float4.
 //  * bf16 <-> f32 conversion: widening is a shift; narrowing is a plain cast to __bf16, which
 //    hipcc lowers to v_cvt_pk_bf16_f32 (round-to-nearest-even, NaN preserving).
@@ -152,7 +152,7 @@ inline DT dtype_of(const at::Tensor& t) {
   }
 }
 
-// Memory-bound grid sizing (Guideline 11): enough blocks to fill 256 CUs x 8, grid-stride rest.
+// Memory-bound grid sizing: enough blocks to fill 256 CUs x 8, grid-stride rest.
 inline int stream_grid(int64_t work_items, int block) {
   int64_t g = (work_items + block - 1) / block;
   if (g > (int64_t)kNumCUs * 8) g = (int64_t)kNumCUs * 8;

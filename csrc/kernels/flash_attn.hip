@@ -9,17 +9,17 @@
 // (ops/transformer/inference/triton/attention.py:263, triton_ops.py:16) and the external
 // flash-attn the FastGen blocked_flash op calls (inference/v2/kernels/ragged_ops/blocked_flash/).
 //
-// CDNA4 design (see /opt/skills/guides/cdna_hip_programming.md §3, §5.5 T2/T10/T12-T14, App. B):
+// CDNA4 design:
 //  * v_mfma_f32_32x32x16_bf16 everywhere; 64-wide waves; one wave owns 32 query rows (fwd, dQ)
 //    or 32 key rows (dK/dV);
 //  * "swapped" products: the forward computes S^T = K Q^T so one lane holds one query's scores
 //    (softmax max/sum are lane-local + one lane^32 exchange, the rescale is a per-lane scalar),
-//    and S^T is consumed directly as the B operand of O^T += V^T P^T (the accumulator-as-operand
-//    identity of guide §3, with its permuted k order), so P never touches LDS;
+//    and S^T is consumed directly as the B operand of O^T += V^T P^T (an accumulator is an operand
+//    whose k order is permuted), so P never touches LDS;
 //  * V^T / K^T / Q^T / dO^T operands come from row-major LDS tiles through ds_read_b64_tr_b16
 //    (hardware transpose), with the XOR-swizzled 256-byte-row image that is conflict-free for
-//    both the row reads (ds_read_b128) and the transposed reads (guide T10, image (b));
-//  * K/V (or Q/dO) tiles are register-staged one tile ahead (T14 issue-early/write-late) into a
+//    both the row reads (ds_read_b128) and the transposed reads;
+//  * K/V (or Q/dO) tiles are register-staged one tile ahead (loads issued early, written late) into a
 //    double-buffered LDS ring: one barrier per tile;
 //  * backward = pre-pass (-delta = -rowsum(dO * O), lse * log2(e)) + dQ kernel (forward-shaped) +
 //    dK/dV kernel (keys on lanes, dK^T/dV^T accumulated in registers across the GQA query heads): no
@@ -48,7 +48,7 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 // Byte offset of 16-byte chunk `ch` (0..D/8-1) of row `row` in a swizzled [rows][D bf16] tile: the
 // chunk index is XORed with a 4-bit function of the row (3 bits when a row has only 8 chunks) so
 // both the row reads (ds_read_b128) and the transposed 4-row reads (ds_read_b64_tr_b16) spread over
-// the banks (guide T10, image (b)); the XOR is an involution, which the direct-to-LDS loader uses.
+// the banks; the XOR is an involution, which the direct-to-LDS loader uses.
 template <int D>
 __device__ __forceinline__ int soff(int row, int ch) {
   constexpr int CH = D / 8;

@@ -12,7 +12,7 @@
 //      the random-LTD scatter back into the full sequence (gather_scatter.cu:72) and the backward of
 //      a unique-index gather.
 //
-// One wave per row and 16 bytes per lane per access (Guideline 13): a 4 KiB bf16 row (H = 2048)
+// One wave per row and 16 bytes per lane per access: a 4 KiB bf16 row (H = 2048)
 // is 4 wave-instructions of 1 KiB, each fully coalesced. Rows are opaque bytes, so every dtype
 // uses the same code; only ``add`` (an elementwise sum) needs the type.
 #include "sxe_common.h"

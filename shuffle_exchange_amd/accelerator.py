@@ -1,7 +1,7 @@
 """Platform layer: one concrete MI355X (ROCm/HIP) device object.
 
 The reference routes every device call through ``get_accelerator()`` (a ~60-method multi-vendor
-abstraction whose source is missing from the snapshot, SURVEY §2.10). This framework targets one
+abstraction whose source is missing from the snapshot). This framework targets one
 platform, so this module is a thin, direct wrapper over ``torch.cuda`` (HIP on ROCm) plus the
 pieces the runtime needs: named stream pools, pinned host buffers, graphs, roctx ranges. The only
 other mode is a host-CPU mode used by the gloo plumbing tests (no dispatch tables, no op builders).

@@ -5,13 +5,13 @@ logger via ``timed_op`` :102-135) and deepspeed/comm/torch.py (``TorchBackend`` 
 ``DS_COMM_*_OFF`` debug toggles :16-88). Differences that matter on MI355X:
 
 * ``isend``/``irecv`` are truly asynchronous (the reference facade calls the blocking send/recv,
-  comm/comm.py:380-389 -- a known quirk, SURVEY §2.7).
+  comm/comm.py:380-389 -- a known quirk).
 * a **group cache** keyed by the member-rank tuple: RCCL communicator creation costs ~100 ms,
   so the Shuffle-exchange reshuffle (reference stage_1_and_2.py:698-711 destroys and recreates
   every communicator) reuses groups it has seen before.
 * a **collective fingerprint**: every collective folds (op, group, numel, dtype) into a per-rank
   running hash; ``verify_fingerprints()`` all-gathers the hashes and raises on divergence. This is
-  the race/ordering detector SURVEY §5.2 asks for (it catches e.g. ranks whose shuffle RNG
+  the race/ordering detector (it catches e.g. ranks whose shuffle RNG
   diverged, which deadlocks or silently mis-averages in the reference).
 * a comms logger reporting per-op latency, algbw and busbw (busbw uses the ring factors of each
   collective, so it is directly comparable to the per-link xGMI bandwidth), and always-on per-op

@@ -1,8 +1,8 @@
 """Environment / native-op report (parity: reference env_report.py, ``ds_report``).
 
 Lists the torch / ROCm / RCCL stack, the visible MI355X devices and, for every native extension,
-whether it is built in-tree and loads, plus the ops it registers. There is no JIT op builder
-(SURVEY §0): the "compatible / installed" columns of the reference collapse into built + loaded.
+whether it is built in-tree and loads, plus the ops it registers. There is no JIT op builder:
+the "compatible / installed" columns of the reference collapse into built + loaded.
 """
 import os
 import shutil

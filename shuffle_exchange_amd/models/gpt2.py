@@ -1,6 +1,6 @@
 """GPT-2 (learned positions, LayerNorm, GELU MLP, tied LM head) on this repo's ops.
 
-Used by the plumbing configuration of BASELINE.json ("GPT-2 small ZeRO-1 on CPU/gloo world_size=2")
+Used by the plumbing configuration (GPT-2 small, ZeRO-1 on the CPU over gloo, two ranks)
 and as the LayerNorm/GELU/bias path of the kernel set. Presets: gpt2 (124M), gpt2-medium, gpt2-large,
 gpt2-tiny (tests).
 """

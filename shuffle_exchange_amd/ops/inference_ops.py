@@ -1,5 +1,5 @@
 """Functional inference-v1 ops (reference ops/transformer/inference/op_binding/*.py, whose
-``InferenceBuilder`` native module is not in the snapshot -- SURVEY 2.5).
+``InferenceBuilder`` native module is not in the snapshot).
 
 The reference wraps each CUDA entry point in an ``*Op`` class configured by
 ``DeepSpeedInferenceConfig``; here every op is a plain function on this framework's gfx950 kernels

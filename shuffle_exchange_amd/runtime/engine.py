@@ -11,8 +11,7 @@ What happens where on MI355X:
 * timers are HIP events (no sync until read); tokens/s and TFLOPs are reported (the reference only
   reports samples/s);
 * the Shuffle-exchange hooks (``shuffle_exchange()``, ``synchronization()``, ``reset_rings()``) are
-  exposed on the engine and can be driven automatically from config (the reference never calls them,
-  SURVEY §0.1).
+  exposed on the engine and can be driven automatically from config (the reference never calls them).
 """
 import os
 import time

@@ -2,7 +2,7 @@
 :93 DynamicLossScaler, :211 CreateLossScaler).
 
 Checkpoints store ``state_dict()`` (plain numbers) instead of the pickled scaler object the
-reference writes (SURVEY §5.4), so they load with ``torch.load(weights_only=True)``.
+reference writes, so they load with ``torch.load(weights_only=True)``.
 """
 import torch
 

@@ -1,6 +1,6 @@
 """Shuffle-exchange: hierarchical ZeRO with inter-slice parameter averaging (the fork's feature).
 
-Semantics (reference runtime/zero/stage_1_and_2.py:163-241, 692-734, 2092-2250; SURVEY §0.1):
+Semantics (reference runtime/zero/stage_1_and_2.py:163-241, 692-734, 2092-2250):
 the ZeRO data-parallel group of W ranks is cut into W/S *slices* of S consecutive ranks. ZeRO
 partitioning, gradient reduce-scatter, grad-norm and the parameter all-gather all happen INSIDE a
 slice. After each optimizer step the bit16 chunk a rank owns is synchronised with the ranks that

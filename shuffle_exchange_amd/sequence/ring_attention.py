@@ -1,6 +1,6 @@
 """Ring attention (context parallelism) over the sequence-parallel group.
 
-SURVEY §2.6 lists ring attention / context parallelism as absent from the reference (its long
+Ring attention / context parallelism is absent from the reference (its long
 context goes through Ulysses all-to-all, FPDT chunking and tiling) and as an optional new feature
 for the xGMI full mesh. This is that feature: every rank keeps its [B, S/p, H, D] chunk of the
 queries and passes the packed [k | v] chunk around the ring with point-to-point sends to the next

@@ -1,4 +1,4 @@
-"""Fault injection for failure-handling tests (SURVEY §5.3; the reference has none).
+"""Fault injection for failure-handling tests (the reference has none).
 
 ``SXE_FAULT`` holds ``;``-separated rules ``<action>@<rank>:<step>``:
   * ``kill@1:3``  -- rank 1 exits with status 17 when the engine reaches global step 3

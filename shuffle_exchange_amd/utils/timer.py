@@ -1,5 +1,5 @@
 """Timers (parity: reference deepspeed/utils/timer.py:44 SynchronizedWallClockTimer, :199
-ThroughputTimer). Adds what the reference lacks (SURVEY §5.5): tokens/s and model TFLOPs/GPU."""
+ThroughputTimer). Adds what the reference lacks: tokens/s and model TFLOPs/GPU."""
 import time
 
 import torch

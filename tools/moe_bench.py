@@ -1,4 +1,4 @@
-"""Mixtral-8x7B training throughput on MI355X (BASELINE.json config "Mixtral 8x7B MoE"): the full
+"""Mixtral-8x7B training throughput on MI355X (Mixtral 8x7B MoE): the full
 architecture (hidden 4096, 8 experts x FFN 14336, top-2, GQA 32/8, vocab 32000) cut to L decoder
 layers so one GPU holds it, ZeRO-3 bf16 AdamW, seq 2048. Reports tokens/s and TFLOP/s counted on
 the ACTIVE parameters (2 of 8 experts per token) plus attention. With one GPU the expert-parallel

@@ -1,4 +1,4 @@
-"""Peak trainable parameters per GPU (the second half of BASELINE.json's headline metric).
+"""Peak trainable parameters per GPU (the second half of the headline metric).
 
 Trains the Llama-3-70B architecture (hidden 8192, 64/8 heads, FFN 28672, vocab 128256) cut to L
 decoder layers -- params = 0.856 B x L + 2.1 B -- with ZeRO-3 bf16 + AdamW (fp32 masters) and
