@@ -10,7 +10,7 @@
 //  * swapped products (S^T = K Q^T: one lane = one query's scores, lane-local softmax) on v_mfma_f32_32x32x16_bf16, the
 //    score accumulator reused as the B operand of O^T += V^T P^T; 128 queries (or keys) a workgroup, K / V (Q / dO) tiles
 //    of 64 rows direct to LDS in rows of D elements, two slots;
-//  * the pair bias is brought into the accumulator's order once a call (pack_pair: 2 x [H, L, L]), in the type it came in:
+//  * the pair bias is brought into the accumulator's order once a call (pack_kernel: 2 x [H, L, L]), in the type it came in:
 //    a lane then reads its 16 scores' biases as 16-byte vectors (lane = query for the forward and dQ, lane = key for
 //    dK / dV and dbias2) one tile ahead. Read in place they are 16 loads of one value, each over 32 rows of the matrix;
 //  * the row mask is packed to fp32 in the log2 domain with -inf behind the last key, which is all the tail masking there

@@ -14,6 +14,8 @@
 //  * K / V tiles go straight from the cache blocks to LDS, two slots, the next tile's load in flight behind this
 //    tile's products; its block id is read a tile ahead;
 //  * few tiles over long histories (one chunk behind 4k tokens) are split along the keys, fp32 partials, one merge.
+// The longest prompts run the training forward instead, 1.0 - 1.05 PFLOP/s where this reaches 0.9 - 0.95: the rule and its figures
+// are in ops/paged_attention.py.
 // Llama-8B heads (32 / 8, D 128), MI355X, a layer: a 3500-token prompt in chunks of 1024 beside 16 decodes took 2170 us a
 // chunk in the 16-row decode kernel (one read of the keys for every 4 tokens), 50 us here and 30 us for the decodes; 12
 // fresh prompts of 20 - 3000 tokens took 630 us in one flash-attention launch a prompt with its padding copies, 172 us here.

@@ -9,14 +9,14 @@ while the HBM time of the step is ~2 ms. The reference captures CUDA graphs only
 * graphs are keyed by (sequence bucket, KV-length bucket), both powers of two, captured lazily on
   first use and sharing one memory pool;
 * all per-step metadata (token ids, positions, cache slots, block tables, lengths) lives in static
-  device buffers refreshed by one pinned H2D copy per dtype before ``replay()``;
+  device buffers refreshed by one pinned H2D copy before ``replay()``;
 * padding sequences point at a reserved scratch KV block and state slot (q_len = kv_len = 1), so every
   row the graph computes is well defined and no real cache slot is touched;
-* the paged-attention grid is fixed per graph by the KV bucket (splits of >= 256 keys, workgroups
-  past a sequence's length exit at once).
+* the paged-attention grid is fixed per graph by the KV bucket (splits of at most 512 keys while their partials
+  are small, ops/paged_attention.choose_balanced_splits; workgroups past a sequence's length exit at once).
 
-MoE models whose expert counts go through the host and sliding windows narrower than the KV bucket run
-eagerly.
+MoE models whose expert counts go through the host, sliding windows narrower than the KV bucket and modules whose
+weights are made anew for every generation (hybrid engine) run eagerly.
 """
 import numpy as np
 import torch

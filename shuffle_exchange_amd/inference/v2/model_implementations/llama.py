@@ -5,11 +5,13 @@ Parity: reference inference/v2/model_implementations/llama_v2/model.py and mixtr
 choices the reference makes through its registry (blocked KV rotary, blocked flash, pre-RMS norm,
 BLAS linear, cutlass MoE GEMM) replaced by this framework's gfx950 kernels:
 
-  * RMSNorm with fused residual add (norm.hip), projections through hipBLASLt,
+  * RMSNorm with fused residual add (norm.hip), projections through hipBLASLt and, for few rows, the
+    decode kernels (skinny_gemm.hip, stream_gemm.hip),
   * RoPE in place on the packed QKV (rope.hip), KV scatter into the blocked cache and paged
     attention (paged_attn.hip; sequences with many new tokens, with or without earlier ones, in one
-    launch of the tile kernel, paged_prefill.hip),
-  * SwiGLU (act.hip); Mixtral experts via the grouped MoE path of moe/,
+    launch of the tile kernel, paged_prefill.hip; the longest prompts, flash_attn.hip),
+  * SwiGLU (act.hip, or in the epilogue of the decode kernels); Mixtral experts routed on the device
+    (experts_kn.hip, experts_kn_tile.hip),
   * only the last token of every sequence goes through the final norm + LM head.
 The weights are the training modules' own parameters (no copy): a trained LlamaForCausalLM /
 MixtralForCausalLM serves directly.

@@ -60,8 +60,8 @@ def _hip(cfg):
 @register("linear", "quantized_weight_only", priority=10)
 class QuantizedWeightLinear:
     """fp8 (W8A16), fp6 (FP6-LLM wf6af16) or fp4 weight-only: decode-sized inputs (<= 16 rows)
-    stream the quantized weight through the skinny MFMA kernels; larger inputs keep the bf16
-    weight on hipBLASLt (the weight is kept for them)."""
+    stream the quantized weight through the decode kernels (skinny_gemm.hip, stream_gemm.hip, mxfp.hip); larger inputs keep
+    the weight as it came (it is kept for them)."""
 
     @staticmethod
     def supports(cfg):
@@ -81,7 +81,7 @@ class QuantizedWeightLinear:
 
 @register("linear", "blas_fp_linear", priority=0)
 class BlasLinear:
-    """bf16 / fp16 / fp32: ops.linear (skinny MFMA kernel for <= 16 rows, hipBLASLt otherwise)."""
+    """bf16 / fp16 / fp32: ops.linear (hand-written kernels for few bf16 rows, hipBLASLt otherwise)."""
 
     @staticmethod
     def supports(cfg):
@@ -99,9 +99,8 @@ class BlasLinear:
 @register("attention", "dense_blocked_attention_flash_prefill", priority=10)
 class PagedAttentionFlashPrefill:
     """Paged decode kernel (paged_attn.hip) for sequences with few new tokens; prompts and chunks of
-    prompts take the tile kernel over the same cache (paged_prefill.hip)."""
-    flash_prefill = True
-    flash_min_tokens = 256
+    prompts take the tile kernel over the same cache (paged_prefill.hip), the longest prompts the training
+    forward (flash_attn.hip): ops/paged_attention.ragged_attention."""
 
     @staticmethod
     def supports(cfg):
@@ -113,11 +112,9 @@ class PagedAttentionFlashPrefill:
 
 @register("attention", "dense_blocked_attention", priority=0)
 class PagedAttention:
-    """Paged attention, also what the heuristics give other head dims (their prompts take the tile
-    kernel, too); pinned by name, the decode kernel runs every token (HIP kernel for head dims 64 / 128 / 256 with optional
-    sliding window; the PyTorch gather path elsewhere -- ops/paged_attention.py)."""
-    flash_prefill = False
-    flash_min_tokens = 1 << 30
+    """What the heuristics give other head dims: the same routes where the kernels cover them (head dims 64 and 256: decode and tile
+    kernel), the PyTorch gather path elsewhere (ops/paged_attention.py). Pinned by name, the decode kernel runs every token;
+    the ragged model looks at the pin, the object itself has no say."""
 
     @staticmethod
     def supports(cfg):
@@ -130,7 +127,8 @@ class PagedAttention:
 # ----------------------------------------------------------------------------------------- moe
 @register("moe", "hip_topk_grouped", priority=10)
 class HipTopKMoE:
-    """Fused softmax + top-k gating kernel (moe.hip), tokens grouped by expert, per-expert GEMMs."""
+    """Routing on the device (experts.hip) and all experts' products in one launch each (experts_kn.hip, experts_kn_tile.hip); sizes
+    these do not cover: fused softmax + top-k gating kernel (moe.hip), tokens grouped by expert, a GEMM per expert."""
     use_hip_gating = True
 
     @staticmethod

@@ -7,8 +7,8 @@ Parity: reference inference/v2/ragged/ -- ``BlockedAllocator`` (blocked_allocato
 
 MI355X-first sizing: the KV cache is one allocation per model ([layers, blocks, 2, nkv, bs, D]),
 sized from a fraction of the free HBM (288 GB per GPU => hundreds of thousands of tokens of
-Llama-3-8B KV at bf16); the batch metadata is built in pinned host buffers and crosses to the GPU
-in one copy per dtype.
+Llama-3-8B KV at bf16); the batch metadata is built in one pinned host buffer and crosses to the GPU
+in one copy.
 """
 import math
 from dataclasses import dataclass, field

@@ -223,8 +223,8 @@ def matmul_fp8(inp, weight, scale, quantization_group_size):
 
 class FP8Weight:
     """Row-scaled FP8 (e4m3) weight of a linear layer, [N, K] -> used through ``ops.linear.linear``:
-    decode-sized inputs (<= 16 rows) stream the FP8 bytes through the skinny MFMA kernel
-    (skinny_gemm.hip, W8A16: weights converted to bf16 in registers, half the HBM bytes of bf16);
+    decode-sized inputs (<= 16 rows) stream the FP8 bytes through the decode kernels
+    (skinny_gemm.hip up to 4 rows, stream_gemm.hip; W8A16: weights converted to bf16 in registers, half the HBM bytes of bf16);
     larger inputs run ``fp8_linear`` on the FP8 matrix cores (activations quantized per row)."""
 
     def __init__(self, w):

@@ -33,8 +33,8 @@ TN_FP32_OUT = os.environ.get("SXE_WGRAD_TN_FP32OUT", "1") == "1"
 # Decode-shaped products (<= 4 rows, no autograd) stream the weight through the MFMA skinny-GEMM
 # kernel (csrc/kernels/skinny_gemm.hip) instead of hipBLASLt's general tiles. Measured on MI355X
 # (tools/skinny_bench.py, profiles/skinny_bench.log), Llama-3-8B shapes, M = 1: o_proj 7.3 vs
-# 11.8 us, gate_up 42 vs 56 us, down 24.8 vs 25.7 us, LM head 169 vs 180 us, QKV 12.4 vs 10.6 us;
-# at M = 8-16 hipBLASLt is as fast or faster (the kernel supports M <= 16).
+# 11.8 us, gate_up 42 vs 56 us, down 24.8 vs 25.7 us, LM head 169 vs 180 us, QKV 12.4 vs 10.6 us. From 5 rows on
+# stream_gemm.hip is the faster kernel (below); this one supports M <= 16.
 SKINNY_MAX_M = int(os.environ.get("SXE_SKINNY_MAX_M", 4))
 
 
