@@ -6,8 +6,9 @@ sizes: Llama-3-8B issues ~10 kernels per layer (norm, QKV GEMM, RoPE, KV append,
 while the HBM time of the step is ~2 ms. The reference captures CUDA graphs only in its v1 engine
 (inference/engine.py ``_create_cuda_graph``); here the v2 engine captures its decode steps:
 
-* graphs are keyed by (sequence bucket, KV-length bucket), both powers of two, captured lazily on
-  first use and sharing one memory pool;
+* graphs are keyed by (sequence bucket, KV-length bucket), both powers of two, and where the attention kernel splits the
+  keys otherwise for them, by whether the sequences are about as long as one another; captured lazily on first use and
+  sharing one memory pool;
 * all per-step metadata (token ids, positions, cache slots, block tables, lengths) lives in static
   device buffers refreshed by one pinned H2D copy before ``replay()``;
 * padding sequences point at a reserved scratch KV block and state slot (q_len = kv_len = 1), so every
@@ -20,6 +21,8 @@ weights are made anew for every generation (hybrid engine) run eagerly.
 """
 import numpy as np
 import torch
+
+from ...ops.paged_attention import choose_balanced_splits, even_lengths
 
 MIN_KV_BUCKET = 256
 
@@ -34,10 +37,11 @@ def _pow2_at_least(n, lo=1):
 class _StaticBatch:
     """RaggedBatch protocol (see ragged.py) over fixed-shape device buffers."""
 
-    def __init__(self, S, max_blocks, kv_bucket, device):
+    def __init__(self, S, max_blocks, kv_bucket, device, even=False):
         self.num_tokens = self.num_seqs = S
         self.max_blocks = max_blocks
         self.max_kv_len = kv_bucket
+        self.even_lengths = even
         n64, n32 = 32 * S, 16 * S + 4 * S * max_blocks  # bytes: one copy brings both
         self.dev = torch.zeros(n64 + n32, dtype=torch.uint8, device=device)
         self.host = torch.zeros(n64 + n32, dtype=torch.uint8, pin_memory=True)
@@ -73,6 +77,7 @@ class DecodeGraphRunner:
                 if t is not None:
                     t[self.scratch_state].zero_()
         self._graphs = {}
+        self._matters = {}
         self._pool = None
         self.replays = 0
 
@@ -91,15 +96,25 @@ class DecodeGraphRunner:
     def _kv_bucket(self, kv_max):
         return max(_pow2_at_least(kv_max, MIN_KV_BUCKET), self.bs)
 
+    def _even(self, S, kvb, seqs):
+        """The sequences are about as long as one another, and attention splits their keys otherwise then."""
+        matters = self._matters.get((S, kvb))
+        if matters is None:
+            nq, nkv, dim = (getattr(self.model, name, None) for name in ("nq", "nkv", "head_dim"))
+            splits = [choose_balanced_splits(S, nkv, kvb, 4 * S * nq * dim, even) for even in (True, False)] if nq and nkv and dim else (1, 1)
+            matters = self._matters[S, kvb] = splits[0] != splits[1]
+        return matters and even_lengths([s.seen_tokens + 1 for s in seqs])
+
     # ------------------------------------------------------------------------------------- run
     def run(self, seqs, tokens):
         S_real = len(seqs)
         S = _pow2_at_least(S_real)
         kvb = self._kv_bucket(max(s.seen_tokens + 1 for s in seqs))
-        key = (S, kvb)
+        even = self._even(S, kvb, seqs)
+        key = (S, kvb, even)
         entry = self._graphs.get(key)
         sb = entry[1] if entry is not None else _StaticBatch(S, (kvb + self.bs - 1) // self.bs, kvb,
-                                                              self.model.device)
+                                                              self.model.device, even)
         self._fill(sb, seqs, tokens)
         if entry is None:
             entry = self._capture(sb)

@@ -17,6 +17,8 @@ from typing import List, Optional
 import numpy as np
 import torch
 
+from ....ops.paged_attention import even_lengths
+
 
 class BlockedAllocator:
     """Free-list allocator of KV block ids (host side, O(1) alloc/free)."""
@@ -215,13 +217,15 @@ class AttentionLists:
     """int32 device lists of one attention over a ragged batch: ``tiles`` [n, 4] (sequence, first token row, tokens, row among
     the token rows that the tiles hold by sequence; None: none), ``tile_rows`` those rows (first row and count of each sequence until
     ``RaggedBatch.tile_rows`` is asked for them), ``tile_keys`` the longest key range; ``seqs`` [m, 2] (sequence, row among
-    ``seq_rows``), ``seq_rows``, ``seq_keys`` the same for the sequences outside the tiles (None: none)."""
+    ``seq_rows``), ``seq_rows``, ``seq_keys`` the same for the sequences outside the tiles (None: none), ``seq_even`` whether they
+    are about as long as one another."""
     tiles: Optional[torch.Tensor]
     tile_rows: object
     tile_keys: int
     seqs: Optional[torch.Tensor]
     seq_rows: Optional[torch.Tensor]
     seq_keys: int
+    seq_even: bool
 
 
 class RaggedBatch:
@@ -327,6 +331,10 @@ class RaggedBatch:
             self._tables[key] = self._upload(rows, 2)
         return self._tables[key]
 
+    @property
+    def even_lengths(self):
+        return even_lengths(self.host_kv_len)
+
     def attention_lists(self, tile, least, done=(), tails=False):
         """What ops/paged_attention.ragged_attention launches, or None if no sequence has ``least`` new tokens: tiles of
         up to ``tile`` tokens of the sequences that have, longest key range first, and the other sequences. ``done``: (sequence,
@@ -352,7 +360,8 @@ class RaggedBatch:
                 d = self._upload([x for t in tiles for x in t[1:]] + flat + rows, 1).view(-1)  # one copy to the device
                 self._tables[key] = AttentionLists(
                     d[:4 * nt].view(nt, 4) if nt else None, held, tiles[0][0] if nt else 0, d[4 * nt:4 * nt + 2 * ns].view(ns, 2) if ns else None,
-                    d[4 * nt + 2 * ns:] if ns else None, max((self.host_kv_len[i] for i in flat[::2]), default=0))
+                    d[4 * nt + 2 * ns:] if ns else None, max((self.host_kv_len[i] for i in flat[::2]), default=0),
+                    even_lengths([self.host_kv_len[i] for i in flat[::2]]))
             else:
                 self._tables[key] = None
         return self._tables[key]

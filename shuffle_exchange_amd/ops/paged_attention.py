@@ -100,20 +100,41 @@ def choose_splits(num_seqs, nkv, max_kv_len, target_wgs=None):
     return max(1, min(want, math.ceil(max(max_kv_len, 1) / PA_MIN_KEYS)))
 
 
-# Keys of a split at most where the batch has a merge launch anyway. Decode step of 4 Llama-8B layers, us at 1024 / 512 / 256:
-# 24 sequences of 270 - 5300 keys 935 / 920 / 937 (1097 with two splits of 4096), 32 of 3000 keys 1012 / 983 / 1020 (987).
+# Keys of a split at most where sequences differ in length. One layer's attention of a decode step, heads 32 / 8 of 128, us with the
+# splits of choose_splits / of at most 512 keys: sequences of 300 - 4000 keys, 16 of them 35 / 26, 32 61 / 44, 64 111 / 85, 128
+# 167 / 152; but all of 4000 keys 44 / 51, 95 / 102, 177 / 195; all of 2000 - 4000 38 / 40, 77 / 79, 145 / 149; 64 of 1000 42 / 50.
 PA_SPLIT_KEYS = 512
+# Lengths are even where the longest is at most this many times the mean (a log-uniform spread over a factor of 2 has 1.4, of 10 2.6).
+PA_EVEN = 1.5
+# Workgroups that run at once, three a CU. Even sequences finish together, so a last round that is nearly empty costs a whole one:
+# 128 sequences of 4000 keys (1024 workgroups a split) 399 / 372 / 363 us with 1 / 2 / 3 splits, 8000 keys 777 / 722 / 704.
+PA_RESIDENT_WGS = 768
 # Bytes of fp32 partials that such short splits may take: 256 decoding sequences keep splits of 512 keys up to 32k keys (heads of
 # 32 x 128), a call of many tokens has the splits of choose_splits, as its partials grow with tokens x splits.
 PA_SPLIT_BYTES = 1 << 28
 
 
-def choose_balanced_splits(num_seqs, nkv, max_kv_len, split_bytes):
-    """``choose_splits``, and no split over PA_SPLIT_KEYS keys: sequences of a batch differ in length, and a workgroup that
+def even_lengths(lengths):
+    """Whether sequences of these lengths keep a batch's workgroups busy alike."""
+    return len(lengths) * max(lengths, default=0) <= PA_EVEN * sum(lengths)
+
+
+def choose_balanced_splits(num_seqs, nkv, max_kv_len, split_bytes, even=False):
+    """``choose_splits``, and no split over PA_SPLIT_KEYS keys: where sequences of a batch differ in length, a workgroup that
     walks a long one alone outlasts the rest. Splits behind a sequence's end exit at once, the merge does not read them.
+    ``even`` (``even_lengths``): as few splits as fill the chip, in rounds that are mostly full.
     ``split_bytes``: partials of one split (rows x heads x head dim, fp32)."""
-    short = min(math.ceil(max_kv_len / PA_SPLIT_KEYS), PA_SPLIT_BYTES // max(1, split_bytes))
-    return max(choose_splits(num_seqs, nkv, max_kv_len), short)
+    splits, most = choose_splits(num_seqs, nkv, max_kv_len), PA_SPLIT_BYTES // max(1, split_bytes)
+    if not even:
+        return max(splits, min(math.ceil(max_kv_len / PA_SPLIT_KEYS), most))
+
+    def full(s):  # share of the resident workgroups that the rounds keep busy
+        rounds = num_seqs * nkv * s / PA_RESIDENT_WGS
+        return 1 if rounds <= 1 else rounds / math.ceil(rounds)
+    if full(splits) > 0.85:
+        return splits
+    more = [s for s in range(splits, splits + 3) if s == splits or (s <= most and max_kv_len >= s * 320)]
+    return max(more, key=full)
 
 
 def paged_attention_parts(q, cache, block_table, q_start, q_len, kv_len, scale, max_kv_len, splits=None):
@@ -159,16 +180,16 @@ def _split_counters(device, n):
     return c
 
 
-def paged_attention(q, cache, block_table, q_start, q_len, kv_len, scale, max_kv_len, splits=None, window=None):
+def paged_attention(q, cache, block_table, q_start, q_len, kv_len, scale, max_kv_len, splits=None, window=None, even=False):
     """q: [T, nq, D] (head stride D); metadata int32 [S]; returns [T, nq, D]. ``window``: sliding
     window length (keys older than ``window`` positions are masked, Mistral / Qwen2). The HIP kernel
     covers head dims 64 / 128 / 256, with or without a window (the window also skips the key chunks
-    it masks entirely)."""
+    it masks entirely). ``even``: the sequences are about as long as one another (``even_lengths``)."""
     if window is not None and max_kv_len <= window:
         window = None
     if native.use_hip(q) and q.shape[-1] in (64, 128, 256):
         if splits is None:
-            splits = choose_balanced_splits(block_table.shape[0], cache.shape[2], max_kv_len, 4 * q.numel())
+            splits = choose_balanced_splits(block_table.shape[0], cache.shape[2], max_kv_len, 4 * q.numel(), even)
         S = block_table.shape[0]
         cnt = (_split_counters(q.device, S * cache.shape[2])
                if PA_LAST_MERGE and splits > 1 and q.shape[0] <= 4 * S else None)
@@ -208,7 +229,7 @@ def _tileable(q, cache, scale):
 def paged_batch_attention(q, cache, batch, scale, window=None):
     """``paged_attention`` of a whole ragged batch."""
     return paged_attention(q, cache, batch.block_table, batch.q_start, batch.q_len, batch.kv_len, scale, batch.max_kv_len,
-                           window=window)
+                           window=window, even=batch.even_lengths)
 
 
 # The longest prompts take the training forward (csrc/kernels/flash_attn.hip) on the new tokens' own keys up to their last multiple of
@@ -264,7 +285,7 @@ def ragged_attention(q, cache, batch, scale, window=None, kv=None):
             rows = batch.tile_rows(x) if splits > 1 else None
             torch.ops.sxe.paged_prefill(*meta, x.tiles, rows, float(scale), int(window or 0), splits, keys, out)
     if lists is not None and lists.seqs is not None:
-        splits = choose_balanced_splits(lists.seqs.shape[0], nkv, lists.seq_keys, 4 * lists.seq_rows.numel() * q.shape[1] * q.shape[2])
+        splits = choose_balanced_splits(lists.seqs.shape[0], nkv, lists.seq_keys, 4 * lists.seq_rows.numel() * q.shape[1] * q.shape[2], lists.seq_even)
         torch.ops.sxe.paged_attention_some(*meta, lists.seqs, lists.seq_rows, float(scale), int(lists.seq_keys), int(splits),
                                            int(window or 0), out)
     return out

@@ -53,3 +53,26 @@ def test_decode_graphs_match_eager():
         b = ee.put([1, 2], [[5], [6]])
         assert ((a - b).norm() / b.norm()).item() < 2e-2
     assert runner.num_graphs == 3  # + (2, 1024)
+
+
+def test_even_and_uneven_lengths(monkeypatch):
+    """A batch whose lengths become uneven inside one KV bucket replays a graph with other key splits."""
+    from shuffle_exchange_amd.models import LlamaForCausalLM, llama_config
+    from shuffle_exchange_amd.ops import paged_attention as PA
+    monkeypatch.setattr(PA, "PA_TARGET_WGS", 4)  # two sequences of two heads fill the chip
+    torch.manual_seed(0)
+    cfg = llama_config("llama-tiny", hidden_size=512, intermediate_size=1024, num_attention_heads=4, num_key_value_heads=2,
+                       vocab_size=512, num_hidden_layers=2, max_position_embeddings=4096)
+    model = LlamaForCausalLM(cfg).to("cuda", torch.bfloat16).eval()
+    eg, ee = _engine(model, True), _engine(model, False)
+    g = torch.Generator().manual_seed(1)
+    for u, n in ((0, 700), (1, 600), (2, 20)):
+        p = torch.randint(0, 512, (n,), generator=g).tolist()
+        eg.put([u], [p])
+        ee.put([u], [p])
+    for live in ([0, 1], [0, 2], [0, 1], [2, 0]):
+        for _ in range(3):
+            toks = [[int(torch.randint(0, 512, (1,), generator=g))] for _ in live]
+            a, b = eg.put(live, toks), ee.put(live, toks)
+            assert ((a - b).norm() / b.norm()).item() < 2e-2, live
+    assert eg._decode_runner().num_graphs == 2 and eg._decode_runner().replays == 12

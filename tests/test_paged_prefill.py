@@ -165,3 +165,23 @@ def test_long_prompt_rule():
     assert PA._flash_prompts(T(32), T(16), b, None) == ((0, 8192), (3, 8960), (5, 4096))
     assert PA._flash_prompts(T(16), T(8), b, None) == ((0, 8192),) and PA._flash_prompts(T(8), T(4), b, None) == ()
     assert PA._flash_prompts(T(32), T(16), b, 4096) == () == PA._flash_prompts(T(32), None, b, None) == PA._flash_prompts(T(32, 64), T(16), b, None)
+
+
+def test_even_lengths():
+    assert PA.even_lengths([]) and PA.even_lengths([7]) and PA.even_lengths([2000, 4000]) and PA.even_lengths([1000] * 30 + [1400])
+    assert not PA.even_lengths([300, 4000]) and not PA.even_lengths([100] * 30 + [1000])
+    b, _ = _batch([(100, 1), (3000, 1), (5, 60)], 16, "cpu")
+    assert not b.even_lengths and not b.attention_lists(32, 9).seq_even
+    b, _ = _batch([(2500, 1), (3000, 1), (5, 60)], 16, "cpu")
+    assert not b.even_lengths and b.attention_lists(32, 9).seq_even
+
+
+@pytest.mark.parametrize("nkv", [1, 4, 8, 32])
+def test_even_splits(nkv):
+    """Even sequences: the fewest splits that fill the chip, or up to two more where the last round would be nearly empty."""
+    for seqs in (1, 3, 16, 32, 50, 64, 96, 100, 128, 256):
+        for keys in (1, 300, 512, 1024, 4096, 131072):
+            plain, n = PA.choose_splits(seqs, nkv, keys), PA.choose_balanced_splits(seqs, nkv, keys, seqs * 16384, True)
+            assert plain <= n <= plain + 2 and (n == plain or keys >= n * 320) and (n == plain or n * seqs * 16384 <= PA.PA_SPLIT_BYTES)
+            if seqs * nkv * plain <= PA.PA_RESIDENT_WGS:
+                assert n == plain
