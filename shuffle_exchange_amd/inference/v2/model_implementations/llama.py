@@ -31,7 +31,7 @@ import torch.nn.functional as F
 
 from ....ops import native
 from ....ops.activation import swiglu
-from ....ops.linear import Linear, is_own_forward, linear
+from ....ops.linear import Linear, glu_faster, glu_linear, is_own_forward, linear
 from ....ops.norm import RMSNorm
 from ....ops.paged_attention import paged_attention_parts, paged_batch_attention, ragged_attention, rope_kv_cache_append
 from ....ops.rows import gather_last
@@ -263,8 +263,7 @@ class RaggedLlama:
             if r is not None:
                 return r
         a, h = norm(x, res)
-        if w is not None:
-            from ....ops.linear import glu_linear
+        if w is not None and glu_faster(T, w):
             mid = glu_linear(a, w)
             if mid is not None:
                 return mid, h

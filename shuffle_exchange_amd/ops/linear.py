@@ -11,6 +11,7 @@ target it behaves exactly like ``torch.nn.functional.linear``. (The reference's 
 Megatron-style ``gradient_accumulation_fusion``; DeepSpeed's ZeRO copies each ``p.grad`` into an
 IPG bucket instead, stage_1_and_2.py:1137-1139.)
 """
+import math
 import os
 import weakref
 
@@ -57,10 +58,38 @@ def _skinny(x, weight, bias):
     return torch.ops.sxe.skinny_gemm(x2, weight, bias).view(*x.shape[:-1], weight.shape[0])
 
 
-# Batched decode: up to 16 rows, and up to 32 of a small weight, take the weight-streaming kernel (csrc/kernels/stream_gemm.hip).
-# Llama-3-8B shapes, us, hipBLASLt / streaming: 16 rows: QKV 14.2 / 14.8, o 15.5 / 9.7, gate | up 63.0 / 47.4, down 25.6 / 25.0,
-# 32000-row head 58.7 / 50.9; 32 rows: o 13.1 / 12.2, 3072 x 2048 11.1 / 6.9, but QKV 15.1 / 16.5, gate | up 53.6 / 53.4.
-STREAM_ROWS, STREAM_ROWS_SMALL, STREAM_SMALL = 16, 32, 1 << 24
+# Batched decode: up to 32 rows take the weight-streaming kernel (csrc/kernels/stream_gemm.hip) where it is the faster one. A workgroup
+# takes 16 columns, so the last round of them over the CUs decides, and long rows of the weight are where the library is good. us,
+# library / streaming, 16 rows: 3072 x 2048 11.2 / 6.0, 4096 x 4096 14.9 / 9.6, 6144 x 4096 14.0 / 14.6, 28672 x 4096 60 / 47,
+# 4096 x 14336 25.5 / 25.3, 15360 x 5120 33.5 / 34.2, 8192 x 8192 28.5 / 28.9; but 5120 x 5120 15.2 / 17.2, 5120 x 13824 31.9 / 39.1,
+# 10240 x 8192 34.1 / 38.4, 2048 x 8192 12.7 / 13.0, 50264 x 768 18.3 / 20.6. 24 rows: 2048 x 2048 8.4 / 5.9, 4096 x 4096
+# 12.8 / 11.6; but 5120 x 3072 11.6 / 13.5, 6144 x 4096 14.4 / 16.1, 1024 x 8192 11.6 / 15.1, 11264 x 2048 14.6 / 15.7.
+STREAM_ROWS, STREAM_ROWS_SMALL = 16, 32
+
+
+def _full_rounds(workgroups):
+    """Share of the CUs that are busy over the rounds that one workgroup a CU makes."""
+    rounds = workgroups / 256
+    return rounds / max(1, math.ceil(rounds))
+
+
+def _stream_faster(rows, N, K):
+    if rows > STREAM_ROWS:
+        return rows <= STREAM_ROWS_SMALL and K <= 4096 and (N <= 4096 or N * K <= 1 << 23)
+    return not (K >= 5120 and N * K >= 1 << 24 and _full_rounds(N / 16) < 0.9) and not (K < 1024 and N > 16384)
+
+
+def glu_faster(rows, weight):
+    """Whether ``glu_linear`` beats the product and the activation's launch. e4m3: always (8 rows of 28672 x 4096 34 / 26 us with the
+    product of skinny_gemm.hip). bf16, four tiles a workgroup, us, with the library's product / here: 16 rows 16384 x 2048
+    20.7 / 17.4, 28672 x 4096 63 / 46, 36864 x 5120 80 / 76, but 57344 x 8192 170 / 183; 24 rows 10240 x 2560 17.9 / 15.9,
+    16384 x 3072 24.4 / 23.3, 28672 x 4096 59 / 52, but 17920 x 2560 25.9 / 30.6, 27648 x 5120 54 / 63, 7168 x 4096 18.1 / 20.7."""
+    if not isinstance(weight, torch.Tensor):
+        return True
+    N, K = weight.shape
+    if rows > STREAM_ROWS and K <= 3072 and N <= 16384:
+        return True
+    return N * K <= 1 << 28 and (rows <= STREAM_ROWS or _full_rounds(N / 64) > 0.85)
 
 
 def _streamable(x2, weight, bias, unit=8):
@@ -74,7 +103,7 @@ def _stream(x, weight, bias):
     if weight.dtype != torch.bfloat16 or not weight.is_cuda:
         return None
     rows = x.numel() // max(1, x.shape[-1])
-    if not SKINNY_MAX_M < rows <= (STREAM_ROWS if weight.numel() > STREAM_SMALL else STREAM_ROWS_SMALL):
+    if rows <= SKINNY_MAX_M or weight.dim() != 2 or not _stream_faster(rows, *weight.shape):
         return None
     x2 = x.reshape(-1, x.shape[-1])
     if not _streamable(x2, weight, bias):
@@ -85,12 +114,14 @@ def _stream(x, weight, bias):
 
 def glu_linear(x, weight):
     """silu(gate) * up of ``linear(x, weight)`` with weight = [gate | up], in ONE launch (stream_gemm.hip): up to 32 rows (16 of an
-    FP8Weight), no autograd; None when not covered. One rounding, of the result."""
+    FP8Weight), no autograd; None when not covered (``glu_faster``: where it pays). One rounding, of the result."""
     wk = _pro_weight(weight)
     if wk is None or SKINNY_MAX_M <= 0 or not x.is_cuda or x.requires_grad or x.dim() != 2 or not native.plain(x):
         return None
     w, sc = wk
-    if not 0 < x.shape[0] <= (32 if sc is None else 16) or w.shape[0] % 32 or not _streamable(x, w, None, 8 if sc is None else 16):
+    if not 0 < x.shape[0] <= (STREAM_ROWS_SMALL if sc is None else STREAM_ROWS) or w.shape[0] % 32:
+        return None
+    if not _streamable(x, w, None, 8 if sc is None else 16):
         return None
     return torch.ops.sxe.stream_gemm(x, w, sc, None, True)
 

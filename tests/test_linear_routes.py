@@ -208,3 +208,20 @@ def test_flops_of_routed_experts(tokens):
     with torch.no_grad(), FlopCounterMode(display=False) as c:
         swiglu_experts(x, routing, up, down)
     assert c.get_total_flops() == 2 * 2 * tokens * (128 * 256 + 128 * 128)
+
+
+def test_streaming_rule():
+    """Which side of the measured lines a product falls on; no size is refused by the rule itself."""
+    from shuffle_exchange_amd.ops.linear import _stream_faster, glu_faster
+    for N, K in ((3072, 2048), (4096, 4096), (28672, 4096), (4096, 14336), (8, 4096), (2048, 5632), (15360, 5120)):
+        assert _stream_faster(5, N, K) and _stream_faster(16, N, K)
+    for N, K in ((5120, 5120), (5120, 13824), (10240, 8192), (50257, 768)):
+        assert not _stream_faster(5, N, K) and not _stream_faster(16, N, K)
+    for N, K in ((2048, 2048), (4096, 4096), (4100, 1032)):
+        assert _stream_faster(17, N, K) and _stream_faster(32, N, K) and not _stream_faster(33, N, K)
+    for N, K in ((5120, 3072), (6144, 4096), (1024, 8192), (11264, 2048)):
+        assert not _stream_faster(17, N, K)
+    w = lambda N, K: torch.empty(N, K, device="meta")  # noqa: E731
+    assert all(glu_faster(16, w(*s)) and glu_faster(24, w(*s)) for s in ((16384, 2048), (16384, 3072), (28672, 4096), (0, 8)))
+    assert all(glu_faster(16, w(*s)) and not glu_faster(24, w(*s)) for s in ((17920, 2560), (27648, 5120), (7168, 4096)))
+    assert not glu_faster(5, w(57344, 8192)) and glu_faster(16, object())
