@@ -545,10 +545,12 @@ __global__ __launch_bounds__(NW * 64) void skinny_gemm_fp8w_kernel(const unsigne
 
 // Tiles and waves of a launch. Narrow tiles read 128 contiguous bytes of a row a load and give small N twice the workgroups;
 // wide ones build the input half as often and leave every wave a super-step where K is small. One row, us, 16 / 8 columns:
-//   bf16 plain 2048 x 2048 4.9 / 4.0, 2048 x 8192 13.7 / 9.4, 4096 x 4096 10.0 / 9.3, 4096 x 14336 28.5 / 26.6, 32000 x 2048
-//   27.1 / 24.9; RMS 3072 x 2048 6.9 / 6.6, 6144 x 4096 14.7 / 13.5, 32000 x 2048 28.2 / 27.7, with SwiGLU 16384 x 2048
+//   bf16 plain 2048 x 2048 5.0 / 3.9, 2048 x 8192 13.0 / 8.8, 4096 x 4096 9.9 / 8.9, 4096 x 14336 27.1 / 25.3, 32000 x 2048
+//   25.2 / 22.6, but 50264 x 768 16.3 / 19.1; four rows 3072 x 8192 14.7 / 15.9, 2560 x 10240 18.7 / 20.1, 128256 x 4096 177 / 186;
+//   RMS 3072 x 2048 6.9 / 6.6, 6144 x 4096 14.7 / 13.5, 32000 x 2048 28.2 / 27.7, with SwiGLU 16384 x 2048
 //   17.1 / 16.6, 28672 x 4096 45.7 / 42.8
-//   e4m3 plain 2048 x 8192 9.1 / 6.9, 4096 x 4096 7.1 / 6.9, 32000 x 2048 16.9 / 18.9; RMS 3072 x 2048 6.0 / 6.7, 5120 x 3072
+//   e4m3 plain 2048 x 8192 8.9 / 6.1, 4096 x 4096 7.3 / 6.6, but 32000 x 2048 15.5 / 17.3, 3072 x 768 3.5 / 3.8; four rows
+//   4096 x 11008 15.1 / 14.5, 4096 x 14336 16.6 / 17.5; RMS 3072 x 2048 6.0 / 6.7, 5120 x 3072
 //   9.1 / 9.0, 6144 x 4096 12.3 / 10.5, 32000 x 4096 30.6 / 33.4, with SwiGLU 28672 x 4096 28.8 / 30.9
 // SwiGLU's and the merge's prologues are long: 2048 x 8192 14.2 / 10.7, but 3072 x 8192 15.2 / 16.5; merge of 16 splits
 // 2048 x 2048 7.9 / 7.1, 3072 x 3072 12.8 / 14.4 (four waves) and 10.5 (eight waves of wide tiles).
@@ -560,7 +562,11 @@ struct Plan {
 inline Plan plan(int mode, int M, int N, int K, bool fp8) {
   const int wide = (N + 15) / 16, ss = fp8 ? kSS8 : kSS;
   bool narrow = M <= kProMaxM;
-  if (mode == PRO_NONE) narrow = narrow && (!fp8 || wide <= kNumCUs);
+  // bf16: not where a wave would be without a super-step, 4 rows of a very wide weight, or long rows on 1 to 2 tiles a CU;
+  // e4m3: not where N already gives every CU a tile, nor for a short K on many tiles or several rows of a long one
+  if (mode == PRO_NONE && !fp8)
+    narrow = narrow && (K > 6 * kSS || wide <= kNumCUs) && (M < kProMaxM || wide <= 2048) && (K < 8192 || wide <= 128 || wide >= 256);
+  else if (mode == PRO_NONE) narrow = narrow && wide <= kNumCUs && (K >= 1024 || wide < 128) && M * K <= 49152;
   else if (mode == PRO_RMS) narrow = M == 1 && K >= 8 * ss && (!fp8 || 2 * wide <= 3 * kNumCUs);
   else if (mode == PRO_SWIGLU) narrow = narrow && 2 * wide <= kNumCUs;
   else if (mode == PRO_MERGE) narrow = narrow && 2 * wide <= kNumCUs && K <= 2048;
