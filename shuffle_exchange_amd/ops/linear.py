@@ -451,10 +451,21 @@ def _autocast_dtype(x):
     return None
 
 
+def _colsum_faster(x):
+    """Whether csrc/kernels/colsum.hip beats the general reduction, us, general / kernel: bf16 128 x 768 6.4 / 5.3, 2048 x 3072
+    17.0 / 5.4, 2048 x 14336 99 / 12, 16384 x 8192 49 / 46; but 16 x 1048576 5.9 / 79, 8192 x 28672 80 / 93, and where rows do not
+    start on 16 bytes 2048 x 1001 12.9 / 21.8, 2048 x 50257 60 / 133, from 4096 rows on 22 / 16 at 1001, 48 / 23 at 3001 columns."""
+    R, N = x.shape
+    if N % 8 or x.stride(0) * x.element_size() % 16 or x.data_ptr() % 16:
+        return R >= 4096 and 64 <= N <= 8192
+    return R >= 128 and N <= 65536 and (N <= 8192 or R < 8192)
+
+
 def column_sum(x, dtype):
-    """``x.sum(0)`` of [R, N] in ``dtype``, accumulated in fp32 (csrc/kernels/colsum.hip; fp64 and recorded sums: torch)."""
-    if (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16, torch.float32) and x.stride(1) == 1
-            and dtype in (x.dtype, torch.float32) and not (torch.is_grad_enabled() and x.requires_grad) and native.plain(x)):
+    """``x.sum(0)`` of [R, N] in ``dtype``, accumulated in fp32 (csrc/kernels/colsum.hip; fp64, recorded sums and sizes where it is
+    not the faster one: torch)."""
+    if (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16, torch.float32) and x.stride(1) == 1 and dtype in (x.dtype, torch.float32)
+            and not (torch.is_grad_enabled() and x.requires_grad) and native.plain(x) and _colsum_faster(x)):
         native.require_hip()
         return torch.ops.sxe.column_sum(x, dtype)
     return x.sum(0) if dtype == x.dtype else x.float().sum(0).to(dtype)

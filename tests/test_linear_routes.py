@@ -103,10 +103,11 @@ def test_traces(rows):
 @gpu
 def test_column_sum_transforms():
     from shuffle_exchange_amd.ops.linear import column_sum
-    x = torch.randn(3, 40, 72, device="cuda")
+    x = torch.randn(3, 400, 72, device="cuda")
     f = lambda a: column_sum(a, a.dtype)  # noqa: E731
-    torch.testing.assert_close(torch.func.vmap(f)(x), x.sum(1), rtol=1e-5, atol=1e-4)
-    torch.testing.assert_close(torch.func.jvp(f, (x[0],), (x[1],))[1], x[1].sum(0), rtol=1e-5, atol=1e-4)
+    # sums of 400 values in another order: 400 x 2^-24 x the sum of magnitudes (330) at most, a tenth of that allowed here
+    torch.testing.assert_close(torch.func.vmap(f)(x), x.sum(1), rtol=1e-5, atol=1e-3)
+    torch.testing.assert_close(torch.func.jvp(f, (x[0],), (x[1],))[1], x[1].sum(0), rtol=1e-5, atol=1e-3)
 
 
 @gpu
@@ -225,3 +226,18 @@ def test_streaming_rule():
     assert all(glu_faster(16, w(*s)) and glu_faster(24, w(*s)) for s in ((16384, 2048), (16384, 3072), (28672, 4096), (0, 8)))
     assert all(glu_faster(16, w(*s)) and not glu_faster(24, w(*s)) for s in ((17920, 2560), (27648, 5120), (7168, 4096)))
     assert not glu_faster(5, w(57344, 8192)) and glu_faster(16, object())
+
+
+@gpu
+@pytest.mark.parametrize("R,N,kernel", [(127, 768, False), (128, 768, True), (4096, 8192, True), (8192, 8192, True), (8192, 8200, False),
+                                        (8191, 8200, True), (4095, 1001, False), (4096, 1001, True), (4096, 63, False), (128, 65544, False)])
+def test_column_sum_rule(R, N, kernel):
+    from shuffle_exchange_amd.ops import linear as L
+    x = torch.randn(R, N, device="cuda").bfloat16()
+    assert L._colsum_faster(x) == kernel
+    want, size = x.double().sum(0), x.double().abs().sum(0)
+    for dtype in (torch.bfloat16, torch.float32):
+        got = L.column_sum(x, dtype)
+        # fp32 sums of at most R / 128 + 14 steps a column (the general reduction has no more), and the rounding of the result
+        assert got.dtype == dtype and ((got.double() - want).abs() <= (R / 128 + 14) * 2 ** -24 * size
+                                       + (2 ** -8 if dtype == torch.bfloat16 else 0) * want.abs() + 1e-30).all()
