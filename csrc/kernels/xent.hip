@@ -13,13 +13,15 @@
 // 116 / 42, gradient 153 / 86; 256 rows 89 / 20 and 86 / 22.
 #include "sxe_common.h"
 #include <torch/library.h>
+#include <type_traits>
 
 namespace sxe {
 
+constexpr float kFltMax = 3.402823466e38f;
 __device__ __forceinline__ void ms_merge(float& m, float& s, float m2, float s2) {
-  const float mn = fmaxf(m, m2);
-  if (mn == -INFINITY) { m = mn; s = 0.f; return; }
-  s = s * __expf(m - mn) + s2 * __expf(m2 - mn);
+  // against a finite reference: nothing but masked logits so far adds nothing (a branch on it costs 10 % where rows are few)
+  const float mn = fmaxf(m, m2), ref = fmaxf(mn, -kFltMax);
+  s = s * __expf(m - ref) + s2 * __expf(m2 - ref);
   m = mn;
 }
 
@@ -28,9 +30,32 @@ template <typename S>
 __device__ __forceinline__ int row_head(const S* row, int V) {
   return min(V, (int)((0 - reinterpret_cast<uintptr_t>(row) / sizeof(S)) & (16 / sizeof(S) - 1)));
 }
-// f8(first, 8 elements) over the 16-byte aligned body of a row, f1(element) over what lies before and behind it (< 8 each)
-template <typename F8, typename F1>
+// How a row is swept. ELEMENTS: short rows off 16 bytes, or gradients that start otherwise than their logits; WHOLE: every row is
+// whole 16-byte vectors; BODY: what lies before and behind the aligned body (< 8 elements each) by single lanes.
+enum Sweep { ELEMENTS, WHOLE, BODY };
+// 8192 rows, us, loss + gradient by ELEMENTS / BODY: 129 columns 15.7 / 18.0, 385 17.7 / 18.4, 513 18.8 / 18.6, 1001 24.8 / 21.7
+constexpr int kBodyMin = 512;
+inline Sweep sweep_of(const at::Tensor& logits, int V) {
+  if (V % 8 == 0 && reinterpret_cast<uintptr_t>(logits.data_ptr()) % 16 == 0) return WHOLE;
+  return V >= kBodyMin ? BODY : ELEMENTS;
+}
+template <typename F>
+void with_sweep(Sweep sw, F f) {
+  if (sw == WHOLE) f(std::integral_constant<Sweep, WHOLE>{});
+  else if (sw == BODY) f(std::integral_constant<Sweep, BODY>{});
+  else f(std::integral_constant<Sweep, ELEMENTS>{});
+}
+// f8(first of 8 aligned elements), f1(element)
+template <Sweep SW, typename F8, typename F1>
 __device__ __forceinline__ void for_row(int V, int head, F8 f8, F1 f1) {
+  if constexpr (SW == ELEMENTS) {
+    for (int c = threadIdx.x; c < V; c += blockDim.x) f1(c);
+    return;
+  }
+  if constexpr (SW == WHOLE) {
+    for (int c = threadIdx.x * 8; c < V; c += blockDim.x * 8) f8(c);
+    return;
+  }
   const int body = (V - head) & ~7;
   for (int c = head + threadIdx.x * 8; c < head + body; c += blockDim.x * 8) f8(c);
   if ((int)threadIdx.x < head) f1(threadIdx.x);
@@ -38,17 +63,17 @@ __device__ __forceinline__ void for_row(int V, int head, F8 f8, F1 f1) {
   if (c < V) f1(c);
 }
 
-template <DT T>
+template <DT T, Sweep SW>
 __device__ __forceinline__ float row_lse(const typename dt_traits<T>::storage* __restrict__ row, int V, int head, float* red) {
   float m = -INFINITY, s = 0.f;
-  for_row(V, head, [&](int c) {
+  for_row<SW>(V, head, [&](int c) {
     float v[8];
     load8<T>(row + c, v);
     float lm = v[0];
 #pragma unroll
     for (int j = 1; j < 8; ++j) lm = fmaxf(lm, v[j]);
     float ls = 0.f;
-    const float ref = lm == -INFINITY ? 0.f : lm;  // eight masked logits add nothing
+    const float ref = fmaxf(lm, -kFltMax);
 #pragma unroll
     for (int j = 0; j < 8; ++j) ls += __expf(v[j] - ref);
     ms_merge(m, s, lm, ls);
@@ -68,7 +93,7 @@ __device__ __forceinline__ float row_lse(const typename dt_traits<T>::storage* _
 }
 
 // mode: 0 = forward only; 1 = forward + in-place gradient with grad = scale * (softmax - onehot)
-template <DT T>
+template <DT T, Sweep SW>
 __global__ void __launch_bounds__(256) xent_kernel(typename dt_traits<T>::storage* __restrict__ logits, int64_t rows, int V,
                                                    const int64_t* __restrict__ target, int64_t ignore_index,
                                                    float* __restrict__ loss, float* __restrict__ lse_out, int mode,
@@ -79,8 +104,8 @@ __global__ void __launch_bounds__(256) xent_kernel(typename dt_traits<T>::storag
     typename dt_traits<T>::storage* row = logits + r * V;
     const int64_t tgt = target[r];
     const bool ign = (tgt == ignore_index);
-    const int head = row_head(row, V);
-    const float lse = row_lse<T>(row, V, head, red);
+    const int head = SW == BODY ? row_head(row, V) : 0;
+    const float lse = row_lse<T, SW>(row, V, head, red);
     if (threadIdx.x == 0) {
       const float xt = ign ? 0.f : to_f32<T>(row[tgt]);
       loss[r] = ign ? 0.f : (lse - xt);
@@ -89,7 +114,7 @@ __global__ void __launch_bounds__(256) xent_kernel(typename dt_traits<T>::storag
     __syncthreads();  // the target logit is read above before the gradient overwrites it
     if (mode == 1) {
       const float sc = ign ? 0.f : scale;
-      for_row(V, head, [&](int c) {
+      for_row<SW>(V, head, [&](int c) {
         float v[8];
         load8<T>(row + c, v);
 #pragma unroll
@@ -100,8 +125,8 @@ __global__ void __launch_bounds__(256) xent_kernel(typename dt_traits<T>::storag
   }
 }
 
-// grad = dloss[r] * (softmax - onehot), written into grad_out (may alias logits). VEC: both start alike against 16 bytes.
-template <DT T, bool VEC>
+// grad = dloss[r] * (softmax - onehot), written into grad_out (may alias logits).
+template <DT T, Sweep SW>
 __global__ void __launch_bounds__(256) xent_bwd_kernel(const typename dt_traits<T>::storage* __restrict__ logits,
                                                        typename dt_traits<T>::storage* __restrict__ grad, int64_t rows, int V,
                                                        const int64_t* __restrict__ target, int64_t ignore_index,
@@ -113,17 +138,13 @@ __global__ void __launch_bounds__(256) xent_bwd_kernel(const typename dt_traits<
     const typename dt_traits<T>::storage* in = logits + r * V;
     typename dt_traits<T>::storage* out = grad + r * V;
     auto one = [&](int c) { out[c] = from_f32<T>(sc * (__expf(to_f32<T>(in[c]) - l) - (c == tgt ? 1.f : 0.f))); };
-    if constexpr (VEC) {
-      for_row(V, row_head(in, V), [&](int c) {
-        float v[8];
-        load8<T>(in + c, v);
+    for_row<SW>(V, SW == BODY ? row_head(in, V) : 0, [&](int c) {
+      float v[8];
+      load8<T>(in + c, v);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = sc * (__expf(v[j] - l) - ((c + j) == tgt ? 1.f : 0.f));
-        store8<T>(out + c, v);
-      }, one);
-    } else {
-      for (int c = threadIdx.x; c < V; c += blockDim.x) one(c);
-    }
+      for (int j = 0; j < 8; ++j) v[j] = sc * (__expf(v[j] - l) - ((c + j) == tgt ? 1.f : 0.f));
+      store8<T>(out + c, v);
+    }, one);
   }
 }
 
@@ -240,12 +261,12 @@ std::tuple<at::Tensor, at::Tensor> xent_fwd(at::Tensor logits, at::Tensor target
   }
   const int grid = (int)std::min<int64_t>(rows, 8192);
   DT d = dtype_of(logits);
-  SXE_DISPATCH_DT(d, TT, {
+  SXE_DISPATCH_DT(d, TT, with_sweep(sweep_of(logits, V), [&](auto sw) {
     using S = typename dt_traits<TT>::storage;
-    hipLaunchKernelGGL((xent_kernel<TT>), dim3(grid), dim3(256), 0, cur_stream(), reinterpret_cast<S*>(logits.data_ptr()),
+    hipLaunchKernelGGL((xent_kernel<TT, decltype(sw)::value>), dim3(grid), dim3(256), 0, cur_stream(), reinterpret_cast<S*>(logits.data_ptr()),
                        rows, V, target.data_ptr<int64_t>(), ignore_index, loss.data_ptr<float>(), lse.data_ptr<float>(),
                        inplace_grad ? 1 : 0, sp, (float)grad_scale);
-  });
+  }));
   SXE_LAUNCH_CHECK();
   return {loss, lse};
 }
@@ -259,12 +280,12 @@ at::Tensor xent_bwd(at::Tensor logits, at::Tensor target, at::Tensor lse, at::Te
   c10::DeviceGuard guard(logits.device());
   at::Tensor grad = inplace ? logits : at::empty_like(logits);
   if (rows == 0) return grad;
-  const bool vec = ((reinterpret_cast<uintptr_t>(logits.data_ptr()) ^ reinterpret_cast<uintptr_t>(grad.data_ptr())) & 15) == 0;
+  const bool alike = ((reinterpret_cast<uintptr_t>(logits.data_ptr()) ^ reinterpret_cast<uintptr_t>(grad.data_ptr())) & 15) == 0;
   const int grid = (int)std::min<int64_t>(rows, 8192);
   DT d = dtype_of(logits);
-  SXE_DISPATCH_DT(d, TT, SXE_DISPATCH_BOOL(vec, VB, {
+  SXE_DISPATCH_DT(d, TT, with_sweep(alike ? sweep_of(logits, V) : ELEMENTS, [&](auto sw) {
     using S = typename dt_traits<TT>::storage;
-    hipLaunchKernelGGL((xent_bwd_kernel<TT, VB>), dim3(grid), dim3(256), 0, cur_stream(),
+    hipLaunchKernelGGL((xent_bwd_kernel<TT, decltype(sw)::value>), dim3(grid), dim3(256), 0, cur_stream(),
                        reinterpret_cast<const S*>(logits.data_ptr()), reinterpret_cast<S*>(grad.data_ptr()), rows, V,
                        target.data_ptr<int64_t>(), ignore_index, lse.data_ptr<float>(), dloss.data_ptr<float>());
   }));

@@ -464,7 +464,8 @@ def _colsum_faster(x):
 def column_sum(x, dtype):
     """``x.sum(0)`` of [R, N] in ``dtype``, accumulated in fp32 (csrc/kernels/colsum.hip; fp64, recorded sums and sizes where it is
     not the faster one: torch)."""
-    if (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16, torch.float32) and x.stride(1) == 1 and dtype in (x.dtype, torch.float32)
+    if (x.is_cuda and x.shape[0] >= 128 and x.dtype in (torch.bfloat16, torch.float16, torch.float32) and x.stride(1) == 1
+            and dtype in (x.dtype, torch.float32)
             and not (torch.is_grad_enabled() and x.requires_grad) and native.plain(x) and _colsum_faster(x)):
         native.require_hip()
         return torch.ops.sxe.column_sum(x, dtype)
