@@ -18,10 +18,13 @@
 namespace sxe {
 
 constexpr float kFltMax = 3.402823466e38f;
+// Running (max, sum) and another one. The products are fused as written, so that a loss does not depend on what surrounds the merge:
+// a sweep rounds what it adds (LANES: what it has) before the sum.
+template <bool LANES>
 __device__ __forceinline__ void ms_merge(float& m, float& s, float m2, float s2) {
   // against a finite reference: nothing but masked logits so far adds nothing (a branch on it costs 10 % where rows are few)
-  const float mn = fmaxf(m, m2), ref = fmaxf(mn, -kFltMax);
-  s = s * __expf(m - ref) + s2 * __expf(m2 - ref);
+  const float mn = fmaxf(m, m2), ref = fmaxf(mn, -kFltMax), e = __expf(m - ref), e2 = __expf(m2 - ref);
+  s = LANES ? __builtin_fmaf(s2, e2, s * e) : __builtin_fmaf(s, e, s2 * e2);
   m = mn;
 }
 
@@ -76,18 +79,18 @@ __device__ __forceinline__ float row_lse(const typename dt_traits<T>::storage* _
     const float ref = fmaxf(lm, -kFltMax);
 #pragma unroll
     for (int j = 0; j < 8; ++j) ls += __expf(v[j] - ref);
-    ms_merge(m, s, lm, ls);
-  }, [&](int c) { ms_merge(m, s, to_f32<T>(row[c]), 1.f); });
+    ms_merge<false>(m, s, lm, ls);
+  }, [&](int c) { ms_merge<false>(m, s, to_f32<T>(row[c]), 1.f); });
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     float m2 = __shfl_xor(m, o, 64), s2 = __shfl_xor(s, o, 64);
-    ms_merge(m, s, m2, s2);
+    ms_merge<true>(m, s, m2, s2);
   }
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   if (lane == 0) { red[2 * w] = m; red[2 * w + 1] = s; }
   __syncthreads();
   float M = red[0], Ssum = red[1];
-  for (int i = 1; i < (int)(blockDim.x >> 6); ++i) ms_merge(M, Ssum, red[2 * i], red[2 * i + 1]);
+  for (int i = 1; i < (int)(blockDim.x >> 6); ++i) ms_merge<true>(M, Ssum, red[2 * i], red[2 * i + 1]);
   __syncthreads();
   return M + __logf(Ssum);
 }

@@ -12,7 +12,7 @@ def _native():
     native.require_hip()
 
 
-@pytest.mark.parametrize("V", [1, 5, 8, 9, 31, 2049, 4100, 50257])
+@pytest.mark.parametrize("V", [1, 5, 8, 9, 31, 511, 513, 2049, 4096, 4100, 50257])
 @pytest.mark.parametrize("offset", [0, 3])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_rows(V, offset, dtype):
