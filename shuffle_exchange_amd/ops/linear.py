@@ -451,20 +451,24 @@ def _autocast_dtype(x):
     return None
 
 
+COLSUM_ROWS = 256
+
+
 def _colsum_faster(x):
-    """Whether csrc/kernels/colsum.hip beats the general reduction, us, general / kernel: bf16 128 x 768 6.4 / 5.3, 2048 x 3072
+    """Whether csrc/kernels/colsum.hip beats the general reduction, us, general / kernel: bf16 256 x 768 8.6 / 3.5, 2048 x 3072
     17.0 / 5.4, 2048 x 14336 99 / 12, 16384 x 8192 49 / 46; but 16 x 1048576 5.9 / 79, 8192 x 28672 80 / 93, and where rows do not
-    start on 16 bytes 2048 x 1001 12.9 / 21.8, 2048 x 50257 60 / 133, from 4096 rows on 22 / 16 at 1001, 48 / 23 at 3001 columns."""
+    start on 16 bytes 2048 x 1001 12.9 / 21.8, 2048 x 50257 60 / 133, from 4096 rows on 22 / 16 at 1001, 48 / 23 at 3001 columns.
+    Steps of fewer rows are bound by the host, where the kernel costs 3 us more: 128 x 768 5.8 / 3.3 on the device, 5.5 / 8.3 there."""
     R, N = x.shape
     if N % 8 or x.stride(0) * x.element_size() % 16 or x.data_ptr() % 16:
         return R >= 4096 and 64 <= N <= 8192
-    return R >= 128 and N <= 65536 and (N <= 8192 or R < 8192)
+    return R >= COLSUM_ROWS and N <= 65536 and (N <= 8192 or R < 8192)
 
 
 def column_sum(x, dtype):
     """``x.sum(0)`` of [R, N] in ``dtype``, accumulated in fp32 (csrc/kernels/colsum.hip; fp64, recorded sums and sizes where it is
     not the faster one: torch)."""
-    if (x.is_cuda and x.shape[0] >= 128 and x.dtype in (torch.bfloat16, torch.float16, torch.float32) and x.stride(1) == 1
+    if (x.is_cuda and x.shape[0] >= COLSUM_ROWS and x.dtype in (torch.bfloat16, torch.float16, torch.float32) and x.stride(1) == 1
             and dtype in (x.dtype, torch.float32)
             and not (torch.is_grad_enabled() and x.requires_grad) and native.plain(x) and _colsum_faster(x)):
         native.require_hip()

@@ -229,8 +229,8 @@ def test_streaming_rule():
 
 
 @gpu
-@pytest.mark.parametrize("R,N,kernel", [(127, 768, False), (128, 768, True), (4096, 8192, True), (8192, 8192, True), (8192, 8200, False),
-                                        (8191, 8200, True), (4095, 1001, False), (4096, 1001, True), (4096, 63, False), (128, 65544, False)])
+@pytest.mark.parametrize("R,N,kernel", [(255, 768, False), (256, 768, True), (4096, 8192, True), (8192, 8192, True), (8192, 8200, False),
+                                        (8191, 8200, True), (4095, 1001, False), (4096, 1001, True), (4096, 63, False), (256, 65544, False)])
 def test_column_sum_rule(R, N, kernel):
     from shuffle_exchange_amd.ops import linear as L
     x = torch.randn(R, N, device="cuda").bfloat16()
