@@ -529,12 +529,11 @@ static bool evo_has(const c10::optional<at::Tensor>& t) { return t.has_value() &
 
 struct EvoCall {
   evo::Args a{};
-  at::Tensor q, k, v, b1, pq, pk;  // keep what the pointers look at
+  at::Tensor q, k, v;  // keep what the pointers look at
   at::ScalarType pair = at::ScalarType::Undefined;
 };
 
-static EvoCall evo_call(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const c10::optional<at::Tensor>& b1,
-                        const c10::optional<at::Tensor>& b2, bool backward) {
+static EvoCall evo_call(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v) {
   SXE_CHECK(q.dim() == 5 && q.sizes() == k.sizes() && q.sizes() == v.sizes(), "evoformer: q/k/v [B, N, L, H, D]");
   for (const at::Tensor* t : {&q, &k, &v})
     SXE_CHECK(t->is_contiguous() && t->scalar_type() == at::kBFloat16, "evoformer: contiguous bf16 q/k/v");
@@ -554,34 +553,42 @@ static EvoCall evo_call(const at::Tensor& q, const at::Tensor& k, const at::Tens
   a.q = reinterpret_cast<const unsigned short*>(c.q.data_ptr());
   a.k = reinterpret_cast<const unsigned short*>(c.k.data_ptr());
   a.v = reinterpret_cast<const unsigned short*>(c.v.data_ptr());
+  return c;
+}
+
+// bias1 and bias2 as the kernels read them: [mask, pq, pk], pq undefined without bias2, pk without a backward to come, too
+static std::vector<at::Tensor> evo_pack(const evo::Args& a, const at::TensorOptions& opt, const c10::optional<at::Tensor>& b1,
+                                        const c10::optional<at::Tensor>& b2, bool backward) {
   const int64_t rows = (int64_t)a.B * a.N;
+  const bool pair = evo_has(b2), has1 = evo_has(b1);
   auto ok = [](const at::Tensor& t) { return t.is_contiguous() && (t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16); };
-  c.b1 = at::empty({rows, a.Lp}, q.options().dtype(at::kFloat));
-  a.b1 = c.b1.data_ptr<float>();
-  if (evo_has(b1)) SXE_CHECK(ok(*b1) && b1->numel() == rows * a.L, "evoformer: bias1 fp32 / bf16 [B, N, 1, 1, L]");
+  if (has1) SXE_CHECK(ok(*b1) && b1->numel() == rows * a.L, "evoformer: bias1 fp32 / bf16 [B, N, 1, 1, L]");
+  if (pair) SXE_CHECK(ok(*b2) && b2->numel() == (int64_t)a.B * a.H * a.L * a.L, "evoformer: bias2 fp32 / bf16 [B, 1, H, L, L]");
+  at::Tensor mask = at::empty({rows, a.Lp}, opt.dtype(at::kFloat)), pq, pk;
+  if (pair) pq = at::empty({(int64_t)a.B * a.H, a.Lp, a.Lp}, b2->options());
+  if (pair && backward) pk = at::empty_like(pq);
+  if (mask.numel() == 0) return {mask, pq, pk};
   const int nt = a.Lp / 32;
-  if (evo_has(b2)) {
-    SXE_CHECK(ok(*b2) && b2->numel() == (int64_t)a.B * a.H * a.L * a.L, "evoformer: bias2 fp32 / bf16 [B, 1, H, L, L]");
-    c.pair = b2->scalar_type();
-    c.pq = at::empty({(int64_t)a.B * a.H, a.Lp, a.Lp}, b2->options());
-    if (backward) c.pk = at::empty_like(c.pq);
-    a.pq = c.pq.data_ptr();
-    a.pk = backward ? c.pk.data_ptr() : nullptr;
-  }
-  if (rows * a.Lp == 0) return c;
   auto pack = [&](auto* t) {
     using T = std::remove_pointer_t<decltype(t)>;
-    const bool pair = evo_has(b2), has1 = evo_has(b1);
     hipLaunchKernelGGL(evo::pack_kernel<T>, pair ? dim3(nt * nt, a.B * a.H + 1) : dim3(64, 1), dim3(256), 0, cur_stream(),
-                       has1 ? b1->data_ptr() : nullptr, has1 && b1->scalar_type() == at::kBFloat16, c.b1.data_ptr<float>(),
-                       rows * a.Lp, pair ? reinterpret_cast<const T*>(b2->data_ptr()) : nullptr,
-                       pair ? reinterpret_cast<T*>(c.pq.data_ptr()) : nullptr,
-                       pair && backward ? reinterpret_cast<T*>(c.pk.data_ptr()) : nullptr, a.L, nt);
+                       has1 ? b1->data_ptr() : nullptr, has1 && b1->scalar_type() == at::kBFloat16, mask.data_ptr<float>(), mask.numel(),
+                       pair ? reinterpret_cast<const T*>(b2->data_ptr()) : nullptr,
+                       pair ? reinterpret_cast<T*>(pq.data_ptr()) : nullptr,
+                       pk.defined() ? reinterpret_cast<T*>(pk.data_ptr()) : nullptr, a.L, nt);
   };
-  if (c.pair == at::kBFloat16) pack((unsigned short*)nullptr);
+  if (pair && b2->scalar_type() == at::kBFloat16) pack((unsigned short*)nullptr);
   else pack((float*)nullptr);
   SXE_LAUNCH_CHECK();
-  return c;
+  return {mask, pq, pk};
+}
+
+static void evo_set_packed(EvoCall& c, const at::Tensor& mask, const c10::optional<at::Tensor>& pq, const c10::optional<at::Tensor>& pk) {
+  c.a.b1 = mask.data_ptr<float>();
+  if (!evo_has(pq)) return;
+  c.pair = pq->scalar_type();
+  c.a.pq = pq->data_ptr();
+  c.a.pk = evo_has(pk) ? pk->data_ptr() : nullptr;
 }
 
 // f(head dim constant, pair bias type tag)
@@ -596,16 +603,20 @@ static void evo_dispatch(int D, at::ScalarType pair, F f) {
   else with(std::integral_constant<int, 64>{});
 }
 
+// -> [o, lse, packed biases of evo_pack]: the backward reads these, not the biases, which the caller may have changed by then
 std::vector<at::Tensor> evoformer_fwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
-                                      const c10::optional<at::Tensor>& b1, const c10::optional<at::Tensor>& b2) {
+                                      const c10::optional<at::Tensor>& b1, const c10::optional<at::Tensor>& b2, bool backward) {
   check_beside(q, {k, v, b1, b2});
   c10::DeviceGuard g(q.device());
-  EvoCall c = evo_call(q, k, v, b1, b2, false);
+  EvoCall c = evo_call(q, k, v);
   evo::Args& a = c.a;
+  auto packed = evo_pack(a, q.options(), b1, b2, backward);
+  evo_set_packed(c, packed[0], packed[1], packed[2]);
   auto o = at::empty_like(q);
   auto lse = at::empty({(int64_t)a.B * a.N, a.H, a.Lp}, q.options().dtype(at::kFloat));
   const int grid = a.B * a.N * a.H * (a.Lp / evo::QB);
-  if (grid == 0) return {o, lse};
+  packed.insert(packed.begin(), {o, lse});
+  if (grid == 0) return packed;
   a.lse = lse.data_ptr<float>();
   evo_dispatch(q.size(4), c.pair, [&](auto d, auto t) {
     constexpr int D = decltype(d)::value;
@@ -613,21 +624,31 @@ std::vector<at::Tensor> evoformer_fwd(const at::Tensor& q, const at::Tensor& k, 
                        a, reinterpret_cast<unsigned short*>(o.data_ptr()));
   });
   SXE_LAUNCH_CHECK();
-  return {o, lse};
+  return packed;
 }
 
 std::vector<at::Tensor> evoformer_bwd(const at::Tensor& dout, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
-                                      const at::Tensor& o, const at::Tensor& lse, const c10::optional<at::Tensor>& b1,
-                                      const c10::optional<at::Tensor>& b2, bool need_db1, bool need_db2) {
-  check_beside(q, {dout, k, v, o, lse, b1, b2});
+                                      const at::Tensor& o, const at::Tensor& lse, const at::Tensor& mask,
+                                      const c10::optional<at::Tensor>& pq, const c10::optional<at::Tensor>& pk, bool need_db1,
+                                      bool need_db2) {
+  check_beside(q, {dout, k, v, o, lse, mask, pq, pk});
   c10::DeviceGuard g(q.device());
-  EvoCall c = evo_call(q, k, v, b1, b2, true);
+  EvoCall c = evo_call(q, k, v);
   evo::Args& a = c.a;
+  SXE_CHECK(mask.numel() == (int64_t)a.B * a.N * a.Lp && mask.scalar_type() == at::kFloat && mask.is_contiguous(),
+            "evoformer_bwd: mask as the forward packed it");
+  SXE_CHECK(evo_has(pq) == evo_has(pk), "evoformer_bwd: both forms of bias2");
+  if (evo_has(pq))
+    for (const at::Tensor* t : {&*pq, &*pk})
+      SXE_CHECK(t->numel() == (int64_t)a.B * a.H * a.Lp * a.Lp && t->is_contiguous() && t->scalar_type() == pq->scalar_type() &&
+                    (t->scalar_type() == at::kFloat || t->scalar_type() == at::kBFloat16) &&
+                    reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "evoformer_bwd: bias2 as the forward packed it");
+  evo_set_packed(c, mask, pq, pk);
   for (const at::Tensor* t : {&dout, &o})
     SXE_CHECK(t->sizes() == q.sizes() && t->is_contiguous() && t->scalar_type() == at::kBFloat16, "evoformer_bwd: dout / o like q");
   SXE_CHECK(lse.numel() == (int64_t)a.B * a.N * a.H * a.Lp && lse.scalar_type() == at::kFloat && lse.is_contiguous(),
             "evoformer_bwd: lse fp32 [B*N, H, Lp]");
-  SXE_CHECK(!need_db2 || evo_has(b2), "evoformer_bwd: gradient of a bias2 that is not there");
+  SXE_CHECK(!need_db2 || evo_has(pq), "evoformer_bwd: gradient of a bias2 that is not there");
   const at::Tensor d = evo_aligned(dout), oo = evo_aligned(o);
   auto stats = at::empty({2, lse.numel()}, lse.options());
   a.dout = reinterpret_cast<const unsigned short*>(d.data_ptr());
@@ -638,7 +659,7 @@ std::vector<at::Tensor> evoformer_bwd(const at::Tensor& dout, const at::Tensor& 
   auto dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
   at::Tensor db1, db2;
   if (need_db1) db1 = at::zeros({a.B, a.N, 1, 1, a.L}, q.options().dtype(at::kFloat));
-  if (need_db2) db2 = at::empty({a.B, 1, a.H, a.L, a.L}, b2->options());
+  if (need_db2) db2 = at::empty({a.B, 1, a.H, a.L, a.L}, pq->options());
   const int grid = a.B * a.N * a.H * (a.Lp / evo::QB);
   if (grid == 0) {
     if (need_db2) db2.zero_();
@@ -682,8 +703,8 @@ std::vector<at::Tensor> evoformer_bwd(const at::Tensor& dout, const at::Tensor& 
 }  // namespace sxe
 
 TORCH_LIBRARY_FRAGMENT(sxe, m) {
-  m.def("evoformer_fwd(Tensor q, Tensor k, Tensor v, Tensor? bias1, Tensor? bias2) -> Tensor[]");
-  m.def("evoformer_bwd(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, Tensor? bias1, Tensor? bias2, "
+  m.def("evoformer_fwd(Tensor q, Tensor k, Tensor v, Tensor? bias1, Tensor? bias2, bool backward=False) -> Tensor[]");
+  m.def("evoformer_bwd(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, Tensor mask, Tensor? pq, Tensor? pk, "
         "bool need_db1, bool need_db2) -> Tensor[]");
 }
 TORCH_LIBRARY_IMPL(sxe, CUDA, m) {

@@ -112,3 +112,24 @@ def test_evoformer_tiles_and_biases(B, N, L, H, D, bias):
     for a, b in zip(grads, rg):
         assert a.dtype == (dt if a.shape != Q.shape else torch.bfloat16)
         assert torch.isfinite(a).all() and (a.double() - b).norm() <= 8e-3 * b.norm() + slack, a.shape
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_evoformer_biases_reused_before_backward(dtype):
+    """A program may write the next crop's mask and pair bias into the same buffers before this crop's backward."""
+    torch.manual_seed(2)
+    mk = lambda *s: torch.randn(*s, device="cuda")
+    Q, K, V, g = (mk(1, 5, 70, 2, 32).bfloat16() for _ in range(4))
+    b1, b2 = mk(1, 5, 1, 1, 70).to(dtype), mk(1, 1, 2, 70, 70).to(dtype)
+
+    def grads(change):
+        ins = [t.detach().clone().requires_grad_(True) for t in (Q, K, V)]
+        m, p = b1.clone(), b2.clone()
+        out = ea.evoformer_attention(*ins, m, p)
+        if change:
+            m.fill_(float("nan"))
+            p.fill_(float("nan"))
+        return torch.autograd.grad(out, ins, g)
+    for a, b in zip(grads(True), grads(False)):
+        assert torch.equal(a, b)
