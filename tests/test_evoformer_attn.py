@@ -133,3 +133,18 @@ def test_evoformer_biases_reused_before_backward(dtype):
         return torch.autograd.grad(out, ins, g)
     for a, b in zip(grads(True), grads(False)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_evoformer_without_gradients():
+    """The call that no backward follows gives the same bits, and a dual tensor's tangent is not dropped without a word."""
+    import torch.autograd.forward_ad as fwAD
+    torch.manual_seed(3)
+    Q, K, V = (torch.randn(1, 5, 70, 2, 32, device="cuda").bfloat16() for _ in range(3))
+    b1, b2 = torch.randn(1, 5, 1, 1, 70, device="cuda"), torch.randn(1, 1, 2, 70, 70, device="cuda").bfloat16().requires_grad_()
+    want = ea.evoformer_attention(Q, K, V, b1, b2)
+    with torch.no_grad():
+        assert torch.equal(ea.evoformer_attention(Q, K, V, b1, b2), want)
+    assert want.requires_grad and not ea.evoformer_attention(Q, K, V, b1).requires_grad
+    with fwAD.dual_level(), pytest.raises((RuntimeError, NotImplementedError)):
+        ea.evoformer_attention(fwAD.make_dual(Q, torch.ones_like(Q)), K, V, b1, None)
