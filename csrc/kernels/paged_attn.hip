@@ -148,11 +148,12 @@ __device__ __forceinline__ int kperm(int g) { return ((g & 1) << 3) | ((g & 2) <
 
 constexpr int PR = 16;  // query rows per pass
 
-template <int D>
+// NT: 16-key tiles per wave chunk. D 128: 32 keys keep three workgroups a CU (148 registers, 33 KB) where 64 keep two: 24
+// sequences of 270 - 5300 keys (heads 32 / 8) 49 against 60 us, 32 of 3000 keys 78 against 82 us. 64 keys are the better form
+// where the workgroups make whole rounds of two a CU and a last round of three would be nearly empty (`wide`: the rule and its
+// figures are in ops/paged_attention.py).
+template <int D, int NT>
 struct PaGeo {
-  // 16-key tiles per wave chunk. D 128: 32 keys keep three workgroups a CU (148 registers, 33 KB) where 64 keep two: 24
-  // sequences of 270 - 5300 keys (heads 32 / 8) 49 against 60 us, 32 of 3000 keys 78 against 82 us
-  static constexpr int NT = D >= 128 ? 2 : 4;
   static constexpr int KC = 16 * NT;           // keys per wave chunk
   static constexpr int KS = D / 32;            // k-steps of the Q K^T product
   static constexpr int DT = D / 16;            // 16-wide d tiles of O^T
@@ -161,10 +162,10 @@ struct PaGeo {
   static constexpr int LDS = (kWaves * VIMG > MERGE ? kWaves * VIMG : MERGE);
 };
 
-template <int D>
-__global__ __launch_bounds__(256, D == 256 ? 1 : 3) void paged_attn_kernel(Args a) {
-  using P = PaGeo<D>;
-  constexpr int NT = P::NT, KC = P::KC, KS = P::KS, DT = P::DT;
+template <int D, int NT>
+__global__ __launch_bounds__(256, D == 256 ? 1 : D * NT > 256 ? 2 : 3) void paged_attn_kernel(Args a) {
+  using P = PaGeo<D, NT>;
+  constexpr int KC = P::KC, KS = P::KS, DT = P::DT;
   extern __shared__ __attribute__((aligned(16))) char smem[];  // V images, then the wave-merge buffer
   __shared__ int64_t koff_lds[kWaves][KC];
   __shared__ float mrg_ml[kWaves][PR][2];
@@ -558,7 +559,7 @@ static at::Tensor paged_attention_impl(const at::Tensor& q, const at::Tensor& ca
                                        double scale, int64_t max_kv_len, int64_t splits, int64_t window,
                                        std::vector<at::Tensor>* parts, const c10::optional<at::Tensor>& counters = {},
                                        const at::Tensor* seqs = nullptr, const at::Tensor* rows = nullptr,
-                                       const at::Tensor* into = nullptr) {
+                                       const at::Tensor* into = nullptr, bool wide = false) {
   check_beside(q, {cache, block_table, q_start, q_len, kv_len, counters});
   SXE_CHECK(q.scalar_type() == at::kBFloat16 && cache.scalar_type() == at::kBFloat16, "bf16 only");
   SXE_CHECK(q.dim() == 3 && q.stride(2) == 1 && q.stride(1) == q.size(2), "q must be [T, nq, D] with head stride D");
@@ -618,18 +619,16 @@ static at::Tensor paged_attention_impl(const at::Tensor& q, const at::Tensor& ca
   }
   dim3 grid(S * nkv, splits);
   SXE_CHECK(D == 128 || D == 64 || D == 256, "paged_attention: head_dim must be 64, 128 or 256");
-  static bool attr_set[3] = {false, false, false};
-  auto launch = [&](void (*kern)(pa::Args), size_t lds, int slot) {
-    if (!attr_set[slot]) {  // > 64 KiB of dynamic LDS must be opted into (gfx950: 160 KiB per CU)
-      SXE_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-      attr_set[slot] = true;
-    }
+  auto launch = [&](auto d, auto nt) {
+    constexpr auto kern = &pa::paged_attn_kernel<decltype(d)::value, decltype(nt)::value>;
+    constexpr int lds = pa::PaGeo<decltype(d)::value, decltype(nt)::value>::LDS;
+    allow_lds<kern>(lds);  // with the static part up to 66 KB
     hipLaunchKernelGGL(kern, grid, dim3(256), lds, cur_stream(), a);
   };
-  if (D == 128) launch(pa::paged_attn_kernel<128>, pa::PaGeo<128>::LDS, 0);
-  else if (D == 256) launch(pa::paged_attn_kernel<256>, pa::PaGeo<256>::LDS, 1);
-  else launch(pa::paged_attn_kernel<64>, pa::PaGeo<64>::LDS, 2);
+  if (D == 128 && wide) launch(std::integral_constant<int, 128>{}, std::integral_constant<int, 4>{});
+  else if (D == 128) launch(std::integral_constant<int, 128>{}, std::integral_constant<int, 2>{});
+  else if (D == 256) launch(std::integral_constant<int, 256>{}, std::integral_constant<int, 2>{});
+  else launch(std::integral_constant<int, 64>{}, std::integral_constant<int, 4>{});
   SXE_LAUNCH_CHECK();
   if (splits > 1 && parts != nullptr) {
     *parts = {part_o, part_ml};
@@ -641,9 +640,9 @@ static at::Tensor paged_attention_impl(const at::Tensor& q, const at::Tensor& ca
 
 at::Tensor paged_attention(const at::Tensor& q, const at::Tensor& cache, const at::Tensor& block_table,
                            const at::Tensor& q_start, const at::Tensor& q_len, const at::Tensor& kv_len, double scale,
-                           int64_t max_kv_len, int64_t splits, int64_t window, const c10::optional<at::Tensor>& counters) {
+                           int64_t max_kv_len, int64_t splits, int64_t window, const c10::optional<at::Tensor>& counters, bool wide) {
   return paged_attention_impl(q, cache, block_table, q_start, q_len, kv_len, scale, max_kv_len, splits, window, nullptr,
-                              counters);
+                              counters, nullptr, nullptr, nullptr, wide);
 }
 
 // The sequences of `seqs` only (int32 [n, 2]: sequence, row of its first partial; rows int32 [R]: token row of every
@@ -651,7 +650,7 @@ at::Tensor paged_attention(const at::Tensor& q, const at::Tensor& cache, const a
 void paged_attention_some(const at::Tensor& q, const at::Tensor& cache, const at::Tensor& block_table,
                           const at::Tensor& q_start, const at::Tensor& q_len, const at::Tensor& kv_len,
                           const at::Tensor& seqs, const at::Tensor& rows, double scale, int64_t max_kv_len, int64_t splits,
-                          int64_t window, at::Tensor out) {
+                          int64_t window, at::Tensor out, bool wide) {
   check_beside(q, {seqs, rows, out});
   SXE_CHECK(seqs.scalar_type() == at::kInt && seqs.is_contiguous() && seqs.dim() == 2 && seqs.size(1) == 2,
             "paged_attention_some: seqs int32 [n, 2]");
@@ -659,7 +658,7 @@ void paged_attention_some(const at::Tensor& q, const at::Tensor& cache, const at
   SXE_CHECK(out.sizes() == q.sizes() && out.is_contiguous() && out.scalar_type() == at::kBFloat16,
             "paged_attention_some: out contiguous bf16 like q");
   paged_attention_impl(q, cache, block_table, q_start, q_len, kv_len, scale, max_kv_len, splits, window, nullptr, {}, &seqs,
-                       &rows, &out);
+                       &rows, &out, wide);
 }
 
 // [out, part_o, part_ml]: with one split `out` is the attention output and the partials are empty;
@@ -685,9 +684,9 @@ TORCH_LIBRARY_FRAGMENT(sxe, m) {
   m.def("rope_kv_cache_append(Tensor(a!) qkv, Tensor cos, Tensor sin, Tensor pos, Tensor(b!) cache, Tensor slots, "
         "int nq, int nkv) -> ()");
   m.def("paged_attention(Tensor q, Tensor cache, Tensor block_table, Tensor q_start, Tensor q_len, Tensor kv_len, "
-        "float scale, int max_kv_len, int splits, int window=0, Tensor(a!)? counters=None) -> Tensor");
+        "float scale, int max_kv_len, int splits, int window=0, Tensor(a!)? counters=None, bool wide=False) -> Tensor");
   m.def("paged_attention_some(Tensor q, Tensor cache, Tensor block_table, Tensor q_start, Tensor q_len, Tensor kv_len, "
-        "Tensor seqs, Tensor rows, float scale, int max_kv_len, int splits, int window, Tensor(a!) out) -> ()");
+        "Tensor seqs, Tensor rows, float scale, int max_kv_len, int splits, int window, Tensor(a!) out, bool wide=False) -> ()");
   m.def("paged_attention_parts(Tensor q, Tensor cache, Tensor block_table, Tensor q_start, Tensor q_len, "
         "Tensor kv_len, float scale, int max_kv_len, int splits, int window=0) -> Tensor[]");
 }

@@ -101,7 +101,7 @@ class DecodeGraphRunner:
         matters = self._matters.get((S, kvb))
         if matters is None:
             nq, nkv, dim = (getattr(self.model, name, None) for name in ("nq", "nkv", "head_dim"))
-            splits = [choose_balanced_splits(S, nkv, kvb, 4 * S * nq * dim, even) for even in (True, False)] if nq and nkv and dim else (1, 1)
+            splits = [choose_balanced_splits(S, nkv, kvb, 4 * S * nq * dim, even, dim) for even in (True, False)] if nq and nkv and dim else (1, 1)
             matters = self._matters[S, kvb] = splits[0] != splits[1]
         return matters and even_lengths([s.seen_tokens + 1 for s in seqs])
 

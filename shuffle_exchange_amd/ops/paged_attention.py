@@ -6,6 +6,7 @@ Cache layout per layer: ``[num_blocks, 2, n_kv_heads, block_size, head_dim]`` (b
 tokens of each sequence over all of its cached keys. Both have PyTorch reference implementations
 (CPU processes / numerics oracles).
 """
+import functools
 import math
 import os
 
@@ -106,9 +107,11 @@ def choose_splits(num_seqs, nkv, max_kv_len, target_wgs=None):
 PA_SPLIT_KEYS = 512
 # Lengths are even where the longest is at most this many times the mean (a log-uniform spread over a factor of 2 has 1.4, of 10 2.6).
 PA_EVEN = 1.5
-# Workgroups that run at once, three a CU. Even sequences finish together, so a last round that is nearly empty costs a whole one:
-# 128 sequences of 4000 keys (1024 workgroups a split) 399 / 372 / 363 us with 1 / 2 / 3 splits, 8000 keys 777 / 722 / 704.
+# Workgroups that run at once, three a CU (other head dims: by registers). Even sequences finish together, so a last round that is nearly
+# empty costs a whole one: 100 sequences (800 workgroups a split) of 2500 keys 221 / 194 us with 1 / 3 splits, but 160 (1280) of 1500
+# 174 / 182; heads of 64, 128 sequences of 12 heads and 4000 keys 278 / 262 with 1 / 2.
 PA_RESIDENT_WGS = 768
+PA_RESIDENT = {64: 1024, 128: PA_RESIDENT_WGS, 256: 256}
 # Bytes of fp32 partials that such short splits may take: 256 decoding sequences keep splits of 512 keys up to 32k keys (heads of
 # 32 x 128), a call of many tokens has the splits of choose_splits, as its partials grow with tokens x splits.
 PA_SPLIT_BYTES = 1 << 28
@@ -119,7 +122,15 @@ def even_lengths(lengths):
     return len(lengths) * max(lengths, default=0) <= PA_EVEN * sum(lengths)
 
 
-def choose_balanced_splits(num_seqs, nkv, max_kv_len, split_bytes, even=False):
+def two_a_cu(workgroups, head_dim):
+    """Whether one split runs better on the kernel's form of 64 keys a wave and two workgroups a CU: these make whole rounds of 512, of
+    768 the last one would be nearly empty. Heads of 128, us, so / one split of the other form / the best number of its splits: 128
+    sequences of 8 kv heads 1500 keys 136 / 156 / 147, 4000 keys 350 / 392 / 360; 32 of 32 kv heads 1000 keys 94 / 106 / 103; a remainder
+    of 512 (64 of 32 kv heads, 2048 workgroups, 1000 to 3000 keys) 183 - 507 / 190 - 523, 256 of 8 379 / 367 at 2000."""
+    return head_dim == 128 and workgroups > 768 and 0 < workgroups % 768 <= 256 and (-workgroups) % 512 < 64
+
+
+def choose_balanced_splits(num_seqs, nkv, max_kv_len, split_bytes, even=False, head_dim=128):
     """``choose_splits``, and no split over PA_SPLIT_KEYS keys: where sequences of a batch differ in length, a workgroup that
     walks a long one alone outlasts the rest. Splits behind a sequence's end exit at once, the merge does not read them.
     ``even`` (``even_lengths``): as few splits as fill the chip, in rounds that are mostly full.
@@ -129,12 +140,20 @@ def choose_balanced_splits(num_seqs, nkv, max_kv_len, split_bytes, even=False):
         return max(splits, min(math.ceil(max_kv_len / PA_SPLIT_KEYS), most))
 
     def full(s):  # share of the resident workgroups that the rounds keep busy
-        rounds = num_seqs * nkv * s / PA_RESIDENT_WGS
+        rounds = num_seqs * nkv * s / PA_RESIDENT.get(head_dim, PA_RESIDENT_WGS)
         return 1 if rounds <= 1 else rounds / math.ceil(rounds)
-    if full(splits) > 0.85:
+    if full(splits) > 0.8 or (splits == 1 and two_a_cu(num_seqs * nkv, head_dim)):
         return splits
     more = [s for s in range(splits, splits + 3) if s == splits or (s <= most and max_kv_len >= s * 320)]
     return max(more, key=full)
+
+
+@functools.lru_cache(maxsize=4096)
+def _decode_plan(num_seqs, nkv, max_kv_len, split_bytes, even, head_dim, tuned):
+    """(splits, two workgroups a CU) of a launch: all layers of a step ask for the same, a microsecond of the host each. ``tuned``: the
+    settings that the choice reads."""
+    splits = choose_balanced_splits(num_seqs, nkv, max_kv_len, split_bytes, even, head_dim)
+    return splits, splits == 1 and two_a_cu(num_seqs * nkv, head_dim)
 
 
 def paged_attention_parts(q, cache, block_table, q_start, q_len, kv_len, scale, max_kv_len, splits=None):
@@ -188,13 +207,15 @@ def paged_attention(q, cache, block_table, q_start, q_len, kv_len, scale, max_kv
     if window is not None and max_kv_len <= window:
         window = None
     if native.use_hip(q) and q.shape[-1] in (64, 128, 256):
+        S, nkv = block_table.shape[0], cache.shape[2]
         if splits is None:
-            splits = choose_balanced_splits(block_table.shape[0], cache.shape[2], max_kv_len, 4 * q.numel(), even)
-        S = block_table.shape[0]
-        cnt = (_split_counters(q.device, S * cache.shape[2])
+            splits, wide = _decode_plan(S, nkv, int(max_kv_len), 4 * q.numel(), even, q.shape[-1], (PA_TARGET_WGS, PA_MIN_KEYS))
+        else:
+            wide = splits == 1 and two_a_cu(S * nkv, q.shape[-1])
+        cnt = (_split_counters(q.device, S * nkv)
                if PA_LAST_MERGE and splits > 1 and q.shape[0] <= 4 * S else None)
         return torch.ops.sxe.paged_attention(q, cache, block_table, q_start, q_len, kv_len, float(scale),
-                                             int(max_kv_len), int(splits), int(window or 0), cnt)
+                                             int(max_kv_len), int(splits), int(window or 0), cnt, wide)
     if q.is_cuda:
         from ..utils.logging import warning_once
         warning_once(f"paged_attention: head_dim={q.shape[-1]} window={window} not covered by the HIP kernel; "
@@ -285,7 +306,9 @@ def ragged_attention(q, cache, batch, scale, window=None, kv=None):
             rows = batch.tile_rows(x) if splits > 1 else None
             torch.ops.sxe.paged_prefill(*meta, x.tiles, rows, float(scale), int(window or 0), splits, keys, out)
     if lists is not None and lists.seqs is not None:
-        splits = choose_balanced_splits(lists.seqs.shape[0], nkv, lists.seq_keys, 4 * lists.seq_rows.numel() * q.shape[1] * q.shape[2], lists.seq_even)
+        n, D = lists.seqs.shape[0], q.shape[2]
+        splits, wide = _decode_plan(n, nkv, lists.seq_keys, 4 * lists.seq_rows.numel() * q.shape[1] * D, lists.seq_even, D,
+                                    (PA_TARGET_WGS, PA_MIN_KEYS))
         torch.ops.sxe.paged_attention_some(*meta, lists.seqs, lists.seq_rows, float(scale), int(lists.seq_keys), int(splits),
-                                           int(window or 0), out)
+                                           int(window or 0), out, wide)
     return out

@@ -185,3 +185,42 @@ def test_even_splits(nkv):
             assert plain <= n <= plain + 2 and (n == plain or keys >= n * 320) and (n == plain or n * seqs * 16384 <= PA.PA_SPLIT_BYTES)
             if seqs * nkv * plain <= PA.PA_RESIDENT_WGS:
                 assert n == plain
+
+
+def test_two_workgroups_a_cu():
+    """Whole rounds of 512 workgroups where the last of 768 is nearly empty, heads of 128 only, and then one split of even sequences."""
+    took = [n for n in range(1, 4000) if PA.two_a_cu(n, 128)]
+    assert {961, 1024, 2560}.issubset(took) and not {1, 512, 768, 960, 1025, 1280, 1536, 1792, 2048, 2304}.intersection(took)
+    assert not PA.two_a_cu(1024, 64) and not PA.two_a_cu(1024, 256)
+    assert PA.choose_balanced_splits(128, 8, 4000, 1 << 21, True) == 1 and PA.choose_balanced_splits(128, 8, 4000, 1 << 21) == 8
+    assert PA.choose_balanced_splits(128, 8, 4000, 1 << 20, True, 64) == 1 and PA.choose_balanced_splits(128, 12, 4000, 1 << 20, True, 64) == 2
+    assert PA.choose_balanced_splits(128, 8, 4000, 1 << 22, True, 256) == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("seqs,nkv,group", [(32, 32, 1), (128, 8, 4), (61, 16, 20)])
+@pytest.mark.parametrize("window", [None, 70])
+def test_wide_chunks_match_reference(seqs, nkv, group, window):
+    """One split on 64 keys a wave (more than 768 workgroups) against the gather: lengths around a wave's and a workgroup's chunk, several
+    passes of 16 rows, blocks in any order, NaN behind a sequence's last key."""
+    PA.native.require_hip()
+    g = torch.Generator(device="cuda").manual_seed(seqs)
+    bs, D, most = 16, 128, 300
+    per = -(-most // bs)
+    lens = [(1, 63, 64, 65, 255, 256, 257, 300)[i % 8] for i in range(seqs)]
+    assert PA.two_a_cu(seqs * nkv, D)
+    cache = torch.full((seqs * per, 2, nkv, bs, D), float("nan"), dtype=torch.bfloat16, device="cuda")
+    bt = torch.randperm(seqs * per, generator=g, device="cuda").to(torch.int32).view(seqs, per)
+    kv = torch.randn(seqs, 2, nkv, most, D, generator=g, device="cuda").bfloat16()
+    for i, n in enumerate(lens):
+        for b in range(-(-n // bs)):
+            m = min(bs, n - b * bs)
+            cache[int(bt[i, b]), :, :, :m] = kv[i, :, :, b * bs:b * bs + m]
+    q = torch.randn(seqs, nkv * group, D, generator=g, device="cuda").bfloat16()
+    one = torch.ones(seqs, dtype=torch.int32, device="cuda")
+    meta = (bt, torch.arange(seqs, dtype=torch.int32, device="cuda"), one, torch.tensor(lens, dtype=torch.int32, device="cuda"))
+    got = [torch.ops.sxe.paged_attention(q, cache, *meta, D ** -0.5, most, 1, window or 0, None, wide) for wide in (True, False)]
+    want = PA.paged_attention_reference(q, cache, *meta, D ** -0.5, window)
+    for y in got:  # bf16 weights and result: two roundings of 2^-9 on values that are averages of unit normals
+        assert not y.isnan().any() and (y.float() - want.float()).norm() <= 2 ** -7 * want.float().norm()
+    assert torch.equal(PA.paged_attention(q, cache, *meta, D ** -0.5, most, window=window, splits=1), got[0])
