@@ -518,7 +518,8 @@ def linear(x, weight, bias=None):
     if grad and weight.requires_grad and hasattr(weight, "_sxe_grad_target"):
         return _Linear.apply(x, weight, bias)
     if (not grad and SKINNY_MAX_M > 0 and x.is_cuda and x.numel() <= max(SKINNY_MAX_M, STREAM_ROWS_SMALL) * x.shape[-1]
-            and _autocast_dtype(x) in (None, torch.bfloat16) and native.plain(x, weight, bias)):
+            and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == torch.bfloat16)
+            and native.plain(x, weight, bias)):
         y = _skinny(x, weight, bias)
         if y is None:
             y = _stream(x, weight, bias)

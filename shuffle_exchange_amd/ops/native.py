@@ -99,18 +99,20 @@ def use_hip(t):
 
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
+# bound once: decode-sized products ask at every call, and each name looked up costs them host time
+_compiling, _tracing, _modes = torch.compiler.is_compiling, torch._C._is_tracing, torch._C._len_torch_dispatch_stack
+_transforms, _batched = _functorch.peek_interpreter_stack, _functorch.is_legacy_batchedtensor
 
 
 def plain(*tensors):
     """A kernel that looks at its operands' memory and has no derivative may take these (None: no operand): no transform's wrapper
     (vmap, jvp, functionalize), no subclass (fake and distributed tensors), and nobody who follows the call by its operators:
     compilation, a trace, forward-mode derivatives."""
-    if (torch.compiler.is_compiling() or torch._C._is_tracing() or fwAD._current_level >= 0
-            or _functorch.peek_interpreter_stack() is not None
-            or (torch._C._len_torch_dispatch_stack() and torch._C._get_dispatch_mode(torch._C._TorchDispatchModeKey.PROXY) is not None)):
+    if (_compiling() or _tracing() or fwAD._current_level >= 0 or _transforms() is not None
+            or (_modes() and torch._C._get_dispatch_mode(torch._C._TorchDispatchModeKey.PROXY) is not None)):
         return False
     for t in tensors:
-        if t is not None and (type(t) not in _PLAIN or _functorch.is_legacy_batchedtensor(t)):
+        if t is not None and (type(t) not in _PLAIN or _batched(t)):
             return False
     return True
 
