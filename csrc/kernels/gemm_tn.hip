@@ -1,0 +1,296 @@
+// Products of many rows on gfx950: y[M, N] = x[M, K] . w[N, K]' (+ bias), both operands with K contiguous, and the same with SwiGLU
+// over w = [gate | up] in the epilogue (y[M, N / 2] = silu(x . gate') * (x . up'), one rounding, of the result). bf16 in and out, fp32
+// sums. skinny_gemm.hip and stream_gemm.hip have the forms for up to 32 rows.
+//
+// What bounds it: at 256 x 256 the card's power. Products of 16 x 16 x 32 run at 1.85 GHz where those of 32 x 32 x 16 run at
+// 1.65 (they read and write half as many sums a flop); behind them LDS, which is busy for 80 % of the products' time.
+//  * Slabs of 64 k, 128-byte rows (a whole cache line a row: with slabs of 32 the L2 answers twice the requests, 1.28 against 1.5
+//    PFLOP/s), by direct-to-LDS loads through the loop of sxe_gemm_loop.h. Of 160 KB, 256 x 256 has room for two slabs of x and three
+//    of w, which comes from memory where x is in a cache (1040 rows, 28672 x 4096 with SwiGLU 218 us the other way, 200 so).
+//  * w rows lie in LDS so that a lane's sums of neighbouring 16-row blocks are 8 neighbouring columns of y: 16-byte stores (8-byte
+//    ones cost 3 % at K = 4096). A round's workgroups end together, and their stores are what is left of its start: 5 % at K = 4096,
+//    13 % at 2048.
+//  * The row tiles of a column block run side by side on one XCD.
+// us, the library / here: 8192 rows, 28672 x 4096 1255 / 1285 (with SwiGLU 1376 / 1290), 4096 x 14336 604 / 630, 4096 x 4096 174 / 184;
+// 7588 rows, 28672 x 4096 with SwiGLU 1390 / 1250, 4096 x 14336 1010 / 620; 1040 rows 238 / 200 and 142 / 110.
+#include "sxe_common.h"
+#include "sxe_gemm_loop.h"
+#include <torch/library.h>
+#include <cmath>
+
+namespace sxe {
+namespace tn {
+using namespace gl;
+
+constexpr int ROW = 2 * BK;
+
+struct Args {
+  const unsigned short *x, *w, *bias;
+  unsigned short* y;
+  float* part;           // splits of K: their sums, [splits, M, N]
+  int64_t ldx, ldw;
+  int M, cols, half, slabs, per, splits;  // columns of y (SwiGLU: half the rows of w); w row that goes with row 0 as up; slabs of K, of a split
+  int tm, tn, gm;        // whole row tiles, column blocks; row tiles that run side by side
+};
+
+// Column of a tile that LDS row r of w holds (SwiGLU: of gate for even blocks of 16 rows, of up for odd ones)
+template <bool GLU>
+__device__ __forceinline__ int column(int r) {
+  const int p = r & 15, b = GLU ? (r >> 5) & 1 : (r >> 4) & 1;
+  return (GLU ? (r >> 6) * 32 : r & ~31) + 8 * (p >> 2) + 4 * b + (p & 3);
+}
+
+template <typename T, bool GLU, bool SPLIT>
+__global__ void __launch_bounds__(T::NTHR, T::WAVES) gemm_kernel(Args a) {
+  constexpr int RT = T::RT, CT = T::CT, NW = T::NW, PA = T::PA, PB = T::PB, BM = T::BM, CB = GLU ? T::BN / 2 : T::BN, X_LDS = T::SA * T::AS;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wr = w / T::WC, wc = w % T::WC;
+  // ---- workgroup -> (split, row tile, column block): neighbours in an XCD's run share w, gm row tiles at a time. The tiles of the
+  // last rows, if these are no whole tile, come behind all others: they take less time and fill the last round
+  const int whole = a.tm * a.tn * a.splits;
+  const bool rest = (int)blockIdx.x >= whole;
+  const int block = rest ? blockIdx.x - whole : blockIdx.x, nwg = rest ? gridDim.x - whole : whole;
+  const int q8 = nwg / 8, r8 = nwg % 8, xcd = block % 8;
+  const int id = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + block / 8;
+  const int nt = rest ? a.tn : a.tm * a.tn, split = SPLIT ? id / nt : 0, tile = SPLIT ? id - split * nt : id;
+  const int per_group = a.gm * a.tn, group = tile / per_group, in = tile - group * per_group, rows = min(a.tm - group * a.gm, a.gm);
+  const int m0 = (rest ? a.tm : group * a.gm + in % rows) * BM, n0 = (rest ? tile : in / rows) * CB;
+  const int first = SPLIT ? split * a.per : 0, ns = SPLIT ? min(a.per, a.slabs - first) : a.slabs;
+
+  // ---- loads: a wave's load is 8 rows, chunk c of row r at place c ^ ((r >> 1) & 7). Rows and columns behind the last, and slabs,
+  // repeat it
+  unsigned xo[PA], wo[PB];
+  const int lr = lane >> 3, lc = 16 * ((lane & 7) ^ (4 * (w & 1) + (lane >> 4)));
+#pragma unroll
+  for (int i = 0; i < PA; ++i) xo[i] = (unsigned)min(8 * (i * NW + w) + lr, a.M - 1 - m0) * (unsigned)(2 * a.ldx) + lc;
+#pragma unroll
+  for (int i = 0; i < PB; ++i) {
+    const int r = 8 * (i * NW + w) + lr, c = min(column<GLU>(r), a.cols - 1 - n0);
+    wo[i] = (unsigned)(c + (GLU && (r & 16) ? a.half : 0)) * (unsigned)(2 * a.ldw) + lc;
+  }
+  const char* xb = reinterpret_cast<const char*>(a.x + m0 * a.ldx + first * BK);
+  const char* wb = reinterpret_cast<const char*>(a.w + n0 * a.ldw + first * BK);
+  const unsigned l0 = lds_base();
+  auto load_x = [&](int i, int slab, unsigned slot) { glds(xo[i], xb + min(slab, ns - 1) * ROW, l0 + slot + (i * NW + w) * 1024); };
+  auto load_w = [&](int i, int slab, unsigned slot) {
+    glds(wo[i], wb + min(slab, ns - 1) * ROW, l0 + X_LDS + slot + (i * NW + w) * 1024);
+  };
+
+  // ---- fragments: row (lane & 15) of a block, chunk 4 s + (lane >> 4) of step s
+  const int l16 = lane & 15, g = lane >> 4;
+  int ao[2], bo[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const int ch = 16 * ((4 * s + g) ^ ((lane >> 1) & 7));
+    ao[s] = (wr * RT * 16 + l16) * ROW + ch;
+    bo[s] = X_LDS + (wc * CT * 16 + l16) * ROW + ch;
+  }
+  auto read_x = [&](bf16x8& f, int s, int i, unsigned slot) { f = *reinterpret_cast<const bf16x8*>(tl::lds + ao[s] + slot + i * 16 * ROW); };
+  auto read_w = [&](bf16x8& f, int s, int j, unsigned slot) { f = *reinterpret_cast<const bf16x8*>(tl::lds + bo[s] + slot + j * 16 * ROW); };
+
+  f32x4 acc[RT][CT];
+  // a tile of fewer rows skips the products of the others
+  const int live = __builtin_amdgcn_readfirstlane(min(max((a.M - m0 - wr * RT * 16 + 15) / 16, 0), RT));
+  loop<T>(acc, ns, false, !rest, live, load_x, load_w, read_x, read_w);
+
+  if constexpr (SPLIT || GLU) {
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+      const int r = m0 + (wr * RT + i) * 16 + l16;
+      if (r >= a.M) continue;
+      if constexpr (SPLIT) {
+        float* p = a.part + ((int64_t)split * a.M + r) * (GLU ? 2 * a.cols : a.cols);
+#pragma unroll
+        for (int j = 0; j < CT; ++j) {
+          const int b = GLU ? (j >> 1) & 1 : j & 1, c = n0 + (GLU ? wc * CT * 8 : (wc * CT + (j & ~1)) * 16) + 8 * g + 4 * b;
+          if (c < a.cols) *reinterpret_cast<f32x4*>(p + c + (GLU && (j & 1) ? a.cols : 0)) = acc[i][j];
+        }
+      } else {
+        const int c = n0 + wc * CT * 8 + 8 * g;
+        if (c >= a.cols) continue;
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float x = acc[i][2 * (e >> 2)][e & 3];
+          v[e] = x * sigmoid(x) * acc[i][2 * (e >> 2) + 1][e & 3];
+        }
+        *reinterpret_cast<u32x4*>(a.y + (int64_t)r * a.cols + c) = u32x4{pack(v[0], v[1]), pack(v[2], v[3]), pack(v[4], v[5]), pack(v[6], v[7])};
+      }
+    }
+  } else {
+    float b[2][8] = {};
+    if (a.bias != nullptr)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) load8<DT::BF16>(a.bias + min(n0 + wc * CT * 16 + 32 * h + 8 * g, a.cols - 8), b[h]);
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+      u32x4 v[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          v[h][e] = pack(acc[i][2 * h + (e >> 1)][2 * (e & 1)] + b[h][2 * e], acc[i][2 * h + (e >> 1)][2 * (e & 1) + 1] + b[h][2 * e + 1]);
+      store_lines(a.y, a.cols, m0 + (wr * RT + i) * 16 + l16, a.M, n0 + wc * CT * 16, a.cols, v);
+    }
+  }
+}
+
+// y from the sums of the splits, 8 columns a thread
+template <bool GLU>
+__global__ void __launch_bounds__(256) sum_kernel(const float* __restrict__ part, const unsigned short* __restrict__ bias,
+                                                  unsigned short* __restrict__ y, int M, int cols, int splits) {
+  const int64_t row = GLU ? 2 * (int64_t)cols : cols, all = M * row;
+  const int per = cols / 8;
+  for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < (int64_t)M * per; i += gridDim.x * 256ll) {
+    const int64_t r = i / per;
+    const int c = 8 * (int)(i - r * per);
+    float v[8], u[8] = {};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = 0.f;
+    for (int s = 0; s < splits; ++s) {
+      const float* p = part + s * all + r * row + c;
+      float t[8];
+      load8<DT::F32>(p, t);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] += t[e];
+      if (GLU) {
+        load8<DT::F32>(p + cols, t);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) u[e] += t[e];
+      }
+    }
+    if (GLU) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] *= sigmoid(v[e]) * u[e];
+    } else if (bias != nullptr) {
+      load8<DT::BF16>(bias + c, u);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] += u[e];
+    }
+    store8<DT::BF16>(y + r * cols + c, v);
+  }
+}
+
+using T256 = Tile<2, 4, 8, 4, 2, 3, 2>;   // 256 x 256
+using T192 = Tile<2, 4, 6, 4, 2, 3, 2>;   // 192 x 256
+using T128 = Tile<2, 4, 4, 4, 3, 3, 2>;   // 128 x 256
+using N128 = Tile<2, 2, 4, 4, 2, 2, 2>;   // 128 x 128, two a CU
+
+// The tile and the splits of K that take least by this account: rounds of workgroups over the CUs, each a start (with the stores of a
+// round, which all its workgroups issue at once) and its slabs; a tile of the last, fewer rows takes 0.62 of a whole one's time and up.
+// us a slab and a start, fitted to 12 weights of 2048 x 2048 to 28672 x 4096 at 25 row counts from 40 to 14000: the choice is 1 %
+// behind the best on average. 256 x 128 and 192 x 128 were never the best.
+struct Form {
+  int bm, bn, at_once;
+  float slab, start;
+};
+constexpr Form kForms[4] = {{256, 256, 256, 1.42f, 9.f}, {192, 256, 256, 1.07f, 14.f}, {128, 256, 256, 0.95f, 3.f}, {128, 128, 512, 1.f, 3.f}};
+struct Plan {
+  int form, splits;
+  float us;
+};
+static Plan plan(int64_t M, int64_t N, int64_t slabs, bool may_split) {
+  Plan best{0, 1, 1e30f};
+  for (int f = 0; f < 4; ++f) {
+    const Form& t = kForms[f];
+    const int64_t cols = (N + t.bn - 1) / t.bn, rest = M % t.bm;
+    for (int s : {1, 2, 3, 4, 6, 8}) {
+      if (s > 1 && (!may_split || slabs < 4 * s || (M + t.bm - 1) / t.bm * cols * s > 600)) break;
+      const float part = 0.62f + 0.38f * rest / t.bm, one = (slabs + s - 1) / s * t.slab + t.start;
+      const int64_t whole = M / t.bm * cols * s, rounds = (whole + t.at_once - 1) / t.at_once;
+      const float idle = rounds * t.at_once - whole, more = rest ? cols * s - idle / part : 0.f;
+      float us = 4.f + rounds * one;
+      if (more > 0.f) us += part * one * std::ceil(more / t.at_once);
+      if (s > 1) us += 4.f + M * N * 4 * (2 * s + 0.5f) / 3.2e6f;
+      if (us < best.us) best = {f, s, us};
+    }
+  }
+  return best;
+}
+
+template <typename T, bool GLU>
+static void launch(Args a, int splits) {
+  constexpr int CB = GLU ? T::BN / 2 : T::BN;
+  a.tm = a.M / T::BM;
+  a.tn = (a.cols + CB - 1) / CB;
+  a.gm = std::max(1, std::min(a.tm, 8));
+  a.splits = splits;
+  const int64_t grid = ((int64_t)a.M + T::BM - 1) / T::BM * a.tn * splits;
+  SXE_CHECK(grid < (1ll << 30), "gemm_tn: too many tiles");
+  if (splits > 1) {
+    allow_lds<&gemm_kernel<T, GLU, true>>(T::LDS);
+    hipLaunchKernelGGL((gemm_kernel<T, GLU, true>), dim3((unsigned)grid), dim3(T::NTHR), T::LDS, cur_stream(), a);
+    hipLaunchKernelGGL(sum_kernel<GLU>, dim3(stream_grid((int64_t)a.M * a.cols / 8, 256)), dim3(256), 0, cur_stream(), a.part, a.bias, a.y,
+                       a.M, a.cols, splits);
+  } else {
+    allow_lds<&gemm_kernel<T, GLU, false>>(T::LDS);
+    hipLaunchKernelGGL((gemm_kernel<T, GLU, false>), dim3((unsigned)grid), dim3(T::NTHR), T::LDS, cur_stream(), a);
+  }
+  SXE_LAUNCH_CHECK();
+}
+
+}  // namespace tn
+
+// x [M, K] (rows may lie apart), w [N, K] (the same), bias [N] or none -> [M, N], glu: [M, N / 2]. tile, splits of K: -1, 0: the plan's
+at::Tensor gemm_tn(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, bool glu, int64_t tile, int64_t splits) {
+  check_beside(x, {w, bias});
+  SXE_CHECK(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 && x.dim() == 2 && w.dim() == 2 &&
+                x.size(1) == w.size(1), "gemm_tn: bf16 x [M, K], w [N, K]");
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0), cols = glu ? N / 2 : N;
+  SXE_CHECK(K > 0 && K % tn::BK == 0 && N > 0 && N % (glu ? 16 : 8) == 0, "gemm_tn: K in multiples of 64, columns of 8");
+  for (const at::Tensor* t : {&x, &w})
+    SXE_CHECK(t->size(0) <= 1 || (t->stride(0) % 8 == 0 && t->stride(0) >= 0), "gemm_tn: rows that start on 16 bytes");
+  SXE_CHECK(x.stride(1) == 1 && w.stride(1) == 1 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+                reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0, "gemm_tn: rows of neighbouring elements that start on 16 bytes");
+  const int64_t ldx = M > 1 ? x.stride(0) : K, ldw = N > 1 ? w.stride(0) : K;
+  SXE_CHECK(M < (1ll << 30) && N < (1ll << 30) && K < (1ll << 30) && 512 * ldx < (1ll << 32) && (glu ? 2 * N * ldw : 512 * ldw) < (1ll << 32),
+            "gemm_tn: sizes beyond 32-bit offsets");
+  const bool has_bias = bias.has_value() && bias->defined();
+  SXE_CHECK(!has_bias || (!glu && bias->scalar_type() == at::kBFloat16 && bias->dim() == 1 && bias->size(0) == N && bias->is_contiguous() &&
+                          reinterpret_cast<uintptr_t>(bias->data_ptr()) % 16 == 0), "gemm_tn: bias bf16 [N]");
+  SXE_CHECK(tile < 4 && splits >= 0 && splits <= 64, "gemm_tn: tile 0 - 3 or -1, splits 0 - 64");
+  c10::DeviceGuard g(x.device());
+  auto y = at::empty({M, cols}, x.options());
+  if (M == 0) return y;
+  tn::Args a{};
+  a.x = reinterpret_cast<const unsigned short*>(x.data_ptr());
+  a.w = reinterpret_cast<const unsigned short*>(w.data_ptr());
+  a.bias = has_bias ? reinterpret_cast<const unsigned short*>(bias->data_ptr()) : nullptr;
+  a.y = reinterpret_cast<unsigned short*>(y.data_ptr());
+  a.ldx = ldx;
+  a.ldw = ldw;
+  a.M = M;
+  a.cols = cols;
+  a.half = cols;
+  a.slabs = K / tn::BK;
+  if (tile < 0) {
+    const tn::Plan p = tn::plan(M, N, a.slabs, splits != 1);
+    tile = p.form;
+    if (splits == 0) splits = p.splits;
+  }
+  splits = std::max<int64_t>(1, splits);
+  a.per = (a.slabs + splits - 1) / splits;
+  const int parts = (a.slabs + a.per - 1) / a.per;  // none of them empty
+  at::Tensor part;
+  if (parts > 1) {
+    part = at::empty({parts, M, N}, x.options().dtype(at::kFloat));
+    a.part = part.data_ptr<float>();
+  }
+  auto run = [&](auto t) {
+    using T = decltype(t);
+    glu ? tn::launch<T, true>(a, parts) : tn::launch<T, false>(a, parts);
+  };
+  switch (tile) {
+    case 0: run(tn::T256{}); break;
+    case 1: run(tn::T192{}); break;
+    case 2: run(tn::T128{}); break;
+    default: run(tn::N128{});
+  }
+  return y;
+}
+
+}  // namespace sxe
+
+TORCH_LIBRARY_FRAGMENT(sxe, m) {
+  m.def("gemm_tn(Tensor x, Tensor w, Tensor? bias, bool glu, int tile=-1, int splits=0) -> Tensor");
+}
+TORCH_LIBRARY_IMPL(sxe, CUDA, m) { m.impl("gemm_tn", &sxe::gemm_tn); }

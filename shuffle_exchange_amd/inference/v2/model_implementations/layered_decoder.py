@@ -283,8 +283,9 @@ ARCHITECTURES = {"Tobinex": (_tobinex_spec, _tobinex_weights), "Bipotar": (_bipo
 
 
 # csrc/kernels sources a checkout with nothing built compiles to serve an architecture
-SERVING_UNITS = {"Tobinex": ("act", "mix_attn", "residual_norm", "skinny_gemm"),
-                 "Bipotar": ("act", "experts", "grouped_gemm", "latent_attn", "linear_attn", "residual_norm", "skinny_gemm")}
+SERVING_UNITS = {"Tobinex": ("act", "gemm_tn", "mix_attn", "residual_norm", "skinny_gemm", "stream_gemm"),
+                 "Bipotar": ("act", "experts", "gemm_tn", "grouped_gemm", "latent_attn", "linear_attn", "residual_norm", "skinny_gemm",
+                             "stream_gemm")}
 
 
 def ensure_library(path):

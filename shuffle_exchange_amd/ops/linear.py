@@ -126,6 +126,56 @@ def glu_linear(x, weight):
     return torch.ops.sxe.stream_gemm(x, w, sc, None, True)
 
 
+# Many rows: csrc/kernels/gemm_tn.hip, 2048 x 2048 to 28672 x 4096, us, library / here. The library's kernels fit whole tiles of 256 rows
+# (8192 rows, 28672 x 4096 1255 / 1285, 4096 x 4096 174 / 184, 4096 x 14336 604 / 630) and fall off at others: 4500 rows, 4096 x 14336
+# 759 / 417, 7300 rows 962 / 596, 5120 x 3072 239 / 191, 9000 rows, 4096 x 4096 338 / 220; at their best 6500 rows, 6144 x 4096 241 / 253,
+# 13000 rows, 3072 x 8192 454 / 504: 5 % less time on average from 1500 rows on. Below, long rows of the weight pay, whose products
+# are split along them: 40 rows, 2048 x 8192 23 / 17, 4096 x 14336 33 / 32, 240 rows 55 / 42, 1100 rows 141 / 114; others do not:
+# 600 rows, 5120 x 3072 26 / 29, 4096 x 4096 28 / 31.
+TILED_ROWS = 1500
+# SwiGLU of the products in one launch, us, product and activation / here: 16384 x 2048, 330 rows 35 / 29, 2100 rows 144 / 112;
+# 28672 x 4096, 330 rows 85 / 73, 1040 rows 226 / 200, 7588 rows 1390 / 1250; but 240 rows of 16384 x 3072 38 / 43, 72 of 28672 x 4096
+# 59 / 67
+TILED_GLU_ROWS = 300
+
+
+def _tiled_faster(rows, N, K):
+    if N < 2048 or K < 2048:
+        return False
+    return rows % 256 != 0 if rows >= TILED_ROWS else STREAM_ROWS_SMALL < rows and K >= 8192 and N <= K
+
+
+def _tileable(x2, weight, bias=None):
+    """The operands that gemm_tn.hip reads: rows of whole 128-byte pieces that start on 16 bytes, offsets in 32 bits."""
+    N, K = weight.shape
+    return (x2.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.is_cuda and x2.stride(1) == 1 and weight.stride(1) == 1
+            and x2.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0 and x2.stride(0) >= K and weight.stride(0) >= K and x2.data_ptr() % 16 == 0
+            and weight.data_ptr() % 16 == 0 and x2.shape[1] == K and K % 64 == 0 and N % 16 == 0 and x2.shape[0] < 1 << 30
+            and x2.stride(0) < 1 << 23 and N * weight.stride(0) < 1 << 31
+            and (bias is None or (_bias_ok(bias, weight) and bias.data_ptr() % 16 == 0)))
+
+
+def _tiled(x, weight, bias):
+    if weight.dim() != 2 or not _tiled_faster(x.numel() // max(1, x.shape[-1]), *weight.shape):
+        return None
+    x2 = x.reshape(-1, x.shape[-1])
+    if not _tileable(x2, weight, bias):
+        return None
+    native.require_hip()
+    return torch.ops.sxe.gemm_tn(x2, weight, bias, False).view(*x.shape[:-1], weight.shape[0])
+
+
+def glu_tiled(x, weight):
+    """silu(gate) * up of ``linear(x, weight)`` with weight = [gate | up], bf16, in ONE launch (gemm_tn.hip): many rows, no autograd; None
+    where the product and the activation's launch are the better or only form. One rounding, of the result."""
+    if (not isinstance(weight, torch.Tensor) or weight.dim() != 2 or x.dim() != 2 or not x.is_cuda or x.requires_grad or not native.plain(x, weight)
+            or x.shape[0] <= TILED_GLU_ROWS or weight.shape[0] < 8192 or weight.shape[1] < 2048 or not _tileable(x, weight)
+            or torch.is_autocast_enabled("cuda")):
+        return None
+    native.require_hip()
+    return torch.ops.sxe.gemm_tn(x, weight, None, True)
+
+
 def _pro_weight(weight):
     """(w, scale) for the fused-prologue skinny kernels: a bf16 [N, K] tensor or an FP8Weight."""
     if isinstance(weight, torch.Tensor):
@@ -517,12 +567,15 @@ def linear(x, weight, bias=None):
     grad = torch.is_grad_enabled() and (weight.requires_grad or x.requires_grad or (bias is not None and bias.requires_grad))
     if grad and weight.requires_grad and hasattr(weight, "_sxe_grad_target"):
         return _Linear.apply(x, weight, bias)
-    if (not grad and SKINNY_MAX_M > 0 and x.is_cuda and x.numel() <= max(SKINNY_MAX_M, STREAM_ROWS_SMALL) * x.shape[-1]
+    if (not grad and SKINNY_MAX_M > 0 and x.is_cuda
             and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == torch.bfloat16)
             and native.plain(x, weight, bias)):
-        y = _skinny(x, weight, bias)
-        if y is None:
-            y = _stream(x, weight, bias)
+        if x.numel() <= max(SKINNY_MAX_M, STREAM_ROWS_SMALL) * x.shape[-1]:
+            y = _skinny(x, weight, bias)
+            if y is None:
+                y = _stream(x, weight, bias)
+        else:
+            y = _tiled(x, weight, bias)
         if y is not None:
             return y
     return F.linear(x, weight, bias)

@@ -1,0 +1,91 @@
+"""Products of many rows (csrc/kernels/gemm_tn.hip) against 64 bits, and the calls of ops/linear.py that take them."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _native():
+    from shuffle_exchange_amd.ops import native
+    native.require_hip()
+
+
+def _operands(M, N, K, apart=0):
+    g = torch.Generator("cuda").manual_seed(M + 3 * N + 7 * K)
+    x = torch.randn(M, K + apart, device="cuda", generator=g).bfloat16()[:, :K]
+    w = (torch.randn(N, K + 2 * apart, device="cuda", generator=g) * K ** -0.5).bfloat16()[:, :K]
+    return x, w, torch.randn(N, device="cuda", generator=g).bfloat16()
+
+
+def _close(y, ref, x, w, factor=1.0):
+    """One rounding to bf16 (2^-9) of fp32 sums of K exact products (each off by at most K 2^-24 of the magnitudes' sum)."""
+    assert y.dtype == torch.bfloat16 and y.shape == ref.shape
+    sums = x.double().abs() @ w.double().abs().t() * x.shape[1] * 2.0 ** -24
+    bound = ref.abs() * 2.0 ** -8 + (sums if sums.shape == ref.shape else sums.amax()) * factor + 1e-30
+    assert bool(((y.double() - ref).abs() <= bound).all())
+
+
+# tiles: 256 x 256, 192 x 256, 128 x 256, 128 x 128, the plan's. Rows around a tile and its 16-row blocks, columns that end inside
+# a store's 8, a lane's 32 and a tile's 256, one slab of K to more than the slots hold
+@pytest.mark.parametrize("tile", [0, 1, 2, 3, -1])
+@pytest.mark.parametrize("splits", [1, 3, 0])
+@pytest.mark.parametrize("M,N,K,apart", [(1, 8, 64, 0), (15, 40, 128, 8), (128, 264, 192, 0), (193, 256, 320, 16), (257, 520, 64, 0),
+                                         (385, 1000, 640, 8), (512, 272, 1024, 0)])
+def test_products(M, N, K, apart, splits, tile):
+    x, w, b = _operands(M, N, K, apart)
+    ref = x.double() @ w.double().t()
+    _close(torch.ops.sxe.gemm_tn(x, w, None, False, tile, splits), ref, x, w)
+    _close(torch.ops.sxe.gemm_tn(x, w, b, False, tile, splits), ref + b.double(), x, w, 2.0)
+    if N % 16 == 0:
+        gate, up = ref.chunk(2, 1)
+        # both sums' errors through silu(gate) up: |silu'| <= 1.1, values up to about 6
+        _close(torch.ops.sxe.gemm_tn(x, w, None, True, tile, splits), F.silu(gate) * up, x, w, 16.0)
+
+
+def test_infinities_and_nan_stay_in_their_rows():
+    x, w, _ = _operands(300, 512, 256)
+    x[7, 3], x[299, 0] = float("inf"), float("nan")
+    for glu in (False, True):
+        y = torch.ops.sxe.gemm_tn(x, w, None, glu)
+        bad = ~torch.isfinite(y).all(1)
+        assert bad.nonzero().flatten().tolist() == [7, 299] and bool(torch.isnan(y[299]).all())
+
+
+@pytest.mark.parametrize("M,N,K,taken", [(1536, 2048, 2048, False), (1537, 2048, 2048, True), (1537, 2040, 2048, False), (300, 2048, 8192, True),
+                                         (33, 2048, 8192, True), (300, 4096, 4096, False)])
+def test_linear_takes_them(M, N, K, taken, monkeypatch):
+    from shuffle_exchange_amd.ops import linear as L
+    x, w, b = _operands(M, N, K)
+    seen = []
+    tiled = L._tiled
+    monkeypatch.setattr(L, "_tiled", lambda *a: seen.append(tiled(*a)) or seen[-1])
+    with torch.no_grad():
+        y = L.linear(x.view(1, M, K), w, b)
+        assert (seen[-1] is not None) == taken
+        _close(y[0], x.double() @ w.double().t() + b.double(), x, w, 2.0)
+        # what the kernel does not read goes where it went before: rows apart by no whole 16 bytes, another type
+        odd = torch.randn(M, K + 4, device="cuda").bfloat16()[:, :K]
+        assert torch.equal(L.linear(odd, w), F.linear(odd, w)) and seen[-1] is None
+        with torch.autocast("cuda", torch.float16):
+            assert L.linear(x, w).dtype == torch.float16
+    n = len(seen)
+    assert L.linear(x.requires_grad_(), w).requires_grad and len(seen) == n
+
+
+def test_captured():
+    """Replays with new inputs; the splits' sums are the graph's own memory."""
+    x, w, _ = _operands(300, 2048, 8192)
+    from shuffle_exchange_amd.ops.linear import linear
+    with torch.no_grad():
+        linear(x, w)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = linear(x, w)
+        for seed in range(3):
+            x.copy_(torch.randn(300, 8192, device="cuda", generator=torch.Generator("cuda").manual_seed(seed)).bfloat16())
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, linear(x, w))
