@@ -6,25 +6,21 @@
 // Reference: inference/v2/kernels/cutlass_ops/moe_gemm/moe_gemm.cu (grouped GEMM over expert-sorted rows). experts_kn.hip has the
 // streaming form for few rows an expert.
 //
-// What bounds it: the matrix cores, fed from LDS. A workgroup takes 256 rows of one expert and 2 x 128 columns (128 of gate and the
-// same of up, whose sums meet in a lane's registers), eight waves of 128 rows x (32 + 32) columns, fp32 sums in registers. Slabs of
-// 32 k (32 KB) arrive by direct loads in a ring of five, four ahead; x rows are gathered on the way. x is read from LDS as it
-// lies, W transposed (ds_read_b64_tr_b16). The two groups of four waves (rows 0 - 127 and the rest, one wave of each on a SIMD)
-// run one barrier apart, with a barrier behind either of a slab's two steps of eight products a wave, so that one group's waits
-// and reads lie under the other's products: 8 experts of 2048 rows, 4096 x 14336, ms of both products 5.9 in step, 5.5 so;
-// ring depth (4 or 5) and the order of loads and reads are within 2 %. The row tiles of an expert and column block run side by
-// side on one XCD, so W comes from memory once. Waves whose 128 rows lie past the expert's rows run no products. 5.5 ms are 1.05
-// PFLOP/s at about 1.9 GHz, matrix cores busy for a good half of the time, no LDS bank conflicts.
+// What bounds it: as in gemm_tn.hip, whose loop this is (sxe_gemm_loop.h). A workgroup takes 256 rows of one expert (128 where the
+// experts have few) and 256 columns (128 of gate and the same of up, whose sums meet in a lane's registers), eight waves of 128 rows
+// x 64 columns (32 + 32). x rows are gathered on the way and read from LDS as they lie, slabs of 64 k rows of W transposed
+// (ds_read_b64_tr_b16). The row tiles of an expert and column block run side by side on one XCD, so W comes from memory once. Blocks
+// of 16 rows past the expert's rows run no products. us, before (32-k slabs, products of 32 x 32 x 16, ring of five) / here: 8 experts of
+// 2048 rows, 4096 x 2 x 14336 3620 / 2991, 14336 x 4096 1911 / 1611 (1.29 PFLOP/s); of 800 rows 1628 / 1358, 785 / 661.
 #include "sxe_common.h"
-#include "sxe_tile.h"
+#include "sxe_gemm_loop.h"
 #include <torch/library.h>
 
 namespace sxe {
 namespace kt {
-using namespace mf;
+using namespace gl;
 
-constexpr int BM = 256, HC = 128, BK = 32, RING = 5, AHEAD = 4, NTHR = 512;
-constexpr int A_BYTES = BM * BK * 2, H_BYTES = BK * HC * 2, SLOT = A_BYTES + 2 * H_BYTES;  // 16 KB, 8 KB, 32 KB: the ring is all 160 KB of LDS
+constexpr int WROW = 512;  // bytes of a slab's k row: 256 columns
 
 struct Args {
   const unsigned short* x;
@@ -38,21 +34,24 @@ struct Args {
   int cols, half;    // columns of y; column of W that goes with column 0 in the second half of a tile
 };
 
+template <int BM>
 __device__ __forceinline__ int tiles_of(const Args& a, int e) {
   if (e >= a.E) return 0;
   const int lo = min(max(a.offs[e], 0), a.R), hi = min(max(a.offs[e + 1], 0), a.R);
   return hi > lo ? (hi - lo + BM - 1) / BM : 0;
 }
 
-template <bool GLU>
-__global__ void __launch_bounds__(NTHR, 2) tile_kernel(Args a) {
-  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wr = w >> 2, wc = w & 3;
+template <typename T, bool GLU>
+__global__ void __launch_bounds__(T::NTHR, T::WAVES) tile_kernel(Args a) {
+  constexpr int RT = T::RT, CT = T::CT, NW = T::NW, PA = T::PA, PB = T::PB, BM = T::BM, X_LDS = T::SA * T::AS, HC = T::BN / 2;
+  static_assert(T::BN == 256 && NW == 8 && PB == 4);
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wr = w / T::WC, wc = w % T::WC;
   // ---- block -> (expert, column block, row tile), row tiles fastest, consecutive ones on one XCD
   constexpr int CB = GLU ? HC : 2 * HC;
   const int tn = (a.cols + CB - 1) / CB;
   int total = 0;
   for (int e0 = 0; e0 < a.E; e0 += 64) {
-    int t = tiles_of(a, e0 + lane);
+    int t = tiles_of<BM>(a, e0 + lane);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
     total += t;
@@ -65,7 +64,7 @@ __global__ void __launch_bounds__(NTHR, 2) tile_kernel(Args a) {
   {
     int before = 0;
     for (int e0 = 0; e0 < a.E; e0 += 64) {
-      const int t = tiles_of(a, e0 + lane);
+      const int t = tiles_of<BM>(a, e0 + lane);
       int inc = t;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
@@ -89,114 +88,86 @@ __global__ void __launch_bounds__(NTHR, 2) tile_kernel(Args a) {
   const int r0 = min(max(a.offs[expert], 0), a.R) + rt * BM, r1 = min(max(a.offs[expert + 1], 0), a.R);
   const int n0 = nt * CB;
 
-  // ---- loads of a slab: wave w brings rows 16 w .. and 128 + 16 w .. of x, k rows 4 w .. of both halves of W
-  const unsigned short* xp[2];
+  // ---- loads: 8 rows of x, chunk c of row r at place c ^ ((r >> 1) & 7); 2 k rows of W, chunk c of row k at place
+  // c ^ (4 (k & 3) + 2 ((k >> 3) & 1)). Slabs behind the last repeat it; the second half of one with 32 k repeats its first
+  const int ns = a.K / BK, last = (a.K + BK - 1) / BK - 1;
+  const bool half = a.K % BK != 0;
+  unsigned xo[PA], wo[2], x_half;
+  {
+    const int c = (lane & 7) ^ (4 * (w & 1) + (lane >> 4));
+    x_half = 16 * (c & 4);
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int r = min(r0 + 128 * i + 16 * w + (lane >> 2), r1 - 1);
-    const int64_t row = a.token != nullptr ? min(max(a.token[r], 0), a.X - 1) : r;
-    xp[i] = a.x + row * a.ldx + 8 * ((lane & 3) ^ ((lane >> 4) & 3));
-  }
-  const unsigned short* wp[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < PA; ++i) {
+      const int r = min(r0 + 8 * (i * NW + w) + (lane >> 3), r1 - 1);
+      const int row = a.token != nullptr ? min(max(a.token[r], 0), a.X - 1) : r - r0;
+      xo[i] = (unsigned)row * (unsigned)(2 * a.ldx) + 16 * c;
+    }
+    const int k = 2 * w + (lane >> 5), p = (lane & 31) ^ (4 * (k & 3) + 2 * ((k >> 3) & 1));
     // a chunk past y's columns repeats the last ones (multiples of 8): its sums are not stored
-    const int c = n0 + (GLU ? 0 : i * HC) + 8 * ((lane & 15) ^ ((lane >> 4) << 2));
-    wp[i] = a.w + ((int64_t)expert * a.K + 4 * w + (lane >> 4)) * a.N + min(c, a.cols - 8) + (GLU ? i * a.half : 0);
+    const int col = GLU ? min(n0 + 8 * (p & 15), a.cols - 8) + (p >= 16 ? a.half : 0) : min(n0 + 8 * p, a.cols - 8);
+    wo[0] = (unsigned)k * (unsigned)(2 * a.N) + 2 * col;
+    wo[1] = wo[0] + (unsigned)(32 * a.N);  // 16 k rows on
   }
-  char* lds = tl::lds;
-  auto load = [&](int slab, int slot) {
-    char* d = lds + slot * SLOT;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) tl::glds16(xp[i] + slab * BK, d + (i * 8 + w) * 1024);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) tl::glds16(wp[i] + (int64_t)slab * BK * a.N, d + A_BYTES + i * H_BYTES + w * 1024);
+  const char* xb = reinterpret_cast<const char*>(a.token != nullptr ? a.x : a.x + r0 * a.ldx);
+  const char* wb = reinterpret_cast<const char*>(a.w + (int64_t)expert * a.K * a.N);
+  const unsigned l0 = lds_base();
+  auto load_x = [&](int i, int slab, unsigned slot) {
+    slab = min(slab, last);
+    glds(xo[i] - (half && slab == last ? x_half : 0), xb + slab * 128, l0 + slot + (i * NW + w) * 1024);
+  };
+  auto load_w = [&](int i, int slab, unsigned slot) {
+    slab = min(slab, last);
+    const int k = slab * BK + (half && slab == last ? 0 : 32 * (i >> 1));
+    glds(wo[i & 1], wb + (int64_t)k * (2 * a.N), l0 + X_LDS + slot + (i * NW + w) * 1024);
   };
 
-  // ---- fragment offsets: x row (lane & 31), chunk 2 s + h; W column 32 wc + (lane & 31), k rows 8 h .. + 7 of a step
-  const int l32 = lane & 31, h = lane >> 5;
-  int ao[2];
+  // ---- fragments: row (lane & 15) of a block of x, chunk 4 s + (lane >> 4) of step s; W: four columns of four k rows a lane,
+  // 8 (lane >> 4) .. and the next four, of which the transposing read makes eight k of one column
+  const int l16 = lane & 15, g = lane >> 4, q = l16 >> 2, p = l16 & 3;
+  int ao[2], bo[CT];
 #pragma unroll
-  for (int s = 0; s < 2; ++s) ao[s] = (wr * 128 + l32) * (BK * 2) + 16 * ((2 * s + h) ^ ((lane >> 2) & 3));
-  const int g = lane >> 4, i16 = lane & 15, q = i16 >> 2, p = i16 & 3;
-  const int bo = A_BYTES + (8 * h + q) * (HC * 2) + 16 * ((4 * wc + 2 * (g & 1) + (p >> 1)) ^ (q << 2)) + 8 * (p & 1);
-
-  f32x16 acc[4][2];
+  for (int s = 0; s < 2; ++s) ao[s] = (wr * RT * 16 + l16) * 128 + 16 * ((4 * s + g) ^ ((lane >> 1) & 7));
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-  bf16x8 fa[2][4], fb[2][2];
-  auto read = [&](int slot, int s) {
-    const char* b = lds + slot * SLOT;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) fa[s][i] = *reinterpret_cast<const bf16x8*>(b + ao[s] + i * 32 * BK * 2);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int o = bo + j * H_BYTES + s * 16 * HC * 2;
-      const i16x4 lo = lds_tr(b, o), hi = lds_tr(b, o + 4 * HC * 2);
-      fb[s][j] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-    }
-  };
-  const bool live = r0 + wr * 128 < r1;
-  auto multiply = [&](int s) {
-    if (!live) return;
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[s][i], fb[s][j], acc[i][j], 0, 0, 0);
-    __builtin_amdgcn_s_setprio(0);
+  for (int j = 0; j < CT; ++j) {
+    const int ch = GLU ? 4 * wc + 2 * (j & 1) + 16 * (j >> 1) : 8 * wc + 2 * j;
+    bo[j] = X_LDS + (8 * g + q) * WROW + 16 * ((ch + (p >> 1)) ^ (4 * q + 2 * (g & 1))) + 8 * (p & 1);
+  }
+  auto read_x = [&](bf16x8& f, int s, int i, unsigned slot) { f = *reinterpret_cast<const bf16x8*>(tl::lds + ao[s] + slot + i * 2048); };
+  auto read_w = [&](bf16x8& f, int s, int j, unsigned slot) {
+    const int o = bo[j] + slot + s * 32 * WROW;
+    const i16x4 lo = lds_tr(tl::lds, o), hi = lds_tr(tl::lds, o + 4 * WROW);
+    f = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
 
-  const int ns = a.K / BK;
+  f32x4 acc[RT][CT];
+  const int live = __builtin_amdgcn_readfirstlane(min(max((r1 - r0 - wr * RT * 16 + 15) / 16, 0), RT));
+  loop<T>(acc, ns, half, r1 - r0 >= BM, live, load_x, load_w, read_x, read_w);
+
+  // two blocks' four columns a lane -> eight of one: lanes of odd groups of 16 take the second block
+  auto pair = [&](const float (&u)[4], const float (&v)[4]) {
+    const auto lo = __builtin_amdgcn_permlane16_swap(pack(u[0], u[1]), pack(v[0], v[1]), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(pack(u[2], u[3]), pack(v[2], v[3]), false, false);
+    return u32x4{lo[0], hi[0], lo[1], hi[1]};
+  };
 #pragma unroll
-  for (int j = 0; j < AHEAD; ++j) load(min(j, ns - 1), j);
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * (AHEAD - 2)) : "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-  read(0, 0);
-  if (wr == 1) __builtin_amdgcn_s_barrier();  // one barrier behind the other group from here on
-  for (int s0 = 0; s0 < ns; s0 += RING) {
+  for (int i = 0; i < RT; ++i) {
+    const int r = r0 + (wr * RT + i) * 16 + l16;
+    float v[CT][4];
 #pragma unroll
-    for (int j = 0; j < RING; ++j) {
-      if (s0 + j >= ns) break;
-      read(j, 1);
-      multiply(0);
-      // this wave's part of slab s + 2 has landed and all of slab s is in its registers. So behind the barrier slab s + 1 is
-      // there, also the part of the group that is a barrier behind, and nobody reads slab s - 1 any more
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(4 * (AHEAD - 3)) : "memory");
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
-      load(min(s0 + j + AHEAD, ns - 1), (j + AHEAD) % RING);  // over slab s - 1 (past the end: the last slab again)
-      read((j + 1) % RING, 0);
-      multiply(1);
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
+    for (int j = 0; j < (GLU ? 2 : CT); ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[j][e] = GLU ? acc[i][j][e] * sigmoid(acc[i][j][e]) * acc[i][j + 2][e] : acc[i][j][e];
+#pragma unroll
+    for (int h = 0; h < (GLU ? 1 : 2); ++h) {
+      const int c = n0 + (GLU ? 32 * wc : 64 * wc + 32 * h) + 16 * (g & 1) + 8 * (g >> 1);
+      const u32x4 out = pair(v[2 * h], v[2 * h + 1]);
+      if (r < r1 && c < a.cols) *reinterpret_cast<u32x4*>(a.y + (int64_t)r * a.cols + c) = out;
     }
   }
-  if (wr == 0) __builtin_amdgcn_s_barrier();  // as many as the other group
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int r = r0 + wr * 128 + 32 * i + (e & 3) + 8 * (e >> 2) + 4 * h;
-      if (r >= r1) continue;
-      unsigned short* yp = a.y + (int64_t)r * a.cols;
-      const int c = n0 + 32 * wc + l32;
-      if constexpr (GLU) {
-        const float v = acc[i][0][e];
-        if (c < a.cols) yp[c] = f32_to_bf16(v / (1.f + expf(-v)) * acc[i][1][e]);
-      } else {
-        if (c < a.cols) yp[c] = f32_to_bf16(acc[i][0][e]);
-        if (c + HC < a.cols) yp[c + HC] = f32_to_bf16(acc[i][1][e]);
-      }
-    }
 }
+
+using T256 = Tile<2, 4, 8, 4, 2, 3, 2>;
+using T128 = Tile<2, 4, 4, 4, 3, 3, 2>;
 
 static Args args(const at::Tensor& x, const at::Tensor& w, const at::Tensor& offs) {
   SXE_CHECK_CUDA(x);
@@ -204,10 +175,11 @@ static Args args(const at::Tensor& x, const at::Tensor& w, const at::Tensor& off
                 w.dim() == 3 && w.is_contiguous() && w.size(1) == x.size(1), "expert tile product: bf16 x [T, K], w [E, K, N]");
   SXE_CHECK(offs.is_cuda() && offs.is_contiguous() && offs.scalar_type() == at::kInt && offs.numel() == w.size(0) + 1,
             "expert tile product: offs int32 [E + 1]");
-  SXE_CHECK(w.size(1) > 0 && w.size(1) % BK == 0 && w.size(2) > 0 && w.size(2) % 16 == 0 && w.size(0) > 0 && w.size(1) < (1 << 30) &&
+  SXE_CHECK(w.size(1) > 0 && w.size(1) % 32 == 0 && w.size(2) > 0 && w.size(2) % 16 == 0 && w.size(0) > 0 && w.size(1) < (1 << 30) &&
                 w.size(2) < (1 << 30) && x.size(0) < (1ll << 31) && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
                 reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0,
             "expert tile product: K in multiples of 32, N of 16, 16-byte aligned operands");
+  SXE_CHECK(w.size(1) < (1 << 23) && w.size(2) < (1 << 26), "expert tile product: sizes beyond 32-bit offsets");
   Args a{};
   a.x = reinterpret_cast<const unsigned short*>(x.data_ptr());
   a.ldx = x.size(1);
@@ -220,15 +192,29 @@ static Args args(const at::Tensor& x, const at::Tensor& w, const at::Tensor& off
   return a;
 }
 
+template <typename T, bool GLU>
+static void launch(const Args& a) {
+  constexpr int CB = GLU ? T::BN / 2 : T::BN;
+  // every expert may end in a part of a tile
+  const int64_t grid = ((int64_t)a.R / T::BM + std::min(a.E, a.R)) * ((a.cols + CB - 1) / CB);
+  SXE_CHECK(grid < (1ll << 31), "expert tile product: too many tiles");
+  allow_lds<&tile_kernel<T, GLU>>(T::LDS);
+  hipLaunchKernelGGL((tile_kernel<T, GLU>), dim3((unsigned)grid), dim3(T::NTHR), T::LDS, cur_stream(), a);
+  SXE_LAUNCH_CHECK();
+}
+// 128 rows a tile where few column blocks make few rounds of workgroups over the CUs and theirs are the shorter ones (a round of 128 rows
+// takes 0.67 of one of 256). Products with h, us, 256 / 128: 4096 columns of 14336 k, 150 rows an expert of eight 271 / 233, 250
+// 318 / 382, 400 581 / 407, 800 661 / 768; 2048 of 8192, 250 170 / 118, 550 187 / 203. Many column blocks: 28672 of 4096 k, 50 rows
+// 379 / 364, 150 403 / 508, 800 1358 / 1481
 template <bool GLU>
 static void launch(const Args& a) {
-  constexpr int CB = GLU ? HC : 2 * HC;
-  // every expert may end in a part of a tile
-  const int64_t grid = ((int64_t)a.R / BM + std::min(a.E, a.R)) * ((a.cols + CB - 1) / CB);
-  SXE_CHECK(grid < (1ll << 31), "expert tile product: too many tiles");
-  allow_lds<&tile_kernel<GLU>>(RING * SLOT);
-  hipLaunchKernelGGL(tile_kernel<GLU>, dim3((unsigned)grid), dim3(NTHR), RING * SLOT, cur_stream(), a);
-  SXE_LAUNCH_CHECK();
+  const int64_t blocks = (a.cols + (GLU ? 127 : 255)) / (GLU ? 128 : 256);
+  auto rounds = [&](int64_t bm) {
+    const int64_t tiles = a.R < bm * a.E ? a.E : a.R / bm + a.E / 2;
+    return (tiles * blocks + kNumCUs - 1) / kNumCUs;
+  };
+  if (blocks <= 32 && 2 * rounds(128) <= 3 * rounds(256)) launch<T128, GLU>(a);
+  else launch<T256, GLU>(a);
 }
 
 }  // namespace kt
@@ -240,7 +226,7 @@ at::Tensor expert_swiglu_kn_tile(const at::Tensor& x, const at::Tensor& w, const
             "expert_swiglu_kn_tile: token int32 [R]");
   auto h = at::empty({token.numel(), w.size(2) / 2}, x.options());
   if (token.numel() == 0) return h;
-  SXE_CHECK(x.size(0) > 0, "expert_swiglu_kn_tile: rows without tokens");
+  SXE_CHECK(x.size(0) > 0 && x.numel() < (1ll << 31), "expert_swiglu_kn_tile: rows without tokens, or x beyond 32-bit offsets");
   c10::DeviceGuard g(x.device());
   a.token = token.data_ptr<int>();
   a.R = token.numel();

@@ -324,11 +324,12 @@ def expert_mlp(h, routing, up, down, act="relu2"):
 
 
 # ---------------------------------------------------- routed SwiGLU experts, weights [E, K, N] as trained
-# Mean rows per expert up to which the streaming kernels are used. One layer of 8 experts, top 2, us streaming / tiles / a library
-# product per expert (with its row counts read back): 4096 x 14336: 32 rows 619 / 635 / 973, 64: 879 / 683 / 1087, 128: 1458 /
-# 788 / 1232, 775: - / 2205 / 2776, 2048: - / 5563 / 5799; 2048 x 8192: 32: 204 / 243 / 500, 64: 300 / 259 / 519, 775: - / 734 /
-# 1101, 2048: - / 1752 / 2001; 3072 x 8192: 32: 293 / 295 / 555.
-KN_ROWS = 40
+# Mean rows per expert up to which the streaming kernels are used; 0.4 of it where an expert has more than KN_LARGE gate | up weights:
+# there the tiles read them at the memory's rate, too. One layer of 8 experts, top 2, us streaming / tiles: 4096 x 14336, 12 rows
+# 528 / 540, 20: 570 / 545, 32: 594 / 549, 64: 916 / 570; 3072 x 8192, 12: 244 / 255, 20: 270 / 258, 40: 291 / 262; 2048 x 8192, 12:
+# 165 / 203, 32: 192 / 208, 50: 211 / 214, 64: 277 / 215. A library product per expert (with its row counts read back), 4096 x 14336:
+# 32: 973, 775: 2776 / 1975, 2048: 5799 / 4700.
+KN_ROWS, KN_LARGE = 40, 1 << 25
 
 
 def swiglu_experts_ok(x, w_gate_up, w_down):
@@ -336,7 +337,7 @@ def swiglu_experts_ok(x, w_gate_up, w_down):
     return (_hip(x) and x.dtype == torch.bfloat16 and w_gate_up.is_cuda and w_gate_up.dtype == torch.bfloat16
             and w_down.dtype == torch.bfloat16 and w_gate_up.is_contiguous() and w_down.is_contiguous()
             and w_gate_up.shape[1] % 32 == 0 and w_gate_up.shape[2] % 128 == 0 and w_down.shape[1] % 32 == 0 and w_down.shape[2] % 128 == 0
-            and w_gate_up.shape[0] <= 1024 and w_gate_up.data_ptr() % 16 == 0 and w_down.data_ptr() % 16 == 0)
+            and w_gate_up.shape[0] <= 1024 and x.numel() < 1 << 31 and w_gate_up.data_ptr() % 16 == 0 and w_down.data_ptr() % 16 == 0)
 
 
 def swiglu_experts(x, routing, w_gate_up, w_down):
@@ -347,7 +348,7 @@ def swiglu_experts(x, routing, w_gate_up, w_down):
     rows, _, slots, offs, active = routing.lists
     x = x.contiguous()
     E, R = w_gate_up.shape[0], rows.numel()
-    if R <= KN_ROWS * E:
+    if R <= KN_ROWS * E * (0.4 if w_gate_up.shape[1] * w_gate_up.shape[2] > KN_LARGE else 1):
         h = torch.ops.sxe.expert_swiglu_kn(x, w_gate_up, offs, active, rows)
         return torch.ops.sxe.expert_down_kn(h, w_down, offs, active, slots, routing.weight)
     h = torch.ops.sxe.expert_swiglu_kn_tile(x, w_gate_up, offs, rows)
