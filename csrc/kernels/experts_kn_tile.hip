@@ -1,7 +1,8 @@
-// Expert products of prefill on gfx950, weights [E, K, N] as they are trained: rows sorted by expert, one launch for all experts,
+// Expert products of prefill and training on gfx950, weights [E, K, N] as they are trained: rows sorted by expert, one launch for all experts,
 // row counts read on the device.
 //   expert_swiglu_kn_tile  h[r] = silu(x[token r] . Wg) * (x[token r] . Wu),  W = [E, K, gate | up]
 //   expert_down_kn_tile    y[r] = h[r] . W[E, K, N]
+//   expert_mm_kn           y[e] = x[e] . W[e], x [E, C, K]: the same number of rows for all (training with a capacity)
 //
 // Reference: inference/v2/kernels/cutlass_ops/moe_gemm/moe_gemm.cu (grouped GEMM over expert-sorted rows). experts_kn.hip has the
 // streaming form for few rows an expert.
@@ -28,16 +29,19 @@ struct Args {
   const int* token;  // row of x for every sorted row; null: the row itself
   int X;             // rows of x
   const unsigned short* w;
-  const int* offs;
+  const int* offs;  // [E + 1]; null: C rows an expert
+  int C;
   unsigned short* y;
   int E, R, K, N;    // N: columns of W
   int cols, half;    // columns of y; column of W that goes with column 0 in the second half of a tile
 };
 
+// first row of an expert
+__device__ __forceinline__ int row_of(const Args& a, int e) { return a.offs != nullptr ? min(max(a.offs[e], 0), a.R) : e * a.C; }
 template <int BM>
 __device__ __forceinline__ int tiles_of(const Args& a, int e) {
   if (e >= a.E) return 0;
-  const int lo = min(max(a.offs[e], 0), a.R), hi = min(max(a.offs[e + 1], 0), a.R);
+  const int lo = row_of(a, e), hi = row_of(a, e + 1);
   return hi > lo ? (hi - lo + BM - 1) / BM : 0;
 }
 
@@ -85,7 +89,7 @@ __global__ void __launch_bounds__(T::NTHR, T::WAVES) tile_kernel(Args a) {
   expert = __builtin_amdgcn_readfirstlane(expert);
   te = __builtin_amdgcn_readfirstlane(te);
   const int local = id - __builtin_amdgcn_readfirstlane(first) * tn, nt = local / te, rt = local - nt * te;
-  const int r0 = min(max(a.offs[expert], 0), a.R) + rt * BM, r1 = min(max(a.offs[expert + 1], 0), a.R);
+  const int r0 = row_of(a, expert) + rt * BM, r1 = row_of(a, expert + 1);
   const int n0 = nt * CB;
 
   // ---- loads: 8 rows of x, chunk c of row r at place c ^ ((r >> 1) & 7); 2 k rows of W, chunk c of row k at place
@@ -169,12 +173,10 @@ __global__ void __launch_bounds__(T::NTHR, T::WAVES) tile_kernel(Args a) {
 using T256 = Tile<2, 4, 8, 4, 2, 3, 2>;
 using T128 = Tile<2, 4, 4, 4, 3, 3, 2>;
 
-static Args args(const at::Tensor& x, const at::Tensor& w, const at::Tensor& offs) {
+static Args args(const at::Tensor& x, const at::Tensor& w) {
   SXE_CHECK_CUDA(x);
   SXE_CHECK(x.scalar_type() == at::kBFloat16 && x.dim() == 2 && x.is_contiguous() && w.is_cuda() && w.scalar_type() == at::kBFloat16 &&
                 w.dim() == 3 && w.is_contiguous() && w.size(1) == x.size(1), "expert tile product: bf16 x [T, K], w [E, K, N]");
-  SXE_CHECK(offs.is_cuda() && offs.is_contiguous() && offs.scalar_type() == at::kInt && offs.numel() == w.size(0) + 1,
-            "expert tile product: offs int32 [E + 1]");
   SXE_CHECK(w.size(1) > 0 && w.size(1) % 32 == 0 && w.size(2) > 0 && w.size(2) % 16 == 0 && w.size(0) > 0 && w.size(1) < (1 << 30) &&
                 w.size(2) < (1 << 30) && x.size(0) < (1ll << 31) && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
                 reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0,
@@ -185,10 +187,16 @@ static Args args(const at::Tensor& x, const at::Tensor& w, const at::Tensor& off
   a.ldx = x.size(1);
   a.X = x.size(0);
   a.w = reinterpret_cast<const unsigned short*>(w.data_ptr());
-  a.offs = offs.data_ptr<int>();
   a.E = w.size(0);
   a.K = w.size(1);
   a.N = w.size(2);
+  return a;
+}
+static Args args(const at::Tensor& x, const at::Tensor& w, const at::Tensor& offs) {
+  Args a = args(x, w);
+  SXE_CHECK(offs.is_cuda() && offs.is_contiguous() && offs.scalar_type() == at::kInt && offs.numel() == w.size(0) + 1,
+            "expert tile product: offs int32 [E + 1]");
+  a.offs = offs.data_ptr<int>();
   return a;
 }
 
@@ -249,13 +257,32 @@ at::Tensor expert_down_kn_tile(const at::Tensor& h, const at::Tensor& w, const a
   return y;
 }
 
+// x [E, C, K], w [E, K, N] -> [E, C, N]
+at::Tensor expert_mm_kn(const at::Tensor& x, const at::Tensor& w) {
+  SXE_CHECK(x.dim() == 3 && x.is_contiguous() && w.dim() == 3 && x.size(0) == w.size(0) && x.device() == w.device() && x.numel() < (1ll << 40) &&
+                x.size(0) * x.size(1) < (1ll << 31), "expert_mm_kn: x [E, C, K], w [E, K, N]");
+  const at::Tensor rows = x.view({-1, x.size(2)});
+  kt::Args a = kt::args(rows, w);
+  auto y = at::empty({x.size(0), x.size(1), w.size(2)}, x.options());
+  if (y.numel() == 0) return y;
+  c10::DeviceGuard g(x.device());
+  a.C = x.size(1);
+  a.R = a.X;
+  a.y = reinterpret_cast<unsigned short*>(y.data_ptr());
+  a.cols = a.N;
+  kt::launch<false>(a);
+  return y;
+}
+
 }  // namespace sxe
 
 TORCH_LIBRARY_FRAGMENT(sxe, m) {
   m.def("expert_swiglu_kn_tile(Tensor x, Tensor w, Tensor offs, Tensor token) -> Tensor");
   m.def("expert_down_kn_tile(Tensor h, Tensor w, Tensor offs) -> Tensor");
+  m.def("expert_mm_kn(Tensor x, Tensor w) -> Tensor");
 }
 TORCH_LIBRARY_IMPL(sxe, CUDA, m) {
   m.impl("expert_swiglu_kn_tile", &sxe::expert_swiglu_kn_tile);
   m.impl("expert_down_kn_tile", &sxe::expert_down_kn_tile);
+  m.impl("expert_mm_kn", &sxe::expert_mm_kn);
 }

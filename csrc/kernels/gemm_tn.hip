@@ -1,6 +1,6 @@
 // Products of many rows on gfx950: y[M, N] = x[M, K] . w[N, K]' (+ bias), both operands with K contiguous, and the same with SwiGLU
 // over w = [gate | up] in the epilogue (y[M, N / 2] = silu(x . gate') * (x . up'), one rounding, of the result). bf16 in and out, fp32
-// sums. skinny_gemm.hip and stream_gemm.hip have the forms for up to 32 rows.
+// sums; also a batch of them in one launch. skinny_gemm.hip and stream_gemm.hip have the forms for up to 32 rows.
 //
 // What bounds it: at 256 x 256 the card's power. Products of 16 x 16 x 32 run at 1.85 GHz where those of 32 x 32 x 16 run at
 // 1.65 (they read and write half as many sums a flop); behind them LDS, which is busy for 80 % of the products' time.
@@ -28,8 +28,9 @@ struct Args {
   const unsigned short *x, *w, *bias;
   unsigned short* y;
   float* part;           // splits of K: their sums, [splits, M, N]
-  int64_t ldx, ldw;
-  int M, cols, half, slabs, per, splits;  // columns of y (SwiGLU: half the rows of w); w row that goes with row 0 as up; slabs of K, of a split
+  int64_t ldx, ldw, bx, bw, by;  // elements from row to row, and from product to product of a batch
+  int M, cols, half, slabs, per, parts;  // columns of y (SwiGLU: half the rows of w); w row that goes with row 0 as up; slabs of K, of a split;
+                                         // splits of K, or products of a batch
   int tm, tn, gm;        // whole row tiles, column blocks; row tiles that run side by side
 };
 
@@ -44,17 +45,17 @@ template <typename T, bool GLU, bool SPLIT>
 __global__ void __launch_bounds__(T::NTHR, T::WAVES) gemm_kernel(Args a) {
   constexpr int RT = T::RT, CT = T::CT, NW = T::NW, PA = T::PA, PB = T::PB, BM = T::BM, CB = GLU ? T::BN / 2 : T::BN, X_LDS = T::SA * T::AS;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wr = w / T::WC, wc = w % T::WC;
-  // ---- workgroup -> (split, row tile, column block): neighbours in an XCD's run share w, gm row tiles at a time. The tiles of the
+  // ---- workgroup -> (split or product, row tile, column block): neighbours in an XCD's run share w, gm row tiles at a time. The tiles of the
   // last rows, if these are no whole tile, come behind all others: they take less time and fill the last round
-  const int whole = a.tm * a.tn * a.splits;
+  const int whole = a.tm * a.tn * a.parts;
   const bool rest = (int)blockIdx.x >= whole;
   const int block = rest ? blockIdx.x - whole : blockIdx.x, nwg = rest ? gridDim.x - whole : whole;
   const int q8 = nwg / 8, r8 = nwg % 8, xcd = block % 8;
   const int id = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + block / 8;
-  const int nt = rest ? a.tn : a.tm * a.tn, split = SPLIT ? id / nt : 0, tile = SPLIT ? id - split * nt : id;
+  const int nt = rest ? a.tn : a.tm * a.tn, part = a.parts > 1 ? id / nt : 0, tile = id - part * nt;
   const int per_group = a.gm * a.tn, group = tile / per_group, in = tile - group * per_group, rows = min(a.tm - group * a.gm, a.gm);
   const int m0 = (rest ? a.tm : group * a.gm + in % rows) * BM, n0 = (rest ? tile : in / rows) * CB;
-  const int first = SPLIT ? split * a.per : 0, ns = SPLIT ? min(a.per, a.slabs - first) : a.slabs;
+  const int first = SPLIT ? part * a.per : 0, ns = SPLIT ? min(a.per, a.slabs - first) : a.slabs;
 
   // ---- loads: a wave's load is 8 rows, chunk c of row r at place c ^ ((r >> 1) & 7). Rows and columns behind the last, and slabs,
   // repeat it
@@ -67,8 +68,8 @@ __global__ void __launch_bounds__(T::NTHR, T::WAVES) gemm_kernel(Args a) {
     const int r = 8 * (i * NW + w) + lr, c = min(column<GLU>(r), a.cols - 1 - n0);
     wo[i] = (unsigned)(c + (GLU && (r & 16) ? a.half : 0)) * (unsigned)(2 * a.ldw) + lc;
   }
-  const char* xb = reinterpret_cast<const char*>(a.x + m0 * a.ldx + first * BK);
-  const char* wb = reinterpret_cast<const char*>(a.w + n0 * a.ldw + first * BK);
+  const char* xb = reinterpret_cast<const char*>(a.x + m0 * a.ldx + (SPLIT ? first * BK : part * a.bx));
+  const char* wb = reinterpret_cast<const char*>(a.w + n0 * a.ldw + (SPLIT ? first * BK : part * a.bw));
   const unsigned l0 = lds_base();
   auto load_x = [&](int i, int slab, unsigned slot) { glds(xo[i], xb + min(slab, ns - 1) * ROW, l0 + slot + (i * NW + w) * 1024); };
   auto load_w = [&](int i, int slab, unsigned slot) {
@@ -98,7 +99,7 @@ __global__ void __launch_bounds__(T::NTHR, T::WAVES) gemm_kernel(Args a) {
       const int r = m0 + (wr * RT + i) * 16 + l16;
       if (r >= a.M) continue;
       if constexpr (SPLIT) {
-        float* p = a.part + ((int64_t)split * a.M + r) * (GLU ? 2 * a.cols : a.cols);
+        float* p = a.part + ((int64_t)part * a.M + r) * (GLU ? 2 * a.cols : a.cols);
 #pragma unroll
         for (int j = 0; j < CT; ++j) {
           const int b = GLU ? (j >> 1) & 1 : j & 1, c = n0 + (GLU ? wc * CT * 8 : (wc * CT + (j & ~1)) * 16) + 8 * g + 4 * b;
@@ -113,7 +114,7 @@ __global__ void __launch_bounds__(T::NTHR, T::WAVES) gemm_kernel(Args a) {
           const float x = acc[i][2 * (e >> 2)][e & 3];
           v[e] = x * sigmoid(x) * acc[i][2 * (e >> 2) + 1][e & 3];
         }
-        *reinterpret_cast<u32x4*>(a.y + (int64_t)r * a.cols + c) = u32x4{pack(v[0], v[1]), pack(v[2], v[3]), pack(v[4], v[5]), pack(v[6], v[7])};
+        *reinterpret_cast<u32x4*>(a.y + part * a.by + (int64_t)r * a.cols + c) = u32x4{pack(v[0], v[1]), pack(v[2], v[3]), pack(v[4], v[5]), pack(v[6], v[7])};
       }
     }
   } else {
@@ -129,7 +130,7 @@ __global__ void __launch_bounds__(T::NTHR, T::WAVES) gemm_kernel(Args a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           v[h][e] = pack(acc[i][2 * h + (e >> 1)][2 * (e & 1)] + b[h][2 * e], acc[i][2 * h + (e >> 1)][2 * (e & 1) + 1] + b[h][2 * e + 1]);
-      store_lines(a.y, a.cols, m0 + (wr * RT + i) * 16 + l16, a.M, n0 + wc * CT * 16, a.cols, v);
+      store_lines(a.y + part * a.by, a.cols, m0 + (wr * RT + i) * 16 + l16, a.M, n0 + wc * CT * 16, a.cols, v);
     }
   }
 }
@@ -188,11 +189,11 @@ struct Plan {
   int form, splits;
   float us;
 };
-static Plan plan(int64_t M, int64_t N, int64_t slabs, bool may_split) {
+static Plan plan(int64_t M, int64_t N, int64_t slabs, bool may_split, int64_t batch) {
   Plan best{0, 1, 1e30f};
   for (int f = 0; f < 4; ++f) {
     const Form& t = kForms[f];
-    const int64_t cols = (N + t.bn - 1) / t.bn, rest = M % t.bm;
+    const int64_t cols = (N + t.bn - 1) / t.bn * batch, rest = M % t.bm;
     for (int s : {1, 2, 3, 4, 6, 8}) {
       if (s > 1 && (!may_split || slabs < 4 * s || (M + t.bm - 1) / t.bm * cols * s > 600)) break;
       const float part = 0.62f + 0.38f * rest / t.bm, one = (slabs + s - 1) / s * t.slab + t.start;
@@ -208,13 +209,13 @@ static Plan plan(int64_t M, int64_t N, int64_t slabs, bool may_split) {
 }
 
 template <typename T, bool GLU>
-static void launch(Args a, int splits) {
+static void launch(Args a, int splits, int batch) {
   constexpr int CB = GLU ? T::BN / 2 : T::BN;
   a.tm = a.M / T::BM;
   a.tn = (a.cols + CB - 1) / CB;
   a.gm = std::max(1, std::min(a.tm, 8));
-  a.splits = splits;
-  const int64_t grid = ((int64_t)a.M + T::BM - 1) / T::BM * a.tn * splits;
+  a.parts = splits * batch;  // one of them is 1
+  const int64_t grid = ((int64_t)a.M + T::BM - 1) / T::BM * a.tn * a.parts;
   SXE_CHECK(grid < (1ll << 30), "gemm_tn: too many tiles");
   if (splits > 1) {
     allow_lds<&gemm_kernel<T, GLU, true>>(T::LDS);
@@ -230,18 +231,18 @@ static void launch(Args a, int splits) {
 
 }  // namespace tn
 
-// x [M, K] (rows may lie apart), w [N, K] (the same), bias [N] or none -> [M, N], glu: [M, N / 2]. tile, splits of K: -1, 0: the plan's
-at::Tensor gemm_tn(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, bool glu, int64_t tile, int64_t splits) {
+// x, w [.., rows, K], one product or a batch
+static at::Tensor gemm_tn_run(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, bool glu, int64_t tile, int64_t splits) {
   check_beside(x, {w, bias});
-  SXE_CHECK(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 && x.dim() == 2 && w.dim() == 2 &&
-                x.size(1) == w.size(1), "gemm_tn: bf16 x [M, K], w [N, K]");
-  const int64_t M = x.size(0), K = x.size(1), N = w.size(0), cols = glu ? N / 2 : N;
+  const int64_t d = x.dim() - 2, batch = d ? x.size(0) : 1, M = x.size(d), K = x.size(d + 1), N = w.size(d), cols = glu ? N / 2 : N;
+  SXE_CHECK(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 && w.size(d + 1) == K && (!d || w.size(0) == batch),
+            "gemm_tn: bf16 x [M, K], w [N, K]");
   SXE_CHECK(K > 0 && K % tn::BK == 0 && N > 0 && N % (glu ? 16 : 8) == 0, "gemm_tn: K in multiples of 64, columns of 8");
   for (const at::Tensor* t : {&x, &w})
-    SXE_CHECK(t->size(0) <= 1 || (t->stride(0) % 8 == 0 && t->stride(0) >= 0), "gemm_tn: rows that start on 16 bytes");
-  SXE_CHECK(x.stride(1) == 1 && w.stride(1) == 1 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
-                reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0, "gemm_tn: rows of neighbouring elements that start on 16 bytes");
-  const int64_t ldx = M > 1 ? x.stride(0) : K, ldw = N > 1 ? w.stride(0) : K;
+    SXE_CHECK((t->size(d) <= 1 || (t->stride(d) % 8 == 0 && t->stride(d) >= 0)) && (!d || batch <= 1 || t->stride(0) % 8 == 0) &&
+                  t->stride(d + 1) == 1 && reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0,
+              "gemm_tn: rows of neighbouring elements that start on 16 bytes");
+  const int64_t ldx = M > 1 ? x.stride(d) : K, ldw = N > 1 ? w.stride(d) : K;
   SXE_CHECK(M < (1ll << 30) && N < (1ll << 30) && K < (1ll << 30) && 512 * ldx < (1ll << 32) && (glu ? 2 * N * ldw : 512 * ldw) < (1ll << 32),
             "gemm_tn: sizes beyond 32-bit offsets");
   const bool has_bias = bias.has_value() && bias->defined();
@@ -249,8 +250,8 @@ at::Tensor gemm_tn(const at::Tensor& x, const at::Tensor& w, const c10::optional
                           reinterpret_cast<uintptr_t>(bias->data_ptr()) % 16 == 0), "gemm_tn: bias bf16 [N]");
   SXE_CHECK(tile < 4 && splits >= 0 && splits <= 64, "gemm_tn: tile 0 - 3 or -1, splits 0 - 64");
   c10::DeviceGuard g(x.device());
-  auto y = at::empty({M, cols}, x.options());
-  if (M == 0) return y;
+  auto y = d ? at::empty({batch, M, cols}, x.options()) : at::empty({M, cols}, x.options());
+  if (y.numel() == 0) return y;
   tn::Args a{};
   a.x = reinterpret_cast<const unsigned short*>(x.data_ptr());
   a.w = reinterpret_cast<const unsigned short*>(w.data_ptr());
@@ -258,16 +259,22 @@ at::Tensor gemm_tn(const at::Tensor& x, const at::Tensor& w, const c10::optional
   a.y = reinterpret_cast<unsigned short*>(y.data_ptr());
   a.ldx = ldx;
   a.ldw = ldw;
+  if (d) {
+    a.bx = x.stride(0);
+    a.bw = w.stride(0);
+    a.by = M * cols;
+  }
   a.M = M;
   a.cols = cols;
   a.half = cols;
   a.slabs = K / tn::BK;
   if (tile < 0) {
-    const tn::Plan p = tn::plan(M, N, a.slabs, splits != 1);
+    const tn::Plan p = tn::plan(M, N, a.slabs, splits != 1, batch);
     tile = p.form;
     if (splits == 0) splits = p.splits;
   }
   splits = std::max<int64_t>(1, splits);
+  SXE_CHECK(splits == 1 || batch == 1, "gemm_tn: a batch or splits");
   a.per = (a.slabs + splits - 1) / splits;
   const int parts = (a.slabs + a.per - 1) / a.per;  // none of them empty
   at::Tensor part;
@@ -277,7 +284,7 @@ at::Tensor gemm_tn(const at::Tensor& x, const at::Tensor& w, const c10::optional
   }
   auto run = [&](auto t) {
     using T = decltype(t);
-    glu ? tn::launch<T, true>(a, parts) : tn::launch<T, false>(a, parts);
+    glu ? tn::launch<T, true>(a, parts, batch) : tn::launch<T, false>(a, parts, batch);
   };
   switch (tile) {
     case 0: run(tn::T256{}); break;
@@ -288,9 +295,25 @@ at::Tensor gemm_tn(const at::Tensor& x, const at::Tensor& w, const c10::optional
   return y;
 }
 
+// x [M, K] (rows may lie apart), w [N, K] (the same), bias [N] or none -> [M, N], glu: [M, N / 2]. tile, splits of K: -1, 0: the plan's
+at::Tensor gemm_tn(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, bool glu, int64_t tile, int64_t splits) {
+  SXE_CHECK(x.dim() == 2 && w.dim() == 2, "gemm_tn: bf16 x [M, K], w [N, K]");
+  return gemm_tn_run(x, w, bias, glu, tile, splits);
+}
+
+// x [B, M, K], w [B, N, K] -> [B, M, N], one launch
+at::Tensor gemm_tn_batch(const at::Tensor& x, const at::Tensor& w, int64_t tile) {
+  SXE_CHECK(x.dim() == 3 && w.dim() == 3, "gemm_tn_batch: bf16 x [B, M, K], w [B, N, K]");
+  return gemm_tn_run(x, w, c10::nullopt, false, tile, 1);
+}
+
 }  // namespace sxe
 
 TORCH_LIBRARY_FRAGMENT(sxe, m) {
   m.def("gemm_tn(Tensor x, Tensor w, Tensor? bias, bool glu, int tile=-1, int splits=0) -> Tensor");
+  m.def("gemm_tn_batch(Tensor x, Tensor w, int tile=-1) -> Tensor");
 }
-TORCH_LIBRARY_IMPL(sxe, CUDA, m) { m.impl("gemm_tn", &sxe::gemm_tn); }
+TORCH_LIBRARY_IMPL(sxe, CUDA, m) {
+  m.impl("gemm_tn", &sxe::gemm_tn);
+  m.impl("gemm_tn_batch", &sxe::gemm_tn_batch);
+}

@@ -14,6 +14,7 @@ import os
 import torch
 import torch.nn as nn
 
+from ..ops import native
 from ..ops.activation import swiglu
 
 # SXE_MOE_DEFER_WGRAD=0: write the expert weight gradients every micro-step (see _GroupedMM)
@@ -87,9 +88,26 @@ class GroupedSwiGLUExperts(nn.Module):
         return grouped_mm(swiglu(grouped_mm(x, self.w_gate_up)), self.w_down)
 
 
+def expert_products(x, w, transposed=False):
+    """x[e] @ w[e] (``transposed``: x[e] @ w[e]^T) of all experts, bf16 x [E, C, .], w [E, K, N], in one launch (csrc/kernels/experts_kn_tile.hip,
+    gemm_tn.hip); None where these do not cover the operands. A library product per expert fills the card only with the rows of one:
+    8 experts, 4096 x 28672, us, 320 rows each 670 / 713 here, 1280 rows 2151 / 1767, transposed 2393 / 578, 3268 / 2007; 14336 x 4096,
+    1110 / 333, 1372 / 908, transposed 434 / 382, 1100 / 825; 2048 x 16384, 1280 rows 657 / 552, transposed 980 / 571."""
+    if not (x.is_cuda and w.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 3 and w.dim() == 3
+            and native.plain(x, w)):
+        return None
+    (E, C, n), (_, K, N) = x.shape, w.shape
+    if (x.is_contiguous() and w.is_contiguous() and E == w.shape[0] and n == (N if transposed else K) and C > 0
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and K % 64 == 0 and N % 64 == 0 and 0 < K < 1 << 22 and 0 < N < 1 << 22
+            and E * C < 1 << 30 and E <= 1024):
+        native.require_hip()
+        return torch.ops.sxe.gemm_tn_batch(x, w) if transposed else torch.ops.sxe.expert_mm_kn(x, w)
+    return None
+
+
 class _GroupedMM(torch.autograd.Function):
-    """y[e] = x[e] @ W[e] for x [E, C, K], W [E, K, N]: one plain 2-D hipBLASLt GEMM per expert,
-    written in place into the output (no stacking copies). Backward: dX per expert in place, and
+    """y[e] = x[e] @ W[e] for x [E, C, K], W [E, K, N]: all experts in one launch (``expert_products``), else one plain 2-D
+    hipBLASLt GEMM per expert, written in place into the output (no stacking copies). Backward: dX the same way, and
     dW straight into the ZeRO gradient buffer of W (fp32 accumulate with beta = 1 inside the GEMM,
     like ops/linear.py) -- autograd's select/stack backward would instead materialise a zeroed
     full-size [E, K, N] gradient per expert and sum them (measured: 36 % of a Mixtral step).
@@ -100,9 +118,11 @@ class _GroupedMM(torch.autograd.Function):
     def forward(ctx, x, w):
         E, C, _ = x.shape
         x = x.contiguous()
-        y = x.new_empty(E, C, w.shape[2])
-        for e in range(E):
-            torch.mm(x[e], w[e], out=y[e])
+        y = expert_products(x, w)
+        if y is None:
+            y = x.new_empty(E, C, w.shape[2])
+            for e in range(E):
+                torch.mm(x[e], w[e], out=y[e])
         ctx.save_for_backward(x, w)
         return y
 
@@ -113,9 +133,11 @@ class _GroupedMM(torch.autograd.Function):
         E = x.shape[0]
         dx = dw = None
         if ctx.needs_input_grad[0]:
-            dx = torch.empty_like(x)
-            for e in range(E):
-                torch.mm(dy[e], w[e].t(), out=dx[e])
+            dx = expert_products(dy, w, transposed=True)
+            if dx is None:
+                dx = torch.empty_like(x)
+                for e in range(E):
+                    torch.mm(dy[e], w[e].t(), out=dx[e])
         if ctx.needs_input_grad[1]:
             from ..ops.linear import grad_target
             tgt = grad_target(w)

@@ -70,6 +70,10 @@ def _register_sxe_formulas():
         def _tiled(x, w, *a, out_shape=None, **kw):
             return 2 * x[0] * w[0] * w[1]
 
+        @register_flop_formula([ops.gemm_tn_batch, ops.expert_mm_kn])
+        def _batched(x, w, *a, out_shape=None, **kw):
+            return 2 * x[0] * x[1] * w[1] * w[2]
+
         def _routed(rows, w):  # every row meets exactly one expert, w [E, K, N]
             return 2 * rows * w[1] * w[2]
 

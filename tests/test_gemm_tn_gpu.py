@@ -74,6 +74,29 @@ def test_linear_takes_them(M, N, K, taken, monkeypatch):
     assert L.linear(x.requires_grad_(), w).requires_grad and len(seen) == n
 
 
+@pytest.mark.parametrize("C", [1, 16, 129, 257, 300])
+@pytest.mark.parametrize("E,K,N", [(1, 64, 128), (3, 192, 320), (8, 64, 576)])
+def test_expert_products(E, C, K, N):
+    """All experts' products in a launch, with the weights as they lie and transposed, and the gradients of the layer that runs them."""
+    from shuffle_exchange_amd.moe.experts import expert_products, grouped_mm
+    g = torch.Generator("cuda").manual_seed(C)
+    x = torch.randn(E, C, K, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(E, K, N, device="cuda", generator=g) * K ** -0.5).bfloat16()
+    dy = torch.randn(E, C, N, device="cuda", generator=g).bfloat16()
+    y, dx = expert_products(x, w), expert_products(dy, w, transposed=True)
+    for tile in range(4):
+        assert torch.equal(torch.ops.sxe.gemm_tn_batch(dy, w, tile), dx)
+    for e in range(E):
+        _close(y[e], x[e].double() @ w[e].double(), x[e], w[e].t())
+        _close(dx[e], dy[e].double() @ w[e].double().t(), dy[e], w[e])
+    xg, wg = x.clone().requires_grad_(), w.clone().requires_grad_()
+    out = grouped_mm(xg, wg)
+    out.backward(dy)
+    assert torch.equal(out, y) and torch.equal(xg.grad, dx)
+    for other in (x[:, :, :K - 32].contiguous(), x.float(), x.transpose(1, 2)):  # not covered: the caller's loop over the experts
+        assert expert_products(other, w) is None
+
+
 def test_captured():
     """Replays with new inputs; the splits' sums are the graph's own memory."""
     x, w, _ = _operands(300, 2048, 8192)
