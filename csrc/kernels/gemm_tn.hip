@@ -231,8 +231,9 @@ static void launch(Args a, int splits, int batch) {
 
 }  // namespace tn
 
-// x, w [.., rows, K], one product or a batch
-static at::Tensor gemm_tn_run(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, bool glu, int64_t tile, int64_t splits) {
+// x, w [.., rows, K], one product or a batch; out: y's sizes where they are not those of one product
+static at::Tensor gemm_tn_run(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, bool glu, int64_t tile, int64_t splits,
+                              at::IntArrayRef out = {}) {
   check_beside(x, {w, bias});
   const int64_t d = x.dim() - 2, batch = d ? x.size(0) : 1, M = x.size(d), K = x.size(d + 1), N = w.size(d), cols = glu ? N / 2 : N;
   SXE_CHECK(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 && w.size(d + 1) == K && (!d || w.size(0) == batch),
@@ -250,7 +251,7 @@ static at::Tensor gemm_tn_run(const at::Tensor& x, const at::Tensor& w, const c1
                           reinterpret_cast<uintptr_t>(bias->data_ptr()) % 16 == 0), "gemm_tn: bias bf16 [N]");
   SXE_CHECK(tile < 4 && splits >= 0 && splits <= 64, "gemm_tn: tile 0 - 3 or -1, splits 0 - 64");
   c10::DeviceGuard g(x.device());
-  auto y = d ? at::empty({batch, M, cols}, x.options()) : at::empty({M, cols}, x.options());
+  auto y = d ? at::empty({batch, M, cols}, x.options()) : out.empty() ? at::empty({M, cols}, x.options()) : at::empty(out, x.options());
   if (y.numel() == 0) return y;
   tn::Args a{};
   a.x = reinterpret_cast<const unsigned short*>(x.data_ptr());
@@ -295,10 +296,14 @@ static at::Tensor gemm_tn_run(const at::Tensor& x, const at::Tensor& w, const c1
   return y;
 }
 
-// x [M, K] (rows may lie apart), w [N, K] (the same), bias [N] or none -> [M, N], glu: [M, N / 2]. tile, splits of K: -1, 0: the plan's
+// x [M, K] (rows may lie apart) or contiguous [.., K], w [N, K] (rows may lie apart), bias [N] or none -> [.., N], glu: [.., N / 2], a tensor
+// of its own. tile, splits of K: -1, 0: the plan's
 at::Tensor gemm_tn(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, bool glu, int64_t tile, int64_t splits) {
-  SXE_CHECK(x.dim() == 2 && w.dim() == 2, "gemm_tn: bf16 x [M, K], w [N, K]");
-  return gemm_tn_run(x, w, bias, glu, tile, splits);
+  SXE_CHECK((x.dim() == 2 || (x.dim() > 2 && x.is_contiguous())) && w.dim() == 2, "gemm_tn: bf16 x [M, K] or contiguous [.., K], w [N, K]");
+  if (x.dim() == 2) return gemm_tn_run(x, w, bias, glu, tile, splits);
+  std::vector<int64_t> out(x.sizes().vec());
+  out.back() = glu ? w.size(0) / 2 : w.size(0);
+  return gemm_tn_run(x.view({-1, x.size(-1)}), w, bias, glu, tile, splits, out);
 }
 
 // x [B, M, K], w [B, N, K] -> [B, M, N], one launch

@@ -215,7 +215,8 @@ class _QKVProjAttn(torch.autograd.Function):
     def forward(ctx, x, w, cos, sin, nq, nkv, causal, scale, pos):
         B, S, H = x.shape
         x2 = x.reshape(-1, H)
-        qkv = F.linear(x2, w).view(B, S, nq + 2 * nkv, -1)
+        from .linear import product
+        qkv = product(x2, w).view(B, S, nq + 2 * nkv, -1)
         if cos is not None:
             torch.ops.sxe.rope_(qkv[:, :, :nq + nkv], cos, sin, pos, S, 0, False)
         q, k, v = qkv[:, :, :nq], qkv[:, :, nq:nq + nkv], qkv[:, :, nq + nkv:]

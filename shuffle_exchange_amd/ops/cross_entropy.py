@@ -17,6 +17,7 @@ import torch
 import torch.nn.functional as F
 
 from . import native
+from .linear import product
 
 
 class _XEnt(torch.autograd.Function):
@@ -80,7 +81,7 @@ class _FusedLinearXEnt(torch.autograd.Function):
             # dual layout: the forward computes only loss + lse; the backward writes the scaled
             # gradient over the logits AND its vocab-major transpose in one pass (xent_grad_dual),
             # so the LM-head weight gradient is a TN GEMM with no transpose of the 4 GB gradient
-            logits = torch.matmul(h2, weight.t())
+            logits = product(h2, weight)
             loss, lse = torch.ops.sxe.xent_fwd(logits, tgt, int(ignore_index), False, None, 1.0)
             ctx.save_for_backward(logits, lse, tgt, inv_n, h2, weight)
             ctx.mode = "dual"
@@ -90,7 +91,7 @@ class _FusedLinearXEnt(torch.autograd.Function):
         if chunk == T:
             # unchunked: keep d(loss)/d(logits) (written over the logits) and do both GEMMs in
             # backward, where the weight-grad GEMM can land directly in the optimizer's buffer
-            logits = torch.matmul(h2, weight.t())
+            logits = product(h2, weight)
             loss, _ = torch.ops.sxe.xent_fwd(logits, tgt, int(ignore_index), need_grad, inv_n, 1.0)
             ctx.save_for_backward(logits if need_grad else None, h2, weight)
             ctx.mode = "dlogits"

@@ -162,7 +162,20 @@ def _tiled(x, weight, bias):
     if not _tileable(x2, weight, bias):
         return None
     native.require_hip()
+    if x.dim() == 2 or x.is_contiguous():  # the result is no view: autograd functions return it, and their callers write to it
+        return torch.ops.sxe.gemm_tn(x, weight, bias, False)
     return torch.ops.sxe.gemm_tn(x2, weight, bias, False).view(*x.shape[:-1], weight.shape[0])
+
+
+def product(x, weight, bias=None):
+    """``F.linear`` for the inside of autograd functions: no graph is built where it runs own kernels (``_tiled``)."""
+    if (weight.shape[0] >= 2048 <= weight.shape[-1] and SKINNY_MAX_M > 0 and x.is_cuda and not torch.is_grad_enabled()
+            and native.plain(x, weight, bias) and (x.dim() == 2 or x.is_contiguous())
+            and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == torch.bfloat16)):
+        y = _tiled(x, weight, bias)
+        if y is not None:
+            return y
+    return F.linear(x, weight, bias)
 
 
 def glu_tiled(x, weight):
@@ -372,8 +385,12 @@ def _tn_ok(gy2, x2):
 # Data-gradient GEMMs dX = dY W run in hipBLASLt's "NN" layout at 1.03-1.35 PF on MI355X; with W^T
 # materialised by the HBM-speed transpose they run in the forward layout at 1.25-1.56 PF
 # (tools/gemm_layout_bench.py, profiles/gemm_layout.log: net -0.03..-0.06 ms per Llama-3-8B layer
-# GEMM, -0.48 ms for the LM head, at 8192 tokens). The transpose reads/writes only the weight.
+# GEMM, -0.48 ms for the LM head, at 8192 tokens). The transpose reads/writes only the weight. Fewer rows pay for it where the
+# product sums over many columns and gemm_tn.hip takes it, us, NN / transpose and own product: 256 rows, 28672 x 4096 170 / 162,
+# 16384 x 3072 93 / 71, 1000 rows 372 / 286, 176 / 128, 32000 x 4096 402 / 320, 16384 x 2048 112 / 89; but 1371 rows of 28672 x 4096
+# 310 / 358; 4096 x 14336, 1000 rows 97 / 130.
 DGRAD_WT_MIN_ELEMS = int(os.environ.get("SXE_DGRAD_WT_MIN_ELEMS", 16 * 2**20))
+DGRAD_WT_LONG = 16384
 
 
 # The transposed weights are constant between optimizer steps: with gradient accumulation each
@@ -441,8 +458,10 @@ def data_grad(gy, w):
     """dX = gy @ w for w [N, K] (gy [..., N])."""
     if (DGRAD_WT_MIN_ELEMS > 0 and gy.is_cuda and gy.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and w.dim() == 2 and w.is_contiguous() and w.numel() >= DGRAD_WT_MIN_ELEMS and w.shape[0] % 64 == 0
-            and w.shape[1] % 64 == 0 and gy.numel() // gy.shape[-1] >= 2048):
-        return torch.matmul(gy, _transposed_weight(w).t())
+            and w.shape[1] % 64 == 0):
+        rows = gy.numel() // gy.shape[-1]
+        if rows >= 2048 or (rows >= 256 and w.shape[0] >= DGRAD_WT_LONG and _tiled_faster(rows, w.shape[1], w.shape[0])):
+            return product(gy, _transposed_weight(w))
     return torch.matmul(gy, w)
 
 
@@ -540,7 +559,7 @@ class _Linear(torch.autograd.Function):
             bias = bias.to(ac) if bias is not None else None
         ctx.save_for_backward(x, weight)
         ctx.has_bias = bias is not None
-        return F.linear(x, weight, bias)
+        return product(x, weight, bias)
 
     @staticmethod
     def backward(ctx, gy):
@@ -567,17 +586,19 @@ def linear(x, weight, bias=None):
     grad = torch.is_grad_enabled() and (weight.requires_grad or x.requires_grad or (bias is not None and bias.requires_grad))
     if grad and weight.requires_grad and hasattr(weight, "_sxe_grad_target"):
         return _Linear.apply(x, weight, bias)
-    if (not grad and SKINNY_MAX_M > 0 and x.is_cuda
-            and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == torch.bfloat16)
-            and native.plain(x, weight, bias)):
-        if x.numel() <= max(SKINNY_MAX_M, STREAM_ROWS_SMALL) * x.shape[-1]:
-            y = _skinny(x, weight, bias)
-            if y is None:
-                y = _stream(x, weight, bias)
-        else:
-            y = _tiled(x, weight, bias)
-        if y is not None:
-            return y
+    if not grad and SKINNY_MAX_M > 0 and x.is_cuda:
+        few = x.numel() <= max(SKINNY_MAX_M, STREAM_ROWS_SMALL) * x.shape[-1]
+        if ((few or weight.shape[0] >= 2048 <= weight.shape[-1])
+                and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == torch.bfloat16)
+                and native.plain(x, weight, bias)):
+            if few:
+                y = _skinny(x, weight, bias)
+                if y is None:
+                    y = _stream(x, weight, bias)
+            else:
+                y = _tiled(x, weight, bias)
+            if y is not None:
+                return y
     return F.linear(x, weight, bias)
 
 

@@ -27,10 +27,9 @@ trains through autograd (no fused MLP exists there); parity is autograd's result
 import os
 
 import torch
-import torch.nn.functional as F
 
 from . import native
-from .linear import Linear, data_grad
+from .linear import Linear, data_grad, product
 
 ACT_SILU = 3
 ENABLED = os.environ.get("SXE_MLP_TN", "1") == "1"
@@ -114,10 +113,10 @@ class _SwiGLUMLP(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, wgu, wd):
         x2 = x.reshape(-1, x.shape[-1])
-        gu = F.linear(x2, wgu)
+        gu = product(x2, wgu)
         v = dual_variant(wd.shape[1])
         h, hT = torch.ops.sxe.gated_act_fwd_dual(gu, ACT_SILU, v)
-        out = F.linear(h, wd)
+        out = product(h, wd)
         del h
         xT = torch.ops.sxe.transpose16(x2) if ctx.needs_input_grad[1] else None
         ctx.save_for_backward(xT, gu, hT, wgu, wd)

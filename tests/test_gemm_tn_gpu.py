@@ -58,7 +58,7 @@ def test_infinities_and_nan_stay_in_their_rows():
 def test_linear_takes_them(M, N, K, taken, monkeypatch):
     from shuffle_exchange_amd.ops import linear as L
     x, w, b = _operands(M, N, K)
-    seen = []
+    seen = [None]
     tiled = L._tiled
     monkeypatch.setattr(L, "_tiled", lambda *a: seen.append(tiled(*a)) or seen[-1])
     with torch.no_grad():
@@ -95,6 +95,32 @@ def test_expert_products(E, C, K, N):
     assert torch.equal(out, y) and torch.equal(xg.grad, dx)
     for other in (x[:, :, :K - 32].contiguous(), x.float(), x.transpose(1, 2)):  # not covered: the caller's loop over the experts
         assert expert_products(other, w) is None
+
+
+@pytest.mark.parametrize("rows", [(3, 515), (1545,), (4, 384)])
+def test_training_products(rows):
+    """Forward and data gradient of a layer that writes its weight gradient itself; its result may be changed in place, as RoPE does."""
+    from shuffle_exchange_amd.ops import linear as L
+    x, w, _ = _operands(1545, 2048, 2048)
+    x = x.contiguous().view(*rows, 2048) if len(rows) == 1 or rows[0] * rows[1] == 1545 else x[:1536].contiguous().view(*rows, 2048)
+    dy = torch.randn(*rows, 2048, device="cuda", generator=torch.Generator("cuda").manual_seed(1)).bfloat16()
+    x.requires_grad_()
+    p = torch.nn.Parameter(w.contiguous())
+    buf = torch.zeros(2048, 2048, device="cuda")
+    p._sxe_grad_target, p._sxe_grad_done = (lambda q: (buf, False)), (lambda q: None)
+    y = L.linear(x, p)
+    _close(y.detach().view(-1, 2048), x.detach().view(-1, 2048).double() @ w.double().t(), x.detach().view(-1, 2048), w)
+    y.view(*rows, 16, 128)[..., :4, :].mul_(2.0)
+    y.backward(dy)
+    d = dy.clone()
+    d.view(*rows, 16, 128)[..., :4, :].mul_(2.0)
+    _close(x.grad.view(-1, 2048), d.view(-1, 2048).double() @ w.double(), d.view(-1, 2048), w.t())
+    want = d.view(-1, 2048).double().t() @ x.detach().view(-1, 2048).double()
+    assert (buf.double() - want).norm() <= 1e-5 * want.norm()
+    # many columns to sum over: few rows take the transposed weight, too
+    wide = (torch.randn(16384, 2048, device="cuda") * 128 ** -1).bfloat16()
+    g = torch.randn(300, 16384, device="cuda").bfloat16()
+    _close(L.data_grad(g, wide), g.double() @ wide.double(), g, wide.t())
 
 
 def test_captured():
