@@ -1,480 +1,340 @@
-// Weight-gradient GEMM for gfx950: C[M, N] (+)= alpha * A^T B with A = dY [K, M] and B = X [K, N]
-// both row-major (the reduction dimension K = tokens is the ROW index of both operands), fp32 C.
+// Weight gradients on gfx950: C[M, N] (+)= alpha * A' B, A = dY [T, M] and B = X [T, N] bf16, both row-major (the sum runs over the tokens,
+// the ROWS of both operands), fp32 C; one product, or one for every expert of a layer in a launch; the tokens in one or two pieces.
 //
-// Why a hand-written kernel: this is the one training GEMM shape class whose operands are both
-// k-strided, and with an fp32 accumulate-in-place output (the ZeRO gradient accumulator) the vendor
-// library runs it 20-35 % below its forward-layout GEMMs on MI355X (measured: 850-1110 TF vs
-// 1260-1610 TF, tools/tune_gemms.py). Here both operands stream row-wise through LDS (global_load_lds,
-// lane-linear image with a source-side XOR swizzle) and are read back TRANSPOSED with
-// ds_read_b64_tr_b16, so no operand ever needs a transposed copy in HBM, and the fp32
-// read-add-write of C happens once per tile in the epilogue.
+// Why a hand-written kernel: this is the one training product whose operands both have the summed index as their rows. The vendor
+// library runs it with an fp32 C at 0.8 - 1.1 PFLOP/s, and with few tokens (626 of each of 8 experts, 3072 x 16384) at 0.48. Here both
+// operands stream through LDS as they lie and are read transposed (ds_read_b64_tr_b16): no operand needs a transposed copy.
 //
-// Geometry: 256 x 256 tile, 8 waves (2 along M x 4 along N), 128 x 64 per wave as 4 x 2
-// v_mfma_f32_32x32x16_bf16 accumulators. K streams through an LDS ring of R slabs of 16 k rows
-// (A and B, two [16][128] halves each: 16 KiB per slab). Phase s:
-//   (a) issues slab s+D (2 LDS-DMA per thread) into the slot of a slab every wave has consumed,
-//   (b) s_waitcnt vmcnt(N) + s_barrier: the slab the NEXT phase reads has landed in every wave's
-//       DMA (D-1 or D-2 slabs stay in flight across each barrier; never vmcnt(0) in the loop),
-//   (c) reads the next phase's fragments (ds_read_b64_tr_b16) into the other register set,
-//   (d) runs its 8 MFMAs on the fragments read one phase earlier.
-// STAGGER: the two wave groups (A rows 0-127 / 128-255: one wave of each per SIMD) run one barrier
-// apart with two barriers per phase, so each SIMD alternates between the groups' MFMA clusters and
-// one group's barrier/wait/read latency hides under the other's MFMAs.
-// Block order: XCD-aware remap + GROUP_M super-rows so blocks on one XCD share A/B tiles in L2.
+// us, the library with fp32 C / the kernel that was here (32 x 32 x 16 products, slabs of 16, whole tiles and 128 tokens only) / here:
+// 28672 x 4096, 8192 tokens 1684 / 1579 / 1481, 2777 tokens 633 / - / 528; 4096 x 4096, 8192 tokens 252 / 221 / 197; 2048 x 2048, 4096 tokens
+// 46 / 85 / 43; 8 experts of 1280 tokens, 4096 x 28672 2696 / 2460 / 2347, of 626, 8192 x 3072 500 / - / 330.
+//
+// What bounds it: as in gemm_tn.hip, whose loop this is (sxe_gemm_loop.h), plus C, 128 MB of fp32 in a round of workgroups. A tile is
+// 256 x 256 (128 x 256 or splits of the tokens where a plan of rounds finds them shorter), slabs of 64 tokens, rows of 256 or 128
+// columns, chunk c (8 columns) of token t at place c ^ (4 (t & 3) + 2 ((t >> 3) & 1)): a transposing read takes 4 columns of 4
+// tokens a lane, the four tokens' 32 bytes from four 64-byte groups of banks, neighbouring groups of lanes from the two halves of
+// these. The tokens behind the last whole slab are cleared to zeros in LDS. Stores take whole cache lines (gl::store_lines).
 #include "sxe_common.h"
+#include "sxe_gemm_loop.h"
 #include <torch/library.h>
+#include <cmath>
 
 namespace sxe {
 namespace wg {
+using namespace gl;
 
-constexpr int BM = 256, BN = 256, SLAB = 16;
-constexpr int NWAVE = 8, NTHR = NWAVE * 64;
-constexpr int ROWB = 256;                   // bytes per LDS row (128 bf16)
-constexpr int HALF = SLAB * ROWB;           // one [16][128] half slab = 4 KiB
-constexpr int SLOT = 4 * HALF;              // A (2 halves) + B (2 halves) = 16 KiB
-constexpr int GROUP_M = 8;  // default super-row height (runtime argument of the kernels)
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef short i16x4 __attribute__((ext_vector_type(4)));
-typedef short i16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-// LDS image of a [k][128] half tile: 16-byte chunk ch of row r sits at chunk position ch ^ swz(r).
-// Only transposed reads touch it: one ds_read_b64_tr_b16 covers rows r0+q (q = 0..3) x 64 bytes per
-// 32-lane half, and the XOR by (q << 2) puts those four rows on four different 64-byte bank
-// groups (conflict-free); the DMA writes whole 256-byte rows and cannot conflict.
-__device__ __forceinline__ int swz(int row) { return (row & 3) << 2; }
-
-__device__ __forceinline__ i16x4 lds_tr(const char* base, int byte_off) {
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      (__attribute__((address_space(3))) i16x4*)(const_cast<char*>(base) + byte_off));
-}
-
-// MFMA operand (A or B of 32x32x16) from a row-major [k][128] LDS half tile, transposed: lane gets
-// column 32*dt + (lane&31); element j of lane half h <- k row row0 + 8*(j>>2) + 4h + (j&3).
-// A and B use the same k permutation, so it cancels in the product.
-// frag_off(dt, lane): the lane's byte offset for row0 = 0; row0 (a multiple of 4) only adds
-// row0 * ROWB, because the swizzle depends on row & 3 alone -- so a phase's reads are one base
-// VGPR per column block + compile-time immediates.
-__device__ __forceinline__ int frag_off(int dt, int lane) {
-  const int g = lane >> 4, i = lane & 15, q = i >> 2, p = i & 3, h = g >> 1;
-  const int ch = 4 * dt + 2 * (g & 1) + (p >> 1);
-  const int row = 4 * h + q;
-  return row * ROWB + 16 * (ch ^ swz(row)) + 8 * (p & 1);
-}
-
-__device__ __forceinline__ bf16x8 frag_at(const char* lane_base, int row0) {
-  i16x4 lo = lds_tr(lane_base, row0 * ROWB);
-  i16x4 hi = lds_tr(lane_base, (row0 + 8) * ROWB);
-  const i16x8 c = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-  return __builtin_bit_cast(bf16x8, c);
-}
-
-// LDS-DMA issued from inline asm: hipcc's waitcnt pass cannot see it, so it does not put a
-// conservative `s_waitcnt vmcnt(0)` in front of every ds_read of the ring (it did with the
-// builtin: the whole prefetch drained each K-step). Completion is tracked by the explicit counted
-// vmcnt + barrier in the main loop. `lds` is the wave-uniform LDS byte address (M0), which the load reads
-// one wait state behind the scalar write at the earliest (s_nop).
-__device__ __forceinline__ void glds16(const void* gsrc, unsigned lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(gsrc) : "memory", "m0");
-}
-
-// Per-thread DMA source/destination of one slab. Wave w moves 4 k rows x 256 bytes of A-half
-// (w>>2)&1 (first instruction) and of B-half (w>>2)&1 (second): rows 4*(w&3) + (lane>>4) of the
-// slab, 16-byte chunk (lane&15) ^ swz(row). Slab j is the same pattern shifted by 16j rows (a
-// scalar offset) into its ring slot.
-struct DmaPlan {
-  const unsigned short* a;  // A source at k row = row-in-slab
-  const unsigned short* b;
-  unsigned lds_a, lds_b;    // LDS byte address of this wave's 1 KiB pieces in slot 0
+struct Args {
+  const unsigned short *a, *b, *a2, *b2;  // first and second piece of the tokens
+  float *c, *part;                        // part: sums of the splits, [splits, M, N]
+  int64_t lda, ldb, ldc;
+  int64_t ba, bb, ba2, bb2, bc;           // elements from expert to expert
+  int M, N, n1, slabs, per, tail, tail2;  // slabs of the first piece, of both, of a split; tokens behind the last slab of each piece
+  int tm, tn, gm, parts;                  // whole row tiles, column blocks; row tiles side by side; splits or experts
+  float alpha;
 };
 
-__device__ __forceinline__ DmaPlan dma_plan(const unsigned short* A, int64_t lda, const unsigned short* B,
-                                            int64_t ldb, int m0, int n0, unsigned lds_base) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int half = (w >> 2) & 1, rq = w & 3;
-  const int row = 4 * rq + (lane >> 4);
-  const int ch = (lane & 15) ^ swz(row);
-  DmaPlan d;
-  d.a = A + (int64_t)row * lda + m0 + half * 128 + ch * 8;
-  d.b = B + (int64_t)row * ldb + n0 + half * 128 + ch * 8;
-  d.lds_a = __builtin_amdgcn_readfirstlane(lds_base + half * HALF + 4 * rq * ROWB);
-  d.lds_b = __builtin_amdgcn_readfirstlane(lds_base + (2 + half) * HALF + 4 * rq * ROWB);
-  return d;
+// offset in LDS of a lane's transposing reads, rows of `bytes`, 16 columns from chunk `ch` on: tokens 8 (lane >> 4) .. and, 4 rows on,
+// the next four
+__device__ __forceinline__ int tr_off(int lane, int bytes, int ch) {
+  const int g = lane >> 4, q = (lane >> 2) & 3, p = lane & 3;
+  return (8 * g + q) * bytes + 16 * ((ch + (p >> 1)) ^ (4 * q + 2 * (g & 1))) + 8 * (p & 1);
 }
 
-__device__ __forceinline__ void load_slab(const DmaPlan& d, int64_t lda, int64_t ldb, int slab, int slot) {
-  const int r = SLAB * slab;
-  glds16(d.a + (int64_t)r * lda, d.lds_a + slot * SLOT);
-  glds16(d.b + (int64_t)r * ldb, d.lds_b + slot * SLOT);
-}
+template <typename T, bool ACCUM, bool SPLIT>
+__global__ void __launch_bounds__(T::NTHR, T::WAVES) wgrad_kernel(Args a) {
+  constexpr int RT = T::RT, CT = T::CT, NW = T::NW, PA = T::PA, PB = T::PB, BM = T::BM, BN = T::BN, X_LDS = T::SA * T::AS;
+  constexpr int XROW = 2 * BM, WROW = 2 * BN, XL = XROW / 16, WL = WROW / 16, XK = 64 / XL, WK = 64 / WL;  // lanes of a row, rows of a load
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wr = w / T::WC, wc = w % T::WC;
+  // ---- workgroup -> (split or expert, row tile, column block), as gemm_tn.hip
+  const int whole = a.tm * a.tn * a.parts;
+  const bool rest = (int)blockIdx.x >= whole;
+  const int block = rest ? blockIdx.x - whole : blockIdx.x, nwg = rest ? gridDim.x - whole : whole;
+  const int q8 = nwg / 8, r8 = nwg % 8, xcd = block % 8;
+  const int id = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + block / 8;
+  const int nt = rest ? a.tn : a.tm * a.tn, part = a.parts > 1 ? id / nt : 0, tile = id - part * nt;
+  const int per_group = a.gm * a.tn, group = tile / per_group, in = tile - group * per_group, rows = min(a.tm - group * a.gm, a.gm);
+  const int m0 = (rest ? a.tm : group * a.gm + in % rows) * BM, n0 = (rest ? tile : in / rows) * BN;
+  const int first = SPLIT ? part * a.per : 0, ns = SPLIT ? min(a.per, a.slabs - first) : a.slabs;
+  const int expert = SPLIT ? 0 : part;
 
-__device__ __forceinline__ int acc_row(int i, int h) { return (i & 3) + 8 * (i >> 2) + 4 * h; }
+  // ---- loads: a wave's are XK (WK) tokens; columns behind the last repeat it
+  const int xk = XK * w + lane / XL, wk = WK * w + lane / WL;
+  const int xc = 2 * min(m0 + 8 * ((lane % XL) ^ (4 * (xk & 3) + 2 * ((xk >> 3) & 1))), a.M - 8);
+  const int wcol = 2 * min(n0 + 8 * ((lane % WL) ^ (4 * (wk & 3) + 2 * ((wk >> 3) & 1))), a.N - 8);
+  const unsigned xo = (unsigned)xk * (unsigned)(2 * a.lda) + xc, wo = (unsigned)wk * (unsigned)(2 * a.ldb) + wcol;
+  const unsigned short *pa = a.a + expert * a.ba, *pb = a.b + expert * a.bb, *pa2 = a.a2 + expert * a.ba2, *pb2 = a.b2 + expert * a.bb2;
+  const unsigned l0 = lds_base();
+  auto tokens_a = [&](int slab) { return slab < a.n1 ? pa + (int64_t)slab * BK * a.lda : pa2 + (int64_t)(slab - a.n1) * BK * a.lda; };
+  auto tokens_b = [&](int slab) { return slab < a.n1 ? pb + (int64_t)slab * BK * a.ldb : pb2 + (int64_t)(slab - a.n1) * BK * a.ldb; };
+  auto load_x = [&](int i, int slab, unsigned slot) {
+    glds(xo, tokens_a(first + min(slab, ns - 1)) + (int64_t)(i * NW * XK) * a.lda, l0 + slot + (i * NW + w) * 1024);
+  };
+  auto load_w = [&](int i, int slab, unsigned slot) {
+    glds(wo, tokens_b(first + min(slab, ns - 1)) + (int64_t)(i * NW * WK) * a.ldb, l0 + X_LDS + slot + (i * NW + w) * 1024);
+  };
 
-// Two K segments (A, B) rows [0, 16 ns1) then (A2, B2) rows [0, K - 16 ns1), same leading dims: the
-// product over the concatenated token axis without materialising the concatenation (the deferred
-// expert weight gradients of moe/experts.py: the stashed micro-step, then the boundary one).
-// ns1 = K / 16 (and A2 = A, B2 = B) for one segment.
-template <bool ACCUM, int R, bool STAGGER, bool NODMA = false, bool SEG2 = false>
-__global__ void __launch_bounds__(NTHR, 1) wgrad_kernel(const unsigned short* __restrict__ A, int64_t lda,
-                                                        const unsigned short* __restrict__ B, int64_t ldb,
-                                                        float* __restrict__ C, int64_t ldc, int M, int N, int K,
-                                                        float alpha, int group_m, const unsigned short* A2,
-                                                        const unsigned short* B2, int ns1) {
-  static_assert(R == 8, "fragment bases assume slots 0-3 / 4-7");
-  constexpr int D = STAGGER ? R - 3 : R - 2;              // prefetch distance in slabs
-  constexpr int WAIT = STAGGER ? 2 * (D - 2) : 2 * (D - 1);  // DMA left in flight at each wait
-  extern __shared__ __attribute__((aligned(1024))) char smem[];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int wr = w >> 2, wc = w & 3;
-  // ---- block -> tile (XCD-aware, grouped along M) ------------------------------------------
-  const int tm = M / BM, tn = N / BN, nwg = tm * tn;
-  const int orig = blockIdx.x;
-  const int q = nwg / 8, r = nwg % 8, xcd = orig % 8;
-  const int wgid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + orig / 8;
-  const int per_group = group_m * tn;
-  const int grp = wgid / per_group;
-  const int first_m = grp * group_m;
-  const int gsz = min(tm - first_m, group_m);
-  const int bm = first_m + (wgid % per_group) % gsz;
-  const int bn = (wgid % per_group) / gsz;
-  const int m0 = bm * BM, n0 = bn * BN;
+  int ao[RT], bo[CT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i) ao[i] = tr_off(lane, XROW, 2 * (wr * RT + i));
+#pragma unroll
+  for (int j = 0; j < CT; ++j) bo[j] = X_LDS + tr_off(lane, WROW, 2 * (wc * CT + j));
+  auto frag = [](bf16x8& f, int o, int four) {
+    const i16x4 lo = lds_tr(tl::lds, o), hi = lds_tr(tl::lds, o + four);
+    f = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  auto read_x = [&](bf16x8& f, int s, int i, unsigned slot) { frag(f, ao[i] + slot + s * 32 * XROW, 4 * XROW); };
+  auto read_w = [&](bf16x8& f, int s, int j, unsigned slot) { frag(f, bo[j] + slot + s * 32 * WROW, 4 * WROW); };
 
-  f32x16 acc[4][2];
+  f32x4 acc[RT][CT];
+  const int live = __builtin_amdgcn_readfirstlane(min(max((a.M - m0 - wr * RT * 16 + 15) / 16, 0), RT));
+  if (ns > 0) {
+    loop<T>(acc, ns, false, !rest, live, load_x, load_w, read_x, read_w);
+  } else {
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
-  const int ns = K / SLAB;  // a multiple of R (host check)
-  bf16x8 fa[2][4], fb[2][2];
-  // per-lane fragment bases: A columns wr*128 .. +128 (4 blocks of 32), B columns
-  // (wc>>1)*128 + (wc&1)*64 .. +64 (2 blocks); slots 0-3 from base 0, slots 4-7 from base 1 (the
-  // ds_read immediate offset field is 16 bits)
-  const char* fbase[2][6];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) fbase[h][i] = smem + 4 * h * SLOT + wr * HALF + frag_off(i, lane);
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-      fbase[h][4 + j] = smem + 4 * h * SLOT + (2 + (wc >> 1)) * HALF + frag_off((wc & 1) * 2 + j, lane);
+      for (int j = 0; j < CT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  auto read_frags = [&](int slot, bf16x8 (&a)[4], bf16x8 (&b)[2]) {
+  // less than a slab of tokens at the end of a piece: zeros behind them, in both operands
+#pragma unroll 1
+  for (int piece = 0; piece < 2; ++piece) {
+    const int tail = piece ? a.tail2 : a.tail;
+    if (tail == 0 || first + ns != a.slabs) continue;
+    __builtin_amdgcn_s_barrier();  // nobody reads the slots any more, and no load writes them
+    asm volatile("" ::: "memory");
+    const unsigned short* ta = piece ? pa2 + (int64_t)(a.slabs - a.n1) * BK * a.lda : pa + (int64_t)a.n1 * BK * a.lda;
+    const unsigned short* tb = piece ? pb2 + (int64_t)(a.slabs - a.n1) * BK * a.ldb : pb + (int64_t)a.n1 * BK * a.ldb;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) a[i] = frag_at(fbase[slot >> 2][i] + (slot & 3) * SLOT, 0);
+    for (int i = 0; i < PA; ++i)
+      glds((unsigned)min(i * NW * XK + xk, tail - 1) * (unsigned)(2 * a.lda) + xc, ta, l0 + (i * NW + w) * 1024);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) b[j] = frag_at(fbase[slot >> 2][4 + j] + (slot & 3) * SLOT, 0);
-  };
-  auto mma = [&](const bf16x8 (&a)[4], const bf16x8 (&b)[2]) {
-    __builtin_amdgcn_s_setprio(1);
+    for (int i = 0; i < PB; ++i)
+      glds((unsigned)min(i * NW * WK + wk, tail - 1) * (unsigned)(2 * a.ldb) + wcol, tb, l0 + X_LDS + (i * NW + w) * 1024);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    for (int o = tail * XROW + threadIdx.x * 16; o < BK * XROW; o += T::NTHR * 16) *reinterpret_cast<u32x4*>(tl::lds + o) = u32x4{0u, 0u, 0u, 0u};
+    for (int o = tail * WROW + threadIdx.x * 16; o < BK * WROW; o += T::NTHR * 16)
+      *reinterpret_cast<u32x4*>(tl::lds + X_LDS + o) = u32x4{0u, 0u, 0u, 0u};
+    __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int s = 0; s < 2; ++s) {
+      bf16x8 fb[CT];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    __builtin_amdgcn_s_setprio(0);
-  };
-  const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
-  const DmaPlan dp = dma_plan(A, lda, B, ldb, m0, n0, lds_base);
-  // one-segment instantiations keep the original single DMA plan (SEG2 = false: no second plan's
-  // registers, no per-slab segment test)
-  const DmaPlan dp2 = SEG2 ? dma_plan(A2, lda, B2, ldb, m0, n0, lds_base) : dp;
-  auto load_any = [&](int slab, int slot) {  // slab in the first or the second K segment (wave-uniform)
-    if (!SEG2 || slab < ns1)
-      load_slab(dp, lda, ldb, slab, slot);
-    else
-      load_slab(dp2, lda, ldb, slab - ns1, slot);
-  };
-  // prologue: slabs 0 .. D-1, then the first phase's fragments
+      for (int j = 0; j < CT; ++j) read_w(fb[j], s, j, 0);
 #pragma unroll
-  for (int j = 0; j < D; ++j) load_any(j, j);
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(WAIT) : "memory");
-  __builtin_amdgcn_s_barrier();
-  read_frags(0, fa[0], fb[0]);
-  if (STAGGER && __builtin_amdgcn_readfirstlane(wr) == 1) __builtin_amdgcn_s_barrier();
-  for (int s0 = 0; s0 < ns; s0 += R) {
+      for (int i = 0; i < RT; ++i) {
+        bf16x8 fa;
+        read_x(fa, s, i, 0);
 #pragma unroll
-    for (int j = 0; j < R; ++j) {  // phase s = s0 + j, slab s in slot j
-      // the surplus DMA of the last D phases (clamped to the last slab) lands in consumed slots
-      if (!NODMA) load_any(min(s0 + j + D, ns - 1), (j + D) % R);
-      if (NODMA)  // ablation (variant 3): the ring is never refilled -- MFMA + LDS + barrier ceiling
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      else
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(WAIT) : "memory");
-      __builtin_amdgcn_s_barrier();
-      read_frags((j + 1) % R, fa[(j + 1) & 1], fb[(j + 1) & 1]);
-      mma(fa[j & 1], fb[j & 1]);
-      if (STAGGER) __builtin_amdgcn_s_barrier();
-    }
-  }
-  if (STAGGER && __builtin_amdgcn_readfirstlane(wr) == 0) __builtin_amdgcn_s_barrier();
-  // ---- epilogue: C (+)= alpha * acc, two accumulator tiles (32 values / lane) per batch so the
-  // C reads are in flight together instead of one dependent round trip per value
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  const int h = lane >> 5, col = lane & 31;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float* rowp[2];
-    float old[2][16];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      rowp[j] = C + (int64_t)(m0 + wr * 128 + i * 32) * ldc + n0 + wc * 64 + j * 32 + col;
-      if (ACCUM) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) old[j][e] = __builtin_nontemporal_load(rowp[j] + (int64_t)acc_row(e, h) * ldc);
+        for (int j = 0; j < CT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa, acc[i][j], 0, 0, 0);
       }
     }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+
+  // ---- a lane has four columns of a row in each block; two lanes with neighbouring rows change one of two neighbouring blocks, so that
+  // a store writes 32 columns of 8 rows, whole lines
+  const int l16 = lane & 15, g = lane >> 4;
+  const bool odd = lane & 1;
+  float* out = SPLIT ? a.part + (int64_t)part * a.M * a.N : a.c + expert * a.bc;
+  const int64_t ld = SPLIT ? a.N : a.ldc;
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+  for (int i = 0; i < RT; ++i) {
+    const int r = m0 + (wr * RT + i) * 16 + (l16 & ~1);
+    float* p[2];
+    f32x4 old[2][2];
+    bool in_row[2], in_col[2];
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const float v = alpha * acc[i][j][e];
-        rowp[j][(int64_t)acc_row(e, h) * ldc] = ACCUM ? old[j][e] + v : v;
+    for (int h = 0; h < 2; ++h) {
+      p[h] = out + (int64_t)(r + h) * ld;
+      in_row[h] = r + h < a.M;
+      in_col[h] = n0 + wc * 64 + 32 * h + 16 * odd + 4 * g < a.N;
+    }
+    if (ACCUM) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+          if (in_row[k] && in_col[h]) old[h][k] = *reinterpret_cast<const f32x4*>(p[k] + n0 + wc * 64 + 32 * h + 16 * odd + 4 * g);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      f32x4 v[2], t;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[0][e] = SPLIT ? acc[i][2 * h][e] : a.alpha * acc[i][2 * h][e];
+        v[1][e] = SPLIT ? acc[i][2 * h + 1][e] : a.alpha * acc[i][2 * h + 1][e];
+        t[e] = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, odd ? v[0][e] : v[1][e]), 0xB1, 0xF, 0xF, true));
       }
+      f32x4 lo = odd ? t : v[0], hi = odd ? v[1] : t;
+      if (ACCUM) lo += old[h][0], hi += old[h][1];
+      const int c = n0 + wc * 64 + 32 * h + 16 * odd + 4 * g;
+      if (in_col[h]) {
+        if (in_row[0]) *reinterpret_cast<f32x4*>(p[0] + c) = lo;
+        if (in_row[1]) *reinterpret_cast<f32x4*>(p[1] + c) = hi;
+      }
+    }
   }
 }
 
-
-// ---------------------------------------------------------------------------------------------
-// Variant 2: 4 waves (one per SIMD), 2 x 2 waves of 128 x 128 (4 x 4 accumulators = 256 fp32 per
-// lane, in AGPRs), slabs of 32 k rows (32 KiB: A and B, two [32][128] halves each) in a ring of 4.
-// Per phase a wave runs 32 MFMAs between barriers (twice the MFMA work per barrier of the 8-wave
-// form) and reads 1 ds_read_b64_tr_b16 per MFMA. Every wave drains its LDS reads (lgkmcnt(0),
-// already complete: they fed this phase) before the barrier, so the slot of the slab consumed in
-// the previous phase can be refilled right after it: prefetch distance 3 slabs.
-namespace w4 {
-constexpr int SLAB = 32, R = 4, D = 3;
-constexpr int NTHR = 256;
-constexpr int HALF = SLAB * ROWB;           // [32][128] bf16 = 8 KiB
-constexpr int SLOT = 4 * HALF;              // 32 KiB
-constexpr int WAIT = 8 * (D - 1);           // DMA per slab per thread = 8
-
-struct Plan {
-  const unsigned short* a;  // A at (k row lane>>4, this lane's swizzled chunk)
-  const unsigned short* b;
-  unsigned lds;             // LDS byte address of slot 0
-};
-
+// C (+)= alpha * the splits' sums, 4 columns a thread
 template <bool ACCUM>
-__global__ void __launch_bounds__(NTHR, 1) kernel(const unsigned short* __restrict__ A, int64_t lda,
-                                                  const unsigned short* __restrict__ B, int64_t ldb,
-                                                  float* __restrict__ C, int64_t ldc, int M, int N, int K,
-                                                  float alpha, int group_m, const unsigned short* A2,
-                                                  const unsigned short* B2, int ns1) {
-  extern __shared__ __attribute__((aligned(1024))) char smem[];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int wr = w >> 1, wc = w & 1;
-  const int tm = M / BM, tn = N / BN, nwg = tm * tn;
-  const int orig = blockIdx.x;
-  const int q = nwg / 8, r = nwg % 8, xcd = orig % 8;
-  const int wgid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + orig / 8;
-  const int per_group = group_m * tn;
-  const int grp = wgid / per_group;
-  const int first_m = grp * group_m;
-  const int gsz = min(tm - first_m, group_m);
-  const int bm = first_m + (wgid % per_group) % gsz;
-  const int bn = (wgid % per_group) / gsz;
-  const int m0 = bm * BM, n0 = bn * BN;
-
-  f32x16 acc[4][4];
+__global__ void __launch_bounds__(256) sum_kernel(const float* __restrict__ part, float* __restrict__ c, int64_t ldc, int M, int N, int splits,
+                                                  float alpha) {
+  const int64_t all = (int64_t)M * N;
+  const int per = N / 4;
+  for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < (int64_t)M * per; i += gridDim.x * 256ll) {
+    const int64_t r = i / per, o = r * N + 4 * (i - r * per);
+    f32x4 s = *reinterpret_cast<const f32x4*>(part + o);
+    for (int k = 1; k < splits; ++k) s += *reinterpret_cast<const f32x4*>(part + k * all + o);
+    f32x4* to = reinterpret_cast<f32x4*>(c + r * ldc + 4 * (i - r * per));
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
-  // DMA: slab rows 4*rq + (lane>>4), rq = 0..7; the 32 wave-instructions of a slab are
-  // (op, half, rq) = (it>>2, (it>>1)&1, (it&1)*4 + w) for it = 0..7
-  Plan pl, pl2;
-  {
-    const int row = lane >> 4;  // row & 3 == (lane >> 4) & 3 for every rq
-    const int ch = (lane & 15) ^ swz(row);
-    pl.a = A + (int64_t)row * lda + m0 + ch * 8;
-    pl.b = B + (int64_t)row * ldb + n0 + ch * 8;
-    pl.lds = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
-    pl2 = pl;
-    pl2.a = A2 + (int64_t)row * lda + m0 + ch * 8;
-    pl2.b = B2 + (int64_t)row * ldb + n0 + ch * 8;
-  }
-  const int ns1_32 = ns1 / 2;  // 16-row slabs of the first segment -> 32-row slabs (host: ns1 even)
-  auto load_slab = [&](int slab_any, int slot) {
-    const bool second = slab_any >= ns1_32;
-    const Plan& P = second ? pl2 : pl;
-    const int slab = second ? slab_any - ns1_32 : slab_any;
-#pragma unroll
-    for (int it = 0; it < 8; ++it) {
-      const int op = it >> 2, half = (it >> 1) & 1, rq = (it & 1) * 4 + w;
-      const int64_t rows = (int64_t)SLAB * slab + 4 * rq;
-      const unsigned short* src = op == 0 ? P.a + rows * lda + half * 128 : P.b + rows * ldb + half * 128;
-      const unsigned dst = __builtin_amdgcn_readfirstlane(pl.lds + slot * SLOT + (op * 2 + half) * HALF + 4 * rq * ROWB);
-      glds16(src, dst);
-    }
-  };
-  // fragment bases: A half wr (columns wr*128 + 32i), B half wc (columns wc*128 + 32j); slots
-  // 0-1 from base 0, slots 2-3 from base 1 (16-bit ds_read immediate offsets)
-  const char* fa_base[2][4];
-  const char* fb_base[2][4];
-#pragma unroll
-  for (int hb = 0; hb < 2; ++hb)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      fa_base[hb][i] = smem + 2 * hb * SLOT + wr * HALF + frag_off(i, lane);
-      fb_base[hb][i] = smem + 2 * hb * SLOT + (2 + wc) * HALF + frag_off(i, lane);
-    }
-  bf16x8 fa[2][2][4], fb[2][2][4];  // [register set][k16 step][block]
-  auto read_frags = [&](int slot, bf16x8 (&a)[2][4], bf16x8 (&b)[2][4]) {
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        a[kk][i] = frag_at(fa_base[slot >> 1][i] + (slot & 1) * SLOT, 16 * kk);
-        b[kk][i] = frag_at(fb_base[slot >> 1][i] + (slot & 1) * SLOT, 16 * kk);
-      }
-  };
-  auto mma = [&](const bf16x8 (&a)[2][4], const bf16x8 (&b)[2][4]) {
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kk][i], b[kk][j], acc[i][j], 0, 0, 0);
-    __builtin_amdgcn_s_setprio(0);
-  };
-  const int ns = K / SLAB;  // a multiple of R (host check)
-#pragma unroll
-  for (int j = 0; j < D; ++j) load_slab(j, j);
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(WAIT) : "memory");
-  __builtin_amdgcn_s_barrier();
-  read_frags(0, fa[0], fb[0]);
-  for (int s0 = 0; s0 < ns; s0 += R) {
-#pragma unroll
-    for (int j = 0; j < R; ++j) {  // phase s = s0 + j: slab s in slot j
-      load_slab(min(s0 + j + D, ns - 1), (j + D) % R);  // surplus DMA at the end lands in consumed slots
-      asm volatile("s_waitcnt vmcnt(%0)\n\ts_waitcnt lgkmcnt(0)" ::"n"(WAIT) : "memory");
-      __builtin_amdgcn_s_barrier();
-      read_frags((j + 1) % R, fa[(j + 1) & 1], fb[(j + 1) & 1]);
-      mma(fa[j & 1], fb[j & 1]);
-    }
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  const int h = lane >> 5, col = lane & 31;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float* rowp[4];
-    float old[4][16];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      rowp[j] = C + (int64_t)(m0 + wr * 128 + i * 32) * ldc + n0 + wc * 128 + j * 32 + col;
-      if (ACCUM) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) old[j][e] = __builtin_nontemporal_load(rowp[j] + (int64_t)acc_row(e, h) * ldc);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const float v = alpha * acc[i][j][e];
-        rowp[j][(int64_t)acc_row(e, h) * ldc] = ACCUM ? old[j][e] + v : v;
-      }
+    for (int e = 0; e < 4; ++e) s[e] *= alpha;
+    *to = ACCUM ? *to + s : s;
   }
 }
-}  // namespace w4
 
-}  // namespace wg
+using T256 = Tile<2, 4, 8, 4, 2, 3, 2>;  // 256 x 256
+using T128 = Tile<2, 4, 4, 4, 3, 3, 2>;  // 128 x 256
 
-bool wgrad_supported(const at::Tensor& a, const at::Tensor& b, const at::Tensor& c) {
-  return a.is_cuda() && a.scalar_type() == at::kBFloat16 && b.scalar_type() == at::kBFloat16 &&
-         c.scalar_type() == at::kFloat && a.dim() == 2 && b.dim() == 2 && c.dim() == 2 && a.stride(1) == 1 &&
-         b.stride(1) == 1 && c.stride(1) == 1 && a.size(0) == b.size(0) && c.size(0) == a.size(1) &&
-         c.size(1) == b.size(1) && a.size(1) % wg::BM == 0 && b.size(1) % wg::BN == 0 && a.size(0) % (8 * wg::SLAB) == 0 &&
-         (reinterpret_cast<uintptr_t>(a.data_ptr()) % 16 == 0) && (reinterpret_cast<uintptr_t>(b.data_ptr()) % 16 == 0) &&
-         a.stride(0) % 8 == 0 && b.stride(0) % 8 == 0;
-}
-
-// c (+)= alpha * a^T @ b ; a: [K, M] bf16, b: [K, N] bf16, c: [M, N] fp32.
-// variant: 0 = 8 lock-step waves, 1 = 8 staggered waves, 2 = 4 waves of 128 x 128, for in-process A/B.
-static void wgrad_launch(const at::Tensor& a, const at::Tensor& b, const at::Tensor& a2, const at::Tensor& b2, int K,
-                         int ns1, at::Tensor c, double alpha, bool accumulate, int64_t variant, bool seg2 = false) {
-  c10::DeviceGuard g(a.device());
-  const int M = a.size(1), N = b.size(1);
-  const int nwg = (M / wg::BM) * (N / wg::BN);
-  const size_t lds = 8 * wg::SLOT;
-  using Kern = void (*)(const unsigned short*, int64_t, const unsigned short*, int64_t, float*, int64_t, int, int,
-                        int, float, int, const unsigned short*, const unsigned short*, int);
-  const int group_m = variant >= 16 ? (int)(variant >> 4) : wg::GROUP_M;  // A/B knob: variant + 16 * group_m
-  variant &= 15;
-  static const Kern kerns[5][2] = {{wg::wgrad_kernel<false, 8, false>, wg::wgrad_kernel<true, 8, false>},
-                                   {wg::wgrad_kernel<false, 8, true>, wg::wgrad_kernel<true, 8, true>},
-                                   {wg::w4::kernel<false>, wg::w4::kernel<true>},
-                                   {wg::wgrad_kernel<false, 8, false, true>, wg::wgrad_kernel<true, 8, false, true>},
-                                   {wg::wgrad_kernel<false, 8, false, false, true>,
-                                    wg::wgrad_kernel<true, 8, false, false, true>}};
-  static bool attr_set = [&] {
-    for (auto& row : kerns)
-      for (Kern k : row)
-        SXE_HIP_CHECK(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    return true;
-  }();
-  (void)attr_set;
-  SXE_CHECK(variant >= 0 && variant <= 3, "wgrad_gemm_: variant must be 0..3");
-  SXE_CHECK(!seg2 || variant == 0, "wgrad_gemm2_: the 8-wave lock-step schedule only");
-  const int nthr = variant == 2 ? wg::w4::NTHR : wg::NTHR;
-  hipLaunchKernelGGL(kerns[seg2 ? 4 : variant][accumulate ? 1 : 0], dim3(nwg), dim3(nthr), lds, cur_stream(),
-                     reinterpret_cast<const unsigned short*>(a.data_ptr()), a.stride(0),
-                     reinterpret_cast<const unsigned short*>(b.data_ptr()), b.stride(0), c.data_ptr<float>(),
-                     c.stride(0), M, N, K, (float)alpha, group_m, reinterpret_cast<const unsigned short*>(a2.data_ptr()),
-                     reinterpret_cast<const unsigned short*>(b2.data_ptr()), ns1);
+template <typename T, bool ACCUM>
+static void launch(Args a, int splits, int experts) {
+  a.tm = a.M / T::BM;
+  a.tn = (a.N + T::BN - 1) / T::BN;
+  a.gm = std::max(1, std::min(a.tm, 8));
+  a.parts = splits * experts;  // one of them is 1
+  const int64_t grid = ((int64_t)a.M + T::BM - 1) / T::BM * a.tn * a.parts;
+  SXE_CHECK(grid < (1ll << 30), "wgrad_gemm: too many tiles");
+  if (splits > 1) {
+    allow_lds<&wgrad_kernel<T, false, true>>(T::LDS);
+    hipLaunchKernelGGL((wgrad_kernel<T, false, true>), dim3((unsigned)grid), dim3(T::NTHR), T::LDS, cur_stream(), a);
+    hipLaunchKernelGGL(sum_kernel<ACCUM>, dim3(stream_grid((int64_t)a.M * a.N / 4, 256)), dim3(256), 0, cur_stream(), a.part, a.c, a.ldc,
+                       a.M, a.N, splits, a.alpha);
+  } else {
+    allow_lds<&wgrad_kernel<T, ACCUM, false>>(T::LDS);
+    hipLaunchKernelGGL((wgrad_kernel<T, ACCUM, false>), dim3((unsigned)grid), dim3(T::NTHR), T::LDS, cur_stream(), a);
+  }
   SXE_LAUNCH_CHECK();
 }
 
-void wgrad_gemm_variant_(const at::Tensor& a, const at::Tensor& b, at::Tensor c, double alpha, bool accumulate,
-                         int64_t variant) {
-  SXE_CHECK(wgrad_supported(a, b, c), "wgrad_gemm_: unsupported shapes/dtypes/strides");
-  const int K = a.size(0);
-  wgrad_launch(a, b, a, b, K, K / wg::SLAB, c, alpha, accumulate, variant);
+// (tile, splits of the tokens) of the least rounds of workgroups over the CUs, us: a slab 1.45 (256 x 256) or 0.82 (128 x 256), a start
+// with C written 14 or 9, read first 12 or 8 more
+static std::pair<int, int> plan(int64_t M, int64_t N, int64_t slabs, int64_t experts, bool accumulate) {
+  std::pair<int, int> best{0, 1};
+  float least = 1e30f;
+  for (int f = 0; f < 2; ++f) {
+    const int64_t tiles = (M + (f ? 127 : 255)) / (f ? 128 : 256) * ((N + 255) / 256) * experts;
+    for (int s : {1, 2, 3, 4, 6, 8}) {
+      if (s > 1 && (experts > 1 || slabs < 4 * s || tiles * s > 600)) break;
+      const float one = (slabs + s) / s * (f ? 0.82f : 1.45f) + (f ? 9.f : 14.f) + (accumulate && s == 1 ? (f ? 8.f : 12.f) : 0.f);
+      float us = (tiles * s + kNumCUs - 1) / kNumCUs * one;
+      if (s > 1) us += 4.f + M * N * 4 * (2 * s + (accumulate ? 2 : 1)) / 3.6e6f;
+      if (us < least) least = us, best = {f, s};
+    }
+  }
+  return best;
 }
 
-static int64_t default_variant(const at::Tensor& a, const at::Tensor& b) {
-  // 8 lock-step waves; super-rows of 4 M-tiles for tall outputs, 8 otherwise (tools/wgrad_exp.py)
-  const int64_t tm = a.size(1) / wg::BM, tn = b.size(1) / wg::BN;
-  return 0 + 16 * (tm >= 4 * tn ? 4 : 8);
+// operands [T, cols] or [E, T, cols], rows that start on 16 bytes
+static void check_tokens(const at::Tensor& t, int64_t d, const char* name) {
+  SXE_CHECK(t.is_cuda() && t.scalar_type() == at::kBFloat16 && t.dim() == d + 2 && t.stride(d + 1) == 1 && t.size(d + 1) % 8 == 0 &&
+                t.size(d + 1) >= 8 && (t.size(d) <= 1 || t.stride(d) % 8 == 0) && (!d || t.size(0) <= 1 || t.stride(0) % 8 == 0) &&
+                reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && (t.size(d) <= 1 || (t.stride(d) > 0 && t.stride(d) < (1 << 24))),
+            "wgrad_gemm: ", name, " bf16 rows of multiples of 8 columns that start on 16 bytes");
+}
+static int64_t row_stride(const at::Tensor& t, int64_t d) { return t.size(d) > 1 ? t.stride(d) : t.size(d + 1); }
+
+static void run(const at::Tensor& x, const at::Tensor& y, const at::Tensor* x2, const at::Tensor* y2, at::Tensor c, double alpha, bool accumulate,
+                int64_t tile, int64_t splits) {
+  check_beside(x, {y, c});
+  const int64_t d = c.dim() - 2;
+  SXE_CHECK(d == 0 || d == 1, "wgrad_gemm: C [M, N] or [E, M, N]");
+  check_tokens(x, d, "A");
+  check_tokens(y, d, "B");
+  const int64_t M = x.size(d + 1), N = y.size(d + 1), experts = d ? c.size(0) : 1;
+  SXE_CHECK(c.scalar_type() == at::kFloat && c.size(d) == M && c.size(d + 1) == N && x.size(d) == y.size(d) && c.stride(d + 1) == 1 &&
+                (M <= 1 || (c.stride(d) % 4 == 0 && c.stride(d) >= N)) && (!d || experts <= 1 || c.stride(0) % 4 == 0) &&
+                (!d || (x.size(0) == experts && y.size(0) == experts)) && reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 == 0 &&
+                M < (1 << 30) && N < (1 << 30) && x.size(d) < (1ll << 31) && experts < (1 << 16),
+            "wgrad_gemm: fp32 C of rows that start on 16 bytes, as many tokens of A and B");
+  c10::DeviceGuard g(x.device());
+  Args a{};
+  a.a = reinterpret_cast<const unsigned short*>(x.data_ptr());
+  a.b = reinterpret_cast<const unsigned short*>(y.data_ptr());
+  a.a2 = a.a;
+  a.b2 = a.b;
+  a.c = c.data_ptr<float>();
+  a.lda = row_stride(x, d);
+  a.ldb = row_stride(y, d);
+  a.ldc = M > 1 ? c.stride(d) : N;
+  a.M = M;
+  a.N = N;
+  a.alpha = alpha;
+  if (d) {
+    a.ba = x.stride(0);
+    a.bb = y.stride(0);
+    a.bc = c.stride(0);
+  }
+  a.n1 = x.size(d) / BK;
+  a.slabs = a.n1;
+  a.tail = x.size(d) % BK;
+  if (x2 != nullptr) {
+    check_beside(x, {*x2, *y2});
+    check_tokens(*x2, d, "A2");
+    check_tokens(*y2, d, "B2");
+    SXE_CHECK(x2->size(d + 1) == M && y2->size(d + 1) == N && x2->size(d) == y2->size(d) && (!d || (x2->size(0) == experts && y2->size(0) == experts)) &&
+                  x2->size(d) < (1ll << 30) && x.size(d) < (1ll << 30), "wgrad_gemm: pieces of the same columns");
+    if (row_stride(*x2, d) != a.lda || row_stride(*y2, d) != a.ldb) {  // one after the other
+      run(x, y, nullptr, nullptr, c, alpha, accumulate, tile, splits);
+      run(*x2, *y2, nullptr, nullptr, c, alpha, true, tile, splits);
+      return;
+    }
+    a.a2 = reinterpret_cast<const unsigned short*>(x2->data_ptr());
+    a.b2 = reinterpret_cast<const unsigned short*>(y2->data_ptr());
+    if (d) {
+      a.ba2 = x2->stride(0);
+      a.bb2 = y2->stride(0);
+    }
+    a.slabs += x2->size(d) / BK;
+    a.tail2 = x2->size(d) % BK;
+  }
+  if (c.numel() == 0) return;
+  if (a.slabs == 0 && a.tail == 0 && a.tail2 == 0) {
+    if (!accumulate) c.zero_();
+    return;
+  }
+  const auto p = plan(M, N, a.slabs, experts, accumulate);
+  if (tile < 0) tile = p.first;
+  if (splits <= 0) splits = p.second;
+  splits = std::max<int64_t>(1, std::min<int64_t>(splits, a.slabs));
+  SXE_CHECK(tile < 2 && (splits == 1 || experts == 1), "wgrad_gemm: tile 0 or 1, experts or splits");
+  a.per = splits > 1 ? (a.slabs + splits - 1) / splits : a.slabs;
+  if (splits > 1) splits = (a.slabs + a.per - 1) / a.per;  // none of them empty
+  at::Tensor part;
+  if (splits > 1) {
+    part = at::empty({splits, M, N}, c.options());
+    a.part = part.data_ptr<float>();
+  }
+  if (tile == 0) accumulate ? launch<T256, true>(a, splits, experts) : launch<T256, false>(a, splits, experts);
+  else accumulate ? launch<T128, true>(a, splits, experts) : launch<T128, false>(a, splits, experts);
 }
 
+}  // namespace wg
+
+// c (+)= alpha * a' b, a [T, M], b [T, N], c [M, N], or all with a leading expert index
 void wgrad_gemm_(const at::Tensor& a, const at::Tensor& b, at::Tensor c, double alpha, bool accumulate) {
-  wgrad_gemm_variant_(a, b, c, alpha, accumulate, default_variant(a, b));
+  wg::run(a, b, nullptr, nullptr, c, alpha, accumulate, -1, 0);
 }
-
-// c (+)= alpha * [a; a2]^T @ [b; b2] (concatenated along K = rows) without the concatenation:
-// a, a2 [K1 | K2, M], b, b2 [K1 | K2, N], equal leading dims, K1 % 32 == 0, (K1 + K2) % 128 == 0
-bool wgrad2_supported(const at::Tensor& a, const at::Tensor& b, const at::Tensor& a2, const at::Tensor& b2,
-                      const at::Tensor& c) {
-  if (a2.dim() != 2 || b2.dim() != 2 || a2.scalar_type() != a.scalar_type() || b2.scalar_type() != b.scalar_type() ||
-      a2.size(1) != a.size(1) || b2.size(1) != b.size(1) || a2.size(0) != b2.size(0) || a2.stride(1) != 1 ||
-      b2.stride(1) != 1 || a2.stride(0) != a.stride(0) || b2.stride(0) != b.stride(0) || a.size(0) % 32 != 0 ||
-      (reinterpret_cast<uintptr_t>(a2.data_ptr()) % 16) != 0 || (reinterpret_cast<uintptr_t>(b2.data_ptr()) % 16) != 0)
-    return false;
-  const int64_t K = a.size(0) + a2.size(0);
-  if (K % (8 * wg::SLAB) != 0) return false;
-  // the one-segment shape checks, with K = K1 + K2
-  return a.is_cuda() && a.scalar_type() == at::kBFloat16 && b.scalar_type() == at::kBFloat16 &&
-         c.scalar_type() == at::kFloat && a.dim() == 2 && b.dim() == 2 && c.dim() == 2 && a.stride(1) == 1 &&
-         b.stride(1) == 1 && c.stride(1) == 1 && a.size(0) == b.size(0) && c.size(0) == a.size(1) &&
-         c.size(1) == b.size(1) && a.size(1) % wg::BM == 0 && b.size(1) % wg::BN == 0 &&
-         (reinterpret_cast<uintptr_t>(a.data_ptr()) % 16 == 0) && (reinterpret_cast<uintptr_t>(b.data_ptr()) % 16 == 0) &&
-         a.stride(0) % 8 == 0 && b.stride(0) % 8 == 0;
+// The same with a tile (0: 256 x 256, 1: 128 x 256, else the plan's) and splits of the tokens (0: the plan's) of the caller's, for comparisons
+void wgrad_gemm_variant_(const at::Tensor& a, const at::Tensor& b, at::Tensor c, double alpha, bool accumulate, int64_t variant) {
+  const int64_t tile = variant & 15;
+  wg::run(a, b, nullptr, nullptr, c, alpha, accumulate, tile < 2 ? tile : -1, variant >> 4);
 }
-
-void wgrad_gemm2_(const at::Tensor& a, const at::Tensor& b, const at::Tensor& a2, const at::Tensor& b2, at::Tensor c,
-                  double alpha, bool accumulate) {
-  SXE_CHECK(wgrad2_supported(a, b, a2, b2, c), "wgrad_gemm2_: unsupported shapes/dtypes/strides");
-  const int K = (int)(a.size(0) + a2.size(0));
-  wgrad_launch(a, b, a2, b2, K, (int)(a.size(0) / wg::SLAB), c, alpha, accumulate, default_variant(a, b), true);
+// c (+)= alpha * [a; a2]' [b; b2] (one after the other along the tokens) without the concatenation
+void wgrad_gemm2_(const at::Tensor& a, const at::Tensor& b, const at::Tensor& a2, const at::Tensor& b2, at::Tensor c, double alpha,
+                  bool accumulate) {
+  wg::run(a, b, &a2, &b2, c, alpha, accumulate, -1, 0);
 }
 
 }  // namespace sxe

@@ -157,16 +157,16 @@ class _GroupedMM(torch.autograd.Function):
                 dy = torch.cat([g for _, g in stash] + [dy], dim=1)
             if tgt is not None:
                 buf, acc = tgt(w)
-                for e in range(E):
-                    if prev is not None:
-                        x1, g1 = prev[0][e], prev[1][e]
-                        if _wgrad2_ok(x1, g1, x[e], dy[e], buf[e]):
-                            torch.ops.sxe.wgrad_gemm2_(x1, g1, x[e], dy[e], buf[e], 1.0, bool(acc))
-                            continue
-                        _expert_wgrad(x1, g1, buf[e], acc)
-                        _expert_wgrad(x[e], dy[e], buf[e], True)
-                        continue
-                    _expert_wgrad(x[e], dy[e], buf[e], acc)
+                be = buf.view(w.shape)
+                if prev is not None and _wgrad2_ok(prev[0], prev[1], x, dy, be):
+                    torch.ops.sxe.wgrad_gemm2_(prev[0], prev[1], x, dy, be, 1.0, bool(acc))
+                elif prev is None and _wgrad_all_ok(x, dy, be):
+                    torch.ops.sxe.wgrad_gemm_(x, dy, be, 1.0, bool(acc))
+                else:
+                    for e in range(E):
+                        if prev is not None:
+                            _expert_wgrad(prev[0][e], prev[1][e], buf[e], acc)
+                        _expert_wgrad(x[e], dy[e], buf[e], acc or prev is not None)
                 w._sxe_grad_done(w)
             else:
                 dw = torch.empty_like(w)
@@ -192,11 +192,16 @@ def _expert_wgrad(xe, ge, be, acc):
         torch.mm(xe.t(), ge, out=be)
 
 
-def _wgrad2_ok(x1, g1, x2, g2, be):
-    """The two-segment wgrad kernel covers [x1; x2]^T [g1; g2] (no concatenated copy)."""
+def _wgrad_all_ok(x, g, be):
+    """The wgrad kernel takes all experts in one launch: x [E, C, K], g [E, C, N], be [E, K, N]."""
     from ..ops.linear import _sxe_wgrad_ok
-    return (_sxe_wgrad_ok(x1, g1, be) and _sxe_wgrad_ok(x2, g2, be) and x1.stride(0) == x2.stride(0)
-            and g1.stride(0) == g2.stride(0))
+    return native.plain(x, g) and x.stride(0) % 8 == 0 and g.stride(0) % 8 == 0 and _sxe_wgrad_ok(x, g, be)
+
+
+def _wgrad2_ok(x1, g1, x2, g2, be):
+    """... and with the tokens of two micro-steps: [x1; x2]^T [g1; g2] of every expert (no concatenated copy)."""
+    return (_wgrad_all_ok(x1, g1, be) and _wgrad_all_ok(x2, g2, be) and x1.stride(1) == x2.stride(1)
+            and g1.stride(1) == g2.stride(1))
 
 
 def grouped_mm(x, w):

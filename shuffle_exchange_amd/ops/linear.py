@@ -350,30 +350,24 @@ def fused_gatenorm_linear(x, norm_weight, gate, eps, weight):
     return torch.ops.sxe.skinny_gemm_gatenorm(x, norm_weight, gate, float(eps), wk[0])
 
 
-# Hand-written weight-gradient GEMM (csrc/kernels/gemm_wgrad.hip: k-major operands read through LDS
-# with ds_read_b64_tr_b16, fp32 accumulate in the epilogue): no transposed copies of dY / X at all.
-# Measured on MI355X at 8192 tokens (tools/wgrad_exp.py, profiles/wgrad_kernel.log): 28672x4096
-# 1.59 ms vs 1.63 (transposes + hipBLASLt TN fp32-out), 4096x14336 0.84 vs 0.89, 4096x4096 0.24 vs
-# 0.25 (NT fp32-out); it loses where its 256x256 tile grid leaves a partial last wave of blocks
-# (6144x4096: 1.5 waves over 256 CUs, see WGRAD_MIN_TILES) and on the LM head, which keep the
-# library paths.
+# Hand-written weight-gradient GEMM (csrc/kernels/gemm_wgrad.hip: both operands read transposed through LDS, fp32 C): no transposed
+# copies of dY / X, any number of tokens. Beside the library's fp32-output product it is the faster one at every size measured, 2048 x
+# 2048 to 32000 x 3072, 300 - 8192 tokens (figures there).
 SXE_WGRAD = os.environ.get("SXE_WGRAD", "1") == "1"
-# smallest non-multiple-of-256 tile count for the hand-written kernel: the fused QKV projection (384
-# tiles, 1.5 waves) wins in isolation at 8192 tokens (0.43 vs 0.46 ms) but not inside the
-# Llama-3-8B step at 16,384 tokens per micro-step (0.78 vs 0.74 ms per call,
-# profiles/r05/bench_llama3_8b_zero3_1gpu_step_final.md, headline_wgrad_norm_ab.log)
-WGRAD_MIN_TILES = int(os.environ.get("SXE_WGRAD_MIN_TILES", "768"))
 
 
 def _sxe_wgrad_ok(gy2, x2, buf):
+    """gy2 [.., T, M], x2 [.., T, N], buf [.., M, N]: one product, or one for every expert."""
     if not (SXE_WGRAD and gy2.is_cuda and buf.dtype == torch.float32 and gy2.dtype == torch.bfloat16
-            and x2.dtype == torch.bfloat16 and buf.is_contiguous() and gy2.stride(1) == 1 and x2.stride(1) == 1):
+            and x2.dtype == torch.bfloat16 and buf.is_contiguous() and gy2.stride(-1) == 1 and x2.stride(-1) == 1):
         return False
-    K, M, N = gy2.shape[0], gy2.shape[1], x2.shape[1]
-    if K % 128 or M % 256 or N % 256 or gy2.stride(0) % 8 or x2.stride(0) % 8 or M * N >= 2 ** 27:
+    K, M, N = gy2.shape[-2], gy2.shape[-1], x2.shape[-1]
+    if M % 8 or N % 8 or M < 64 or N < 64 or K == 0 or gy2.stride(-2) % 8 or x2.stride(-2) % 8:
         return False
-    tiles = (M // 256) * (N // 256)
-    return tiles % 256 == 0 or tiles >= WGRAD_MIN_TILES
+    if not native.plain(gy2, x2):  # traced: no memory to look at, sizes whose operands start on 16 bytes
+        return K % 128 == 0 and M % 256 == 0 and N % 256 == 0
+    return (gy2.data_ptr() % 16 == 0 and x2.data_ptr() % 16 == 0 and buf.data_ptr() % 16 == 0 and max(gy2.stride(-2), x2.stride(-2)) < 1 << 24
+            and min(gy2.stride(-2), x2.stride(-2)) > 0 and max(M, N, K) < 1 << 30)
 
 
 def _tn_ok(gy2, x2):

@@ -11,6 +11,7 @@ framework registers formulas for its own HIP ops (flash attention fwd/bwd, paged
 no generic counter could know. Module attribution comes from the counter's module tracker;
 latencies from HIP events around each module's forward.
 """
+import math
 import time
 from collections import defaultdict
 
@@ -94,8 +95,8 @@ def _register_sxe_formulas():
             return 2 * x[0] * w[1] * w[2]
 
         @register_flop_formula(ops.wgrad_gemm_)
-        def _wgrad(a, b, *rest, out_shape=None, **kw):  # c (+)= a^T b, a [K, M], b [K, N]
-            return 2 * a[0] * a[1] * b[1]
+        def _wgrad(a, b, *rest, out_shape=None, **kw):  # c (+)= a^T b, a [.., K, M], b [.., K, N]
+            return 2 * math.prod(a) * b[-1]
     except Exception:  # formulas are optional; generic ops are still counted
         pass
 

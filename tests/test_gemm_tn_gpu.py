@@ -123,6 +123,33 @@ def test_training_products(rows):
     _close(L.data_grad(g, wide), g.double() @ wide.double(), g, wide.t())
 
 
+# tokens: inside a slab of 64, whole slabs, more than the slots hold, pieces that end inside a slab; sizes that end inside a tile of 256 or
+# 128, a block of 16, a store of 4 columns; one product or three
+@pytest.mark.parametrize("E,T,T2,M,N", [(0, 1, 0, 8, 8), (0, 63, 0, 264, 40), (0, 64, 0, 128, 256), (0, 577, 0, 192, 1000), (0, 640, 0, 256, 512),
+                                        (0, 128, 72, 256, 264), (0, 100, 30, 136, 256), (3, 70, 0, 264, 128), (3, 90, 65, 264, 128)])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_weight_gradients(E, T, T2, M, N, accumulate):
+    g = torch.Generator("cuda").manual_seed(T + M)
+    batch = (E,) if E else ()
+    a, b, a2, b2 = [torch.randn(*batch, t, n + 8, device="cuda", generator=g).bfloat16()[..., :n] for t in (T, T2) for n in (M, N)]
+    before = torch.randn(*batch, M, N, device="cuda", generator=g)
+    sums = a.double().transpose(-1, -2) @ b.double() + a2.double().transpose(-1, -2) @ b2.double()
+    want = 0.5 * sums + (before.double() if accumulate else 0)
+    # fp32 sums of T exact products each: T 2^-24 of the magnitudes' sum
+    bound = (a.double().abs().transpose(-1, -2) @ b.double().abs() + a2.double().abs().transpose(-1, -2) @ b2.double().abs()) * (T + T2 + 8) * 2.0 ** -24
+    bound += (want.abs() + before.double().abs()) * 2.0 ** -22
+    forms = [None] if T2 or E else [None, 0, 1, 16 * 3, 16 * 2 + 1]  # 256 x 256, 128 x 256, splits
+    for form in forms:
+        c = before.clone() if accumulate else torch.full_like(before, float("nan"))
+        if T2:
+            torch.ops.sxe.wgrad_gemm2_(a, b, a2, b2, c, 0.5, accumulate)
+        elif form is None:
+            torch.ops.sxe.wgrad_gemm_(a, b, c, 0.5, accumulate)
+        else:
+            torch.ops.sxe.wgrad_gemm_variant_(a, b, c, 0.5, accumulate, form)
+        assert bool(((c.double() - want).abs() <= bound).all()), form
+
+
 def test_captured():
     """Replays with new inputs; the splits' sums are the graph's own memory."""
     x, w, _ = _operands(300, 2048, 8192)
