@@ -487,6 +487,250 @@ __global__ void __launch_bounds__(NWF * 64, (fwd_min_waves<D, NWF>())) fwd_kerne
 }
 
 // =============================================================================================
+// Forward, eight waves: the two waves of a SIMD take turns. A tile is two phases of a wave, the
+// matrix phase (V product of the tile before, scores of this one: 32 MFMAs at D 128, ~1024 clocks)
+// and the softmax phase (~1050 clocks of vector work), and waves 4..7 run one phase behind waves
+// 0..3, so that each SIMD has one wave on its matrix core and the other on its vector units; a
+// barrier ends every phase. With both waves in step, as one barrier per tile leaves them, the phases
+// added up instead: at [1, 32768, 4, 1, 128] causal 47 % of the matrix clocks were busy, and 56 %
+// are now. What bounds it at that size is power (the clock falls as the units fill): 1207 -> 1114
+// us; [1, 8192, 8, 2, 128] 244 -> 208, [4, 2048, 32, 8, 128] 196 -> 178, [1, 16384, 4, 1, 64] 365 ->
+// 300, [2, 1024, 12, 12, 64] 29 -> 25. In the matrix phase the operand reads run twelve ahead of the
+// products (the compiler's own order runs two ahead and waits for each: 7 % slower at S 8192).
+// dQ and dK/dV, whose vector share is smaller and which have no registers left for reads ahead, were
+// slower this way (1515 -> 1690 and 2410 -> 3170 us at S 32768) and keep one barrier per tile.
+// =============================================================================================
+template <int D>
+struct PPState {
+  bf16x8 qf[D / 16];
+  f32x16 oacc[D / 32], s[2];
+  bf16x8 p[4];
+  float m, l;
+};
+// O^T += V^T P^T of a tile of KT keys, or of its first half
+template <int D>
+__device__ __forceinline__ void pp_pv(const LaneOffs<D>& lo, PPState<D>& st, const char* vt, bool half = false) {
+#pragma unroll
+  for (int s2 = 0; s2 < 4; ++s2) {
+    if (s2 == 2 && half) break;
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt)
+      st.oacc[dt] = mfma(lds_tr_at(vt + 16 * s2 * 2 * D, lo.tr[dt]), st.p[s2], st.oacc[dt]);
+  }
+}
+// S^T = K Q^T of a tile, the two 32-key halves in turn (two chains of dependent products)
+template <int D>
+__device__ __forceinline__ void pp_qk(const LaneOffs<D>& lo, PPState<D>& st, const char* kt) {
+  st.s[0] = zero16();
+  st.s[1] = zero16();
+#pragma unroll
+  for (int t2 = 0; t2 < D / 16; ++t2)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) st.s[j] = mfma(lds_row_at(kt + 32 * j * 2 * D, lo.row[t2]), st.qf[t2], st.s[j]);
+}
+// as in fwd_tile; leaves the tile's probabilities as the V product's operand in st.p
+template <int D>
+__device__ __forceinline__ void pp_softmax(PPState<D>& st, float c, int kbase, int qpos, int r, int h, bool diag,
+                                           bool tail, int kvlen, const uint8_t* lrow, int blk) {
+  if (diag || tail || lrow) {
+    // first masked row of this lane (diagonal or end of the keys); opaque, so the compares keep
+    // compile-time row constants
+    int lim = kvlen - kbase - 4 * h;
+    if (diag) lim = min(lim, qpos + r + 1 - kbase - 4 * h);
+    asm volatile("" : "+v"(lim));
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      bool b0 = true, b1 = true;
+      if (lrow) {
+        b0 = lrow[(kbase + 32 * j) / blk] != 0;
+        b1 = lrow[(kbase + 32 * j + 16) / blk] != 0;
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (32 * j + acc_row(i, 0) >= lim || !(i < 8 ? b0 : b1)) st.s[j][i] = -INFINITY;
+    }
+  }
+  float mx = -INFINITY;
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, st.s[j][i]);
+  mx = fmaxf(mx, xor32(mx)) * c;
+  const bool grow = mx > st.m + 8.f;
+  const float mnew = grow ? mx : st.m;
+  const float mref = (mnew == -INFINITY) ? 0.f : mnew;
+  const float alpha = fast_exp2(st.m - mref);
+  float ps = 0.f;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float e = fast_exp2(__builtin_fmaf(st.s[j][i], c, -mref));
+      st.s[j][i] = e;
+      ps += e;
+    }
+    st.p[2 * j] = acc_to_b(st.s[j], 0);
+    st.p[2 * j + 1] = acc_to_b(st.s[j], 1);
+  }
+  st.l = st.l * alpha + ps;
+  st.m = mnew;
+  if (__any(grow)) {
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) st.oacc[dt][i] *= alpha;
+  }
+  // computed in this phase, not sunk to their use in the next one
+#pragma unroll
+  for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(st.p[i]));
+}
+template <bool SPARSE, int D>
+__global__ void __launch_bounds__(512, 1) fwd_pp_kernel(
+    const unsigned short* __restrict__ q, Strides qs, const unsigned short* __restrict__ k, Strides ks,
+    const unsigned short* __restrict__ v, Strides vs, unsigned short* __restrict__ o, Strides os,
+    float* __restrict__ lse, int B, int H, int Hk, int Sq, int Sk, float scale, int causal, Sparse sp, int kvlen,
+    int qoff) {
+  constexpr int ROWB = 2 * D, TILE = KT * ROWB, NWF = 8, QBF = NWF * QW;
+  int* tlist = reinterpret_cast<int*>(smem + 4 * TILE) + 1;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, h = lane >> 5;
+  const int nqb = Sq / QBF;
+  int bh, qb;
+  map_block(nqb, B * H, causal != 0, bh, qb);
+  const int b = bh / H, head = bh - b * H;
+  const int kh = head / (H / Hk);
+  const int q0 = qb * QBF + w * QW;
+  const int qpos = q0 + qoff;
+  const unsigned short* qp = q + b * qs.b + head * qs.h;
+  const unsigned short* kp = k + b * ks.b + kh * ks.h;
+  const unsigned short* vp = v + b * vs.b + kh * vs.h;
+  const float c = scale * LOG2E;
+  PPState<D> st;
+#pragma unroll
+  for (int t = 0; t < D / 16; ++t)
+    st.qf[t] = *reinterpret_cast<const bf16x8*>(qp + (int64_t)(q0 + r) * qs.s + 16 * t + 8 * h);
+#pragma unroll
+  for (int t = 0; t < D / 32; ++t) st.oacc[t] = zero16();
+  st.m = -INFINITY;
+  st.l = 0.f;
+  const int kend = causal ? min(Sk, (qb + 1) * QBF + qoff) : Sk;
+  const int nkt = (max(kend, 0) + KT - 1) / KT;
+  const int ntiles = SPARSE ? build_tile_list(sp, head, 0, nkt, KT, qb * QBF, qb * QBF + QBF, true, tlist) : nkt;
+  auto tile_at = [&](int i) { return SPARSE ? tlist[i] : i; };
+  const uint8_t* lrow = SPARSE ? sp.layout + ((int64_t)head * sp.nb + (q0 + r) / sp.blk) * sp.nb : nullptr;
+  // two slots of K tiles, then two of V tiles
+  if (ntiles > 0) tile_glds<KT, D, NWF>(kp, ks.s, tile_at(0) * KT, smem);
+  vm_wait_all();
+  __syncthreads();
+  LaneOffs<D> lo;
+  lo.init(lane);
+  // At phase 2 t (waves 0..3 in the matrix phase of tile t, waves 4..7 in the softmax of tile t - 1)
+  // K tile t + 1 and V tile t set out, both wanted from phase 2 t + 2 on; the tiles whose slots they
+  // take, K t - 1 and V t - 2, were last read in phase 2 t - 1.
+  auto issue = [&](int t, int slot) {
+    if (t + 1 < ntiles) tile_glds<KT, D, NWF>(kp, ks.s, tile_at(t + 1) * KT, smem + (slot ^ 1) * TILE);
+    if (t < ntiles) tile_glds<KT, D, NWF>(vp, vs.s, tile_at(t) * KT, smem + (2 + slot) * TILE);
+  };
+  // tiles this wave's queries see: the first `nact` (the list ascends)
+  int nact = ntiles;
+  if (causal)
+    while (nact > 0 && tile_at(nact - 1) * KT > qpos + QW - 1) --nact;
+  auto sphase = [&](int t) {
+    if (t >= nact) return;
+    const int kbase = tile_at(t) * KT;
+    pp_softmax<D>(st, c, kbase, qpos, r, h, causal && (kbase + KT - 1 > qpos), kbase + KT > kvlen, kvlen, lrow,
+                  SPARSE ? sp.blk : 1);
+  };
+  // V product of tile t - 1, scores of tile t
+  auto mphase = [&](int slot) {
+    __builtin_amdgcn_s_setprio(1);
+    pp_pv<D>(lo, st, smem + (2 + (slot ^ 1)) * TILE);
+    pp_qk<D>(lo, st, smem + slot * TILE);
+    // operand reads (0x100) ahead of the products (0x008): a V fragment is two reads, a K fragment one
+    __builtin_amdgcn_sched_group_barrier(0x100, 12, 0);
+#pragma unroll
+    for (int i = 0; i < D / 8; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < D / 8; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_s_setprio(0);
+  };
+  // Steps 1 .. ntiles of one side; both sides pass two barriers in each. The steady ones (1 .. nact - 1)
+  // run unrolled by two, so that slots are constants; the rest keep nothing of theirs in registers.
+  auto sweep = [&](auto first) {
+    constexpr bool FIRST = decltype(first)::value;  // waves 0..3
+    auto step = [&](int t, int slot) {
+      issue(t, slot);
+      if (FIRST) mphase(slot);
+      else sphase(t - 1);
+      __syncthreads();
+      if (FIRST) sphase(t);
+      else mphase(slot);
+      vm_wait_all();
+      __syncthreads();
+    };
+    int t = 1;
+    for (; t + 1 < nact; t += 2) {
+      step(t, 1);
+      step(t + 1, 0);
+    }
+    for (; t <= ntiles; ++t) {
+      auto tailm = [&] {
+        if (t < nact) {
+          mphase(t & 1);
+        } else if (t == nact) {
+          // keys 32..63 of the last tile that all follow this wave's last query are left out: their
+          // values are no factor of the result (0 x NaN would be seen)
+          const int kbase = tile_at(t - 1) * KT;
+          pp_pv<D>(lo, st, smem + (2 + ((t - 1) & 1)) * TILE,
+                   !SPARSE && causal && kbase + KT <= kvlen && kbase + 32 > qpos + QW - 1);
+        }
+      };
+      issue(t, t & 1);
+      if (FIRST) tailm();
+      else sphase(t - 1);
+      __syncthreads();
+      if (FIRST) sphase(t);
+      else tailm();
+      vm_wait_all();
+      __syncthreads();
+    }
+  };
+  issue(0, 0);
+  if (w < 4) {
+    if (nact > 0) pp_qk<D>(lo, st, smem);
+    __syncthreads();
+    sphase(0);
+    vm_wait_all();
+    __syncthreads();
+    sweep(std::true_type{});
+  } else {
+    __syncthreads();
+    if (nact > 0) pp_qk<D>(lo, st, smem);
+    vm_wait_all();
+    __syncthreads();
+    sweep(std::false_type{});
+  }
+  const float lt = st.l + __shfl_xor(st.l, 32, 64);
+  const float inv = lt > 0.f ? 1.f / lt : 0.f;  // a fully masked row outputs zeros
+  unsigned short* op = o + b * os.b + head * os.h + (int64_t)(q0 + r) * os.s;
+#pragma unroll
+  for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+    for (int rg = 0; rg < 4; ++rg) {
+      u16x4 pk;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pk[e] = f32_to_bf16(st.oacc[dt][4 * rg + e] * inv);
+      *reinterpret_cast<u16x4*>(op + 32 * dt + 8 * rg + 4 * h) = pk;
+    }
+  if (h == 0) lse[((int64_t)b * H + head) * Sq + q0 + r] = lt > 0.f ? (st.m + log2f(lt)) * LN2 : INFINITY;
+}
+
+// =============================================================================================
 // Backward pre-pass, per (batch, head, query) row: -delta = -sum_d dO * O and lse * log2(e) (fp32),
 // D/8 threads per row. (Computing delta inside the dQ kernel instead -- it holds the dO rows --
 // measured neutral: the dQ prologue's extra O load cost what the launch saved.)
@@ -981,8 +1225,8 @@ static std::vector<at::Tensor> fwd_impl_d(at::Tensor q, at::Tensor k, at::Tensor
       set_lds_limit(&fa::fwd_kernel<true, 8, D>, mx);
       set_lds_limit(&fa::fwd_kernel<false, 4, D, true>, mx);
       set_lds_limit(&fa::fwd_kernel<true, 4, D, true>, mx);
-      set_lds_limit(&fa::fwd_kernel<false, 8, D, true>, mx);
-      set_lds_limit(&fa::fwd_kernel<true, 8, D, true>, mx);
+      set_lds_limit(&fa::fwd_pp_kernel<false, D>, mx);
+      set_lds_limit(&fa::fwd_pp_kernel<true, D>, mx);
     }
     attr = true;
   }
@@ -1000,7 +1244,7 @@ static std::vector<at::Tensor> fwd_impl_d(at::Tensor q, at::Tensor k, at::Tensor
   if constexpr (D < 256) {
     if (fwd_dma()) {
       if (wide)
-        sp.layout ? launch(fa::fwd_kernel<true, 8, D, true>, 8) : launch(fa::fwd_kernel<false, 8, D, true>, 8);
+        sp.layout ? launch(fa::fwd_pp_kernel<true, D>, 8) : launch(fa::fwd_pp_kernel<false, D>, 8);
       else
         sp.layout ? launch(fa::fwd_kernel<true, 4, D, true>, 4) : launch(fa::fwd_kernel<false, 4, D, true>, 4);
       SXE_LAUNCH_CHECK();

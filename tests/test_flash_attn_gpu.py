@@ -297,6 +297,36 @@ def test_flash_fwd_variants(dma, waves, causal, B, Sq, Sk, H, Hk, D, monkeypatch
     assert (lse - lse2).abs().max().item() < 2e-2
 
 
+@pytest.mark.parametrize("Sq,Sk,kv_len,qoff,causal", [(256, 128, 64, 0, False),    # one tile
+                                                       (256, 128, 65, 0, False),    # and one key
+                                                       (256, 256, 200, 0, True),    # rows past the keys
+                                                       (512, 128, 128, -384, True),  # rows that see nothing
+                                                       (256, 640, 640, 384, True),
+                                                       (512, 512, 512, 17, True)])   # diagonal inside tiles
+@pytest.mark.parametrize("D", [64, 128])
+def test_flash_fwd_waves_in_turns(D, Sq, Sk, kv_len, qoff, causal, monkeypatch):
+    """The eight-wave forward, whose waves take turns at the matrix core, does per query what the
+    four-wave one does in the same order: the outputs and LSEs are the same bits."""
+    from shuffle_exchange_amd.ops import native
+    native.require_hip()
+    torch.manual_seed(3)
+    q = torch.randn(2, Sq, 4, D, device="cuda", dtype=torch.bfloat16)
+    k = torch.randn(2, Sk, 2, D, device="cuda", dtype=torch.bfloat16)
+    v = torch.randn(2, Sk, 2, D, device="cuda", dtype=torch.bfloat16)
+    out = []
+    for waves in ("8", "4"):
+        monkeypatch.setenv("SXE_FA_FWD_WAVES", waves)
+        out.append(torch.ops.sxe.flash_attn_fwd(q, k, v, causal, D ** -0.5, kv_len, qoff))
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+    if causal and qoff == 0:  # a value that no query before it sees, at the start of half a tile
+        v[:, 96] = float("nan")
+        k[:, 96] = float("inf")
+        for waves in ("8", "4"):
+            monkeypatch.setenv("SXE_FA_FWD_WAVES", waves)
+            assert torch.ops.sxe.flash_attn_fwd(q, k, v, causal, D ** -0.5, kv_len, qoff)[0][:, :96].isfinite().all()
+
+
 def _chunked_reference(q, k, v, do, causal, chunk=1024):
     """fp32 attention output and gradients for long sequences, one query block at a time (the full
     score matrix of S = 16k would not be materialised at once). q [B, S, H, D], k/v [B, S, Hk, D]."""
