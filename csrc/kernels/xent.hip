@@ -240,6 +240,195 @@ at::Tensor xent_grad_dual(at::Tensor logits, at::Tensor target, at::Tensor lse, 
   return gT;
 }
 
+// ------------------------------------------------------------------------ vocabulary-major logits
+// Logits as [V, ld] bf16 with a token per column: of an odd vocabulary the rows are whole 16-byte
+// vectors only this way round (ld, the tokens rounded up, is a multiple of 64), so the head's three
+// products run on aligned operands. A thread owns 8 columns and every 4th to 32nd row of its block's
+// share, four in flight; both passes stream. 50257 rows, us, loss / gradient, a workgroup a row of
+// token-major logits against this: 2048 tokens 34 / 89 against 47 / 94, 8192 145 / 340 against 165 /
+// 310, 512 16 / 19 against 22 / 26; what the products gain is a multiple of that (see head_cross_entropy).
+template <int LANES>  // of a row
+struct ColBlock {
+  static constexpr int COLS = 8 * LANES, ROWS = 256 / LANES;
+};
+
+template <int LANES>
+__global__ void __launch_bounds__(256) xent_cols_part_kernel(const unsigned short* __restrict__ x, int64_t ld, int V, int rows_per,
+                                                             float2* __restrict__ part) {
+  constexpr int COLS = ColBlock<LANES>::COLS, ROWS = ColBlock<LANES>::ROWS;
+  __shared__ float2 red[ROWS][COLS + 1];
+  const int cx = threadIdx.x % LANES * 8, ry = threadIdx.x / LANES;
+  const int64_t c = (int64_t)blockIdx.x * COLS + cx;
+  const int r0 = blockIdx.y * rows_per, r1 = min(V, r0 + rows_per);
+  float m[8], s[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    m[j] = -INFINITY;
+    s[j] = 0.f;
+  }
+  if (c < ld) {
+    int r = r0 + ry;
+    for (; r + 3 * ROWS < r1; r += 4 * ROWS) {
+      float v[4][8];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) load8<DT::BF16>(x + (r + u * ROWS) * ld + c, v[u]);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float lm = fmaxf(fmaxf(v[0][j], v[1][j]), fmaxf(v[2][j], v[3][j])), ref = fmaxf(lm, -kFltMax);
+        ms_merge<false>(m[j], s[j], lm, (__expf(v[0][j] - ref) + __expf(v[1][j] - ref)) + (__expf(v[2][j] - ref) + __expf(v[3][j] - ref)));
+      }
+    }
+    for (; r < r1; r += ROWS) {
+      float v[8];
+      load8<DT::BF16>(x + r * ld + c, v);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ms_merge<false>(m[j], s[j], v[j], 1.f);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) red[ry][cx + j] = float2{m[j], s[j]};
+  __syncthreads();
+  for (int i = threadIdx.x; i < COLS; i += 256) {
+    const int64_t col = (int64_t)blockIdx.x * COLS + i;
+    if (col >= ld) break;
+    float2 a = red[0][i];
+    for (int g = 1; g < ROWS; ++g) ms_merge<true>(a.x, a.y, red[g][i].x, red[g][i].y);
+    part[blockIdx.y * ld + col] = a;
+  }
+}
+
+// the shares' (max, sum) to loss and LSE: 16 tokens a block, 16 threads a token
+__global__ void __launch_bounds__(256) xent_cols_loss_kernel(const unsigned short* __restrict__ x, int64_t ld, int64_t tokens, int shares,
+                                                             const float2* __restrict__ part, const int64_t* __restrict__ target,
+                                                             int64_t ignore_index, float* __restrict__ loss, float* __restrict__ lse) {
+  __shared__ float2 red[16][17];
+  const int cx = threadIdx.x & 15, ry = threadIdx.x >> 4;
+  const int64_t t = (int64_t)blockIdx.x * 16 + cx;
+  float2 a{-INFINITY, 0.f};
+  if (t < tokens)
+    for (int g = ry; g < shares; g += 16) {
+      const float2 b = part[g * ld + t];
+      ms_merge<true>(a.x, a.y, b.x, b.y);
+    }
+  red[ry][cx] = a;
+  __syncthreads();
+  if (ry != 0 || t >= tokens) return;
+  for (int g = 1; g < 16; ++g) ms_merge<true>(a.x, a.y, red[g][cx].x, red[g][cx].y);
+  const float l = a.x + __logf(a.y);
+  const int64_t tgt = target[t];
+  loss[t] = tgt == ignore_index ? 0.f : l - bf16_to_f32(x[tgt * ld + t]);
+  lse[t] = l;
+}
+
+// dloss[t] * (softmax - onehot); columns behind the last token are zeros
+template <int LANES>
+__global__ void __launch_bounds__(256) xent_cols_bwd_kernel(const unsigned short* __restrict__ x, unsigned short* __restrict__ grad,
+                                                            int64_t ld, int V, int64_t tokens, int rows_per,
+                                                            const int64_t* __restrict__ target, int64_t ignore_index,
+                                                            const float* __restrict__ lse, const float* __restrict__ dloss) {
+  const int64_t c = (int64_t)blockIdx.x * ColBlock<LANES>::COLS + threadIdx.x % LANES * 8;
+  if (c >= ld) return;
+  float l[8], sc[8];
+  int tgt[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const bool in = c + j < tokens;
+    const int64_t t = in ? target[c + j] : ignore_index;
+    tgt[j] = (int)t;
+    sc[j] = t == ignore_index ? 0.f : dloss[c + j];
+    l[j] = in ? lse[c + j] : 0.f;
+  }
+  const int r0 = blockIdx.y * rows_per, r1 = min(V, r0 + rows_per);
+  constexpr int ROWS = ColBlock<LANES>::ROWS;
+  auto put = [&](float (&v)[8], int r) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = c + j < tokens ? sc[j] * (__expf(v[j] - l[j]) - (r == tgt[j] ? 1.f : 0.f)) : 0.f;
+    store8<DT::BF16>(grad + r * ld + c, v);
+  };
+  int r = r0 + threadIdx.x / LANES;
+  for (; r + 3 * ROWS < r1; r += 4 * ROWS) {
+    float v[4][8];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) load8<DT::BF16>(x + (r + u * ROWS) * ld + c, v[u]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) put(v[u], r + u * ROWS);
+  }
+  for (; r < r1; r += ROWS) {
+    float v[8];
+    load8<DT::BF16>(x + r * ld + c, v);
+    put(v, r);
+  }
+}
+
+// f(blocks across, rows of a block, shares of the vocabulary) for blocks of `lanes`: 2048 blocks where there are that many of 64
+// rows or more (the loss reads a (max, sum) of each column of each: 4096 blocks cost it 8 % at 2048 columns)
+template <typename F>
+static void col_blocks(int lanes, int V, int64_t ld, F f) {
+  const int64_t across = (ld + 8 * lanes - 1) / (8 * lanes);
+  const int64_t want = std::min<int64_t>(std::max<int64_t>(1, 2048 / across), (V + 63) / 64);
+  const int per = (int)((V + want - 1) / want);
+  f(dim3(across, (V + per - 1) / per), per);
+}
+
+static void xent_cols_checks(const at::Tensor& x, const at::Tensor& target) {
+  SXE_CHECK(x.dim() == 2 && x.is_contiguous() && x.scalar_type() == at::kBFloat16 && x.size(1) % 8 == 0 && x.size(0) > 0 &&
+                x.size(0) < (1ll << 30) && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0,
+            "xent_cols: bf16 logits [vocab, columns], columns in multiples of 8");
+  SXE_CHECK(target.is_cuda() && target.scalar_type() == at::kLong && target.is_contiguous() && target.numel() > 0 &&
+                target.numel() <= x.size(1), "xent_cols: int64 targets, one for each of the first columns");
+}
+
+std::tuple<at::Tensor, at::Tensor> xent_cols_fwd(at::Tensor logits, at::Tensor target, int64_t ignore_index) {
+  xent_cols_checks(logits, target);
+  c10::DeviceGuard guard(logits.device());
+  const int V = (int)logits.size(0);
+  const int64_t ld = logits.size(1), tokens = target.numel();
+  auto f = logits.options().dtype(at::kFloat);
+  auto loss = at::empty({tokens}, f), lse = at::empty({tokens}, f);
+  auto* x = reinterpret_cast<const unsigned short*>(logits.data_ptr());
+  // pieces of 256 bytes of a row: with whole waves a row 2048 columns take 51 us for 47, 512 columns 35 for 22
+  auto run = [&](auto lanes) {
+    constexpr int LANES = decltype(lanes)::value;
+    col_blocks(LANES, V, ld, [&](dim3 grid, int per) {
+      auto part = at::empty({(int64_t)grid.y, ld, 2}, f);
+      auto* pp = reinterpret_cast<float2*>(part.data_ptr<float>());
+      hipLaunchKernelGGL(xent_cols_part_kernel<LANES>, grid, dim3(256), 0, cur_stream(), x, ld, V, per, pp);
+      SXE_LAUNCH_CHECK();
+      hipLaunchKernelGGL(xent_cols_loss_kernel, dim3((tokens + 15) / 16), dim3(256), 0, cur_stream(), x, ld, tokens, (int)grid.y, pp,
+                         target.data_ptr<int64_t>(), ignore_index, loss.data_ptr<float>(), lse.data_ptr<float>());
+    });
+  };
+  if (ld > 64) run(std::integral_constant<int, 16>{});
+  else run(std::integral_constant<int, 8>{});
+  SXE_LAUNCH_CHECK();
+  return {loss, lse};
+}
+
+at::Tensor xent_cols_bwd(at::Tensor logits, at::Tensor target, at::Tensor lse, at::Tensor dloss, int64_t ignore_index) {
+  xent_cols_checks(logits, target);
+  for (const at::Tensor* t : {&lse, &dloss})
+    SXE_CHECK(t->is_cuda() && t->scalar_type() == at::kFloat && t->is_contiguous() && t->numel() == target.numel(),
+              "xent_cols: fp32 lse and dloss [tokens]");
+  c10::DeviceGuard guard(logits.device());
+  const int V = (int)logits.size(0);
+  const int64_t ld = logits.size(1);
+  auto grad = at::empty_like(logits);
+  // whole waves a row where that leaves few of them idle: 8192 columns 309 us, 361 in pieces of 256 bytes
+  auto run = [&](auto lanes) {
+    constexpr int LANES = decltype(lanes)::value;
+    col_blocks(LANES, V, ld, [&](dim3 grid, int per) {
+      hipLaunchKernelGGL(xent_cols_bwd_kernel<LANES>, grid, dim3(256), 0, cur_stream(),
+                         reinterpret_cast<const unsigned short*>(logits.data_ptr()), reinterpret_cast<unsigned short*>(grad.data_ptr()), ld,
+                         V, target.numel(), per, target.data_ptr<int64_t>(), ignore_index, lse.data_ptr<float>(), dloss.data_ptr<float>());
+    });
+  };
+  if (ld >= 2048 || ld % 512 == 0) run(std::integral_constant<int, 64>{});
+  else if (ld > 64) run(std::integral_constant<int, 16>{});
+  else run(std::integral_constant<int, 8>{});
+  SXE_LAUNCH_CHECK();
+  return grad;
+}
+
 static void xent_checks(const at::Tensor& logits, const at::Tensor& target) {
   SXE_CHECK(logits.dim() == 2 && logits.is_contiguous(), "xent: logits must be contiguous [rows, vocab]");
   SXE_CHECK(target.scalar_type() == at::kLong && target.numel() == logits.size(0) && target.is_contiguous(),
@@ -301,9 +490,13 @@ at::Tensor xent_bwd(at::Tensor logits, at::Tensor target, at::Tensor lse, at::Te
 TORCH_LIBRARY_FRAGMENT(sxe, m) {
   m.def("xent_fwd(Tensor(a!) logits, Tensor target, int ignore_index, bool inplace_grad, Tensor? scale, float grad_scale) -> (Tensor, Tensor)");
   m.def("xent_bwd(Tensor(a!) logits, Tensor target, Tensor lse, Tensor dloss, int ignore_index, bool inplace) -> Tensor");
+  m.def("xent_cols_fwd(Tensor logits, Tensor target, int ignore_index) -> (Tensor, Tensor)");
+  m.def("xent_cols_bwd(Tensor logits, Tensor target, Tensor lse, Tensor dloss, int ignore_index) -> Tensor");
   m.def("xent_grad_dual(Tensor(a!) logits, Tensor target, Tensor lse, int ignore_index, Tensor scale_a, Tensor? scale_b) -> Tensor");
 }
 TORCH_LIBRARY_IMPL(sxe, CUDA, m) {
+  m.impl("xent_cols_fwd", &sxe::xent_cols_fwd);
+  m.impl("xent_cols_bwd", &sxe::xent_cols_bwd);
   m.impl("xent_grad_dual", &sxe::xent_grad_dual);
   m.impl("xent_fwd", &sxe::xent_fwd);
   m.impl("xent_bwd", &sxe::xent_bwd);

@@ -12,7 +12,7 @@ import torch.nn.functional as F
 
 from ..ops.activation import bias_gelu
 from ..ops.attention import attention
-from ..ops.cross_entropy import cross_entropy
+from ..ops.cross_entropy import head_cross_entropy
 from ..ops.linear import Embedding, Linear
 from ..ops.norm import LayerNorm
 from ..runtime.zero.partition_parameters import local_shard
@@ -103,8 +103,8 @@ class GPT2LMHeadModel(nn.Module):
         x = self.wte(input_ids) + self.wpe(pos)[None]
         for blk in self.h:
             x = blk(x)
-        logits = F.linear(self.ln_f(x), self.wte.weight)
+        x = self.ln_f(x)
         if labels is None:
-            return logits
+            return F.linear(x, self.wte.weight)
         tgt = torch.cat([labels[:, 1:], torch.full_like(labels[:, :1], -100)], dim=1)
-        return cross_entropy(logits, tgt)
+        return head_cross_entropy(x, self.wte.weight, tgt)

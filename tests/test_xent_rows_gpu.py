@@ -47,3 +47,41 @@ def test_rows(V, offset, dtype):
     torch.ops.sxe.xent_fwd(keep, tgt, -100, True, None, 0.25)
     full = torch.where((tgt == -100)[:, None], 0., 0.25 * ((ref - lse[:, None]).exp() - one))
     torch.testing.assert_close(keep.double(), full, **tol)
+
+
+@pytest.mark.parametrize("tokens", [1, 63, 64, 130, 500, 2100])  # columns behind the last token, of a block, blocks of each width
+@pytest.mark.parametrize("V", [65, 129, 1001, 9999])        # one share and several, rounds of 64 rows and their rest
+def test_column_head_matches_fp64(V, tokens):
+    """The head with a token per column. The logits are sums of 64 products rounded once to bf16 (|x| < 6: a probability moves by
+    2^-9 of |x| at most), a gradient is rounded once, a product of them once more: 2^-9 (6 + 2) of a norm."""
+    from shuffle_exchange_amd.ops.cross_entropy import head_cross_entropy, _columns_ok
+    g = torch.Generator("cuda").manual_seed(V + tokens)
+    h = torch.randn(1, tokens, 64, generator=g, device="cuda").bfloat16().requires_grad_()
+    w = torch.randn(V, 64, generator=g, device="cuda").mul_(0.125).bfloat16().requires_grad_()
+    tgt = torch.randint(0, V, (1, tokens), generator=g, device="cuda")
+    tgt[0, tokens // 2 + 1:tokens // 2 + 3] = -100
+    assert _columns_ok(h, w, tgt)
+    loss = head_cross_entropy(h, w, tgt)
+    h2, w2 = h.detach().double().requires_grad_(), w.detach().double().requires_grad_()
+    want = torch.nn.functional.cross_entropy((h2 @ w2.t())[0], tgt[0])
+    (0.5 * loss).backward()
+    (0.5 * want).backward()
+    assert abs(loss.item() - want.item()) < 6 * 2 ** -9
+    for a, b in ((h.grad, h2.grad), (w.grad, w2.grad)):
+        assert (a.double() - b).norm() <= 2 ** -6 * b.norm()
+
+
+def test_column_head_masked_vocabulary():
+    """Rows of -inf logits (a hidden state of infinities) and a share with nothing else: NaN and zeros where the row form has them."""
+    x = torch.randn(200, 64, device="cuda").bfloat16()
+    x[:120] = float("-inf")
+    x[:, 3] = float("nan")
+    tgt = torch.full((64,), 150, device="cuda")
+    loss, lse = torch.ops.sxe.xent_cols_fwd(x, tgt, -100)
+    rows, rlse = torch.ops.sxe.xent_fwd(x.t().contiguous(), tgt, -100, False, None, 1.0)
+    torch.testing.assert_close(loss, rows, equal_nan=True, rtol=1e-5, atol=1e-5)  # sums of 200 terms in another order: 200 * 2^-24
+    torch.testing.assert_close(lse, rlse, equal_nan=True, rtol=1e-5, atol=1e-5)
+    dl = torch.ones(64, device="cuda")
+    got = torch.ops.sxe.xent_cols_bwd(x, tgt, rlse, dl, -100)
+    want = torch.ops.sxe.xent_bwd(x.t().contiguous(), tgt, rlse, dl, -100, False).t()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
