@@ -8,6 +8,8 @@
 //      a vocab-parallel embedding), last-token logits gather (ragged_ops/logits_gather/
 //      logits_gather.cu:20; ``add`` folds the fused-residual sum x + res into the gather), and the
 //      random-LTD token gather (ops/random_ltd/gather_scatter.cu:22).
+//  * embedding_grad(gy [N, W], idx [N], rows) -> [rows, W]: the sum of the rows of gy that share an
+//      index, in their order and in fp32; rows that no index names are zeros.
 //  * scatter_rows_(dst [R, W], idx [N], src [N, W]): dst[idx[i]] = src[i] (indices unique):
 //      the random-LTD scatter back into the full sequence (gather_scatter.cu:72) and the backward of
 //      a unique-index gather.
@@ -70,6 +72,100 @@ __global__ void __launch_bounds__(256) scatter_kernel(u32x4* __restrict__ dst, c
     const u32x4* a = src + row * chunks;
     for (int c = lane; c < chunks; c += 64) o[c] = a[c];
   }
+}
+
+// -------------------------------------------------------------------------------- embedding gradient
+// The library's kernel for up to 3072 tokens walks them one after another (2048 tokens of 768: 97 us), its
+// other one is a radix sort of some ten launches. Here the tokens are ranked by (index, position) by
+// counting -- every wave of a block compares 64 tokens with a part of the others, N^2 compares in all,
+// which is why the caller stops at 16384 of them -- and a block then sums 64 columns of 32 ranks:
+// 2048 tokens of 768 into 50257 rows 24 us, of which the zeros of the result are 12; 4096 wide into
+// 32000 rows, us, the library / this: 512 tokens 75 / 42, 2048 182 / 59, 8192 328 / 121, 16384 598 / 212
+// (zeros 33); half of the tokens the same: 2048 211 / 102, 16384 605 / 566.
+constexpr int RANK_TILE = 8192;
+template <typename I>
+__global__ void __launch_bounds__(1024) rank_kernel(const I* __restrict__ idx, int n, int rows, int* __restrict__ order,
+                                                    int* __restrict__ sorted) {
+  __shared__ __attribute__((aligned(16))) int ids[RANK_TILE];
+  __shared__ int count[16][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, t = blockIdx.x * 64 + lane;
+  // an index out of range counts as row `rows`, which is not written
+  auto id_of = [&](int j) {
+    const I x = idx[j];
+    return x >= 0 && x < rows ? (int)x : rows;
+  };
+  const int mine = t < n ? id_of(t) : 0;
+  int below = 0;
+  for (int j0 = 0; j0 < n; j0 += RANK_TILE) {
+    const int m = min(RANK_TILE, (n - j0 + 63) / 64 * 64), part = m / 16;
+    __syncthreads();
+    for (int j = threadIdx.x; j < m; j += 1024) ids[j] = j0 + j < n ? id_of(j0 + j) : 0x7fffffff;
+    __syncthreads();
+    for (int j = w * part; j < (w + 1) * part; j += 4) {
+      const int4 x = *reinterpret_cast<const int4*>(ids + j);
+      const int at = j0 + j;
+      below += (x.x < mine || (x.x == mine && at < t)) + (x.y < mine || (x.y == mine && at + 1 < t)) +
+               (x.z < mine || (x.z == mine && at + 2 < t)) + (x.w < mine || (x.w == mine && at + 3 < t));
+    }
+  }
+  count[w][lane] = below;
+  __syncthreads();
+  if (w != 0 || t >= n) return;
+  for (int i = 1; i < 16; ++i) below += count[i][lane];
+  order[below] = t;
+  sorted[below] = mine;
+}
+
+// Eight lanes a rank, eight columns a lane. A run of one index is summed by the block it starts in, which
+// follows it over the blocks behind.
+template <DT T>
+__global__ void __launch_bounds__(256) run_sum_kernel(const typename dt_traits<T>::storage* __restrict__ gy, int64_t W, int n, int rows,
+                                                      const int* __restrict__ order, const int* __restrict__ sorted,
+                                                      typename dt_traits<T>::storage* __restrict__ out) {
+  __shared__ float sum[32][65];
+  const int g = threadIdx.x >> 3, cl = (threadIdx.x & 7) * 8, p0 = blockIdx.x * 32, p = p0 + g;
+  const int64_t c = (int64_t)blockIdx.y * 64 + cl;
+  const bool in = c < W;
+  auto add_row = [&](int at, float (&v)[8]) {
+    float x[8];
+    load8<T>(gy + (int64_t)order[at] * W + c, x);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] += x[j];
+  };
+  const int id = p < n ? sorted[p] : rows;
+  const bool start = id < rows && (p == 0 || sorted[p - 1] != id);
+  float v[8] = {};
+  if (in && id < rows) add_row(p, v);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) sum[g][cl + j] = v[j];
+  __syncthreads();
+  const int end = min(n, p0 + 32);
+  int q = p + 1;
+  if (start)
+    for (; q < end && sorted[q] == id; ++q)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] += sum[q - p0][cl + j];
+  // the run over the block's end, if it starts here: each group adds up its share of it, then the groups'
+  const int last = sorted[end - 1];
+  if (end < n && last < rows && sorted[end] == last && (p0 == 0 || sorted[p0 - 1] != last)) {
+    float x[8] = {};
+    for (int q0 = end; q0 < n && sorted[q0] == last; q0 += 256) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int at = q0 + 32 * u + g;
+        if (in && at < n && sorted[at] == last) add_row(at, x);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sum[g][cl + j] = x[j];
+    __syncthreads();
+    if (start && id == last)
+      for (int i = 0; i < 32; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] += sum[i][cl + j];
+  }
+  if (start && in) store8<T>(out + (int64_t)id * W + c, v);
 }
 
 }  // namespace rows
@@ -147,13 +243,44 @@ void scatter_rows_(at::Tensor dst, const at::Tensor& idx, const at::Tensor& src)
   SXE_LAUNCH_CHECK();
 }
 
+at::Tensor embedding_grad(const at::Tensor& gy, const at::Tensor& idx, int64_t rows) {
+  SXE_CHECK_CUDA(gy);
+  const int64_t n = idx.numel();
+  SXE_CHECK(gy.dim() == 2 && gy.is_contiguous() && gy.size(1) % 8 == 0 && reinterpret_cast<uintptr_t>(gy.data_ptr()) % 16 == 0,
+            "embedding_grad: gy [N, W], W a multiple of 8");
+  SXE_CHECK(idx.is_cuda() && idx.is_contiguous() && n == gy.size(0) && (idx.scalar_type() == at::kLong || idx.scalar_type() == at::kInt),
+            "embedding_grad: idx int32/int64 [N]");
+  SXE_CHECK(rows >= 0 && rows < 0x7fffffff && n < (1 << 24) && gy.size(1) < (1 << 20), "embedding_grad: sizes");
+  c10::DeviceGuard g(gy.device());
+  auto out = at::zeros({rows, gy.size(1)}, gy.options());
+  if (n == 0 || out.numel() == 0) return out;
+  auto scratch = at::empty({2, n}, idx.options().dtype(at::kInt));
+  int *order = scratch.data_ptr<int>(), *sorted = order + n;
+  const dim3 grid((n + 63) / 64);
+  if (idx.scalar_type() == at::kLong)
+    hipLaunchKernelGGL(rows::rank_kernel<int64_t>, grid, dim3(1024), 0, cur_stream(), idx.data_ptr<int64_t>(), (int)n, (int)rows, order, sorted);
+  else
+    hipLaunchKernelGGL(rows::rank_kernel<int32_t>, grid, dim3(1024), 0, cur_stream(), idx.data_ptr<int32_t>(), (int)n, (int)rows, order, sorted);
+  SXE_LAUNCH_CHECK();
+  SXE_DISPATCH_DT(dtype_of(gy), TT, {
+    using S = typename dt_traits<TT>::storage;
+    hipLaunchKernelGGL(rows::run_sum_kernel<TT>, dim3((n + 31) / 32, (gy.size(1) + 63) / 64), dim3(256), 0, cur_stream(),
+                       reinterpret_cast<const S*>(gy.data_ptr()), gy.size(1), (int)n, (int)rows, order, sorted,
+                       reinterpret_cast<S*>(out.data_ptr()));
+  });
+  SXE_LAUNCH_CHECK();
+  return out;
+}
+
 }  // namespace sxe
 
 TORCH_LIBRARY_FRAGMENT(sxe, m) {
   m.def("gather_rows(Tensor src, Tensor idx, int offset=0, Tensor? add=None) -> Tensor");
+  m.def("embedding_grad(Tensor gy, Tensor idx, int rows) -> Tensor");
   m.def("scatter_rows_(Tensor(a!) dst, Tensor idx, Tensor src) -> ()");
 }
 TORCH_LIBRARY_IMPL(sxe, CUDA, m) {
   m.impl("gather_rows", &sxe::gather_rows);
+  m.impl("embedding_grad", &sxe::embedding_grad);
   m.impl("scatter_rows_", &sxe::scatter_rows_);
 }

@@ -627,8 +627,38 @@ class Linear(torch.nn.Linear):
         return linear(x, self.weight, None if skip_bias else self.bias)
 
 
+class _Embed(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, ids, weight):
+        ctx.save_for_backward(ids)
+        ctx.rows = weight.shape[0]
+        return F.embedding(ids, weight)
+
+    @staticmethod
+    def backward(ctx, gy):
+        ids, = ctx.saved_tensors
+        if (torch.is_grad_enabled() and gy.requires_grad) or not native.plain(gy, ids):  # a derivative of the gradient is asked for
+            return None, torch.ops.aten.embedding_dense_backward(gy, ids, ctx.rows, -1, False)
+        g2 = gy.reshape(-1, gy.shape[-1])
+        if not g2.is_contiguous() or g2.data_ptr() % 16:
+            g2 = g2.clone(memory_format=torch.contiguous_format)
+        return None, torch.ops.sxe.embedding_grad(g2, ids.reshape(-1).contiguous(), ctx.rows)
+
+
+EMBED_GRAD_IDS = 16384  # indices up to which ranking them by comparison is the faster way to their gradient (rows.hip)
+
+
 class Embedding(torch.nn.Embedding):
-    """``nn.Embedding`` with the constructor-time N(0, init_std) init of ``Linear``."""
+    """``nn.Embedding`` with the constructor-time N(0, init_std) init of ``Linear`` and, on the GPU, a gradient of its own."""
+
+    def forward(self, input):
+        w = self.weight
+        if (w.is_cuda and torch.is_grad_enabled() and w.requires_grad and self.padding_idx is None and self.max_norm is None
+                and not self.scale_grad_by_freq and not self.sparse and isinstance(input, torch.Tensor) and 0 < input.numel() <= EMBED_GRAD_IDS
+                and w.dim() == 2 and w.shape[1] % 8 == 0 and w.dtype in (torch.bfloat16, torch.float16, torch.float32)
+                and input.device == w.device and input.dtype in (torch.int64, torch.int32) and native.use_hip(w) and native.plain(w, input)):
+            return _Embed.apply(input, w)
+        return super().forward(input)
 
     def __init__(self, num_embeddings, embedding_dim, init_std=None, **kw):
         super().__init__(num_embeddings, embedding_dim, **kw)

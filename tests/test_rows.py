@@ -68,3 +68,29 @@ def test_rows_gpu(dtype):
     native.require_hip()
     _check("cuda", dtype)
     _check_tokens("cuda", dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens", [1, 31, 64, 65, 333, 8200])  # blocks of 32 ranks, 64 tokens, stages of 8192
+@pytest.mark.parametrize("kind", ["random", "few", "one"])       # runs within a block, over several, over all of them
+@pytest.mark.parametrize("dtype,W", [(torch.bfloat16, 72), (torch.float32, 64), (torch.float16, 128)])
+def test_embedding_gradient(tokens, kind, dtype, W):
+    """Against sums in fp64: fp32 sums of n terms (2^-24 n of their magnitudes at the most), rounded once. Twice the same bits."""
+    from shuffle_exchange_amd.ops import native
+    from shuffle_exchange_amd.ops.linear import Embedding
+    native.require_hip()
+    g = torch.Generator("cuda").manual_seed(tokens)
+    V = 1000
+    ids = torch.randint(0, {"random": V, "few": 3, "one": 1}[kind], (tokens,), generator=g, device="cuda") + (5 if kind != "random" else 0)
+    emb = Embedding(V, W, device="cuda", dtype=dtype)
+    gy = torch.randn(tokens, W, generator=g, device="cuda").to(dtype)
+    y = emb(ids)
+    assert type(y.grad_fn).__name__ == "_EmbedBackward" and torch.equal(y, emb.weight[ids])
+    got = torch.autograd.grad(y, emb.weight, gy, retain_graph=True)[0]
+    want = torch.zeros(V, W, device="cuda", dtype=torch.float64).index_add_(0, ids, gy.double())
+    size = torch.zeros(V, W, device="cuda", dtype=torch.float64).index_add_(0, ids, gy.double().abs())
+    n = torch.bincount(ids, minlength=V)[:, None]
+    eps = {torch.bfloat16: 2 ** -8, torch.float16: 2 ** -11, torch.float32: 2 ** -24}[dtype]
+    assert bool(((got.double() - want).abs() <= eps * want.abs() + 2 ** -24 * n * size + 2 ** -25).all())
+    assert torch.equal(got, torch.autograd.grad(y, emb.weight, gy)[0])
+    assert torch.equal(got, torch.ops.sxe.embedding_grad(gy, ids.int(), V))

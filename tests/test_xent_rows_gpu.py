@@ -52,8 +52,8 @@ def test_rows(V, offset, dtype):
 @pytest.mark.parametrize("tokens", [1, 63, 64, 130, 500, 2100])  # columns behind the last token, of a block, blocks of each width
 @pytest.mark.parametrize("V", [65, 129, 1001, 9999])        # one share and several, rounds of 64 rows and their rest
 def test_column_head_matches_fp64(V, tokens):
-    """The head with a token per column. The logits are sums of 64 products rounded once to bf16 (|x| < 6: a probability moves by
-    2^-9 of |x| at most), a gradient is rounded once, a product of them once more: 2^-9 (6 + 2) of a norm."""
+    """The head with a token per column. A logit (|x| < 6) is rounded to bf16, and with it the loss moves by 2 * 6 * 2^-8 at most. A
+    probability moves by 2^-8 |x|, in a norm by less than 2 * 2^-8; the gradient is rounded and so is the product of it: 2^-8 (2 + 2)."""
     from shuffle_exchange_amd.ops.cross_entropy import head_cross_entropy, _columns_ok
     g = torch.Generator("cuda").manual_seed(V + tokens)
     h = torch.randn(1, tokens, 64, generator=g, device="cuda").bfloat16().requires_grad_()
@@ -66,7 +66,7 @@ def test_column_head_matches_fp64(V, tokens):
     want = torch.nn.functional.cross_entropy((h2 @ w2.t())[0], tgt[0])
     (0.5 * loss).backward()
     (0.5 * want).backward()
-    assert abs(loss.item() - want.item()) < 6 * 2 ** -9
+    assert abs(loss.item() - want.item()) < 12 * 2 ** -8
     for a, b in ((h.grad, h2.grad), (w.grad, w2.grad)):
         assert (a.double() - b).norm() <= 2 ** -6 * b.norm()
 
