@@ -218,9 +218,15 @@ __device__ __forceinline__ int build_tile_list(const Sparse sp, int head, int t_
   return list[-1];
 }
 
-// Heavy-first mapping of the flat block index onto (b, head, row-block) for the causal triangle.
+// Heavy-first mapping of the flat block index onto (b, head, row-block) for the causal triangle. A grid
+// of four-wave workgroups that is resident at once, two on a CU, is not evened out by the order in which
+// they finish: its second half runs backwards, so that the CU with the heaviest first workgroup has the
+// lightest second one (causal, forward [1, 8192, 8, 2, 128] 204 -> 191 us, backward 700 -> 671;
+// [1, 16384, 4, 1, 128] 393 -> 360 and 1352 -> 1268).
 __device__ __forceinline__ void map_block(int nblk, int BH, bool heavy_last_index, int& bh, int& blk) {
-  const int idx = blockIdx.x;
+  int idx = blockIdx.x;
+  const int grid = nblk * BH;
+  if (blockDim.x == 256 && grid > kNumCUs && grid <= 2 * kNumCUs && idx >= kNumCUs) idx = grid - 1 - (idx - kNumCUs);
   const int rank = idx / BH;
   bh = idx - rank * BH;
   blk = heavy_last_index ? (nblk - 1 - rank) : rank;
@@ -1189,14 +1195,24 @@ static int env_int(const char* name, int dflt) {
   const char* e = std::getenv(name);
   return (e != nullptr && *e != 0) ? std::atoi(e) : dflt;
 }
-// 4-wave forward workgroups only when forced (SXE_FA_FWD_WAVES=4): 8 waves are equal or faster on
-// every measured shape -- causal equal at head dims 64 / 128, non-causal 3-7 % faster
-// (profiles/r05/attn_fwd_waves_ab.log, attn_fwd_waves_d64_ab.log; one earlier box showed 4 waves
-// 6 % ahead at D64 causal, which a second box did not reproduce)
-static bool fwd_narrow(int D) {
-  (void)D;
-  return env_int("SXE_FA_FWD_WAVES", 8) == 4;
+// Rows of 256 or 128 queries a workgroup, by how many of 256 there are (`blocks`), us, eight waves / four.
+// Forward, causal: up to one workgroup of 256 a CU the heaviest of them sets the time, and four waves
+// alone on a CU are the faster half of it: 64 blocks, D 128, S 4096 94 / 88, 128 blocks, S 8192 187 / 178,
+// 256 blocks, S 16384 374 / 360; beyond, eight waves are: 512 blocks, S 2048 84 / 95, S 8192 258 / 318, 1024
+// blocks, S 2048 169 / 175. D 64: 256 blocks, S 8192 153 / 147, 512 blocks, S 2048 58 / 54, S 4096 99 / 98,
+// S 8192 173 / 188, 1024 blocks, S 2048 115 / 93. Not causal: 128 blocks, D 128, S 8192 194 / 184, 256 blocks
+// 252 / 350, 512 blocks 513 / 607; D 64 154 / 138, 173 / 226, 337 / 359.
+// dQ (with dK / dV), causal: D 128, 128 blocks, S 8192 655 / 624, 256 blocks 699 / 691, 512 blocks, S 2048
+// 321 / 330, S 4096 536 / 586, S 8192 935 / 1009; D 64, 512 blocks, S 2048 189 / 176, S 4096 339 / 332, S 8192
+// 574 / 580. Not causal: D 128, 128 blocks, S 8192 1790 / 1738, 256 blocks 1863 / 1935, 512 blocks 2226 /
+// 2394; D 64 1220 / 1194, 1229 / 1297, 1440 / 1470.
+static bool fwd_wide(int D, int64_t blocks, int Sq, bool causal) {
+  return causal ? blocks > kNumCUs && (D == 128 || Sq >= 8192) : blocks > kNumCUs / 2;
 }
+static bool dq_wide(int D, int64_t blocks, int Sq, bool causal) {
+  return causal ? blocks > kNumCUs && (D == 128 || Sq >= 8192) : blocks >= kNumCUs;
+}
+// SXE_FA_FWD_WAVES = 4 / 8 forces the forward's
 static bool fwd_dma() { return env_int("SXE_FA_FWD_DMA", 1) != 0; }
 
 template <typename F>
@@ -1226,12 +1242,17 @@ static std::vector<at::Tensor> fwd_impl_d(at::Tensor q, at::Tensor k, at::Tensor
       set_lds_limit(&fa::fwd_kernel<false, 4, D, true>, mx);
       set_lds_limit(&fa::fwd_kernel<true, 4, D, true>, mx);
       set_lds_limit(&fa::fwd_pp_kernel<false, D>, mx);
+      if constexpr (D == 64) {
+        set_lds_limit(&fa::fwd_kernel<false, 8, D, true>, mx);
+        set_lds_limit(&fa::fwd_kernel<true, 8, D, true>, mx);
+      }
       set_lds_limit(&fa::fwd_pp_kernel<true, D>, mx);
     }
     attr = true;
   }
-  // 8 waves share each staged K/V tile when the query axis allows; head dim 256 runs 4 (register budget)
-  const bool wide = D < 256 && Sq % 256 == 0 && !fwd_narrow(D);
+  // 8 waves share each staged K/V tile where that pays and the query axis allows; head dim 256 runs 4 (register budget)
+  const int fww = env_int("SXE_FA_FWD_WAVES", 0);
+  const bool wide = D < 256 && Sq % 256 == 0 && (fww == 8 || (fww != 4 && (sp.layout || fwd_wide(D, (int64_t)B * H * Sq / 256, Sq, causal))));
   const int grid = (Sq / fa::QB) * B * H;
   auto launch = [&](auto kern, int nwf) {
     hipLaunchKernelGGL(kern, dim3(nwf == 8 ? grid / 2 : grid), dim3(nwf * 64), lds, cur_stream(),
@@ -1243,7 +1264,17 @@ static std::vector<at::Tensor> fwd_impl_d(at::Tensor q, at::Tensor k, at::Tensor
   };
   if constexpr (D < 256) {
     if (fwd_dma()) {
-      if (wide)
+      // Head dim 64 fits two eight-wave workgroups on a CU if their waves keep in step, and without a diagonal, or with a layout, that
+      // is the faster form (us, in step / in turns: [4, 2048, 32, 8, 64] 166 / 185, [4, 2048, 16, 4, 64] 88 / 96, [1, 8192, 16, 4, 64]
+      // 332 / 335; block-sparse, 9 of 64 blocks of 64 a row, 16 heads, 4 x 2048 49 / 63, 2 x 8192 95 / 134, head dim 128 172 / 166)
+      bool in_step = false;
+      if constexpr (D == 64) {
+        in_step = wide && (sp.layout || (!causal && (int64_t)B * H * Sq / 256 >= 2 * kNumCUs && fww == 0));
+        if (in_step) sp.layout ? launch(fa::fwd_kernel<true, 8, D, true>, 8) : launch(fa::fwd_kernel<false, 8, D, true>, 8);
+      }
+      if (in_step)
+        ;
+      else if (wide)
         sp.layout ? launch(fa::fwd_pp_kernel<true, D>, 8) : launch(fa::fwd_pp_kernel<false, D>, 8);
       else
         sp.layout ? launch(fa::fwd_kernel<true, 4, D, true>, 4) : launch(fa::fwd_kernel<false, 4, D, true>, 4);
@@ -1318,10 +1349,9 @@ static void bwd_impl_d(at::Tensor dout, at::Tensor q, at::Tensor k, at::Tensor v
     }
     attr_set = true;
   }
-  // 8-wave dQ workgroups from 8k queries on (auto; SXE_FA_DQ_WAVES=4 / 8 forces): 1.5-2 % faster
-  // fwd+bwd at S8k / S32k, neutral at 2k (profiles/r05/attn_bwd_waves_ab.log)
+  // 8-wave dQ workgroups (SXE_FA_DQ_WAVES=4 / 8 forces)
   const int dqw = env_int("SXE_FA_DQ_WAVES", 0);
-  const bool dq8 = D < 256 && Sq % 256 == 0 && (dqw == 8 || (dqw == 0 && Sq >= 8192));
+  const bool dq8 = D < 256 && Sq % 256 == 0 && (dqw == 8 || (dqw == 0 && (sp.layout ? Sq >= 8192 : dq_wide(D, (int64_t)B * H * Sq / 256, Sq, causal))));
   auto* dqk = sp.layout ? fa::dq_kernel<true, D> : fa::dq_kernel<false, D>;
   if constexpr (D < 256) {
     if (dq8) dqk = sp.layout ? fa::dq_kernel<true, D, 8> : fa::dq_kernel<false, D, 8>;
@@ -1347,8 +1377,10 @@ static void bwd_impl_d(at::Tensor dout, at::Tensor q, at::Tensor k, at::Tensor v
   // 36.4 / 36.2 / 37.3; B1 S32k H4/1 4.75 / 6.14 / 9.15 (profiles/r05/attn_dkdv_hpw_sweep.log)
   int hpw = sp.layout != nullptr ? 1 : env_int("SXE_FA_DKDV_HPW", 0);
   if (hpw == 0) {
-    int64_t cap = (int64_t)B * H * (Sk / fa::QB) / (4 * kNumCUs);
-    if (Sk >= 8192 && cap > 2) cap = 2;
+    // not causal: every workgroup's load is the same, two of them a CU are enough (one KV head a workgroup / this, us, fwd+bwd's
+    // backward: [1, 4096, 4, 1, 128] 879 / 333, [1, 8192, 8, 2, 128] 2194 / 921, [4, 2048, 16, 4, 128] 684 / 571)
+    int64_t cap = (int64_t)B * H * (Sk / fa::QB) / ((causal ? 4 : 2) * kNumCUs);
+    if (causal && Sk >= 8192 && cap > 2) cap = 2;
     for (int d = H / Hk; d >= 1; --d)
       if ((H / Hk) % d == 0 && d <= cap) {
         hpw = d;
@@ -1356,7 +1388,7 @@ static void bwd_impl_d(at::Tensor dout, at::Tensor q, at::Tensor k, at::Tensor v
       }
   }
   if (hpw < 1 || (H / Hk) % hpw != 0) hpw = 1;
-  const bool split = sp.layout != nullptr || (causal && H / Hk > hpw);
+  const bool split = sp.layout != nullptr || H / Hk > hpw;
   const bool partials = split && H / hpw > Hk;
   const int np = H / hpw;  // partial head groups
   // head dim 256: dV and dK in one sweep (S once, 256 accumulators, a few spilled registers; default)
@@ -1364,9 +1396,10 @@ static void bwd_impl_d(at::Tensor dout, at::Tensor q, at::Tensor k, at::Tensor v
   // fwd+bwd (profiles/r05/attn_d256_one_sweep_ab.log)
   const bool one_sweep = D >= 256 && env_int("SXE_FA_DKDV_ONE_SWEEP", 1) != 0;
   // head dim 128: 8-wave dK/dV workgroups of 256 keys (SXE_FA_DKDV_WAVES=8, read per call)
-  // (auto from 8k keys on, as the dQ kernel; SXE_FA_DKDV_WAVES=4 / 8 forces)
+  // (auto: block-sparse from 8k keys on; dense, us, 8 / 4 waves: [1, 8192, 4, 1, 128] 699 / 628, [1, 32768, 4, 1, 128] 3762 / 3692,
+  // [2, 4096, 16, 4, 128] 544 / 536, not causal [1, 8192, 16, 4, 128] 2530 / 2226; SXE_FA_DKDV_WAVES=4 / 8 forces)
   const int kvw = env_int("SXE_FA_DKDV_WAVES", 0);
-  const bool kv8 = D == 128 && Sk % 256 == 0 && (kvw == 8 || (kvw == 0 && Sk >= 8192));
+  const bool kv8 = D == 128 && Sk % 256 == 0 && (kvw == 8 || (kvw == 0 && sp.layout && Sk >= 8192));
   const size_t lds_kv = (kv8 ? fa::KVL<D, 256>::VBLK : G_::VBLK) + 2 * G_::SLOT + (sp.layout ? kListBytes : 0);
   at::Tensor pk, pv;
   if (partials) {

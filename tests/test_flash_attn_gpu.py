@@ -327,6 +327,34 @@ def test_flash_fwd_waves_in_turns(D, Sq, Sk, kv_len, qoff, causal, monkeypatch):
             assert torch.ops.sxe.flash_attn_fwd(q, k, v, causal, D ** -0.5, kv_len, qoff)[0][:, :96].isfinite().all()
 
 
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,S,H,Hk,D", [(1, 4096, 10, 2, 64),   # 320 workgroups of 128 rows: the second half of the grid runs backwards
+                                        (1, 2176, 20, 5, 128),  # 340, no whole 256 rows
+                                        (1, 2048, 64, 16, 128),  # 512 of 256: eight waves; K/V heads fill the chip
+                                        (4, 1024, 64, 16, 64),  # 1024 of 256
+                                        (1, 512, 8, 1, 128)])   # dK / dV of 8 query heads in parts
+def test_flash_default_launch_rules(B, S, H, Hk, D, causal, monkeypatch):
+    """The launches that the sizes choose against the fp32 oracle, per head (bf16 results of fp32 sums: as the tests above)."""
+    A = _no_sdpa(monkeypatch)
+    torch.manual_seed(5)
+    q = torch.randn(B, S, H, D, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+    k = torch.randn(B, S, Hk, D, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+    v = torch.randn(B, S, Hk, D, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+    do = torch.randn(B, S, H, D, device="cuda", dtype=torch.bfloat16)
+    o = A.attention(q, k, v, causal=causal)
+    o.backward(do)
+    G = H // Hk
+    for hk in (0, Hk - 1):
+        q2, do2 = (t[:, :, hk * G:(hk + 1) * G].detach().float() for t in (q, do))
+        q2.requires_grad_()
+        k2, v2 = (t[:, :, hk:hk + 1].detach().float().requires_grad_() for t in (k, v))
+        o2 = A.reference_attention(q2, k2, v2, causal=causal)
+        o2.backward(do2)
+        assert _rel(o[:, :, hk * G:(hk + 1) * G], o2) < 1e-2
+        assert _rel(q.grad[:, :, hk * G:(hk + 1) * G], q2.grad) < 2e-2
+        assert _rel(k.grad[:, :, hk:hk + 1], k2.grad) < 2e-2 and _rel(v.grad[:, :, hk:hk + 1], v2.grad) < 2e-2
+
+
 def _chunked_reference(q, k, v, do, causal, chunk=1024):
     """fp32 attention output and gradients for long sequences, one query block at a time (the full
     score matrix of S = 16k would not be materialised at once). q [B, S, H, D], k/v [B, S, Hk, D]."""
