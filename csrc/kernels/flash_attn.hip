@@ -19,8 +19,8 @@
 //  * V^T / K^T / Q^T / dO^T operands come from row-major LDS tiles through ds_read_b64_tr_b16
 //    (hardware transpose), with the XOR-swizzled 256-byte-row image that is conflict-free for
 //    both the row reads (ds_read_b128) and the transposed reads;
-//  * K/V (or Q/dO) tiles are register-staged one tile ahead (loads issued early, written late) into a
-//    double-buffered LDS ring: one barrier per tile;
+//  * K/V (or Q/dO) tiles go straight to LDS one tile ahead, into a double-buffered ring: one barrier
+//    per tile, or two phases of a tile in which the waves of a SIMD take turns (fwd_pp_kernel);
 //  * backward = pre-pass (-delta = -rowsum(dO * O), lse * log2(e)) + dQ kernel (forward-shaped) +
 //    dK/dV kernel (keys on lanes, dK^T/dV^T accumulated in registers across the GQA query heads): no
 //    atomics, deterministic.
