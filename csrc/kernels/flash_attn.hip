@@ -221,8 +221,8 @@ __device__ __forceinline__ int build_tile_list(const Sparse sp, int head, int t_
 // Heavy-first mapping of the flat block index onto (b, head, row-block) for the causal triangle. A grid
 // of four-wave workgroups that is resident at once, two on a CU, is not evened out by the order in which
 // they finish: its second half runs backwards, so that the CU with the heaviest first workgroup has the
-// lightest second one (causal, forward [1, 8192, 8, 2, 128] 204 -> 191 us, backward 700 -> 671;
-// [1, 16384, 4, 1, 128] 393 -> 360 and 1352 -> 1268).
+// lightest second one (causal, backward [1, 8192, 8, 2, 128] 700 -> 671 us, [1, 16384, 4, 1, 128]
+// 1352 -> 1268).
 __device__ __forceinline__ void map_block(int nblk, int BH, bool heavy_last_index, int& bh, int& blk) {
   int idx = blockIdx.x;
   const int grid = nblk * BH;
@@ -590,21 +590,26 @@ __device__ __forceinline__ void pp_softmax(PPState<D>& st, float c, int kbase, i
 #pragma unroll
   for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(st.p[i]));
 }
-template <bool SPARSE, int D>
+// PAIRED: the two waves of a SIMD also share 32 queries (128 a workgroup) and take every other tile of
+// theirs, 128 keys a step; their sums meet at the end. Twice the workgroups with half the chain of tiles:
+// for grids that do not fill the chip, and causal ones that wait for their heaviest workgroup.
+template <bool SPARSE, int D, bool PAIRED = false>
 __global__ void __launch_bounds__(512, 1) fwd_pp_kernel(
     const unsigned short* __restrict__ q, Strides qs, const unsigned short* __restrict__ k, Strides ks,
     const unsigned short* __restrict__ v, Strides vs, unsigned short* __restrict__ o, Strides os,
     float* __restrict__ lse, int B, int H, int Hk, int Sq, int Sk, float scale, int causal, Sparse sp, int kvlen,
     int qoff) {
-  constexpr int ROWB = 2 * D, TILE = KT * ROWB, NWF = 8, QBF = NWF * QW;
-  int* tlist = reinterpret_cast<int*>(smem + 4 * TILE) + 1;
+  constexpr int ROWB = 2 * D, TILE = KT * ROWB, NWF = 8, QBF = (PAIRED ? 4 : 8) * QW;
+  constexpr int KS = PAIRED ? 2 * KT : KT, STEP = KS * ROWB;  // keys of a step, bytes of them
+  int* tlist = reinterpret_cast<int*>(smem + 4 * STEP) + 1;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, h = lane >> 5;
   const int nqb = Sq / QBF;
   int bh, qb;
   map_block(nqb, B * H, causal != 0, bh, qb);
   const int b = bh / H, head = bh - b * H;
   const int kh = head / (H / Hk);
-  const int q0 = qb * QBF + w * QW;
+  const int pair = PAIRED ? w >> 2 : 0;
+  const int q0 = qb * QBF + (PAIRED ? w & 3 : w) * QW;
   const int qpos = q0 + qoff;
   const unsigned short* qp = q + b * qs.b + head * qs.h;
   const unsigned short* kp = k + b * ks.b + kh * ks.h;
@@ -619,12 +624,13 @@ __global__ void __launch_bounds__(512, 1) fwd_pp_kernel(
   st.m = -INFINITY;
   st.l = 0.f;
   const int kend = causal ? min(Sk, (qb + 1) * QBF + qoff) : Sk;
-  const int nkt = (max(kend, 0) + KT - 1) / KT;
-  const int ntiles = SPARSE ? build_tile_list(sp, head, 0, nkt, KT, qb * QBF, qb * QBF + QBF, true, tlist) : nkt;
+  const int nkt = (max(kend, 0) + KS - 1) / KS;  // Sk is a multiple of 128
+  const int ntiles = SPARSE ? build_tile_list(sp, head, 0, nkt, KS, qb * QBF, qb * QBF + QBF, true, tlist) : nkt;
   auto tile_at = [&](int i) { return SPARSE ? tlist[i] : i; };
+  auto key_of = [&](int i) { return tile_at(i) * KS + pair * KT; };  // first key of this wave's tile
   const uint8_t* lrow = SPARSE ? sp.layout + ((int64_t)head * sp.nb + (q0 + r) / sp.blk) * sp.nb : nullptr;
   // two slots of K tiles, then two of V tiles
-  if (ntiles > 0) tile_glds<KT, D, NWF>(kp, ks.s, tile_at(0) * KT, smem);
+  if (ntiles > 0) tile_glds<KS, D, NWF>(kp, ks.s, tile_at(0) * KS, smem);
   vm_wait_all();
   __syncthreads();
   LaneOffs<D> lo;
@@ -633,24 +639,25 @@ __global__ void __launch_bounds__(512, 1) fwd_pp_kernel(
   // K tile t + 1 and V tile t set out, both wanted from phase 2 t + 2 on; the tiles whose slots they
   // take, K t - 1 and V t - 2, were last read in phase 2 t - 1.
   auto issue = [&](int t, int slot) {
-    if (t + 1 < ntiles) tile_glds<KT, D, NWF>(kp, ks.s, tile_at(t + 1) * KT, smem + (slot ^ 1) * TILE);
-    if (t < ntiles) tile_glds<KT, D, NWF>(vp, vs.s, tile_at(t) * KT, smem + (2 + slot) * TILE);
+    if (t + 1 < ntiles) tile_glds<KS, D, NWF>(kp, ks.s, tile_at(t + 1) * KS, smem + (slot ^ 1) * STEP);
+    if (t < ntiles) tile_glds<KS, D, NWF>(vp, vs.s, tile_at(t) * KS, smem + (2 + slot) * STEP);
   };
   // tiles this wave's queries see: the first `nact` (the list ascends)
   int nact = ntiles;
   if (causal)
-    while (nact > 0 && tile_at(nact - 1) * KT > qpos + QW - 1) --nact;
+    while (nact > 0 && key_of(nact - 1) > qpos + QW - 1) --nact;
   auto sphase = [&](int t) {
     if (t >= nact) return;
-    const int kbase = tile_at(t) * KT;
+    const int kbase = key_of(t);
     pp_softmax<D>(st, c, kbase, qpos, r, h, causal && (kbase + KT - 1 > qpos), kbase + KT > kvlen, kvlen, lrow,
                   SPARSE ? sp.blk : 1);
   };
+  const char* mine = smem + pair * TILE;
   // V product of tile t - 1, scores of tile t
   auto mphase = [&](int slot) {
     __builtin_amdgcn_s_setprio(1);
-    pp_pv<D>(lo, st, smem + (2 + (slot ^ 1)) * TILE);
-    pp_qk<D>(lo, st, smem + slot * TILE);
+    pp_pv<D>(lo, st, mine + (2 + (slot ^ 1)) * STEP);
+    pp_qk<D>(lo, st, mine + slot * STEP);
     // operand reads (0x100) ahead of the products (0x008): a V fragment is two reads, a K fragment one
     __builtin_amdgcn_sched_group_barrier(0x100, 12, 0);
 #pragma unroll
@@ -691,8 +698,8 @@ __global__ void __launch_bounds__(512, 1) fwd_pp_kernel(
         } else if (t == nact) {
           // keys 32..63 of the last tile that all follow this wave's last query are left out: their
           // values are no factor of the result (0 x NaN would be seen)
-          const int kbase = tile_at(t - 1) * KT;
-          pp_pv<D>(lo, st, smem + (2 + ((t - 1) & 1)) * TILE,
+          const int kbase = key_of(t - 1);
+          pp_pv<D>(lo, st, mine + (2 + ((t - 1) & 1)) * STEP,
                    !SPARSE && causal && kbase + KT <= kvlen && kbase + 32 > qpos + QW - 1);
         }
       };
@@ -708,7 +715,7 @@ __global__ void __launch_bounds__(512, 1) fwd_pp_kernel(
   };
   issue(0, 0);
   if (w < 4) {
-    if (nact > 0) pp_qk<D>(lo, st, smem);
+    if (nact > 0) pp_qk<D>(lo, st, mine);
     __syncthreads();
     sphase(0);
     vm_wait_all();
@@ -716,10 +723,31 @@ __global__ void __launch_bounds__(512, 1) fwd_pp_kernel(
     sweep(std::true_type{});
   } else {
     __syncthreads();
-    if (nact > 0) pp_qk<D>(lo, st, smem);
+    if (nact > 0) pp_qk<D>(lo, st, mine);
     vm_wait_all();
     __syncthreads();
     sweep(std::false_type{});
+  }
+  if constexpr (PAIRED) {  // nothing is in flight to the ring and nobody reads it any more
+    float* part = reinterpret_cast<float*>(smem) + (w & 3) * (D / 2 + 2) * 64 + lane;
+    if (pair) {
+#pragma unroll
+      for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) part[(16 * dt + i) * 64] = st.oacc[dt][i];
+      part[D / 2 * 64] = st.m;
+      part[(D / 2 + 1) * 64] = st.l;
+    }
+    __syncthreads();
+    if (pair) return;
+    const float m1 = part[D / 2 * 64], mx = fmaxf(st.m, m1), ref = mx == -INFINITY ? 0.f : mx;
+    const float e0 = fast_exp2(st.m - ref), e1 = fast_exp2(m1 - ref);
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) st.oacc[dt][i] = __builtin_fmaf(part[(16 * dt + i) * 64], e1, st.oacc[dt][i] * e0);
+    st.l = __builtin_fmaf(part[(D / 2 + 1) * 64], e1, st.l * e0);
+    st.m = mx;
   }
   const float lt = st.l + __shfl_xor(st.l, 32, 64);
   const float inv = lt > 0.f ? 1.f / lt : 0.f;  // a fully masked row outputs zeros
@@ -1195,13 +1223,13 @@ static int env_int(const char* name, int dflt) {
   const char* e = std::getenv(name);
   return (e != nullptr && *e != 0) ? std::atoi(e) : dflt;
 }
-// Rows of 256 or 128 queries a workgroup, by how many of 256 there are (`blocks`), us, eight waves / four.
-// Forward, causal: up to one workgroup of 256 a CU the heaviest of them sets the time, and four waves
-// alone on a CU are the faster half of it: 64 blocks, D 128, S 4096 94 / 88, 128 blocks, S 8192 187 / 178,
-// 256 blocks, S 16384 374 / 360; beyond, eight waves are: 512 blocks, S 2048 84 / 95, S 8192 258 / 318, 1024
-// blocks, S 2048 169 / 175. D 64: 256 blocks, S 8192 153 / 147, 512 blocks, S 2048 58 / 54, S 4096 99 / 98,
-// S 8192 173 / 188, 1024 blocks, S 2048 115 / 93. Not causal: 128 blocks, D 128, S 8192 194 / 184, 256 blocks
-// 252 / 350, 512 blocks 513 / 607; D 64 154 / 138, 173 / 226, 337 / 359.
+// By how many workgroups of 256 queries there are (`blocks`), us, eight waves of 256 / four of 128 / eight in pairs of 128.
+// Forward, causal: up to one workgroup of 256 a CU the heaviest of them sets the time. D 128, 64 blocks, S 4096
+// 100 / 88 / 58, 128 blocks, S 8192 184 / 175 / 117, 256 blocks, S 1024 36 / 33 / 35, S 8192 197 / 190 / 151, S 16384 395 / 370 /
+// 284, 512 blocks, S 2048 83 / 92 / 100, S 8192 266 / 323 / 298, 1024 blocks, S 2048 167 / 170 / 210; D 64, 128 blocks, S 8192
+// 148 / 139 / 85, 256 blocks 155 / 148 / 103, 512 blocks, S 2048 59 / 55 / 68, S 4096 100 / 101 / 120, S 8192 185 / 193 / 206,
+// 1024 blocks, S 2048 115 / 95 / 134. Not causal: D 128, 64 blocks, S 4096 105 / 92 / 64, 128 blocks, S 8192 196 / 186 / 143, 256
+// blocks 253 / 299 / 283, 512 blocks 501 / 571 / 559; D 64 82 / 74 / 45, 150 / 138 / 92, 168 / 202 / 184, 331 / 347 / 359.
 // dQ (with dK / dV), causal: D 128, 128 blocks, S 8192 655 / 624, 256 blocks 699 / 691, 512 blocks, S 2048
 // 321 / 330, S 4096 536 / 586, S 8192 935 / 1009; D 64, 512 blocks, S 2048 189 / 176, S 4096 339 / 332, S 8192
 // 574 / 580. Not causal: D 128, 128 blocks, S 8192 1790 / 1738, 256 blocks 1863 / 1935, 512 blocks 2226 /
@@ -1212,7 +1240,8 @@ static bool fwd_wide(int D, int64_t blocks, int Sq, bool causal) {
 static bool dq_wide(int D, int64_t blocks, int Sq, bool causal) {
   return causal ? blocks > kNumCUs && (D == 128 || Sq >= 8192) : blocks >= kNumCUs;
 }
-// SXE_FA_FWD_WAVES = 4 / 8 forces the forward's
+static bool fwd_paired(int64_t blocks128, bool causal) { return blocks128 <= (causal ? 2 : 1) * kNumCUs; }
+// SXE_FA_FWD_WAVES = 4 / 8 / 16 (pairs) forces the forward's
 static bool fwd_dma() { return env_int("SXE_FA_FWD_DMA", 1) != 0; }
 
 template <typename F>
@@ -1230,7 +1259,7 @@ static std::vector<at::Tensor> fwd_impl_d(at::Tensor q, at::Tensor k, at::Tensor
   auto o = at::empty({B, Sq, H, D}, q.options());
   auto lse = at::empty({B, H, Sq}, q.options().dtype(at::kFloat));
   constexpr int ROWB = 2 * D;
-  const size_t lds = 4 * fa::KT * ROWB + (sp.layout ? kListBytes : 0);
+  size_t lds = 4 * fa::KT * ROWB + (sp.layout ? kListBytes : 0);
   static bool attr = false;
   if (!attr) {
     const size_t mx = 4 * fa::KT * ROWB + kListBytes;
@@ -1247,6 +1276,7 @@ static std::vector<at::Tensor> fwd_impl_d(at::Tensor q, at::Tensor k, at::Tensor
         set_lds_limit(&fa::fwd_kernel<true, 8, D, true>, mx);
       }
       set_lds_limit(&fa::fwd_pp_kernel<true, D>, mx);
+      set_lds_limit(&fa::fwd_pp_kernel<false, D, true>, 2 * 4 * fa::KT * ROWB);
     }
     attr = true;
   }
@@ -1272,8 +1302,18 @@ static std::vector<at::Tensor> fwd_impl_d(at::Tensor q, at::Tensor k, at::Tensor
         in_step = wide && (sp.layout || (!causal && (int64_t)B * H * Sq / 256 >= 2 * kNumCUs && fww == 0));
         if (in_step) sp.layout ? launch(fa::fwd_kernel<true, 8, D, true>, 8) : launch(fa::fwd_kernel<false, 8, D, true>, 8);
       }
+      const bool paired = !sp.layout && (fww == 0 ? !wide && fwd_paired(grid, causal) : fww == 16);
       if (in_step)
         ;
+      else if (paired) {
+        lds = 2 * 4 * fa::KT * ROWB;
+        hipLaunchKernelGGL((fa::fwd_pp_kernel<false, D, true>), dim3(grid), dim3(512), lds, cur_stream(),
+                       reinterpret_cast<const unsigned short*>(q.data_ptr()), strides_of(q),
+                       reinterpret_cast<const unsigned short*>(k.data_ptr()), strides_of(k),
+                       reinterpret_cast<const unsigned short*>(v.data_ptr()), strides_of(v),
+                       reinterpret_cast<unsigned short*>(o.data_ptr()), strides_of(o), lse.data_ptr<float>(), B, H, Hk,
+                       Sq, Sk, (float)scale, causal ? 1 : 0, sp, kvlen, qoff);
+      }
       else if (wide)
         sp.layout ? launch(fa::fwd_pp_kernel<true, D>, 8) : launch(fa::fwd_pp_kernel<false, D>, 8);
       else

@@ -319,10 +319,17 @@ def test_flash_fwd_waves_in_turns(D, Sq, Sk, kv_len, qoff, causal, monkeypatch):
         out.append(torch.ops.sxe.flash_attn_fwd(q, k, v, causal, D ** -0.5, kv_len, qoff))
     for a, b in zip(*out):
         assert torch.equal(a, b)
+    # in pairs the sums of every other tile meet at the end, each against a maximum of its own: the probabilities are
+    # rounded to bf16 at other places (2^-8 of each, twice, of sum p |v|), and so is the result
+    size = torch.ops.sxe.flash_attn_fwd(q, k, v.abs(), causal, D ** -0.5, kv_len, qoff)[0].float()
+    monkeypatch.setenv("SXE_FA_FWD_WAVES", "16")
+    o, lse = torch.ops.sxe.flash_attn_fwd(q, k, v, causal, D ** -0.5, kv_len, qoff)
+    assert bool(((o.float() - out[1][0].float()).abs() <= 2 ** -7 * (out[1][0].float().abs() + 1.01 * size)).all())
+    torch.testing.assert_close(lse, out[1][1], rtol=2 ** -18, atol=2 ** -16)
     if causal and qoff == 0:  # a value that no query before it sees, at the start of half a tile
         v[:, 96] = float("nan")
         k[:, 96] = float("inf")
-        for waves in ("8", "4"):
+        for waves in ("8", "4", "16"):
             monkeypatch.setenv("SXE_FA_FWD_WAVES", waves)
             assert torch.ops.sxe.flash_attn_fwd(q, k, v, causal, D ** -0.5, kv_len, qoff)[0][:, :96].isfinite().all()
 
