@@ -847,7 +847,9 @@ __device__ __forceinline__ void dq_tile(const LaneOffs<D>& lo, const char* kt, c
 // NWF waves per workgroup, 32 queries each: 8 (256 queries) shares every staged K/V tile among twice
 // the queries of 4 -- half the L2-to-LDS tile traffic per query, at one workgroup per CU
 // (SXE_FA_DQ_WAVES, read per call; Sq a multiple of 256, head dims 64 / 128)
-template <bool SPARSE, int D, int NWF = 4>
+// PAIRED (of 8): waves w and w + 4 share 32 queries and take every other tile of theirs, 128 keys a
+// step; their sums meet at the end (see fwd_pp_kernel)
+template <bool SPARSE, int D, int NWF = 4, bool PAIRED = false>
 __global__ void __launch_bounds__(NWF * 64, (NWF == 8 ? 1 : bwd_min_waves<D>())) dq_kernel(
     const unsigned short* __restrict__ q, Strides qs, const unsigned short* __restrict__ k, Strides ks,
     const unsigned short* __restrict__ v, Strides vs, const unsigned short* __restrict__ dout, Strides dos,
@@ -855,16 +857,17 @@ __global__ void __launch_bounds__(NWF * 64, (NWF == 8 ? 1 : bwd_min_waves<D>()))
     int B, int H, int Hk, int Sq, int Sk, float scale, int causal, Sparse sp, int kvlen, int qoff) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int ROWB = 2 * D;
-  constexpr int BUF = 2 * KT * ROWB;
-  int* tlist = reinterpret_cast<int*>(smem + 4 * KT * ROWB) + 1;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 31, h = lane >> 5;
-  constexpr int QBF = NWF * QW;
+  constexpr int KS = PAIRED ? 2 * KT : KT, BUF = 2 * KS * ROWB;  // keys of a step, ring slot
+  int* tlist = reinterpret_cast<int*>(smem + 2 * BUF) + 1;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, h = lane >> 5;
+  constexpr int QBF = (PAIRED ? NWF / 2 : NWF) * QW;
+  const int pair = PAIRED ? w >> 2 : 0;
   const int nqb = Sq / QBF;
   int bh, qb;
   map_block(nqb, B * H, causal != 0, bh, qb);
   const int b = bh / H, head = bh - b * H;
   const int kh = head / (H / Hk);
-  const int q0 = qb * QBF + w * QW;
+  const int q0 = qb * QBF + (PAIRED ? w & 3 : w) * QW;
   const int qpos = q0 + qoff;
   const unsigned short* qp = q + b * qs.b + head * qs.h;
   const unsigned short* dop = dout + b * dos.b + head * dos.h;
@@ -873,13 +876,13 @@ __global__ void __launch_bounds__(NWF * 64, (NWF == 8 ? 1 : bwd_min_waves<D>()))
   const float c = scale * LOG2E;
   const int64_t lrow = ((int64_t)b * H + head) * Sq + q0 + r;
   const int kend = causal ? min(Sk, (qb + 1) * QBF + qoff) : Sk;
-  const int nkt = (max(kend, 0) + KT - 1) / KT;
-  const int ntiles = SPARSE ? build_tile_list(sp, head, 0, nkt, KT, qb * QBF, qb * QBF + QBF, true, tlist) : nkt;
+  const int nkt = (max(kend, 0) + KS - 1) / KS;
+  const int ntiles = SPARSE ? build_tile_list(sp, head, 0, nkt, KS, qb * QBF, qb * QBF + QBF, true, tlist) : nkt;
   auto tile_at = [&](int i) { return SPARSE ? tlist[i] : i; };
   const uint8_t* lay_row = SPARSE ? sp.layout + ((int64_t)head * sp.nb + (q0 + r) / sp.blk) * sp.nb : nullptr;
   if (ntiles > 0) {
-    tile_glds<KT, D, NWF>(kp, ks.s, tile_at(0) * KT, smem);
-    tile_glds<KT, D, NWF>(vp, vs.s, tile_at(0) * KT, smem + KT * ROWB);
+    tile_glds<KS, D, NWF>(kp, ks.s, tile_at(0) * KS, smem);
+    tile_glds<KS, D, NWF>(vp, vs.s, tile_at(0) * KS, smem + KS * ROWB);
   }
 
   const float lse2 = lse[lrow] * LOG2E;
@@ -905,14 +908,14 @@ __global__ void __launch_bounds__(NWF * 64, (NWF == 8 ? 1 : bwd_min_waves<D>()))
   auto step = [&](const int t, auto slot) {
     constexpr int CUR = decltype(slot)::value;
     if (t + 1 < ntiles) {
-      tile_glds<KT, D, NWF>(kp, ks.s, tile_at(t + 1) * KT, smem + (CUR ^ 1) * BUF);
-      tile_glds<KT, D, NWF>(vp, vs.s, tile_at(t + 1) * KT, smem + (CUR ^ 1) * BUF + KT * ROWB);
+      tile_glds<KS, D, NWF>(kp, ks.s, tile_at(t + 1) * KS, smem + (CUR ^ 1) * BUF);
+      tile_glds<KS, D, NWF>(vp, vs.s, tile_at(t + 1) * KS, smem + (CUR ^ 1) * BUF + KS * ROWB);
     }
-    const int kbase = tile_at(t) * KT;
+    const int kbase = tile_at(t) * KS + pair * KT;
     const bool active = !causal || kbase <= qpos + QW - 1;
     if (active) {
-      const char* kt = smem + CUR * BUF;
-      const char* vt = smem + CUR * BUF + KT * ROWB;
+      const char* kt = smem + CUR * BUF + pair * KT * ROWB;
+      const char* vt = kt + KS * ROWB;
       const bool diag = causal && (kbase + KT - 1 > qpos);
       const bool tail = kbase + KT > kvlen;
       if (SPARSE || diag || tail)
@@ -928,6 +931,21 @@ __global__ void __launch_bounds__(NWF * 64, (NWF == 8 ? 1 : bwd_min_waves<D>()))
   for (int t = 0; t < ntiles; t += 2) {
     step(t, std::integral_constant<int, 0>{});
     if (t + 1 < ntiles) step(t + 1, std::integral_constant<int, 1>{});
+  }
+  if constexpr (PAIRED) {  // nothing is in flight to the ring and nobody reads it any more
+    float* part = reinterpret_cast<float*>(smem) + (w & 3) * (D / 2) * 64 + lane;
+    if (pair) {
+#pragma unroll
+      for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) part[(16 * dt + i) * 64] = dqacc[dt][i];
+    }
+    __syncthreads();
+    if (pair) return;
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) dqacc[dt][i] += part[(16 * dt + i) * 64];
   }
   unsigned short* op = dq + b * dqs.b + head * dqs.h + (int64_t)(q0 + r) * dqs.s;
 #pragma unroll
@@ -1240,7 +1258,10 @@ static bool fwd_wide(int D, int64_t blocks, int Sq, bool causal) {
 static bool dq_wide(int D, int64_t blocks, int Sq, bool causal) {
   return causal ? blocks > kNumCUs && (D == 128 || Sq >= 8192) : blocks >= kNumCUs;
 }
-static bool fwd_paired(int64_t blocks128, bool causal) { return blocks128 <= (causal ? 2 : 1) * kNumCUs; }
+// dQ's pairs against four waves (with dK / dV), causal: D 128, 64 blocks, S 4096 348 / 291, 128 blocks, S 8192 669 / 559, 256
+// blocks, S 1024 132 / 130, S 8192 725 / 632, S 16384 1395 / 1233, 512 blocks, S 2048 333 / 363, S 8192 1018 / 1017; D 64, 128 blocks
+// 430 / 370, 256 blocks 448 / 392. Not causal: D 128, 128 blocks, S 8192 689 / 602, 256 blocks, S 1024 173 / 199, S 8192 961 / 953.
+static bool fa_paired(int64_t blocks128, bool causal) { return blocks128 <= (causal ? 2 : 1) * kNumCUs; }
 // SXE_FA_FWD_WAVES = 4 / 8 / 16 (pairs) forces the forward's
 static bool fwd_dma() { return env_int("SXE_FA_FWD_DMA", 1) != 0; }
 
@@ -1302,7 +1323,7 @@ static std::vector<at::Tensor> fwd_impl_d(at::Tensor q, at::Tensor k, at::Tensor
         in_step = wide && (sp.layout || (!causal && (int64_t)B * H * Sq / 256 >= 2 * kNumCUs && fww == 0));
         if (in_step) sp.layout ? launch(fa::fwd_kernel<true, 8, D, true>, 8) : launch(fa::fwd_kernel<false, 8, D, true>, 8);
       }
-      const bool paired = !sp.layout && (fww == 0 ? !wide && fwd_paired(grid, causal) : fww == 16);
+      const bool paired = !sp.layout && (fww == 0 ? !wide && fa_paired(grid, causal) : fww == 16);
       if (in_step)
         ;
       else if (paired) {
@@ -1373,6 +1394,7 @@ static void bwd_impl_d(at::Tensor dout, at::Tensor q, at::Tensor k, at::Tensor v
     if constexpr (D < 256) {
       set_lds_limit(&fa::dq_kernel<false, D, 8>, 4 * fa::KT * ROWB + kListBytes);
       set_lds_limit(&fa::dq_kernel<true, D, 8>, 4 * fa::KT * ROWB + kListBytes);
+      set_lds_limit(&fa::dq_kernel<false, D, 8, true>, 8 * fa::KT * ROWB);
     }
     set_lds_limit(&fa::dkdv_kernel<false, D>, lds_kv_max);
     set_lds_limit(&fa::dkdv_kernel<true, D>, lds_kv_max);
@@ -1392,12 +1414,14 @@ static void bwd_impl_d(at::Tensor dout, at::Tensor q, at::Tensor k, at::Tensor v
   // 8-wave dQ workgroups (SXE_FA_DQ_WAVES=4 / 8 forces)
   const int dqw = env_int("SXE_FA_DQ_WAVES", 0);
   const bool dq8 = D < 256 && Sq % 256 == 0 && (dqw == 8 || (dqw == 0 && (sp.layout ? Sq >= 8192 : dq_wide(D, (int64_t)B * H * Sq / 256, Sq, causal))));
+  const bool dqp = D < 256 && !sp.layout && (dqw == 16 || (dqw == 0 && !dq8 && fa_paired(B * H * (int64_t)(Sq / fa::QB), causal)));
   auto* dqk = sp.layout ? fa::dq_kernel<true, D> : fa::dq_kernel<false, D>;
   if constexpr (D < 256) {
     if (dq8) dqk = sp.layout ? fa::dq_kernel<true, D, 8> : fa::dq_kernel<false, D, 8>;
+    if (dqp) dqk = fa::dq_kernel<false, D, 8, true>;
   }
   hipLaunchKernelGGL(dqk, dim3((Sq / (dq8 ? 2 * fa::QB : fa::QB)) * B * H),
-                     dim3(dq8 ? 512 : 256), lds_dq, cur_stream(),
+                     dim3(dq8 || dqp ? 512 : 256), dqp ? 8 * fa::KT * ROWB : lds_dq, cur_stream(),
                      reinterpret_cast<const unsigned short*>(q.data_ptr()), strides_of(q),
                      reinterpret_cast<const unsigned short*>(k.data_ptr()), strides_of(k),
                      reinterpret_cast<const unsigned short*>(v.data_ptr()), strides_of(v),

@@ -334,6 +334,26 @@ def test_flash_fwd_waves_in_turns(D, Sq, Sk, kv_len, qoff, causal, monkeypatch):
             assert torch.ops.sxe.flash_attn_fwd(q, k, v, causal, D ** -0.5, kv_len, qoff)[0][:, :96].isfinite().all()
 
 
+@pytest.mark.parametrize("Sq,Sk,causal", [(256, 128, False), (128, 384, True), (384, 384, True), (512, 128, True)])
+@pytest.mark.parametrize("D", [64, 128])
+def test_flash_dq_pairs(D, Sq, Sk, causal, monkeypatch):
+    """dQ by pairs of waves that take every other tile (none, one, or a different number of them): the four-wave form's products,
+    their fp32 sums of 2 Sk / 64 terms added in another order (2^-24 of their sizes each, far below) and rounded once to bf16."""
+    torch.manual_seed(4)
+    q, do = (torch.randn(2, Sq, 4, D, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    k, v = (torch.randn(2, Sk, 2, D, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    o, lse = torch.ops.sxe.flash_attn_fwd(q, k, v, causal, D ** -0.5)
+    out = []
+    for waves in ("4", "16"):
+        monkeypatch.setenv("SXE_FA_DQ_WAVES", waves)
+        g = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+        torch.ops.sxe.flash_attn_bwd(do, q, k, v, o, lse, *g, causal, D ** -0.5)
+        out.append(g)
+    (a, ak, av), (b, bk, bv) = out
+    assert torch.equal(ak, bk) and torch.equal(av, bv)
+    assert bool(((a.float() - b.float()).abs() <= 2 ** -7 * a.float().abs() + 2 ** -18).all())
+
+
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("B,S,H,Hk,D", [(1, 4096, 10, 2, 64),   # 320 workgroups of 128 rows: the second half of the grid runs backwards
                                         (1, 2176, 20, 5, 128),  # 340, no whole 256 rows
