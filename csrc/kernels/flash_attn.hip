@@ -273,6 +273,19 @@ __device__ __forceinline__ void tile_glds(const unsigned short* base, int64_t ro
     glds16(base + (int64_t)(row0 + row) * row_stride + ch * 8, lds + n * 1024);
   }
 }
+// the same by four of the workgroup's waves, `w` among them
+template <int ROWS, int D>
+__device__ __forceinline__ void quad_glds(const unsigned short* base, int64_t row_stride, int row0, char* lds, int w) {
+  constexpr int CH = D / 8, RPK = 64 / CH;
+  static_assert(ROWS % (RPK * 4) == 0, "tile rows must split evenly over the waves");
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int i = 0; i < ROWS / RPK / 4; ++i) {
+    const int n = i * 4 + w, row = RPK * n + lane / CH;
+    const int ch = (lane % CH) ^ ((((row & 3) << 2) | ((row >> 2) & 3)) & (CH >= 16 ? 15 : CH - 1));
+    glds16(base + (int64_t)(row0 + row) * row_stride + ch * 8, lds + n * 1024);
+  }
+}
 // s_waitcnt vmcnt(0) through the builtin (expcnt / lgkmcnt fields left at their maxima), not inline
 // asm: the compiler's wait-count pass then knows every load it tracks has landed, so it does not
 // keep counting the operand loads issued before a tile loop as pending inside the loop (where its
@@ -859,7 +872,8 @@ __global__ void __launch_bounds__(NWF * 64, (NWF == 8 ? 1 : bwd_min_waves<D>()))
   constexpr int ROWB = 2 * D;
   constexpr int KS = PAIRED ? 2 * KT : KT, BUF = 2 * KS * ROWB;  // keys of a step, ring slot
   int* tlist = reinterpret_cast<int*>(smem + 2 * BUF) + 1;
-  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, h = lane >> 5;
+  const int lane = threadIdx.x & 63, w = PAIRED ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6,  // uniform elsewhere: 4 % slower
+            r = lane & 31, h = lane >> 5;
   constexpr int QBF = (PAIRED ? NWF / 2 : NWF) * QW;
   const int pair = PAIRED ? w >> 2 : 0;
   const int nqb = Sq / QBF;
@@ -1036,7 +1050,9 @@ __device__ __forceinline__ void dkdv_tile(const LaneOffs<D>& lo, const char* slo
 // NWK waves per workgroup, 32 keys each: 8 (256 keys, head dim 128; SXE_FA_DKDV_WAVES, read per
 // call) shares every staged Q / dO tile among twice the keys of 4 -- half the L2-to-LDS traffic per
 // key, at one workgroup per CU
-template <bool SPLIT, int D, int PART = 3, int NWK = 4>
+// PAIRED (of 8): waves w and w + 4 share 32 keys and take every other query tile, each side loading its
+// own; their sums meet at the end
+template <bool SPLIT, int D, int PART = 3, int NWK = 4, bool PAIRED = false>
 __global__ void __launch_bounds__(NWK * 64, (NWK == 8 ? 1 : bwd_min_waves<D>())) dkdv_kernel(
     const unsigned short* __restrict__ q, Strides qs, const unsigned short* __restrict__ k, Strides ks,
     const unsigned short* __restrict__ v, Strides vs, const unsigned short* __restrict__ dout, Strides dos,
@@ -1044,15 +1060,17 @@ __global__ void __launch_bounds__(NWK * 64, (NWK == 8 ? 1 : bwd_min_waves<D>()))
     unsigned short* __restrict__ dv, Strides dvs, float* __restrict__ pk, float* __restrict__ pv, int B, int H,
     int Hk, int Sq, int Sk, float scale, int causal, Sparse sp, int qoff, int hpw) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  constexpr int KB = NWK * QW;  // keys per workgroup
+  constexpr int KB = (PAIRED ? NWK / 2 : NWK) * QW;  // keys per workgroup
+  constexpr int NT = PAIRED ? 2 : 1;                 // query tiles of a step
   using G_ = KVL<D, KB>;
   char* vblk = smem;
   char* ring = smem + G_::VBLK;
-  int* tlist = reinterpret_cast<int*>(ring + 2 * G_::SLOT) + 1;
+  int* tlist = reinterpret_cast<int*>(ring + 2 * NT * G_::SLOT) + 1;
   // w via readfirstlane: the compiler then knows it (and k0, the causal `diag` test) is wave-uniform,
   // so the diagonal mask is a scalar branch rather than per-lane selects on every tile
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31,
             h = lane >> 5;
+  const int pair = PAIRED ? w >> 2 : 0, wk = PAIRED ? w & 3 : w;
   const int nkb = Sk / KB;
   int bh, kb;
   const int G = SPLIT ? hpw : H / Hk;  // query heads swept by this workgroup (sparse: 1)
@@ -1061,7 +1079,7 @@ __global__ void __launch_bounds__(NWK * 64, (NWK == 8 ? 1 : bwd_min_waves<D>()))
   const int b = bh / HB, hsel = bh - b * HB;
   const int hq0 = hsel * G;             // first query head swept by this workgroup
   const int kh = hq0 / (H / Hk);
-  const int k0 = kb * KB + w * QW;  // this wave's first key
+  const int k0 = kb * KB + wk * QW;  // this wave's first key
   const unsigned short* kp = k + b * ks.b + kh * ks.h;
   const unsigned short* vp = v + b * vs.b + kh * vs.h;
   const float c = scale * LOG2E;
@@ -1087,15 +1105,23 @@ __global__ void __launch_bounds__(NWK * 64, (NWK == 8 ? 1 : bwd_min_waves<D>()))
         ++is_h;
       }
     }
-    tile_glds<QT, D, NWK>(q + b * qs.b + hq * qs.h, qs.s, qt0, slot);
-    tile_glds<QT, D, NWK>(dout + b * dos.b + hq * dos.h, dos.s, qt0, slot + G_::TILE);
-    if (w == 0) {  // 64 lanes x 4 B: lse[32] then delta[32]
+    if constexpr (PAIRED) {
+      if ((it & 1) != pair) return;  // waves 0..3 load the even tiles, 4..7 the odd ones: each side its own
+      quad_glds<QT, D>(q + b * qs.b + hq * qs.h, qs.s, qt0, slot, wk);
+      quad_glds<QT, D>(dout + b * dos.b + hq * dos.h, dos.s, qt0, slot + G_::TILE, wk);
+    } else {
+      tile_glds<QT, D, NWK>(q + b * qs.b + hq * qs.h, qs.s, qt0, slot);
+      tile_glds<QT, D, NWK>(dout + b * dos.b + hq * dos.h, dos.s, qt0, slot + G_::TILE);
+    }
+    if (wk == 0) {  // 64 lanes x 4 B: lse[32] then delta[32]
       const int64_t lr = ((int64_t)b * H + hq) * Sq + qt0 + (lane & 31);
       glds4(lane < 32 ? (const void*)(lse + lr) : (const void*)(delta + lr), slot + 2 * G_::TILE);
     }
   };
   if constexpr ((PART & 2) != 0) tile_glds<KB, D, NWK>(vp, vs.s, kb * KB, vblk);
-  if (total > 0) issue(0, ring);
+#pragma unroll
+  for (int u = 0; u < NT; ++u)
+    if (u < total) issue(u, ring + u * G_::SLOT);
   bf16x8 kf[D / 16];
 #pragma unroll
   for (int t = 0; t < D / 16; ++t)
@@ -1118,20 +1144,52 @@ __global__ void __launch_bounds__(NWK * 64, (NWK == 8 ? 1 : bwd_min_waves<D>()))
   // unrolled by two: compile-time ring slot, hoisted LDS offsets (see fwd_kernel)
   auto step = [&](const int it, auto slotc) {
     constexpr int CUR = decltype(slotc)::value;
-    const int qt0 = sp.layout ? tlist[it] * QT : c_q;
+    int qt0 = sp.layout ? tlist[it] * QT : c_q;
     c_q = c_q + QT >= Sq ? qstart : c_q + QT;
-    const bool active = !causal || (qt0 + QT - 1 + qoff >= k0);
+    bool mine = true;
+    if constexpr (PAIRED) {  // tiles it and it + 1 (which there may not be)
+      if (pair) qt0 = c_q;
+      c_q = c_q + QT >= Sq ? qstart : c_q + QT;
+      mine = it + pair < total;
+    }
+    const bool active = mine && (!causal || (qt0 + QT - 1 + qoff >= k0));
     const bool diag = causal && (qt0 + qoff < k0 + QW);
-    if (it + 1 < total) issue(it + 1, ring + (CUR ^ 1) * G_::SLOT);
+    if constexpr (PAIRED) {
+      if (it + 2 < total) issue(it + 2, ring + (CUR ^ 1) * 2 * G_::SLOT);
+      if (it + 3 < total) issue(it + 3, ring + ((CUR ^ 1) * 2 + 1) * G_::SLOT);
+    } else {
+      if (it + 1 < total) issue(it + 1, ring + (CUR ^ 1) * G_::SLOT);
+    }
     if (active)
-      dkdv_tile<true, D, PART>(lo, ring + CUR * G_::SLOT, vblk, kf, dka, dva, c, qt0, k0, w, r, h, lane, diag, sp,
-                               hq0, kbl, qoff);
+      dkdv_tile<true, D, PART>(lo, ring + (CUR * NT + pair) * G_::SLOT, vblk, kf, dka, dva, c, qt0, k0, wk, r, h, lane, diag,
+                               sp, hq0, kbl, qoff);
     vm_wait_all();
     __syncthreads();
   };
-  for (int it = 0; it < total; it += 2) {
+  for (int it = 0; it < total; it += 2 * NT) {
     step(it, std::integral_constant<int, 0>{});
-    if (it + 1 < total) step(it + 1, std::integral_constant<int, 1>{});
+    if (it + NT < total) step(it + NT, std::integral_constant<int, 1>{});
+  }
+  if constexpr (PAIRED) {  // nothing is in flight to LDS and nobody reads it any more
+    float* part = reinterpret_cast<float*>(smem) + wk * D * 64 + lane;
+    if (pair) {
+#pragma unroll
+      for (int t = 0; t < D / 32; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          part[(16 * t + i) * 64] = dka[t][i];
+          part[(D / 2 + 16 * t + i) * 64] = dva[t][i];
+        }
+    }
+    __syncthreads();
+    if (pair) return;
+#pragma unroll
+    for (int t = 0; t < D / 32; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        dka[t][i] += part[(16 * t + i) * 64];
+        dva[t][i] += part[(D / 2 + 16 * t + i) * 64];
+      }
   }
   if (SPLIT && pk != nullptr) {  // fp32 partials, layout [B, Sk, H / hpw, D] contiguous
     float* kp32 = pk + (((int64_t)b * Sk + k0 + r) * HB + hsel) * D;
@@ -1261,6 +1319,9 @@ static bool dq_wide(int D, int64_t blocks, int Sq, bool causal) {
 // dQ's pairs against four waves (with dK / dV), causal: D 128, 64 blocks, S 4096 348 / 291, 128 blocks, S 8192 669 / 559, 256
 // blocks, S 1024 132 / 130, S 8192 725 / 632, S 16384 1395 / 1233, 512 blocks, S 2048 333 / 363, S 8192 1018 / 1017; D 64, 128 blocks
 // 430 / 370, 256 blocks 448 / 392. Not causal: D 128, 128 blocks, S 8192 689 / 602, 256 blocks, S 1024 173 / 199, S 8192 961 / 953.
+// dK / dV's (with dQ in pairs): causal, D 128, 64 blocks, S 4096 291 / 223, 128 blocks, S 8192 575 / 439, 256 blocks, S 1024 132 / 127,
+// S 8192 666 / 548, S 16384 1266 / 1042, 512 blocks, S 2048 335 / 367, S 8192 1017 / 1044; D 64, 128 blocks 376 / 295, 256 blocks
+// 420 / 347. Not causal: D 128, 128 blocks, S 8192 624 / 511, 256 blocks, S 1024 174 / 218, S 8192 969 / 990.
 static bool fa_paired(int64_t blocks128, bool causal) { return blocks128 <= (causal ? 2 : 1) * kNumCUs; }
 // SXE_FA_FWD_WAVES = 4 / 8 / 16 (pairs) forces the forward's
 static bool fwd_dma() { return env_int("SXE_FA_FWD_DMA", 1) != 0; }
@@ -1470,8 +1531,8 @@ static void bwd_impl_d(at::Tensor dout, at::Tensor q, at::Tensor k, at::Tensor v
     pk = at::empty({B, Sk, np, D}, q.options().dtype(at::kFloat));
     pv = at::empty({B, Sk, np, D}, q.options().dtype(at::kFloat));
   }
-  auto launch = [&](auto kern, int heads, int nwk = 4) {
-    hipLaunchKernelGGL(kern, dim3((Sk / (nwk * fa::QW)) * B * heads), dim3(nwk * 64), lds_kv, cur_stream(),
+  auto launch = [&](auto kern, int heads, int nwk = 4, size_t lds = 0) {
+    hipLaunchKernelGGL(kern, dim3((Sk / (nwk * fa::QW)) * B * heads), dim3(lds ? 512 : nwk * 64), lds ? lds : lds_kv, cur_stream(),
                        reinterpret_cast<const unsigned short*>(q.data_ptr()), strides_of(q),
                        reinterpret_cast<const unsigned short*>(k.data_ptr()), strides_of(k),
                        reinterpret_cast<const unsigned short*>(v.data_ptr()), strides_of(v),
@@ -1490,6 +1551,16 @@ static void bwd_impl_d(at::Tensor dout, at::Tensor q, at::Tensor k, at::Tensor v
         launch(fa::dkdv_kernel<SP, D, 1>, heads);
         SXE_LAUNCH_CHECK();
         launch(fa::dkdv_kernel<SP, D, 2>, heads);
+        return;
+      }
+    }
+    if constexpr (D < 256) {
+      if (!sp.layout && (kvw == 16 || (kvw == 0 && fa_paired((int64_t)(Sk / fa::QB) * B * heads, causal)))) {
+        const size_t lds = std::max<size_t>(G_::VBLK + 4 * G_::SLOT, 4 * D * 64 * sizeof(float));
+        static bool once = false;
+        if (!once) set_lds_limit(&fa::dkdv_kernel<SP, D, 3, 8, true>, lds);
+        once = true;
+        launch(fa::dkdv_kernel<SP, D, 3, 8, true>, heads, 4, lds);
         return;
       }
     }

@@ -336,9 +336,10 @@ def test_flash_fwd_waves_in_turns(D, Sq, Sk, kv_len, qoff, causal, monkeypatch):
 
 @pytest.mark.parametrize("Sq,Sk,causal", [(256, 128, False), (128, 384, True), (384, 384, True), (512, 128, True)])
 @pytest.mark.parametrize("D", [64, 128])
-def test_flash_dq_pairs(D, Sq, Sk, causal, monkeypatch):
-    """dQ by pairs of waves that take every other tile (none, one, or a different number of them): the four-wave form's products,
-    their fp32 sums of 2 Sk / 64 terms added in another order (2^-24 of their sizes each, far below) and rounded once to bf16."""
+def test_flash_bwd_pairs(D, Sq, Sk, causal, monkeypatch):
+    """dQ and dK / dV by pairs of waves that take every other tile (none, one, or a different number of them): the four-wave form's
+    products, their fp32 sums of a few tiles added in another order (2^-24 of the sizes of the terms each, which are below 16 here) and
+    rounded once to bf16."""
     torch.manual_seed(4)
     q, do = (torch.randn(2, Sq, 4, D, device="cuda", dtype=torch.bfloat16) for _ in range(2))
     k, v = (torch.randn(2, Sk, 2, D, device="cuda", dtype=torch.bfloat16) for _ in range(2))
@@ -346,12 +347,11 @@ def test_flash_dq_pairs(D, Sq, Sk, causal, monkeypatch):
     out = []
     for waves in ("4", "16"):
         monkeypatch.setenv("SXE_FA_DQ_WAVES", waves)
-        g = [torch.full_like(t, float("nan")) for t in (q, k, v)]
-        torch.ops.sxe.flash_attn_bwd(do, q, k, v, o, lse, *g, causal, D ** -0.5)
-        out.append(g)
-    (a, ak, av), (b, bk, bv) = out
-    assert torch.equal(ak, bk) and torch.equal(av, bv)
-    assert bool(((a.float() - b.float()).abs() <= 2 ** -7 * a.float().abs() + 2 ** -18).all())
+        monkeypatch.setenv("SXE_FA_DKDV_WAVES", waves)
+        out.append([torch.full_like(t, float("nan")) for t in (q, k, v)])
+        torch.ops.sxe.flash_attn_bwd(do, q, k, v, o, lse, *out[-1], causal, D ** -0.5)
+    for a, b in zip(*out):
+        assert bool(((a.float() - b.float()).abs() <= 2 ** -7 * a.float().abs() + 2 ** -18).all())
 
 
 @pytest.mark.parametrize("causal", [True, False])
