@@ -68,8 +68,8 @@ def _register_sxe_formulas():
             return 2 * x[0] * w[0] * w[1]
 
         @register_flop_formula(ops.gemm_tn)
-        def _tiled(x, w, *a, out_shape=None, **kw):
-            return 2 * x[0] * w[0] * w[1]
+        def _tiled(x, w, *a, out_shape=None, **kw):  # x [.., K]
+            return 2 * math.prod(x) * w[0]
 
         @register_flop_formula([ops.gemm_tn_batch, ops.expert_mm_kn])
         def _batched(x, w, *a, out_shape=None, **kw):
@@ -97,6 +97,10 @@ def _register_sxe_formulas():
         @register_flop_formula(ops.wgrad_gemm_)
         def _wgrad(a, b, *rest, out_shape=None, **kw):  # c (+)= a^T b, a [.., K, M], b [.., K, N]
             return 2 * math.prod(a) * b[-1]
+
+        @register_flop_formula(ops.wgrad_gemm2_)
+        def _wgrad2(a, b, a2, b2, *rest, out_shape=None, **kw):  # c (+)= [a; a2]^T [b; b2]
+            return 2 * (math.prod(a) + math.prod(a2)) * b[-1]
     except Exception:  # formulas are optional; generic ops are still counted
         pass
 

@@ -76,3 +76,33 @@ def test_hip_ops_have_flop_formulas():
         torch.ops.sxe.flash_attn_fwd(q, q, q, True, 0.088)
     expect = 2 * 2 * 512 * 256 + 2 * 300 * 384 * 256 + 2 * 256 * 512 * 768 + 4 * 2 * 128 * 128 * 128 // 2
     assert fc.get_total_flops() == expect
+
+
+@pytest.mark.gpu
+def test_products_of_many_rows_and_experts_are_counted():
+    """Every row of a batch of sequences, every expert, both micro-steps of a deferred weight gradient."""
+    from shuffle_exchange_amd.ops import native
+    from shuffle_exchange_amd.ops.linear import linear
+    from torch.utils.flop_counter import FlopCounterMode
+    from shuffle_exchange_amd.profiling.flops_profiler.profiler import _register_sxe_formulas
+    native.require_hip()
+    _register_sxe_formulas()
+
+    def t(*shape):
+        return torch.randn(*shape, device="cuda", dtype=torch.bfloat16)
+
+    def count(f):
+        with FlopCounterMode(display=False) as fc:
+            f()
+        return fc.get_total_flops()
+    x, w = t(5, 515, 2048), t(2048, 2048)
+    assert count(lambda: torch.ops.sxe.gemm_tn(x, w, None, False)) == 2 * 5 * 515 * 2048 * 2048
+    with torch.no_grad():  # whichever product it takes
+        assert count(lambda: linear(x, w)) == 2 * 5 * 515 * 2048 * 2048
+    assert count(lambda: torch.ops.sxe.gemm_tn(t(70, 128), t(256, 128), None, True)) == 2 * 70 * 256 * 128
+    e, we = t(3, 40, 128), t(3, 128, 192)
+    assert count(lambda: torch.ops.sxe.expert_mm_kn(e, we)) == 2 * 3 * 40 * 128 * 192
+    assert count(lambda: torch.ops.sxe.gemm_tn_batch(t(3, 40, 192), we)) == 2 * 3 * 40 * 128 * 192
+    c = torch.zeros(3, 128, 192, device="cuda")
+    assert count(lambda: torch.ops.sxe.wgrad_gemm_(e, t(3, 40, 192), c, 1.0, False)) == 2 * 3 * 40 * 128 * 192
+    assert count(lambda: torch.ops.sxe.wgrad_gemm2_(e, t(3, 40, 192), t(3, 24, 128), t(3, 24, 192), c, 1.0, False)) == 2 * 3 * 64 * 128 * 192
