@@ -63,6 +63,8 @@ class _ColumnHeadXEnt(torch.autograd.Function):
         if h2.shape[0] % 64:
             h2 = F.pad(h2, (0, 0, 0, -h2.shape[0] % 64))
         h2 = h2.contiguous()
+        if h2.data_ptr() % 16:  # a view that starts inside a vector
+            h2 = h2.clone()
         logits = torch.ops.sxe.gemm_tn(weight, h2, None, False)
         loss, lse = torch.ops.sxe.xent_cols_fwd(logits, tgt, int(ignore_index))
         ctx.save_for_backward(logits, lse, tgt, h2, weight)

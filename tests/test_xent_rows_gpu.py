@@ -71,6 +71,23 @@ def test_column_head_matches_fp64(V, tokens):
         assert (a.double() - b).norm() <= 2 ** -6 * b.norm()
 
 
+@pytest.mark.parametrize("tokens", [64, 65])  # as they are, rounded up
+def test_column_head_of_unaligned_states(tokens):
+    """Hidden states that start off 16 bytes give what their copy gives."""
+    from shuffle_exchange_amd.ops.cross_entropy import head_cross_entropy, _columns_ok
+    g = torch.Generator("cuda").manual_seed(tokens)
+    w = torch.randn(1001, 128, generator=g, device="cuda").mul_(0.1).bfloat16().requires_grad_()
+    tgt = torch.randint(0, 1001, (1, tokens), generator=g, device="cuda")
+    flat = torch.randn(tokens * 128 + 1, generator=g, device="cuda").bfloat16()
+    got = []
+    for h in (flat[1:].view(1, tokens, 128), flat[1:].clone().view(1, tokens, 128)):
+        h.requires_grad_()
+        assert _columns_ok(h, w, tgt)
+        loss = head_cross_entropy(h, w, tgt)
+        got.append((loss.detach(), *torch.autograd.grad(loss, (h, w))))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
 def test_column_head_masked_vocabulary():
     """Rows of -inf logits (a hidden state of infinities) and a share with nothing else: NaN and zeros where the row form has them."""
     x = torch.randn(200, 64, device="cuda").bfloat16()
