@@ -1331,6 +1331,15 @@ static void set_lds_limit(F* f, size_t bytes) {
   SXE_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)bytes));
 }
+// the opt-ins `f` of a kernel family, once on every device of the process
+template <typename F>
+static void on_each_device(std::atomic<uint64_t>& done, F f) {
+  int dev = 0;
+  SXE_HIP_CHECK(hipGetDevice(&dev));
+  if (dev < 64 && (done.load(std::memory_order_relaxed) >> dev & 1)) return;
+  f();
+  if (dev < 64) done.fetch_or(1ull << dev, std::memory_order_relaxed);
+}
 
 // kv_len: valid keys (the rest of the padded key axis is masked); qoff: causal offset (query i sees
 // keys <= i + qoff), default Sk - Sq (bottom-right aligned)
@@ -1342,8 +1351,8 @@ static std::vector<at::Tensor> fwd_impl_d(at::Tensor q, at::Tensor k, at::Tensor
   auto lse = at::empty({B, H, Sq}, q.options().dtype(at::kFloat));
   constexpr int ROWB = 2 * D;
   size_t lds = 4 * fa::KT * ROWB + (sp.layout ? kListBytes : 0);
-  static bool attr = false;
-  if (!attr) {
+  static std::atomic<uint64_t> attr{0};
+  on_each_device(attr, [&] {
     const size_t mx = 4 * fa::KT * ROWB + kListBytes;
     set_lds_limit(&fa::fwd_kernel<false, 4, D>, mx);
     set_lds_limit(&fa::fwd_kernel<true, 4, D>, mx);
@@ -1360,8 +1369,7 @@ static std::vector<at::Tensor> fwd_impl_d(at::Tensor q, at::Tensor k, at::Tensor
       set_lds_limit(&fa::fwd_pp_kernel<true, D>, mx);
       set_lds_limit(&fa::fwd_pp_kernel<false, D, true>, 2 * 4 * fa::KT * ROWB);
     }
-    attr = true;
-  }
+  });
   // 8 waves share each staged K/V tile where that pays and the query axis allows; head dim 256 runs 4 (register budget)
   const int fww = env_int("SXE_FA_FWD_WAVES", 0);
   const bool wide = D < 256 && Sq % 256 == 0 && (fww == 8 || (fww != 4 && (sp.layout || fwd_wide(D, (int64_t)B * H * Sq / 256, Sq, causal))));
@@ -1448,8 +1456,8 @@ static void bwd_impl_d(at::Tensor dout, at::Tensor q, at::Tensor k, at::Tensor v
   SXE_LAUNCH_CHECK();
   const size_t lds_dq = 4 * fa::KT * ROWB + (sp.layout ? kListBytes : 0);
   const size_t lds_kv_max = G_::VBLK + 2 * G_::SLOT + kListBytes;
-  static bool attr_set = false;
-  if (!attr_set) {  // > 64 KiB of dynamic LDS must be opted into (gfx950 has 160 KiB per CU)
+  static std::atomic<uint64_t> attr_set{0};
+  on_each_device(attr_set, [&] {  // > 64 KiB of dynamic LDS must be opted into (gfx950 has 160 KiB per CU)
     set_lds_limit(&fa::dq_kernel<false, D>, 4 * fa::KT * ROWB + kListBytes);
     set_lds_limit(&fa::dq_kernel<true, D>, 4 * fa::KT * ROWB + kListBytes);
     if constexpr (D < 256) {
@@ -1470,8 +1478,7 @@ static void bwd_impl_d(at::Tensor dout, at::Tensor q, at::Tensor k, at::Tensor v
       set_lds_limit(&fa::dkdv_kernel<false, D, 2>, lds_kv_max);
       set_lds_limit(&fa::dkdv_kernel<true, D, 2>, lds_kv_max);
     }
-    attr_set = true;
-  }
+  });
   // 8-wave dQ workgroups (SXE_FA_DQ_WAVES=4 / 8 forces)
   const int dqw = env_int("SXE_FA_DQ_WAVES", 0);
   const bool dq8 = D < 256 && Sq % 256 == 0 && (dqw == 8 || (dqw == 0 && (sp.layout ? Sq >= 8192 : dq_wide(D, (int64_t)B * H * Sq / 256, Sq, causal))));
@@ -1557,9 +1564,7 @@ static void bwd_impl_d(at::Tensor dout, at::Tensor q, at::Tensor k, at::Tensor v
     if constexpr (D < 256) {
       if (!sp.layout && (kvw == 16 || (kvw == 0 && fa_paired((int64_t)(Sk / fa::QB) * B * heads, causal)))) {
         const size_t lds = std::max<size_t>(G_::VBLK + 4 * G_::SLOT, 4 * D * 64 * sizeof(float));
-        static bool once = false;
-        if (!once) set_lds_limit(&fa::dkdv_kernel<SP, D, 3, 8, true>, lds);
-        once = true;
+        allow_lds<&fa::dkdv_kernel<SP, D, 3, 8, true>>((int)lds);
         launch(fa::dkdv_kernel<SP, D, 3, 8, true>, heads, 4, lds);
         return;
       }
