@@ -1,4 +1,4 @@
-// The inner loop of the 16 x 16 x 32 bf16 products (gemm_tn.hip, experts_kn_tile.hip): WR x WC waves, each RT x CT blocks of 16 x 16
+// The inner loop of the 16 x 16 x 32 bf16 products (gemm_tn.hip, experts_kn_tile.hip, gemm_wgrad.hip): WR x WC waves, each RT x CT blocks of 16 x 16
 // fp32 sums, whose operands x and w stream through LDS in slabs of 64 k, SA and SB of them at once.
 //  * The loads of a slab (a wave's are PA of x and PB of w, 1 KB each) are spread over three quarters of a slab's time: a wave that
 //    issues them at once waits in front of the full address queue with its products behind it (8192 rows, 28672 x 4096, 1.20 against
@@ -34,8 +34,18 @@ __device__ __forceinline__ unsigned lds_base() {
   return __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)tl::lds);
 }
 __device__ __forceinline__ unsigned pack(float a, float b) { return (unsigned)f32_to_bf16(a) | ((unsigned)f32_to_bf16(b) << 16); }
-// one unit in the last place of 32 bits each; a correct quotient costs 10 % of a tile of 4096 k
-__device__ __forceinline__ float sigmoid(float x) { return __builtin_amdgcn_rcpf(1.f + fast_exp2(-LOG2E * x)); }
+// x / (1 + exp(-x)). FULL: to 32 bits, off by less than 5 * 2^-24 of itself (x / (1.f + expf(-x)): 3, but the quotient costs 10 % of a
+// tile of 4096 k): what rounding -LOG2E * x and LOG2E left out is put back behind the exponent; below -87 it goes to -0. Else as
+// x / (1.f + __expf(-x)), whose exponent is off as -LOG2E * x is rounded: 17 * 2^-24 at x = -16, 66 at -87.
+template <bool FULL>
+__device__ __forceinline__ float silu(float x) {
+  constexpr float kLow = 1.92596299e-8f;  // log2(e) - LOG2E
+  if constexpr (!FULL) return x * __builtin_amdgcn_rcpf(1.f + fast_exp2(-LOG2E * x));
+  const float c = __builtin_amdgcn_fmed3f(x, -88.f, 150.f), t = -LOG2E * c;
+  const float left = __builtin_fmaf(-kLow, c, __builtin_fmaf(-LOG2E, c, -t)), e = fast_exp2(t);
+  const float d = 1.f + __builtin_fmaf(e, LN2 * left, e), r = __builtin_amdgcn_rcpf(d);
+  return x * __builtin_fmaf(__builtin_fmaf(-d, r, 1.f), r, r);
+}
 
 // acc[i][j] = sums over ns slabs of (w block j)' x (x block i): a lane has row lane & 15 of x and the four rows 4 (lane >> 4) .. of w.
 //   load_x(i, slab, slot), load_w(i, slab, slot): the wave's i-th load of a slab to a slot (byte offset in x's or w's part of LDS);

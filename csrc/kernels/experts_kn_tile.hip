@@ -160,7 +160,7 @@ __global__ void __launch_bounds__(T::NTHR, T::WAVES) tile_kernel(Args a) {
 #pragma unroll
     for (int j = 0; j < (GLU ? 2 : CT); ++j)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[j][e] = GLU ? acc[i][j][e] * sigmoid(acc[i][j][e]) * acc[i][j + 2][e] : acc[i][j][e];
+      for (int e = 0; e < 4; ++e) v[j][e] = GLU ? silu<true>(acc[i][j][e]) * acc[i][j + 2][e] : acc[i][j][e];
 #pragma unroll
     for (int h = 0; h < (GLU ? 1 : 2); ++h) {
       const int c = n0 + (GLU ? 32 * wc : 64 * wc + 32 * h) + 16 * (g & 1) + 8 * (g >> 1);

@@ -111,8 +111,7 @@ __global__ void __launch_bounds__(T::NTHR, T::WAVES) gemm_kernel(Args a) {
         float v[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const float x = acc[i][2 * (e >> 2)][e & 3];
-          v[e] = x * sigmoid(x) * acc[i][2 * (e >> 2) + 1][e & 3];
+          v[e] = silu<false>(acc[i][2 * (e >> 2)][e & 3]) * acc[i][2 * (e >> 2) + 1][e & 3];
         }
         *reinterpret_cast<u32x4*>(a.y + part * a.by + (int64_t)r * a.cols + c) = u32x4{pack(v[0], v[1]), pack(v[2], v[3]), pack(v[4], v[5]), pack(v[6], v[7])};
       }
@@ -161,7 +160,7 @@ __global__ void __launch_bounds__(256) sum_kernel(const float* __restrict__ part
     }
     if (GLU) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] *= sigmoid(v[e]) * u[e];
+      for (int e = 0; e < 8; ++e) v[e] = silu<false>(v[e]) * u[e];
     } else if (bias != nullptr) {
       load8<DT::BF16>(bias + c, u);
 #pragma unroll

@@ -73,6 +73,35 @@ def test_tile_kernels(T, E, k, K, I, N, skew):
         assert (y[r].double() - wy).norm() <= 3e-3 * wy.norm()
 
 
+def _tile_activation(gate, up):
+    """silu(gate) up of [I, 64] pairs that the products hold exactly, one term each."""
+    offs, rows = torch.tensor([0, 64], device="cuda", dtype=torch.int32), torch.arange(64, device="cuda", dtype=torch.int32)
+    return torch.ops.sxe.expert_swiglu_kn_tile(torch.eye(64, device="cuda").bfloat16(), torch.cat([gate, up]).t().contiguous()[None], offs, rows)
+
+
+def test_tile_activation_in_32_bits():
+    """A million gates whose exponents are large. A value that is off by e of itself before the rounding to bf16 rounds the other way with
+    a chance of 2^8 e at the most (a spacing is 2^-8 of the value, or more): 5 units of 2^-24 let 80 of 2^20 differ, four standard
+    deviations more are 116."""
+    g = torch.Generator("cuda").manual_seed(3)
+    gate = -(16 + 64 * torch.rand(16384, 64, device="cuda", generator=g)).bfloat16()
+    up = (1 + torch.rand(16384, 64, device="cuda", generator=g)).bfloat16()
+    y = _tile_activation(gate, up)
+    want = (torch.nn.functional.silu(gate.double()) * up.double()).t()
+    assert int((y != want.bfloat16()).sum()) <= 116
+    torch.testing.assert_close(y.double(), want, rtol=2 ** -8, atol=0)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), -500.0, -88.5, -87.0, -0.0])
+def test_tile_activation_of_extremes(value):
+    """As x / (1 + exp(-x)) in 32 bits: NaN of -inf, zeros far below (from -87 on, where the result is under 2^-119)."""
+    gate = torch.zeros(128, 64, device="cuda").bfloat16()
+    gate[:, 5] = value
+    y = _tile_activation(gate, torch.ones_like(gate))[5]
+    v = gate[:, 5].double()
+    torch.testing.assert_close(y.double(), v / (1 + (-v).exp()), equal_nan=True, rtol=2 ** -8, atol=2.0 ** -119)
+
+
 def test_mixtral_decode_graphs_match_eager():
     from shuffle_exchange_amd.inference.v2 import RaggedInferenceEngineConfig, build_engine
     from shuffle_exchange_amd.models import MixtralForCausalLM, mixtral_config
