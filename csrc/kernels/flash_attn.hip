@@ -219,14 +219,17 @@ __device__ __forceinline__ int build_tile_list(const Sparse sp, int head, int t_
 }
 
 // Heavy-first mapping of the flat block index onto (b, head, row-block) for the causal triangle. A grid
-// of four-wave workgroups that is resident at once, two on a CU, is not evened out by the order in which
-// they finish: its second half runs backwards, so that the CU with the heaviest first workgroup has the
-// lightest second one (causal, backward [1, 8192, 8, 2, 128] 700 -> 671 us, [1, 16384, 4, 1, 128]
-// 1352 -> 1268).
-__device__ __forceinline__ void map_block(int nblk, int BH, bool heavy_last_index, int& bh, int& blk) {
+// of four-wave workgroups that is resident at once, two on a CU (TWO; head dim 256 has one), is not evened
+// out by the order in which they finish: its second half runs backwards, so that the CU with the heaviest
+// first workgroup has the lightest second one (causal, backward [1, 8192, 8, 2, 128] 700 -> 671 us,
+// [1, 16384, 4, 1, 128] 1352 -> 1268). Few row-blocks are near each other in weight and lose more by the
+// heads' order than that gives (512 workgroups, S 512, head dim 128, forward and backward 97 -> 100 us; 64 62 -> 65).
+template <bool TWO>
+__device__ __forceinline__ void map_block(int nblk, int BH, bool causal, bool heavy_last_index, int& bh, int& blk) {
   int idx = blockIdx.x;
   const int grid = nblk * BH;
-  if (blockDim.x == 256 && grid > kNumCUs && grid <= 2 * kNumCUs && idx >= kNumCUs) idx = grid - 1 - (idx - kNumCUs);
+  if (TWO && causal && nblk >= 16 && blockDim.x == 256 && grid > kNumCUs && grid <= 2 * kNumCUs && idx >= kNumCUs)
+    idx = grid - 1 - (idx - kNumCUs);
   const int rank = idx / BH;
   bh = idx - rank * BH;
   blk = heavy_last_index ? (nblk - 1 - rank) : rank;
@@ -406,7 +409,7 @@ __global__ void __launch_bounds__(NWF * 64, (fwd_min_waves<D, NWF>())) fwd_kerne
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 31, h = lane >> 5;
   const int nqb = Sq / QBF;
   int bh, qb;
-  map_block(nqb, B * H, causal != 0, bh, qb);
+  map_block<(D < 256 && !SPARSE)>(nqb, B * H, causal != 0, causal != 0, bh, qb);
   const int b = bh / H, head = bh - b * H;
   const int kh = head / (H / Hk);
   const int q0 = qb * QBF + w * QW;  // this wave's first query
@@ -618,7 +621,7 @@ __global__ void __launch_bounds__(512, 1) fwd_pp_kernel(
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, h = lane >> 5;
   const int nqb = Sq / QBF;
   int bh, qb;
-  map_block(nqb, B * H, causal != 0, bh, qb);
+  map_block<(D < 256 && !SPARSE)>(nqb, B * H, causal != 0, causal != 0, bh, qb);
   const int b = bh / H, head = bh - b * H;
   const int kh = head / (H / Hk);
   const int pair = PAIRED ? w >> 2 : 0;
@@ -878,7 +881,7 @@ __global__ void __launch_bounds__(NWF * 64, (NWF == 8 ? 1 : bwd_min_waves<D>()))
   const int pair = PAIRED ? w >> 2 : 0;
   const int nqb = Sq / QBF;
   int bh, qb;
-  map_block(nqb, B * H, causal != 0, bh, qb);
+  map_block<(D < 256 && !SPARSE)>(nqb, B * H, causal != 0, causal != 0, bh, qb);
   const int b = bh / H, head = bh - b * H;
   const int kh = head / (H / Hk);
   const int q0 = qb * QBF + (PAIRED ? w & 3 : w) * QW;
@@ -1075,7 +1078,7 @@ __global__ void __launch_bounds__(NWK * 64, (NWK == 8 ? 1 : bwd_min_waves<D>()))
   int bh, kb;
   const int G = SPLIT ? hpw : H / Hk;  // query heads swept by this workgroup (sparse: 1)
   const int HB = H / G;                 // workgroups along the head axis
-  map_block(nkb, B * HB, false, bh, kb);  // key block 0 is the heaviest under causality
+  map_block<(D < 256)>(nkb, B * HB, causal && !sp.layout, false, bh, kb);  // key block 0 is the heaviest under causality
   const int b = bh / HB, hsel = bh - b * HB;
   const int hq0 = hsel * G;             // first query head swept by this workgroup
   const int kh = hq0 / (H / Hk);
