@@ -1302,30 +1302,40 @@ static int env_int(const char* name, int dflt) {
   const char* e = std::getenv(name);
   return (e != nullptr && *e != 0) ? std::atoi(e) : dflt;
 }
-// By how many workgroups of 256 queries there are (`blocks`), us, eight waves of 256 / four of 128 / eight in pairs of 128.
-// Forward, causal: up to one workgroup of 256 a CU the heaviest of them sets the time. D 128, 64 blocks, S 4096
-// 100 / 88 / 58, 128 blocks, S 8192 184 / 175 / 117, 256 blocks, S 1024 36 / 33 / 35, S 8192 197 / 190 / 151, S 16384 395 / 370 /
-// 284, 512 blocks, S 2048 83 / 92 / 100, S 8192 266 / 323 / 298, 1024 blocks, S 2048 167 / 170 / 210; D 64, 128 blocks, S 8192
-// 148 / 139 / 85, 256 blocks 155 / 148 / 103, 512 blocks, S 2048 59 / 55 / 68, S 4096 100 / 101 / 120, S 8192 185 / 193 / 206,
-// 1024 blocks, S 2048 115 / 95 / 134. Not causal: D 128, 64 blocks, S 4096 105 / 92 / 64, 128 blocks, S 8192 196 / 186 / 143, 256
-// blocks 253 / 299 / 283, 512 blocks 501 / 571 / 559; D 64 82 / 74 / 45, 150 / 138 / 92, 168 / 202 / 184, 331 / 347 / 359.
-// dQ (with dK / dV), causal: D 128, 128 blocks, S 8192 655 / 624, 256 blocks 699 / 691, 512 blocks, S 2048
-// 321 / 330, S 4096 536 / 586, S 8192 935 / 1009; D 64, 512 blocks, S 2048 189 / 176, S 4096 339 / 332, S 8192
-// 574 / 580. Not causal: D 128, 128 blocks, S 8192 1790 / 1738, 256 blocks 1863 / 1935, 512 blocks 2226 /
-// 2394; D 64 1220 / 1194, 1229 / 1297, 1440 / 1470.
-static bool fwd_wide(int D, int64_t blocks, int Sq, bool causal) {
-  return causal ? blocks > kNumCUs && (D == 128 || Sq >= 8192) : blocks > kNumCUs / 2;
+// Which workgroups run, by their number and the length of the chain of tiles that each goes through. us, head dim 128 unless said,
+// n workgroups of 128 rows at sequence length S (measured at S 128 to 4096 with n 64 to 4096, causal and not).
+//
+// Eight waves of 256 rows in turns against four of 128: half as many workgroups, one a CU. Causal, n 1024, S 512 46 / 45, S 1024 56 /
+// 63, S 4096 138 / 163; n 2048, S 256 76 / 67, S 1024 120 / 120, S 2048 179 / 188. Not causal, n 384, S 1024 34 / 39, n 512, S 2048 69 / 78,
+// n 1024, S 2048 139 / 155. Head dim 64, causal: up to S 4096 four are as fast or faster (n 1024, S 2048 57 / 54, n 4096 254 / 198); not
+// causal, n 512, S 2048 45 / 52, but n 768 87 / 70: 1.5 rounds of workgroups over the CUs; from n 1024 on the waves keep in step, two
+// workgroups a CU (below).
+static bool fwd_wide(int D, int64_t n, int Sq, bool causal) {
+  if (causal) return n > 2 * kNumCUs && Sq >= (D == 128 ? 1024 : 8192);
+  return n > kNumCUs && (D == 128 || n <= 2 * kNumCUs || n >= 4 * kNumCUs);
 }
-static bool dq_wide(int D, int64_t blocks, int Sq, bool causal) {
-  return causal ? blocks > kNumCUs && (D == 128 || Sq >= 8192) : blocks >= kNumCUs;
+// Pairs of waves on 128 rows against four waves: half the chain where there is at most one workgroup a CU (n 256, S 256 causal 13.3 /
+// 13.1, not causal 14.1 / 12.7, S 512 16.6 / 18.5, 17.7 / 17.9, S 4096 62 / 90, 74 / 92), or two, the heaviest of which the others wait
+// for: causal, n 512, S 512 28 / 24, S 1024 34.6 / 33.5, S 2048 50 / 55, S 4096 81 / 99; n 384, S 512 25 / 22, S 1024 30 / 31, S 2048 41 / 52.
+static bool fwd_paired(int64_t n, int Sk, bool causal) {
+  return n <= kNumCUs ? Sk >= (causal ? 256 : 512) : causal && n <= 2 * kNumCUs && Sk >= 1024;
 }
-// dQ's pairs against four waves (with dK / dV), causal: D 128, 64 blocks, S 4096 348 / 291, 128 blocks, S 8192 669 / 559, 256
-// blocks, S 1024 132 / 130, S 8192 725 / 632, S 16384 1395 / 1233, 512 blocks, S 2048 333 / 363, S 8192 1018 / 1017; D 64, 128 blocks
-// 430 / 370, 256 blocks 448 / 392. Not causal: D 128, 128 blocks, S 8192 689 / 602, 256 blocks, S 1024 173 / 199, S 8192 961 / 953.
-// dK / dV's (with dQ in pairs): causal, D 128, 64 blocks, S 4096 291 / 223, 128 blocks, S 8192 575 / 439, 256 blocks, S 1024 132 / 127,
-// S 8192 666 / 548, S 16384 1266 / 1042, 512 blocks, S 2048 335 / 367, S 8192 1017 / 1044; D 64, 128 blocks 376 / 295, 256 blocks
-// 420 / 347. Not causal: D 128, 128 blocks, S 8192 624 / 511, 256 blocks, S 1024 174 / 218, S 8192 969 / 990.
-static bool fa_paired(int64_t blocks128, bool causal) { return blocks128 <= (causal ? 2 : 1) * kNumCUs; }
+// dQ, eight waves against four (with dK / dV of four): causal, n 1024, S 512 144 / 139, S 1024 187 / 190, S 2048 283 / 287, S 4096 484 /
+// 499; n 2048, S 256 240 / 228, S 1024 406 / 394, S 2048 605 / 605, S 4096 1000 / 1031. Not causal, n 1024, S 512 179 / 176, S 1024 290 /
+// 292, S 2048 500 / 520, S 4096 896 / 943. Head dim 64: up to S 4096 four (n 2048, S 2048 324 / 303; not causal 553 / 542).
+static bool dq_wide(int D, int64_t n, int Sq, bool causal) {
+  return n >= (causal ? 2 * kNumCUs + 1 : 2 * kNumCUs) && Sq >= (D == 128 ? 2048 : 8192);
+}
+// Backward, pairs of both / of dK and dV / none: n 256, causal, S 256 42.9 / 40.0 / 41.7, S 512 54.5 / 53.9 / 59.3, S 1024 79 / 82 / 96,
+// S 4096 229 / 251 / 318; not causal, S 256 47 / 42 / 44, S 512 59 / 56 / 62, S 1024 86 / 86 / 99. n 512, causal, S 512 92 / 79 / 76,
+// S 1024 115 / 107 / 111, S 2048 169 / 167 / 188, S 4096 282 / 296 / 344. Head dim 64, n 256, S 256 26.2 / 27.1 / 28.2, n 512, S 512
+// 51 / 49 / 46, S 1024 67 / 69 / 71.
+static bool dq_paired(int D, int64_t n, int Sk, bool causal) {
+  return n <= kNumCUs ? Sk >= (D == 64 ? 256 : 512) : causal && n <= 2 * kNumCUs && Sk >= (D == 64 ? 1024 : 2048);
+}
+static bool dkdv_paired(int64_t n, int Sq, bool causal) {
+  return n <= kNumCUs ? Sq >= 256 : causal && n <= 2 * kNumCUs && Sq >= 1024;
+}
 // SXE_FA_FWD_WAVES = 4 / 8 / 16 (pairs) forces the forward's
 static bool fwd_dma() { return env_int("SXE_FA_FWD_DMA", 1) != 0; }
 
@@ -1375,7 +1385,7 @@ static std::vector<at::Tensor> fwd_impl_d(at::Tensor q, at::Tensor k, at::Tensor
   });
   // 8 waves share each staged K/V tile where that pays and the query axis allows; head dim 256 runs 4 (register budget)
   const int fww = env_int("SXE_FA_FWD_WAVES", 0);
-  const bool wide = D < 256 && Sq % 256 == 0 && (fww == 8 || (fww != 4 && (sp.layout || fwd_wide(D, (int64_t)B * H * Sq / 256, Sq, causal))));
+  const bool wide = D < 256 && Sq % 256 == 0 && (fww == 8 || (fww != 4 && (sp.layout || fwd_wide(D, (int64_t)B * H * Sq / fa::QB, Sq, causal))));
   const int grid = (Sq / fa::QB) * B * H;
   auto launch = [&](auto kern, int nwf) {
     hipLaunchKernelGGL(kern, dim3(nwf == 8 ? grid / 2 : grid), dim3(nwf * 64), lds, cur_stream(),
@@ -1395,7 +1405,7 @@ static std::vector<at::Tensor> fwd_impl_d(at::Tensor q, at::Tensor k, at::Tensor
         in_step = wide && (sp.layout || (!causal && (int64_t)B * H * Sq / 256 >= 2 * kNumCUs && fww == 0));
         if (in_step) sp.layout ? launch(fa::fwd_kernel<true, 8, D, true>, 8) : launch(fa::fwd_kernel<false, 8, D, true>, 8);
       }
-      const bool paired = !sp.layout && (fww == 0 ? !wide && fa_paired(grid, causal) : fww == 16);
+      const bool paired = !sp.layout && (fww == 0 ? !wide && fwd_paired(grid, Sk, causal) : fww == 16);
       if (in_step)
         ;
       else if (paired) {
@@ -1484,8 +1494,8 @@ static void bwd_impl_d(at::Tensor dout, at::Tensor q, at::Tensor k, at::Tensor v
   });
   // 8-wave dQ workgroups (SXE_FA_DQ_WAVES=4 / 8 forces)
   const int dqw = env_int("SXE_FA_DQ_WAVES", 0);
-  const bool dq8 = D < 256 && Sq % 256 == 0 && (dqw == 8 || (dqw == 0 && (sp.layout ? Sq >= 8192 : dq_wide(D, (int64_t)B * H * Sq / 256, Sq, causal))));
-  const bool dqp = D < 256 && !sp.layout && (dqw == 16 || (dqw == 0 && !dq8 && fa_paired(B * H * (int64_t)(Sq / fa::QB), causal)));
+  const bool dq8 = D < 256 && Sq % 256 == 0 && (dqw == 8 || (dqw == 0 && (sp.layout ? Sq >= 8192 : dq_wide(D, (int64_t)B * H * Sq / fa::QB, Sq, causal))));
+  const bool dqp = D < 256 && !sp.layout && (dqw == 16 || (dqw == 0 && !dq8 && dq_paired(D, B * H * (int64_t)(Sq / fa::QB), Sk, causal)));
   auto* dqk = sp.layout ? fa::dq_kernel<true, D> : fa::dq_kernel<false, D>;
   if constexpr (D < 256) {
     if (dq8) dqk = sp.layout ? fa::dq_kernel<true, D, 8> : fa::dq_kernel<false, D, 8>;
@@ -1565,7 +1575,7 @@ static void bwd_impl_d(at::Tensor dout, at::Tensor q, at::Tensor k, at::Tensor v
       }
     }
     if constexpr (D < 256) {
-      if (!sp.layout && (kvw == 16 || (kvw == 0 && fa_paired((int64_t)(Sk / fa::QB) * B * heads, causal)))) {
+      if (!sp.layout && (kvw == 16 || (kvw == 0 && dkdv_paired((int64_t)(Sk / fa::QB) * B * heads, Sq, causal)))) {
         const size_t lds = std::max<size_t>(G_::VBLK + 4 * G_::SLOT, 4 * D * 64 * sizeof(float));
         allow_lds<&fa::dkdv_kernel<SP, D, 3, 8, true>>((int)lds);
         launch(fa::dkdv_kernel<SP, D, 3, 8, true>, heads, 4, lds);
