@@ -370,6 +370,13 @@ def _sxe_wgrad_ok(gy2, x2, buf):
             and min(gy2.stride(-2), x2.stride(-2)) > 0 and max(M, N, K) < 1 << 30)
 
 
+def _wgrad_faster(T, M, N):
+    """us, the library with transposed copies or without / own, each call on another dW: 28672 x 4096, 128 tokens 200 / 196, 512 262 / 241;
+    128256 x 4096, 128 845 / 773, 2048 2298 / 2096, 8192 7361 / 6912; 57344 x 8192, 512 947 / 920, 2048 1898 / 1894; but few tokens of
+    large weights of rows 32 KB apart, 57344 x 8192, 128 754 / 832, 256 800 / 841, 16384 x 8192 224 / 240, 242 / 251."""
+    return T >= 512 or M * N < 1 << 27 or N % 8192 != 0
+
+
 def _tn_ok(gy2, x2):
     return (gy2.is_cuda and gy2.dtype == torch.bfloat16 and x2.dtype == torch.bfloat16 and TN_MIN_ELEMS > 0
             and gy2.shape[1] * x2.shape[1] >= TN_MIN_ELEMS and gy2.shape[0] % 64 == 0 and gy2.shape[1] % 64 == 0
@@ -478,7 +485,7 @@ def write_weight_grad(w, gy2, x2):
     if tgt is None:
         return False
     buf, accumulate = tgt(w)
-    if _sxe_wgrad_ok(gy2, x2, buf):
+    if _sxe_wgrad_ok(gy2, x2, buf) and _wgrad_faster(gy2.shape[0], gy2.shape[1], x2.shape[1]):
         torch.ops.sxe.wgrad_gemm_(gy2, x2, buf, 1.0, bool(accumulate))
     elif _tn_ok(gy2, x2) and buf.is_contiguous():
         a, b = torch.ops.sxe.transpose16(gy2), torch.ops.sxe.transpose16(x2).t()

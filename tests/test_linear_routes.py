@@ -241,3 +241,11 @@ def test_column_sum_rule(R, N, kernel):
         # fp32 sums of at most R / 128 + 14 steps a column (the general reduction has no more), and the rounding of the result
         assert got.dtype == dtype and ((got.double() - want).abs() <= (R / 128 + 14) * 2 ** -24 * size
                                        + (2 ** -8 if dtype == torch.bfloat16 else 0) * want.abs() + 1e-30).all()
+
+
+@pytest.mark.parametrize("T,M,N,own", [(256, 57344, 8192, False), (512, 57344, 8192, True), (128, 16384, 8192, False), (256, 8192, 8192, True),
+                                       (128, 128256, 4096, True), (64, 28672, 4096, True)])
+def test_weight_gradient_rule(T, M, N, own):
+    """Few tokens of the largest weights whose rows lie 32 KB apart are the library's."""
+    from shuffle_exchange_amd.ops.linear import _wgrad_faster
+    assert _wgrad_faster(T, M, N) == own
