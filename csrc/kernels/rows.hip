@@ -9,7 +9,8 @@
 //      logits_gather.cu:20; ``add`` folds the fused-residual sum x + res into the gather), and the
 //      random-LTD token gather (ops/random_ltd/gather_scatter.cu:22).
 //  * embedding_grad(gy [N, W], idx [N], rows) -> [rows, W]: the sum of the rows of gy that share an
-//      index, in their order and in fp32; rows that no index names are zeros.
+//      index, in fp32 and always in the same order (theirs, but that of many is 32 sums of every 32nd);
+//      rows that no index names are zeros.
 //  * scatter_rows_(dst [R, W], idx [N], src [N, W]): dst[idx[i]] = src[i] (indices unique):
 //      the random-LTD scatter back into the full sequence (gather_scatter.cu:72) and the backward of
 //      a unique-index gather.
@@ -150,10 +151,23 @@ __global__ void __launch_bounds__(256) run_sum_kernel(const typename dt_traits<T
   if (end < n && last < rows && sorted[end] == last && (p0 == 0 || sorted[p0 - 1] != last)) {
     float x[8] = {};
     for (int q0 = end; q0 < n && sorted[q0] == last; q0 += 256) {
+      // eight rows at once, those behind the run too: asked for one by one, each waits for its place in the order and then for itself
+      int row[8];
+      bool of[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        const int at = q0 + 32 * u + g;
-        if (in && at < n && sorted[at] == last) add_row(at, x);
+        const int at = q0 + 32 * u + g, near = min(at, n - 1);
+        row[u] = order[near];
+        of[u] = at < n && sorted[near] == last;
+      }
+      if (in) {
+        float y[8][8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) load8<T>(gy + (int64_t)row[u] * W + c, y[u]);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) x[j] = of[u] ? x[j] + y[u][j] : x[j];
       }
     }
     __syncthreads();
