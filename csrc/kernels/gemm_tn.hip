@@ -175,32 +175,44 @@ using T192 = Tile<2, 4, 6, 4, 2, 3, 2>;   // 192 x 256
 using T128 = Tile<2, 4, 4, 4, 3, 3, 2>;   // 128 x 256
 using N128 = Tile<2, 2, 4, 4, 2, 2, 2>;   // 128 x 128, two a CU
 
-// The tile and the splits of K that take least by this account: rounds of workgroups over the CUs, each a start (with the stores of a
-// round, which all its workgroups issue at once) and its slabs; a tile of the last, fewer rows takes 0.62 of a whole one's time and up.
-// us a slab and a start, fitted to 12 weights of 2048 x 2048 to 28672 x 4096 at 25 row counts from 40 to 14000: the choice is 1 %
-// behind the best on average. 256 x 128 and 192 x 128 were never the best.
+// The tile and the splits of K that take least by this account: rounds of workgroups over the CUs, each its slabs and a start (with the
+// stores of a round, which all its workgroups issue at once); the tiles of the last, fewer rows take 0.93 of a whole one's time and up,
+// and run on the CUs that the last round of whole ones leaves idle before they lengthen it. us a slab and a start, fitted to 32 weights
+// of 2048 x 2048 to 28672 x 4096 at 33 to 13000 rows with every tile and split (433 sizes): the choice is 0.6 % behind the best on
+// average, 12 % at the most; with the same rest tiles counted as running one after another on an idle CU it was 1.1 and 42 %
+// (1573 rows, 5120 x 5120, 107 us for 80). 256 x 128 and 192 x 128 were never the best.
 struct Form {
   int bm, bn, at_once;
   float slab, start;
 };
-constexpr Form kForms[4] = {{256, 256, 256, 1.42f, 9.f}, {192, 256, 256, 1.07f, 14.f}, {128, 256, 256, 0.95f, 3.f}, {128, 128, 512, 1.f, 3.f}};
+constexpr Form kForms[4] = {{256, 256, 256, 1.24f, 0.4f}, {192, 256, 256, 0.96f, 2.5f}, {128, 256, 256, 0.79f, 2.4f}, {128, 128, 512, 1.02f, 1.7f}};
+constexpr float kAlone = 0.87f;  // a slab's time of a tile of the last form that has a CU to itself
 struct Plan {
   int form, splits;
   float us;
 };
+// when `rest` tiles of `part` rounds each, on `slots` of which `idle` are free a round earlier, end behind `rounds` rounds
+static float end_of(int64_t rounds, int64_t idle, int64_t slots, int64_t rest, float part) {
+  if (rest == 0) return rounds;
+  // k tiles on each idle slot, the others joining in behind the last round; no slot takes more than k + 2 by then
+  for (int64_t k = std::max<int64_t>(1, rest / slots - 2);; ++k) {
+    const float idle_ends = rounds - 1 + k * part, others = std::max(0.f, idle_ends - rounds);
+    if (idle > 0 && idle * k + (slots - idle) * (int64_t)(others / part + 1e-5f) >= rest) return std::max<float>(rounds, idle_ends);
+    if (idle * (int64_t)((1 + k * part) / part + 1e-5f) + (slots - idle) * k >= rest) return rounds + k * part;
+  }
+}
 static Plan plan(int64_t M, int64_t N, int64_t slabs, bool may_split, int64_t batch) {
   Plan best{0, 1, 1e30f};
   for (int f = 0; f < 4; ++f) {
     const Form& t = kForms[f];
     const int64_t cols = (N + t.bn - 1) / t.bn * batch, rest = M % t.bm;
     for (int s : {1, 2, 3, 4, 6, 8}) {
-      if (s > 1 && (!may_split || slabs < 4 * s || (M + t.bm - 1) / t.bm * cols * s > 600)) break;
-      const float part = 0.62f + 0.38f * rest / t.bm, one = (slabs + s - 1) / s * t.slab + t.start;
+      const int64_t tiles = (M + t.bm - 1) / t.bm * cols * s;
+      if (s > 1 && (!may_split || slabs < 4 * s || tiles > 600)) break;
+      const float one = (slabs + s - 1) / s * t.slab * (f == 3 && tiles <= kNumCUs ? kAlone : 1.f) + t.start;
       const int64_t whole = M / t.bm * cols * s, rounds = (whole + t.at_once - 1) / t.at_once;
-      const float idle = rounds * t.at_once - whole, more = rest ? cols * s - idle / part : 0.f;
-      float us = 4.f + rounds * one;
-      if (more > 0.f) us += part * one * std::ceil(more / t.at_once);
-      if (s > 1) us += 4.f + M * N * 4 * (2 * s + 0.5f) / 3.2e6f;
+      float us = one * end_of(rounds, rounds * t.at_once - whole, t.at_once, rest ? cols * s : 0, 0.93f + 0.07f * rest / t.bm);
+      if (s > 1) us += 6.8f + M * N * 4 * (2 * s + 0.5f) / 6.9e6f;
       if (us < best.us) best = {f, s, us};
     }
   }
