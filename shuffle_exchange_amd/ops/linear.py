@@ -167,11 +167,15 @@ def _tiled(x, weight, bias):
     return torch.ops.sxe.gemm_tn(x2, weight, bias, False).view(*x.shape[:-1], weight.shape[0])
 
 
+def _own_products(x, weight, bias=None):
+    """Whether ``product`` may run own kernels: no graph is recorded, nobody follows the call by its operators."""
+    return (SKINNY_MAX_M > 0 and x.is_cuda and not torch.is_grad_enabled() and native.plain(x, weight, bias) and (x.dim() == 2 or x.is_contiguous())
+            and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == torch.bfloat16))
+
+
 def product(x, weight, bias=None):
     """``F.linear`` for the inside of autograd functions: no graph is built where it runs own kernels (``_tiled``)."""
-    if (weight.shape[0] >= 2048 <= weight.shape[-1] and SKINNY_MAX_M > 0 and x.is_cuda and not torch.is_grad_enabled()
-            and native.plain(x, weight, bias) and (x.dim() == 2 or x.is_contiguous())
-            and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == torch.bfloat16)):
+    if weight.shape[0] >= 2048 <= weight.shape[-1] and _own_products(x, weight, bias):
         y = _tiled(x, weight, bias)
         if y is not None:
             return y
@@ -386,12 +390,8 @@ def _tn_ok(gy2, x2):
 # Data-gradient GEMMs dX = dY W run in hipBLASLt's "NN" layout at 1.03-1.35 PF on MI355X; with W^T
 # materialised by the HBM-speed transpose they run in the forward layout at 1.25-1.56 PF
 # (tools/gemm_layout_bench.py, profiles/gemm_layout.log: net -0.03..-0.06 ms per Llama-3-8B layer
-# GEMM, -0.48 ms for the LM head, at 8192 tokens). The transpose reads/writes only the weight. Fewer rows pay for it where the
-# product sums over many columns and gemm_tn.hip takes it, us, NN / transpose and own product: 256 rows, 28672 x 4096 170 / 162,
-# 16384 x 3072 93 / 71, 1000 rows 372 / 286, 176 / 128, 32000 x 4096 402 / 320, 16384 x 2048 112 / 89; but 1371 rows of 28672 x 4096
-# 310 / 358; 4096 x 14336, 1000 rows 97 / 130.
+# GEMM, -0.48 ms for the LM head, at 8192 tokens). The transpose reads/writes only the weight.
 DGRAD_WT_MIN_ELEMS = int(os.environ.get("SXE_DGRAD_WT_MIN_ELEMS", 16 * 2**20))
-DGRAD_WT_LONG = 16384
 
 
 # The transposed weights are constant between optimizer steps: with gradient accumulation each
@@ -413,6 +413,7 @@ def invalidate_transposed_weights():
 
 
 def _transpose16(t):
+    native.require_hip()
     return torch.ops.sxe.transpose16(t)
 
 
@@ -455,13 +456,23 @@ def configure_transposed_weight_cache(enabled, free_bytes=None):
     return cap
 
 
+def _wt_few_faster(rows, N, K):
+    """Whether fewer than 2048 rows pay for the transpose of w [N, K], too: where the product sums over many columns and gemm_tn.hip takes
+    it. us, NN / transpose and own product: 256 rows, 28672 x 4096 206 / 171, 16384 x 2048 81 / 60, 1000 rows 350 / 268, 141 / 95, 32000 x
+    3072 314 / 261; 1819 rows, 16384 x 2048 1.18, 1808, 32000 x 3072 1.49; but 1962 rows, 28672 x 3072 0.82; 1371 rows, 28672 x 4096
+    308 / 338; 512 rows, 16384 x 4096 0.94, 57344 x 4096, 640 rows 0.74, 16384 x 8192 0.70, 400 rows, 128256 x 4096 829 / 1022."""
+    if not 256 <= rows <= 1900 or not 16384 <= N <= 49152 or not _tiled_faster(rows, K, N):
+        return False
+    return K <= 3072 or (K <= 5120 and N >= 20480 and rows <= 1280)
+
+
 def data_grad(gy, w):
     """dX = gy @ w for w [N, K] (gy [..., N])."""
     if (DGRAD_WT_MIN_ELEMS > 0 and gy.is_cuda and gy.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and w.dim() == 2 and w.is_contiguous() and w.numel() >= DGRAD_WT_MIN_ELEMS and w.shape[0] % 64 == 0
             and w.shape[1] % 64 == 0):
         rows = gy.numel() // gy.shape[-1]
-        if rows >= 2048 or (rows >= 256 and w.shape[0] >= DGRAD_WT_LONG and _tiled_faster(rows, w.shape[1], w.shape[0])):
+        if rows >= 2048 or (_wt_few_faster(rows, *w.shape) and gy.is_contiguous() and gy.data_ptr() % 16 == 0 and _own_products(gy, w)):
             return product(gy, _transposed_weight(w))
     return torch.matmul(gy, w)
 

@@ -249,3 +249,38 @@ def test_weight_gradient_rule(T, M, N, own):
     """Few tokens of the largest weights whose rows lie 32 KB apart are the library's."""
     from shuffle_exchange_amd.ops.linear import _wgrad_faster
     assert _wgrad_faster(T, M, N) == own
+
+
+@pytest.mark.parametrize("rows,N,K,own", [(255, 28672, 4096, False), (256, 28672, 4096, True), (1280, 28672, 4096, True), (1371, 28672, 4096, False),
+                                          (1819, 16384, 2048, True), (1962, 28672, 3072, False), (512, 16384, 4096, False), (256, 57344, 8192, False),
+                                          (400, 128256, 4096, False), (640, 57344, 4096, False), (1000, 27648, 5120, True), (1792, 16384, 2048, False)])
+def test_transposed_weight_rule(rows, N, K, own):
+    from shuffle_exchange_amd.ops.linear import _wt_few_faster
+    assert _wt_few_faster(rows, N, K) == own
+
+
+@gpu
+def test_data_gradient_of_few_rows(monkeypatch):
+    """The weight is transposed only for the own product: not where a graph is recorded (the transpose has no derivative), nor where the
+    library's products are asked for."""
+    from shuffle_exchange_amd.ops import linear as L, native
+    native.require_hip()
+    g = torch.Generator("cuda").manual_seed(2)
+    w = (torch.randn(16384, 2048, generator=g, device="cuda") / 128).bfloat16()
+    gy = torch.randn(300, 16384, generator=g, device="cuda").bfloat16()
+    seen = []
+    transposed = L._transposed_weight
+    monkeypatch.setattr(L, "_transposed_weight", lambda t: seen.append(1) or transposed(t))
+    want = gy.double() @ w.double()
+    with torch.no_grad():
+        dx = L.data_grad(gy, w)
+        assert seen == [1] and (dx.double() - want).norm() <= 6e-3 * want.norm()
+        assert torch.equal(L.data_grad(F.pad(gy, (0, 4))[:, :16384], w), gy @ w) and seen == [1]  # rows off 16 bytes
+    wg = w.clone().requires_grad_()
+    with torch.enable_grad():
+        dx = L.data_grad(gy, wg)
+        dw, = torch.autograd.grad(dx, wg, torch.ones_like(dx))
+    assert seen == [1] and (dw.double() - (gy.double().t() @ torch.ones_like(dx).double())).norm() <= 6e-3 * dw.double().norm()
+    monkeypatch.setattr(L, "SKINNY_MAX_M", 0)
+    with torch.no_grad():
+        assert torch.equal(L.data_grad(gy, w), gy @ w) and seen == [1]
