@@ -126,13 +126,16 @@ def glu_linear(x, weight):
     return torch.ops.sxe.stream_gemm(x, w, sc, None, True)
 
 
-# Many rows: csrc/kernels/gemm_tn.hip, 2048 x 2048 to 28672 x 4096, us, library / here. The library's kernels fit whole tiles of 256 rows
-# (8192 rows, 28672 x 4096 1255 / 1285, 4096 x 4096 174 / 184, 4096 x 14336 604 / 630) and fall off at others: 4500 rows, 4096 x 14336
-# 759 / 417, 7300 rows 962 / 596, 5120 x 3072 239 / 191, 9000 rows, 4096 x 4096 338 / 220; at their best 6500 rows, 6144 x 4096 241 / 253,
-# 13000 rows, 3072 x 8192 454 / 504: 5 % less time on average from 1500 rows on. Below, long rows of the weight pay, whose products
-# are split along them: 40 rows, 2048 x 8192 23 / 17, 4096 x 14336 33 / 32, 240 rows 55 / 42, 1100 rows 141 / 114; others do not:
-# 600 rows, 5120 x 3072 26 / 29, 4096 x 4096 28 / 31.
-TILED_ROWS = 1500
+# Many rows: csrc/kernels/gemm_tn.hip, us, library / here. The library's kernels fit whole tiles of 256 rows (8192 rows, 28672 x 4096
+# 1255 / 1285, 4096 x 4096 174 / 184) and many other counts, but by far not all: 6695 rows, 5120 x 5120 1.59 times as long, 7584, 4096 x 14336
+# 1.68, 2716, 6144 x 4096 1.69, 8810, 4096 x 4096 1.57, 2588, 16384 x 3072 1.52; where it fits it is up to 10 % ahead (3072 x 3072, 1630 rows
+# 39 / 44; 32000 x 4096, 4000 rows 0.94). From 1500 to 13000 rows the library takes 1.085 times as long on average (17 weights of 2048 x
+# 2048 to 32000 x 4096, 14 counts each); further on 1.03 at equal weights, 1.01 to 1.02 in all, and more than 2 % less for every third count
+# (3072 x 8192, 19089 rows 666 / 736).
+# Fewer rows, long rows of the weight, whose products are split along them: 1.5 times on average, 40 rows, 8192 x 28672 127 / 88, 4096 x 14336
+# 33 / 32, 200 rows 55 / 40, 1100 rows, 3072 x 8192 70 / 64; but up to 128 rows (few workgroups, or rows 32 KB apart) 64 rows, 8192 x 8192 33 / 39,
+# 128 rows, 2048 x 8192 21 / 25, 33 rows, 2048 x 16384 0.74; others do not: 600 rows, 5120 x 3072 26 / 29, 4096 x 4096 28 / 31.
+TILED_ROWS, TILED_ROWS_MOST = 1500, 13000
 # SwiGLU of the products in one launch, us, product and activation / here: 16384 x 2048, 330 rows 35 / 29, 2100 rows 144 / 112;
 # 28672 x 4096, 330 rows 85 / 73, 1040 rows 226 / 200, 7588 rows 1390 / 1250; but 240 rows of 16384 x 3072 38 / 43, 72 of 28672 x 4096
 # 59 / 67
@@ -142,7 +145,11 @@ TILED_GLU_ROWS = 300
 def _tiled_faster(rows, N, K):
     if N < 2048 or K < 2048:
         return False
-    return rows % 256 != 0 if rows >= TILED_ROWS else STREAM_ROWS_SMALL < rows and K >= 8192 and N <= K
+    if rows >= TILED_ROWS:
+        return rows < TILED_ROWS_MOST and rows % 256 != 0
+    if rows <= 128 and (N >= K or K % 16384 == 0 or (rows > 64 and N < 3072)):
+        return False
+    return STREAM_ROWS_SMALL < rows and K >= 8192 and N <= K
 
 
 def _tileable(x2, weight, bias=None):
@@ -175,7 +182,7 @@ def _own_products(x, weight, bias=None):
 
 def product(x, weight, bias=None):
     """``F.linear`` for the inside of autograd functions: no graph is built where it runs own kernels (``_tiled``)."""
-    if weight.shape[0] >= 2048 <= weight.shape[-1] and _own_products(x, weight, bias):
+    if weight.dim() == 2 and _tiled_faster(x.numel() // max(1, x.shape[-1]), *weight.shape) and _own_products(x, weight, bias):
         y = _tiled(x, weight, bias)
         if y is not None:
             return y
@@ -599,8 +606,10 @@ def linear(x, weight, bias=None):
     if grad and weight.requires_grad and hasattr(weight, "_sxe_grad_target"):
         return _Linear.apply(x, weight, bias)
     if not grad and SKINNY_MAX_M > 0 and x.is_cuda:
-        few = x.numel() <= max(SKINNY_MAX_M, STREAM_ROWS_SMALL) * x.shape[-1]
-        if ((few or weight.shape[0] >= 2048 <= weight.shape[-1])
+        n, K = x.numel(), x.shape[-1]
+        few = n <= max(SKINNY_MAX_M, STREAM_ROWS_SMALL) * K
+        # the sizes first: a call that stays with the library is host-bound at a few hundred rows, and what follows is 2 us
+        if ((few or (weight.dim() == 2 and _tiled_faster(n // K, *weight.shape)))
                 and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == torch.bfloat16)
                 and native.plain(x, weight, bias)):
             if few:

@@ -251,6 +251,15 @@ def test_weight_gradient_rule(T, M, N, own):
     assert _wgrad_faster(T, M, N) == own
 
 
+@pytest.mark.parametrize("rows,N,K,own", [(1499, 4096, 4096, False), (1501, 4096, 4096, True), (1536, 4096, 4096, False), (12999, 3072, 8192, True),
+                                          (13001, 3072, 8192, False), (31000, 4096, 4096, False), (600, 4096, 14336, True), (33, 8192, 8192, False),
+                                          (200, 8192, 8192, True), (33, 2048, 8192, True), (100, 2048, 8192, False), (64, 6144, 16384, False),
+                                          (200, 6144, 16384, True), (100, 8192, 28672, True), (600, 2040, 8192, False)])
+def test_many_row_rule(rows, N, K, own):
+    from shuffle_exchange_amd.ops.linear import _tiled_faster
+    assert _tiled_faster(rows, N, K) == own
+
+
 @pytest.mark.parametrize("rows,N,K,own", [(255, 28672, 4096, False), (256, 28672, 4096, True), (1280, 28672, 4096, True), (1371, 28672, 4096, False),
                                           (1819, 16384, 2048, True), (1962, 28672, 3072, False), (512, 16384, 4096, False), (256, 57344, 8192, False),
                                           (400, 128256, 4096, False), (640, 57344, 4096, False), (1000, 27648, 5120, True), (1792, 16384, 2048, False)])
