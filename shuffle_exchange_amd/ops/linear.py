@@ -138,8 +138,8 @@ def glu_linear(x, weight):
 TILED_ROWS, TILED_ROWS_MOST = 1500, 13000
 # SwiGLU of the products in one launch, us, product and activation / here: 16384 x 2048, 330 rows 35 / 29, 2100 rows 144 / 112;
 # 28672 x 4096, 330 rows 85 / 73, 1040 rows 226 / 200, 7588 rows 1390 / 1250; but 240 rows of 16384 x 3072 38 / 43, 72 of 28672 x 4096
-# 59 / 67
-TILED_GLU_ROWS = 300
+# 59 / 67, and of weights beyond 2^28 elements 493 rows, 57344 x 8192 0.90, 1423 rows 1.02, 3000 rows 1.12
+TILED_GLU_ROWS, TILED_GLU_ROWS_LARGE = 300, 1024
 
 
 def _tiled_faster(rows, N, K):
@@ -194,7 +194,7 @@ def glu_tiled(x, weight):
     where the product and the activation's launch are the better or only form. One rounding, of the result."""
     if (not isinstance(weight, torch.Tensor) or weight.dim() != 2 or x.dim() != 2 or not x.is_cuda or x.requires_grad or not native.plain(x, weight)
             or x.shape[0] <= TILED_GLU_ROWS or weight.shape[0] < 8192 or weight.shape[1] < 2048 or not _tileable(x, weight)
-            or torch.is_autocast_enabled("cuda")):
+            or (weight.numel() > 1 << 28 and x.shape[0] <= TILED_GLU_ROWS_LARGE) or SKINNY_MAX_M <= 0 or torch.is_autocast_enabled("cuda")):
         return None
     native.require_hip()
     return torch.ops.sxe.gemm_tn(x, weight, None, True)

@@ -293,3 +293,17 @@ def test_data_gradient_of_few_rows(monkeypatch):
     monkeypatch.setattr(L, "SKINNY_MAX_M", 0)
     with torch.no_grad():
         assert torch.equal(L.data_grad(gy, w), gy @ w) and seen == [1]
+
+
+@gpu
+def test_glu_rule_and_switch(monkeypatch):
+    """SwiGLU of many rows in the product's launch, not of few rows of the largest weights, nor where the library's products are asked for."""
+    from shuffle_exchange_amd.ops import linear as L
+    w = torch.zeros(8192, 2048, device="cuda", dtype=torch.bfloat16)
+    x = torch.zeros(301, 2048, device="cuda", dtype=torch.bfloat16)
+    large = torch.empty(1, 8192, device="cuda", dtype=torch.bfloat16).expand(32776, 8192)  # never read
+    xl = torch.zeros(1024, 8192, device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        assert L.glu_tiled(x, w) is not None and L.glu_tiled(x[:300], w) is None and L.glu_tiled(xl, large) is None
+        monkeypatch.setattr(L, "SKINNY_MAX_M", 0)
+        assert L.glu_tiled(x, w) is None
