@@ -52,35 +52,46 @@ def cross_entropy(logits, target, ignore_index=-100, reduction="mean"):
     return per_tok.sum() / n
 
 
+def _column_states(h):
+    """[tokens, K] of the hidden states, rounded up to 64 tokens by zeros, whole 16-byte vectors."""
+    h2 = h.reshape(-1, h.shape[-1])
+    if h2.shape[0] % 64:
+        h2 = F.pad(h2, (0, 0, 0, -h2.shape[0] % 64))
+    h2 = h2.contiguous()
+    return h2.clone() if h2.data_ptr() % 16 else h2  # a view that starts inside a vector
+
+
 class _ColumnHeadXEnt(torch.autograd.Function):
     """LM head and loss over logits with a token per column (``xent_cols_fwd``): the logits, the data gradient and the weight gradient
-    are products of whole 16-byte vectors although a row of logits is not. The tokens are rounded up by rows of zeros."""
+    are products of whole 16-byte vectors although a row of logits is not."""
 
     @staticmethod
     def forward(ctx, h, weight, target, ignore_index):
-        h2 = h.reshape(-1, h.shape[-1])
         tgt = target.reshape(-1).contiguous()
-        if h2.shape[0] % 64:
-            h2 = F.pad(h2, (0, 0, 0, -h2.shape[0] % 64))
-        h2 = h2.contiguous()
-        if h2.data_ptr() % 16:  # a view that starts inside a vector
-            h2 = h2.clone()
-        logits = torch.ops.sxe.gemm_tn(weight, h2, None, False)
+        logits = torch.ops.sxe.gemm_tn(weight, _column_states(h), None, False)
         loss, lse = torch.ops.sxe.xent_cols_fwd(logits, tgt, int(ignore_index))
-        ctx.save_for_backward(logits, lse, tgt, h2, weight)
-        ctx.ignore_index, ctx.hshape = int(ignore_index), h.shape
+        ctx.save_for_backward(logits, lse, tgt, h, weight)
+        ctx.ignore_index = int(ignore_index)
         return loss.view(target.shape)
 
     @staticmethod
     def backward(ctx, dloss):
-        logits, lse, tgt, h2, weight = ctx.saved_tensors
-        g = torch.ops.sxe.xent_cols_bwd(logits, tgt, lse, dloss.reshape(-1).float().contiguous(), ctx.ignore_index)
+        logits, lse, tgt, h, weight = ctx.saved_tensors
+        g = torch.ops.sxe.xent_cols_bwd(logits, tgt, lse, dloss.detach().reshape(-1).float().contiguous(), ctx.ignore_index)
         del logits
         dh = dw = None
+        if torch.is_grad_enabled():  # derivatives of these products may be asked for, which the kernels below do not have
+            g = g[:, :tgt.numel()]
+            if ctx.needs_input_grad[0]:
+                dh = (g.t() @ weight).view(h.shape)
+            if ctx.needs_input_grad[1]:
+                dw = g @ h.reshape(-1, h.shape[-1])
+            return dh, dw, None, None
+        h2 = _column_states(h)
         if ctx.needs_input_grad[0]:  # contracts the vocabulary: the form of a weight gradient, in fp32 parts
             dh = torch.empty(h2.shape, device=h2.device, dtype=torch.float32)
             torch.ops.sxe.wgrad_gemm_(g, weight, dh, 1.0, False)
-            dh = dh[:tgt.numel()].to(h2.dtype).view(ctx.hshape)
+            dh = dh[:tgt.numel()].to(h2.dtype).view(h.shape)
         if ctx.needs_input_grad[1]:
             dw = torch.ops.sxe.gemm_tn(g, torch.ops.sxe.transpose16(h2), None, False)
         return dh, dw, None, None

@@ -88,6 +88,26 @@ def test_column_head_of_unaligned_states(tokens):
     assert all(torch.equal(a, b) for a, b in zip(*got))
 
 
+@pytest.mark.parametrize("tokens", [64, 70])
+def test_column_head_gradients_of_gradients(tokens):
+    """What a recorded backward gives, and its derivatives with respect to the head's two operands (the softmax's own derivative is not
+    among them, as over a token per row): as the product and the row form give them, up to the roundings of logits and gradients
+    (see above: 2^-6 of the norm)."""
+    from shuffle_exchange_amd.ops.cross_entropy import cross_entropy, head_cross_entropy, _columns_ok
+    g = torch.Generator("cuda").manual_seed(tokens)
+    h = torch.randn(1, tokens, 64, generator=g, device="cuda").bfloat16().requires_grad_()
+    w = torch.randn(1001, 64, generator=g, device="cuda").mul_(0.125).bfloat16().requires_grad_()
+    tgt = torch.randint(0, 1001, (1, tokens), generator=g, device="cuda")
+    vh, vw = torch.randn_like(h), torch.randn_like(w)
+    assert _columns_ok(h, w, tgt)
+    got = []
+    for loss in (head_cross_entropy(h, w, tgt), cross_entropy(torch.nn.functional.linear(h, w), tgt)):
+        dh, dw = torch.autograd.grad(loss, (h, w), create_graph=True)
+        got.append((dh.detach(), dw.detach(), torch.autograd.grad(dh, w, vh, retain_graph=True)[0], torch.autograd.grad(dw, h, vw)[0]))
+    for a, b in zip(*got):
+        assert (a.double() - b.double()).norm() <= 2 ** -6 * b.double().norm()
+
+
 def test_column_head_masked_vocabulary():
     """Rows of -inf logits (a hidden state of infinities) and a share with nothing else: NaN and zeros where the row form has them."""
     x = torch.randn(200, 64, device="cuda").bfloat16()
