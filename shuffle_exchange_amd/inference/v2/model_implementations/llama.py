@@ -31,7 +31,7 @@ import torch.nn.functional as F
 
 from ....ops import native
 from ....ops.activation import swiglu
-from ....ops.linear import Linear, glu_faster, glu_linear, glu_tiled, is_own_forward, linear
+from ....ops.linear import Linear, STREAM_ROWS_SMALL, TILED_GLU_ROWS, glu_faster, glu_linear, glu_tiled, is_own_forward, linear
 from ....ops.norm import RMSNorm
 from ....ops.paged_attention import paged_attention_parts, paged_batch_attention, ragged_attention, rope_kv_cache_append
 from ....ops.rows import gather_last
@@ -252,7 +252,8 @@ class RaggedLlama:
         many tokens, the norm in its prologue up to 4."""
         mlp, norm, T = layer.mlp, layer.post_attention_layernorm, x.shape[0]
         w = None
-        if (self.tps is None and (T > self.FUSE_MAX_T or self._fusable(T)) and self.device.type == "cuda"
+        few = T <= STREAM_ROWS_SMALL  # between these and the many rows there is no such product: host-bound passes, and asking is 10 us a layer
+        if (self.tps is None and (few or T > TILED_GLU_ROWS) and (T > self.FUSE_MAX_T or self._fusable(T)) and self.device.type == "cuda"
                 and getattr(mlp.gate_up_proj, "bias", None) is None and native.hip_available()):
             w = self._wobj(mlp.gate_up_proj, li, "gu")
             if T > 16 and self.qw is not None:  # quantized layers run more than 16 rows on the weight as it came
@@ -264,7 +265,7 @@ class RaggedLlama:
                 return r
         a, h = norm(x, res)
         if w is not None:
-            mid = (glu_linear(a, w) if glu_faster(T, w) else None) if T <= 32 else glu_tiled(a, w)
+            mid = (glu_linear(a, w) if glu_faster(T, w) else None) if few else glu_tiled(a, w)
             if mid is not None:
                 return mid, h
         return swiglu(self._proj(mlp.gate_up_proj, a, li, "gu")), h

@@ -678,6 +678,13 @@ EMBED_GRAD_IDS = 16384  # indices up to which ranking them by comparison is the 
 class Embedding(torch.nn.Embedding):
     """``nn.Embedding`` with the constructor-time N(0, init_std) init of ``Linear`` and, on the GPU, a gradient of its own."""
 
+    def __init__(self, num_embeddings, embedding_dim, init_std=None, **kw):
+        super().__init__(num_embeddings, embedding_dim, **kw)
+        if init_std is not None:
+            with torch.no_grad():
+                self.weight.normal_(0.0, init_std)
+            self._sxe_inited = True
+
     def forward(self, input):
         w = self.weight
         if (w.is_cuda and torch.is_grad_enabled() and w.requires_grad and self.padding_idx is None and self.max_norm is None
@@ -686,10 +693,3 @@ class Embedding(torch.nn.Embedding):
                 and input.device == w.device and input.dtype in (torch.int64, torch.int32) and native.use_hip(w) and native.plain(w, input)):
             return _Embed.apply(input, w)
         return super().forward(input)
-
-    def __init__(self, num_embeddings, embedding_dim, init_std=None, **kw):
-        super().__init__(num_embeddings, embedding_dim, **kw)
-        if init_std is not None:
-            with torch.no_grad():
-                self.weight.normal_(0.0, init_std)
-            self._sxe_inited = True

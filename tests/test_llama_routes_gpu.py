@@ -52,6 +52,19 @@ def test_gate_up_routes(tokens, quant, monkeypatch):
     assert _rel(got, want) < 2e-2
 
 
+def test_gate_up_of_a_short_prompt_asks_for_no_launch(monkeypatch):
+    """Between the few and the many rows nothing takes gate, up and the activation in one launch, and a pass is bound by its host."""
+    from shuffle_exchange_amd.inference.v2.model_implementations import llama
+    seen = []
+    for name in ("glu_tiled", "glu_linear", "glu_faster"):
+        monkeypatch.setattr(llama, name, lambda *a: seen.append(1))
+    engine = _engine(_model())
+    for uid, (tokens, asked) in enumerate([(33, False), (300, False), (301, True)]):
+        seen.clear()
+        engine.put([uid], [list(range(tokens))])
+        assert bool(seen) == asked, tokens
+
+
 @pytest.mark.parametrize("tokens", [2, 8, 40])
 @pytest.mark.parametrize("which", ["qkv_proj", "o_proj", "gate_up_proj", "down_proj"])
 def test_lora_modules(tokens, which):
