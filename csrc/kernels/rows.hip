@@ -80,9 +80,9 @@ __global__ void __launch_bounds__(256) scatter_kernel(u32x4* __restrict__ dst, c
 // other one is a radix sort of some ten launches. Here the tokens are ranked by (index, position) by
 // counting -- every wave of a block compares 64 tokens with a part of the others, N^2 compares in all,
 // which is why the caller stops at 16384 of them -- and a block then sums 64 columns of 32 ranks:
-// 2048 tokens of 768 into 50257 rows 24 us, of which the zeros of the result are 12; 4096 wide into
-// 32000 rows, us, the library / this: 512 tokens 75 / 42, 2048 182 / 59, 8192 328 / 121, 16384 598 / 212
-// (zeros 33); half of the tokens the same: 2048 211 / 102, 16384 605 / 566.
+// 2048 tokens of 768 into 50257 rows 27 us, of which the zeros of the result are 12; 4096 wide into
+// 32000 rows, us, the library / this: 512 tokens 74 / 42, 2048 180 / 59, 8192 329 / 121, 16384 600 / 214
+// (zeros 33); half of the tokens the same: 2048 190 / 87, 16384 625 / 302; all 16384 in two rows 364 / 224.
 constexpr int RANK_TILE = 8192;
 template <typename I>
 __global__ void __launch_bounds__(1024) rank_kernel(const I* __restrict__ idx, int n, int rows, int* __restrict__ order,
@@ -151,23 +151,25 @@ __global__ void __launch_bounds__(256) run_sum_kernel(const typename dt_traits<T
   if (end < n && last < rows && sorted[end] == last && (p0 == 0 || sorted[p0 - 1] != last)) {
     float x[8] = {};
     for (int q0 = end; q0 < n && sorted[q0] == last; q0 += 256) {
-      // eight rows at once, those behind the run too: asked for one by one, each waits for its place in the order and then for itself
-      int row[8];
-      bool of[8];
+      // All of the next 256 ranks: four places, then four rows at once (eight cost the kernel a quarter of its waves). One by one, each waits
+      // for its place and then for itself; but so the last ranks of a run, as rows that are not of it cost as much as its own.
+      if (in && q0 + 255 < n && sorted[q0 + 255] == last) {
+#pragma unroll 1
+        for (int u0 = 0; u0 < 8; u0 += 4) {
+          float y[4][8];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) load8<T>(gy + (int64_t)order[q0 + 32 * (u0 + u) + g] * W + c, y[u]);
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x[j] += y[u][j];
+        }
+        continue;
+      }
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        const int at = q0 + 32 * u + g, near = min(at, n - 1);
-        row[u] = order[near];
-        of[u] = at < n && sorted[near] == last;
-      }
-      if (in) {
-        float y[8][8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) load8<T>(gy + (int64_t)row[u] * W + c, y[u]);
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-#pragma unroll
-          for (int j = 0; j < 8; ++j) x[j] = of[u] ? x[j] + y[u][j] : x[j];
+        const int at = q0 + 32 * u + g;
+        if (in && at < n && sorted[at] == last) add_row(at, x);
       }
     }
     __syncthreads();
