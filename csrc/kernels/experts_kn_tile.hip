@@ -12,7 +12,8 @@
 // x 64 columns (32 + 32). x rows are gathered on the way and read from LDS as they lie, slabs of 64 k rows of W transposed
 // (ds_read_b64_tr_b16). The row tiles of an expert and column block run side by side on one XCD, so W comes from memory once. Blocks
 // of 16 rows past the expert's rows run no products. us, before (32-k slabs, products of 32 x 32 x 16, ring of five) / here: 8 experts of
-// 2048 rows, 4096 x 2 x 14336 3620 / 2991, 14336 x 4096 1911 / 1611 (1.29 PFLOP/s); of 800 rows 1628 / 1358, 785 / 661.
+// 2048 rows, 4096 x 2 x 14336 3620 / 2991, 14336 x 4096 1911 / 1611 (1.29 PFLOP/s); of 800 rows 1628 / 1358, 785 / 661. SwiGLU to 32 bits
+// (gl::silu) has since added 1 - 2 % to the products with gate and up: of 800 rows, on one card, 1287 -> 1307.
 #include "sxe_common.h"
 #include "sxe_gemm_loop.h"
 #include <torch/library.h>

@@ -5,9 +5,9 @@
 // library runs it with an fp32 C at 0.8 - 1.1 PFLOP/s, and with few tokens (626 of each of 8 experts, 3072 x 16384) at 0.48. Here both
 // operands stream through LDS as they lie and are read transposed (ds_read_b64_tr_b16): no operand needs a transposed copy.
 //
-// us, the library with fp32 C / the kernel that was here (32 x 32 x 16 products, slabs of 16, whole tiles and 128 tokens only) / here:
-// 28672 x 4096, 8192 tokens 1684 / 1579 / 1481, 2777 tokens 633 / - / 528; 4096 x 4096, 8192 tokens 252 / 221 / 197; 2048 x 2048, 4096 tokens
-// 46 / 85 / 43; 8 experts of 1280 tokens, 4096 x 28672 2696 / 2460 / 2347, of 626, 8192 x 3072 500 / - / 330.
+// us, the library with fp32 C, with transposed copies or without / here, each call on another C: 28672 x 4096, 8192 tokens 1603 / 1520,
+// 2048 513 / 466, 256 221 / 209; 4096 x 4096, 8192 tokens 253 / 215, 512 47 / 40; 128256 x 4096, 4096 tokens 3846 / 3644; 2048 x 2048, 4096 tokens
+// 49 / 48; 8 experts of 256 tokens, 4096 x 28672 1890 / 1517.
 //
 // What bounds it: as in gemm_tn.hip, whose loop this is (sxe_gemm_loop.h), plus C, 128 MB of fp32 in a round of workgroups. A tile is
 // 256 x 256 (128 x 256 or splits of the tokens where a plan of rounds finds them shorter), slabs of 64 tokens, rows of 256 or 128

@@ -91,8 +91,9 @@ class GroupedSwiGLUExperts(nn.Module):
 def expert_products(x, w, transposed=False):
     """x[e] @ w[e] (``transposed``: x[e] @ w[e]^T) of all experts, bf16 x [E, C, .], w [E, K, N], in one launch (csrc/kernels/experts_kn_tile.hip,
     gemm_tn.hip); None where these do not cover the operands. A library product per expert fills the card only with the rows of one:
-    8 experts, 4096 x 28672, us, 320 rows each 670 / 713 here, 1280 rows 2151 / 1767, transposed 2393 / 578, 3268 / 2007; 14336 x 4096,
-    1110 / 333, 1372 / 908, transposed 434 / 382, 1100 / 825; 2048 x 16384, 1280 rows 657 / 552, transposed 980 / 571."""
+    8 experts, 4096 x 28672, us, 320 rows each 753 / 749 here, 1280 rows 2273 / 1776, transposed 2438 / 508, 3289 / 2012; 14336 x 4096,
+    1164 / 330, 1455 / 936, transposed 443 / 385, 1174 / 847; 2048 x 16384, 1280 rows 695 / 548, transposed 987 / 563. Of 4 to 2560 rows
+    each nothing was more than 4 % slower but 4 rows transposed of 3072 x 16384 (0.91)."""
     if not (x.is_cuda and w.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 3 and w.dim() == 3
             and native.plain(x, w)):
         return None

@@ -20,11 +20,10 @@ import torch.nn.functional as F
 
 from . import native
 
-# Large weight-gradient GEMMs (MLP projections, LM head) run faster as two HBM-speed transposes +
-# a forward-layout ("TN") bf16 GEMM + an fp32 accumulate than as one fp32-output GEMM in the
-# token-major "NT" layout: hipBLASLt reaches 1.47-1.61 PF in TN vs 1.06-1.19 PF in NT on MI355X
-# (tools/wgrad_layout_exp.py, tools/wgrad_tn_exp.py: -0.13 ms per 28672x4096 / 4096x14336 call,
-# -0.47 ms for the 128256x4096 LM head, at K = 8192 tokens). Smaller weights keep the fused path.
+# Large weight gradients that gemm_wgrad.hip does not take (bf16 reduce-scatter slots, few tokens of the largest weights, SXE_WGRAD=0) run
+# faster as two HBM-speed transposes + a forward-layout ("TN") GEMM than in the token-major "NT" layout: hipBLASLt reaches
+# 1.47-1.61 PF in TN vs 1.06-1.19 PF in NT on MI355X (tools/wgrad_layout_exp.py, tools/wgrad_tn_exp.py: -0.13 ms per 28672x4096 /
+# 4096x14336 call, -0.47 ms for the 128256x4096 LM head, at K = 8192 tokens).
 TN_MIN_ELEMS = int(os.environ.get("SXE_WGRAD_TN_MIN_ELEMS", 32 * 2**20))
 # TN weight gradient into an fp32 accumulator: one fp32-output GEMM with beta = 1 (hipBLASLt "BSS"
 # kernels), or (SXE_WGRAD_TN_FP32OUT=0) the bf16-output TN GEMM -- the faster kernel family -- plus
@@ -362,8 +361,9 @@ def fused_gatenorm_linear(x, norm_weight, gate, eps, weight):
 
 
 # Hand-written weight-gradient GEMM (csrc/kernels/gemm_wgrad.hip: both operands read transposed through LDS, fp32 C): no transposed
-# copies of dY / X, any number of tokens. Beside the library's fp32-output product it is the faster one at every size measured, 2048 x
-# 2048 to 32000 x 3072, 300 - 8192 tokens (figures there).
+# copies of dY / X, any number of tokens. Beside the library's fp32-output product, with transposed copies or without, it is the faster one
+# from 768 x 768 to 128256 x 4096 at 128 - 16384 tokens (figures there), but for 1024 and 2048 tokens of 2048 x 2048 (24 us for 22, 34 for
+# 31) and what ``_wgrad_faster`` leaves out.
 SXE_WGRAD = os.environ.get("SXE_WGRAD", "1") == "1"
 
 

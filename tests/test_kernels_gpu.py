@@ -274,8 +274,8 @@ def test_fp8_quantize():
 @pytest.mark.parametrize("K,M,N", [(128, 256, 256), (1024, 768, 512), (2048, 512, 1280)])
 @pytest.mark.parametrize("accumulate", [True, False])
 def test_wgrad_gemm_vs_fp32_reference(variant, K, M, N, accumulate):
-    """Hand-written k-major weight-gradient GEMM (gemm_wgrad.hip, every schedule variant and a
-    non-default block order) == fp32 reference of C (+)= alpha * A^T B."""
+    """Hand-written k-major weight-gradient GEMM (gemm_wgrad.hip: tiles of 256 and 128 rows, the plan's choice, four splits of
+    the tokens) == fp32 reference of C (+)= alpha * A^T B."""
     g = torch.Generator(device="cuda").manual_seed(K + M + N)
     a = torch.randn(K, M, device="cuda", generator=g).bfloat16()
     b = torch.randn(K, N, device="cuda", generator=g).bfloat16()

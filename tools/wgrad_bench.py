@@ -20,7 +20,7 @@ for K, M, N in [(128, 256, 256), (512, 512, 768), (1024, 768, 512), (8192, 256, 
     b = torch.randn(K, N, device="cuda", dtype=torch.bfloat16)
     c = torch.randn(M, N, device="cuda")
     ref = c.double() + 0.5 * (a.double().t() @ b.double())
-    for v in (0, 1, 2):
+    for v in (0, 1, 2):  # tiles of 256 x 256, of 128 x 256, the plan's choice
         cc = c.clone()
         torch.ops.sxe.wgrad_gemm_variant_(a, b, cc, 0.5, True, v)
         err = ((cc.double() - ref).norm() / ref.norm()).item()
@@ -43,10 +43,10 @@ for (Mo, Ni) in [(6144, 4096), (4096, 4096), (28672, 4096), (4096, 14336), (1282
     def tn_fp32():
         d1, x1 = torch.ops.sxe.transpose16(gy), torch.ops.sxe.transpose16(x)
         torch.ops.aten.addmm.dtype_out(acc2, d1, x1.t(), torch.float32, beta=1, alpha=1, out=acc2)
-    arms = {"v0 accum": lambda: torch.ops.sxe.wgrad_gemm_variant_(gy, x, acc, 1.0, True, 0),
-            "v1 accum": lambda: torch.ops.sxe.wgrad_gemm_variant_(gy, x, acc, 1.0, True, 1),
-            "v2 accum": lambda: torch.ops.sxe.wgrad_gemm_variant_(gy, x, acc, 1.0, True, 2),
-            "v2 overwrite": lambda: torch.ops.sxe.wgrad_gemm_variant_(gy, x, acc, 1.0, False, 2),
+    arms = {"256x256 accum": lambda: torch.ops.sxe.wgrad_gemm_variant_(gy, x, acc, 1.0, True, 0),
+            "128x256 accum": lambda: torch.ops.sxe.wgrad_gemm_variant_(gy, x, acc, 1.0, True, 1),
+            "plan accum": lambda: torch.ops.sxe.wgrad_gemm_variant_(gy, x, acc, 1.0, True, 2),
+            "plan overwrite": lambda: torch.ops.sxe.wgrad_gemm_variant_(gy, x, acc, 1.0, False, 2),
             "hipBLASLt NT fp32": lambda: torch.ops.aten.addmm.dtype_out(acc2, gy.t(), x, torch.float32, beta=1,
                                                                          alpha=1, out=acc2),
             "transposes+TN fp32": tn_fp32}

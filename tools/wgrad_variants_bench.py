@@ -1,7 +1,7 @@
 """Weight-gradient GEMM variants at the Llama-3-8B headline micro-step (16,384 tokens), fp32 accumulator:
-  nt32   : hipBLASLt fp32-out, beta = 1, token-major operands (the current QKV path)
+  nt32   : hipBLASLt fp32-out, beta = 1, token-major operands
   hand   : csrc/kernels/gemm_wgrad.hip k-major kernel (fp32 accumulate)
-  tn+T32 : two transposes + TN fp32-out beta = 1 (the current LM-head path)
+  tn+T32 : two transposes + TN fp32-out beta = 1
   tn32   : TN fp32-out beta = 1 with operands already token-minor (producers write them)
   tn16   : TN bf16-out + fp32 add, operands already token-minor (the MLP path)
   T      : cost of the two transposes alone
