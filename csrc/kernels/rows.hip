@@ -260,7 +260,7 @@ void scatter_rows_(at::Tensor dst, const at::Tensor& idx, const at::Tensor& src)
 }
 
 at::Tensor embedding_grad(const at::Tensor& gy, const at::Tensor& idx, int64_t rows) {
-  SXE_CHECK_CUDA(gy);
+  check_beside(gy, {idx});
   const int64_t n = idx.numel();
   SXE_CHECK(gy.dim() == 2 && gy.is_contiguous() && gy.size(1) % 8 == 0 && reinterpret_cast<uintptr_t>(gy.data_ptr()) % 16 == 0,
             "embedding_grad: gy [N, W], W a multiple of 8");

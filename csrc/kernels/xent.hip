@@ -371,6 +371,7 @@ static void col_blocks(int lanes, int V, int64_t ld, F f) {
 }
 
 static void xent_cols_checks(const at::Tensor& x, const at::Tensor& target) {
+  check_beside(x, {target});
   SXE_CHECK(x.dim() == 2 && x.is_contiguous() && x.scalar_type() == at::kBFloat16 && x.size(1) % 8 == 0 && x.size(0) > 0 &&
                 x.size(0) < (1ll << 30) && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0,
             "xent_cols: bf16 logits [vocab, columns], columns in multiples of 8");
@@ -406,6 +407,7 @@ std::tuple<at::Tensor, at::Tensor> xent_cols_fwd(at::Tensor logits, at::Tensor t
 
 at::Tensor xent_cols_bwd(at::Tensor logits, at::Tensor target, at::Tensor lse, at::Tensor dloss, int64_t ignore_index) {
   xent_cols_checks(logits, target);
+  check_beside(logits, {lse, dloss});
   for (const at::Tensor* t : {&lse, &dloss})
     SXE_CHECK(t->is_cuda() && t->scalar_type() == at::kFloat && t->is_contiguous() && t->numel() == target.numel(),
               "xent_cols: fp32 lse and dloss [tokens]");

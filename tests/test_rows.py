@@ -94,3 +94,19 @@ def test_embedding_gradient(tokens, kind, dtype, W):
     assert bool(((got.double() - want).abs() <= eps * want.abs() + 2 ** -24 * n * size + 2 ** -25).all())
     assert torch.equal(got, torch.autograd.grad(y, emb.weight, gy)[0])
     assert torch.equal(got, torch.ops.sxe.embedding_grad(gy, ids.int(), V))
+
+
+@pytest.mark.gpu
+def test_operands_elsewhere_are_refused():
+    """Indices, targets and row sums in host memory (or on another GPU, as the same check finds) raise; no kernel gets their addresses."""
+    from shuffle_exchange_amd.ops import native
+    native.require_hip()
+    gy, ids = torch.zeros(4, 64, device="cuda"), torch.zeros(4, dtype=torch.long)
+    with pytest.raises(RuntimeError, match="an operand is on"):
+        torch.ops.sxe.embedding_grad(gy, ids, 10)
+    x = torch.zeros(65, 64, device="cuda", dtype=torch.bfloat16)
+    with pytest.raises(RuntimeError, match="an operand is on"):
+        torch.ops.sxe.xent_cols_fwd(x, ids, -100)
+    f = torch.zeros(4)
+    with pytest.raises(RuntimeError, match="an operand is on"):
+        torch.ops.sxe.xent_cols_bwd(x, ids.cuda(), f, f, -100)
