@@ -68,15 +68,17 @@ class _ColumnHeadXEnt(torch.autograd.Function):
     @staticmethod
     def forward(ctx, h, weight, target, ignore_index):
         tgt = target.reshape(-1).contiguous()
-        logits = torch.ops.sxe.gemm_tn(weight, _column_states(h), None, False)
+        h2 = _column_states(h)
+        logits = torch.ops.sxe.gemm_tn(weight, h2, None, False)
         loss, lse = torch.ops.sxe.xent_cols_fwd(logits, tgt, int(ignore_index))
-        ctx.save_for_backward(logits, lse, tgt, h, weight)
+        # the rows that were rounded up are kept beside h: making them again costs 2368 x 768 a fill and a copy, 8 us
+        ctx.save_for_backward(logits, lse, tgt, h, h2 if h2.data_ptr() != h.data_ptr() else None, weight)
         ctx.ignore_index = int(ignore_index)
         return loss.view(target.shape)
 
     @staticmethod
     def backward(ctx, dloss):
-        logits, lse, tgt, h, weight = ctx.saved_tensors
+        logits, lse, tgt, h, h2, weight = ctx.saved_tensors
         g = torch.ops.sxe.xent_cols_bwd(logits, tgt, lse, dloss.detach().reshape(-1).float().contiguous(), ctx.ignore_index)
         del logits
         dh = dw = None
@@ -87,7 +89,7 @@ class _ColumnHeadXEnt(torch.autograd.Function):
             if ctx.needs_input_grad[1]:
                 dw = g @ h.reshape(-1, h.shape[-1])
             return dh, dw, None, None
-        h2 = _column_states(h)
+        h2 = _column_states(h) if h2 is None else h2
         if ctx.needs_input_grad[0]:  # contracts the vocabulary: the form of a weight gradient, in fp32 parts
             dh = torch.empty(h2.shape, device=h2.device, dtype=torch.float32)
             torch.ops.sxe.wgrad_gemm_(g, weight, dh, 1.0, False)
