@@ -159,6 +159,16 @@ inline int stream_grid(int64_t work_items, int block) {
   return (int)(g < 1 ? 1 : g);
 }
 
+// the opt-ins `f` of a kernel family, once on every device of the process
+template <typename F>
+inline void on_each_device(std::atomic<uint64_t>& done, F f) {
+  int dev = 0;
+  SXE_HIP_CHECK(hipGetDevice(&dev));
+  if (dev < 64 && (done.load(std::memory_order_relaxed) >> dev & 1)) return;
+  f();
+  if (dev < 64) done.fetch_or(1ull << dev, std::memory_order_relaxed);
+}
+
 inline hipStream_t cur_stream() { return at::hip::getCurrentHIPStream().stream(); }
 
 }  // namespace sxe

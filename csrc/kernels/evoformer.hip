@@ -5,25 +5,27 @@
 // Reference: ops/deepspeed4science/evoformer_attn.py (CUTLASS kernels of csrc/deepspeed4science,
 // not in the snapshot; kMax = 64 there too).
 //
-// What bounds it: with D = 32 a score costs 4 matrix-core cycles and ~11 VALU ones (bias, exponent, sums, rounding), so
-// every access and instruction a score has to pay for counts. Structure:
+// What bounds it: with D = 32 the vector work of a score (exponent 8 clocks a wave's instruction, every other 4) beside two to four
+// products of it, and how little of the two the two or three waves of a SIMD overlap: at 1 x 128 x 384, 8 heads of 32, the vector units
+// are busy 70 % of the forward's time, 40 to 45 % of the backward's, the matrix cores 22 to 29 %. Structure:
 //  * swapped products (S^T = K Q^T: one lane = one query's scores, lane-local softmax) on v_mfma_f32_32x32x16_bf16, the
-//    score accumulator reused as the B operand of O^T += V^T P^T; 128 queries (or keys) a workgroup, K / V (Q / dO) tiles
-//    of 64 rows direct to LDS in rows of D elements, two slots;
-//  * the pair bias is brought into the accumulator's order once a call (pack_kernel: 2 x [H, L, L]), in the type it came in:
-//    a lane then reads its 16 scores' biases as 16-byte vectors (lane = query for the forward and dQ, lane = key for
-//    dK / dV and dbias2) one tile ahead. Read in place they are 16 loads of one value, each over 32 rows of the matrix;
-//  * the row mask is packed to fp32 in the log2 domain with -inf behind the last key, which is all the tail masking there
-//    is; rows behind L are read from a row of zeros;
-//  * dbias2 = sum of dS over the N rows has a kernel of its own that keeps a 64 x 128 tile of it in registers while it
-//    walks the rows (a third recomputation of dS costs less than L x L atomics a row and is deterministic); where that
-//    gives too few workgroups the rows are split and the parts added up by a last pass. dbias1: per-lane sums, one atomic
-//    a key;
-//  * delta = rowsum(dO O) is formed in the dQ kernel, which leaves it and the log2-domain LSE to the other two.
-// MSA row attention 1 x 128 x 384, 8 heads of 32, bf16 biases, MI355X, forward + backward: 1595 us with biases read in
-// place, dbias2 by atomics and delta by torch; see the kernels below for what each takes now.
-#include "sxe_common.h"
-#include "sxe_tile.h"
+//    score accumulator reused as the B operand of O^T += V^T P^T; 128 queries (or keys) a workgroup, K / V (Q / dO) rows
+//    direct to LDS, two slots;
+//  * the scores' accumulator starts at the pair bias: packed once a call (pack_kernel: 2 x [H, L, L]) in the accumulator's order, in
+//    fp32 and in the products' domain, so that adding it costs no instruction (converted, scaled and added per score it was three of
+//    about ten). Two of the N rows share a workgroup and its biases' registers (64 KB of biases a tile of 128 x 128 and row each else:
+//    forward 68 us, 59 shared);
+//  * the row mask of the kernels with queries on the lanes, and LSE and delta of those with keys on them, come in by one more product
+//    each: three bf16 parts of the fp32 number times ones. As rows of LDS floats they cost four broadcast reads and 16 instructions a
+//    tile each;
+//  * the mask is -inf behind the last key, which is all the tail masking there is; rows behind L are read as zeros;
+//  * dbias2 = sum of dS over the N rows stays in registers while a workgroup walks the rows; up to 384 keys of head dim 32 together
+//    with dQ (dq_pair_kernel), else in a kernel of its own (dpair_kernel). Where that gives too few workgroups the rows are split and the
+//    parts added up by a last pass. dbias1: per-lane sums, one atomic a key;
+//  * delta = rowsum(dO O) is formed in the dQ kernels, which leave it and the LSE to the others.
+// MSA row attention 1 x 128 x 384, 8 heads of 32, bf16 biases, MI355X, forward + backward: 278 us with biases added per score, dQ and
+// dbias2 apart (forward 62, dQ 68, dK / dV 76, dbias2 79); 238 now (forward 58, dQ + dbias2 95, dK / dV 83).
+#include "sxe_gemm_loop.h"
 #include <torch/library.h>
 #include <type_traits>
 
@@ -31,138 +33,225 @@ namespace sxe {
 namespace evo {
 using namespace tl;
 
-constexpr int NW = 4, QB = 32 * NW, KT = 64;  // waves, rows of a workgroup, rows of a streamed tile
-constexpr int TAIL = 2 * KT * 4;              // bytes of a slot's two fp32 rows
+constexpr int NW = 4, QB = 32 * NW, KT = 64;  // waves, rows of a workgroup, streamed rows of a step
+constexpr float FAR = 1.1e9f;                 // biases beyond it are this far: sums of them stay finite, exp() of them stays 0
 
 __device__ const __attribute__((aligned(128))) unsigned short kZeroRow[64] = {0};
 
 struct Args {
   const unsigned short *q, *k, *v, *dout, *o;
-  const float* b1;        // packed row mask [B N, Lp]
-  const void *pq, *pk;    // packed pair bias, lane = query / lane = key; null: none
-  float *lse, *lse2, *ndelta;  // [B N, H, Lp]: natural log; log2 domain, -delta
+  const unsigned short* km;  // row mask as an MFMA operand [B N, Lp, 16]
+  const float* mask;         // row mask [B N, Lp], log2 domain
+  const float *pq, *pk;      // packed pair bias, lane = query / lane = key; null: none
+  float* lse;                // [B N, H, Lp], log2 domain
+  unsigned short *sl, *sd;   // -LSE and -delta as MFMA operands [B N, H, Lp, 16]
   int B, N, L, H, Lp;
-  float c;                // log2(e) / sqrt(D)
+  float c;                   // log2(e) / sqrt(D)
 };
 
+// x in three bf16 parts, which is all of its 24 bits; inf and NaN in the first
+__device__ __forceinline__ void split3(float x, unsigned short* to) {
+  to[0] = f32_to_bf16(x);
+  const float hi = bf16_to_f32(to[0]);
+  const bool finite = fabsf(hi) < INFINITY;
+  const float rest = finite ? x - hi : 0.f;
+  to[1] = f32_to_bf16(rest);
+  to[2] = f32_to_bf16(rest - bf16_to_f32(to[1]));
+}
+// The two halves of an operand row [16]: the parts of x, zeros. Lane half hf holds k = 8 hf ..: a row times `ones` is x.
+__device__ __forceinline__ u32x4 split_half(float x, int hf) {
+  unsigned short h[3];
+  split3(x, h);
+  return hf ? u32x4{0u, 0u, 0u, 0u} : u32x4{h[0] | (unsigned)h[1] << 16, h[2], 0u, 0u};
+}
+__device__ __forceinline__ bf16x8 ones() {
+  return __builtin_bit_cast(bf16x8, u32x4{0x3f803f80u, 0x3f80u, 0u, 0u});
+}
+__device__ __forceinline__ float bounded(float x) {  // inf and NaN stay
+  return x < -FAR && x > -INFINITY ? -FAR : x > FAR && x < INFINITY ? FAR : x;
+}
+
 // ------------------------------------------------------------------------------------ bias packing
-// One launch for both. bias1 (null: none) [B N, L] -> [B N, Lp] fp32 * log2(e), -inf behind L: the blocks of the last grid row.
-// bias2 [B H, L, L] -> 32 x 32 tiles in accumulator order: element (tile (a, b), half i / 8, lane, i % 8) is the value of
-// register i of that lane. pq: lane = query of tile row a, registers = keys of b; pk (may be null): lane = key of tile row
-// a, registers = queries of b. Grid: (nt * nt, B H + 1), nt = Lp / 32; without bias2 (64, 1).
+// One launch for both. bias1 (null: none) [B N, L] -> mask [B N, Lp] * log2(e) and km [B N, Lp, 16] * sqrt(D), -inf behind L:
+// the blocks of the first grid row. A row whose largest bias is far below zero (every key masked by a large
+// finite number) is moved up to zero: the softmax is the same, and its scores keep their fractions.
+// bias2 [B H, L, L] * sqrt(D) -> 32 x 32 fp32 tiles in accumulator order: element (tile (a, b), quarter i / 4, lane, i % 4) is
+// the value of register i of that lane. pq: lane = query of tile row a, registers = keys of b; pk (may be null): lane = key of
+// tile row a, registers = queries of b. Grid: (nt * nt, B H + 1), nt = Lp / 32; without bias2 (64, 1).
 template <typename T>
-__global__ void __launch_bounds__(256) pack_kernel(const void* __restrict__ b1, int b1_bf16, float* __restrict__ mask, int64_t n1,
-                                                   const T* __restrict__ b2, T* __restrict__ pq, T* __restrict__ pk, int L, int nt) {
-  if (blockIdx.y == gridDim.y - 1) {
+__global__ void __launch_bounds__(256) pack_kernel(const void* __restrict__ b1, int b1_bf16, float* __restrict__ mask,
+                                                   unsigned short* __restrict__ km, int64_t rows, const T* __restrict__ b2,
+                                                   float* __restrict__ pq, float* __restrict__ pk, int L, int nt, float root) {
+  auto value = [](auto t) { return sizeof(t) == 2 ? bf16_to_f32((unsigned short)t) : (float)t; };
+  if (blockIdx.y == 0) {
+    __shared__ float tops[4];
     const int Lp = 32 * nt;
-    for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < n1; i += gridDim.x * 256ll) {
-      const int key = i % Lp;
-      const int64_t at = i / Lp * L + key;
-      float x = 0.f;
-      if (b1 != nullptr && key < L)
-        x = b1_bf16 ? bf16_to_f32(reinterpret_cast<const unsigned short*>(b1)[at]) : reinterpret_cast<const float*>(b1)[at];
-      mask[i] = key < L ? x * LOG2E : -INFINITY;
+    for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
+      auto at = [&](int key) {
+        if (key >= L) return -INFINITY;
+        const int64_t i = row * L + key;
+        const float x = b1 == nullptr ? 0.f : b1_bf16 ? bf16_to_f32(reinterpret_cast<const unsigned short*>(b1)[i])
+                                                      : reinterpret_cast<const float*>(b1)[i];
+        return x * LOG2E == -INFINITY ? -INFINITY : x;
+      };
+      float top = -INFINITY;
+      if (b1 != nullptr)
+        for (int key = threadIdx.x; key < L; key += 256) top = fmaxf(top, at(key));
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) top = fmaxf(top, __shfl_xor(top, o));
+      if ((threadIdx.x & 63) == 0) tops[threadIdx.x >> 6] = top;
+      __syncthreads();
+      top = fmaxf(fmaxf(tops[0], tops[1]), fmaxf(tops[2], tops[3]));
+      __syncthreads();
+      const float up = top < -1e4f && top > -INFINITY ? top : 0.f;
+      for (int key = threadIdx.x; key < Lp; key += 256) {
+        const float x = bounded(at(key) - up);
+        mask[row * Lp + key] = x * LOG2E;
+        u32x4* to = reinterpret_cast<u32x4*>(km + (row * Lp + key) * 16);
+        to[0] = split_half(x * root, 0);
+        to[1] = split_half(0.f, 1);
+      }
     }
     return;
   }
-  __shared__ T t[32][33];
+  __shared__ float t[32][33];
   const int a = blockIdx.x / nt, b = blockIdx.x - a * nt;
-  const T* src = b2 + (int64_t)blockIdx.y * L * L;
+  const int64_t bh = blockIdx.y - 1;
+  const T* src = b2 + bh * L * L;
   for (int i = threadIdx.x; i < 1024; i += 256) {
     const int q = 32 * a + i / 32, k = 32 * b + i % 32;
-    t[i / 32][i % 32] = q < L && k < L ? src[(int64_t)q * L + k] : (T)0;
+    t[i / 32][i % 32] = q < L && k < L ? bounded(value(src[(int64_t)q * L + k])) * root : 0.f;
   }
   __syncthreads();
-  const int64_t tiles = (int64_t)blockIdx.y * nt * nt;
-  for (int i = threadIdx.x; i < 1024; i += 256) {
-    const int reg = (i >> 9) * 8 + (i & 7), lane = (i >> 3) & 63, r = acc_row(reg, lane >> 5);
-    pq[(tiles + (int64_t)a * nt + b) * 1024 + i] = t[lane & 31][r];
-    if (pk != nullptr) pk[(tiles + (int64_t)b * nt + a) * 1024 + i] = t[r][lane & 31];
+  const int64_t tiles = bh * nt * nt;
+  const int g = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 31;
+  f32x4 x, y;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int at = acc_row(4 * g + e, lane >> 5);
+    x[e] = t[r][at];
+    y[e] = t[at][r];
   }
+  *reinterpret_cast<f32x4*>(pq + (tiles + (int64_t)a * nt + b) * 1024 + threadIdx.x * 4) = x;
+  if (pk != nullptr) *reinterpret_cast<f32x4*>(pk + (tiles + (int64_t)b * nt + a) * 1024 + threadIdx.x * 4) = y;
 }
 
-struct NoBias {};
 // waves a SIMD: what the registers allow without spills
-template <int D, typename BT>
-constexpr int min_waves() { return D == 32 && !std::is_same<BT, float>::value ? 3 : 2; }
-// a lane's 16 biases of one 32 x 32 tile
-template <typename BT>
-struct Bias {
-  u32x4 v[sizeof(BT)];
-  __device__ __forceinline__ void load(const void* packed, int64_t tile, int lane) {
-    const char* p = reinterpret_cast<const char*>(packed) + (tile * 1024 + lane * 8) * sizeof(BT);
+template <int D>
+constexpr int min_waves() { return D == 32 ? 3 : 2; }
+// a lane's 16 biases of one 32 x 32 tile: where the accumulator of the scores starts
+template <bool PAIR>
+__device__ __forceinline__ f32x16 load_bias(const float* packed, int64_t tile, int lane) {
+  f32x16 x = zero16();
+  if constexpr (PAIR) {
+    const float* p = packed + tile * 1024 + lane * 4;
 #pragma unroll
-    for (int i = 0; i < (int)sizeof(BT); ++i)  // halves are 512 elements apart, a half is sizeof(BT) / 2 vectors
-      v[i] = *reinterpret_cast<const u32x4*>(p + (sizeof(BT) == 2 ? i * 1024 : (i >> 1) * 2048 + (i & 1) * 16));
-  }
-  __device__ __forceinline__ float at(int i) const {
-    if constexpr (sizeof(BT) == 2) {
-      const unsigned x = v[i >> 3][(i & 7) >> 1];
-      return __uint_as_float(i & 1 ? x & 0xffff0000u : x << 16);
-    } else {
-      return __uint_as_float(v[i >> 2][i & 3]);
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 y = *reinterpret_cast<const f32x4*>(p + 256 * g);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[4 * g + e] = y[e];
     }
   }
-};
-template <>
-struct Bias<NoBias> {
-  __device__ __forceinline__ void load(const void*, int64_t, int) {}
-};
-// (bias1 + bias2) * log2(e); m: the packed bias1
-template <typename BT>
-__device__ __forceinline__ float bias_term(const Bias<BT>& b, int i, float m) {
-  if constexpr (std::is_same<BT, NoBias>::value) return m;
-  else return __builtin_fmaf(b.at(i), LOG2E, m);
+  return x;
 }
 
-__device__ __forceinline__ void glds4(const void* src, char* dst) {
-  const unsigned a = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)lds +
-                                                    (unsigned)(dst - lds));
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(a), "v"(src) : "memory", "m0");
+// Rows of one (b, n), head h, that arrive 16 bytes a lane through a buffer resource: its length is the rows that are there, and what
+// is read behind it is zeros. A lane's offset and a wave's resource stay, the base moves: nothing is left to do a load.
+struct Rows {
+  const unsigned short* x;
+  int left;  // rows from x on
+  __device__ __forceinline__ u32x4 resource(int most, int64_t rs) const {
+    const uint64_t p = reinterpret_cast<uint64_t>(x);
+    auto uniform = [](unsigned v) { return (unsigned)__builtin_amdgcn_readfirstlane(v); };
+    return u32x4{uniform((unsigned)p), uniform((unsigned)(p >> 32) & 0xffffu), uniform((unsigned)(min(max(left, 0), most) * (int)rs) * 2u),
+                 0x00020000u};
+  }
+};
+// 1 KB: as gl::glds, from a resource
+__device__ __forceinline__ void blds(unsigned off, const u32x4& res, unsigned dst) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(dst), "v"(off), "s"(res) : "memory", "m0");
 }
-
-// rows row0 .. of x (rows of one (b, n), head h) to LDS; rows behind L are zeros
+// a lane's byte offset for KB i of a tile: 1024 / (2 D) rows each
 template <int D>
-__device__ __forceinline__ void load_rows(char* dst, const unsigned short* x, int64_t rs, int row0, int L) {
-  load_tile<KT, D, NW>(dst, D / 8, [&](int r) { return row0 + r < L ? x + (int64_t)(row0 + r) * rs : kZeroRow; });
+__device__ __forceinline__ unsigned row_off(int i, int lane, int64_t rs) {
+  const int r = i * (512 / D) + lane / (D / 8);
+  return (unsigned)(r * (int)rs + (lane % (D / 8) ^ swz<D>(r)) * 8) * 2;
 }
+
+// Streamed rows: a step takes KT / NN rows of two arrays from each of NN of the N rows, 2 NN tiles in LDS. A wave's loads of a
+// step are LOADS KB of one tile.
+template <int D, int NN>
+struct Stream {
+  static constexpr int ROWS = KT / NN, TILE = ROWS * 2 * D, SLOT = 2 * NN * TILE, PART = TILE / 1024, LOADS = 2 * NN * PART / NW;
+  static_assert(LOADS * NW == 2 * NN * PART && PART % LOADS == 0);
+  Rows rows;
+  unsigned off[LOADS];
+  int at;
+  int64_t rs;
+  // x, y: the first rows of the first of the NN; step: elements from one to the next, the last of them `last`
+  __device__ __forceinline__ void init(const unsigned short* x, const unsigned short* y, int64_t step, int last, int64_t rs_, int L, int w,
+                                       int lane) {
+    at = LOADS * w, rs = rs_;
+    const int tile = at / PART;
+    rows = {(tile & 1 ? y : x) + min(tile >> 1, last) * step, L};
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) off[i] = row_off<D>(at % PART + i, lane, rs);
+  }
+  // the next ROWS rows
+  __device__ __forceinline__ void load(char* slot) {
+    const unsigned dst = gl::lds_base() + (unsigned)(slot - lds) + at * 1024;
+    const u32x4 res = rows.resource(ROWS, rs);
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) blds(off[i], res, dst + i * 1024);
+    rows.x += ROWS * rs, rows.left -= ROWS;
+  }
+};
+// Said to be global memory: a load through a pointer chosen between the two would be a flat one, and every wait for LDS would
+// wait for it, too.
+template <typename T>
+using Global = __attribute__((address_space(1))) T;
 template <int D>
 __device__ __forceinline__ void frags(bf16x8 (&f)[D / 16], const unsigned short* x, int64_t rs, int row, int L, int hf) {
 #pragma unroll
   for (int t = 0; t < D / 16; ++t)
-    f[t] = *reinterpret_cast<const bf16x8*>((row < L ? x + (int64_t)row * rs : kZeroRow) + 16 * t + 8 * hf);
+    f[t] = *reinterpret_cast<const Global<bf16x8>*>((row < L ? (const Global<unsigned short>*)(x + (int64_t)row * rs)
+                                                             : (const Global<unsigned short>*)kZeroRow) + 16 * t + 8 * hf);
 }
-// four floats of each register group of a lane half: rows 8 g + 4 hf .. of an LDS row of floats
-struct Rows16 {
-  f32x4 x[4];
-  __device__ __forceinline__ void load(const char* p, int first, int hf) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g) x[g] = *reinterpret_cast<const f32x4*>(p + 4 * (first + 8 * g + 4 * hf));
-  }
-  __device__ __forceinline__ float at(int i) const { return x[i >> 2][i & 3]; }
-};
+
+// where a lane's half of its row is in an array of operand rows [16]
+__device__ __forceinline__ int lane_row(int lane) { return (lane & 31) * 16 + (lane >> 5) * 8; }
+// log2-domain LSE from the reference exponent and the sum. Without a key, behind L, and where the pair bias alone puts every
+// score of the row so far out that fp32 has no fractions there, it is large: the probabilities of the backward are 0.
+__device__ __forceinline__ float row_lse(bool in, float m, float l) {
+  return in && l > 0.f && fabsf(m) < 1.6e7f ? m + log2f(l) : 1e30f;
+}
 
 struct Place {
-  int b, n, h, blk, bn;
-  int64_t rs, base, row;  // row stride; element of (b, n, 0, h, 0); row of the [B N, H, Lp] arrays
+  int b, n, h, blk, bn, last;  // n, bn: the first of the workgroup's rows, n + last its last
+  int64_t rs, base, row;       // row stride; element of (b, n, 0, h, 0); row of the [B N, H, Lp] arrays
+  int64_t step, srow;          // from one n to the next
 };
 // The N rows that share a pair-bias tile are neighbours in the grid. (A row's blocks and heads on one XCD instead measured
 // the same: K / V traffic does not bound these kernels.)
-template <int D>
+template <int D, int NN>
 __device__ __forceinline__ Place place(const Args& a) {
   Place p;
   int idx = blockIdx.x;
-  p.n = idx % a.N;
-  idx /= a.N;
+  const int nn = (a.N + NN - 1) / NN;
+  p.n = idx % nn * NN;
+  idx /= nn;
   const int nblk = a.Lp / QB;
   p.blk = idx % nblk;
   idx /= nblk;
   p.h = idx % a.H;
   p.b = idx / a.H;
   p.bn = p.b * a.N + p.n;
+  p.last = min(NN - 1, a.N - 1 - p.n);
   p.rs = (int64_t)a.H * D;
-  p.base = (int64_t)p.bn * a.L * p.rs + (int64_t)p.h * D;
-  p.row = ((int64_t)p.bn * a.H + p.h) * a.Lp;
+  p.step = a.L * p.rs;
+  p.srow = (int64_t)a.H * a.Lp;
+  p.base = p.bn * p.step + (int64_t)p.h * D;
+  p.row = p.bn * p.srow + (int64_t)p.h * a.Lp;
   return p;
 }
 
@@ -173,261 +262,347 @@ __device__ __forceinline__ void store_rows(const f32x16 (&acc)[D / 32], unsigned
 }
 
 // ------------------------------------------------------------------------------------ forward
-template <int D, typename BT>
-__global__ void __launch_bounds__(256, (min_waves<D, BT>())) fwd_kernel(Args a, unsigned short* __restrict__ out) {
-  constexpr int TILE = KT * 2 * D, SLOT = 2 * TILE + TAIL;
+// A workgroup takes the same 128 queries of NN of the N rows; a step is two 32 x 32 tiles a wave, one of each row (NN = 2) or two of
+// the one.
+template <int D, bool PAIR, int NN>
+__global__ void __launch_bounds__(256, (min_waves<D>())) fwd_kernel(Args a, unsigned short* __restrict__ out) {
+  using St = Stream<D, NN>;
+  constexpr int SUB = 2 / NN;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, hf = lane >> 5;
-  const Place p = place<D>(a);
+  const Place p = place<D, NN>(a);
   const int q0 = p.blk * QB + 32 * w, q = q0 + r, nt32 = a.Lp / 32;
   const int64_t tiles = (((int64_t)p.b * a.H + p.h) * nt32 + q0 / 32) * nt32;
-  bf16x8 qf[D / 16];
-  frags<D>(qf, a.q + p.base, p.rs, q, a.L, hf);
-  f32x16 o[D / 32];
+  const unsigned short* km = a.km + (int64_t)p.bn * a.Lp * 16;
+  const int lr = lane_row(lane);
+  bf16x8 qf[NN][D / 16];
+  f32x16 o[NN][D / 32];
+  float m[NN], l[NN];
 #pragma unroll
-  for (int t = 0; t < D / 32; ++t) o[t] = zero16();
-  float m = -INFINITY, l = 0.f;
-  const int n = (a.L + KT - 1) / KT;
-  auto load = [&](int t, char* slot) {
-    load_rows<D>(slot, a.k + p.base, p.rs, t * KT, a.L);
-    load_rows<D>(slot + TILE, a.v + p.base, p.rs, t * KT, a.L);
-    if (w == 0) glds4(a.b1 + (int64_t)p.bn * a.Lp + t * KT + lane, slot + 2 * TILE);
+  for (int i = 0; i < NN; ++i) {
+    frags<D>(qf[i], a.q + p.base + min(i, p.last) * p.step, p.rs, q, a.L, hf);
+#pragma unroll
+    for (int t = 0; t < D / 32; ++t) o[i][t] = zero16();
+    m[i] = -INFINITY, l[i] = 0.f;
+  }
+  const int n = (a.L + St::ROWS - 1) / St::ROWS;
+  St st;
+  st.init(a.k + p.base, a.v + p.base, p.step, p.last, p.rs, a.L, w, lane);
+  f32x16 bias[SUB];
+  bf16x8 kmf[2];
+  auto load = [&](int t) {
+    st.load(lds + (t & 1) * St::SLOT);
+#pragma unroll
+    for (int j = 0; j < SUB; ++j) bias[j] = load_bias<PAIR>(a.pq, tiles + SUB * t + j, lane);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      kmf[u] = *reinterpret_cast<const bf16x8*>(km + (int64_t)min(u % NN, p.last) * a.Lp * 16 + 512 * (SUB * t + u / NN) + lr);
   };
-  Bias<BT> bias[2], next[2];
-  load(0, lds);
-#pragma unroll
-  for (int j = 0; j < 2; ++j) next[j].load(a.pq, tiles + j, lane);
+  load(0);
   wait_loads();
   __syncthreads();
   LaneOffs<D> lo;
   lo.init(lane);
   for (int t = 0; t < n; ++t) {
-    const char* kt = lds + (t & 1) * SLOT;
-    const char* vt = kt + TILE;
+    const char* slot = lds + (t & 1) * St::SLOT;
+    f32x16 s[2];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) bias[j] = next[j];
-    if (t + 1 < n) {
-      load(t + 1, lds + ((t & 1) ^ 1) * SLOT);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) next[j].load(a.pq, tiles + 2 * (t + 1) + j, lane);
-    }
+    for (int u = 0; u < 2; ++u) s[u] = mfma(kmf[u], ones(), bias[u / NN]);
+    if (t + 1 < n) load(t + 1);
     if (q0 < a.L) {
-      f32x16 s[2];
-      float mx = -INFINITY;
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        s[j] = zero16();
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
-        for (int t2 = 0; t2 < D / 16; ++t2) s[j] = mfma(row_at(kt + 32 * j * 2 * D, lo.row[t2]), qf[t2], s[j]);
-        Rows16 mask;
-        mask.load(vt + TILE, 32 * j, hf);
+        for (int t2 = 0; t2 < D / 16; ++t2)
+          s[u] = mfma(row_at(slot + 2 * St::TILE * (u % NN) + 64 * D * (u / NN), lo.row[t2]), qf[u % NN][t2], s[u]);
+      bf16x8 vf[2][2][D / 32];  // read here: in front of their products the wave would wait for each
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          s[j][i] = __builtin_fmaf(s[j][i], a.c, bias_term(bias[j], i, mask.at(i)));
-          mx = fmaxf(mx, s[j][i]);
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+          for (int dt = 0; dt < D / 32; ++dt)
+            vf[u][s2][dt] = tr_at(slot + 2 * St::TILE * (u % NN) + St::TILE + (32 * (u / NN) + 16 * s2) * 2 * D, lo.tr[dt]);
+      if constexpr (D == 32) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < NN; ++i) {
+        float mx = -INFINITY;
+#pragma unroll
+        for (int u = i; u < 2; u += NN)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[u][e]);
+        mx = fmaxf(mx, xor32(mx)) * a.c;
+        const bool grow = mx > m[i] + 8.f;  // lazy rescale: p <= 2^8
+        const float mnew = grow ? mx : m[i], mref = mnew == -INFINITY ? 0.f : mnew, alpha = fast_exp2(m[i] - mref);
+        float ps = 0.f;
+#pragma unroll
+        for (int u = i; u < 2; u += NN)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            s[u][e] = fast_exp2(__builtin_fmaf(s[u][e], a.c, -mref));
+            ps += s[u][e];
+          }
+        l[i] = l[i] * alpha + ps;
+        m[i] = mnew;
+        if (__any(grow)) {
+          asm volatile("");  // stays a branch
+#pragma unroll
+          for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) o[i][dt][e] *= alpha;
         }
       }
-      mx = fmaxf(mx, xor32(mx));
-      const bool grow = mx > m + 8.f;  // lazy rescale: p <= 2^8
-      const float mnew = grow ? mx : m, mref = mnew == -INFINITY ? 0.f : mnew, alpha = fast_exp2(m - mref);
-      float ps = 0.f;
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          s[j][i] = fast_exp2(s[j][i] - mref);
-          ps += s[j][i];
-        }
-      l = l * alpha + ps;
-      m = mnew;
-      if (__any(grow)) {
-#pragma unroll
-        for (int dt = 0; dt < D / 32; ++dt)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
-          const bf16x8 pb = acc_to_b(s[j], s2);
+          const bf16x8 pb = acc_to_b(s[u], s2);
 #pragma unroll
-          for (int dt = 0; dt < D / 32; ++dt) o[dt] = mfma(tr_at(vt + (32 * j + 16 * s2) * 2 * D, lo.tr[dt]), pb, o[dt]);
+          for (int dt = 0; dt < D / 32; ++dt)
+            o[u % NN][dt] = mfma(vf[u][s2][dt], pb, o[u % NN][dt]);
         }
     }
     wait_loads();
     __syncthreads();
   }
-  l += xor32(l);
-  if (q < a.L) store_rows<D>(o, out + p.base + (int64_t)q * p.rs, l > 0.f ? 1.f / l : 0.f, hf);
-  if (hf == 0) a.lse[p.row + q] = q < a.L && l > 0.f ? (m + log2f(l)) * LN2 : INFINITY;
+#pragma unroll
+  for (int i = 0; i < NN; ++i) {
+    if (i > p.last) break;
+    l[i] += xor32(l[i]);
+    if (q < a.L) store_rows<D>(o[i], out + p.base + i * p.step + (int64_t)q * p.rs, l[i] > 0.f ? 1.f / l[i] : 0.f, hf);
+    if (hf == 0) a.lse[p.row + i * p.srow + q] = row_lse(q < a.L, m[i], l[i]);
+  }
 }
 
 // ----------------------------------------------------------------------------------------- dQ
-template <int D, typename BT>
-__global__ void __launch_bounds__(256, (min_waves<D, BT>())) dq_kernel(Args a, unsigned short* __restrict__ dq) {
-  constexpr int TILE = KT * 2 * D, SLOT = 2 * TILE + TAIL;
-  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, hf = lane >> 5;
-  const Place p = place<D>(a);
-  const int q0 = p.blk * QB + 32 * w, q = q0 + r, nt32 = a.Lp / 32;
-  const int64_t tiles = (((int64_t)p.b * a.H + p.h) * nt32 + q0 / 32) * nt32;
-  bf16x8 qf[D / 16], df[D / 16], of[D / 16];
-  frags<D>(qf, a.q + p.base, p.rs, q, a.L, hf);
-  frags<D>(df, a.dout + p.base, p.rs, q, a.L, hf);
-  frags<D>(of, a.o + p.base, p.rs, q, a.L, hf);
-  const int n = (a.L + KT - 1) / KT;
-  auto load = [&](int t, char* slot) {
-    load_rows<D>(slot, a.k + p.base, p.rs, t * KT, a.L);
-    load_rows<D>(slot + TILE, a.v + p.base, p.rs, t * KT, a.L);
-    if (w == 0) glds4(a.b1 + (int64_t)p.bn * a.Lp + t * KT + lane, slot + 2 * TILE);
-  };
-  Bias<BT> bias[2], next[2];
-  load(0, lds);
-#pragma unroll
-  for (int j = 0; j < 2; ++j) next[j].load(a.pq, tiles + j, lane);
-  const float lse2 = a.lse[p.row + q] * LOG2E;
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+// delta = rowsum(dO O) of a lane's query, and what the kernels with keys on the lanes read of it
+template <int D>
+__device__ __forceinline__ float row_delta(const bf16x8 (&df)[D / 16], const bf16x8 (&of)[D / 16]) {
   float delta = 0.f;
 #pragma unroll
   for (int t = 0; t < D / 16; ++t)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) delta += (float)df[t][e] * (float)of[t][e];
-  delta += xor32(delta);
-  if (hf == 0) {
-    a.lse2[p.row + q] = lse2;
-    a.ndelta[p.row + q] = -delta;
+    for (int e = 0; e < 8; e += 2)
+      delta = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{df[t][e], df[t][e + 1]}, bf16x2{of[t][e], of[t][e + 1]}, delta, false);
+  return delta + xor32(delta);
+}
+__device__ __forceinline__ void store_stats(const Args& a, int64_t row, float lse, float delta, int hf) {
+  *reinterpret_cast<u32x4*>(a.sl + row * 16 + 8 * hf) = split_half(-lse / a.c, hf);
+  *reinterpret_cast<u32x4*>(a.sd + row * 16 + 8 * hf) = split_half(-delta, hf);
+}
+
+template <int D, bool PAIR, int NN>
+__global__ void __launch_bounds__(256, 2) dq_kernel(Args a, unsigned short* __restrict__ dq) {
+  using St = Stream<D, NN>;
+  constexpr int SUB = 2 / NN;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, hf = lane >> 5;
+  const Place p = place<D, NN>(a);
+  const int q0 = p.blk * QB + 32 * w, q = q0 + r, nt32 = a.Lp / 32;
+  const int64_t tiles = (((int64_t)p.b * a.H + p.h) * nt32 + q0 / 32) * nt32;
+  const unsigned short* km = a.km + (int64_t)p.bn * a.Lp * 16;
+  const int lr = lane_row(lane);
+  bf16x8 qf[NN][D / 16], df[NN][D / 16];
+  f32x16 acc[NN][D / 32];
+  float lse[NN], delta[NN];
+  const int n = (a.L + St::ROWS - 1) / St::ROWS;
+  St st;
+  st.init(a.k + p.base, a.v + p.base, p.step, p.last, p.rs, a.L, w, lane);
+  f32x16 bias[SUB];
+  bf16x8 kmf[2];
+  auto load = [&](int t) {
+    st.load(lds + (t & 1) * St::SLOT);
+#pragma unroll
+    for (int j = 0; j < SUB; ++j) bias[j] = load_bias<PAIR>(a.pq, tiles + SUB * t + j, lane);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      kmf[u] = *reinterpret_cast<const bf16x8*>(km + (int64_t)min(u % NN, p.last) * a.Lp * 16 + 512 * (SUB * t + u / NN) + lr);
+  };
+  load(0);
+#pragma unroll
+  for (int i = 0; i < NN; ++i) {
+    const int64_t base = p.base + min(i, p.last) * p.step, row = p.row + min(i, p.last) * p.srow + q;
+    bf16x8 of[D / 16];
+    frags<D>(qf[i], a.q + base, p.rs, q, a.L, hf);
+    frags<D>(df[i], a.dout + base, p.rs, q, a.L, hf);
+    frags<D>(of, a.o + base, p.rs, q, a.L, hf);
+    lse[i] = a.lse[row], delta[i] = row_delta<D>(df[i], of);
+    store_stats(a, row, lse[i], delta[i], hf);
+#pragma unroll
+    for (int t = 0; t < D / 32; ++t) acc[i][t] = zero16();
   }
-  f32x16 acc[D / 32], nd;
-#pragma unroll
-  for (int t = 0; t < D / 32; ++t) acc[t] = zero16();
-#pragma unroll
-  for (int i = 0; i < 16; ++i) nd[i] = -delta;
   wait_loads();
   __syncthreads();
   LaneOffs<D> lo;
   lo.init(lane);
   for (int t = 0; t < n; ++t) {
-    const char* kt = lds + (t & 1) * SLOT;
-    const char* vt = kt + TILE;
+    const char* slot = lds + (t & 1) * St::SLOT;
+    f32x16 s[2], dp[2];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) bias[j] = next[j];
-    if (t + 1 < n) {
-      load(t + 1, lds + ((t & 1) ^ 1) * SLOT);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) next[j].load(a.pq, tiles + 2 * (t + 1) + j, lane);
-    }
+    for (int u = 0; u < 2; ++u) s[u] = mfma(kmf[u], ones(), bias[u / NN]);
+    if (t + 1 < n) load(t + 1);
     if (q0 < a.L) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        f32x16 s = zero16(), dp = nd;
+      for (int u = 0; u < 2; ++u) {
+        const char* kt = slot + 2 * St::TILE * (u % NN) + 64 * D * (u / NN);
+        dp[u] = zero16();
 #pragma unroll
         for (int t2 = 0; t2 < D / 16; ++t2) {
-          s = mfma(row_at(kt + 32 * j * 2 * D, lo.row[t2]), qf[t2], s);
-          dp = mfma(row_at(vt + 32 * j * 2 * D, lo.row[t2]), df[t2], dp);
+          s[u] = mfma(row_at(kt, lo.row[t2]), qf[u % NN][t2], s[u]);
+          dp[u] = mfma(row_at(kt + St::TILE, lo.row[t2]), df[u % NN][t2], dp[u]);
         }
-        Rows16 mask;
-        mask.load(vt + TILE, 32 * j, hf);
+      }
 #pragma unroll
-        for (int i = 0; i < 16; ++i)
-          s[i] = fast_exp2(__builtin_fmaf(s[i], a.c, bias_term(bias[j], i, mask.at(i))) - lse2) * dp[i];  // dS^T
+      for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s[u][e] = fast_exp2(__builtin_fmaf(s[u][e], a.c, -lse[u % NN])) * (dp[u][e] - delta[u % NN]);  // dS^T
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
-          const bf16x8 db = acc_to_b(s, s2);
+          const bf16x8 db = acc_to_b(s[u], s2);
 #pragma unroll
-          for (int dt = 0; dt < D / 32; ++dt) acc[dt] = mfma(tr_at(kt + (32 * j + 16 * s2) * 2 * D, lo.tr[dt]), db, acc[dt]);
+          for (int dt = 0; dt < D / 32; ++dt)
+            acc[u % NN][dt] = mfma(tr_at(slot + 2 * St::TILE * (u % NN) + (32 * (u / NN) + 16 * s2) * 2 * D, lo.tr[dt]), db, acc[u % NN][dt]);
         }
       }
     }
     wait_loads();
     __syncthreads();
   }
-  if (q < a.L) store_rows<D>(acc, dq + p.base + (int64_t)q * p.rs, a.c * LN2, hf);
+#pragma unroll
+  for (int i = 0; i < NN; ++i)
+    if (i <= p.last && q < a.L) store_rows<D>(acc[i], dq + p.base + i * p.step + (int64_t)q * p.rs, a.c * LN2, hf);
 }
 
 // -------------------------------------------------------------------------------------- dK, dV
-// Keys on the lanes; Q / dO tiles and their LSE / -delta stream by.
-template <int D>
-__device__ __forceinline__ void load_query_tile(const Args& a, const unsigned short* q, const unsigned short* d, int64_t rs,
-                                                int64_t row, int q0, char* slot, int w, int lane) {
-  constexpr int TILE = KT * 2 * D;
-  load_rows<D>(slot, q, rs, q0, a.L);
-  load_rows<D>(slot + TILE, d, rs, q0, a.L);
-  if (w == 0) glds4(a.lse2 + row + q0 + lane, slot + 2 * TILE);
-  if (w == 1) glds4(a.ndelta + row + q0 + lane, slot + 2 * TILE + KT * 4);
-}
-
-// P and dS [query][key] of 32 queries of a slot, keys on the lanes (queries behind L: LSE inf, so P = 0)
-template <int D, typename BT>
-__device__ __forceinline__ void score_grads(f32x16& pr, f32x16& ds, const char* slot, int j, const LaneOffs<D>& lo,
-                                            const bf16x8 (&kf)[D / 16], const bf16x8 (&vf)[D / 16], const Bias<BT>& bias, float mask,
-                                            float c, int hf) {
-  constexpr int TILE = KT * 2 * D;
-  Rows16 ls, nd;
-  ls.load(slot + 2 * TILE, 32 * j, hf);
-  nd.load(slot + 2 * TILE + KT * 4, 32 * j, hf);
-  pr = zero16();
-#pragma unroll
-  for (int i = 0; i < 16; ++i) ds[i] = nd.at(i);
-#pragma unroll
-  for (int t = 0; t < D / 16; ++t) {
-    pr = mfma(row_at(slot + 32 * j * 2 * D, lo.row[t]), kf[t], pr);
-    ds = mfma(row_at(slot + TILE + 32 * j * 2 * D, lo.row[t]), vf[t], ds);
+// Keys on the lanes; Q / dO tiles and their -LSE / -delta rows stream by.
+template <int D, int NN>
+struct QueryStream : Stream<D, NN> {
+  using S = Stream<D, NN>;
+  static constexpr int STAT = S::ROWS * 32, SLOT = S::SLOT + 2 * NN * STAT;  // bytes of one statistic's rows
+  static_assert(2 * NN * STAT == 1024 * NW);
+  const unsigned short* stat;
+  // base: element of the first row and head; row: of the [B N, H, Lp] arrays
+  __device__ __forceinline__ void init(const Args& a, int64_t base, int64_t row, int64_t step, int64_t srow, int last, int64_t rs, int w,
+                                       int lane) {
+    S::init(a.q + base, a.dout + base, step, last, rs, a.L, w, lane);
+    constexpr int PARTS = STAT / 1024;  // a wave's KB: which statistic of which row, which part of it
+    const int s = w / PARTS;
+    stat = (s & 1 ? a.sd : a.sl) + (row + min(s >> 1, last) * srow) * 16 + w % PARTS * 512;
   }
+  __device__ __forceinline__ void load(char* slot, int w, int lane) {
+    S::load(slot);
+    gl::glds(lane * 16, stat, gl::lds_base() + (unsigned)(slot - lds) + S::SLOT + w * 1024);
+    stat += S::ROWS * 16;
+  }
+};
+
+// The operands of tile u of a slot, 32 queries, and its products: S - LSE and dP - delta [query][key], keys on the lanes (queries behind
+// L: LSE large, so P = 0)
+template <int D, int NN>
+struct QueryTile {
+  using St = QueryStream<D, NN>;
+  bf16x8 lse, delta, q[D / 16], d[D / 16];
+  __device__ __forceinline__ void read(const char* slot, int u, const LaneOffs<D>& lo, int lr) {
+    const char* stat = slot + St::S::SLOT + 2 * St::STAT * (u % NN) + 1024 * (u / NN) + 2 * lr;
+    const char* tile = slot + 2 * St::TILE * (u % NN) + 64 * D * (u / NN);
+    lse = row_at(stat, 0);
+    delta = row_at(stat, St::STAT);
+#pragma unroll
+    for (int t = 0; t < D / 16; ++t) {
+      q[t] = row_at(tile, lo.row[t]);
+      d[t] = row_at(tile + St::TILE, lo.row[t]);
+    }
+  }
+  __device__ __forceinline__ void products(f32x16& pr, f32x16& ds, const bf16x8 (&kf)[D / 16], const bf16x8 (&vf)[D / 16],
+                                           const f32x16& bias) const {
+    pr = mfma(lse, ones(), bias);
+    ds = mfma(delta, ones(), zero16());
+#pragma unroll
+    for (int t = 0; t < D / 16; ++t) {
+      pr = mfma(q[t], kf[t], pr);
+      ds = mfma(d[t], vf[t], ds);
+    }
+  }
+};
+__device__ __forceinline__ void score_grads(f32x16& pr, f32x16& ds, float mask, float c) {
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
-    pr[i] = fast_exp2(__builtin_fmaf(pr[i], c, bias_term(bias, i, mask)) - ls.at(i));
+    pr[i] = fast_exp2(__builtin_fmaf(pr[i], c, mask));
     ds[i] *= pr[i];
   }
 }
 
-template <int D, typename BT>
-__global__ void __launch_bounds__(256, (min_waves<D, BT>())) dkdv_kernel(Args a, unsigned short* __restrict__ dk,
-                                                                   unsigned short* __restrict__ dv, float* __restrict__ db1) {
-  constexpr int TILE = KT * 2 * D, SLOT = 2 * TILE + TAIL;
+template <int D, bool PAIR, int NN, bool DB1>
+__global__ void __launch_bounds__(256, 2) dkdv_kernel(Args a, unsigned short* __restrict__ dk,
+                                                                     unsigned short* __restrict__ dv, float* __restrict__ db1) {
+  using St = QueryStream<D, NN>;
+  constexpr int SUB = 2 / NN;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, hf = lane >> 5;
-  const Place p = place<D>(a);
-  const int k0 = p.blk * QB + 32 * w, key = k0 + r, nt32 = a.Lp / 32;
+  const Place p = place<D, NN>(a);
+  const int k0 = p.blk * QB + 32 * w, key = k0 + r, nt32 = a.Lp / 32, lr = lane_row(lane);
   const int64_t tiles = (((int64_t)p.b * a.H + p.h) * nt32 + k0 / 32) * nt32;
-  bf16x8 kf[D / 16], vf[D / 16];
-  frags<D>(kf, a.k + p.base, p.rs, key, a.L, hf);
-  frags<D>(vf, a.v + p.base, p.rs, key, a.L, hf);
-  const float mask = a.b1[(int64_t)p.bn * a.Lp + key];
-  f32x16 dka[D / 32], dva[D / 32];
+  bf16x8 kf[NN][D / 16], vf[NN][D / 16];
+  f32x16 dka[NN][D / 32], dva[NN][D / 32];
+  float mask[NN], b1acc[NN];
+  St st;
+  st.init(a, p.base, p.row, p.step, p.srow, p.last, p.rs, w, lane);
+  f32x16 bias[SUB];
+  auto load = [&](int t) {
+    st.load(lds + (t & 1) * St::SLOT, w, lane);
 #pragma unroll
-  for (int t = 0; t < D / 32; ++t) dka[t] = dva[t] = zero16();
-  float b1acc = 0.f;
-  const int n = (a.L + KT - 1) / KT;
-  Bias<BT> bias[2], next[2];
-  load_query_tile<D>(a, a.q + p.base, a.dout + p.base, p.rs, p.row, 0, lds, w, lane);
+    for (int j = 0; j < SUB; ++j) bias[j] = load_bias<PAIR>(a.pk, tiles + SUB * t + j, lane);
+  };
+  load(0);
 #pragma unroll
-  for (int j = 0; j < 2; ++j) next[j].load(a.pk, tiles + j, lane);
+  for (int i = 0; i < NN; ++i) {
+    const int64_t base = p.base + min(i, p.last) * p.step;
+    frags<D>(kf[i], a.k + base, p.rs, key, a.L, hf);
+    frags<D>(vf[i], a.v + base, p.rs, key, a.L, hf);
+    mask[i] = a.mask[(int64_t)(p.bn + min(i, p.last)) * a.Lp + key];
+    b1acc[i] = 0.f;
+#pragma unroll
+    for (int t = 0; t < D / 32; ++t) dka[i][t] = dva[i][t] = zero16();
+  }
+  const int n = (a.L + St::ROWS - 1) / St::ROWS;
   wait_loads();
   __syncthreads();
   LaneOffs<D> lo;
   lo.init(lane);
   for (int t = 0; t < n; ++t) {
-    const char* slot = lds + (t & 1) * SLOT;
+    const char* slot = lds + (t & 1) * St::SLOT;
+    f32x16 pr[2], ds[2];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) bias[j] = next[j];
-    if (t + 1 < n) {
-      load_query_tile<D>(a, a.q + p.base, a.dout + p.base, p.rs, p.row, (t + 1) * KT, lds + ((t & 1) ^ 1) * SLOT, w, lane);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) next[j].load(a.pk, tiles + 2 * (t + 1) + j, lane);
+    for (int u = 0; u < 2; ++u) {
+      QueryTile<D, NN> x;
+      x.read(slot, u, lo, lr);
+      __builtin_amdgcn_sched_barrier(0);
+      x.products(pr[u], ds[u], kf[u % NN], vf[u % NN], bias[u / NN]);
     }
+    if (t + 1 < n) load(t + 1);
     if (k0 < a.L) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        f32x16 pr, ds;
-        score_grads<D>(pr, ds, slot, j, lo, kf, vf, bias[j], mask, a.c, hf);
-        if (db1 != nullptr) {
+      for (int u = 0; u < 2; ++u) {
+        const char* tile = slot + 2 * St::TILE * (u % NN) + 64 * D * (u / NN);
+        bf16x8 df[2][D / 32], qf[2][D / 32];  // read here: in front of their products the wave would wait for each
 #pragma unroll
-          for (int i = 0; i < 16; ++i) b1acc += ds[i];
+        for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+          for (int dt = 0; dt < D / 32; ++dt) {
+            df[s2][dt] = tr_at(tile + St::TILE + 32 * D * s2, lo.tr[dt]);
+            qf[s2][dt] = tr_at(tile + 32 * D * s2, lo.tr[dt]);
+          }
+        if constexpr (D == 32) __builtin_amdgcn_sched_barrier(0);
+        score_grads(pr[u], ds[u], mask[u % NN], a.c);
+        if constexpr (DB1) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) b1acc[u % NN] += ds[u][i];
         }
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
-          const bf16x8 pb = acc_to_b(pr, s2), db = acc_to_b(ds, s2);
+          const bf16x8 pb = acc_to_b(pr[u], s2), db = acc_to_b(ds[u], s2);
 #pragma unroll
           for (int dt = 0; dt < D / 32; ++dt) {
-            dva[dt] = mfma(tr_at(slot + TILE + (32 * j + 16 * s2) * 2 * D, lo.tr[dt]), pb, dva[dt]);  // dV^T += dO^T P
-            dka[dt] = mfma(tr_at(slot + (32 * j + 16 * s2) * 2 * D, lo.tr[dt]), db, dka[dt]);         // dK^T += Q^T dS
+            dva[u % NN][dt] = mfma(df[s2][dt], pb, dva[u % NN][dt]);  // dV^T += dO^T P
+            dka[u % NN][dt] = mfma(qf[s2][dt], db, dka[u % NN][dt]);  // dK^T += Q^T dS
           }
         }
       }
@@ -436,30 +611,195 @@ __global__ void __launch_bounds__(256, (min_waves<D, BT>())) dkdv_kernel(Args a,
     __syncthreads();
   }
   if (key >= a.L) return;
-  if (db1 != nullptr) {
-    b1acc += xor32(b1acc);
-    if (hf == 0) atomicAdd(db1 + (int64_t)p.bn * a.L + key, b1acc);
+#pragma unroll
+  for (int i = 0; i < NN; ++i) {
+    if (i > p.last) break;
+    if constexpr (DB1) {
+      b1acc[i] += xor32(b1acc[i]);
+      if (hf == 0) atomicAdd(db1 + (int64_t)(p.bn + i) * a.L + key, b1acc[i]);
+    }
+    store_rows<D>(dka[i], dk + p.base + i * p.step + (int64_t)key * p.rs, a.c * LN2, hf);
+    store_rows<D>(dva[i], dv + p.base + i * p.step + (int64_t)key * p.rs, 1.f, hf);
   }
-  store_rows<D>(dka, dk + p.base + (int64_t)key * p.rs, a.c * LN2, hf);
-  store_rows<D>(dva, dv + p.base + (int64_t)key * p.rs, 1.f, hf);
+}
+
+// ------------------------------------------------------------------------------ dQ and dbias2 together
+// A workgroup has 32 QW queries of one (b, h) and all keys (KEYS of them are Lp), and walks rows_per of the N rows: QW x KG waves, each 32 queries x J tiles
+// of 32 keys, whose biases and dbias2 stay in its registers; the scores are formed once for both gradients. The KG partial sums of
+// dQ go through LDS, and are added up while the next row's scores are formed. part: fp32 [parts, B H, tiles, tiles, 1024], the
+// packed order of pq. Grid: (query tiles * B H, parts), heads fastest.
+template <int QW, int KG, int J>
+struct DqPair {
+  static constexpr int D = 32, NWG = QW * KG, QUERIES = 32 * QW, KEYS = 32 * KG * J, ROWS = KEYS * 2 * D, QROWS = QUERIES * 2 * D;
+  static constexpr int SLOT = 2 * ROWS + 3 * QROWS, RED = NWG * 4096;  // K, V, Q, dO, O
+  static constexpr int NR = 2 * SLOT + 2 * RED <= 160 * 1024 ? 2 : 1, LDS = 2 * SLOT + NR * RED;
+  static_assert(NWG == 8 && LDS <= 160 * 1024);
+};
+template <int QW, int KG, int J>
+__global__ void __launch_bounds__(512, 2) dq_pair_kernel(Args a, unsigned short* __restrict__ dq, float* __restrict__ part, int rows_per) {
+  using C = DqPair<QW, KG, J>;
+  constexpr int D = 32;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), hf = lane >> 5;
+  const int qw = w % QW, kg = w / QW, nt32 = a.Lp / 32, nbh = a.B * a.H, bh = blockIdx.x % nbh, h = bh % a.H, b = bh / a.H;
+  const int qb = C::QUERIES * (blockIdx.x / nbh), q = qb + 32 * qw + (lane & 31), t0 = kg * J;
+  const int64_t rs = (int64_t)a.H * D, step = a.L * rs;
+  const int n0 = blockIdx.y * rows_per, n1 = min(a.N, n0 + rows_per);
+  const int64_t tiles = ((int64_t)bh * nt32 + qb / 32 + qw) * nt32 + t0;
+  const unsigned lbase = gl::lds_base();
+  f32x16 bias[J], dpair[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    bias[j] = load_bias<true>(a.pq, tiles + j, lane);
+    dpair[j] = zero16();
+  }
+  bf16x8 kmn[J];
+  float lsen;
+  // A wave loads K's or V's rows 16 (w / 2) .. of every 64, 16 rows of Q or dO and, the first waves, 16 of O
+  constexpr int QP = C::QUERIES / 16;
+  const int64_t first = ((int64_t)b * a.N + n0) * step + (int64_t)h * D;
+  Rows kv = {(w & 1 ? a.v : a.k) + first, a.L}, qd = {(w < QP ? a.q : a.dout) + first + qb * rs, a.L - qb}, oo = {a.o + first + qb * rs, a.L - qb};
+  const unsigned koff = row_off<D>(w / 2, lane, rs), qoff = row_off<D>(w % QP, lane, rs);
+  const float* lsep = a.lse + (((int64_t)b * a.N + n0) * a.H + h) * a.Lp + q;
+  const unsigned short* kmp = a.km + (((int64_t)b * a.N + n0) * a.Lp + 32 * t0) * 16 + lane_row(lane);
+  auto load = [&](int n) {
+    const unsigned dst = lbase + ((n - n0) & 1) * C::SLOT;
+    const u32x4 kres = kv.resource(C::KEYS, rs), qres = qd.resource(C::QUERIES, rs);
+#pragma unroll
+    for (int i = 0; i < C::KEYS / 64; ++i)
+      blds(koff + i * (unsigned)(128 * rs), kres, dst + (w & 1) * C::ROWS + (w / 2 + 4 * i) * 1024);
+    if (w < 2 * QP) blds(qoff, qres, dst + 2 * C::ROWS + w * 1024);
+    if (w < QP) blds(qoff, oo.resource(C::QUERIES, rs), dst + 2 * C::ROWS + (2 * QP + w) * 1024);
+    lsen = *lsep;
+#pragma unroll
+    for (int j = 0; j < J; ++j) kmn[j] = *reinterpret_cast<const bf16x8*>(kmp + 512 * j);
+    kv.x += step, qd.x += step, oo.x += step, lsep += (int64_t)a.H * a.Lp, kmp += a.Lp * 16;
+  };
+  // dQ of row n: four values a thread
+  auto reduce = [&](int n) {
+    if (threadIdx.x >= 256 * QW) return;
+    const int qt = threadIdx.x >> 8, i = threadIdx.x & 255, qq = qb + 32 * qt + (i & 31);
+    const char* red = lds + 2 * C::SLOT + (C::NR == 2 ? (n - n0) & 1 : 0) * C::RED + 16 * i;
+    f32x4 x = *reinterpret_cast<const f32x4*>(red + qt * 4096);
+#pragma unroll
+    for (int g = 1; g < KG; ++g) x += *reinterpret_cast<const f32x4*>(red + (g * QW + qt) * 4096);
+    if (qq >= a.L) return;
+    const float s = a.c * LN2;
+    const unsigned lo = gl::pack(x[0] * s, x[1] * s), hi = gl::pack(x[2] * s, x[3] * s);
+    unsigned short* to = dq + ((int64_t)b * a.N + n) * step + (int64_t)h * D + (int64_t)qq * rs + 8 * (i >> 6) + 4 * (i >> 5 & 1);
+    *reinterpret_cast<unsigned long long*>(to) = (unsigned long long)lo | (unsigned long long)hi << 32;
+  };
+  LaneOffs<D> lo;
+  lo.init(lane);
+  if (n0 < n1) load(n0);
+  wait_loads();
+  __syncthreads();
+  for (int n = n0; n < n1; ++n) {
+    const char* slot = lds + ((n - n0) & 1) * C::SLOT;
+    const char *kt = slot + t0 * 2048, *qt = slot + 2 * C::ROWS + qw * 2048;
+    bf16x8 qf[2], df[2], of[2], km[J];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      df[t] = row_at(qt + C::QROWS, lo.row[t]);
+      of[t] = row_at(qt + 2 * C::QROWS, lo.row[t]);
+      qf[t] = row_at(qt, lo.row[t]);
+    }
+    const float lse = lsen, delta = row_delta<D>(df, of);
+    const u32x4 nd = split_half(-delta, hf);
+    if (kg == 0) {
+      const int64_t row = (((int64_t)b * a.N + n) * a.H + h) * a.Lp + q;
+      *reinterpret_cast<u32x4*>(a.sl + row * 16 + 8 * hf) = split_half(-lse / a.c, hf);
+      *reinterpret_cast<u32x4*>(a.sd + row * 16 + 8 * hf) = nd;
+    }
+#pragma unroll
+    for (int j = 0; j < J; ++j) km[j] = kmn[j];
+    if (n + 1 < n1) load(n + 1);
+    if (n > n0) reduce(n - 1);
+    f32x16 acc = zero16();
+    // operands are read one use ahead: left to itself the compiler reads each in front of its product and waits
+    bf16x8 kf[2], vf[2], tr[2];
+    auto read = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        kf[t] = row_at(kt + 2048 * j, lo.row[t]);
+        vf[t] = row_at(kt + C::ROWS + 2048 * j, lo.row[t]);
+      }
+    };
+    read(0);
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      f32x16 s = mfma(km[j], ones(), bias[j]), dp = mfma(ones(), __builtin_bit_cast(bf16x8, nd), zero16());
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        s = mfma(kf[t], qf[t], s);
+        dp = mfma(vf[t], df[t], dp);
+      }
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2) tr[s2] = tr_at(kt + 2048 * j + 1024 * s2, lo.tr[0]);
+      if (j + 1 < J) read(j + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s[e] = fast_exp2(__builtin_fmaf(s[e], a.c, -lse));
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        s[e] *= dp[e];  // dS^T
+        dpair[j][e] += s[e];
+      }
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2) acc = mfma(tr[s2], acc_to_b(s, s2), acc);
+    }
+    if constexpr (C::NR == 1) __syncthreads();
+    char* red = lds + 2 * C::SLOT + (C::NR == 2 ? (n - n0) & 1 : 0) * C::RED + w * 4096 + 16 * lane;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) *reinterpret_cast<f32x4*>(red + 1024 * g) = f32x4{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+    wait_loads();
+    __syncthreads();
+  }
+  if (n0 < n1) reduce(n1 - 1);
+  float* out = part + ((int64_t)blockIdx.y * nbh * nt32 * nt32 + tiles) * 1024 + 4 * lane;
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<f32x4*>(out + 1024 * j + 256 * g) = f32x4{dpair[j][4 * g], dpair[j][4 * g + 1], dpair[j][4 * g + 2], dpair[j][4 * g + 3]};
+}
+
+// packed parts -> dbias2 [B H, L, L]; a 32 x 32 tile a workgroup, grid (tiles * tiles, B H) with tiles = ceil(L / 32)
+template <typename T>
+__global__ void __launch_bounds__(256) dpair_tiles_kernel(const float* __restrict__ part, T* __restrict__ out, int64_t stride, int parts, int L,
+                                                          int nt32) {
+  __shared__ float t[32][33];
+  const int tl = (L + 31) / 32, ta = blockIdx.x / tl, tb = blockIdx.x - ta * tl, g = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const float* src = part + (((int64_t)blockIdx.y * nt32 + ta) * nt32 + tb) * 1024 + 4 * threadIdx.x;
+  f32x4 x = {0.f, 0.f, 0.f, 0.f};
+  for (int p = 0; p < parts; ++p) x += *reinterpret_cast<const f32x4*>(src + p * stride);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) t[lane & 31][acc_row(4 * g + e, lane >> 5)] = x[e];
+  __syncthreads();
+  for (int i = threadIdx.x; i < 1024; i += 256) {
+    const int q = 32 * ta + i / 32, k = 32 * tb + i % 32;
+    if (q >= L || k >= L) continue;
+    T* to = out + ((int64_t)blockIdx.y * L + q) * L + k;
+    if constexpr (sizeof(T) == 2) *to = f32_to_bf16(t[i / 32][i % 32]);
+    else *to = t[i / 32][i % 32];
+  }
 }
 
 // -------------------------------------------------------------------------------------- dbias2
 // A workgroup holds dbias2 of 64 queries x 128 keys of one (b, h) and walks rows_per of the N rows. part: fp32 [parts,
 // B H, L, L]. Grid: (query tiles * key blocks * B H, parts), heads fastest: with 8 heads an XCD walks one head's rows
 // (82 us at 128 x 384 x 8 heads of 32; 103 us with the tiles of a head spread over the XCDs).
-template <int D, typename BT>
-__global__ void __launch_bounds__(256, (min_waves<D, BT>())) dpair_kernel(Args a, float* __restrict__ part, int rows_per) {
-  constexpr int TILE = KT * 2 * D, SLOT = 2 * TILE + TAIL;
+template <int D>
+__global__ void __launch_bounds__(256, (min_waves<D>())) dpair_kernel(Args a, float* __restrict__ part, int rows_per) {
+  using St = QueryStream<D, 1>;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, hf = lane >> 5;
-  const int nqt = (a.L + KT - 1) / KT, nkb = a.Lp / QB, nt32 = a.Lp / 32;
+  const int nqt = (a.L + KT - 1) / KT, nkb = a.Lp / QB, nt32 = a.Lp / 32, lr = lane_row(lane);
   const int nbh = a.B * a.H, bh = blockIdx.x % nbh, kb = blockIdx.x / nbh % nkb, qt = blockIdx.x / nbh / nkb;
   const int h = bh % a.H, b = bh / a.H;
   const int k0 = kb * QB + 32 * w, key = k0 + r, q0 = qt * KT;
   const int64_t rs = (int64_t)a.H * D;
-  Bias<BT> bias[2];
+  f32x16 bias[2];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) bias[j].load(a.pk, ((int64_t)bh * nt32 + k0 / 32) * nt32 + 2 * qt + j, lane);
+  for (int j = 0; j < 2; ++j) bias[j] = load_bias<true>(a.pk, ((int64_t)bh * nt32 + k0 / 32) * nt32 + 2 * qt + j, lane);
   const int n0 = blockIdx.y * rows_per, n1 = min(a.N, n0 + rows_per);
   f32x16 acc[2] = {zero16(), zero16()};
   bf16x8 kf[D / 16], vf[D / 16], kn[D / 16], vn[D / 16];
@@ -467,10 +807,13 @@ __global__ void __launch_bounds__(256, (min_waves<D, BT>())) dpair_kernel(Args a
   auto load = [&](int n, char* slot) {
     const int bn = b * a.N + n;
     const int64_t base = (int64_t)bn * a.L * rs + (int64_t)h * D;
-    load_query_tile<D>(a, a.q + base, a.dout + base, rs, ((int64_t)bn * a.H + h) * a.Lp, q0, slot, w, lane);
+    St st;
+    st.init(a, base, ((int64_t)bn * a.H + h) * a.Lp, 0, 0, 0, rs, w, lane);
+    st.rows.x += q0 * rs, st.rows.left -= q0, st.stat += q0 * 16;
+    st.load(slot, w, lane);
     frags<D>(kn, a.k + base, rs, key, a.L, hf);
     frags<D>(vn, a.v + base, rs, key, a.L, hf);
-    maskn = a.b1[(int64_t)bn * a.Lp + key];
+    maskn = a.mask[(int64_t)bn * a.Lp + key];
   };
   if (n0 < n1) load(n0, lds);
   wait_loads();
@@ -485,12 +828,15 @@ __global__ void __launch_bounds__(256, (min_waves<D, BT>())) dpair_kernel(Args a
       vf[t] = vn[t];
     }
     mask = maskn;
-    if (n + 1 < n1) load(n + 1, lds + (cur ^ 1) * SLOT);
+    if (n + 1 < n1) load(n + 1, lds + (cur ^ 1) * St::SLOT);
     if (k0 < a.L) {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         f32x16 pr, ds;
-        score_grads<D>(pr, ds, lds + cur * SLOT, j, lo, kf, vf, bias[j], mask, a.c, hf);
+        QueryTile<D, 1> x;
+        x.read(lds + cur * St::SLOT, j, lo, lr);
+        x.products(pr, ds, kf, vf, bias[j]);
+        score_grads(pr, ds, mask, a.c);
         acc[j] += ds;
       }
     }
@@ -530,7 +876,7 @@ static bool evo_has(const c10::optional<at::Tensor>& t) { return t.has_value() &
 struct EvoCall {
   evo::Args a{};
   at::Tensor q, k, v;  // keep what the pointers look at
-  at::ScalarType pair = at::ScalarType::Undefined;
+  bool pair = false;
 };
 
 static EvoCall evo_call(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v) {
@@ -556,7 +902,8 @@ static EvoCall evo_call(const at::Tensor& q, const at::Tensor& k, const at::Tens
   return c;
 }
 
-// bias1 and bias2 as the kernels read them: [mask, pq, pk], pq undefined without bias2, pk without a backward to come, too
+// bias1 and bias2 as the kernels read them: [mask, pair]; mask fp32 [9, B N, Lp]: the mask, then km; pair fp32 [1 or 2, B H, Lp, Lp]: pq
+// and, where a backward is to come, pk; undefined without bias2
 static std::vector<at::Tensor> evo_pack(const evo::Args& a, const at::TensorOptions& opt, const c10::optional<at::Tensor>& b1,
                                         const c10::optional<at::Tensor>& b2, bool backward) {
   const int64_t rows = (int64_t)a.B * a.N;
@@ -564,44 +911,46 @@ static std::vector<at::Tensor> evo_pack(const evo::Args& a, const at::TensorOpti
   auto ok = [](const at::Tensor& t) { return t.is_contiguous() && (t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16); };
   if (has1) SXE_CHECK(ok(*b1) && b1->numel() == rows * a.L, "evoformer: bias1 fp32 / bf16 [B, N, 1, 1, L]");
   if (pair) SXE_CHECK(ok(*b2) && b2->numel() == (int64_t)a.B * a.H * a.L * a.L, "evoformer: bias2 fp32 / bf16 [B, 1, H, L, L]");
-  at::Tensor mask = at::empty({rows, a.Lp}, opt.dtype(at::kFloat)), pq, pk;
-  if (pair) pq = at::empty({(int64_t)a.B * a.H, a.Lp, a.Lp}, b2->options());
-  if (pair && backward) pk = at::empty_like(pq);
-  if (mask.numel() == 0) return {mask, pq, pk};
+  at::Tensor mask = at::empty({9, rows, a.Lp}, opt.dtype(at::kFloat)), packed;
+  if (pair) packed = at::empty({backward ? 2 : 1, (int64_t)a.B * a.H, a.Lp, a.Lp}, mask.options());
+  if (mask.numel() == 0) return {mask, packed};
   const int nt = a.Lp / 32;
+  float* pq = pair ? packed.data_ptr<float>() : nullptr;
   auto pack = [&](auto* t) {
     using T = std::remove_pointer_t<decltype(t)>;
     hipLaunchKernelGGL(evo::pack_kernel<T>, pair ? dim3(nt * nt, a.B * a.H + 1) : dim3(64, 1), dim3(256), 0, cur_stream(),
-                       has1 ? b1->data_ptr() : nullptr, has1 && b1->scalar_type() == at::kBFloat16, mask.data_ptr<float>(), mask.numel(),
-                       pair ? reinterpret_cast<const T*>(b2->data_ptr()) : nullptr,
-                       pair ? reinterpret_cast<T*>(pq.data_ptr()) : nullptr,
-                       pk.defined() ? reinterpret_cast<T*>(pk.data_ptr()) : nullptr, a.L, nt);
+                       has1 ? b1->data_ptr() : nullptr, has1 && b1->scalar_type() == at::kBFloat16, mask.data_ptr<float>(),
+                       reinterpret_cast<unsigned short*>(mask.data_ptr<float>() + rows * a.Lp), rows,
+                       pair ? reinterpret_cast<const T*>(b2->data_ptr()) : nullptr, pq,
+                       pair && backward ? pq + packed.numel() / 2 : nullptr, a.L, nt, mf::LOG2E / a.c);
   };
   if (pair && b2->scalar_type() == at::kBFloat16) pack((unsigned short*)nullptr);
   else pack((float*)nullptr);
   SXE_LAUNCH_CHECK();
-  return {mask, pq, pk};
+  return {mask, packed};
 }
 
-static void evo_set_packed(EvoCall& c, const at::Tensor& mask, const c10::optional<at::Tensor>& pq, const c10::optional<at::Tensor>& pk) {
-  c.a.b1 = mask.data_ptr<float>();
-  if (!evo_has(pq)) return;
-  c.pair = pq->scalar_type();
-  c.a.pq = pq->data_ptr();
-  c.a.pk = evo_has(pk) ? pk->data_ptr() : nullptr;
+static void evo_set_packed(EvoCall& c, const at::Tensor& mask, const c10::optional<at::Tensor>& pair) {
+  c.a.mask = mask.data_ptr<float>();
+  c.a.km = reinterpret_cast<const unsigned short*>(c.a.mask + mask.numel() / 9);
+  if (!evo_has(pair)) return;
+  c.pair = true;
+  c.a.pq = pair->data_ptr<float>();
+  c.a.pk = pair->size(0) == 2 ? c.a.pq + pair->numel() / 2 : nullptr;
 }
 
-// f(head dim constant, pair bias type tag)
+// f(head dim constant, with a pair bias or without)
 template <typename F>
-static void evo_dispatch(int D, at::ScalarType pair, F f) {
+static void evo_dispatch(int D, bool pair, F f) {
   auto with = [&](auto d) {
-    if (pair == at::kBFloat16) f(d, (unsigned short)0);
-    else if (pair == at::kFloat) f(d, 0.f);
-    else f(d, evo::NoBias{});
+    if (pair) f(d, std::true_type{});
+    else f(d, std::false_type{});
   };
   if (D == 32) with(std::integral_constant<int, 32>{});
   else with(std::integral_constant<int, 64>{});
 }
+
+static int evo_grid(const evo::Args& a, int rows) { return a.B * ((a.N + rows - 1) / rows) * a.H * (a.Lp / evo::QB); }
 
 // -> [o, lse, packed biases of evo_pack]: the backward reads these, not the biases, which the caller may have changed by then
 std::vector<at::Tensor> evoformer_fwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
@@ -611,17 +960,18 @@ std::vector<at::Tensor> evoformer_fwd(const at::Tensor& q, const at::Tensor& k, 
   EvoCall c = evo_call(q, k, v);
   evo::Args& a = c.a;
   auto packed = evo_pack(a, q.options(), b1, b2, backward);
-  evo_set_packed(c, packed[0], packed[1], packed[2]);
+  evo_set_packed(c, packed[0], packed[1]);
   auto o = at::empty_like(q);
   auto lse = at::empty({(int64_t)a.B * a.N, a.H, a.Lp}, q.options().dtype(at::kFloat));
-  const int grid = a.B * a.N * a.H * (a.Lp / evo::QB);
+  const int grid = evo_grid(a, 1);
   packed.insert(packed.begin(), {o, lse});
   if (grid == 0) return packed;
   a.lse = lse.data_ptr<float>();
   evo_dispatch(q.size(4), c.pair, [&](auto d, auto t) {
     constexpr int D = decltype(d)::value;
-    hipLaunchKernelGGL((evo::fwd_kernel<D, decltype(t)>), dim3(grid), dim3(256), 2 * (2 * evo::KT * 2 * D + evo::TAIL), cur_stream(),
-                       a, reinterpret_cast<unsigned short*>(o.data_ptr()));
+    constexpr int NN = 2, LDS = 2 * evo::Stream<D, NN>::SLOT;
+    hipLaunchKernelGGL((evo::fwd_kernel<D, decltype(t)::value, NN>), dim3(evo_grid(a, NN)), dim3(256), LDS, cur_stream(), a,
+                       reinterpret_cast<unsigned short*>(o.data_ptr()));
   });
   SXE_LAUNCH_CHECK();
   return packed;
@@ -629,38 +979,38 @@ std::vector<at::Tensor> evoformer_fwd(const at::Tensor& q, const at::Tensor& k, 
 
 std::vector<at::Tensor> evoformer_bwd(const at::Tensor& dout, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
                                       const at::Tensor& o, const at::Tensor& lse, const at::Tensor& mask,
-                                      const c10::optional<at::Tensor>& pq, const c10::optional<at::Tensor>& pk, bool need_db1,
-                                      bool need_db2) {
-  check_beside(q, {dout, k, v, o, lse, mask, pq, pk});
+                                      const c10::optional<at::Tensor>& pair, bool need_db1, c10::optional<at::ScalarType> db2_type) {
+  const bool need_db2 = db2_type.has_value();
+  check_beside(q, {dout, k, v, o, lse, mask, pair});
   c10::DeviceGuard g(q.device());
   EvoCall c = evo_call(q, k, v);
   evo::Args& a = c.a;
-  SXE_CHECK(mask.numel() == (int64_t)a.B * a.N * a.Lp && mask.scalar_type() == at::kFloat && mask.is_contiguous(),
-            "evoformer_bwd: mask as the forward packed it");
-  SXE_CHECK(evo_has(pq) == evo_has(pk), "evoformer_bwd: both forms of bias2");
-  if (evo_has(pq))
-    for (const at::Tensor* t : {&*pq, &*pk})
-      SXE_CHECK(t->numel() == (int64_t)a.B * a.H * a.Lp * a.Lp && t->is_contiguous() && t->scalar_type() == pq->scalar_type() &&
-                    (t->scalar_type() == at::kFloat || t->scalar_type() == at::kBFloat16) &&
-                    reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "evoformer_bwd: bias2 as the forward packed it");
-  evo_set_packed(c, mask, pq, pk);
+  auto packed = [](const at::Tensor& t, int64_t numel) {
+    return t.numel() == numel && t.scalar_type() == at::kFloat && t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  SXE_CHECK(packed(mask, 9 * (int64_t)a.B * a.N * a.Lp), "evoformer_bwd: mask as the forward packed it");
+  if (evo_has(pair))
+    SXE_CHECK(pair->dim() == 4 && pair->size(0) == 2 && packed(*pair, 2 * (int64_t)a.B * a.H * a.Lp * a.Lp),
+              "evoformer_bwd: bias2 as the forward packed it, in both forms");
+  SXE_CHECK(!need_db2 || *db2_type == at::kFloat || *db2_type == at::kBFloat16, "evoformer_bwd: gradient of bias2 in fp32 / bf16");
+  evo_set_packed(c, mask, pair);
   for (const at::Tensor* t : {&dout, &o})
     SXE_CHECK(t->sizes() == q.sizes() && t->is_contiguous() && t->scalar_type() == at::kBFloat16, "evoformer_bwd: dout / o like q");
   SXE_CHECK(lse.numel() == (int64_t)a.B * a.N * a.H * a.Lp && lse.scalar_type() == at::kFloat && lse.is_contiguous(),
             "evoformer_bwd: lse fp32 [B*N, H, Lp]");
-  SXE_CHECK(!need_db2 || evo_has(pq), "evoformer_bwd: gradient of a bias2 that is not there");
+  SXE_CHECK(!need_db2 || evo_has(pair), "evoformer_bwd: gradient of a bias2 that is not there");
   const at::Tensor d = evo_aligned(dout), oo = evo_aligned(o);
-  auto stats = at::empty({2, lse.numel()}, lse.options());
+  auto stats = at::empty({2, lse.numel(), 16}, q.options());
   a.dout = reinterpret_cast<const unsigned short*>(d.data_ptr());
   a.o = reinterpret_cast<const unsigned short*>(oo.data_ptr());
   a.lse = lse.data_ptr<float>();
-  a.lse2 = stats.data_ptr<float>();
-  a.ndelta = a.lse2 + lse.numel();
+  a.sl = reinterpret_cast<unsigned short*>(stats.data_ptr());
+  a.sd = a.sl + 16 * lse.numel();
   auto dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
   at::Tensor db1, db2;
   if (need_db1) db1 = at::zeros({a.B, a.N, 1, 1, a.L}, q.options().dtype(at::kFloat));
-  if (need_db2) db2 = at::empty({a.B, 1, a.H, a.L, a.L}, pq->options());
-  const int grid = a.B * a.N * a.H * (a.Lp / evo::QB);
+  if (need_db2) db2 = at::empty({a.B, 1, a.H, a.L, a.L}, q.options().dtype(*db2_type));
+  const int grid = evo_grid(a, 1);
   if (grid == 0) {
     if (need_db2) db2.zero_();
     return {dq, dk, dv, need_db1 ? db1 : at::Tensor(), need_db2 ? db2 : at::Tensor()};
@@ -670,20 +1020,54 @@ std::vector<at::Tensor> evoformer_bwd(const at::Tensor& dout, const at::Tensor& 
   auto* dvp = reinterpret_cast<unsigned short*>(dv.data_ptr());
   evo_dispatch(q.size(4), c.pair, [&](auto dd, auto t) {
     constexpr int D = decltype(dd)::value;
-    using BT = decltype(t);
-    const size_t lds = 2 * (2 * evo::KT * 2 * D + evo::TAIL);
-    hipLaunchKernelGGL((evo::dq_kernel<D, BT>), dim3(grid), dim3(256), lds, cur_stream(), a, dqp);
-    hipLaunchKernelGGL((evo::dkdv_kernel<D, BT>), dim3(grid), dim3(256), lds, cur_stream(), a, dkp, dvp,
-                       need_db1 ? db1.data_ptr<float>() : nullptr);
-    if constexpr (!std::is_same<BT, evo::NoBias>::value) if (need_db2) {
+    constexpr bool PAIR = decltype(t)::value;
+    constexpr int NN = 2, NK = D == 32 ? 2 : 1, LDS = 2 * evo::Stream<D, NN>::SLOT, LDSK = 2 * evo::QueryStream<D, NK>::SLOT;
+    bool both = false;
+    if constexpr (PAIR && D == 32) {
+      both = need_db2 && a.L <= 384;
+      auto run = [&](auto cfg, auto kernel, int queries) {
+        constexpr int LDSB = decltype(cfg)::LDS;
+        static std::atomic<uint64_t> done{0};
+        on_each_device(done, [&] {
+          SXE_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, LDSB));
+        });
+        const int wgs = (a.L + queries - 1) / queries * a.B * a.H, most = std::max(1, std::min(a.N, kNumCUs / wgs));
+        const int rows_per = (a.N + most - 1) / most, parts = (a.N + rows_per - 1) / rows_per;
+        const int64_t stride = (int64_t)a.B * a.H * a.Lp * a.Lp;
+        auto part = at::empty({parts, stride}, q.options().dtype(at::kFloat));
+        hipLaunchKernelGGL(kernel, dim3(wgs, parts), dim3(512), LDSB, cur_stream(), a, dqp, part.template data_ptr<float>(), rows_per);
+        const int tl = (a.L + 31) / 32;
+        const dim3 gs(tl * tl, a.B * a.H);
+        if (db2.scalar_type() == at::kFloat)
+          hipLaunchKernelGGL(evo::dpair_tiles_kernel<float>, gs, dim3(256), 0, cur_stream(), part.template data_ptr<float>(),
+                             db2.data_ptr<float>(), stride, parts, a.L, a.Lp / 32);
+        else
+          hipLaunchKernelGGL(evo::dpair_tiles_kernel<unsigned short>, gs, dim3(256), 0, cur_stream(), part.template data_ptr<float>(),
+                             reinterpret_cast<unsigned short*>(db2.data_ptr()), stride, parts, a.L, a.Lp / 32);
+      };
+      if (both) {
+        if (a.L <= 128) run(evo::DqPair<2, 4, 1>{}, evo::dq_pair_kernel<2, 4, 1>, 64);
+        else if (a.L <= 256) run(evo::DqPair<2, 4, 2>{}, evo::dq_pair_kernel<2, 4, 2>, 64);
+        else run(evo::DqPair<2, 4, 3>{}, evo::dq_pair_kernel<2, 4, 3>, 64);
+      }
+    }
+    if (!both) hipLaunchKernelGGL((evo::dq_kernel<D, PAIR, NN>), dim3(evo_grid(a, NN)), dim3(256), LDS, cur_stream(), a, dqp);
+    auto dkdv = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(evo_grid(a, NK)), dim3(256), LDSK, cur_stream(), a, dkp, dvp,
+                         need_db1 ? db1.data_ptr<float>() : nullptr);
+    };
+    if (need_db1) dkdv(evo::dkdv_kernel<D, PAIR, NK, true>);
+    else dkdv(evo::dkdv_kernel<D, PAIR, NK, false>);
+    if constexpr (PAIR) if (need_db2 && !both) {
+      constexpr int LDSP = 2 * evo::QueryStream<D, 1>::SLOT;
       // as many parts as all run at once (a part of at least 8 rows): a second, part-filled round costs more than the
       // longer walk
       const int wgs = (a.L + evo::KT - 1) / evo::KT * (a.Lp / evo::QB) * a.B * a.H;
-      const int most = std::max(1, std::min((a.N + 7) / 8, evo::min_waves<D, BT>() * kNumCUs / wgs));
+      const int most = std::max(1, std::min((a.N + 7) / 8, evo::min_waves<D>() * kNumCUs / wgs));
       const int rows_per = (a.N + most - 1) / most, parts = (a.N + rows_per - 1) / rows_per;
       const bool direct = parts == 1 && db2.scalar_type() == at::kFloat;
       auto part = direct ? db2 : at::empty({parts, db2.numel()}, q.options().dtype(at::kFloat));
-      hipLaunchKernelGGL((evo::dpair_kernel<D, BT>), dim3(wgs, parts), dim3(256), lds, cur_stream(), a, part.template data_ptr<float>(),
+      hipLaunchKernelGGL((evo::dpair_kernel<D>), dim3(wgs, parts), dim3(256), LDSP, cur_stream(), a, part.template data_ptr<float>(),
                          rows_per);
       if (!direct) {
         const dim3 gs(stream_grid(db2.numel(), 256));
@@ -704,8 +1088,8 @@ std::vector<at::Tensor> evoformer_bwd(const at::Tensor& dout, const at::Tensor& 
 
 TORCH_LIBRARY_FRAGMENT(sxe, m) {
   m.def("evoformer_fwd(Tensor q, Tensor k, Tensor v, Tensor? bias1, Tensor? bias2, bool backward=False) -> Tensor[]");
-  m.def("evoformer_bwd(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, Tensor mask, Tensor? pq, Tensor? pk, "
-        "bool need_db1, bool need_db2) -> Tensor[]");
+  m.def("evoformer_bwd(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, Tensor mask, Tensor? pair, "
+        "bool need_db1, ScalarType? db2) -> Tensor[]");
 }
 TORCH_LIBRARY_IMPL(sxe, CUDA, m) {
   m.impl("evoformer_fwd", &sxe::evoformer_fwd);

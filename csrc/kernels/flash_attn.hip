@@ -1344,16 +1344,6 @@ static void set_lds_limit(F* f, size_t bytes) {
   SXE_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)bytes));
 }
-// the opt-ins `f` of a kernel family, once on every device of the process
-template <typename F>
-static void on_each_device(std::atomic<uint64_t>& done, F f) {
-  int dev = 0;
-  SXE_HIP_CHECK(hipGetDevice(&dev));
-  if (dev < 64 && (done.load(std::memory_order_relaxed) >> dev & 1)) return;
-  f();
-  if (dev < 64) done.fetch_or(1ull << dev, std::memory_order_relaxed);
-}
-
 // kv_len: valid keys (the rest of the padded key axis is masked); qoff: causal offset (query i sees
 // keys <= i + qoff), default Sk - Sq (bottom-right aligned)
 template <int D>

@@ -69,17 +69,20 @@ class EvoformerFusedAttention(torch.autograd.Function):
     def forward(ctx, q, k, v, bias1=None, bias2=None):
         q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
         # the packed biases are what the backward reads: the biases themselves may change between the two
-        o, lse, mask, pq, pk = torch.ops.sxe.evoformer_fwd(q, k, v, _bias(bias1), _bias(bias2), any(ctx.needs_input_grad))
-        ctx.save_for_backward(q, k, v, o, lse, mask, pq, pk)
+        b1, b2 = _bias(bias1), _bias(bias2)
+        o, lse, mask, pair = torch.ops.sxe.evoformer_fwd(q, k, v, b1, b2, any(ctx.needs_input_grad))
+        ctx.save_for_backward(q, k, v, o, lse, mask, pair)
+        ctx.pair_dtype = None if b2 is None else b2.dtype
         ctx.bias_dtypes = (bias1.dtype if bias1 is not None else None, bias2.dtype if bias2 is not None else None)
         return o
 
     @staticmethod
     def backward(ctx, do):
-        q, k, v, o, lse, mask, pq, pk = ctx.saved_tensors
+        q, k, v, o, lse, mask, pair = ctx.saved_tensors
         need1 = ctx.bias_dtypes[0] is not None and ctx.needs_input_grad[3]
         need2 = ctx.bias_dtypes[1] is not None and ctx.needs_input_grad[4]
-        dq, dk, dv, db1, db2 = torch.ops.sxe.evoformer_bwd(do.contiguous().to(q.dtype), q, k, v, o, lse, mask, pq, pk, need1, need2)
+        dq, dk, dv, db1, db2 = torch.ops.sxe.evoformer_bwd(do.contiguous().to(q.dtype), q, k, v, o, lse, mask, pair, need1,
+                                                           ctx.pair_dtype if need2 else None)
         db1 = db1.to(ctx.bias_dtypes[0]) if need1 else None
         db2 = db2.to(ctx.bias_dtypes[1]) if need2 else None
         return dq, dk, dv, db1, db2

@@ -148,3 +148,28 @@ def test_evoformer_without_gradients():
     assert want.requires_grad and not ea.evoformer_attention(Q, K, V, b1).requires_grad
     with fwAD.dual_level(), pytest.raises((RuntimeError, NotImplementedError)):
         ea.evoformer_attention(fwAD.make_dual(Q, torch.ones_like(Q)), K, V, b1, None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,L", [(32, 127), (32, 128), (32, 129), (32, 256), (32, 257), (32, 383), (32, 384), (32, 385), (64, 65), (64, 257)])
+@pytest.mark.parametrize("N", [1, 2, 7])
+def test_evoformer_key_blocks(D, L, N):
+    """Edges of the key blocks that dQ and the pair bias' gradient share, odd and even numbers of rows, and a row whose keys are all
+    masked by the same finite number: its softmax is that of the other terms."""
+    torch.manual_seed(4)
+    B, H = 2, 3
+    mk = lambda *s: torch.randn(*s, device="cuda")
+    Q, K, V, g = (mk(B, N, L, H, D).bfloat16() for _ in range(4))
+    b1 = (mk(B, N, 1, 1, L) > 1).float() * -1e9
+    b1[..., 0] = 0
+    b1[1, N - 1] = -1e9
+    ins = [t.requires_grad_(True) for t in (Q, K, V, b1, (mk(B, 1, H, L, L) * 2).bfloat16())]
+    out = ea.evoformer_attention(*ins)
+    grads = torch.autograd.grad(out, ins, g)
+    ref = [t.detach().double().requires_grad_(True) for t in ins]
+    q, k, v = (t.transpose(-2, -3) for t in ref[:3])
+    want = (torch.softmax(q @ k.transpose(-1, -2) / D ** 0.5 + ref[3] + ref[4], -1) @ v).transpose(-2, -3)
+    # as above: p, ds and the results are rounded to 8 bits, 4 x 2^-9
+    assert (out.double() - want).norm() <= 8e-3 * want.norm()
+    for a, b in zip(grads, torch.autograd.grad(want, ref, g.double())):
+        assert torch.isfinite(a).all() and (a.double() - b).norm() <= 8e-3 * b.norm(), a.shape
