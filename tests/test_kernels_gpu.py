@@ -73,6 +73,31 @@ def test_multi_tensor_adam_matches_flat():
         assert _rel(p, r) < 1e-5
 
 
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("gdt", [torch.float32, torch.bfloat16])
+def test_multi_tensor_adam_sizes(offset, gdt):
+    """Edges of a workgroup's 1024 and an entry's 65536 elements, tensors that start on 16 bytes and 4 bytes behind; what lies
+    between the tensors stays."""
+    torch.manual_seed(1)
+    sizes = [1, 3, 4, 1021, 1023, 1024, 1025, 4099, 65535, 65536, 65537, 131073]
+    room = [torch.randn(n + 8, device="cuda") for n in sizes]
+    cut = lambda ts: [t[4 + offset:4 + offset + n] for t, n in zip(ts, sizes)]
+    m, v = [torch.zeros_like(t) for t in room], [torch.zeros_like(t) for t in room]
+    lp = [torch.zeros_like(t, dtype=torch.bfloat16) for t in room]
+    g = [torch.randn_like(t).to(gdt) for t in room]
+    before = [t.clone() for t in room]
+    torch.ops.sxe.multi_tensor_adam_(cut(room), cut(g), cut(m), cut(v), cut(lp), None, None, 1e-2, 0.9, 0.95, 1e-8, 0.1, 1, True, True, 1.0)
+    for t, b, gr, h, mm, vv in zip(cut(room), cut(before), cut(g), cut(lp), cut(m), cut(v)):
+        gd = gr.double()
+        want = b.double() * (1 - 1e-3) - 1e-2 * gd / (gd.abs() + 1e-8)
+        # a handful of fp32 roundings, and those of the moments' corrections, which the update of 1e-2 sees: 16 ulp of the larger
+        assert (t.double() - want).abs().max() <= 16 * 2.0 ** -24 * want.abs().max().clamp_min(1)
+        assert torch.equal(h, t.bfloat16())
+        assert (mm.double() - 0.1 * gd).norm() <= 1e-6 * gd.norm() and (vv.double() - 0.05 * gd * gd).norm() <= 1e-6 * (gd * gd).norm()
+    for t, b, n in zip(room, before, sizes):
+        assert torch.equal(t[:4 + offset], b[:4 + offset]) and torch.equal(t[4 + offset + n:], b[4 + offset + n:])
+
+
 @pytest.mark.parametrize("H", [128, 1000, 4096, 8192])
 @pytest.mark.parametrize("residual", [False, True])
 @pytest.mark.parametrize("rows", [1, 185, 300])  # <= 256 rows and H >= 1024: block-per-row forward
