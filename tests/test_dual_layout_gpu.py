@@ -165,3 +165,16 @@ def test_acc2_bf16_kernel():
     assert torch.equal(d, ref)
     torch.ops.sxe.acc2_bf16_(d, a, b, False)
     assert torch.equal(d, a.float() + b.float())
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 1023, 2047, 2048, 2049, 4100, 100003])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_acc2_bf16_sizes(n, accumulate):
+    """Edges of a workgroup's 2048 elements; what lies behind the operands stays."""
+    torch.manual_seed(0)
+    room = torch.randn(n + 8, device="cuda")
+    a, b = (torch.randn(n + 8, device="cuda").bfloat16() for _ in range(2))
+    want = room.clone()
+    want[:n] = (want[:n] if accumulate else 0) + a[:n].float() + b[:n].float()
+    torch.ops.sxe.acc2_bf16_(room[:n], a[:n], b[:n], accumulate)
+    assert torch.equal(room, want)
