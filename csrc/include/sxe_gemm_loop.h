@@ -162,5 +162,18 @@ __device__ __forceinline__ void store_lines(unsigned short* y, int64_t ld, int r
   }
 }
 
+// zeros to a tile of y: rows x cols (a multiple of 8) from `y` on
+__device__ __forceinline__ void clear_tile(unsigned short* y, int64_t ld, int rows, int cols) {
+  const int per = cols / 8;
+  for (int i = threadIdx.x; i < rows * per; i += blockDim.x) *reinterpret_cast<u32x4*>(y + (i / per) * ld + i % per * 8) = u32x4{0u, 0u, 0u, 0u};
+}
+
 }  // namespace gl
+
+// rows in use of each of `n` blocks of rows, or null
+inline const int* used_rows(const c10::optional<at::Tensor>& t, int64_t n) {
+  if (!t.has_value() || !t->defined()) return nullptr;
+  SXE_CHECK(t->is_cuda() && t->scalar_type() == at::kInt && t->is_contiguous() && t->numel() == n, "rows in use: int32, one number for each of ", n);
+  return t->data_ptr<int>();
+}
 }  // namespace sxe

@@ -2,7 +2,8 @@
 // row counts read on the device.
 //   expert_swiglu_kn_tile  h[r] = silu(x[token r] . Wg) * (x[token r] . Wu),  W = [E, K, gate | up]
 //   expert_down_kn_tile    y[r] = h[r] . W[E, K, N]
-//   expert_mm_kn           y[e] = x[e] . W[e], x [E, C, K]: the same number of rows for all (training with a capacity)
+//   expert_mm_kn           y[e] = x[e] . W[e], x [E, C, K]: the same number of rows for all (training with a capacity); the rows behind
+//                          those in use are cleared, not multiplied
 //
 // Reference: inference/v2/kernels/cutlass_ops/moe_gemm/moe_gemm.cu (grouped GEMM over expert-sorted rows). experts_kn.hip has the
 // streaming form for few rows an expert.
@@ -32,6 +33,7 @@ struct Args {
   const unsigned short* w;
   const int* offs;  // [E + 1]; null: C rows an expert
   int C;
+  const int* rows;  // [E] of the C rows that are not zeros, the first ones; null: all
   unsigned short* y;
   int E, R, K, N;    // N: columns of W
   int cols, half;    // columns of y; column of W that goes with column 0 in the second half of a tile
@@ -92,6 +94,12 @@ __global__ void __launch_bounds__(T::NTHR, T::WAVES) tile_kernel(Args a) {
   const int local = id - __builtin_amdgcn_readfirstlane(first) * tn, nt = local / te, rt = local - nt * te;
   const int r0 = row_of(a, expert) + rt * BM, r1 = row_of(a, expert + 1);
   const int n0 = nt * CB;
+  int used = r1 - r0;  // rows of the tile with products
+  if (a.rows != nullptr) used = __builtin_amdgcn_readfirstlane(min(used, a.rows[expert] - rt * BM));
+  if (used <= 0 && a.rows != nullptr) {
+    clear_tile(a.y + (int64_t)r0 * a.cols + n0, a.cols, min(BM, r1 - r0), min(CB, a.cols - n0));
+    return;
+  }
 
   // ---- loads: 8 rows of x, chunk c of row r at place c ^ ((r >> 1) & 7); 2 k rows of W, chunk c of row k at place
   // c ^ (4 (k & 3) + 2 ((k >> 3) & 1)). Slabs behind the last repeat it; the second half of one with 32 k repeats its first
@@ -145,8 +153,8 @@ __global__ void __launch_bounds__(T::NTHR, T::WAVES) tile_kernel(Args a) {
   };
 
   f32x4 acc[RT][CT];
-  const int live = __builtin_amdgcn_readfirstlane(min(max((r1 - r0 - wr * RT * 16 + 15) / 16, 0), RT));
-  loop<T>(acc, ns, half, r1 - r0 >= BM, live, load_x, load_w, read_x, read_w);
+  const int live = __builtin_amdgcn_readfirstlane(min(max((used - wr * RT * 16 + 15) / 16, 0), RT));
+  loop<T>(acc, ns, half, used >= BM, live, load_x, load_w, read_x, read_w);
 
   // two blocks' four columns a lane -> eight of one: lanes of odd groups of 16 take the second block
   auto pair = [&](const float (&u)[4], const float (&v)[4]) {
@@ -258,8 +266,9 @@ at::Tensor expert_down_kn_tile(const at::Tensor& h, const at::Tensor& w, const a
   return y;
 }
 
-// x [E, C, K], w [E, K, N] -> [E, C, N]
-at::Tensor expert_mm_kn(const at::Tensor& x, const at::Tensor& w) {
+// x [E, C, K], w [E, K, N] -> [E, C, N]; used int32 [E]: x[e, used[e]:] is zeros, and so is y
+at::Tensor expert_mm_kn(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& used) {
+  check_beside(x, {w, used});
   SXE_CHECK(x.dim() == 3 && x.is_contiguous() && w.dim() == 3 && x.size(0) == w.size(0) && x.device() == w.device() && x.numel() < (1ll << 40) &&
                 x.size(0) * x.size(1) < (1ll << 31), "expert_mm_kn: x [E, C, K], w [E, K, N]");
   const at::Tensor rows = x.view({-1, x.size(2)});
@@ -268,6 +277,7 @@ at::Tensor expert_mm_kn(const at::Tensor& x, const at::Tensor& w) {
   if (y.numel() == 0) return y;
   c10::DeviceGuard g(x.device());
   a.C = x.size(1);
+  a.rows = used_rows(used, w.size(0));
   a.R = a.X;
   a.y = reinterpret_cast<unsigned short*>(y.data_ptr());
   a.cols = a.N;
@@ -280,7 +290,7 @@ at::Tensor expert_mm_kn(const at::Tensor& x, const at::Tensor& w) {
 TORCH_LIBRARY_FRAGMENT(sxe, m) {
   m.def("expert_swiglu_kn_tile(Tensor x, Tensor w, Tensor offs, Tensor token) -> Tensor");
   m.def("expert_down_kn_tile(Tensor h, Tensor w, Tensor offs) -> Tensor");
-  m.def("expert_mm_kn(Tensor x, Tensor w) -> Tensor");
+  m.def("expert_mm_kn(Tensor x, Tensor w, Tensor? rows=None) -> Tensor");
 }
 TORCH_LIBRARY_IMPL(sxe, CUDA, m) {
   m.impl("expert_swiglu_kn_tile", &sxe::expert_swiglu_kn_tile);

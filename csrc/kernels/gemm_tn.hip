@@ -27,6 +27,7 @@ constexpr int ROW = 2 * BK;
 struct Args {
   const unsigned short *x, *w, *bias;
   unsigned short* y;
+  const int* rows;       // of a batch: rows of each product that are not zeros, the first ones; null: all
   float* part;           // splits of K: their sums, [splits, M, N]
   int64_t ldx, ldw, bx, bw, by;  // elements from row to row, and from product to product of a batch
   int M, cols, half, slabs, per, parts;  // columns of y (SwiGLU: half the rows of w); w row that goes with row 0 as up; slabs of K, of a split;
@@ -56,6 +57,14 @@ __global__ void __launch_bounds__(T::NTHR, T::WAVES) gemm_kernel(Args a) {
   const int per_group = a.gm * a.tn, group = tile / per_group, in = tile - group * per_group, rows = min(a.tm - group * a.gm, a.gm);
   const int m0 = (rest ? a.tm : group * a.gm + in % rows) * BM, n0 = (rest ? tile : in / rows) * CB;
   const int first = SPLIT ? part * a.per : 0, ns = SPLIT ? min(a.per, a.slabs - first) : a.slabs;
+  int used = a.M - m0;  // rows of the tile with products
+  if (!SPLIT && a.rows != nullptr) {
+    used = __builtin_amdgcn_readfirstlane(min(used, a.rows[part] - m0));
+    if (used <= 0) {
+      clear_tile(a.y + part * a.by + (int64_t)m0 * a.cols + n0, a.cols, min(BM, a.M - m0), min(CB, a.cols - n0));
+      return;
+    }
+  }
 
   // ---- loads: a wave's load is 8 rows, chunk c of row r at place c ^ ((r >> 1) & 7). Rows and columns behind the last, and slabs,
   // repeat it
@@ -90,8 +99,8 @@ __global__ void __launch_bounds__(T::NTHR, T::WAVES) gemm_kernel(Args a) {
 
   f32x4 acc[RT][CT];
   // a tile of fewer rows skips the products of the others
-  const int live = __builtin_amdgcn_readfirstlane(min(max((a.M - m0 - wr * RT * 16 + 15) / 16, 0), RT));
-  loop<T>(acc, ns, false, !rest, live, load_x, load_w, read_x, read_w);
+  const int live = __builtin_amdgcn_readfirstlane(min(max((used - wr * RT * 16 + 15) / 16, 0), RT));
+  loop<T>(acc, ns, false, used >= BM, live, load_x, load_w, read_x, read_w);
 
   if constexpr (SPLIT || GLU) {
 #pragma unroll
@@ -244,8 +253,8 @@ static void launch(Args a, int splits, int batch) {
 
 // x, w [.., rows, K], one product or a batch; out: y's sizes where they are not those of one product
 static at::Tensor gemm_tn_run(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, bool glu, int64_t tile, int64_t splits,
-                              at::IntArrayRef out = {}) {
-  check_beside(x, {w, bias});
+                              at::IntArrayRef out = {}, const c10::optional<at::Tensor>& rows = c10::nullopt) {
+  check_beside(x, {w, bias, rows});
   const int64_t d = x.dim() - 2, batch = d ? x.size(0) : 1, M = x.size(d), K = x.size(d + 1), N = w.size(d), cols = glu ? N / 2 : N;
   SXE_CHECK(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 && w.size(d + 1) == K && (!d || w.size(0) == batch),
             "gemm_tn: bf16 x [M, K], w [N, K]");
@@ -271,6 +280,7 @@ static at::Tensor gemm_tn_run(const at::Tensor& x, const at::Tensor& w, const c1
   a.y = reinterpret_cast<unsigned short*>(y.data_ptr());
   a.ldx = ldx;
   a.ldw = ldw;
+  a.rows = used_rows(rows, batch);
   if (d) {
     a.bx = x.stride(0);
     a.bw = w.stride(0);
@@ -317,17 +327,17 @@ at::Tensor gemm_tn(const at::Tensor& x, const at::Tensor& w, const c10::optional
   return gemm_tn_run(x.view({-1, x.size(-1)}), w, bias, glu, tile, splits, out);
 }
 
-// x [B, M, K], w [B, N, K] -> [B, M, N], one launch
-at::Tensor gemm_tn_batch(const at::Tensor& x, const at::Tensor& w, int64_t tile) {
+// x [B, M, K], w [B, N, K] -> [B, M, N], one launch; rows int32 [B]: x[b, rows[b]:] is zeros, and so is y
+at::Tensor gemm_tn_batch(const at::Tensor& x, const at::Tensor& w, int64_t tile, const c10::optional<at::Tensor>& rows) {
   SXE_CHECK(x.dim() == 3 && w.dim() == 3, "gemm_tn_batch: bf16 x [B, M, K], w [B, N, K]");
-  return gemm_tn_run(x, w, c10::nullopt, false, tile, 1);
+  return gemm_tn_run(x, w, c10::nullopt, false, tile, 1, {}, rows);
 }
 
 }  // namespace sxe
 
 TORCH_LIBRARY_FRAGMENT(sxe, m) {
   m.def("gemm_tn(Tensor x, Tensor w, Tensor? bias, bool glu, int tile=-1, int splits=0) -> Tensor");
-  m.def("gemm_tn_batch(Tensor x, Tensor w, int tile=-1) -> Tensor");
+  m.def("gemm_tn_batch(Tensor x, Tensor w, int tile=-1, Tensor? rows=None) -> Tensor");
 }
 TORCH_LIBRARY_IMPL(sxe, CUDA, m) {
   m.impl("gemm_tn", &sxe::gemm_tn);

@@ -25,6 +25,7 @@ using namespace gl;
 
 struct Args {
   const unsigned short *a, *b, *a2, *b2;  // first and second piece of the tokens
+  const int *rows, *rows2;                // tokens of each expert's piece that are not zeros, the first ones; null: all
   float *c, *part;                        // part: sums of the splits, [splits, M, N]
   int64_t lda, ldb, ldc;
   int64_t ba, bb, ba2, bb2, bc;           // elements from expert to expert
@@ -54,8 +55,20 @@ __global__ void __launch_bounds__(T::NTHR, T::WAVES) wgrad_kernel(Args a) {
   const int nt = rest ? a.tn : a.tm * a.tn, part = a.parts > 1 ? id / nt : 0, tile = id - part * nt;
   const int per_group = a.gm * a.tn, group = tile / per_group, in = tile - group * per_group, rows = min(a.tm - group * a.gm, a.gm);
   const int m0 = (rest ? a.tm : group * a.gm + in % rows) * BM, n0 = (rest ? tile : in / rows) * BN;
-  const int first = SPLIT ? part * a.per : 0, ns = SPLIT ? min(a.per, a.slabs - first) : a.slabs;
   const int expert = SPLIT ? 0 : part;
+  // slabs with tokens other than zeros: of the first piece, of both
+  int n1 = a.n1, slabs = a.slabs, tails[2] = {a.tail, a.tail2};
+  if (!SPLIT && (a.rows != nullptr || a.rows2 != nullptr)) {
+    auto in_use = [&](const int* rows, int n, int& tail) {
+      if (rows == nullptr) return n;
+      const int used = __builtin_amdgcn_readfirstlane(max(rows[expert], 0));
+      if (used <= n * BK) tail = 0;
+      return min(n, (used + BK - 1) / BK);
+    };
+    n1 = in_use(a.rows, a.n1, tails[0]);
+    slabs = n1 + in_use(a.rows2, a.slabs - a.n1, tails[1]);
+  }
+  const int first = SPLIT ? part * a.per : 0, ns = SPLIT ? min(a.per, slabs - first) : slabs;
 
   // ---- loads: a wave's are XK (WK) tokens; columns behind the last repeat it
   const int xk = XK * w + lane / XL, wk = WK * w + lane / WL;
@@ -64,8 +77,8 @@ __global__ void __launch_bounds__(T::NTHR, T::WAVES) wgrad_kernel(Args a) {
   const unsigned xo = (unsigned)xk * (unsigned)(2 * a.lda) + xc, wo = (unsigned)wk * (unsigned)(2 * a.ldb) + wcol;
   const unsigned short *pa = a.a + expert * a.ba, *pb = a.b + expert * a.bb, *pa2 = a.a2 + expert * a.ba2, *pb2 = a.b2 + expert * a.bb2;
   const unsigned l0 = lds_base();
-  auto tokens_a = [&](int slab) { return slab < a.n1 ? pa + (int64_t)slab * BK * a.lda : pa2 + (int64_t)(slab - a.n1) * BK * a.lda; };
-  auto tokens_b = [&](int slab) { return slab < a.n1 ? pb + (int64_t)slab * BK * a.ldb : pb2 + (int64_t)(slab - a.n1) * BK * a.ldb; };
+  auto tokens_a = [&](int slab) { return slab < n1 ? pa + (int64_t)slab * BK * a.lda : pa2 + (int64_t)(slab - n1) * BK * a.lda; };
+  auto tokens_b = [&](int slab) { return slab < n1 ? pb + (int64_t)slab * BK * a.ldb : pb2 + (int64_t)(slab - n1) * BK * a.ldb; };
   auto load_x = [&](int i, int slab, unsigned slot) {
     glds(xo, tokens_a(first + min(slab, ns - 1)) + (int64_t)(i * NW * XK) * a.lda, l0 + slot + (i * NW + w) * 1024);
   };
@@ -98,8 +111,8 @@ __global__ void __launch_bounds__(T::NTHR, T::WAVES) wgrad_kernel(Args a) {
   // less than a slab of tokens at the end of a piece: zeros behind them, in both operands
 #pragma unroll 1
   for (int piece = 0; piece < 2; ++piece) {
-    const int tail = piece ? a.tail2 : a.tail;
-    if (tail == 0 || first + ns != a.slabs) continue;
+    const int tail = tails[piece];
+    if (tail == 0 || first + ns != slabs) continue;
     __builtin_amdgcn_s_barrier();  // nobody reads the slots any more, and no load writes them
     asm volatile("" ::: "memory");
     const unsigned short* ta = piece ? pa2 + (int64_t)(a.slabs - a.n1) * BK * a.lda : pa + (int64_t)a.n1 * BK * a.lda;
@@ -254,8 +267,9 @@ static void check_tokens(const at::Tensor& t, int64_t d, const char* name) {
 static int64_t row_stride(const at::Tensor& t, int64_t d) { return t.size(d) > 1 ? t.stride(d) : t.size(d + 1); }
 
 static void run(const at::Tensor& x, const at::Tensor& y, const at::Tensor* x2, const at::Tensor* y2, at::Tensor c, double alpha, bool accumulate,
-                int64_t tile, int64_t splits) {
-  check_beside(x, {y, c});
+                int64_t tile, int64_t splits, const c10::optional<at::Tensor>& rows = c10::nullopt,
+                const c10::optional<at::Tensor>& rows2 = c10::nullopt) {
+  check_beside(x, {y, c, rows, rows2});
   const int64_t d = c.dim() - 2;
   SXE_CHECK(d == 0 || d == 1, "wgrad_gemm: C [M, N] or [E, M, N]");
   check_tokens(x, d, "A");
@@ -284,6 +298,10 @@ static void run(const at::Tensor& x, const at::Tensor& y, const at::Tensor* x2, 
     a.bb = y.stride(0);
     a.bc = c.stride(0);
   }
+  if (d) {  // of experts only
+    a.rows = used_rows(rows, experts);
+    a.rows2 = used_rows(rows2, experts);
+  }
   a.n1 = x.size(d) / BK;
   a.slabs = a.n1;
   a.tail = x.size(d) % BK;
@@ -294,8 +312,8 @@ static void run(const at::Tensor& x, const at::Tensor& y, const at::Tensor* x2, 
     SXE_CHECK(x2->size(d + 1) == M && y2->size(d + 1) == N && x2->size(d) == y2->size(d) && (!d || (x2->size(0) == experts && y2->size(0) == experts)) &&
                   x2->size(d) < (1ll << 30) && x.size(d) < (1ll << 30), "wgrad_gemm: pieces of the same columns");
     if (row_stride(*x2, d) != a.lda || row_stride(*y2, d) != a.ldb) {  // one after the other
-      run(x, y, nullptr, nullptr, c, alpha, accumulate, tile, splits);
-      run(*x2, *y2, nullptr, nullptr, c, alpha, true, tile, splits);
+      run(x, y, nullptr, nullptr, c, alpha, accumulate, tile, splits, rows);
+      run(*x2, *y2, nullptr, nullptr, c, alpha, true, tile, splits, rows2);
       return;
     }
     a.a2 = reinterpret_cast<const unsigned short*>(x2->data_ptr());
@@ -331,8 +349,9 @@ static void run(const at::Tensor& x, const at::Tensor& y, const at::Tensor* x2, 
 }  // namespace wg
 
 // c (+)= alpha * a' b, a [T, M], b [T, N], c [M, N], or all with a leading expert index
-void wgrad_gemm_(const at::Tensor& a, const at::Tensor& b, at::Tensor c, double alpha, bool accumulate) {
-  wg::run(a, b, nullptr, nullptr, c, alpha, accumulate, -1, 0);
+// (rows int32 [E]: a[e, rows[e]:] or b[e, rows[e]:] is zeros, as far as 64 tokens go from there on both are)
+void wgrad_gemm_(const at::Tensor& a, const at::Tensor& b, at::Tensor c, double alpha, bool accumulate, const c10::optional<at::Tensor>& rows) {
+  wg::run(a, b, nullptr, nullptr, c, alpha, accumulate, -1, 0, rows);
 }
 // The same with a tile (0: 256 x 256, 1: 128 x 256, else the plan's) and splits of the tokens (0: the plan's) of the caller's, for comparisons
 void wgrad_gemm_variant_(const at::Tensor& a, const at::Tensor& b, at::Tensor c, double alpha, bool accumulate, int64_t variant) {
@@ -341,16 +360,17 @@ void wgrad_gemm_variant_(const at::Tensor& a, const at::Tensor& b, at::Tensor c,
 }
 // c (+)= alpha * [a; a2]' [b; b2] (one after the other along the tokens) without the concatenation
 void wgrad_gemm2_(const at::Tensor& a, const at::Tensor& b, const at::Tensor& a2, const at::Tensor& b2, at::Tensor c, double alpha,
-                  bool accumulate) {
-  wg::run(a, b, &a2, &b2, c, alpha, accumulate, -1, 0);
+                  bool accumulate, const c10::optional<at::Tensor>& rows, const c10::optional<at::Tensor>& rows2) {
+  wg::run(a, b, &a2, &b2, c, alpha, accumulate, -1, 0, rows, rows2);
 }
 
 }  // namespace sxe
 
 TORCH_LIBRARY_FRAGMENT(sxe, m) {
-  m.def("wgrad_gemm_(Tensor a, Tensor b, Tensor(a!) c, float alpha, bool accumulate) -> ()");
+  m.def("wgrad_gemm_(Tensor a, Tensor b, Tensor(a!) c, float alpha, bool accumulate, Tensor? rows=None) -> ()");
   m.def("wgrad_gemm_variant_(Tensor a, Tensor b, Tensor(a!) c, float alpha, bool accumulate, int variant) -> ()");
-  m.def("wgrad_gemm2_(Tensor a, Tensor b, Tensor a2, Tensor b2, Tensor(a!) c, float alpha, bool accumulate) -> ()");
+  m.def("wgrad_gemm2_(Tensor a, Tensor b, Tensor a2, Tensor b2, Tensor(a!) c, float alpha, bool accumulate, Tensor? rows=None, "
+        "Tensor? rows2=None) -> ()");
 }
 TORCH_LIBRARY_IMPL(sxe, CUDA, m) {
   m.impl("wgrad_gemm_", &sxe::wgrad_gemm_);

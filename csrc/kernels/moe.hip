@@ -169,6 +169,27 @@ __global__ void __launch_bounds__(NT) combine_bwd_kernel(const typename dt_trait
   }
 }
 
+// slots[i] = expert * C + location of a kept assignment i, else -1; slot_src (filled with -1) its inverse; rows (zeros): slots of each
+// expert up to its last one in use. The workgroups' largest go to rows through LDS, a handful of atomics each.
+__global__ void __launch_bounds__(256) tables_kernel(const int64_t* __restrict__ expert, const int64_t* __restrict__ location,
+                                                     const bool* __restrict__ keep, int64_t n, int64_t C, int E, int64_t* __restrict__ slots,
+                                                     int64_t* __restrict__ slot_src, int* __restrict__ rows) {
+  extern __shared__ int most[];
+  for (int e = threadIdx.x; e < E; e += 256) most[e] = 0;
+  __syncthreads();
+  for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < n; i += gridDim.x * 256ll) {
+    const int64_t e = expert[i], c = location[i];
+    const bool in = keep[i] && e >= 0 && e < E && c >= 0 && c < C;
+    slots[i] = in ? e * C + c : -1;
+    if (!in) continue;
+    slot_src[e * C + c] = i;
+    atomicMax(&most[e], (int)c + 1);
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < E; e += 256)
+    if (most[e] > 0) atomicMax(rows + e, most[e]);
+}
+
 inline int row_grid(int64_t rows) { return (int)std::max<int64_t>(1, std::min<int64_t>(rows, (int64_t)kNumCUs * 16)); }
 
 }  // namespace moe
@@ -202,6 +223,25 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> moe_topk_softmax(const at::Tensor
 static void check_rows(const at::Tensor& t, const char* name) {
   SXE_CHECK(t.is_cuda() && t.dim() == 2 && t.is_contiguous() && t.size(1) % 8 == 0, name,
             ": contiguous GPU [rows, H] with H % 8 == 0");
+}
+
+// expert, location int64 [S, k], keep bool -> slots [S, k], slot_src [E C], rows int32 [E]
+std::tuple<at::Tensor, at::Tensor, at::Tensor> moe_tables(const at::Tensor& expert, const at::Tensor& location, const at::Tensor& keep, int64_t C,
+                                                          int64_t E) {
+  check_beside(expert, {location, keep});
+  SXE_CHECK(expert.scalar_type() == at::kLong && location.scalar_type() == at::kLong && keep.scalar_type() == at::kBool &&
+                expert.is_contiguous() && location.is_contiguous() && keep.is_contiguous() && expert.sizes() == location.sizes() &&
+                expert.sizes() == keep.sizes(), "moe_tables: contiguous int64 expert, location and bool keep of one shape");
+  SXE_CHECK(E >= 1 && E <= 8192 && C >= 0 && C < (1ll << 31), "moe_tables: up to 8192 experts of 2^31 slots");
+  c10::DeviceGuard g(expert.device());
+  auto slots = at::empty_like(expert), src = at::full({E * C}, -1, expert.options()), rows = at::zeros({E}, expert.options().dtype(at::kInt));
+  const int64_t n = expert.numel();
+  if (n == 0) return {slots, src, rows};
+  hipLaunchKernelGGL(moe::tables_kernel, dim3((unsigned)std::min<int64_t>((n + 255) / 256, kNumCUs)), dim3(256), E * sizeof(int), cur_stream(),
+                     expert.data_ptr<int64_t>(), location.data_ptr<int64_t>(), keep.data_ptr<bool>(), n, C, (int)E, slots.data_ptr<int64_t>(),
+                     src.data_ptr<int64_t>(), rows.data_ptr<int>());
+  SXE_LAUNCH_CHECK();
+  return {slots, src, rows};
 }
 
 at::Tensor moe_dispatch(const at::Tensor& x, const at::Tensor& slot_src, int64_t k) {
@@ -286,12 +326,14 @@ std::tuple<at::Tensor, at::Tensor> moe_combine_bwd(const at::Tensor& gy, const a
 
 TORCH_LIBRARY_FRAGMENT(sxe, m) {
   m.def("moe_topk_softmax(Tensor logits, int k) -> (Tensor, Tensor, Tensor)");
+  m.def("moe_tables(Tensor expert, Tensor location, Tensor keep, int capacity, int experts) -> (Tensor, Tensor, Tensor)");
   m.def("moe_dispatch(Tensor x, Tensor slot_src, int k) -> Tensor");
   m.def("moe_gather_sum(Tensor src, Tensor slots, Tensor? coef) -> Tensor");
   m.def("moe_combine_bwd(Tensor gy, Tensor expert_out, Tensor slot_src, Tensor w) -> (Tensor, Tensor)");
 }
 TORCH_LIBRARY_IMPL(sxe, CUDA, m) {
   m.impl("moe_topk_softmax", &sxe::moe_topk_softmax);
+  m.impl("moe_tables", &sxe::moe_tables);
   m.impl("moe_dispatch", &sxe::moe_dispatch);
   m.impl("moe_gather_sum", &sxe::moe_gather_sum);
   m.impl("moe_combine_bwd", &sxe::moe_combine_bwd);

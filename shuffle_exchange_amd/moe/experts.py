@@ -77,7 +77,8 @@ class GroupedSwiGLUExperts(nn.Module):
             setattr(self, name, new)
         self.tp_group = tp_group
 
-    def forward(self, x):
+    def forward(self, x, rows=None):
+        """``rows`` (int32 [E_local], may be None): rows of each expert that may be other than zero, the first ones."""
         # x: [E_local, C, H] -> [E_local, C, 2I] -> SwiGLU (one HIP launch for all experts) -> [E_local, C, H]
         # (the dense MLP's token-minor weight-gradient scheme, ops/mlp.py, measured no faster here: the
         # experts reduce over only C capacity tokens -- Mixtral-arch 8 layers 311.8 vs 309.9 ms/step)
@@ -85,12 +86,13 @@ class GroupedSwiGLUExperts(nn.Module):
             from ..module_inject.layers import copy_to_tp, reduce_from_tp
             x = copy_to_tp(x, self.tp_group)
             return reduce_from_tp(grouped_mm(swiglu(grouped_mm(x, self.w_gate_up)), self.w_down), self.tp_group)
-        return grouped_mm(swiglu(grouped_mm(x, self.w_gate_up)), self.w_down)
+        return grouped_mm(swiglu(grouped_mm(x, self.w_gate_up, rows)), self.w_down, rows)
 
 
-def expert_products(x, w, transposed=False):
+def expert_products(x, w, transposed=False, rows=None):
     """x[e] @ w[e] (``transposed``: x[e] @ w[e]^T) of all experts, bf16 x [E, C, .], w [E, K, N], in one launch (csrc/kernels/experts_kn_tile.hip,
-    gemm_tn.hip); None where these do not cover the operands. A library product per expert fills the card only with the rows of one:
+    gemm_tn.hip); None where these do not cover the operands. ``rows`` (int32 [E] on the device, or None): x[e, rows[e]:] is zeros, and so is
+    what comes of it. A library product per expert fills the card only with the rows of one:
     8 experts, 4096 x 28672, us, 320 rows each 753 / 749 here, 1280 rows 2273 / 1776, transposed 2438 / 508, 3289 / 2012; 14336 x 4096,
     1164 / 330, 1455 / 936, transposed 443 / 385, 1174 / 847; 2048 x 16384, 1280 rows 695 / 548, transposed 987 / 563. Of 4 to 2560 rows
     each nothing was more than 4 % slower but 4 rows transposed of 3072 x 16384 (0.91)."""
@@ -102,7 +104,7 @@ def expert_products(x, w, transposed=False):
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and K % 64 == 0 and N % 64 == 0 and 0 < K < 1 << 22 and 0 < N < 1 << 22
             and E * C < 1 << 30 and E <= 1024):
         native.require_hip()
-        return torch.ops.sxe.gemm_tn_batch(x, w) if transposed else torch.ops.sxe.expert_mm_kn(x, w)
+        return torch.ops.sxe.gemm_tn_batch(x, w, -1, rows) if transposed else torch.ops.sxe.expert_mm_kn(x, w, rows)
     return None
 
 
@@ -116,25 +118,25 @@ class _GroupedMM(torch.autograd.Function):
     lookup-only path faulted on MI355X at Mixtral sizes (illegal address in the autograd thread)."""
 
     @staticmethod
-    def forward(ctx, x, w):
+    def forward(ctx, x, w, rows=None):
         E, C, _ = x.shape
         x = x.contiguous()
-        y = expert_products(x, w)
+        y = expert_products(x, w, rows=rows)
         if y is None:
             y = x.new_empty(E, C, w.shape[2])
             for e in range(E):
                 torch.mm(x[e], w[e], out=y[e])
-        ctx.save_for_backward(x, w)
+        ctx.save_for_backward(x, w, rows)
         return y
 
     @staticmethod
     def backward(ctx, dy):
-        x, w = ctx.saved_tensors
+        x, w, rows = ctx.saved_tensors
         dy = dy.contiguous()
         E = x.shape[0]
         dx = dw = None
         if ctx.needs_input_grad[0]:
-            dx = expert_products(dy, w, transposed=True)
+            dx = expert_products(dy, w, transposed=True, rows=rows)
             if dx is None:
                 dx = torch.empty_like(x)
                 for e in range(E):
@@ -147,22 +149,23 @@ class _GroupedMM(torch.autograd.Function):
                 # before the accumulation boundary: keep (x, dy) and write the weight gradient once, at
                 # the boundary, over all micro-steps' tokens -- one fp32 write of the expert's gradient
                 # per step instead of a write plus a read-modify-write per micro-step
-                w.__dict__.setdefault("_sxe_wstash", []).append((x, dy))
-                return dx, None
+                w.__dict__.setdefault("_sxe_wstash", []).append((x, dy, rows))
+                return dx, None, None
             stash = w.__dict__.pop("_sxe_wstash", None)
             prev = None  # one stashed micro-step: its (x, dy) are the first K segment of the product
             if stash and len(stash) == 1:
                 prev = stash[0]
             elif stash:
-                x = torch.cat([a for a, _ in stash] + [x], dim=1)
-                dy = torch.cat([g for _, g in stash] + [dy], dim=1)
+                x = torch.cat([a for a, _, _ in stash] + [x], dim=1)
+                dy = torch.cat([g for _, g, _ in stash] + [dy], dim=1)
+                rows = None
             if tgt is not None:
                 buf, acc = tgt(w)
                 be = buf.view(w.shape)
                 if prev is not None and _wgrad2_ok(prev[0], prev[1], x, dy, be):
-                    torch.ops.sxe.wgrad_gemm2_(prev[0], prev[1], x, dy, be, 1.0, bool(acc))
+                    torch.ops.sxe.wgrad_gemm2_(prev[0], prev[1], x, dy, be, 1.0, bool(acc), prev[2], rows)
                 elif prev is None and _wgrad_all_ok(x, dy, be):
-                    torch.ops.sxe.wgrad_gemm_(x, dy, be, 1.0, bool(acc))
+                    torch.ops.sxe.wgrad_gemm_(x, dy, be, 1.0, bool(acc), rows)
                 else:
                     for e in range(E):
                         if prev is not None:
@@ -173,7 +176,7 @@ class _GroupedMM(torch.autograd.Function):
                 dw = torch.empty_like(w)
                 for e in range(E):
                     torch.mm(x[e].t(), dy[e], out=dw[e])
-        return dx, dw
+        return dx, dw, None
 
 
 def _expert_wgrad(xe, ge, be, acc):
@@ -205,8 +208,9 @@ def _wgrad2_ok(x1, g1, x2, g2, be):
             and g1.stride(1) == g2.stride(1))
 
 
-def grouped_mm(x, w):
-    return _GroupedMM.apply(x, w)
+def grouped_mm(x, w, rows=None):
+    """``rows``: as ``expert_products``; the rows behind them of the gradient of the result are taken to be zeros, too."""
+    return _GroupedMM.apply(x, w, rows)
 
 
 def flush_deferred_wgrad(w):
@@ -215,8 +219,8 @@ def flush_deferred_wgrad(w):
     stash = w.__dict__.pop("_sxe_wstash", None)
     if not stash:
         return
-    x = torch.cat([a for a, _ in stash], dim=1)
-    dy = torch.cat([g for _, g in stash], dim=1)
+    x = torch.cat([a for a, _, _ in stash], dim=1)
+    dy = torch.cat([g for _, g, _ in stash], dim=1)
     defer, w._sxe_grad_defer = w._sxe_grad_defer, None
     try:
         _GroupedMM.backward(_FlushCtx(x, w), dy)
@@ -228,4 +232,4 @@ class _FlushCtx:
     needs_input_grad = (False, True)
 
     def __init__(self, x, w):
-        self.saved_tensors = (x, w)
+        self.saved_tensors = (x, w, None)

@@ -281,10 +281,11 @@ class MOELayer(nn.Module):
         E = self.ep_size * self.num_local_experts
         C = r.capacity
         k = r.expert.shape[1]
-        from ..ops.moe import combine, dispatch, routing_tables
+        from ..ops.moe import combine, dispatch, slot_tables
+        from .experts import GroupedSwiGLUExperts
         # slots[t, c] = expert * C + position (-1 dropped) and its inverse slot_src[E * C]: dispatch
         # and combine are then atomic-free row gathers (csrc/kernels/moe.hip on the GPU)
-        slots, slot_src = routing_tables(r.expert, r.location, r.keep, C, E)
+        slots, slot_src, rows = slot_tables(r.expert, r.location, r.keep, C, E)
         disp = dispatch(xt, slots, slot_src)
         ep, nle, tp = self.ep_size, self.num_local_experts, self.tp
         from .mappings import drop_tokens, gather_tokens
@@ -299,7 +300,10 @@ class MOELayer(nn.Module):
             Ce = C
         # local experts see [E_local, ep*Ce, H]
         disp = disp.reshape(ep, nle, Ce, H).transpose(0, 1).reshape(nle, ep * Ce, H)
-        out = self.experts(disp)
+        if rows is not None and ep == 1 and tp == 1 and getattr(type(self.experts), "forward", None) is GroupedSwiGLUExperts.forward:
+            out = self.experts(disp, rows=rows)  # the slots behind an expert's last one are zeros: its products leave them out
+        else:
+            out = self.experts(disp)
         out = out.view(nle, ep, Ce, H).transpose(0, 1).reshape(ep * nle, Ce, H)
         if self.expert_tp:
             out = drop_tokens(out, 1, self.tp_group)

@@ -106,7 +106,7 @@ def _transpose16(x):
 
 
 @_reg("sxe::wgrad_gemm_")
-def _wgrad(a, b, c, alpha, accumulate):
+def _wgrad(a, b, c, alpha, accumulate, rows=None):
     return None
 
 

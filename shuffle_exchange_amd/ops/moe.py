@@ -49,12 +49,21 @@ def topk_softmax(logits, k):
 
 
 def routing_tables(expert, location, keep, capacity, num_experts):
+    return slot_tables(expert, location, keep, capacity, num_experts)[:2]
+
+
+def slot_tables(expert, location, keep, capacity, num_experts):
+    """``routing_tables`` and, on the GPU, int32 [E]: each expert's slots up to its last one in use (else None). One kernel, and no
+    number comes back to the host (the boolean indices below are two waits a layer)."""
+    if (_hip(expert) and expert.dtype == location.dtype == torch.int64 and keep.dtype == torch.bool and num_experts <= 8192
+            and native.plain(expert, location, keep)):
+        return torch.ops.sxe.moe_tables(expert.contiguous(), location.contiguous(), keep.contiguous(), int(capacity), int(num_experts))
     slots = torch.where(keep, expert * capacity + location, torch.full_like(expert, -1)).contiguous()
     flat = slots.reshape(-1)
     kept = flat >= 0
     slot_src = torch.full((num_experts * capacity,), -1, dtype=torch.int64, device=expert.device)
     slot_src.index_copy_(0, flat[kept], torch.arange(flat.numel(), device=expert.device)[kept])
-    return slots, slot_src
+    return slots, slot_src, None
 
 
 class _Dispatch(torch.autograd.Function):

@@ -165,3 +165,39 @@ def test_captured():
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(y, linear(x, w))
+
+
+@pytest.mark.parametrize("C", [1, 64, 100, 256, 320, 700])
+def test_expert_products_of_rows_in_use(C):
+    """Rows behind those in use are zeros and left out: the same bits as all rows, for no row, a row, edges of slabs and tiles, all rows; both
+    products, and the weight gradient in one piece and in two, with tokens that end inside a slab."""
+    from shuffle_exchange_amd.moe.experts import expert_products
+    E, K, N = 6, 128, 320
+    g = torch.Generator("cuda").manual_seed(C)
+    R = lambda *s: torch.randn(*s, device="cuda", generator=g).bfloat16()
+    w = R(E, K, N) * K ** -0.5
+
+    def piece(used):
+        rows = torch.tensor([min(C, u) for u in used], device="cuda", dtype=torch.int32)
+        live = torch.arange(C, device="cuda")[None, :, None] < rows[:, None, None]
+        return rows, R(E, C, K) * live, R(E, C, N) * live
+    a, b = piece((0, 1, 63, 64, 257, C)), piece((65, 0, 256, 128, 1, C - 1))
+    nan = lambda *s: torch.full(s, float("nan"), device="cuda", dtype=torch.bfloat16)
+    for rows, x, dy in (a, b):
+        nan(E, C, N), nan(E, C, K)  # what the results' memory may hold before
+        assert torch.equal(expert_products(x, w, rows=rows), expert_products(x, w))
+        assert torch.equal(expert_products(dy, w, transposed=True, rows=rows), expert_products(dy, w, transposed=True))
+        for tile in range(4):
+            assert torch.equal(torch.ops.sxe.gemm_tn_batch(dy, w, tile, rows), torch.ops.sxe.gemm_tn_batch(dy, w, tile))
+    for accumulate in (False, True):
+        def both(f):
+            out = [torch.randn(E, K, N, device="cuda", generator=torch.Generator("cuda").manual_seed(1)) for _ in range(2)]
+            f(out[0], False), f(out[1], True)
+            assert torch.equal(*out)
+        both(lambda c, r: torch.ops.sxe.wgrad_gemm_(a[1], a[2], c, 0.5, accumulate, a[0] if r else None))
+        both(lambda c, r: torch.ops.sxe.wgrad_gemm2_(a[1], a[2], b[1], b[2], c, 1.0, accumulate, a[0] if r else None, b[0] if r else None))
+        both(lambda c, r: torch.ops.sxe.wgrad_gemm2_(a[1], a[2], b[1], b[2], c, 1.0, accumulate, None, b[0] if r else None))
+    with pytest.raises(RuntimeError):
+        expert_products(a[1], w, rows=a[0].long())
+    with pytest.raises(RuntimeError):
+        expert_products(a[1], w, rows=a[0][:-1])

@@ -122,3 +122,20 @@ def test_moe_layer_gpu_kernels_match_cpu_path(_hip):
     yg.sum().backward()
     for (n, a), (_, b) in zip(layer.named_parameters(), gpu.named_parameters()):
         assert torch.allclose(b.grad.cpu(), a.grad, atol=1e-4), n
+
+
+@pytest.mark.parametrize("S,k,E,C", [(1, 1, 1, 1), (300, 2, 8, 48), (700, 1, 5, 700), (4097, 2, 64, 160)])
+def test_slot_tables(S, k, E, C):
+    """The tables of the kernel and those of the plain operators; rows up to each expert's last slot in use, gaps before it or not."""
+    from shuffle_exchange_amd.ops import moe as M
+    torch.manual_seed(S)
+    order = torch.randperm(E * C)[:S * k]
+    if order.numel() < S * k:
+        order = torch.cat([order, torch.zeros(S * k - order.numel(), dtype=torch.long)])
+    keep = (torch.rand(S, k) < 0.8) & (torch.arange(S * k).view(S, k) < E * C)
+    expert, loc = (order // C).view(S, k), (order % C).view(S, k)
+    want = M.slot_tables(expert, loc, keep, C, E)
+    slots, src, rows = M.slot_tables(expert.cuda(), loc.cuda(), keep.cuda(), C, E)
+    assert want[2] is None and torch.equal(slots.cpu(), want[0]) and torch.equal(src.cpu(), want[1])
+    used = (want[1].view(E, C) >= 0) * torch.arange(1, C + 1)
+    assert rows.dtype == torch.int32 and torch.equal(rows.cpu().long(), used.amax(1))
