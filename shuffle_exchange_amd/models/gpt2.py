@@ -11,7 +11,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from ..ops.activation import bias_gelu
-from ..ops.attention import attention
+from ..ops.attention import attention_qkv_rope
 from ..ops.cross_entropy import head_cross_entropy
 from ..ops.linear import Embedding, Linear
 from ..ops.norm import LayerNorm
@@ -72,10 +72,10 @@ class GPT2Block(nn.Module):
     def forward(self, x):
         B, S, H = x.shape
         d = self.head_dim
-        qkv = self.c_attn(self.ln_1(x)).view(B, S, 3, self.n_head, d)
-        o = attention(qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2], causal=True)
-        x = x + self.c_proj(o.reshape(B, S, self.n_head * d))
-        m = bias_gelu(self.c_fc(self.ln_2(x), skip_bias=True), self.c_fc.bias)
+        # q, k and v as they lie: their gradients are written side by side, where slices' would be padded with zeros and added up
+        o = attention_qkv_rope(self.c_attn(self.ln_1(x)).view(B, S, 3 * self.n_head, d), self.n_head, self.n_head)
+        y, x = self.ln_2(self.c_proj(o.reshape(B, S, self.n_head * d)), residual=x)
+        m = bias_gelu(self.c_fc(y, skip_bias=True), self.c_fc.bias)
         return x + self.mlp_proj(m)
 
 

@@ -161,8 +161,9 @@ def _tileable(x2, weight, bias=None):
             and (bias is None or (_bias_ok(bias, weight) and bias.data_ptr() % 16 == 0)))
 
 
-def _tiled(x, weight, bias):
-    if weight.dim() != 2 or not _tiled_faster(x.numel() // max(1, x.shape[-1]), *weight.shape):
+def _tiled(x, weight, bias, faster=False):
+    """gemm_tn.hip, where it covers the operands and is the faster one (``faster``: as the caller has found), else None."""
+    if weight.dim() != 2 or not (faster or _tiled_faster(x.numel() // max(1, x.shape[-1]), *weight.shape)):
         return None
     x2 = x.reshape(-1, x.shape[-1])
     if not _tileable(x2, weight, bias):
@@ -179,10 +180,23 @@ def _own_products(x, weight, bias=None):
             and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == torch.bfloat16))
 
 
+# Products of training with narrow weights, up to this many multiplications. A call of the library costs the host 19.5 us whatever its size, one
+# of gemm_tn.hip 6, and its kernels are about as fast; us on the device, library / here: 2048 rows, 2304 x 768 17 / 14, 3072 x 768 16 / 15,
+# 768 x 768 10 / 12, 768 x 3072 19 / 25, 1280 x 5120 37 / 37, 300 rows 8 / 12, 8 / 12, 6 / 11, 9 / 16, 18 / 23. Behind it the device decides:
+# 8192 rows, 768 x 3072 39 / 36, 4096 x 1024 57 / 60, 8192 x 1536, 8192 rows 158 / 168.
+NARROW_WORK = 10 ** 10
+
+
+def _narrow(rows, N, K):
+    """A weight that ``_tiled_faster`` leaves to the library for its width, and a product whose call costs more than its work."""
+    return (N < 2048 or K < 2048) and N >= 512 and K >= 512 and rows > STREAM_ROWS_SMALL and rows * N * K <= NARROW_WORK
+
+
 def product(x, weight, bias=None):
     """``F.linear`` for the inside of autograd functions: no graph is built where it runs own kernels (``_tiled``)."""
-    if weight.dim() == 2 and _tiled_faster(x.numel() // max(1, x.shape[-1]), *weight.shape) and _own_products(x, weight, bias):
-        y = _tiled(x, weight, bias)
+    rows = x.numel() // max(1, x.shape[-1])
+    if weight.dim() == 2 and (_tiled_faster(rows, *weight.shape) or _narrow(rows, *weight.shape)) and _own_products(x, weight, bias):
+        y = _tiled(x, weight, bias, True)
         if y is not None:
             return y
     return F.linear(x, weight, bias)
@@ -473,6 +487,22 @@ def _wt_few_faster(rows, N, K):
     return K <= 3072 or (K <= 5120 and N >= 20480 and rows <= 1280)
 
 
+def _narrow_data_grad(gy, w):
+    """gy @ w of ``_narrow`` weights: up to 1280 rows of the weight by the product that reads them as they lie (experts_kn_tile.hip, one
+    expert), else with the transpose, which the splits of gemm_tn.hip make up for. us on the device, library / as they lie / transposed,
+    2048 rows: 768 x 3072 18 / 17 / 21, 768 x 768 12 / 14 / 15, 1280 x 5120 36 / 32 / 35, 2304 x 768 24 / 28 / 27, 3072 x 768 30 / 35 / 28,
+    300 rows 14 / 33 / 20; on the host 19 / 8 / 13. None where they do not cover the operands."""
+    N, K = w.shape
+    if not (_narrow(gy.numel() // max(1, gy.shape[-1]), N, K) and gy.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and N % 64 == 0
+            and K % 64 == 0 and gy.is_contiguous() and w.is_cuda and w.is_contiguous() and gy.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and _own_products(gy, w)):
+        return None
+    native.require_hip()
+    if N <= 1280:
+        return torch.ops.sxe.expert_mm_kn(gy.view(1, -1, N), w.unsqueeze(0)).view(*gy.shape[:-1], K)
+    return torch.ops.sxe.gemm_tn(gy, _transposed_weight(w), None, False)
+
+
 def data_grad(gy, w):
     """dX = gy @ w for w [N, K] (gy [..., N])."""
     if (DGRAD_WT_MIN_ELEMS > 0 and gy.is_cuda and gy.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
@@ -481,6 +511,10 @@ def data_grad(gy, w):
         rows = gy.numel() // gy.shape[-1]
         if rows >= 2048 or (_wt_few_faster(rows, *w.shape) and gy.is_contiguous() and gy.data_ptr() % 16 == 0 and _own_products(gy, w)):
             return product(gy, _transposed_weight(w))
+    if gy.is_cuda and w.dim() == 2:
+        dx = _narrow_data_grad(gy, w)
+        if dx is not None:
+            return dx
     return torch.matmul(gy, w)
 
 

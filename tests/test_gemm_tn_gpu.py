@@ -201,3 +201,50 @@ def test_expert_products_of_rows_in_use(C):
         expert_products(a[1], w, rows=a[0].long())
     with pytest.raises(RuntimeError):
         expert_products(a[1], w, rows=a[0][:-1])
+
+
+@pytest.mark.parametrize("N,K", [(512, 512), (768, 3072), (2304, 768), (1344, 1088), (3072, 768)])
+@pytest.mark.parametrize("rows", [33, 300, 1025])
+def test_narrow_products_of_training(N, K, rows):
+    """Weights that are narrow one way, inside autograd functions: forward with a bias and data gradient on the own products, and what they do
+    not cover on the library's."""
+    from shuffle_exchange_amd.ops import linear as L
+    g = torch.Generator("cuda").manual_seed(rows)
+    R = lambda *s: torch.randn(*s, device="cuda", generator=g).bfloat16()
+    x, w, b, dy = R(rows, K), R(N, K) * K ** -0.5, R(N), R(rows, N)
+    with torch.no_grad():
+        assert L._narrow(rows, N, K) and not L._narrow(32, N, K) and not L._narrow(10 ** 10 // (N * K) + 1, N, K)
+        y = L.product(x, w, b)
+        _close(y, x.double() @ w.double().t() + b.double(), x, w)
+        assert torch.equal(L.product(x.view(1, rows, K), w, b)[0], y)
+        dx = L._narrow_data_grad(dy, w)
+        _close(dx, dy.double() @ w.double(), dy, w.t())
+        assert torch.equal(L.data_grad(dy.view(1, rows, N), w)[0], dx)
+        odd = R(rows + 1, N + 1)[1:, 1:]  # rows that start off 16 bytes
+        assert L._narrow_data_grad(odd, w) is None and L._narrow_data_grad(dy.float(), w.float()) is None
+        _close(L.data_grad(odd, w), odd.double() @ w.double(), odd, w.t())
+    assert L._narrow_data_grad(dy.requires_grad_(), w) is None  # a graph is recorded
+
+
+def test_gpt2_block_packed_attention():
+    """Attention over the projection as it lies and the residual inside the second norm: values and gradients of the block by plain operators."""
+    from shuffle_exchange_amd.models.gpt2 import GPT2Block, gpt2_config
+    import torch.nn.functional as F
+    torch.manual_seed(0)
+    cfg = gpt2_config("gpt2-tiny", n_embd=128, n_head=2)
+    blk = GPT2Block(cfg).cuda().bfloat16()
+    x = torch.randn(2, 70, 128, device="cuda").bfloat16().requires_grad_()
+    dy = torch.randn(2, 70, 128, device="cuda").bfloat16()
+    y = blk(x)
+    got = torch.autograd.grad(y, [x, *blk.parameters()], dy)
+    P = {n: p.detach().double().requires_grad_() for n, p in blk.named_parameters()}
+    xd = x.detach().double().requires_grad_()
+    ln = lambda t, n: F.layer_norm(t, (128,), P[n + ".weight"], P[n + ".bias"], 1e-5)
+    lin = lambda t, n: t @ P[n + ".weight"].t() + P[n + ".bias"]
+    q, k, v = (t.transpose(1, 2) for t in lin(ln(xd, "ln_1"), "c_attn").view(2, 70, 3, 2, 64).unbind(2))
+    s = (q @ k.transpose(-1, -2) / 8).masked_fill(torch.ones(70, 70, device="cuda", dtype=torch.bool).triu(1), float("-inf"))
+    h = xd + lin((s.softmax(-1) @ v).transpose(1, 2).reshape(2, 70, 128), "c_proj")
+    want = h + lin(F.gelu(lin(ln(h, "ln_2"), "c_fc"), approximate="tanh"), "mlp_proj")
+    assert (y.double() - want).norm() <= 4e-3 * want.norm()  # roundings to 8 bits of the sums: 2^-9 each
+    for a, b in zip(got, torch.autograd.grad(want, [xd, *P.values()], dy.double())):
+        assert (a.double() - b).norm() <= 2e-2 * b.norm(), a.shape  # a chain of a dozen of them
