@@ -17,6 +17,7 @@ struct ColsumArgs {  // blockIdx.z picks the matrix
   const void* in[2];
   void* out[2];
   int64_t R, N, ld, rows;  // rows of a split
+  bool add[2];             // fp32 out: add to what is there
 };
 
 template <DT T, DT O, bool VEC>
@@ -65,7 +66,10 @@ __global__ void __launch_bounds__(1024) colsum_kernel(ColsumArgs a) {
     float t = 0.f;
 #pragma unroll
     for (int w = 0; w < 16; ++w) t += red[w][threadIdx.x];
-    static_cast<typename dt_traits<O>::storage*>(a.out[blockIdx.z])[(int64_t)blockIdx.y * a.N + n] = from_f32<O>(t);
+    auto* out = static_cast<typename dt_traits<O>::storage*>(a.out[blockIdx.z]) + (int64_t)blockIdx.y * a.N + n;
+    if constexpr (O == DT::F32)
+      if (a.add[blockIdx.z]) t += *out;
+    *out = from_f32<O>(t);
   }
 }
 
@@ -80,19 +84,20 @@ void colsum_launch(const ColsumArgs& a, int splits, int mats) {
   SXE_LAUNCH_CHECK();
 }
 
-// one or two matrices of R > 0 rows and N > 0 columns, row stride ld; out: N elements of O each
+// one or two matrices of R > 0 rows and N > 0 columns, row stride ld; out: N elements of O each, where `add` (fp32 only) added to
 template <DT T, DT O>
-void colsum(const void* const (&in)[2], void* const (&out)[2], int64_t R, int64_t N, int64_t ld, int mats, const at::TensorOptions& opt) {
+void colsum(const void* const (&in)[2], void* const (&out)[2], int64_t R, int64_t N, int64_t ld, int mats, const at::TensorOptions& opt,
+            bool add0 = false, bool add1 = false) {
   SXE_CHECK(N <= 64ll * 0x7fffffff, "column sum: columns");
   if (R <= kColsumRows) {
-    colsum_launch<T, O>({{in[0], in[1]}, {out[0], out[1]}, R, N, ld, R}, 1, mats);
+    colsum_launch<T, O>({{in[0], in[1]}, {out[0], out[1]}, R, N, ld, R, {add0, add1}}, 1, mats);
     return;
   }
   const int64_t splits = std::min<int64_t>((R + 1023) / 1024, 256), rows = (R + splits - 1) / splits;
   auto part = at::empty({mats, splits, N}, opt.dtype(at::kFloat));
   float* p = part.data_ptr<float>();
-  colsum_launch<T, DT::F32>({{in[0], in[1]}, {p, p + splits * N}, R, N, ld, rows}, (int)splits, mats);
-  colsum_launch<DT::F32, O>({{p, p + splits * N}, {out[0], out[1]}, splits, N, N, splits}, 1, mats);
+  colsum_launch<T, DT::F32>({{in[0], in[1]}, {p, p + splits * N}, R, N, ld, rows, {false, false}}, (int)splits, mats);
+  colsum_launch<DT::F32, O>({{p, p + splits * N}, {out[0], out[1]}, splits, N, N, splits, {add0, add1}}, 1, mats);
 }
 
 }  // namespace sxe

@@ -307,8 +307,9 @@ std::vector<at::Tensor> norm_fwd(at::Tensor x, c10::optional<at::Tensor> residua
 }
 
 // Returns (dx, dweight_fp32, dbias_fp32_or_empty). `dres` (optional) is added into dx.
-std::vector<at::Tensor> norm_bwd(at::Tensor dy, at::Tensor x, at::Tensor rstd, c10::optional<at::Tensor> mean,
-                                 at::Tensor weight, c10::optional<at::Tensor> dres, bool layernorm) {
+// dw, db: where the gradients go, fp32 [H] of the caller's that they are written or added to; or undefined: new tensors
+static std::vector<at::Tensor> norm_bwd_run(at::Tensor dy, at::Tensor x, at::Tensor rstd, c10::optional<at::Tensor> mean, at::Tensor weight,
+                                            c10::optional<at::Tensor> dres, bool layernorm, at::Tensor dw, bool add_w, at::Tensor db, bool add_b) {
   SXE_CHECK(dy.is_contiguous() && x.is_contiguous() && weight.is_contiguous(), "norm_bwd: contiguous");
   const int H = (int)x.size(-1);
   const int64_t rows = x.numel() / H;
@@ -322,7 +323,12 @@ std::vector<at::Tensor> norm_bwd(at::Tensor dy, at::Tensor x, at::Tensor rstd, c
   auto dw_part = at::empty({grid, H}, x.options().dtype(at::kFloat));
   auto db_part = layernorm ? at::empty({grid, H}, x.options().dtype(at::kFloat)) : at::empty({0}, x.options().dtype(at::kFloat));
   if (rows == 0) {
-    return {dx, at::zeros({H}, x.options().dtype(at::kFloat)), layernorm ? at::zeros({H}, x.options().dtype(at::kFloat)) : db_part};
+    if (!dw.defined()) dw = at::zeros({H}, dw_part.options());
+    else if (!add_w) dw.zero_();
+    if (!layernorm) db = db_part;
+    else if (!db.defined()) db = at::zeros({H}, dw_part.options());
+    else if (!add_b) db.zero_();
+    return {dx, dw, db};
   }
   const size_t lds = (size_t)4 * H * sizeof(float);
   SXE_CHECK(lds <= 160 * 1024, "norm_bwd: hidden too large for LDS reduction");
@@ -341,10 +347,28 @@ std::vector<at::Tensor> norm_bwd(at::Tensor dy, at::Tensor x, at::Tensor rstd, c
                        layernorm ? db_part.data_ptr<float>() : nullptr, rows, H);
   })))));
   SXE_LAUNCH_CHECK();
-  auto dw = at::empty({H}, dw_part.options()), db = layernorm ? at::empty({H}, dw_part.options()) : db_part;
+  if (!dw.defined()) dw = at::empty({H}, dw_part.options());
+  if (!layernorm) db = db_part;
+  else if (!db.defined()) db = at::empty({H}, dw_part.options());
   colsum<DT::F32, DT::F32>({dw_part.data_ptr(), db_part.data_ptr()}, {dw.data_ptr(), db.data_ptr()}, grid, H, H, layernorm ? 2 : 1,
-                           dw_part.options());
+                           dw_part.options(), add_w, add_b);
   return {dx, dw, db};
+}
+
+std::vector<at::Tensor> norm_bwd(at::Tensor dy, at::Tensor x, at::Tensor rstd, c10::optional<at::Tensor> mean,
+                                 at::Tensor weight, c10::optional<at::Tensor> dres, bool layernorm) {
+  return norm_bwd_run(dy, x, rstd, mean, weight, dres, layernorm, {}, false, {}, false);
+}
+
+// -> dx; the gradients of weight and bias (layer norms) are written or added to dw and db
+at::Tensor norm_bwd_into(at::Tensor dy, at::Tensor x, at::Tensor rstd, c10::optional<at::Tensor> mean, at::Tensor weight,
+                         c10::optional<at::Tensor> dres, bool layernorm, at::Tensor dw, bool add_w, c10::optional<at::Tensor> db, bool add_b) {
+  check_beside(x, {dy, rstd, mean, weight, dres, dw, db});
+  const bool has_db = db.has_value() && db->defined();
+  SXE_CHECK(has_db == layernorm, "norm_bwd_into: db of layer norms");
+  for (const at::Tensor* t : {&dw, has_db ? &*db : &dw})
+    SXE_CHECK(t->scalar_type() == at::kFloat && t->is_contiguous() && t->numel() == x.size(-1), "norm_bwd_into: fp32 dw, db [H]");
+  return norm_bwd_run(dy, x, rstd, mean, weight, dres, layernorm, dw, add_w, has_db ? *db : at::Tensor(), add_b)[0];
 }
 
 }  // namespace sxe
@@ -352,8 +376,11 @@ std::vector<at::Tensor> norm_bwd(at::Tensor dy, at::Tensor x, at::Tensor rstd, c
 TORCH_LIBRARY_FRAGMENT(sxe, m) {
   m.def("norm_fwd(Tensor x, Tensor? residual, Tensor weight, Tensor? bias, float eps, bool layernorm) -> Tensor[]");
   m.def("norm_bwd(Tensor dy, Tensor x, Tensor rstd, Tensor? mean, Tensor weight, Tensor? dres, bool layernorm) -> Tensor[]");
+  m.def("norm_bwd_into(Tensor dy, Tensor x, Tensor rstd, Tensor? mean, Tensor weight, Tensor? dres, bool layernorm, Tensor(a!) dw, bool add_w, "
+        "Tensor(b!)? db, bool add_b) -> Tensor");
 }
 TORCH_LIBRARY_IMPL(sxe, CUDA, m) {
   m.impl("norm_fwd", &sxe::norm_fwd);
   m.impl("norm_bwd", &sxe::norm_bwd);
+  m.impl("norm_bwd_into", &sxe::norm_bwd_into);
 }

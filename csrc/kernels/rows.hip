@@ -20,6 +20,7 @@
 // uses the same code; only ``add`` (an elementwise sum) needs the type.
 #include "sxe_common.h"
 #include <torch/library.h>
+#include <type_traits>
 
 namespace sxe {
 namespace rows {
@@ -118,11 +119,11 @@ __global__ void __launch_bounds__(1024) rank_kernel(const I* __restrict__ idx, i
 }
 
 // Eight lanes a rank, eight columns a lane. A run of one index is summed by the block it starts in, which
-// follows it over the blocks behind.
-template <DT T>
+// follows it over the blocks behind. O: void, rows of gy's type are stored; float, fp32 rows are added to.
+template <DT T, typename O>
 __global__ void __launch_bounds__(256) run_sum_kernel(const typename dt_traits<T>::storage* __restrict__ gy, int64_t W, int n, int rows,
-                                                      const int* __restrict__ order, const int* __restrict__ sorted,
-                                                      typename dt_traits<T>::storage* __restrict__ out) {
+                                                      const int* __restrict__ order, const int* __restrict__ sorted, void* __restrict__ out) {
+  using S = typename dt_traits<T>::storage;
   __shared__ float sum[32][65];
   const int g = threadIdx.x >> 3, cl = (threadIdx.x & 7) * 8, p0 = blockIdx.x * 32, p = p0 + g;
   const int64_t c = (int64_t)blockIdx.y * 64 + cl;
@@ -181,7 +182,17 @@ __global__ void __launch_bounds__(256) run_sum_kernel(const typename dt_traits<T
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] += sum[i][cl + j];
   }
-  if (start && in) store8<T>(out + (int64_t)id * W + c, v);
+  if (!start || !in) return;
+  if constexpr (std::is_same<O, void>::value) {
+    store8<T>(static_cast<S*>(out) + (int64_t)id * W + c, v);
+  } else {  // fp32 sums that are there already: a run has one workgroup a column, its row nobody else
+    float x[8];
+    float* to = static_cast<float*>(out) + (int64_t)id * W + c;
+    load8<DT::F32>(to, x);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] += x[j];
+    store8<DT::F32>(to, v);
+  }
 }
 
 }  // namespace rows
@@ -259,17 +270,15 @@ void scatter_rows_(at::Tensor dst, const at::Tensor& idx, const at::Tensor& src)
   SXE_LAUNCH_CHECK();
 }
 
-at::Tensor embedding_grad(const at::Tensor& gy, const at::Tensor& idx, int64_t rows) {
-  check_beside(gy, {idx});
-  const int64_t n = idx.numel();
+// the gradients of equal indices added up: out [rows, W] of gy's type, zeros to start with, or (into) fp32 sums that they are added to
+static void embedding_run(const at::Tensor& gy, const at::Tensor& idx, at::Tensor& out, bool into) {
+  const int64_t n = idx.numel(), rows = out.size(0);
   SXE_CHECK(gy.dim() == 2 && gy.is_contiguous() && gy.size(1) % 8 == 0 && reinterpret_cast<uintptr_t>(gy.data_ptr()) % 16 == 0,
             "embedding_grad: gy [N, W], W a multiple of 8");
   SXE_CHECK(idx.is_cuda() && idx.is_contiguous() && n == gy.size(0) && (idx.scalar_type() == at::kLong || idx.scalar_type() == at::kInt),
             "embedding_grad: idx int32/int64 [N]");
   SXE_CHECK(rows >= 0 && rows < 0x7fffffff && n < (1 << 24) && gy.size(1) < (1 << 20), "embedding_grad: sizes");
-  c10::DeviceGuard g(gy.device());
-  auto out = at::zeros({rows, gy.size(1)}, gy.options());
-  if (n == 0 || out.numel() == 0) return out;
+  if (n == 0 || out.numel() == 0) return;
   auto scratch = at::empty({2, n}, idx.options().dtype(at::kInt));
   int *order = scratch.data_ptr<int>(), *sorted = order + n;
   const dim3 grid((n + 63) / 64);
@@ -280,12 +289,30 @@ at::Tensor embedding_grad(const at::Tensor& gy, const at::Tensor& idx, int64_t r
   SXE_LAUNCH_CHECK();
   SXE_DISPATCH_DT(dtype_of(gy), TT, {
     using S = typename dt_traits<TT>::storage;
-    hipLaunchKernelGGL(rows::run_sum_kernel<TT>, dim3((n + 31) / 32, (gy.size(1) + 63) / 64), dim3(256), 0, cur_stream(),
-                       reinterpret_cast<const S*>(gy.data_ptr()), gy.size(1), (int)n, (int)rows, order, sorted,
-                       reinterpret_cast<S*>(out.data_ptr()));
+    auto kern = into ? rows::run_sum_kernel<TT, float> : rows::run_sum_kernel<TT, void>;
+    hipLaunchKernelGGL(kern, dim3((n + 31) / 32, (gy.size(1) + 63) / 64), dim3(256), 0, cur_stream(),
+                       reinterpret_cast<const S*>(gy.data_ptr()), gy.size(1), (int)n, (int)rows, order, sorted, out.data_ptr());
   });
   SXE_LAUNCH_CHECK();
+}
+
+at::Tensor embedding_grad(const at::Tensor& gy, const at::Tensor& idx, int64_t rows) {
+  check_beside(gy, {idx});
+  SXE_CHECK(gy.dim() == 2 && rows >= 0 && rows < 0x7fffffff, "embedding_grad: gy [N, W]");
+  c10::DeviceGuard g(gy.device());
+  auto out = at::zeros({rows, gy.size(1)}, gy.options());
+  embedding_run(gy, idx, out, false);
   return out;
+}
+
+// out fp32 [rows, W] += the same, without a tensor of rows x W between: 2048 tokens of 50257 x 768 8.7 us beside 13 for clearing one,
+// 32 for reading it back and 35 where it met another gradient
+void embedding_grad_(const at::Tensor& gy, const at::Tensor& idx, at::Tensor out) {
+  check_beside(gy, {idx, out});
+  SXE_CHECK(out.scalar_type() == at::kFloat && out.dim() == 2 && out.is_contiguous() && gy.dim() == 2 && out.size(1) == gy.size(1) &&
+                reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0, "embedding_grad_: fp32 out [rows, W] that starts on 16 bytes");
+  c10::DeviceGuard g(gy.device());
+  embedding_run(gy, idx, out, true);
 }
 
 }  // namespace sxe
@@ -293,10 +320,12 @@ at::Tensor embedding_grad(const at::Tensor& gy, const at::Tensor& idx, int64_t r
 TORCH_LIBRARY_FRAGMENT(sxe, m) {
   m.def("gather_rows(Tensor src, Tensor idx, int offset=0, Tensor? add=None) -> Tensor");
   m.def("embedding_grad(Tensor gy, Tensor idx, int rows) -> Tensor");
+  m.def("embedding_grad_(Tensor gy, Tensor idx, Tensor(a!) out) -> ()");
   m.def("scatter_rows_(Tensor(a!) dst, Tensor idx, Tensor src) -> ()");
 }
 TORCH_LIBRARY_IMPL(sxe, CUDA, m) {
   m.impl("gather_rows", &sxe::gather_rows);
   m.impl("embedding_grad", &sxe::embedding_grad);
+  m.impl("embedding_grad_", &sxe::embedding_grad_);
   m.impl("scatter_rows_", &sxe::scatter_rows_);
 }

@@ -57,16 +57,20 @@ class _BiasAct(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, bias, act):
         x = x.contiguous()
+        from .linear import keep_local
         ctx.save_for_backward(x, bias)
         ctx.act = act
+        ctx.bias = keep_local(bias)
         return torch.ops.sxe.bias_act_fwd(x, bias, act)
 
     @staticmethod
     def backward(ctx, dy):
         x, bias = ctx.saved_tensors
         dx = torch.ops.sxe.bias_act_bwd(dy.contiguous(), x, bias, ctx.act)
-        from .linear import column_sum
-        db = column_sum(dx.view(-1, dx.shape[-1]), bias.dtype) if bias is not None else None
+        from .linear import column_sum, write_bias_grad
+        db, d2 = None, dx.view(-1, dx.shape[-1])
+        if bias is not None and not (ctx.needs_input_grad[1] and write_bias_grad(ctx.bias, d2)):
+            db = column_sum(d2, bias.dtype)
         return dx, db, None
 
 

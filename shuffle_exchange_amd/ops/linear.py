@@ -531,6 +531,41 @@ def grad_target(w):
     return tgt
 
 
+def local_grad_target(p):
+    """``grad_target`` of a parameter whose gradient only this rank ever adds up, in fp32 (``_sxe_grad_local``): (buffer, whether it holds
+    a sum), for gradients that may come in several pieces or besides autograd's. None elsewhere, and where hooks of the parameter's
+    gradient want to see it."""
+    if (p is None or not getattr(p, "_sxe_grad_local", False) or p._backward_hooks
+            or len(getattr(p, "_post_accumulate_grad_hooks", None) or ()) > 1):
+        return None
+    tgt = grad_target(p)
+    if tgt is None:
+        return None
+    buf, accumulate = tgt(p)
+    return (buf, bool(accumulate)) if buf.dtype == torch.float32 and buf.is_contiguous() else None
+
+
+def keep_local(p):
+    """``p`` for an autograd function to ask for its target in the backward, if it may have one (not a saved tensor: its values are not
+    read, and may change until then)."""
+    return p if getattr(p, "_sxe_grad_local", False) else None
+
+
+def write_bias_grad(b, gy2):
+    """The column sums of gy2 into the optimizer's buffer of ``b`` (``keep_local``), in fp32: one launch instead of the sum, autograd's
+    accumulation and a conversion. True if written."""
+    if b is None or not (gy2.is_cuda and gy2.dtype in (torch.bfloat16, torch.float16, torch.float32) and gy2.stride(1) == 1
+                         and native.plain(gy2)) or torch.is_grad_enabled():
+        return False
+    tgt = local_grad_target(b)
+    if tgt is None:
+        return False
+    native.require_hip()
+    torch.ops.sxe.column_sum_(gy2, tgt[0].view(-1), tgt[1])
+    b._sxe_grad_done(b)
+    return True
+
+
 def write_weight_grad(w, gy2, x2):
     """dW = gy2^T @ x2 into the optimizer-provided target of `w`; returns True if handled."""
     tgt = grad_target(w)
@@ -612,6 +647,7 @@ class _Linear(torch.autograd.Function):
             bias = bias.to(ac) if bias is not None else None
         ctx.save_for_backward(x, weight)
         ctx.has_bias = bias is not None
+        ctx.bias = keep_local(bias)
         return product(x, weight, bias)
 
     @staticmethod
@@ -628,7 +664,7 @@ class _Linear(torch.autograd.Function):
             x2 = x.reshape(-1, x.shape[-1])
             if not write_weight_grad(wp, gy2, x2):
                 dw = gy2.t() @ x2
-        if ctx.has_bias and ctx.needs_input_grad[2]:
+        if ctx.has_bias and ctx.needs_input_grad[2] and not write_bias_grad(ctx.bias, gy2):
             db = column_sum(gy2, gy2.dtype)
         return dx, dw, db
 
@@ -693,6 +729,7 @@ class _Embed(torch.autograd.Function):
     def forward(ctx, ids, weight):
         ctx.save_for_backward(ids)
         ctx.rows = weight.shape[0]
+        ctx.weight = keep_local(weight)
         return F.embedding(ids, weight)
 
     @staticmethod
@@ -703,7 +740,15 @@ class _Embed(torch.autograd.Function):
         g2 = gy.reshape(-1, gy.shape[-1])
         if not g2.is_contiguous() or g2.data_ptr() % 16:
             g2 = g2.clone(memory_format=torch.contiguous_format)
-        return None, torch.ops.sxe.embedding_grad(g2, ids.reshape(-1).contiguous(), ctx.rows)
+        ids = ids.reshape(-1).contiguous()
+        tgt = None if torch.is_grad_enabled() else local_grad_target(ctx.weight)
+        if tgt is not None and tgt[0].data_ptr() % 16 == 0 and tgt[0].shape == (ctx.rows, g2.shape[1]):
+            if not tgt[1]:
+                tgt[0].zero_()
+            torch.ops.sxe.embedding_grad_(g2, ids, tgt[0])  # only the rows that tokens took
+            ctx.weight._sxe_grad_done(ctx.weight)
+            return None, None
+        return None, torch.ops.sxe.embedding_grad(g2, ids, ctx.rows)
 
 
 EMBED_GRAD_IDS = 16384  # indices up to which ranking them by comparison is the faster way to their gradient (rows.hip)

@@ -35,6 +35,8 @@ class _NormFn(torch.autograd.Function):
         ctx.layernorm = layernorm
         ctx.has_res = residual is not None
         ctx.has_bias = bias is not None
+        from .linear import keep_local
+        ctx.local = (keep_local(weight), keep_local(bias))
         ctx.shape = shape
         y = y.view(shape)
         if residual is not None:
@@ -47,9 +49,20 @@ class _NormFn(torch.autograd.Function):
         H = ctx.shape[-1]
         dy2 = dy.contiguous().view(-1, H)
         dres = dh.contiguous().view(-1, H) if (ctx.has_res and dh is not None) else None
+        from .linear import grad_target, local_grad_target
+        lw, lb = ctx.local
+        if lw is not None and ctx.needs_input_grad[2] and (ctx.needs_input_grad[3] and lb is not None) == ctx.layernorm and not torch.is_grad_enabled():
+            tw, tb = local_grad_target(lw), local_grad_target(lb)
+            if tw is not None and (tb is not None) == ctx.layernorm:  # both sums straight into the optimizer's buffers
+                dx = torch.ops.sxe.norm_bwd_into(dy2, hin, rstd, mean, weight, dres, bool(ctx.layernorm), tw[0].view(-1), tw[1],
+                                                 tb[0].view(-1) if tb is not None else None, tb is not None and tb[1])
+                for p in (lw, lb):
+                    if p is not None:
+                        p._sxe_grad_done(p)
+                dx = dx.view(ctx.shape)
+                return dx, (dx if ctx.has_res else None), None, None, None, None
         dx, dw, db = torch.ops.sxe.norm_bwd(dy2, hin, rstd, mean, weight, dres, bool(ctx.layernorm))
         dx = dx.view(ctx.shape)
-        from .linear import grad_target
         tgt_fn = grad_target(weight)
         if tgt_fn is not None and ctx.needs_input_grad[2]:
             # the fp32 dgamma goes straight into the optimizer's buffer (no bf16 round trip, no

@@ -73,7 +73,7 @@ class ZeroOptimizerBase:
         for units in self.units:
             for u in units:
                 for p in u.params:
-                    for a in ("_sxe_grad_target", "_sxe_grad_done"):
+                    for a in ("_sxe_grad_target", "_sxe_grad_done", "_sxe_grad_local"):
                         if hasattr(p, a):
                             delattr(p, a)
 

@@ -140,8 +140,9 @@ class ZeroStage12Optimizer(ZeroOptimizerBase):
                 # bf16 reduce-scatter staging slot (S > 1) directly
                 p._sxe_grad_target = self._grad_target
                 p._sxe_grad_done = self._grad_done
-                if u.topo.S == 1:  # only this rank ever writes the accumulator: safe to write it late
+                if u.topo.S == 1:  # only this rank ever writes the accumulator: safe to write it late, and more than once
                     p._sxe_grad_defer = self._grad_defer
+                    p._sxe_grad_local = True
 
     def _grad_target(self, p):
         u = self.param_unit[p]

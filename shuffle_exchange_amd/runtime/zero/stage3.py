@@ -426,6 +426,8 @@ class ZeroStage3Optimizer(ZeroOptimizerBase):
             p._sxe_grad_target = self._grad_target
             p._sxe_grad_done = self._grad_done
             p._sxe_grad_defer = self._grad_defer
+            if u.persistent and self.S == 1:
+                p._sxe_grad_local = True
 
     def _grad_defer(self, p):
         """May a weight-gradient producer hold this micro-step's contribution and write it with a

@@ -415,3 +415,96 @@ def test_lamb_kernels_vs_torch_reference():
     assert _rel(m.cpu(), ref_m) < 1e-6 and _rel(v.cpu(), ref_v) < 1e-6
     assert _rel(p.cpu(), out) < 1e-6
     assert torch.equal(lp, p.bfloat16())
+
+
+@pytest.mark.parametrize("R,N", [(1, 1), (3, 64), (130, 5), (2048, 768), (2049, 2304)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_column_sum_into(R, N, dtype):
+    """The sums that ``column_sum`` gives in fp32, written over or added to what is there: one launch and splits, odd columns."""
+    torch.manual_seed(R)
+    x, base = torch.randn(R, N, device="cuda").to(dtype), torch.randn(N, device="cuda")
+    want = torch.ops.sxe.column_sum(x, torch.float32)
+    for accumulate in (False, True):
+        out = base.clone()
+        torch.ops.sxe.column_sum_(x, out, accumulate)
+        assert torch.equal(out, want + base if accumulate else want)
+    out = base.clone()
+    torch.ops.sxe.column_sum_(x[:0], out, True)
+    assert torch.equal(out, base)
+    torch.ops.sxe.column_sum_(x[:0], out, False)
+    assert not out.any()
+
+
+@pytest.mark.parametrize("layernorm", [False, True])
+@pytest.mark.parametrize("rows,H", [(0, 64), (1, 64), (37, 768), (2500, 1000)])
+def test_norm_bwd_into(layernorm, rows, H):
+    torch.manual_seed(rows)
+    x, dy, res = (torch.randn(rows, H, device="cuda").bfloat16() for _ in range(3))
+    w, b = torch.randn(H, device="cuda").bfloat16(), torch.randn(H, device="cuda").bfloat16()
+    y, rstd, mean, _ = torch.ops.sxe.norm_fwd(x, None, w, b if layernorm else None, 1e-5, layernorm)
+    args = (dy, x, rstd, mean if layernorm else None, w, res, layernorm)
+    dx, dw, db = torch.ops.sxe.norm_bwd(*args)
+    for add_w, add_b in ((False, False), (True, False), (False, True), (True, True)):
+        base = torch.randn(2, H, device="cuda")
+        got = base.clone()
+        d = torch.ops.sxe.norm_bwd_into(*args, got[0], add_w, got[1] if layernorm else None, add_b)
+        assert torch.equal(d, dx) and torch.equal(got[0], dw + base[0] if add_w else dw)
+        assert torch.equal(got[1], (db + base[1] if add_b else db) if layernorm else base[1])
+
+
+@pytest.mark.parametrize("n,rows,W", [(1, 1, 8), (100, 7, 72), (1000, 50257, 768), (3000, 3, 64)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_embedding_grad_into(n, rows, W, dtype):
+    """Runs within a block and over many, rows that no index takes stay as they are, indices out of range are left out."""
+    torch.manual_seed(n)
+    idx = torch.randint(0, rows, (n,), device="cuda")
+    idx[n // 2] = rows if n > 1 else 0
+    gy, base = torch.randn(n, W, device="cuda").to(dtype), torch.randn(rows, W, device="cuda")
+    out = base.clone()
+    torch.ops.sxe.embedding_grad_(gy, idx, out)
+    keep = idx < rows
+    want = base.double().index_add(0, idx[keep], gy[keep].double())
+    # fp32 sums of up to n terms in some order
+    size = base.double().abs().index_add(0, idx[keep], gy[keep].double().abs())
+    assert ((out.double() - want).abs() <= 2.0 ** -24 * (4 + n / rows + n ** 0.5) * size).all()
+    untouched = torch.ones(rows, dtype=torch.bool, device="cuda").index_fill(0, idx[keep], False)
+    assert torch.equal(out[untouched], base[untouched])
+
+
+def test_gradients_into_the_optimizers_buffers():
+    """Biases, norms and an embedding whose parameters have a buffer of the optimizer's: the gradients that autograd gives, added up over
+    two passes; a parameter with a hook of its own still hands its gradient to autograd."""
+    from shuffle_exchange_amd.ops.activation import bias_gelu
+    from shuffle_exchange_amd.ops.linear import Embedding, Linear
+    from shuffle_exchange_amd.ops.norm import LayerNorm, RMSNorm
+    torch.manual_seed(0)
+    emb, norm, rms, lin = Embedding(50, 64), LayerNorm(64), RMSNorm(64), Linear(64, 128)
+    mods = torch.nn.ModuleList([emb, norm, rms, lin]).cuda().bfloat16()
+    bias = torch.nn.Parameter(torch.randn(128, device="cuda").bfloat16())
+    ids = torch.randint(0, 50, (2, 150), device="cuda")
+    dy = torch.randn(2, 150, 128, device="cuda").bfloat16()
+    params = [*mods.parameters(), bias]
+
+    def run():
+        x = emb(ids)
+        h, r = norm(x, residual=x)
+        (bias_gelu(lin(rms(h)), bias) * dy).sum().backward()
+    run()
+    want = [2 * p.grad.float() for p in params]
+    bufs, valid = {p: torch.full(p.shape, float("nan"), device="cuda") for p in params}, set()
+
+    def done(p):
+        valid.add(p)
+    for p in params:
+        p.grad = None
+        p._sxe_grad_target, p._sxe_grad_done, p._sxe_grad_local = (lambda q: (bufs[q], q in valid)), done, True
+    for _ in range(2):
+        run()
+    assert len(valid) == len(params) and all(p.grad is None for p in params)
+    for p, w in zip(params, want):  # autograd's were rounded to 8 bits, twice where a parameter's pieces met
+        assert (bufs[p] - w).norm() <= 2 ** -7 * w.norm()
+    seen = []
+    handle = lin.bias.register_hook(lambda g: seen.append(g))
+    run()
+    assert len(seen) == 1 and lin.bias.grad is not None
+    handle.remove()
