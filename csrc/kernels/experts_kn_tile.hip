@@ -48,59 +48,12 @@ __device__ __forceinline__ int tiles_of(const Args& a, int e) {
   return hi > lo ? (hi - lo + BM - 1) / BM : 0;
 }
 
+// The tile of rows r0 .. r1 of an expert (T::BM of them at most, `used` of them with products), columns from n0 on
 template <typename T, bool GLU>
-__global__ void __launch_bounds__(T::NTHR, T::WAVES) tile_kernel(Args a) {
+__device__ __forceinline__ void run_tile(const Args& a, int expert, int r0, int r1, int n0, int used) {
   constexpr int RT = T::RT, CT = T::CT, NW = T::NW, PA = T::PA, PB = T::PB, BM = T::BM, X_LDS = T::SA * T::AS, HC = T::BN / 2;
   static_assert(T::BN == 256 && NW == 8 && PB == 4);
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wr = w / T::WC, wc = w % T::WC;
-  // ---- block -> (expert, column block, row tile), row tiles fastest, consecutive ones on one XCD
-  constexpr int CB = GLU ? HC : 2 * HC;
-  const int tn = (a.cols + CB - 1) / CB;
-  int total = 0;
-  for (int e0 = 0; e0 < a.E; e0 += 64) {
-    int t = tiles_of<BM>(a, e0 + lane);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
-    total += t;
-  }
-  const int nwg = __builtin_amdgcn_readfirstlane(total) * tn, orig = blockIdx.x;
-  if (orig >= nwg) return;
-  const int q8 = nwg / 8, r8 = nwg % 8, xcd = orig % 8;
-  const int id = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + orig / 8;
-  int expert = 0, first = 0, te = 1;
-  {
-    int before = 0;
-    for (int e0 = 0; e0 < a.E; e0 += 64) {
-      const int t = tiles_of<BM>(a, e0 + lane);
-      int inc = t;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int v = __shfl_up(inc, o, 64);
-        if (lane >= o) inc += v;
-      }
-      const unsigned long long hit = __ballot((before + inc) * tn > id);
-      if (hit) {
-        const int l = __builtin_ctzll(hit);
-        expert = e0 + l;
-        te = __shfl(t, l, 64);
-        first = before + __shfl(inc, l, 64) - te;
-        break;
-      }
-      before += __shfl(inc, 63, 64);
-    }
-  }
-  expert = __builtin_amdgcn_readfirstlane(expert);
-  te = __builtin_amdgcn_readfirstlane(te);
-  const int local = id - __builtin_amdgcn_readfirstlane(first) * tn, nt = local / te, rt = local - nt * te;
-  const int r0 = row_of(a, expert) + rt * BM, r1 = row_of(a, expert + 1);
-  const int n0 = nt * CB;
-  int used = r1 - r0;  // rows of the tile with products
-  if (a.rows != nullptr) used = __builtin_amdgcn_readfirstlane(min(used, a.rows[expert] - rt * BM));
-  if (used <= 0 && a.rows != nullptr) {
-    clear_tile(a.y + (int64_t)r0 * a.cols + n0, a.cols, min(BM, r1 - r0), min(CB, a.cols - n0));
-    return;
-  }
-
   // ---- loads: 8 rows of x, chunk c of row r at place c ^ ((r >> 1) & 7); 2 k rows of W, chunk c of row k at place
   // c ^ (4 (k & 3) + 2 ((k >> 3) & 1)). Slabs behind the last repeat it; the second half of one with 32 k repeats its first
   const int ns = a.K / BK, last = (a.K + BK - 1) / BK - 1;
@@ -181,6 +134,72 @@ __global__ void __launch_bounds__(T::NTHR, T::WAVES) tile_kernel(Args a) {
 
 using T256 = Tile<2, 4, 8, 4, 2, 3, 2>;
 using T128 = Tile<2, 4, 4, 4, 3, 3, 2>;
+using T64 = Tile<2, 4, 2, 4, 3, 3, 2>;
+
+// An expert's last tile, of fewer rows, runs as one of 64 or 128 rows (as gemm_tn.hip): six prompts of 50 to 2000
+// tokens through two layers of 8 experts of 4096 x 14336, with the layers' other products, 4.48 / 4.44 ms
+template <typename T, bool GLU>
+__global__ void __launch_bounds__(T::NTHR, T::WAVES) tile_kernel(Args a) {
+  constexpr int BM = T::BM, HC = T::BN / 2;
+  const int lane = threadIdx.x & 63;
+  // ---- block -> (expert, column block, row tile), row tiles fastest, consecutive ones on one XCD
+  constexpr int CB = GLU ? HC : 2 * HC;
+  const int tn = (a.cols + CB - 1) / CB;
+  int total = 0;
+  for (int e0 = 0; e0 < a.E; e0 += 64) {
+    int t = tiles_of<BM>(a, e0 + lane);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+    total += t;
+  }
+  const int nwg = __builtin_amdgcn_readfirstlane(total) * tn, orig = blockIdx.x;
+  if (orig >= nwg) return;
+  const int q8 = nwg / 8, r8 = nwg % 8, xcd = orig % 8;
+  const int id = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + orig / 8;
+  int expert = 0, first = 0, te = 1;
+  {
+    int before = 0;
+    for (int e0 = 0; e0 < a.E; e0 += 64) {
+      const int t = tiles_of<BM>(a, e0 + lane);
+      int inc = t;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += v;
+      }
+      const unsigned long long hit = __ballot((before + inc) * tn > id);
+      if (hit) {
+        const int l = __builtin_ctzll(hit);
+        expert = e0 + l;
+        te = __shfl(t, l, 64);
+        first = before + __shfl(inc, l, 64) - te;
+        break;
+      }
+      before += __shfl(inc, 63, 64);
+    }
+  }
+  expert = __builtin_amdgcn_readfirstlane(expert);
+  te = __builtin_amdgcn_readfirstlane(te);
+  const int local = id - __builtin_amdgcn_readfirstlane(first) * tn, nt = local / te, rt = local - nt * te;
+  const int r0 = row_of(a, expert) + rt * BM, r1 = row_of(a, expert + 1);
+  const int n0 = nt * CB;
+  int used = r1 - r0;  // rows of the tile with products
+  if (a.rows != nullptr) used = __builtin_amdgcn_readfirstlane(min(used, a.rows[expert] - rt * BM));
+  if (used <= 0 && a.rows != nullptr) {
+    clear_tile(a.y + (int64_t)r0 * a.cols + n0, a.cols, min(BM, r1 - r0), min(CB, a.cols - n0));
+    return;
+  }
+  static_assert(T64::LDS <= T::LDS && (BM <= 128 || T128::LDS <= T::LDS) && T64::NTHR == T::NTHR && T128::NTHR == T::NTHR);
+  if (used <= BM / 2) {
+    const int there = min(BM, r1 - r0), small = used <= 64 ? T64::BM : T128::BM;
+    if (there > small)  // rows that are not in use
+      clear_tile(a.y + (int64_t)(r0 + small) * a.cols + n0, a.cols, there - small, min(CB, a.cols - n0));
+    if (used <= 64 || BM <= 128) run_tile<T64, GLU>(a, expert, r0, r1, n0, used);
+    else run_tile<T128, GLU>(a, expert, r0, r1, n0, used);
+    return;
+  }
+  run_tile<T, GLU>(a, expert, r0, r1, n0, used);
+}
 
 static Args args(const at::Tensor& x, const at::Tensor& w) {
   SXE_CHECK_CUDA(x);

@@ -42,30 +42,11 @@ __device__ __forceinline__ int column(int r) {
   return (GLU ? (r >> 6) * 32 : r & ~31) + 8 * (p >> 2) + 4 * b + (p & 3);
 }
 
+// The tile of `used` rows from row m0 on (T::BM rows are stored, as far as there are), columns from n0 on, ns slabs from `first` on
 template <typename T, bool GLU, bool SPLIT>
-__global__ void __launch_bounds__(T::NTHR, T::WAVES) gemm_kernel(Args a) {
-  constexpr int RT = T::RT, CT = T::CT, NW = T::NW, PA = T::PA, PB = T::PB, BM = T::BM, CB = GLU ? T::BN / 2 : T::BN, X_LDS = T::SA * T::AS;
+__device__ __forceinline__ void run_tile(const Args& a, int m0, int n0, int part, int first, int ns, int used) {
+  constexpr int RT = T::RT, CT = T::CT, NW = T::NW, PA = T::PA, PB = T::PB, BM = T::BM, X_LDS = T::SA * T::AS;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wr = w / T::WC, wc = w % T::WC;
-  // ---- workgroup -> (split or product, row tile, column block): neighbours in an XCD's run share w, gm row tiles at a time. The tiles of the
-  // last rows, if these are no whole tile, come behind all others: they take less time and fill the last round
-  const int whole = a.tm * a.tn * a.parts;
-  const bool rest = (int)blockIdx.x >= whole;
-  const int block = rest ? blockIdx.x - whole : blockIdx.x, nwg = rest ? gridDim.x - whole : whole;
-  const int q8 = nwg / 8, r8 = nwg % 8, xcd = block % 8;
-  const int id = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + block / 8;
-  const int nt = rest ? a.tn : a.tm * a.tn, part = a.parts > 1 ? id / nt : 0, tile = id - part * nt;
-  const int per_group = a.gm * a.tn, group = tile / per_group, in = tile - group * per_group, rows = min(a.tm - group * a.gm, a.gm);
-  const int m0 = (rest ? a.tm : group * a.gm + in % rows) * BM, n0 = (rest ? tile : in / rows) * CB;
-  const int first = SPLIT ? part * a.per : 0, ns = SPLIT ? min(a.per, a.slabs - first) : a.slabs;
-  int used = a.M - m0;  // rows of the tile with products
-  if (!SPLIT && a.rows != nullptr) {
-    used = __builtin_amdgcn_readfirstlane(min(used, a.rows[part] - m0));
-    if (used <= 0) {
-      clear_tile(a.y + part * a.by + (int64_t)m0 * a.cols + n0, a.cols, min(BM, a.M - m0), min(CB, a.cols - n0));
-      return;
-    }
-  }
-
   // ---- loads: a wave's load is 8 rows, chunk c of row r at place c ^ ((r >> 1) & 7). Rows and columns behind the last, and slabs,
   // repeat it
   unsigned xo[PA], wo[PB];
@@ -143,6 +124,50 @@ __global__ void __launch_bounds__(T::NTHR, T::WAVES) gemm_kernel(Args a) {
   }
 }
 
+// The last tiles, of fewer rows, run as tiles of 64 or 128 rows: one of 256 with empty blocks of rows takes 0.93 of a whole one's time, as
+// its loads and barriers stay. 28672 x 4096 with SwiGLU, us: 1040 rows 202 / 184, 1088 214 / 188, 1152 234 / 201 (1024: 181).
+using T256 = Tile<2, 4, 8, 4, 2, 3, 2>;   // 256 x 256
+using T192 = Tile<2, 4, 6, 4, 2, 3, 2>;   // 192 x 256
+using T128 = Tile<2, 4, 4, 4, 3, 3, 2>;   // 128 x 256
+using T64 = Tile<2, 4, 2, 4, 3, 3, 2>;    // 64 x 256
+using N128 = Tile<2, 2, 4, 4, 2, 2, 2>;   // 128 x 128, two a CU
+
+template <typename T, bool GLU, bool SPLIT>
+__global__ void __launch_bounds__(T::NTHR, T::WAVES) gemm_kernel(Args a) {
+  constexpr int BM = T::BM, CB = GLU ? T::BN / 2 : T::BN;
+  // ---- workgroup -> (split or product, row tile, column block): neighbours in an XCD's run share w, gm row tiles at a time. The tiles of the
+  // last rows, if these are no whole tile, come behind all others: they take less time and fill the last round
+  const int whole = a.tm * a.tn * a.parts;
+  const bool rest = (int)blockIdx.x >= whole;
+  const int block = rest ? blockIdx.x - whole : blockIdx.x, nwg = rest ? gridDim.x - whole : whole;
+  const int q8 = nwg / 8, r8 = nwg % 8, xcd = block % 8;
+  const int id = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + block / 8;
+  const int nt = rest ? a.tn : a.tm * a.tn, part = a.parts > 1 ? id / nt : 0, tile = id - part * nt;
+  const int per_group = a.gm * a.tn, group = tile / per_group, in = tile - group * per_group, rows = min(a.tm - group * a.gm, a.gm);
+  const int m0 = (rest ? a.tm : group * a.gm + in % rows) * BM, n0 = (rest ? tile : in / rows) * CB;
+  const int first = SPLIT ? part * a.per : 0, ns = SPLIT ? min(a.per, a.slabs - first) : a.slabs;
+  int used = a.M - m0;  // rows of the tile with products
+  if (!SPLIT && a.rows != nullptr) {
+    used = __builtin_amdgcn_readfirstlane(min(used, a.rows[part] - m0));
+    if (used <= 0) {
+      clear_tile(a.y + part * a.by + (int64_t)m0 * a.cols + n0, a.cols, min(BM, a.M - m0), min(CB, a.cols - n0));
+      return;
+    }
+  }
+  if constexpr (T::BN == 256) {
+    static_assert(T64::LDS <= T::LDS && (BM <= 128 || T128::LDS <= T::LDS) && T64::NTHR == T::NTHR && T128::NTHR == T::NTHR);
+    if (used <= (BM > 128 ? 128 : 64)) {
+      const int there = min(BM, a.M - m0), small = used <= 64 ? T64::BM : T128::BM;
+      if (!SPLIT && there > small)  // rows that are not in use
+        clear_tile(a.y + part * a.by + (int64_t)(m0 + small) * a.cols + n0, a.cols, there - small, min(CB, a.cols - n0));
+      if (used <= 64 || BM <= 128) run_tile<T64, GLU, SPLIT>(a, m0, n0, part, first, ns, used);
+      else run_tile<T128, GLU, SPLIT>(a, m0, n0, part, first, ns, used);
+      return;
+    }
+  }
+  run_tile<T, GLU, SPLIT>(a, m0, n0, part, first, ns, used);
+}
+
 // y from the sums of the splits, 8 columns a thread
 template <bool GLU>
 __global__ void __launch_bounds__(256) sum_kernel(const float* __restrict__ part, const unsigned short* __restrict__ bias,
@@ -179,17 +204,12 @@ __global__ void __launch_bounds__(256) sum_kernel(const float* __restrict__ part
   }
 }
 
-using T256 = Tile<2, 4, 8, 4, 2, 3, 2>;   // 256 x 256
-using T192 = Tile<2, 4, 6, 4, 2, 3, 2>;   // 192 x 256
-using T128 = Tile<2, 4, 4, 4, 3, 3, 2>;   // 128 x 256
-using N128 = Tile<2, 2, 4, 4, 2, 2, 2>;   // 128 x 128, two a CU
-
 // The tile and the splits of K that take least by this account: rounds of workgroups over the CUs, each its slabs and a start (with the
-// stores of a round, which all its workgroups issue at once); the tiles of the last, fewer rows take 0.93 of a whole one's time and up,
-// and run on the CUs that the last round of whole ones leaves idle before they lengthen it. us a slab and a start, fitted to 32 weights
-// of 2048 x 2048 to 28672 x 4096 at 33 to 13000 rows with every tile and split (433 sizes): the choice is 0.6 % behind the best on
-// average, 12 % at the most; with the same rest tiles counted as running one after another on an idle CU it was 1.1 and 42 %
-// (1573 rows, 5120 x 5120, 107 us for 80). 256 x 128 and 192 x 128 were never the best.
+// stores of a round, which all its workgroups issue at once); the tiles of the last, fewer rows take what those of 64 or 128 rows take, or
+// 0.93 of a whole one's time and up, and run on the CUs that the last round of whole ones leaves idle before they lengthen it. us a slab
+// and a start, fitted to 32 weights of 2048 x 2048 to 28672 x 4096 at 33 to 13000 rows with every tile and split (433 sizes); with the
+// small last tiles the choice is 0.3 % behind the best on average and 11 % at the most over 200 sizes of 260 to 12000 rows.
+// 256 x 128 and 192 x 128 were never the best.
 struct Form {
   int bm, bn, at_once;
   float slab, start;
@@ -203,12 +223,17 @@ struct Plan {
 // when `rest` tiles of `part` rounds each, on `slots` of which `idle` are free a round earlier, end behind `rounds` rounds
 static float end_of(int64_t rounds, int64_t idle, int64_t slots, int64_t rest, float part) {
   if (rest == 0) return rounds;
-  // k tiles on each idle slot, the others joining in behind the last round; no slot takes more than k + 2 by then
-  for (int64_t k = std::max<int64_t>(1, rest / slots - 2);; ++k) {
-    const float idle_ends = rounds - 1 + k * part, others = std::max(0.f, idle_ends - rounds);
-    if (idle > 0 && idle * k + (slots - idle) * (int64_t)(others / part + 1e-5f) >= rest) return std::max<float>(rounds, idle_ends);
-    if (idle * (int64_t)((1 + k * part) / part + 1e-5f) + (slots - idle) * k >= rest) return rounds + k * part;
-  }
+  const auto fit = [&](float end) {
+    const auto of = [&](float time) { return time > 0 ? (int64_t)(time / part + 1e-4f) : 0; };
+    return idle * of(end - rounds + 1) + (slots - idle) * of(end - rounds) >= rest;
+  };
+  // The last to end is the k-th on a slot that was idle, or the k-th on another. An idle slot takes 3 more at the most, as no part is below 0.5
+  float first = 1e30f, second = 1e30f;
+  for (int64_t k = std::max<int64_t>(1, rest / slots); idle > 0 && first > 1e29f; ++k)
+    if (fit(rounds - 1 + k * part)) first = rounds - 1 + k * part;
+  for (int64_t k = std::max<int64_t>(1, rest / slots - 3); second > 1e29f; ++k)
+    if (fit(rounds + k * part)) second = rounds + k * part;
+  return std::max<float>(rounds, std::min(first, second));
 }
 static Plan plan(int64_t M, int64_t N, int64_t slabs, bool may_split, int64_t batch) {
   Plan best{0, 1, 1e30f};
@@ -220,7 +245,10 @@ static Plan plan(int64_t M, int64_t N, int64_t slabs, bool may_split, int64_t ba
       if (s > 1 && (!may_split || slabs < 4 * s || tiles > 600)) break;
       const float one = (slabs + s - 1) / s * t.slab * (f == 3 && tiles <= kNumCUs ? kAlone : 1.f) + t.start;
       const int64_t whole = M / t.bm * cols * s, rounds = (whole + t.at_once - 1) / t.at_once;
-      float us = one * end_of(rounds, rounds * t.at_once - whole, t.at_once, rest ? cols * s : 0, 0.93f + 0.07f * rest / t.bm);
+      const float part = f == 3 || rest > (t.bm > 128 ? 128 : 64)
+                             ? 0.93f + 0.07f * rest / t.bm
+                             : ((slabs + s - 1) / s * (rest <= 64 ? 0.62f : kForms[2].slab) + kForms[2].start) / one;
+      float us = one * end_of(rounds, rounds * t.at_once - whole, t.at_once, rest ? cols * s : 0, part);
       if (s > 1) us += 6.8f + M * N * 4 * (2 * s + 0.5f) / 6.9e6f;
       if (us < best.us) best = {f, s, us};
     }

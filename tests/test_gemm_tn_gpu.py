@@ -44,6 +44,26 @@ def test_products(M, N, K, apart, splits, tile):
         _close(torch.ops.sxe.gemm_tn(x, w, None, True, tile, splits), F.silu(gate) * up, x, w, 16.0)
 
 
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("M", [base + rest for base in (0, 768) for rest in (1, 63, 64, 65, 127, 128, 129)])
+def test_small_last_tiles(M, splits):
+    """The last rows run as a tile of 64 or 128 rows: the sums are those of whole tiles, in the same order, whichever tile the rest has, and
+    rows behind it that are not in use, zeros, stay zeros."""
+    x, w, b = _operands(M, 528, 320)
+    ref = x.double() @ w.double().t()
+    for glu in (False, True):
+        got = [torch.ops.sxe.gemm_tn(x, w, None if glu else b, glu, tile, splits) for tile in range(4)]
+        assert all(torch.equal(got[0], y) for y in got[1:])
+    _close(torch.ops.sxe.gemm_tn(x, w, None, False, 0, splits), ref, x, w)
+    rows = torch.tensor([M // 2, M], device="cuda", dtype=torch.int32)
+    xb, wb = torch.stack((x, x)), torch.stack((w, w))
+    xb[0, M // 2:] = 0
+    for tile in range(4):
+        y = torch.ops.sxe.gemm_tn_batch(xb, wb, tile, rows)
+        assert not y[0, M // 2:].any() and torch.equal(y[0, :M // 2], y[1, :M // 2])
+        _close(y[1], ref, x, w)
+
+
 def test_infinities_and_nan_stay_in_their_rows():
     x, w, _ = _operands(300, 512, 256)
     x[7, 3], x[299, 0] = float("inf"), float("nan")
