@@ -134,7 +134,10 @@ def glu_linear(x, weight):
 # Fewer rows, long rows of the weight, whose products are split along them: 1.5 times on average, 40 rows, 8192 x 28672 127 / 88, 4096 x 14336
 # 33 / 32, 200 rows 55 / 40, 1100 rows, 3072 x 8192 70 / 64; but up to 128 rows (few workgroups, or rows 32 KB apart) 64 rows, 8192 x 8192 33 / 39,
 # 128 rows, 2048 x 8192 21 / 25, 33 rows, 2048 x 16384 0.74; others do not: 600 rows, 5120 x 3072 26 / 29, 4096 x 4096 28 / 31.
+# From 1025 rows to 1500, wide weights: 1.07 times on average (20 of them, 11 counts each), 1040 rows, 6144 x 4096 55 / 49, 1208, 50304 x
+# 2048 1.27, 1351, 7680 x 2560 1.14, 1237, 28672 x 8192 0.94; but 4608 x 4096 0.96, 4096 x 4096 0.89, 3072 x 3072 0.92; up to 1024 rows 0.96.
 TILED_ROWS, TILED_ROWS_MOST = 1500, 13000
+TILED_ROWS_WIDE, TILED_WIDE, TILED_WIDE_WORK = 1024, 6144, 18 * 10 ** 6
 # SwiGLU of the products in one launch, us, product and activation / here: 16384 x 2048, 330 rows 35 / 29, 2100 rows 144 / 112;
 # 28672 x 4096, 330 rows 85 / 73, 1040 rows 226 / 200, 7588 rows 1390 / 1250; but 240 rows of 16384 x 3072 38 / 43, 72 of 28672 x 4096
 # 59 / 67, and of weights beyond 2^28 elements 493 rows, 57344 x 8192 0.90, 1423 rows 1.02, 3000 rows 1.12
@@ -144,7 +147,7 @@ TILED_GLU_ROWS, TILED_GLU_ROWS_LARGE = 300, 1024
 def _tiled_faster(rows, N, K):
     if N < 2048 or K < 2048:
         return False
-    if rows >= TILED_ROWS:
+    if rows >= TILED_ROWS or (rows > TILED_ROWS_WIDE and N >= TILED_WIDE and N * K >= TILED_WIDE_WORK):
         return rows < TILED_ROWS_MOST and rows % 256 != 0
     if rows <= 128 and (N >= K or K % 16384 == 0 or (rows > 64 and N < 3072)):
         return False

@@ -94,6 +94,12 @@ def test_linear_takes_them(M, N, K, taken, monkeypatch):
     assert L.linear(x.requires_grad_(), w).requires_grad and len(seen) == n
 
 
+def test_wide_weights_rule():
+    from shuffle_exchange_amd.ops.linear import _tiled_faster as own
+    assert own(1025, 6144, 3072) and own(1499, 6144, 3072) and not own(1024, 6144, 3072) and not own(1280, 6144, 3072)
+    assert not own(1025, 6128, 3072) and not own(1025, 6144, 2048)
+
+
 @pytest.mark.parametrize("C", [1, 16, 129, 257, 300])
 @pytest.mark.parametrize("E,K,N", [(1, 64, 128), (3, 192, 320), (8, 64, 576)])
 def test_expert_products(E, C, K, N):
