@@ -29,6 +29,11 @@ namespace sxe {
 
 constexpr int kWave = 64;
 constexpr int kNumCUs = 256;
+// Whether a decode product reads its weight past the caches (nontemporal loads): a weight of a quarter of the last one's 256 MB is gone from it
+// by the next token, with the rest of its model, and makes room for what is read again. us, 16 rows, through the caches / past them:
+// 28672 x 4096 47 / 43, 32000 x 4096 50 / 46, 4096 x 14336 24.4 / 22.8, 4096 x 4096 9.3 / 9.5; where all weights stay in it, 4096 x 4096
+// 6.7 / 7.8, 28672 x 4096 38 / 42; 16 sequences over two layers of 8 experts of 4096 x 14336, a token 1268 / 1178.
+inline bool read_once(int64_t bytes) { return bytes >= 64ll << 20; }
 
 // Dynamic LDS beyond the default limit of 64 KB: a kernel is opted in once on every device.
 template <auto KERN>

@@ -37,7 +37,7 @@ struct Args {
 __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 
 // grid (column tiles, experts that may have rows, K splits)
-template <int MB, bool GATE>
+template <int MB, bool GATE, bool ONCE>
 __global__ void __launch_bounds__(64 * NW, MB == 1 ? 4 : MB == 2 ? 3 : 2) expert_kn_kernel(Args a) {
   extern __shared__ __attribute__((aligned(16))) float part[];  // [NW][16][LDP]
   if ((int)blockIdx.y >= a.active[0]) return;
@@ -68,7 +68,10 @@ __global__ void __launch_bounds__(64 * NW, MB == 1 ? 4 : MB == 2 ? 3 : 2) expert
       for (int u = 0; u < U; ++u) {
         const int k = 32 * min(s + u, s1 - 1);  // past the share: read again, not used
 #pragma unroll
-        for (int j = 0; j < 8; ++j) wf[u][j] = *reinterpret_cast<const u32x4*>(w + (int64_t)(k + j) * a.N);
+        for (int j = 0; j < 8; ++j) {
+          const auto* p = reinterpret_cast<const u32x4*>(w + (int64_t)(k + j) * a.N);
+          wf[u][j] = ONCE ? __builtin_nontemporal_load(p) : *p;
+        }
 #pragma unroll
         for (int m = 0; m < MB; ++m) xf[m][u] = *reinterpret_cast<const u32x4*>(xr[m] + k);
       }
@@ -149,11 +152,12 @@ template <bool GATE>
 void launch(const Args& a, hipStream_t stream) {
   const dim3 grid(a.N / COLS, std::min(a.E, a.R), a.splits);
   const size_t lds = sizeof(float) * NW * 16 * LDP;
-  auto go = [&](auto mb) {
-    constexpr auto kern = &expert_kn_kernel<decltype(mb)::value, GATE>;
+  auto with = [&](auto mb, auto once) {
+    constexpr auto kern = &expert_kn_kernel<decltype(mb)::value, GATE, decltype(once)::value>;
     allow_lds<kern>((int)lds);
     hipLaunchKernelGGL(kern, grid, dim3(64 * NW), lds, stream, a);
   };
+  auto go = [&](auto mb) { read_once(2ll * a.E * a.N * a.K) ? with(mb, std::true_type{}) : with(mb, std::false_type{}); };
   // blocks of 16 rows that share a pass: twice the mean, so that an uneven routing seldom takes a second pass
   if (a.R <= 8 * a.E) go(std::integral_constant<int, 1>{});
   else if (a.R <= 16 * a.E) go(std::integral_constant<int, 2>{});

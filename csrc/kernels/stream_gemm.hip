@@ -71,7 +71,7 @@ __device__ __forceinline__ void exchange(u32x4 (&r)[4], bool odd1, bool odd2) {
 
 // A wave's operands of one piece of K: 256 bytes of every row of W (128 columns of bf16, 256 of e4m3) and the same columns of x.
 // After the exchange lane (row, g) holds chunk 4 g + c of 16 bytes of its row in register c.
-template <bool FP8, int MB, int NT>
+template <bool FP8, int MB, int NT, bool ONCE>
 struct Piece {
   static constexpr int PIECE = FP8 ? 256 : 128, XL = FP8 ? 2 : 1;
   u32x4 w[NT][4], x[MB][XL][4];
@@ -85,7 +85,8 @@ struct Piece {
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         w[t][u] = u32x4{0u, 0u, 0u, 0u};
-        if (win) w[t][u] = *reinterpret_cast<const u32x4*>(wr[t] + u * ldw + (int64_t)kw * (FP8 ? 1 : 2));
+        const auto* p = reinterpret_cast<const u32x4*>(wr[t] + u * ldw + (int64_t)kw * (FP8 ? 1 : 2));
+        if (win) w[t][u] = ONCE ? __builtin_nontemporal_load(p) : *p;
       }
 #pragma unroll
     for (int h = 0; h < XL; ++h) {
@@ -120,7 +121,7 @@ struct Piece {
   }
 };
 
-template <bool FP8, int MB, int NT, bool GLU>
+template <bool FP8, int MB, int NT, bool GLU, bool ONCE>
 __global__ void __launch_bounds__(64 * NW, 2) stream_gemm_kernel(Args a) {
   __shared__ f32x4 red[NW][NT][64];
   constexpr int OT = GLU ? NT / 2 : NT;  // tiles of output columns
@@ -148,7 +149,7 @@ __global__ void __launch_bounds__(64 * NW, 2) stream_gemm_kernel(Args a) {
     for (int t = 0; t < NT; ++t) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // (the next piece in flight behind this one's products halves the workgroups on a CU and gains nothing)
-  using P = Piece<FP8, MB, NT>;
+  using P = Piece<FP8, MB, NT, ONCE>;
   for (int k0 = wave * P::PIECE; k0 < a.K; k0 += NW * P::PIECE) {
     P p;
     p.load(wr, ldw, xr, k0, a.K, c);
@@ -242,19 +243,24 @@ at::Tensor stream_gemm(const at::Tensor& x, const at::Tensor& w, const c10::opti
   const int nt = glu ? (!fp8 && N % 64 == 0 ? 4 : 2) : all >= 384 && (fp8 || M > 16) ? 2 : 1;
   const dim3 grid((all + nt - 1) / nt);
   auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(64 * st::NW), 0, cur_stream(), a); };
-  auto rows = [&](auto mb) {
+  auto rows = [&](auto mb, auto nontemporal) {
     constexpr int MB = decltype(mb)::value;
+    constexpr bool ONCE = decltype(nontemporal)::value;
     if (fp8) {
-      if (glu) go(st::stream_gemm_kernel<true, MB, 2, true>);
-      else nt == 2 ? go(st::stream_gemm_kernel<true, MB, 2, false>) : go(st::stream_gemm_kernel<true, MB, 1, false>);
+      if (glu) go(st::stream_gemm_kernel<true, MB, 2, true, ONCE>);
+      else nt == 2 ? go(st::stream_gemm_kernel<true, MB, 2, false, ONCE>) : go(st::stream_gemm_kernel<true, MB, 1, false, ONCE>);
     } else if (glu) {
-      nt == 4 ? go(st::stream_gemm_kernel<false, MB, 4, true>) : go(st::stream_gemm_kernel<false, MB, 2, true>);
+      nt == 4 ? go(st::stream_gemm_kernel<false, MB, 4, true, ONCE>) : go(st::stream_gemm_kernel<false, MB, 2, true, ONCE>);
     } else {
-      nt == 2 ? go(st::stream_gemm_kernel<false, MB, 2, false>) : go(st::stream_gemm_kernel<false, MB, 1, false>);
+      nt == 2 ? go(st::stream_gemm_kernel<false, MB, 2, false, ONCE>) : go(st::stream_gemm_kernel<false, MB, 1, false, ONCE>);
     }
   };
-  if (M <= 16) rows(std::integral_constant<int, 1>{});
-  else rows(std::integral_constant<int, 2>{});
+  auto blocks = [&](auto nontemporal) {
+    if (M <= 16) rows(std::integral_constant<int, 1>{}, nontemporal);
+    else rows(std::integral_constant<int, 2>{}, nontemporal);
+  };
+  if (read_once(N * K * (fp8 ? 1 : 2))) blocks(std::true_type{});
+  else blocks(std::false_type{});
   SXE_LAUNCH_CHECK();
   return y;
 }

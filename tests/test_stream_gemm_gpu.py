@@ -48,6 +48,22 @@ def test_gated(M, N, K, fp8):
     assert got.shape == (M, N // 2) and (got.double() - want).norm() < 3e-3 * want.norm()
 
 
+@pytest.mark.parametrize("M", [5, 17])
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("fp8,N,K", [(False, 8256, 4112), (True, 16416, 4112), (True, 16448, 4096)])
+def test_weights_read_past_the_caches(M, fp8, N, K, glu):
+    """From 64 MB on the weight is loaded another way: the same bits as of its pieces, which are smaller."""
+    x, w, s, _ = _operands(M, N, K, fp8, M + N + K)
+    got = torch.ops.sxe.stream_gemm(x, w, s, None, glu)
+    half = N // 2
+    for a in range(0, half if glu else N, 2064):
+        b = min(a + 2064, half if glu else N)
+        part = torch.cat((w[a:b], w[half + a:half + b])) if glu else w[a:b]
+        scale = None if s is None else torch.cat((s[a:b], s[half + a:half + b])) if glu else s[a:b]
+        assert part.numel() * part.element_size() < 64 << 20
+        assert torch.equal(got[:, a:b], torch.ops.sxe.stream_gemm(x, part.contiguous(), scale, None, glu))
+
+
 def test_linear_routes_by_rows():
     """The rule's two sides agree: the streaming kernel, the library and the few-row kernel within one rounding of each other."""
     from shuffle_exchange_amd.ops.fp_quantizer import FP8Weight

@@ -24,7 +24,8 @@ def _reference(x, logits, k, w_gu, w_down):
 
 
 @pytest.mark.parametrize("T", [1, 2, 7, 16, 33, 100, 256])
-@pytest.mark.parametrize("E,k,K,I,N", [(8, 2, 256, 192, 128), (4, 1, 32, 64, 256), (8, 2, 2080, 1088, 384), (3, 3, 96, 64, 128)])
+@pytest.mark.parametrize("E,k,K,I,N", [(8, 2, 256, 192, 128), (4, 1, 32, 64, 256), (8, 2, 2080, 1088, 384), (3, 3, 96, 64, 128),
+                                       (8, 2, 2080, 1088, 4096)])  # the last: from 64 MB on weights are loaded another way
 @pytest.mark.parametrize("skew", [False, True])
 def test_streaming_kernels(T, E, k, K, I, N, skew, monkeypatch):
     from shuffle_exchange_amd.ops import moe
