@@ -62,7 +62,10 @@ def _skinny(x, weight, bias):
 # library / streaming, 16 rows: 3072 x 2048 11.2 / 6.0, 4096 x 4096 14.9 / 9.6, 6144 x 4096 14.0 / 14.6, 28672 x 4096 60 / 47,
 # 4096 x 14336 25.5 / 25.3, 15360 x 5120 33.5 / 34.2, 8192 x 8192 28.5 / 28.9; but 5120 x 5120 15.2 / 17.2, 5120 x 13824 31.9 / 39.1,
 # 10240 x 8192 34.1 / 38.4, 2048 x 8192 12.7 / 13.0, 50264 x 768 18.3 / 20.6. 24 rows: 2048 x 2048 8.4 / 5.9, 4096 x 4096
-# 12.8 / 11.6; but 5120 x 3072 11.6 / 13.5, 6144 x 4096 14.4 / 16.1, 1024 x 8192 11.6 / 15.1, 11264 x 2048 14.6 / 15.7.
+# 12.8 / 11.6; but 5120 x 3072 11.6 / 13.5, 6144 x 4096 14.4 / 16.1, 1024 x 8192 11.6 / 15.1, 11264 x 2048 14.6 / 15.7. Wide weights, 32
+# columns a workgroup, in a captured sequence of weights that are each read once, 24 rows: 32000 x 4096 60.6 / 52.2, 32000 x 2048 32.5 /
+# 27.6, 128256 x 4096 191 / 186, 65536 x 4096 121 / 99, 16384 x 4096 31.8 / 29.8, 8192 x 3072 18.4 / 13.9 (32 rows: 64000 x 2560 60.7 /
+# 62.4, 32000 x 3072 37.2 / 38.3); but 12288 x 4096 23.6 / 26.9, 9216 x 3072 17.1 / 19.5, 8192 x 4096 16.7 / 18.3.
 STREAM_ROWS, STREAM_ROWS_SMALL = 16, 32
 
 
@@ -74,7 +77,8 @@ def _full_rounds(workgroups):
 
 def _stream_faster(rows, N, K):
     if rows > STREAM_ROWS:
-        return rows <= STREAM_ROWS_SMALL and K <= 4096 and (N <= 4096 or N * K <= 1 << 23)
+        return rows <= STREAM_ROWS_SMALL and K <= 4096 and (N <= 4096 or N * K <= 1 << 23 or ((N >= 16384 or K <= 3072)
+                                                                                              and _full_rounds(N / 32) > 0.93))
     return not (K >= 5120 and N * K >= 1 << 24 and _full_rounds(N / 16) < 0.9) and not (K < 1024 and N > 16384)
 
 

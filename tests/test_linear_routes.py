@@ -307,3 +307,10 @@ def test_glu_rule_and_switch(monkeypatch):
         assert L.glu_tiled(x, w) is not None and L.glu_tiled(x[:300], w) is None and L.glu_tiled(xl, large) is None
         monkeypatch.setattr(L, "SKINNY_MAX_M", 0)
         assert L.glu_tiled(x, w) is None
+
+
+@pytest.mark.parametrize("rows,N,K,own", [(17, 32000, 4096, True), (32, 16384, 4096, True), (24, 8192, 4096, False), (24, 8192, 3072, True),
+                                          (24, 9216, 3072, False), (33, 32000, 4096, False), (24, 32000, 4104, False)])
+def test_few_row_rule_of_wide_weights(rows, N, K, own):
+    from shuffle_exchange_amd.ops.linear import _stream_faster
+    assert _stream_faster(rows, N, K) == own
