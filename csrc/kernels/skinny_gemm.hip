@@ -467,26 +467,19 @@ inline int pick_nw(int tiles, int ss_total, int min_ss, int wg8_per_cu) {
 
 // ---- FP8-weight variant (W8A16: e4m3 weights, per-output-row fp32 scale, bf16 activations) ----
 // Same structure; each lane streams 16 bytes = 16 weights per load and converts them to bf16 in
-// registers (v_cvt_f32_fp8; e4m3 values are exact in bf16), so the weight bytes -- the whole
+// registers (e4m3 values are exact in bf16), so the weight bytes -- the whole
 // cost of a decode GEMM -- are halved. MFMA step (j, h) of a 512-wide super-step uses
 // K = k0 + 64 j + 16 g + 8 h + [0, 8) for lane group g, for weights and activations alike.
 constexpr int kSS8 = 512;
 
 __device__ __forceinline__ bf16x8 fp8x8_to_bf16(uint2 w) {
-  // byte-selected v_cvt_f32_fp8 (byte b of the word -> element b): explicit order, e4m3 is exact
-  // in bf16 so the top half of the f32 bit pattern is the bf16 value
-  bf16x8 r;
-#define SXE_FP8_BYTE(word, b) (short)(__builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_f32_fp8((int)(word), b)) >> 16)
-  r[0] = SXE_FP8_BYTE(w.x, 0);
-  r[1] = SXE_FP8_BYTE(w.x, 1);
-  r[2] = SXE_FP8_BYTE(w.x, 2);
-  r[3] = SXE_FP8_BYTE(w.x, 3);
-  r[4] = SXE_FP8_BYTE(w.y, 0);
-  r[5] = SXE_FP8_BYTE(w.y, 1);
-  r[6] = SXE_FP8_BYTE(w.y, 2);
-  r[7] = SXE_FP8_BYTE(w.y, 3);
-#undef SXE_FP8_BYTE
-  return r;
+  // exact, two an instruction (at a scale of 1), of the lower or the upper half of a word
+  unsigned r __attribute__((ext_vector_type(4)));
+  r[0] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w.x, 1.f, false));
+  r[1] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w.x, 1.f, true));
+  r[2] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w.y, 1.f, false));
+  r[3] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w.y, 1.f, true));
+  return __builtin_bit_cast(bf16x8, r);
 }
 
 template <int NW, int MODE, int CW>

@@ -36,15 +36,14 @@ struct Args {
 __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
-// 8 e4m3 bytes -> bf16 (exact: the upper half of the fp32 value)
+// 8 e4m3 bytes -> bf16, exact, two an instruction (at a scale of 1). By way of fp32, three for two, it took 28672 x 4096, 8 rows, gated
+// 28.6 us, now 26.3, 32000 x 4096 28.8 / 26.5, 4096 x 4096 7.6 / 7.5 (with loads past the caches)
 __device__ __forceinline__ u32x4 widen(unsigned lo, unsigned hi) {
   u32x4 r;
-#define SXE_W(word, b) __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_f32_fp8((int)(word), b))
-  r[0] = __builtin_amdgcn_perm(SXE_W(lo, 1), SXE_W(lo, 0), 0x07060302u);
-  r[1] = __builtin_amdgcn_perm(SXE_W(lo, 3), SXE_W(lo, 2), 0x07060302u);
-  r[2] = __builtin_amdgcn_perm(SXE_W(hi, 1), SXE_W(hi, 0), 0x07060302u);
-  r[3] = __builtin_amdgcn_perm(SXE_W(hi, 3), SXE_W(hi, 2), 0x07060302u);
-#undef SXE_W
+  r[0] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.f, false));
+  r[1] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.f, true));
+  r[2] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.f, false));
+  r[3] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.f, true));
   return r;
 }
 

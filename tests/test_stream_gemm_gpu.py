@@ -37,6 +37,15 @@ def test_plain(M, N, K, fp8):
         assert (got.double() - want).norm() < 3e-3 * want.norm()
 
 
+def test_every_e4m3_value_is_exact():
+    w = torch.arange(256, device="cuda", dtype=torch.uint8).view(16, 16)
+    one = torch.ones(16, device="cuda")
+    y = torch.ops.sxe.stream_gemm(torch.eye(16, device="cuda").bfloat16(), torch.where(w & 127 == 127, 0, w), one, None, False)
+    want = torch.where(w & 127 == 127, 0, w).view(torch.float8_e4m3fn).float()
+    assert torch.equal(y.float(), want.T) and not torch.ops.sxe.stream_gemm(torch.ones(1, 16, device="cuda").bfloat16(), w, one, None,
+                                                                            False)[:, 7::8].isfinite().any()
+
+
 @pytest.mark.parametrize("M", [5, 16, 32])
 @pytest.mark.parametrize("N,K", [(32, 32), (96, 512), (64, 4096), (28672, 128)])
 @pytest.mark.parametrize("fp8", [False, True])
