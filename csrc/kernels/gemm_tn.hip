@@ -28,7 +28,8 @@ struct Args {
   const unsigned short *x, *w, *bias;
   unsigned short* y;
   const int* rows;       // of a batch: rows of each product that are not zeros, the first ones; null: all
-  float* part;           // splits of K: their sums, [splits, M, N]
+  float* part;           // splits of K: their sums, [splits, M, N]; or y in fp32, one split
+  bool add;              // y in fp32: added to what is there
   int64_t ldx, ldw, bx, bw, by;  // elements from row to row, and from product to product of a batch
   int M, cols, half, slabs, per, parts;  // columns of y (SwiGLU: half the rows of w); w row that goes with row 0 as up; slabs of K, of a split;
                                          // splits of K, or products of a batch
@@ -93,7 +94,9 @@ __device__ __forceinline__ void run_tile(const Args& a, int m0, int n0, int part
 #pragma unroll
         for (int j = 0; j < CT; ++j) {
           const int b = GLU ? (j >> 1) & 1 : j & 1, c = n0 + (GLU ? wc * CT * 8 : (wc * CT + (j & ~1)) * 16) + 8 * g + 4 * b;
-          if (c < a.cols) *reinterpret_cast<f32x4*>(p + c + (GLU && (j & 1) ? a.cols : 0)) = acc[i][j];
+          if (c >= a.cols) continue;
+          f32x4* to = reinterpret_cast<f32x4*>(p + c + (GLU && (j & 1) ? a.cols : 0));
+          *to = a.add ? *to + acc[i][j] : acc[i][j];
         }
       } else {
         const int c = n0 + wc * CT * 8 + 8 * g;
@@ -265,10 +268,10 @@ static void launch(Args a, int splits, int batch) {
   a.parts = splits * batch;  // one of them is 1
   const int64_t grid = ((int64_t)a.M + T::BM - 1) / T::BM * a.tn * a.parts;
   SXE_CHECK(grid < (1ll << 30), "gemm_tn: too many tiles");
-  if (splits > 1) {
+  if (a.part != nullptr) {
     allow_lds<&gemm_kernel<T, GLU, true>>(T::LDS);
     hipLaunchKernelGGL((gemm_kernel<T, GLU, true>), dim3((unsigned)grid), dim3(T::NTHR), T::LDS, cur_stream(), a);
-    hipLaunchKernelGGL(sum_kernel<GLU>, dim3(stream_grid((int64_t)a.M * a.cols / 8, 256)), dim3(256), 0, cur_stream(), a.part, a.bias, a.y,
+    if (splits > 1) hipLaunchKernelGGL(sum_kernel<GLU>, dim3(stream_grid((int64_t)a.M * a.cols / 8, 256)), dim3(256), 0, cur_stream(), a.part, a.bias, a.y,
                        a.M, a.cols, splits);
   } else {
     allow_lds<&gemm_kernel<T, GLU, false>>(T::LDS);
@@ -279,10 +282,11 @@ static void launch(Args a, int splits, int batch) {
 
 }  // namespace tn
 
-// x, w [.., rows, K], one product or a batch; out: y's sizes where they are not those of one product
+// x, w [.., rows, K], one product or a batch; out: y's sizes where they are not those of one product; into: y in fp32, written or added to
 static at::Tensor gemm_tn_run(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, bool glu, int64_t tile, int64_t splits,
-                              at::IntArrayRef out = {}, const c10::optional<at::Tensor>& rows = c10::nullopt) {
-  check_beside(x, {w, bias, rows});
+                              at::IntArrayRef out = {}, const c10::optional<at::Tensor>& rows = c10::nullopt,
+                              const c10::optional<at::Tensor>& into = c10::nullopt, bool add = false) {
+  check_beside(x, {w, bias, rows, into});
   const int64_t d = x.dim() - 2, batch = d ? x.size(0) : 1, M = x.size(d), K = x.size(d + 1), N = w.size(d), cols = glu ? N / 2 : N;
   SXE_CHECK(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 && w.size(d + 1) == K && (!d || w.size(0) == batch),
             "gemm_tn: bf16 x [M, K], w [N, K]");
@@ -299,13 +303,18 @@ static at::Tensor gemm_tn_run(const at::Tensor& x, const at::Tensor& w, const c1
                           reinterpret_cast<uintptr_t>(bias->data_ptr()) % 16 == 0), "gemm_tn: bias bf16 [N]");
   SXE_CHECK(tile < 4 && splits >= 0 && splits <= 64, "gemm_tn: tile 0 - 3 or -1, splits 0 - 64");
   c10::DeviceGuard g(x.device());
-  auto y = d ? at::empty({batch, M, cols}, x.options()) : out.empty() ? at::empty({M, cols}, x.options()) : at::empty(out, x.options());
+  auto y = into.has_value() ? *into : d ? at::empty({batch, M, cols}, x.options()) : out.empty() ? at::empty({M, cols}, x.options()) : at::empty(out, x.options());
   if (y.numel() == 0) return y;
   tn::Args a{};
   a.x = reinterpret_cast<const unsigned short*>(x.data_ptr());
   a.w = reinterpret_cast<const unsigned short*>(w.data_ptr());
   a.bias = has_bias ? reinterpret_cast<const unsigned short*>(bias->data_ptr()) : nullptr;
-  a.y = reinterpret_cast<unsigned short*>(y.data_ptr());
+  if (into.has_value()) {
+    a.part = y.data_ptr<float>();
+    a.add = add;
+  } else {
+    a.y = reinterpret_cast<unsigned short*>(y.data_ptr());
+  }
   a.ldx = ldx;
   a.ldw = ldw;
   a.rows = used_rows(rows, batch);
@@ -355,6 +364,13 @@ at::Tensor gemm_tn(const at::Tensor& x, const at::Tensor& w, const c10::optional
   return gemm_tn_run(x.view({-1, x.size(-1)}), w, bias, glu, tile, splits, out);
 }
 
+// c [M, N] fp32 (+)= x [M, K] . w [N, K]^T: a weight gradient whose operands lie with the tokens side by side
+void gemm_tn_into(const at::Tensor& x, const at::Tensor& w, at::Tensor c, bool add, int64_t tile) {
+  SXE_CHECK(x.dim() == 2 && w.dim() == 2 && c.dim() == 2 && c.size(0) == x.size(0) && c.size(1) == w.size(0) && c.scalar_type() == at::kFloat &&
+                c.is_contiguous() && reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 == 0, "gemm_tn_into: bf16 x [M, K], w [N, K], fp32 c [M, N]");
+  gemm_tn_run(x, w, c10::nullopt, false, tile, 1, {}, c10::nullopt, c, add);
+}
+
 // x [B, M, K], w [B, N, K] -> [B, M, N], one launch; rows int32 [B]: x[b, rows[b]:] is zeros, and so is y
 at::Tensor gemm_tn_batch(const at::Tensor& x, const at::Tensor& w, int64_t tile, const c10::optional<at::Tensor>& rows) {
   SXE_CHECK(x.dim() == 3 && w.dim() == 3, "gemm_tn_batch: bf16 x [B, M, K], w [B, N, K]");
@@ -365,9 +381,11 @@ at::Tensor gemm_tn_batch(const at::Tensor& x, const at::Tensor& w, int64_t tile,
 
 TORCH_LIBRARY_FRAGMENT(sxe, m) {
   m.def("gemm_tn(Tensor x, Tensor w, Tensor? bias, bool glu, int tile=-1, int splits=0) -> Tensor");
+  m.def("gemm_tn_into(Tensor x, Tensor w, Tensor(a!) c, bool add, int tile=-1) -> ()");
   m.def("gemm_tn_batch(Tensor x, Tensor w, int tile=-1, Tensor? rows=None) -> Tensor");
 }
 TORCH_LIBRARY_IMPL(sxe, CUDA, m) {
   m.impl("gemm_tn", &sxe::gemm_tn);
+  m.impl("gemm_tn_into", &sxe::gemm_tn_into);
   m.impl("gemm_tn_batch", &sxe::gemm_tn_batch);
 }

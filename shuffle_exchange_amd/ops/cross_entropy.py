@@ -17,7 +17,7 @@ import torch
 import torch.nn.functional as F
 
 from . import native
-from .linear import product
+from .linear import keep_local, local_grad_target, product
 
 
 class _XEnt(torch.autograd.Function):
@@ -74,6 +74,7 @@ class _ColumnHeadXEnt(torch.autograd.Function):
         # the rows that were rounded up are kept beside h: making them again costs 2368 x 768 a fill and a copy, 8 us
         ctx.save_for_backward(logits, lse, tgt, h, h2 if h2.data_ptr() != h.data_ptr() else None, weight)
         ctx.ignore_index = int(ignore_index)
+        ctx.weight = keep_local(weight)
         return loss.view(target.shape)
 
     @staticmethod
@@ -95,7 +96,13 @@ class _ColumnHeadXEnt(torch.autograd.Function):
             torch.ops.sxe.wgrad_gemm_(g, weight, dh, 1.0, False)
             dh = dh[:tgt.numel()].to(h2.dtype).view(h.shape)
         if ctx.needs_input_grad[1]:
-            dw = torch.ops.sxe.gemm_tn(g, torch.ops.sxe.transpose16(h2), None, False)
+            into = local_grad_target(ctx.weight)
+            # in fp32 into the optimizer's buffer: no gradient of the table is written, read and added up besides
+            if into is not None and into[0].shape == weight.shape and into[0].data_ptr() % 16 == 0:
+                torch.ops.sxe.gemm_tn_into(g, torch.ops.sxe.transpose16(h2), *into)
+                ctx.weight._sxe_grad_done(ctx.weight)
+            else:
+                dw = torch.ops.sxe.gemm_tn(g, torch.ops.sxe.transpose16(h2), None, False)
         return dh, dw, None, None
 
 

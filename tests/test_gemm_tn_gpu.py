@@ -64,6 +64,42 @@ def test_small_last_tiles(M, splits):
         _close(y[1], ref, x, w)
 
 
+@pytest.mark.parametrize("tile", [0, 1, 2, 3, -1])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (129, 264, 192), (321, 776, 640)])
+def test_products_in_32_bits(M, N, K, tile):
+    """Written to and added to a buffer in fp32: the sums before their rounding; nothing behind it is touched."""
+    x, w, _ = _operands(M, N, K)
+    ref, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    behind = torch.full((M * N + 8,), float("nan"), device="cuda")
+    c = behind[:M * N].view(M, N)
+    for times in (1, 2):  # each sum is off by at most K 2^-24 of the magnitudes' sum
+        torch.ops.sxe.gemm_tn_into(x, w, c, times == 2, tile)
+        assert bool(((c.double() - times * ref).abs() <= times * (K + 2) * 2.0 ** -24 * size).all())
+    assert bool(behind[M * N:].isnan().all())
+    with pytest.raises(RuntimeError):
+        torch.ops.sxe.gemm_tn_into(x, w, c[:, :-1], False)
+
+
+def test_head_gradient_into_the_optimizers_buffer():
+    """A table that embeds and ends a model: both gradients meet in the buffer, as autograd's sum of them does."""
+    from shuffle_exchange_amd.ops.cross_entropy import head_cross_entropy
+    from shuffle_exchange_amd.ops.linear import Embedding
+    torch.manual_seed(0)
+    emb = Embedding(515, 128).cuda().bfloat16()
+    ids = torch.randint(0, 515, (2, 75), device="cuda")
+    p, valid = emb.weight, []
+
+    def run():
+        head_cross_entropy(emb(ids), p, ids).backward()
+    run()
+    want, p.grad = 2 * p.grad.float(), None
+    buf = torch.full(p.shape, float("nan"), device="cuda")
+    p._sxe_grad_target, p._sxe_grad_done, p._sxe_grad_local = (lambda q: (buf, bool(valid))), valid.append, True
+    run()
+    run()
+    assert len(valid) == 4 and p.grad is None and (buf - want).norm() <= 2 ** -7 * want.norm()  # autograd's pieces were rounded to 8 bits
+
+
 def test_infinities_and_nan_stay_in_their_rows():
     x, w, _ = _operands(300, 512, 256)
     x[7, 3], x[299, 0] = float("inf"), float("nan")
