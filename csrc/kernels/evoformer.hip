@@ -27,6 +27,7 @@
 // dbias2 apart (forward 62, dQ 68, dK / dV 76, dbias2 79); 238 now (forward 58, dQ + dbias2 95, dK / dV 83).
 #include "sxe_gemm_loop.h"
 #include <torch/library.h>
+#include <climits>
 #include <type_traits>
 
 namespace sxe {
@@ -263,9 +264,9 @@ __device__ __forceinline__ void store_rows(const f32x16 (&acc)[D / 32], unsigned
 
 // ------------------------------------------------------------------------------------ forward
 // A workgroup takes the same 128 queries of NN of the N rows; a step is two 32 x 32 tiles a wave, one of each row (NN = 2) or two of
-// the one.
+// the one. Which: evo_single.
 template <int D, bool PAIR, int NN>
-__global__ void __launch_bounds__(256, (min_waves<D>())) fwd_kernel(Args a, unsigned short* __restrict__ out) {
+__global__ void __launch_bounds__(256, (NN == 1 ? 3 : min_waves<D>())) fwd_kernel(Args a, unsigned short* __restrict__ out) {
   using St = Stream<D, NN>;
   constexpr int SUB = 2 / NN;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, hf = lane >> 5;
@@ -309,19 +310,23 @@ __global__ void __launch_bounds__(256, (min_waves<D>())) fwd_kernel(Args a, unsi
     for (int u = 0; u < 2; ++u) s[u] = mfma(kmf[u], ones(), bias[u / NN]);
     if (t + 1 < n) load(t + 1);
     if (q0 < a.L) {
+      constexpr bool EARLY = D == 32 || NN == 2;  // else operands just ahead of their products: 161 registers, three waves a SIMD
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+      for (int u = 0; u < 2; ++u) {
+        if constexpr (!EARLY) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int t2 = 0; t2 < D / 16; ++t2)
           s[u] = mfma(row_at(slot + 2 * St::TILE * (u % NN) + 64 * D * (u / NN), lo.row[t2]), qf[u % NN][t2], s[u]);
-      bf16x8 vf[2][2][D / 32];  // read here: in front of their products the wave would wait for each
+      }
+      bf16x8 vf[2][2][D / 32];  // read here where registers allow: in front of their products the wave would wait for each
+      auto values = [&](int u, int s2) {
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+        for (int dt = 0; dt < D / 32; ++dt)
+          vf[u][s2][dt] = tr_at(slot + 2 * St::TILE * (u % NN) + St::TILE + (32 * (u / NN) + 16 * s2) * 2 * D, lo.tr[dt]);
+      };
 #pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-          for (int dt = 0; dt < D / 32; ++dt)
-            vf[u][s2][dt] = tr_at(slot + 2 * St::TILE * (u % NN) + St::TILE + (32 * (u / NN) + 16 * s2) * 2 * D, lo.tr[dt]);
+      for (int i = 0; i < 4; ++i)
+        if constexpr (EARLY) values(i / 2, i % 2);
       if constexpr (D == 32) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < NN; ++i) {
@@ -355,6 +360,10 @@ __global__ void __launch_bounds__(256, (min_waves<D>())) fwd_kernel(Args a, unsi
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
+          if constexpr (!EARLY) {
+            __builtin_amdgcn_sched_barrier(0);
+            values(u, s2);
+          }
           const bf16x8 pb = acc_to_b(s[u], s2);
 #pragma unroll
           for (int dt = 0; dt < D / 32; ++dt)
@@ -952,6 +961,16 @@ static void evo_dispatch(int D, bool pair, F f) {
 
 static int evo_grid(const evo::Args& a, int rows) { return a.B * ((a.N + rows - 1) / rows) * a.H * (a.Lp / evo::QB); }
 
+// Whether the forward and dQ take one of the N rows a workgroup: two share the pair bias, but grids of up to `most` workgroups a CU are
+// better off with twice as many. us of all launches, two rows / one (128 queries, 8 heads; workgroups of two rows): forward, head dim
+// 64, three waves a SIMD instead of two, 20 x 500 (320) 43.1 / 36.8, 64 x 256 (512) 31.2 / 27.7, 128 x 384 (1536) 89.8 / 77.9; but 256 x
+// 512, 4 heads (2048) 131 / 134, 8 heads 281 / 295; without a pair bias 82.2 / 66.2 at 1536, 257 / 221 at 4096; head dim 32: 20 x 500
+// 34.4 / 30.7, 512 22.8 / 22.0, 800 24.1 / 23.7; but 960 56.4 / 57.6, 1024 26.6 / 30.6. Backward with dQ that way, head dim 64: 320
+// 117 / 110, 520 100.6 / 98.1, 800 102.6 / 103.1, 2048 578 / 584, head dim 32, 500 keys: 320 88.9 / 84.3, 960 180.3 / 180.4. Without a
+// pair bias, head dim 32, forward 60 x 500 (960) 43.9 / 38.1, 1536 49.3 / 44.8, backward 106 / 96, 123 / 120; but 4096 156 / 169, 447 /
+// 464, and 64 keys (1024), where a second row has its first step at once, 15.4 / 18.2, 29.6 / 35.6.
+static bool evo_single(const evo::Args& a, int64_t most) { return evo_grid(a, 2) <= most * kNumCUs; }
+
 // -> [o, lse, packed biases of evo_pack]: the backward reads these, not the biases, which the caller may have changed by then
 std::vector<at::Tensor> evoformer_fwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
                                       const c10::optional<at::Tensor>& b1, const c10::optional<at::Tensor>& b2, bool backward) {
@@ -969,9 +988,14 @@ std::vector<at::Tensor> evoformer_fwd(const at::Tensor& q, const at::Tensor& k, 
   a.lse = lse.data_ptr<float>();
   evo_dispatch(q.size(4), c.pair, [&](auto d, auto t) {
     constexpr int D = decltype(d)::value;
-    constexpr int NN = 2, LDS = 2 * evo::Stream<D, NN>::SLOT;
-    hipLaunchKernelGGL((evo::fwd_kernel<D, decltype(t)::value, NN>), dim3(evo_grid(a, NN)), dim3(256), LDS, cur_stream(), a,
-                       reinterpret_cast<unsigned short*>(o.data_ptr()));
+    constexpr bool PAIR = decltype(t)::value;
+    auto rows = [&](auto nn) {
+      constexpr int NN = decltype(nn)::value, LDS = 2 * evo::Stream<D, NN>::SLOT;
+      hipLaunchKernelGGL((evo::fwd_kernel<D, PAIR, NN>), dim3(evo_grid(a, NN)), dim3(256), LDS, cur_stream(), a,
+                         reinterpret_cast<unsigned short*>(o.data_ptr()));
+    };
+    if (evo_single(a, D == 64 ? (PAIR ? 7 : INT_MAX) : !PAIR && a.L > 128 ? 6 : 3)) rows(std::integral_constant<int, 1>{});
+    else rows(std::integral_constant<int, 2>{});
   });
   SXE_LAUNCH_CHECK();
   return packed;
@@ -1021,7 +1045,7 @@ std::vector<at::Tensor> evoformer_bwd(const at::Tensor& dout, const at::Tensor& 
   evo_dispatch(q.size(4), c.pair, [&](auto dd, auto t) {
     constexpr int D = decltype(dd)::value;
     constexpr bool PAIR = decltype(t)::value;
-    constexpr int NN = 2, NK = D == 32 ? 2 : 1, LDS = 2 * evo::Stream<D, NN>::SLOT, LDSK = 2 * evo::QueryStream<D, NK>::SLOT;
+    constexpr int NK = D == 32 && PAIR ? 2 : 1, LDSK = 2 * evo::QueryStream<D, NK>::SLOT;
     bool both = false;
     if constexpr (PAIR && D == 32) {
       both = need_db2 && a.L <= 384;
@@ -1051,7 +1075,14 @@ std::vector<at::Tensor> evoformer_bwd(const at::Tensor& dout, const at::Tensor& 
         else run(evo::DqPair<2, 4, 3>{}, evo::dq_pair_kernel<2, 4, 3>, 64);
       }
     }
-    if (!both) hipLaunchKernelGGL((evo::dq_kernel<D, PAIR, NN>), dim3(evo_grid(a, NN)), dim3(256), LDS, cur_stream(), a, dqp);
+    auto dq_rows = [&](auto nn) {
+      constexpr int NN = decltype(nn)::value, LDS = 2 * evo::Stream<D, NN>::SLOT;
+      hipLaunchKernelGGL((evo::dq_kernel<D, PAIR, NN>), dim3(evo_grid(a, NN)), dim3(256), LDS, cur_stream(), a, dqp);
+    };
+    if (!both) {
+      if (evo_single(a, !PAIR && a.L > 128 ? 6 : 3)) dq_rows(std::integral_constant<int, 1>{});
+      else dq_rows(std::integral_constant<int, 2>{});
+    }
     auto dkdv = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3(evo_grid(a, NK)), dim3(256), LDSK, cur_stream(), a, dkp, dvp,
                          need_db1 ? db1.data_ptr<float>() : nullptr);

@@ -173,3 +173,25 @@ def test_evoformer_key_blocks(D, L, N):
     assert (out.double() - want).norm() <= 8e-3 * want.norm()
     for a, b in zip(grads, torch.autograd.grad(want, ref, g.double())):
         assert torch.isfinite(a).all() and (a.double() - b).norm() <= 8e-3 * b.norm(), a.shape
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,N,L", [(32, 191, 40), (32, 193, 40), (64, 191, 40), (64, 193, 40), (64, 447, 40), (64, 449, 40), (32, 49, 400)])
+@pytest.mark.parametrize("pair", [True, False])
+def test_evoformer_rows_of_a_workgroup(D, N, L, pair):
+    """Both sides of the grids from which on a workgroup takes two of the N rows, with a last workgroup of one."""
+    torch.manual_seed(6)
+    H = 8
+    mk = lambda *s: torch.randn(*s, device="cuda")
+    ins = [mk(1, N, L, H, D).bfloat16() for _ in range(3)] + [(mk(1, N, 1, 1, L) > 1).float() * -30.0]
+    g = mk(1, N, L, H, D).bfloat16()
+    ins = [t.requires_grad_(True) for t in ins + ([(mk(1, 1, H, L, L) * 2).bfloat16()] if pair else [])]
+    out = ea.evoformer_attention(*ins)
+    grads = torch.autograd.grad(out, ins, g)
+    ref = [t.detach().double().requires_grad_(True) for t in ins]
+    q, k, v = (t.transpose(-2, -3) for t in ref[:3])
+    want = (torch.softmax(sum(ref[4:], q @ k.transpose(-1, -2).contiguous() / D ** 0.5 + ref[3]), -1) @ v).transpose(-2, -3)
+    # as above: p, ds and the results are rounded to 8 bits, 4 x 2^-9
+    assert (out.double() - want).norm() <= 8e-3 * want.norm()
+    for a, b in zip(grads, torch.autograd.grad(want, ref, g.double())):
+        assert torch.isfinite(a).all() and (a.double() - b).norm() <= 8e-3 * b.norm(), a.shape
