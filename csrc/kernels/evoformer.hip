@@ -310,7 +310,7 @@ __global__ void __launch_bounds__(256, (NN == 1 ? 3 : min_waves<D>())) fwd_kerne
     for (int u = 0; u < 2; ++u) s[u] = mfma(kmf[u], ones(), bias[u / NN]);
     if (t + 1 < n) load(t + 1);
     if (q0 < a.L) {
-      constexpr bool EARLY = D == 32 || NN == 2;  // else operands just ahead of their products: 161 registers, three waves a SIMD
+      constexpr bool EARLY = D == 32 || NN == 2;  // else operands one product ahead: 167 registers, three waves a SIMD
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         if constexpr (!EARLY) __builtin_amdgcn_sched_barrier(0);
@@ -326,7 +326,7 @@ __global__ void __launch_bounds__(256, (NN == 1 ? 3 : min_waves<D>())) fwd_kerne
       };
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        if constexpr (EARLY) values(i / 2, i % 2);
+        if (EARLY || i < 1) values(i / 2, i % 2);
       if constexpr (D == 32) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < NN; ++i) {
@@ -362,7 +362,8 @@ __global__ void __launch_bounds__(256, (NN == 1 ? 3 : min_waves<D>())) fwd_kerne
         for (int s2 = 0; s2 < 2; ++s2) {
           if constexpr (!EARLY) {
             __builtin_amdgcn_sched_barrier(0);
-            values(u, s2);
+            const int next = 2 * u + s2 + 1;
+            if (next < 4) values(next / 2, next % 2);
           }
           const bf16x8 pb = acc_to_b(s[u], s2);
 #pragma unroll
@@ -963,8 +964,9 @@ static int evo_grid(const evo::Args& a, int rows) { return a.B * ((a.N + rows - 
 
 // Whether the forward and dQ take one of the N rows a workgroup: two share the pair bias, but grids of up to `most` workgroups a CU are
 // better off with twice as many. us of all launches, two rows / one (128 queries, 8 heads; workgroups of two rows): forward, head dim
-// 64, three waves a SIMD instead of two, 20 x 500 (320) 43.1 / 36.8, 64 x 256 (512) 31.2 / 27.7, 128 x 384 (1536) 89.8 / 77.9; but 256 x
-// 512, 4 heads (2048) 131 / 134, 8 heads 281 / 295; without a pair bias 82.2 / 66.2 at 1536, 257 / 221 at 4096; head dim 32: 20 x 500
+// 64, three waves a SIMD instead of two, 20 x 500 (320) 43.1 / 36.8, 64 x 256 (512) 31.2 / 27.7, 128 x 384 (1536) 89.8 / 77.9 (values
+// read right before their products; one product ahead 126 x 359 goes from 49.5 to 47.5, 8 heads 84.4 to 82.0); but 256 x 512, 4 heads
+// (2048) 131 / 134, 8 heads 281 / 295; without a pair bias 82.2 / 66.2 at 1536, 257 / 221 at 4096; head dim 32: 20 x 500
 // 34.4 / 30.7, 512 22.8 / 22.0, 800 24.1 / 23.7; but 960 56.4 / 57.6, 1024 26.6 / 30.6. Backward with dQ that way, head dim 64: 320
 // 117 / 110, 520 100.6 / 98.1, 800 102.6 / 103.1, 2048 578 / 584, head dim 32, 500 keys: 320 88.9 / 84.3, 960 180.3 / 180.4. Without a
 // pair bias, head dim 32, forward 60 x 500 (960) 43.9 / 38.1, 1536 49.3 / 44.8, backward 106 / 96, 123 / 120; but 4096 156 / 169, 447 /
