@@ -508,8 +508,8 @@ def _narrow_data_grad(gy, w):
     300 rows 14 / 33 / 20; on the host 19 / 8 / 13. None where they do not cover the operands."""
     N, K = w.shape
     if not (_narrow(gy.numel() // max(1, gy.shape[-1]), N, K) and gy.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and N % 64 == 0
-            and K % 64 == 0 and gy.is_contiguous() and w.is_cuda and w.is_contiguous() and gy.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and _own_products(gy, w)):
+            and K % 64 == 0 and gy.is_contiguous() and w.is_cuda and w.is_contiguous() and _own_products(gy, w)
+            and gy.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):  # last: compilation has no memory to look at
         return None
     native.require_hip()
     if N <= 1280:
@@ -523,7 +523,7 @@ def data_grad(gy, w):
             and w.dim() == 2 and w.is_contiguous() and w.numel() >= DGRAD_WT_MIN_ELEMS and w.shape[0] % 64 == 0
             and w.shape[1] % 64 == 0):
         rows = gy.numel() // gy.shape[-1]
-        if rows >= 2048 or (_wt_few_faster(rows, *w.shape) and gy.is_contiguous() and gy.data_ptr() % 16 == 0 and _own_products(gy, w)):
+        if rows >= 2048 or (_wt_few_faster(rows, *w.shape) and gy.is_contiguous() and _own_products(gy, w) and gy.data_ptr() % 16 == 0):
             return product(gy, _transposed_weight(w))
     if gy.is_cuda and w.dim() == 2:
         dx = _narrow_data_grad(gy, w)

@@ -295,6 +295,31 @@ def test_data_gradient_of_few_rows(monkeypatch):
         assert torch.equal(L.data_grad(gy, w), gy @ w) and seen == [1]
 
 
+@pytest.mark.parametrize("rows,N,K", [(512, 2048, 512), (2048, 1024, 2816), (300, 2304, 768), (300, 16384, 2048)])
+def test_products_of_training_compile(rows, N, K):
+    """No question that compilation cannot answer (where an operand lies) is on the way of a product or its data gradient: without a
+    GPU, on fake tensors of one."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from shuffle_exchange_amd.ops.linear import data_grad, product
+
+    class Product(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x, w):
+            ctx.save_for_backward(x, w)
+            return product(x, w)
+
+        @staticmethod
+        def backward(ctx, gy):
+            x, w = ctx.saved_tensors
+            return data_grad(gy, w), gy.t() @ x
+    torch._dynamo.reset()
+    with FakeTensorMode():
+        x, w = (torch.empty(n, K, device="cuda", dtype=torch.bfloat16, requires_grad=True) for n in (rows, N))
+        y = torch.compile(Product.apply, fullgraph=True, backend=lambda graph, inputs: graph)(x, w)
+    assert y.shape == (rows, N)
+
+
 @gpu
 def test_glu_rule_and_switch(monkeypatch):
     """SwiGLU of many rows in the product's launch, not of few rows of the largest weights, nor where the library's products are asked for."""
