@@ -74,11 +74,14 @@ __device__ __forceinline__ float bounded(float x) {  // inf and NaN stay
 
 // ------------------------------------------------------------------------------------ bias packing
 // One launch for both. bias1 (null: none) [B N, L] -> mask [B N, Lp] * log2(e) and km [B N, Lp, 16] * sqrt(D), -inf behind L:
-// the blocks of the first grid row. A row whose largest bias is far below zero (every key masked by a large
-// finite number) is moved up to zero: the softmax is the same, and its scores keep their fractions.
+// the blocks of the first grid row. A row of either bias whose largest value is far below zero (every key masked by a large
+// finite number) is moved up to zero, one of bias1 far above it down: the softmax is the same, and its scores keep their
+// fractions. (One of bias2 is read whole only where a tile's part of it lies there.)
 // bias2 [B H, L, L] * sqrt(D) -> 32 x 32 fp32 tiles in accumulator order: element (tile (a, b), quarter i / 4, lane, i % 4) is
 // the value of register i of that lane. pq: lane = query of tile row a, registers = keys of b; pk (may be null): lane = key of
 // tile row a, registers = queries of b. Grid: (nt * nt, B H + 1), nt = Lp / 32; without bias2 (64, 1).
+constexpr float MASKED = 1e4f;
+__device__ __forceinline__ float lift(float top) { return top < -MASKED && top > -INFINITY ? top : 0.f; }
 template <typename T>
 __global__ void __launch_bounds__(256) pack_kernel(const void* __restrict__ b1, int b1_bf16, float* __restrict__ mask,
                                                    unsigned short* __restrict__ km, int64_t rows, const T* __restrict__ b2,
@@ -104,7 +107,7 @@ __global__ void __launch_bounds__(256) pack_kernel(const void* __restrict__ b1, 
       __syncthreads();
       top = fmaxf(fmaxf(tops[0], tops[1]), fmaxf(tops[2], tops[3]));
       __syncthreads();
-      const float up = top < -1e4f && top > -INFINITY ? top : 0.f;
+      const float up = top > MASKED && top < INFINITY ? top : lift(top);
       for (int key = threadIdx.x; key < Lp; key += 256) {
         const float x = bounded(at(key) - up);
         mask[row * Lp + key] = x * LOG2E;
@@ -119,10 +122,26 @@ __global__ void __launch_bounds__(256) pack_kernel(const void* __restrict__ b1, 
   const int a = blockIdx.x / nt, b = blockIdx.x - a * nt;
   const int64_t bh = blockIdx.y - 1;
   const T* src = b2 + bh * L * L;
-  for (int i = threadIdx.x; i < 1024; i += 256) {
-    const int q = 32 * a + i / 32, k = 32 * b + i % 32;
-    t[i / 32][i % 32] = q < L && k < L ? bounded(value(src[(int64_t)q * L + k])) * root : 0.f;
+  const int r0 = threadIdx.x / 8, q = 32 * a + r0, k = 32 * b + 4 * (threadIdx.x % 8);  // eight threads a row
+  const T* row = src + (int64_t)q * L;
+  auto row_top = [](float y) {
+#pragma unroll
+    for (int o = 4; o > 0; o >>= 1) y = fmaxf(y, __shfl_xor(y, o));
+    return y;
+  };
+  float v[4], top = -INFINITY;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    v[e] = q < L && k + e < L ? value(row[k + e]) : 0.f;
+    if (k + e < L) top = fmaxf(top, v[e]);
   }
+  float up = lift(row_top(top));
+  if (up != 0.f) {  // (so q < L: the others' values are zeros)
+    for (int i = threadIdx.x % 8; i < L; i += 8) top = fmaxf(top, value(row[i]));
+    up = lift(row_top(top));
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) t[r0][4 * (threadIdx.x % 8) + e] = bounded(v[e] - up) * root;  // behind L they meet a mask of -inf, or zeros
   __syncthreads();
   const int64_t tiles = bh * nt * nt;
   const int g = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 31;

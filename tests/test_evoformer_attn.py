@@ -195,3 +195,38 @@ def test_evoformer_rows_of_a_workgroup(D, N, L, pair):
     assert (out.double() - want).norm() <= 8e-3 * want.norm()
     for a, b in zip(grads, torch.autograd.grad(want, ref, g.double())):
         assert torch.isfinite(a).all() and (a.double() - b).norm() <= 8e-3 * b.norm(), a.shape
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,N,L", [(32, 5, 70), (32, 5, 257), (32, 5, 400), (32, 200, 40), (64, 5, 133), (64, 400, 40)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_evoformer_masked_queries(D, N, L, dtype):
+    """Queries whose keys are all masked by one large finite number of the pair bias: their softmax is that of the other terms, forward
+    and backward, also where they share keys with a part of the row mask; and a row mask that is large above zero."""
+    torch.manual_seed(7)
+    H = 8
+    mk = lambda *s: torch.randn(*s, device="cuda")
+    Q, K, V, g = (mk(1, N, L, H, D).bfloat16() for _ in range(4))
+    b1 = (mk(1, N, 1, 1, L) > 1).float() * -1e9
+    b1[..., 0] = 0
+    b1[0, 1] = mk(L) + 3e4
+    b1[0, 2] = 0
+    b1[0, 2, 0, 0, 0] = 1e9
+    b2 = (mk(1, 1, H, L, L) * 2).to(dtype)
+    b2[0, 0, 1] = -1e9
+    b2[0, 0, 2, L - 1] = -3e8
+    b2[0, 0, 3, 5] = -20480.0 + (mk(L) > 0) * -128.0
+    b2[0, 0, 4, 3, 1:] = -1e9  # a key is left: nothing to move
+    b2[0, 0, 5, :, L // 3:] = -1e9
+    ins = [t.requires_grad_(True) for t in (Q, K, V, b1, b2)]
+    out = ea.evoformer_attention(*ins)
+    grads = torch.autograd.grad(out, ins, g)
+    ref = [t.detach().double().requires_grad_(True) for t in ins]
+    q, k, v = (t.transpose(-2, -3) for t in ref[:3])
+    want = (torch.softmax(q @ k.transpose(-1, -2).contiguous() / D ** 0.5 + ref[3] + ref[4], -1) @ v).transpose(-2, -3)
+    # p, ds and the results are rounded to 8 bits, 4 x 2^-9
+    assert (out.double() - want).norm() <= 8e-3 * want.norm()
+    for a, b in zip(grads, torch.autograd.grad(want, ref, g.double())):
+        assert torch.isfinite(a).all() and (a.double() - b).norm() <= 8e-3 * b.norm(), a.shape
+        if a.shape == Q.shape:  # and of the head whose keys are all masked alone
+            assert (a[:, :, :, 1].double() - b[:, :, :, 1]).norm() <= 8e-3 * b[:, :, :, 1].norm()
