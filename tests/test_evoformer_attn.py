@@ -177,7 +177,7 @@ def test_evoformer_key_blocks(D, L, N):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("D,N,L", [(32, 191, 40), (32, 193, 40), (64, 191, 40), (64, 193, 40), (64, 447, 40), (64, 449, 40), (32, 49, 400)])
-@pytest.mark.parametrize("pair", [True, False])
+@pytest.mark.parametrize("pair", [torch.bfloat16, torch.float32, None])
 def test_evoformer_rows_of_a_workgroup(D, N, L, pair):
     """Both sides of the grids from which on a workgroup takes two of the N rows, with a last workgroup of one."""
     torch.manual_seed(6)
@@ -185,7 +185,7 @@ def test_evoformer_rows_of_a_workgroup(D, N, L, pair):
     mk = lambda *s: torch.randn(*s, device="cuda")
     ins = [mk(1, N, L, H, D).bfloat16() for _ in range(3)] + [(mk(1, N, 1, 1, L) > 1).float() * -30.0]
     g = mk(1, N, L, H, D).bfloat16()
-    ins = [t.requires_grad_(True) for t in ins + ([(mk(1, 1, H, L, L) * 2).bfloat16()] if pair else [])]
+    ins = [t.requires_grad_(True) for t in ins + ([(mk(1, 1, H, L, L) * 2).to(pair)] if pair else [])]
     out = ea.evoformer_attention(*ins)
     grads = torch.autograd.grad(out, ins, g)
     ref = [t.detach().double().requires_grad_(True) for t in ins]
@@ -230,3 +230,13 @@ def test_evoformer_masked_queries(D, N, L, dtype):
         assert torch.isfinite(a).all() and (a.double() - b).norm() <= 8e-3 * b.norm(), a.shape
         if a.shape == Q.shape:  # and of the head whose keys are all masked alone
             assert (a[:, :, :, 1].double() - b[:, :, :, 1]).norm() <= 8e-3 * b[:, :, :, 1].norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,N,dtype", [(64, 400, torch.bfloat16), (32, 191, torch.bfloat16), (32, 193, torch.bfloat16), (64, 3, torch.float32)])
+def test_evoformer_packed_biases(D, N, dtype):
+    """What the forward keeps for the backward: the pair bias in its own type, and a key of the mask takes 20 bytes."""
+    q = torch.randn(1, N, 40, 8, D, device="cuda").bfloat16()
+    b2 = torch.randn(1, 1, 8, 40, 40, device="cuda").to(dtype)
+    _, _, mask, pair = torch.ops.sxe.evoformer_fwd(q, q, q, None, b2, True)
+    assert pair.dtype == dtype and pair.shape == (2, 8, 128, 128) and mask.nbytes == 20 * N * 128
