@@ -69,7 +69,7 @@ class _BiasAct(torch.autograd.Function):
         dx = torch.ops.sxe.bias_act_bwd(dy.contiguous(), x, bias, ctx.act)
         from .linear import column_sum, write_bias_grad
         db, d2 = None, dx.view(-1, dx.shape[-1])
-        if bias is not None and not (ctx.needs_input_grad[1] and write_bias_grad(ctx.bias, d2)):
+        if bias is not None and not (ctx.needs_input_grad[1] and write_bias_grad(ctx.bias, d2, ctx)):
             db = column_sum(d2, bias.dtype)
         return dx, db, None
 

@@ -545,12 +545,24 @@ def grad_target(w):
     return tgt
 
 
-def local_grad_target(p):
-    """``grad_target`` of a parameter whose gradient only this rank ever adds up, in fp32 (``_sxe_grad_local``): (buffer, whether it holds
-    a sum), for gradients that may come in several pieces or besides autograd's. None elsewhere, and where hooks of the parameter's
-    gradient want to see it."""
+def _accumulates(ctx, p):
+    """Whether the backward that runs ``ctx`` adds the gradient of ``p`` up: not ``torch.autograd.grad``, which returns it, nor a backward
+    of other ``inputs``. 1 us."""
+    for node, _ in ctx.next_functions:
+        if node is not None and getattr(node, "variable", None) is p:
+            try:
+                return torch._C._will_engine_execute_node(node)
+            except RuntimeError:  # the gradient of p itself is asked for
+                return False
+    return False
+
+
+def local_grad_target(p, ctx):
+    """``grad_target`` of a parameter whose gradient only this rank ever adds up, in fp32 (``_sxe_grad_local``), in the backward of
+    ``ctx``: (buffer, whether it holds a sum), for gradients that may come in several pieces or besides autograd's. None elsewhere, where
+    hooks of the parameter's gradient want to see it, and where the caller of autograd does."""
     if (p is None or not getattr(p, "_sxe_grad_local", False) or p._backward_hooks
-            or len(getattr(p, "_post_accumulate_grad_hooks", None) or ()) > 1):
+            or len(getattr(p, "_post_accumulate_grad_hooks", None) or ()) > 1 or not native.plain(p) or not _accumulates(ctx, p)):
         return None
     tgt = grad_target(p)
     if tgt is None:
@@ -565,13 +577,13 @@ def keep_local(p):
     return p if getattr(p, "_sxe_grad_local", False) else None
 
 
-def write_bias_grad(b, gy2):
+def write_bias_grad(b, gy2, ctx):
     """The column sums of gy2 into the optimizer's buffer of ``b`` (``keep_local``), in fp32: one launch instead of the sum, autograd's
     accumulation and a conversion. True if written."""
     if b is None or not (gy2.is_cuda and gy2.dtype in (torch.bfloat16, torch.float16, torch.float32) and gy2.stride(1) == 1
                          and native.plain(gy2)) or torch.is_grad_enabled():
         return False
-    tgt = local_grad_target(b)
+    tgt = local_grad_target(b, ctx)
     if tgt is None:
         return False
     native.require_hip()
@@ -678,7 +690,7 @@ class _Linear(torch.autograd.Function):
             x2 = x.reshape(-1, x.shape[-1])
             if not write_weight_grad(wp, gy2, x2):
                 dw = gy2.t() @ x2
-        if ctx.has_bias and ctx.needs_input_grad[2] and not write_bias_grad(ctx.bias, gy2):
+        if ctx.has_bias and ctx.needs_input_grad[2] and not write_bias_grad(ctx.bias, gy2, ctx):
             db = column_sum(gy2, gy2.dtype)
         return dx, dw, db
 
@@ -755,7 +767,7 @@ class _Embed(torch.autograd.Function):
         if not g2.is_contiguous() or g2.data_ptr() % 16:
             g2 = g2.clone(memory_format=torch.contiguous_format)
         ids = ids.reshape(-1).contiguous()
-        tgt = None if torch.is_grad_enabled() else local_grad_target(ctx.weight)
+        tgt = None if torch.is_grad_enabled() else local_grad_target(ctx.weight, ctx)
         if tgt is not None and tgt[0].data_ptr() % 16 == 0 and tgt[0].shape == (ctx.rows, g2.shape[1]):
             if not tgt[1]:
                 tgt[0].zero_()

@@ -52,7 +52,7 @@ class _NormFn(torch.autograd.Function):
         from .linear import grad_target, local_grad_target
         lw, lb = ctx.local
         if lw is not None and ctx.needs_input_grad[2] and (ctx.needs_input_grad[3] and lb is not None) == ctx.layernorm and not torch.is_grad_enabled():
-            tw, tb = local_grad_target(lw), local_grad_target(lb)
+            tw, tb = local_grad_target(lw, ctx), local_grad_target(lb, ctx)
             if tw is not None and (tb is not None) == ctx.layernorm:  # both sums straight into the optimizer's buffers
                 dx = torch.ops.sxe.norm_bwd_into(dy2, hin, rstd, mean, weight, dres, bool(ctx.layernorm), tw[0].view(-1), tw[1],
                                                  tb[0].view(-1) if tb is not None else None, tb is not None and tb[1])

@@ -508,3 +508,31 @@ def test_gradients_into_the_optimizers_buffers():
     run()
     assert len(seen) == 1 and lin.bias.grad is not None
     handle.remove()
+
+
+def test_gradients_that_autograd_is_asked_for():
+    """``torch.autograd.grad`` with respect to parameters that have a buffer of the optimizer's returns their gradients, and a backward of
+    other inputs leaves their buffers alone."""
+    from shuffle_exchange_amd.ops.activation import bias_gelu
+    from shuffle_exchange_amd.ops.cross_entropy import head_cross_entropy
+    from shuffle_exchange_amd.ops.linear import Embedding, Linear
+    from shuffle_exchange_amd.ops.norm import LayerNorm
+    torch.manual_seed(0)
+    emb, norm, lin = Embedding(515, 128).cuda().bfloat16(), LayerNorm(128).cuda().bfloat16(), Linear(128, 128).cuda().bfloat16()
+    bias = torch.nn.Parameter(torch.randn(128, device="cuda").bfloat16())
+    ids = torch.randint(0, 515, (2, 150), device="cuda")
+    params = [emb.weight, norm.bias, lin.bias, bias]
+    start = torch.randn(2, 150, 128, device="cuda").bfloat16().requires_grad_()
+
+    def loss():
+        return head_cross_entropy(bias_gelu(lin(norm(emb(ids) + start)), bias), emb.weight, ids)
+    want = torch.autograd.grad(loss(), params)
+    bufs, valid = {p: torch.full(p.shape, float("nan"), device="cuda") for p in (*params, norm.weight, lin.weight)}, set()
+    for p in bufs:
+        p._sxe_grad_target, p._sxe_grad_done, p._sxe_grad_local = (lambda q: (bufs[q], q in valid)), valid.add, True
+    for g, w in zip(torch.autograd.grad(loss(), params), want):
+        assert g.dtype == w.dtype and torch.equal(g, w)
+    loss().backward(inputs=[start])
+    assert start.grad is not None and not valid & set(params) and all(p.grad is None for p in params)
+    loss().backward()
+    assert valid == set(bufs)

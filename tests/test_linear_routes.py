@@ -320,6 +320,34 @@ def test_products_of_training_compile(rows, N, K):
     assert y.shape == (rows, N)
 
 
+def test_optimizers_buffer_is_for_backward():
+    """``local_grad_target``: where the backward adds a parameter's gradient up, not where its caller asks for it or for others."""
+    from shuffle_exchange_amd.ops.linear import keep_local, local_grad_target
+    p, q, buf, seen = torch.nn.Parameter(torch.ones(3)), torch.nn.Parameter(torch.ones(3)), torch.zeros(3), []
+    p._sxe_grad_target, p._sxe_grad_local = (lambda t: (buf, False)), True
+    assert keep_local(q) is None
+
+    class Scale(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, number, x, w):
+            ctx.w = keep_local(w)
+            return number * x * w
+
+        @staticmethod
+        def backward(ctx, gy):
+            seen.append(local_grad_target(ctx.w, ctx) is not None)
+            return None, gy, gy
+    run = lambda: Scale.apply(1.0, q * 2, p).sum()  # noqa: E731
+    run().backward()
+    run().backward(inputs=[q])
+    torch.autograd.grad(run(), [p])
+    torch.autograd.grad(run(), [q])
+    assert seen == [True, False, False, False]
+    p.grad = None
+    run().backward(inputs=[p])
+    assert seen[4]
+
+
 @gpu
 def test_glu_rule_and_switch(monkeypatch):
     """SwiGLU of many rows in the product's launch, not of few rows of the largest weights, nor where the library's products are asked for."""
