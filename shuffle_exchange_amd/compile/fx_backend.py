@@ -22,6 +22,7 @@ import itertools
 
 import torch
 
+from ..ops.linear import drop_grad_target
 from ..utils.logging import log_dist
 from .fx_graph import GraphParams, ProfilingInterpreter, insert_grad_reduce, reduce_order, sink_reduces
 
@@ -152,9 +153,7 @@ def compile_fx(engine, cfg, compile_kwargs=None):
     for p in engine.module.parameters():
         # weight-gradient GEMMs writing straight into ZeRO buffers (ops/linear.py) are an eager-mode
         # shortcut with Python side effects inside backward; the graph's reduce nodes replace them
-        for a in ("_sxe_grad_target", "_sxe_grad_done"):
-            if hasattr(p, a):
-                delattr(p, a)
+        drop_grad_target(p)
     if any(p.is_cuda for p in engine.module.parameters()):
         from ..ops import native
         native.require_hip()  # loaded before tracing: the dispatch predicates then stay lock-free

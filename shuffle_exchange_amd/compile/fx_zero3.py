@@ -31,6 +31,7 @@ import logging
 
 import torch
 
+from ..ops.linear import drop_grad_target
 from ..utils.logging import log_dist
 from .fx_backend import FXCompiler, _ACTIVE
 from .fx_graph import GraphParams, insert_grad_reduce, output_node, sink_reduces, reduce_order
@@ -229,9 +230,7 @@ def compile_fx_zero3(engine, cfg, compile_kwargs=None):
     opt = engine.optimizer
     assert hasattr(opt, "fgroups"), "compile_fx_zero3 needs the ZeRO-3 optimizer"
     for p in engine.module.parameters():
-        for a in ("_sxe_grad_target", "_sxe_grad_done"):
-            if hasattr(p, a):
-                delattr(p, a)
+        drop_grad_target(p)
     if any(p.is_cuda for p in engine.module.parameters()):
         from ..ops import native
         native.require_hip()  # loaded before tracing: the dispatch predicates then stay lock-free

@@ -545,6 +545,12 @@ def grad_target(w):
     return tgt
 
 
+def drop_grad_target(p):
+    """Give the gradient of ``p`` back to autograd: nothing of the optimizer's direct target stays on the parameter."""
+    for a in ("_sxe_grad_target", "_sxe_grad_done", "_sxe_grad_local"):
+        p.__dict__.pop(a, None)
+
+
 def _accumulates(ctx, p):
     """Whether the backward that runs ``ctx`` adds the gradient of ``p`` up: not ``torch.autograd.grad``, which returns it, nor a backward
     of other ``inputs``. 1 us."""

@@ -15,6 +15,7 @@ ZeRO optimizer reduces everything in one epilogue and steps.
 import torch
 
 from ... import comm as dist
+from ...ops.linear import drop_grad_target
 from ...utils.logging import log_dist
 from ..engine import SXEEngine
 from . import schedule as S
@@ -50,9 +51,7 @@ class PipelineEngine(SXEEngine):
             self.data_iterator = iter(RepeatingLoader(self.training_dataloader))
         # tied weights are summed across stages before the ZeRO reduction: keep their grads in .grad
         for p in self.module.tied_parameters():
-            for a in ("_sxe_grad_target", "_sxe_grad_done"):
-                if hasattr(p, a):
-                    delattr(p, a)
+            drop_grad_target(p)
         n_local = sum(p.numel() for p in self.module.parameters())
         log_dist(f"pipeline: {self.num_stages} stages, micro_batches={self.micro_batches}, stage {self.stage_id} "
                  f"holds {n_local} params", ranks=[0])

@@ -12,6 +12,7 @@ import torch
 
 from ... import comm as dist
 from ...ops import optim as fused
+from ...ops.linear import drop_grad_target
 from ...utils.logging import log_dist
 
 
@@ -73,9 +74,7 @@ class ZeroOptimizerBase:
         for units in self.units:
             for u in units:
                 for p in u.params:
-                    for a in ("_sxe_grad_target", "_sxe_grad_done", "_sxe_grad_local"):
-                        if hasattr(p, a):
-                            delattr(p, a)
+                    drop_grad_target(p)
 
     # --------------------------------------------------------------------------------------------
     def _init_master(self):

@@ -357,3 +357,25 @@ def _case_moe_load(rank, world, tmp):
 def test_load_moe_state_dict_static(tmp_path):
     res = run_dist(_case_moe_load, 2, str(tmp_path))
     assert all(ok for ok, _ in res) and res[0][1] > 0
+
+
+# --------------------------------------------------------------------------- gradients given back to autograd
+def _case_dropped_targets(rank, world, stage, how):
+    import shuffle_exchange_amd as sxe
+    model, cfg = _tiny()
+    ds = {"train_micro_batch_size_per_gpu": 2, "zero_optimization": {"stage": stage},
+          "optimizer": {"type": "AdamW", "params": {"lr": 1e-2}}, "compile": {"deepcompile": True, "fx_zero3": True}}
+    eng, _, _, _ = sxe.initialize(model=model, config=ds)
+    names = lambda: {a for p in model.parameters() for a in p.__dict__ if a.startswith("_sxe_grad_")}  # noqa: E731
+    before = names()
+    eng.compile() if how == "compile" else eng.optimizer.destroy()
+    return before, names()
+
+
+@pytest.mark.parametrize("stage", [2, 3])
+@pytest.mark.parametrize("how", ["compile", "destroy"])
+def test_nothing_of_the_direct_targets_stays(stage, how):
+    """A compiled engine's gradients come from its graphs, a destroyed one's from autograd: no parameter says that it has a buffer."""
+    (before, after), = run_dist(_case_dropped_targets, 1, stage, how)
+    assert {"_sxe_grad_target", "_sxe_grad_local"} <= before
+    assert not after & {"_sxe_grad_target", "_sxe_grad_done", "_sxe_grad_local"}
