@@ -13,7 +13,7 @@ import torch.nn.functional as F
 from ..ops.activation import bias_gelu
 from ..ops.attention import attention_qkv_rope
 from ..ops.cross_entropy import head_cross_entropy
-from ..ops.linear import Embedding, Linear
+from ..ops.linear import Embedding, Linear, is_own_forward
 from ..ops.norm import LayerNorm
 from ..runtime.zero.partition_parameters import local_shard
 
@@ -74,7 +74,12 @@ class GPT2Block(nn.Module):
         d = self.head_dim
         # q, k and v as they lie: their gradients are written side by side, where slices' would be padded with zeros and added up
         o = attention_qkv_rope(self.c_attn(self.ln_1(x)).view(B, S, 3 * self.n_head, d), self.n_head, self.n_head)
-        y, x = self.ln_2(self.c_proj(o.reshape(B, S, self.n_head * d)), residual=x)
+        a = self.c_proj(o.reshape(B, S, self.n_head * d))
+        if is_own_forward(self.ln_2, LayerNorm):
+            y, x = self.ln_2(a, residual=x)
+        else:  # a norm of the program's own, or one that it looks at
+            x = x + a
+            y = self.ln_2(x)
         m = bias_gelu(self.c_fc(y, skip_bias=True), self.c_fc.bias)
         return x + self.mlp_proj(m)
 
