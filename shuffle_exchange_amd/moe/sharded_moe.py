@@ -300,7 +300,8 @@ class MOELayer(nn.Module):
             Ce = C
         # local experts see [E_local, ep*Ce, H]
         disp = disp.reshape(ep, nle, Ce, H).transpose(0, 1).reshape(nle, ep * Ce, H)
-        if rows is not None and ep == 1 and tp == 1 and getattr(type(self.experts), "forward", None) is GroupedSwiGLUExperts.forward:
+        if (rows is not None and ep == 1 and tp == 1 and "forward" not in vars(self.experts)
+                and getattr(type(self.experts), "forward", None) is GroupedSwiGLUExperts.forward):
             out = self.experts(disp, rows=rows)  # the slots behind an expert's last one are zeros: its products leave them out
         else:
             out = self.experts(disp)

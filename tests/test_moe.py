@@ -73,3 +73,23 @@ def test_mixtral_trains_with_expert_parallelism(stage):
     res = run_dist(C.case_mixtral_train, 2, stage)
     for r in res:
         assert r["losses"][-1] < r["losses"][0]
+
+
+def test_experts_with_a_forward_of_their_own(monkeypatch):
+    """A forward set on the instance takes the slots alone, also where the numbers of slots in use are known (as on the GPU)."""
+    from shuffle_exchange_amd.moe import MoE
+    from shuffle_exchange_amd.ops import moe as M
+    from shuffle_exchange_amd.parallel import groups
+    torch.manual_seed(0)
+    groups.reset()
+    moe = MoE(32, None, num_experts=4, ep_size=1, k=1, capacity_factor=4.0, min_capacity=64, use_rts=False, intermediate_size=48)
+    moe._groups_ready = True
+    x = torch.randn(2, 10, 32)
+    want = moe(x)[0]
+    tables = M.slot_tables
+    monkeypatch.setattr(M, "slot_tables", lambda *a: (*tables(*a)[:2], torch.full((4,), a[3], dtype=torch.int32)))
+    assert torch.equal(moe(x)[0], want)
+    experts, seen = moe.deepspeed_moe.experts, []
+    own = experts.forward
+    experts.forward = lambda slots: (seen.append(slots.shape[0]), own(slots))[1]
+    assert torch.equal(moe(x)[0], want) and seen == [4]
