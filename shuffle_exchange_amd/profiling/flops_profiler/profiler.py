@@ -67,7 +67,7 @@ def _register_sxe_formulas():
         def _stream(x, w, *a, out_shape=None, **kw):
             return 2 * x[0] * w[0] * w[1]
 
-        @register_flop_formula(ops.gemm_tn)
+        @register_flop_formula([ops.gemm_tn, ops.gemm_tn_into])
         def _tiled(x, w, *a, out_shape=None, **kw):  # x [.., K]
             return 2 * math.prod(x) * w[0]
 

@@ -196,6 +196,26 @@ def test_flops_are_counted(rows):
 
 
 @gpu
+def test_flops_of_a_head_with_a_buffer():
+    """A column-wise head's products, forward, dh and dW: the same count where dW goes into the optimizer's buffer."""
+    from torch.utils.flop_counter import FlopCounterMode
+
+    from shuffle_exchange_amd.ops.cross_entropy import head_cross_entropy
+    from shuffle_exchange_amd.profiling.flops_profiler.profiler import _register_sxe_formulas
+    _register_sxe_formulas()
+    w = torch.nn.Parameter(torch.randn(515, 128, device="cuda").bfloat16())
+    h, ids = torch.randn(2, 64, 128, device="cuda").bfloat16().requires_grad_(), torch.randint(0, 515, (2, 64), device="cuda")
+    buf, done, counts = torch.zeros(515, 128, device="cuda"), [], []
+    for _ in range(2):
+        with FlopCounterMode(display=False) as c:
+            head_cross_entropy(h, w, ids).backward()
+        counts.append(c.get_total_flops())
+        w.grad = None
+        w._sxe_grad_target, w._sxe_grad_done, w._sxe_grad_local = (lambda p: (buf, False)), done.append, True
+    assert done and counts == [3 * 2 * 128 * 515 * 128] * 2
+
+
+@gpu
 @pytest.mark.parametrize("tokens", [3, 200])
 def test_flops_of_routed_experts(tokens):
     from torch.utils.flop_counter import FlopCounterMode
