@@ -195,9 +195,12 @@ def _own_products(x, weight, bias=None):
 
 
 # Products of training with narrow weights, up to this many multiplications. A call of the library costs the host 19.5 us whatever its size, one
-# of gemm_tn.hip 6, and its kernels are about as fast; us on the device, library / here: 2048 rows, 2304 x 768 17 / 14, 3072 x 768 16 / 15,
-# 768 x 768 10 / 12, 768 x 3072 19 / 25, 1280 x 5120 37 / 37, 300 rows 8 / 12, 8 / 12, 6 / 11, 9 / 16, 18 / 23. Behind it the device decides:
-# 8192 rows, 768 x 3072 39 / 36, 4096 x 1024 57 / 60, 8192 x 1536, 8192 rows 158 / 168.
+# of gemm_tn.hip 6, which is what steps of this size wait for: GPT-2, four layers, ZeRO-1, us a step with the library / here, 64 tokens 4790 /
+# 4095, 1024 4288 / 3728, 2100 5035 / 4629, 4096 4446 / 3908, 7000 5943 / 5958. On the device most of them take longer, the step's kernels 1720 /
+# 1810, 2280 / 2410, 3360 / 3360, 3840 / 3890, 5940 / 6040 together; single ones, 2048 rows, 2304 x 768 16.6 / 13.8, 3072 x 768 15.6 / 14.8,
+# 768 x 768 9.3 / 11.9, 768 x 3072 19 / 25, 512 x 2048 12 / 24, 300 rows 7.7 / 11.5, 7.9 / 11.6, 7.0 / 11.2, 9.1 / 15.2, 8.4 / 12.6. So not where
+# a graph is captured, whose replays cost the host nothing, nor behind this limit: 8192 rows, 768 x 3072 39 / 36, 4096 x 1024 57 / 60,
+# 8192 x 1536 158 / 168.
 NARROW_WORK = 10 ** 10
 
 
@@ -206,13 +209,18 @@ def _narrow(rows, N, K):
     return (N < 2048 or K < 2048) and N >= 512 and K >= 512 and rows > STREAM_ROWS_SMALL and rows * N * K <= NARROW_WORK
 
 
+_capturing = torch.cuda.is_current_stream_capturing
+
+
 def product(x, weight, bias=None):
     """``F.linear`` for the inside of autograd functions: no graph is built where it runs own kernels (``_tiled``)."""
     rows = x.numel() // max(1, x.shape[-1])
-    if weight.dim() == 2 and (_tiled_faster(rows, *weight.shape) or _narrow(rows, *weight.shape)) and _own_products(x, weight, bias):
-        y = _tiled(x, weight, bias, True)
-        if y is not None:
-            return y
+    if weight.dim() == 2:
+        faster = _tiled_faster(rows, *weight.shape)
+        if (faster or _narrow(rows, *weight.shape)) and _own_products(x, weight, bias) and (faster or not _capturing()):
+            y = _tiled(x, weight, bias, True)
+            if y is not None:
+                return y
     return F.linear(x, weight, bias)
 
 
@@ -505,11 +513,12 @@ def _narrow_data_grad(gy, w):
     """gy @ w of ``_narrow`` weights: up to 1280 rows of the weight by the product that reads them as they lie (experts_kn_tile.hip, one
     expert), else with the transpose, which the splits of gemm_tn.hip make up for. us on the device, library / as they lie / transposed,
     2048 rows: 768 x 3072 18 / 17 / 21, 768 x 768 12 / 14 / 15, 1280 x 5120 36 / 32 / 35, 2304 x 768 24 / 28 / 27, 3072 x 768 30 / 35 / 28,
-    300 rows 14 / 33 / 20; on the host 19 / 8 / 13. None where they do not cover the operands."""
+    300 rows 8.7 / 13.7 / 17, 7.3 / 13 / 14, 14 / 19 / 27, 11.5 / 27 / 19, 14 / 33 / 20; on the host 19 / 8 / 13, which decides, as above.
+    None where they do not cover the operands and where a graph is captured."""
     N, K = w.shape
     if not (_narrow(gy.numel() // max(1, gy.shape[-1]), N, K) and gy.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and N % 64 == 0
             and K % 64 == 0 and gy.is_contiguous() and w.is_cuda and w.is_contiguous() and _own_products(gy, w)
-            and gy.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):  # last: compilation has no memory to look at
+            and gy.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and not _capturing()):  # last: compilation has no memory to look at
         return None
     native.require_hip()
     if N <= 1280:

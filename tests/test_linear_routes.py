@@ -369,6 +369,35 @@ def test_optimizers_buffer_is_for_backward():
 
 
 @gpu
+def test_narrow_products_of_a_captured_step(monkeypatch):
+    """Own kernels for what the host would wait for; in a captured graph, where it waits for nothing, the library's."""
+    from shuffle_exchange_amd.ops import linear as L
+    x, w, b = _operands(300, N=768, K=512)
+    wide = _operands(300, N=2048, K=8192)  # the own product's on the device, too
+    gy, took = F.linear(x, w), []
+    for name in ("_tiled", "_narrow_data_grad"):
+        monkeypatch.setattr(L, name, lambda *a, own=getattr(L, name): took.append(own(*a)) or took[-1])
+
+    def run():
+        took.clear()
+        return [L.product(x, w, b), L.data_grad(gy, w), L.product(*wide[:2])], [t is not None for t in took]
+    with torch.no_grad():
+        want, own = run()
+        assert own == [True, True, True]
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            got, own = run()
+        assert own == [False, True]  # the data gradient's and the wide product
+        for _ in range(3):
+            for t in got:
+                t.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            for t, o in zip(got, want):
+                _close(t, o)
+
+
+@gpu
 def test_glu_rule_and_switch(monkeypatch):
     """SwiGLU of many rows in the product's launch, not of few rows of the largest weights, nor where the library's products are asked for."""
     from shuffle_exchange_amd.ops import linear as L
