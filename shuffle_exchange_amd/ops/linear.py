@@ -592,11 +592,18 @@ def keep_local(p):
     return p if getattr(p, "_sxe_grad_local", False) else None
 
 
+# Elements up to which column sums go into the optimizer's buffer by colsum.hip whether it is the faster reduction or not: what follows a
+# general one (autograd's accumulation and the conversion, two launches and 20 us of the host) costs more than it gains. us, general /
+# kernel: 128 x 768 6.6 / 3.6, 64 x 50257 5.6 / 10.1, 33 x 65544 4.9 / 8.3, 2048 x 1001 13 / 22; behind it 2048 x 3001 23 / 28, 1000 x 50257
+# 32 / 72, 2048 x 50257 60 / 134, 16 x 1048576 6 / 83.
+BIAS_GRAD_ELEMS = 1 << 22
+
+
 def write_bias_grad(b, gy2, ctx):
     """The column sums of gy2 into the optimizer's buffer of ``b`` (``keep_local``), in fp32: one launch instead of the sum, autograd's
     accumulation and a conversion. True if written."""
     if b is None or not (gy2.is_cuda and gy2.dtype in (torch.bfloat16, torch.float16, torch.float32) and gy2.stride(1) == 1
-                         and native.plain(gy2)) or torch.is_grad_enabled():
+                         and native.plain(gy2)) or torch.is_grad_enabled() or not (gy2.numel() <= BIAS_GRAD_ELEMS or _colsum_faster(gy2)):
         return False
     tgt = local_grad_target(b, ctx)
     if tgt is None:

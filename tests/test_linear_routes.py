@@ -398,6 +398,19 @@ def test_narrow_products_of_a_captured_step(monkeypatch):
 
 
 @gpu
+@pytest.mark.parametrize("R,N,kernel", [(128, 768, True), (64, 50257, True), (2048, 3072, True), (1000, 50257, False), (16, 524288, False)])
+def test_bias_gradient_rule(R, N, kernel):
+    """Into the optimizer's buffer by the kernel where that is the faster way; else autograd gets the general reduction's sums."""
+    from shuffle_exchange_amd.ops.linear import _Linear
+    x, w, b = torch.zeros(R, 8, device="cuda").bfloat16(), torch.zeros(N, 8, device="cuda").bfloat16(), torch.nn.Parameter(torch.zeros(N, device="cuda").bfloat16())
+    buf, done = torch.zeros(N, device="cuda"), []
+    b._sxe_grad_target, b._sxe_grad_done, b._sxe_grad_local = (lambda p: (buf, False)), done.append, True
+    _Linear.apply(x, w, b).backward(torch.ones(R, N, device="cuda").bfloat16())
+    got = buf if kernel else b.grad.float()
+    assert bool(done) == kernel and (b.grad is None) == kernel and torch.equal(got, torch.full_like(buf, R).bfloat16().float())
+
+
+@gpu
 def test_glu_rule_and_switch(monkeypatch):
     """SwiGLU of many rows in the product's launch, not of few rows of the largest weights, nor where the library's products are asked for."""
     from shuffle_exchange_amd.ops import linear as L
