@@ -73,6 +73,27 @@ def test_multi_tensor_adam_matches_flat():
         assert _rel(p, r) < 1e-5
 
 
+def test_multi_tensor_adam_groups():
+    """Tensors of every number of workgroups, in no order: each as the flat kernel updates it alone."""
+    torch.manual_seed(0)
+    sizes = [1024 * k + d for k in (1, 2, 4, 8, 16, 32, 64, 128) for d in (-1, 0, 1)] + [1, 3 * 1024, 40 * 1024, 65536 * 3 + 5, 768]
+    sizes = [sizes[i] for i in torch.randperm(len(sizes))]
+    mk = lambda: [torch.rand(n, device="cuda") for n in sizes]  # noqa: E731
+    p, g, m, v = mk(), mk(), mk(), mk()
+    lp = [t.bfloat16() for t in p]
+    args = (None, None, 1e-2, 0.9, 0.95, 1e-8, 0.1, 3, True, True, 0.5)
+    for same in (sizes, sizes[:1], [n for n in sizes if 2048 < n <= 4096]):
+        at = [sizes.index(n) for n in same]
+        cut = lambda ts: [ts[i].clone() for i in at]  # noqa: E731
+        one, many = [cut(ts) for ts in (p, g, m, v, lp)], [cut(ts) for ts in (p, g, m, v, lp)]
+        torch.ops.sxe.multi_tensor_adam_(*many, *args)
+        for ts in zip(*one):
+            torch.ops.sxe.multi_tensor_adam_(*([t] for t in ts), *args)
+        for a, b in zip(one, many):
+            assert all(torch.equal(x, y) for x, y in zip(a, b))
+        assert not any(torch.equal(x, p[i]) for x, i in zip(many[0], at))
+
+
 @pytest.mark.parametrize("offset", [0, 1])
 @pytest.mark.parametrize("gdt", [torch.float32, torch.bfloat16])
 def test_multi_tensor_adam_sizes(offset, gdt):
