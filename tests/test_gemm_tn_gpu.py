@@ -80,6 +80,29 @@ def test_products_in_32_bits(M, N, K, tile):
         torch.ops.sxe.gemm_tn_into(x, w, c[:, :-1], False)
 
 
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+@pytest.mark.parametrize("M,N,K,splits", [(1, 8, 128, 2), (129, 264, 320, 2), (321, 776, 640, 3), (65, 40, 704, 8)])
+def test_split_products_in_32_bits(M, N, K, splits, tile):
+    """The same of products that are split along K, and of a few rows and many tokens, which the plan splits."""
+    x, w, _ = _operands(M, N, K)
+    ref, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    behind = torch.full((M * N + 8,), float("nan"), device="cuda")
+    c = behind[:M * N].view(M, N)
+    for times in (1, 2):
+        torch.ops.sxe.gemm_tn_into(x, w, c, times == 2, tile, splits)
+        assert bool(((c.double() - times * ref).abs() <= times * (K + 2 + splits) * 2.0 ** -24 * size).all())
+    assert bool(behind[M * N:].isnan().all())
+
+
+def test_a_small_tables_gradient_fills_the_card():
+    """515 x 768 of 8192 tokens have 15 tiles: split along the tokens, as the product in bf16 is, to the same sums."""
+    x, w, _ = _operands(515, 768, 8192)
+    c, one = torch.zeros(515, 768, device="cuda"), torch.zeros(515, 768, device="cuda")
+    torch.ops.sxe.gemm_tn_into(x, w, c, False)
+    torch.ops.sxe.gemm_tn_into(x, w, one, False, -1, 1)
+    assert torch.equal(c.bfloat16(), torch.ops.sxe.gemm_tn(x, w, None, False)) and not torch.equal(c, one)
+
+
 def test_head_gradient_into_the_optimizers_buffer():
     """A table that embeds and ends a model: both gradients meet in the buffer, as autograd's sum of them does."""
     from shuffle_exchange_amd.ops.cross_entropy import head_cross_entropy
