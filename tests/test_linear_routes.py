@@ -431,7 +431,8 @@ def test_few_row_rule_of_wide_weights(rows, N, K, own):
     assert _stream_faster(rows, N, K) == own
 
 
-@pytest.mark.parametrize("rows,N,K,own", [(17, 4096, 14336, True), (32, 8192, 28672, True), (24, 4096, 11008, True), (24, 4096, 24576, True),
+@pytest.mark.parametrize("rows,N,K,own", [(17, 4096, 14336, False), (24, 4096, 14336, True), (32, 8192, 28672, True), (24, 4096, 11008, True),
+                                          (24, 4096, 24576, True), (17, 8192, 5120, False), (17, 8192, 5632, True),
                                           (24, 4096, 16384, False), (24, 4096, 8192, False), (33, 4096, 14336, False), (24, 3840, 15360, False),
                                           (24, 5120, 13824, False), (24, 2048, 22016, False), (24, 12288, 12288, False)])
 def test_few_row_rule_of_long_rows(rows, N, K, own):
