@@ -23,7 +23,7 @@ struct AdamHP {
 };
 
 // Adam moves 28 - 30 bytes a parameter and is bound by memory alone. What its streams reach depends on how a launch walks them: a
-// workgroup takes 256 vectors and ends (1 KB of each of eight streams at a time, neighbours side by side), and loads and stores pass by
+// workgroup takes 256 vectors of four and ends (4 KB of each fp32 stream, 2 KB of a 16-bit one, neighbours side by side), and loads and stores pass by
 // the caches, which a step of this size only empties of what comes next. 2^28 parameters with bf16 copies, TB/s: workgroups that walk
 // 64 K elements each 5.0, 4 K 5.3, 1 K 5.5; around the caches 5.2, 5.6, 6.1; only the stores 5.0, 5.3.
 template <typename V>

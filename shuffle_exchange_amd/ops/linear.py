@@ -66,10 +66,13 @@ def _skinny(x, weight, bias):
 # columns a workgroup, in a captured sequence of weights that are each read once, 24 rows: 32000 x 4096 60.6 / 52.2, 32000 x 2048 32.5 /
 # 27.6, 128256 x 4096 191 / 186, 65536 x 4096 121 / 99, 16384 x 4096 31.8 / 29.8, 8192 x 3072 18.4 / 13.9 (32 rows: 64000 x 2560 60.7 /
 # 62.4, 32000 x 3072 37.2 / 38.3); but 12288 x 4096 23.6 / 26.9, 9216 x 3072 17.1 / 19.5, 8192 x 4096 16.7 / 18.3. Long rows, a workgroup
-# for every CU, 24 rows, the same way: 4096 x 9216 21.3 / 19.5, 4096 x 11008 31.5 / 24.1, 4096 x 14336 30.9 / 30.0 (17 rows 28.3 / 29.1, 32 rows
-# 30.2 / 30.0), 4096 x 22016 124 / 44, 4096 x 24576 135 / 47, 8192 x 5120 19.6 / 19.8, 8192 x 14336 48.6 / 48.0, 8192 x 28672 89.1 / 89.8; but rows
-# whose starts fall on the same channels, 4096 x 8192 17.9 / 18.7, 4096 x 16384 33.4 / 35.9, 8192 x 8192 29.9 / 33.2, and 3840 x 15360 30.1 /
-# 31.5, 12288 x 12288 64.2 / 66.6.
+# for every CU, weights that are each read once, 17 / 32 rows: the library is slow where rows are no whole pieces of 1 KB, 4096 x 11008 30.3 / 23.4,
+# 29.8 / 24.9, 4096 x 14080 35.5 / 27.2, 34.7 / 29.4, or longer than 32 KB, 4096 x 18432 119 / 35, 121 / 37, 4096 x 28672 173 / 51, 177 / 55, else
+# level with it, 4096 x 12288 23.5 / 24.5, 26.3 / 26.1, 4096 x 14336 27.6 / 28.0, 30.6 / 30.1, 4096 x 15360 28.4 / 29.9, 31.4 / 31.8 (in a
+# decode step with four such layers, us a step, 17 rows 695 / 694, 20 701 / 695, 24 706 / 702, 28 714 / 712, 32 723 / 723); with
+# 32 columns a workgroup 8192 x 5632 20.0 / 19.4, 20.9 / 20.3, 8192 x 12288 41.6 / 37.9, 42.6 / 40.4, 8192 x 28672 90.4 / 83.9, 103 / 90, 7936 x
+# 11008 51.4 / 38.2, 52.8 / 39.5, but 8192 x 5120 18.8 / 19.0, 19.4 / 19.8. Not rows whose starts fall on the same channels, 24 rows, 4096 x 8192
+# 17.9 / 18.7, 4096 x 16384 33.4 / 35.9, 8192 x 8192 29.9 / 33.2, nor 3840 x 15360 30.1 / 31.5, 12288 x 12288 64.2 / 66.6.
 STREAM_ROWS, STREAM_ROWS_SMALL = 16, 32
 
 
@@ -82,8 +85,11 @@ def _full_rounds(workgroups):
 def _stream_faster(rows, N, K):
     if rows > STREAM_ROWS:
         if K > 4096:
-            return (rows <= STREAM_ROWS_SMALL and 4096 <= N <= 8192 and N * K >= 1 << 25 and (K > 16384 or K % 8192 != 0)
-                    and _full_rounds(N / (32 if N >= 6144 else 16)) > 0.95)
+            if rows > STREAM_ROWS_SMALL or not 4096 <= N <= 8192 or N * K < 1 << 25 or (K <= 16384 and K % 8192 == 0):
+                return False
+            if N >= 6144:
+                return K > 5120 and _full_rounds(N / 32) > 0.95
+            return (K > 16384 or K % 512 != 0 or rows >= 20) and _full_rounds(N / 16) > 0.95
         return rows <= STREAM_ROWS_SMALL and K <= 4096 and (N <= 4096 or N * K <= 1 << 23 or ((N >= 16384 or K <= 3072)
                                                                                               and _full_rounds(N / 32) > 0.93))
     return not (K >= 5120 and N * K >= 1 << 24 and _full_rounds(N / 16) < 0.9) and not (K < 1024 and N > 16384)

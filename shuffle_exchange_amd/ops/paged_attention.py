@@ -104,10 +104,11 @@ def choose_splits(num_seqs, nkv, max_kv_len, target_wgs=None):
 # Keys of a split at most where sequences differ in length. One layer's attention of a decode step, heads 32 / 8 of 128, us with the
 # splits of choose_splits / of at most 512 keys: sequences of 300 - 4000 keys, 16 of them 35 / 26, 32 61 / 44, 64 111 / 85, 128
 # 167 / 152; but all of 4000 keys 44 / 51, 95 / 102, 177 / 195; all of 2000 - 4000 38 / 40, 77 / 79, 145 / 149; 64 of 1000 42 / 50.
-# Half of them where even then all workgroups run at once: a workgroup's few chunks one after the other are what the call takes. With the
-# merge, 512 / 256 keys: 8 sequences of 256 - 3000 keys 23.0 / 20.7, 16 of 200 - 2500 26.3 / 22.7; 24 of 256 - 6000 (2304 workgroups) a
-# step of four layers 841 / 850, 40 of 100 - 3000 (1920) of two 432 / 438; heads of 64
-# 13.9 / 13.1, 17.8 / 16.3, of 256, one workgroup a CU, 29.2 / 33.7.
+# Half of them where the splits of 512 keys all run at once (so the launch has up to twice as many workgroups as do, of which those behind
+# a sequence's end exit at once): a workgroup's few chunks one after the other are what the call takes. With the merge, 512 / 256 keys:
+# 8 sequences of 256 - 3000 keys 23.0 / 20.7, 16 of 200 - 2500 (640, then 1280 workgroups) 26.3 / 22.7; 24 of 256 - 6000 (2304, not
+# halved) a step of four layers 841 / 850, 40 of 100 - 3000 (1920) of two 432 / 438; heads of 64 13.9 / 13.1, 17.8 / 16.3, of 256, one
+# workgroup a CU, 29.2 / 33.7.
 PA_SPLIT_KEYS = 512
 # Lengths are even where the longest is at most this many times the mean (a log-uniform spread over a factor of 2 has 1.4, of 10 2.6).
 PA_EVEN = 1.5

@@ -177,7 +177,7 @@ def test_even_lengths():
 
 
 def test_short_splits_of_few_uneven_sequences():
-    for seqs, nkv, keys, dim in ((8, 8, 3000, 128), (16, 8, 3072, 128), (2, 4, 512, 64), (3, 2, 10, 64)):  # all at once: 256 keys
+    for seqs, nkv, keys, dim in ((8, 8, 3000, 128), (16, 8, 3072, 128), (2, 4, 512, 64), (3, 2, 10, 64)):  # splits of 512 keys would all run at once
         assert PA.choose_balanced_splits(seqs, nkv, keys, 1 << 10, False, dim) == max(PA.choose_splits(seqs, nkv, keys), -(-keys // 256))
     for seqs, nkv, keys, dim in ((16, 8, 3073, 128), (24, 8, 6000, 128), (4, 8, 3000, 256)):
         assert PA.choose_balanced_splits(seqs, nkv, keys, 1 << 10, False, dim) == max(PA.choose_splits(seqs, nkv, keys), -(-keys // 512))
