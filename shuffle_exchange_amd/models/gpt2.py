@@ -13,7 +13,7 @@ import torch.nn.functional as F
 from ..ops.activation import bias_gelu
 from ..ops.attention import attention_qkv_rope
 from ..ops.cross_entropy import head_cross_entropy
-from ..ops.linear import Embedding, Linear, is_own_forward
+from ..ops.linear import Embedding, Linear, is_own_call
 from ..ops.norm import LayerNorm
 from ..runtime.zero.partition_parameters import local_shard
 
@@ -75,7 +75,7 @@ class GPT2Block(nn.Module):
         # q, k and v as they lie: their gradients are written side by side, where slices' would be padded with zeros and added up
         o = attention_qkv_rope(self.c_attn(self.ln_1(x)).view(B, S, 3 * self.n_head, d), self.n_head, self.n_head)
         a = self.c_proj(o.reshape(B, S, self.n_head * d))
-        if is_own_forward(self.ln_2, LayerNorm):
+        if is_own_call(self.ln_2, LayerNorm):
             y, x = self.ln_2(a, residual=x)
         else:  # a norm of the program's own, or one that it looks at
             x = x + a

@@ -755,6 +755,16 @@ def is_own_forward(mod, *types):
             and not every._global_forward_hooks and not every._global_forward_pre_hooks)
 
 
+def is_own_call(mod, *types):
+    """A caller may choose the arguments of ``mod(...)``: it runs the forward of one of ``types``, and nobody looks at what goes in, comes
+    out or flows back (the optimizer's hooks that wait for parameters do not)."""
+    every = torch.nn.modules.module
+    return (type(mod) in types and "forward" not in mod.__dict__ and not mod._forward_hooks and not mod._backward_hooks
+            and not mod._backward_pre_hooks and all(getattr(h, "_sxe_wait", False) for h in mod._forward_pre_hooks.values())
+            and not every._global_forward_hooks and not every._global_forward_pre_hooks and not every._global_backward_hooks
+            and not every._global_backward_pre_hooks)
+
+
 class Linear(torch.nn.Linear):
     """``nn.Linear`` whose GEMMs go through ``linear`` (fused weight-grad into ZeRO buffers).
     AutoTP swaps it for a column/row-parallel layer with the same call signature.

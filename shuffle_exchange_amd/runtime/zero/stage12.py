@@ -392,6 +392,7 @@ class ZeroStage12Optimizer(ZeroOptimizerBase):
                 ev = self._pending_events.pop(u, None)
                 if ev is not None:
                     cur.wait_event(ev)
+        pre._sxe_wait = True
         return pre
 
     def _post_step_exchange(self):
