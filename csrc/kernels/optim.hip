@@ -222,7 +222,7 @@ void multi_tensor_adam_(at::TensorList p, at::TensorList g, at::TensorList m, at
   if (nt == 0) return;
   SXE_CHECK(g.size() == nt && m.size() == nt && v.size() == nt, "multi_tensor_adam_: list sizes");
   SXE_CHECK(lp.size() == 0 || lp.size() == nt, "multi_tensor_adam_: lp list size");
-  std::vector<MTChunk> host;
+  std::vector<MTChunk> host, less[kGroups];  // entries of kChunk elements, and of fewer
   DT gd = dtype_of(g[0]);
   DT ld = lp.size() ? dtype_of(lp[0]) : DT::BF16;
   for (size_t i = 0; i < nt; ++i) {
@@ -238,11 +238,11 @@ void multi_tensor_adam_(at::TensorList p, at::TensorList g, at::TensorList m, at
       c.v = v[i].data_ptr<float>() + s;
       c.lp = lp.size() ? static_cast<char*>(lp[i].data_ptr()) + s * lp[i].element_size() : nullptr;
       c.n = std::min<int64_t>(kChunk, n - s);
-      host.push_back(c);
+      (c.n == kChunk ? host : less[mt_group(c.n)]).push_back(c);
     }
   }
+  for (const auto& group : less) host.insert(host.end(), group.begin(), group.end());
   if (host.empty()) return;
-  std::stable_sort(host.begin(), host.end(), [](const MTChunk& a, const MTChunk& b) { return mt_group(a.n) < mt_group(b.n); });
   c10::DeviceGuard guard(p[0].device());
   auto bytes = (int64_t)(host.size() * sizeof(MTChunk));
   auto h = at::empty({bytes}, at::TensorOptions().dtype(at::kByte).pinned_memory(true));
