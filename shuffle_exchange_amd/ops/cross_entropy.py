@@ -96,7 +96,7 @@ class _ColumnHeadXEnt(torch.autograd.Function):
             torch.ops.sxe.wgrad_gemm_(g, weight, dh, 1.0, False)
             dh = dh[:tgt.numel()].to(h2.dtype).view(h.shape)
         if ctx.needs_input_grad[1]:
-            into = local_grad_target(ctx.weight, ctx)
+            into = local_grad_target(ctx.weight, ctx) if native.plain(dloss) else None
             # in fp32 into the optimizer's buffer: no gradient of the table is written, read and added up besides
             if into is not None and into[0].shape == weight.shape and into[0].data_ptr() % 16 == 0:
                 torch.ops.sxe.gemm_tn_into(g, torch.ops.sxe.transpose16(h2), *into)

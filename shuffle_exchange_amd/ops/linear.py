@@ -580,10 +580,11 @@ def _accumulates(ctx, p):
 
 def local_grad_target(p, ctx):
     """``grad_target`` of a parameter whose gradient only this rank ever adds up, in fp32 (``_sxe_grad_local``), in the backward of
-    ``ctx``: (buffer, whether it holds a sum), for gradients that may come in several pieces or besides autograd's. None elsewhere, where
-    hooks of the parameter's gradient want to see it, and where the caller of autograd does."""
+    ``ctx``, whose gradient the caller has found ``native.plain``: (buffer, whether it holds a sum), for gradients that may come in several
+    pieces or besides autograd's. None elsewhere, where hooks of the parameter's gradient want to see it, and where the caller of
+    autograd does."""
     if (p is None or not getattr(p, "_sxe_grad_local", False) or p._backward_hooks
-            or len(getattr(p, "_post_accumulate_grad_hooks", None) or ()) > 1 or not native.plain(p) or not _accumulates(ctx, p)):
+            or len(getattr(p, "_post_accumulate_grad_hooks", None) or ()) > 1 or not _accumulates(ctx, p)):
         return None
     tgt = grad_target(p)
     if tgt is None:

@@ -51,7 +51,7 @@ class _NormFn(torch.autograd.Function):
         dres = dh.contiguous().view(-1, H) if (ctx.has_res and dh is not None) else None
         from .linear import grad_target, local_grad_target
         lw, lb = ctx.local
-        if lw is not None and ctx.needs_input_grad[2] and (ctx.needs_input_grad[3] and lb is not None) == ctx.layernorm and not torch.is_grad_enabled():
+        if lw is not None and ctx.needs_input_grad[2] and (ctx.needs_input_grad[3] and lb is not None) == ctx.layernorm and not torch.is_grad_enabled() and native.plain(dy2):
             tw, tb = local_grad_target(lw, ctx), local_grad_target(lb, ctx)
             if tw is not None and (tb is not None) == ctx.layernorm:  # both sums straight into the optimizer's buffers
                 dx = torch.ops.sxe.norm_bwd_into(dy2, hin, rstd, mean, weight, dres, bool(ctx.layernorm), tw[0].view(-1), tw[1],
