@@ -3,8 +3,9 @@
 // Parity: reference csrc/quantization (``quantize`` / ``dequantize`` / ``swizzle_quant`` /
 // ``quantized_reduction``, symmetric int8 / int4) and ops/fp_quantizer (FP8 e4m3 with per-group
 // scales). MI355X design:
-//  * one wave per quantization group (group sizes are multiples of 64): a lane handles
-//    group/64 contiguous values, the absmax is a wave butterfly, no LDS;
+//  * one wave per quantization group (group sizes are multiples of 64): a lane handles every 64th pair of neighbouring values, so
+//    that pairs which share a byte (int4) or are converted together (FP8) are whole at every group size, also where a lane has an odd
+//    number of values, and no lane reads or writes beyond the group; the absmax is a wave butterfly, no LDS;
 //  * int4 packs two values per byte (low nibble first), int8 as-is, scales fp32 per group;
 //  * FP8 e4m3 conversion uses CDNA4's hardware converters (v_cvt_pk_fp8_f32 via the
 //    __builtin_amdgcn_cvt_pk_fp8_f32 builtin, OCP e4m3 on gfx950) and v_cvt_f32_fp8 back;
@@ -21,22 +22,21 @@ __global__ void quant_kernel(const typename dt_traits<T>::storage* __restrict x,
   const int lane = threadIdx.x & 63;
   const int64_t wid = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6;
   const int64_t nw = ((int64_t)gridDim.x * blockDim.x) >> 6;
-  const int per = group / 64;
   constexpr float qmax = BITS == 8 ? 127.f : 7.f;
   for (int64_t gi = wid; gi < n_groups; gi += nw) {
-    const typename dt_traits<T>::storage* src = x + gi * group + lane * per;
+    const typename dt_traits<T>::storage* src = x + gi * group;
     float m = 0.f;
-    for (int i = 0; i < per; ++i) m = fmaxf(m, fabsf(to_f32<T>(src[i])));
+    for (int i = 2 * lane; i < group; i += 128) m = fmaxf(m, fmaxf(fabsf(to_f32<T>(src[i])), fabsf(to_f32<T>(src[i + 1]))));
     m = wave_max(m);
     const float s = m > 0.f ? m / qmax : 1.f;
     const float inv = 1.f / s;
     if (lane == 0) scales[gi] = s;
     if constexpr (BITS == 8) {
-      int8_t* dst = reinterpret_cast<int8_t*>(q) + gi * group + lane * per;
-      for (int i = 0; i < per; ++i) dst[i] = (int8_t)fmaxf(-qmax, fminf(qmax, rintf(to_f32<T>(src[i]) * inv)));
+      int8_t* dst = reinterpret_cast<int8_t*>(q) + gi * group;
+      for (int i = lane; i < group; i += 64) dst[i] = (int8_t)fmaxf(-qmax, fminf(qmax, rintf(to_f32<T>(src[i]) * inv)));
     } else {
-      uint8_t* dst = q + (gi * group + lane * per) / 2;
-      for (int i = 0; i < per; i += 2) {
+      uint8_t* dst = q + gi * group / 2;
+      for (int i = 2 * lane; i < group; i += 128) {
         const int a = (int)fmaxf(-qmax, fminf(qmax, rintf(to_f32<T>(src[i]) * inv)));
         const int b = (int)fmaxf(-qmax, fminf(qmax, rintf(to_f32<T>(src[i + 1]) * inv)));
         dst[i / 2] = (uint8_t)((a & 0xF) | ((b & 0xF) << 4));
@@ -94,18 +94,17 @@ __global__ void fp8_quant_kernel(const typename dt_traits<T>::storage* __restric
   const int lane = threadIdx.x & 63;
   const int64_t wid = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6;
   const int64_t nw = ((int64_t)gridDim.x * blockDim.x) >> 6;
-  const int per = group / 64;
   constexpr float fmax8 = 448.f;
   for (int64_t gi = wid; gi < n_groups; gi += nw) {
-    const typename dt_traits<T>::storage* src = x + gi * group + lane * per;
+    const typename dt_traits<T>::storage* src = x + gi * group;
     float m = 0.f;
-    for (int i = 0; i < per; ++i) m = fmaxf(m, fabsf(to_f32<T>(src[i])));
+    for (int i = 2 * lane; i < group; i += 128) m = fmaxf(m, fmaxf(fabsf(to_f32<T>(src[i])), fabsf(to_f32<T>(src[i + 1]))));
     m = wave_max(m);
     const float s = m > 0.f ? m / fmax8 : 1.f;
     const float inv = 1.f / s;
     if (lane == 0) scales[gi] = s;
-    uint8_t* dst = q + gi * group + lane * per;
-    for (int i = 0; i < per; i += 2) {
+    uint8_t* dst = q + gi * group;
+    for (int i = 2 * lane; i < group; i += 128) {
       const float a = fmaxf(-fmax8, fminf(fmax8, to_f32<T>(src[i]) * inv));
       const float b = fmaxf(-fmax8, fminf(fmax8, to_f32<T>(src[i + 1]) * inv));
       const int packed = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false);

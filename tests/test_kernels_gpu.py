@@ -316,6 +316,26 @@ def test_fp8_quantize():
     assert ((out.float() - x.float()).norm() / x.float().norm()) < 0.05
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kind", ["fp8", 8, 4])
+@pytest.mark.parametrize("group", [64, 192, 576, 640])
+def test_quantize_groups_of_their_own_scale(kind, dt, group):
+    """Groups in which 64 lanes have one or an odd number of values each, neighbours 256 times apart: every code is its own group's. What
+    divides by the scale multiplies by its reciprocal here, so a value beside a rounding boundary may be a code off."""
+    from shuffle_exchange_amd.ops import quantizer as Q
+    n = 33
+    x = (torch.randn(n, group, device="cuda") * 256.0 ** (torch.arange(n, device="cuda") % 2)[:, None]).to(dt)
+    if kind == "fp8":
+        q, s = Q.quantize_fp8(x, group)
+        got, step = q.view(torch.float8_e4m3fn).float(), 2.0 ** -4 * x.float().abs() / s[:, None] + 2.0 ** -10
+    else:
+        q, s = Q.quantize(x, group, kind)
+        got, step = Q.dequantize(q, torch.ones_like(s), group, kind, dtype=torch.float32), 0.5
+    assert torch.allclose(s, x.float().abs().amax(1) / {"fp8": 448.0, 8: 127.0, 4: 7.0}[kind], rtol=1e-6)
+    want = x.float() / s[:, None]
+    assert ((got.view(n, group) - want).abs() <= step * (1 + 2.0 ** -12)).all()  # half a code (subnormal fp8 codes are 2^-9 apart)
+
+
 @pytest.mark.parametrize("variant", [0, 1, 2, 16 * 4])
 @pytest.mark.parametrize("K,M,N", [(128, 256, 256), (1024, 768, 512), (2048, 512, 1280)])
 @pytest.mark.parametrize("accumulate", [True, False])
