@@ -33,8 +33,9 @@ def test_plain(M, N, K, fp8):
     for bias in (None, b):
         got = torch.ops.sxe.stream_gemm(x, w, s, bias, False)
         want = x.double() @ ref.T + (0 if bias is None else b.double())
-        # products of bf16 are exact in fp32; left are fp32 sums and the rounding of the result (2^-9)
-        assert (got.double() - want).norm() < 3e-3 * want.norm()
+        # products of bf16 are exact in fp32; left are fp32 sums and the rounding of the result: at most 2^-8 of a value (just above a power
+        # of two), which a result of four values with a bias drawn anew each time comes near
+        assert (got.double() - want).norm() < 1.01 * 2 ** -8 * want.norm()
 
 
 def test_every_e4m3_value_is_exact():
