@@ -22,6 +22,15 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int NW = 8;  // waves of a workgroup
 
+// What is done with the sums: EPI_PLAIN bf16 (+ bias); EPI_GLU silu(gate) * up; and those of a decoder's layer, whose norms and RoPE are no
+// launches of their own: EPI_RES adds the residual stream, EPI_ROPE rotates q and k and appends k and v to the paged cache, EPI_NGLU and
+// EPI_HEAD (fp32 result) are the other two products behind a norm. A norm between two products is split over both: the first one's
+// epilogue holds the new residual stream and leaves (stream x norm weight) in bf16 for the next product and its tiles' sums of squares; the
+// next one adds those up (rows x tiles, 32 KB at most, behind its first operand loads) and multiplies its sums by 1 / rms. The operand is
+// rounded once, as a norm's result is; the product and the sum are no longer rounded before they meet the stream.
+// A launch costs a step ~4.7 us whatever it does: a layer of 4096 x 4096 / 28672 x 4096 has 6 of them, 9 before.
+enum Epi { EPI_PLAIN, EPI_GLU, EPI_RES, EPI_ROPE, EPI_NGLU, EPI_HEAD };
+
 struct Args {
   const unsigned short* x;
   int64_t ldx;
@@ -31,6 +40,21 @@ struct Args {
   const unsigned short* bias;  // or null
   unsigned short* y;
   int M, N, K;
+  // behind a norm (ROPE, NGLU, HEAD; part null: x is normed): sums of squares [parts, mp] of the rows' tiles
+  const float* part;
+  int parts, mp;  // mp: M rounded up to 8, 16 or 32
+  float eps;
+  float* yf;  // HEAD
+  // RES: y = bf16(stream * gw)
+  const unsigned short *res, *gw;
+  int64_t ldr;
+  unsigned short* h;  // [M, N], the new stream
+  float* sums;        // [N / 16, mp]
+  // ROPE: w's rows are nq + 2 nkv heads of 128
+  const float *rcos, *rsin;  // [positions, 64]
+  const int64_t *pos, *slots;
+  unsigned short* cache;  // [blocks, 2, nkv, bs, 128]
+  int nq, nkv, bs;
 };
 
 __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
@@ -120,20 +144,32 @@ struct Piece {
   }
 };
 
-template <bool FP8, int MB, int NT, bool GLU, bool ONCE>
+// HALF (up to 8 rows): a tile of 8 columns, each twice. The matrix core's rows 0 - 7 have one half of a piece's K, rows 8 - 15 the other one,
+// of W and of x alike, and the two blocks of the result that belong together are added: no lane loads what another one does, and there are
+// twice the workgroups, each with half the pieces one behind the other.
+template <bool FP8, int MB, int NT, int EPI, bool ONCE, bool HALF = false>
 __global__ void __launch_bounds__(64 * NW, 2) stream_gemm_kernel(Args a) {
-  __shared__ f32x4 red[NW][NT][64];
+  static_assert(!HALF || (MB == 1 && NT == 1), "");
+  constexpr bool GLU = EPI == EPI_GLU || EPI == EPI_NGLU, NORMED = EPI >= EPI_ROPE;
   constexpr int OT = GLU ? NT / 2 : NT;  // tiles of output columns
+  constexpr int TC = HALF ? 8 : 16, PAIRS = TC * NT / 2;
+  __shared__ f32x4 red[NW][NT][64];
+  __shared__ float squares[NORMED ? NW : 1][NORMED ? 32 : 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16 * OT, half = a.N / 2;
-  const int j = lane & 3, quad0 = l16 & 12, c = 4 * g + j;
+  const int half = a.N / 2;
+  const int j = lane & 3, quad0 = l16 & (TC - 4), c = 4 * g + j;
+  // ROPE: a workgroup has both halves of what it rotates, as two tiles or as the halves of one; else NT tiles side by side
+  const int n0 = EPI == EPI_ROPE ? (int)(blockIdx.x / (64 / PAIRS)) * 128 + (int)(blockIdx.x % (64 / PAIRS)) * PAIRS : (int)blockIdx.x * TC * OT;
+  auto column = [&](int t, int q) {  // of column q (a multiple of 4) of tile t
+    if constexpr (EPI == EPI_ROPE) return NT == 2 ? n0 + 64 * t + q : HALF ? n0 + 16 * q : n0 + (q & 4) + 8 * (q & 8);
+    return GLU ? n0 + 16 * (t % OT) + (t / OT) * half + q : n0 + 16 * t + q;
+  };
+  // what this lane finishes: 4 columns of row frow of tile `wave` (HALF: the four groups of 16 lanes do the same)
+  const int frow = HALF ? lane & 7 : l16, fq = HALF ? (lane & 8) / 2 : 4 * g;
   // tiles start inside W (N a multiple of 4: a quad's rows all do or none); what lies past the end repeats the last rows
   const char* wr[NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int n = (GLU ? n0 + 16 * (t % OT) + (t / OT) * half : n0 + 16 * t) + quad0;
-    wr[t] = static_cast<const char*>(a.w) + (int64_t)min(n, a.N - 4) * a.ldw * (FP8 ? 1 : 2);
-  }
+  for (int t = 0; t < NT; ++t) wr[t] = static_cast<const char*>(a.w) + (int64_t)min(column(t, quad0), a.N - 4) * a.ldw * (FP8 ? 1 : 2);
   const int64_t ldw = a.ldw * (FP8 ? 1 : 2);
   const unsigned short* xr[MB][4];
 #pragma unroll
@@ -149,12 +185,159 @@ __global__ void __launch_bounds__(64 * NW, 2) stream_gemm_kernel(Args a) {
 
   // (the next piece in flight behind this one's products halves the workgroups on a CU and gains nothing)
   using P = Piece<FP8, MB, NT, ONCE>;
-  for (int k0 = wave * P::PIECE; k0 < a.K; k0 += NW * P::PIECE) {
+  constexpr int STEP = HALF ? 2 * P::PIECE : P::PIECE;
+  int k0 = wave * STEP + (HALF ? (l16 >> 3) * P::PIECE : 0);
+  // what the epilogue reads is on its way beside the first piece
+  u16x4 res[MB], gw;
+  f32x4 cs[MB], sn[MB];
+  int64_t slot[MB];
+  if constexpr (EPI >= EPI_RES) {
+    int64_t at[MB];
+    if constexpr (EPI == EPI_ROPE) {
+#pragma unroll
+      for (int m = 0; m < MB; ++m) {
+        const int row = min(16 * m + frow, a.M - 1);
+        at[m] = a.pos[row];
+        slot[m] = a.slots[row];
+      }
+    }
+    P p;
+    p.load(wr, ldw, xr, k0, a.K, c);
+    if (EPI == EPI_RES && wave < OT) {
+      const int n = min(column(wave, fq), a.N - 4);
+      gw = *reinterpret_cast<const u16x4*>(a.gw + n);
+#pragma unroll
+      for (int m = 0; m < MB; ++m) res[m] = *reinterpret_cast<const u16x4*>(a.res + (int64_t)min(16 * m + frow, a.M - 1) * a.ldr + n);
+    }
+    if (EPI == EPI_ROPE && wave < OT) {
+#pragma unroll
+      for (int m = 0; m < MB; ++m) {
+        const int64_t o = at[m] * 64 + (column(wave, fq) & 63);
+        cs[m] = *reinterpret_cast<const f32x4*>(a.rcos + o);
+        sn[m] = *reinterpret_cast<const f32x4*>(a.rsin + o);
+      }
+    }
+    if constexpr (NORMED) {
+      if (a.part != nullptr) {  // a thread always has the same 4 rows: 512 is a multiple of mp / 4
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+        const int quads = a.mp / 4;
+        for (int i = threadIdx.x; i < a.parts * quads; i += 64 * NW) s += reinterpret_cast<const f32x4*>(a.part)[i];
+        for (int d = quads; d < 64; d *= 2)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) s[q] += __shfl_xor(s[q], d, 64);
+        if (lane < quads) *reinterpret_cast<f32x4*>(&squares[wave][4 * lane]) = s;
+      }
+    }
+    p.multiply(acc, odd1, odd2);
+    k0 += NW * STEP;
+  }
+  for (; k0 - (HALF ? (l16 >> 3) * P::PIECE : 0) < a.K; k0 += NW * STEP) {
     P p;
     p.load(wr, ldw, xr, k0, a.K, c);
     p.multiply(acc, odd1, odd2);
   }
   // lane: columns 4 g .. + 3 of row l16 of every tile
+  auto finish = [&](int m, int t) {
+    const int row = 16 * m + frow, n = column(t, fq);
+    float rinv = 1.f;
+    if constexpr (NORMED) {
+      if (a.part != nullptr) {
+        float s = 0.f;
+#pragma unroll
+        for (int v = 0; v < NW; ++v) s += squares[v][min(row, a.mp - 1)];
+        rinv = rsqrtf(s / (float)a.K + a.eps);
+      }
+    }
+    auto sum = [&](int tile, int other, int col) {  // other: of the other half of the tile's columns
+      f32x4 s;
+      if constexpr (HALF) {  // of the waves 2 (lane / 16) and the next, then of all
+        const int at = frow + 16 * ((fq >> 2) ^ other), v = lane >> 4;
+        s = red[2 * v][tile][at] + red[2 * v][tile][at + 40] + red[2 * v + 1][tile][at] + red[2 * v + 1][tile][at + 40];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          s[q] += __shfl_xor(s[q], 16, 64);
+          s[q] += __shfl_xor(s[q], 32, 64);
+        }
+      } else {
+        const int at = other ? lane ^ 32 : lane;
+        s = red[0][tile][at];
+#pragma unroll
+        for (int v = 1; v < NW; ++v) s += red[v][tile][at];
+      }
+      if (FP8) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s[q] *= a.scale[min(col + q, a.N - 1)];
+      }
+      if (NORMED) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s[q] *= rinv;
+      } else if (a.bias != nullptr) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s[q] += bf16_to_f32(a.bias[min(col + q, a.N - 1)]);
+      }
+      return s;
+    };
+    f32x4 v = sum(t, 0, n);
+    const int cols = GLU ? half : a.N;
+    if constexpr (GLU) {
+      const f32x4 up = sum(t + OT, 0, n + half);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] = v[q] / (1.f + expf(-v[q])) * up[q];
+    }
+    if constexpr (EPI == EPI_ROPE) {
+      const f32x4 other = NT == 2 ? sum(1 - t, 0, n ^ 64) : sum(0, 1, n ^ 64);
+      if (n < (a.nq + a.nkv) * 128) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = v[q] * cs[m][q] + (n & 64 ? other[q] : -other[q]) * sn[m][q];
+      }
+    }
+    u16x4 o;
+    if constexpr (EPI == EPI_RES) {
+      float s = 0.f;
+      u16x4 hs;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        hs[q] = f32_to_bf16(v[q] + bf16_to_f32(res[m][q]));
+        const float h = bf16_to_f32(hs[q]);
+        s += h * h;
+        o[q] = f32_to_bf16(h * bf16_to_f32(gw[q]));
+      }
+      if constexpr (HALF) {
+        s += __shfl_xor(s, 8, 64);
+      } else {
+        s += __shfl_xor(s, 16, 64);
+        s += __shfl_xor(s, 32, 64);
+      }
+      if (n >= a.N || row >= a.mp) return;  // a whole tile, or rows that have no place
+      if (HALF && lane >= 16) return;
+      if (fq == 0) a.sums[(int64_t)(n / TC) * a.mp + row] = row < a.M ? s : 0.f;
+      if (row < a.M) *reinterpret_cast<u16x4*>(a.h + (int64_t)row * a.N + n) = hs;
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) o[q] = f32_to_bf16(v[q]);
+    }
+    if (row >= a.M || (HALF && lane >= 16)) return;
+    if constexpr (EPI == EPI_HEAD) {
+      if (n < a.N) *reinterpret_cast<f32x4*>(a.yf + (int64_t)row * a.N + n) = v;
+      return;
+    }
+    if constexpr (EPI == EPI_ROPE) {
+      const int head = n >> 7;
+      if (head >= a.nq && slot[m] >= 0) {
+        const int kv = head >= a.nq + a.nkv ? 1 : 0, hh = head - a.nq - kv * a.nkv;
+        const int64_t blk = slot[m] / a.bs, off = slot[m] - blk * a.bs;
+        *reinterpret_cast<u16x4*>(a.cache + (((blk * 2 + kv) * a.nkv + hh) * a.bs + off) * 128 + (n & 127)) = o;
+      }
+    }
+    unsigned short* yp = a.y + (int64_t)row * cols + n;
+    if (n + 4 <= cols && cols % 4 == 0) {
+      *reinterpret_cast<u16x4*>(yp) = o;
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (n + q < cols) yp[q] = o[q];
+    }
+  };
 #pragma unroll
   for (int m = 0; m < MB; ++m) {
     if (16 * m >= a.M) break;
@@ -162,50 +345,16 @@ __global__ void __launch_bounds__(64 * NW, 2) stream_gemm_kernel(Args a) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) red[wave][t][lane] = acc[m][t];
     __syncthreads();
-    for (int i = threadIdx.x; i < OT * 64; i += 64 * NW) {
-      const int t = i >> 6, ln = i & 63, row = 16 * m + (ln & 15), n = n0 + 16 * t + 4 * (ln >> 4);
-      auto sum = [&](int tile, int col) {
-        f32x4 s = red[0][tile][ln];
-#pragma unroll
-        for (int v = 1; v < NW; ++v) s += red[v][tile][ln];
-        if (FP8) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) s[q] *= a.scale[min(col + q, a.N - 1)];
-        }
-        if (a.bias != nullptr) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) s[q] += bf16_to_f32(a.bias[min(col + q, a.N - 1)]);
-        }
-        return s;
-      };
-      f32x4 v = sum(t, n);
-      const int cols = GLU ? half : a.N;
-      if constexpr (GLU) {
-        const f32x4 up = sum(t + OT, n + half);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = v[q] / (1.f + expf(-v[q])) * up[q];
-      }
-      if (row >= a.M) continue;
-      unsigned short* yp = a.y + (int64_t)row * cols + n;
-      if (n + 4 <= cols && cols % 4 == 0) {
-        u16x4 o;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) o[q] = f32_to_bf16(v[q]);
-        *reinterpret_cast<u16x4*>(yp) = o;
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if (n + q < cols) yp[q] = f32_to_bf16(v[q]);
-      }
-    }
+    if (wave < OT) finish(m, wave);
   }
 }
 
 }  // namespace st
 
-// x [M, K] bf16, w [N, K] bf16, or e4m3 bytes with wscale fp32 [N]; bias bf16 [N] or None; glu: w = gate | up
-at::Tensor stream_gemm(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& wscale,
-                       const c10::optional<at::Tensor>& bias, bool glu) {
+namespace {
+// the operands that all forms have: x [M, K] bf16, w [N, K] bf16, or e4m3 bytes with wscale fp32 [N]; -> whether w is e4m3
+bool operands(st::Args& a, const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& wscale,
+              const c10::optional<at::Tensor>& bias) {
   check_beside(x, {w, wscale, bias});
   const bool fp8 = wscale.has_value() && wscale->defined();
   SXE_CHECK(x.scalar_type() == at::kBFloat16 && x.dim() == 2 && x.stride(1) == 1 && w.is_cuda() && w.dim() == 2 && w.stride(1) == 1 &&
@@ -216,8 +365,6 @@ at::Tensor stream_gemm(const at::Tensor& x, const at::Tensor& w, const c10::opti
   SXE_CHECK(K % unit == 0 && w.stride(0) % unit == 0 && x.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
                 reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0, "stream_gemm: K and the rows must allow 16-byte loads");
   SXE_CHECK(N % 4 == 0, "stream_gemm: N a multiple of 4");
-  SXE_CHECK(!glu || N % 32 == 0, "stream_gemm: gate and up of a multiple of 16 columns");
-  st::Args a{};
   if (fp8) {
     SXE_CHECK(wscale->scalar_type() == at::kFloat && wscale->is_contiguous() && wscale->numel() == N, "stream_gemm: wscale fp32 [N]");
     a.scale = wscale->data_ptr<float>();
@@ -226,41 +373,166 @@ at::Tensor stream_gemm(const at::Tensor& x, const at::Tensor& w, const c10::opti
     SXE_CHECK(bias->scalar_type() == at::kBFloat16 && bias->is_contiguous() && bias->numel() == N, "stream_gemm: bias bf16 [N]");
     a.bias = reinterpret_cast<const unsigned short*>(bias->data_ptr());
   }
-  c10::DeviceGuard gd(x.device());
-  auto y = at::empty({M, glu ? N / 2 : N}, x.options());
   a.x = reinterpret_cast<const unsigned short*>(x.data_ptr());
   a.ldx = x.stride(0);
   a.w = w.data_ptr();
   a.ldw = w.stride(0);
-  a.y = reinterpret_cast<unsigned short*>(y.data_ptr());
   a.M = M;
   a.N = N;
   a.K = K;
-  // tiles a workgroup: more of them for fewer reads of x, fewer for more workgroups. 28672 x 4096, us at 1 / 2 / 4 tiles: bf16,
-  // 16 rows 47 / 50 / 47, 32 rows 57 / 53 / 53; e4m3, 8 rows 32 / 29 / 35; 4096 x 4096: bf16 9.7 / 12.9 / 16, e4m3 7.3 / 8.5 / 12.4
-  const int64_t all = (N + 15) / 16;
-  const int nt = glu ? (!fp8 && N % 64 == 0 ? 4 : 2) : all >= 384 && (fp8 || M > 16) ? 2 : 1;
-  const dim3 grid((all + nt - 1) / nt);
-  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(64 * st::NW), 0, cur_stream(), a); };
-  auto rows = [&](auto mb, auto nontemporal) {
-    constexpr int MB = decltype(mb)::value;
-    constexpr bool ONCE = decltype(nontemporal)::value;
-    if (fp8) {
-      if (glu) go(st::stream_gemm_kernel<true, MB, 2, true, ONCE>);
-      else nt == 2 ? go(st::stream_gemm_kernel<true, MB, 2, false, ONCE>) : go(st::stream_gemm_kernel<true, MB, 1, false, ONCE>);
-    } else if (glu) {
-      nt == 4 ? go(st::stream_gemm_kernel<false, MB, 4, true, ONCE>) : go(st::stream_gemm_kernel<false, MB, 2, true, ONCE>);
-    } else {
-      nt == 2 ? go(st::stream_gemm_kernel<false, MB, 2, false, ONCE>) : go(st::stream_gemm_kernel<false, MB, 1, false, ONCE>);
-    }
-  };
+  a.mp = M <= 8 ? 8 : M <= 16 ? 16 : 32;
+  return fp8;
+}
+
+// the sums of squares that stream_gemm_res left for x's rows, or none: x is normed
+void normed_by(st::Args& a, const at::Tensor& x, const c10::optional<at::Tensor>& part, double eps) {
+  if (!part.has_value() || !part->defined()) return;
+  check_beside(x, {*part});
+  SXE_CHECK(part->scalar_type() == at::kFloat && part->dim() == 2 && part->is_contiguous() && part->size(1) == a.mp && part->size(0) > 0 &&
+                part->size(0) < (1 << 24) && reinterpret_cast<uintptr_t>(part->data_ptr()) % 16 == 0, "stream_gemm: sums fp32 [tiles, rows]");
+  a.part = part->data_ptr<float>();
+  a.parts = part->size(0);
+  a.eps = (float)eps;
+}
+
+// the kernel of M's rows and of weights that are read past the caches or through them: run(one or two blocks of rows, past the caches)
+template <class F>
+void by_rows(const st::Args& a, bool fp8, F run) {
   auto blocks = [&](auto nontemporal) {
-    if (M <= 16) rows(std::integral_constant<int, 1>{}, nontemporal);
-    else rows(std::integral_constant<int, 2>{}, nontemporal);
+    if (a.M <= 16) run(std::integral_constant<int, 1>{}, nontemporal);
+    else run(std::integral_constant<int, 2>{}, nontemporal);
   };
-  if (read_once(N * K * (fp8 ? 1 : 2))) blocks(std::true_type{});
+  if (read_once((int64_t)a.N * a.K * (fp8 ? 1 : 2))) blocks(std::true_type{});
   else blocks(std::false_type{});
   SXE_LAUNCH_CHECK();
+}
+
+// tiles a workgroup: more of them for fewer reads of x, fewer for more workgroups. e4m3, 28672 x 4096, 8 rows, us at 1 / 2 / 4 tiles 32 / 29 /
+// 35, 4096 x 4096 7.3 / 8.5 / 12.4; bf16, 4096 x 4096, 16 rows 9.7 / 12.9 / 16
+int plain_tiles(const st::Args& a, bool fp8) { return (a.N + 15) / 16 >= 384 && (fp8 || a.M > 16) ? 2 : 1; }
+
+// Half tiles where whole ones give half of the CUs no work: 2048 columns, up to 8 rows, a decode step of three layers of hidden 2048, ff 8192 with
+// the head 189 / 180 us bf16, 148 / 142 e4m3; but 2560 columns (160 tiles) 230 / 236 and 180 / 187, 4096 (256) 367 / 380 and 266 / 284
+bool halves(const st::Args& a) { return a.M <= 8 && a.N <= 2048; }
+
+template <int EPI>
+void launch(const st::Args& a, bool fp8, int nt) {
+  if constexpr (EPI != st::EPI_GLU && EPI != st::EPI_NGLU) {
+    if (halves(a)) {
+      const dim3 grid((a.N + 7) / 8);
+      auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(64 * st::NW), 0, cur_stream(), a); };
+      by_rows(a, fp8, [&](auto, auto nontemporal) {
+        constexpr bool ONCE = decltype(nontemporal)::value;
+        fp8 ? go(st::stream_gemm_kernel<true, 1, 1, EPI, ONCE, true>) : go(st::stream_gemm_kernel<false, 1, 1, EPI, ONCE, true>);
+      });
+      return;
+    }
+  }
+  const dim3 grid(((a.N + 15) / 16 + nt - 1) / nt);
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(64 * st::NW), 0, cur_stream(), a); };
+  constexpr bool GLU = EPI == st::EPI_GLU || EPI == st::EPI_NGLU;
+  by_rows(a, fp8, [&](auto mb, auto nontemporal) {
+    constexpr int MB = decltype(mb)::value;
+    constexpr bool ONCE = decltype(nontemporal)::value;
+    if constexpr (GLU) {
+      // a tile of gate and one of up; two of each leave a workgroup a CU, steps of three layers, us, two / one: 4096, 14336 1 row 358 / 340, 8
+      // rows 372 / 355, 16 397 / 379, 32 467 / 455; 4096, 11008 32 rows 544 / 509; 3072, 8192 235 / 234, 300 / 297; 2048, 8192 180 / 177, 218 / 216
+      fp8 ? go(st::stream_gemm_kernel<true, MB, 2, EPI, ONCE>) : go(st::stream_gemm_kernel<false, MB, 2, EPI, ONCE>);
+    } else if (fp8) {
+      nt == 2 ? go(st::stream_gemm_kernel<true, MB, 2, EPI, ONCE>) : go(st::stream_gemm_kernel<true, MB, 1, EPI, ONCE>);
+    } else {
+      nt == 2 ? go(st::stream_gemm_kernel<false, MB, 2, EPI, ONCE>) : go(st::stream_gemm_kernel<false, MB, 1, EPI, ONCE>);
+    }
+  });
+}
+}  // namespace
+
+// (+ bias bf16 [N] or None); glu: w = gate | up
+at::Tensor stream_gemm(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& wscale,
+                       const c10::optional<at::Tensor>& bias, bool glu) {
+  st::Args a{};
+  const bool fp8 = operands(a, x, w, wscale, bias);
+  SXE_CHECK(!glu || a.N % 32 == 0, "stream_gemm: gate and up of a multiple of 16 columns");
+  c10::DeviceGuard gd(x.device());
+  auto y = at::empty({a.M, glu ? a.N / 2 : a.N}, x.options());
+  a.y = reinterpret_cast<unsigned short*>(y.data_ptr());
+  if (glu) launch<st::EPI_GLU>(a, fp8, 2);
+  else launch<st::EPI_PLAIN>(a, fp8, plain_tiles(a, fp8));
+  return y;
+}
+
+// h = res + x . w^T (+ bias), and what a product of rms_norm(h) * gw needs: -> [bf16(h * gw), h, sums of h^2 [N / 16, rows]]
+std::vector<at::Tensor> stream_gemm_res(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& wscale,
+                                        const c10::optional<at::Tensor>& bias, const at::Tensor& res, const at::Tensor& gw) {
+  st::Args a{};
+  const bool fp8 = operands(a, x, w, wscale, bias);
+  check_beside(x, {res, gw});
+  SXE_CHECK(a.N % 16 == 0, "stream_gemm_res: whole tiles of 16 columns");
+  SXE_CHECK(res.scalar_type() == at::kBFloat16 && res.dim() == 2 && res.size(0) == a.M && res.size(1) == a.N && res.stride(1) == 1 &&
+                res.stride(0) % 4 == 0 && reinterpret_cast<uintptr_t>(res.data_ptr()) % 8 == 0, "stream_gemm_res: res bf16 [M, N]");
+  SXE_CHECK(gw.scalar_type() == at::kBFloat16 && gw.is_contiguous() && gw.numel() == a.N && reinterpret_cast<uintptr_t>(gw.data_ptr()) % 8 == 0,
+            "stream_gemm_res: gw bf16 [N]");
+  c10::DeviceGuard gd(x.device());
+  auto y = at::empty({a.M, a.N}, x.options()), h = at::empty({a.M, a.N}, x.options());
+  auto sums = at::empty({a.N / (halves(a) ? 8 : 16), a.mp}, x.options().dtype(at::kFloat));
+  a.y = reinterpret_cast<unsigned short*>(y.data_ptr());
+  a.h = reinterpret_cast<unsigned short*>(h.data_ptr());
+  a.sums = sums.data_ptr<float>();
+  a.res = reinterpret_cast<const unsigned short*>(res.data_ptr());
+  a.ldr = res.stride(0);
+  a.gw = reinterpret_cast<const unsigned short*>(gw.data_ptr());
+  launch<st::EPI_RES>(a, fp8, plain_tiles(a, fp8));
+  return {y, h, sums};
+}
+
+// of x . w^T / rms (sums of stream_gemm_res; None: x is normed): silu(gate) * up in bf16 (glu), or the product in fp32
+at::Tensor stream_gemm_normed(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& wscale,
+                              const c10::optional<at::Tensor>& part, double eps, bool glu) {
+  st::Args a{};
+  const bool fp8 = operands(a, x, w, wscale, c10::nullopt);
+  normed_by(a, x, part, eps);
+  SXE_CHECK(!glu || a.N % 32 == 0, "stream_gemm_normed: gate and up of a multiple of 16 columns");
+  c10::DeviceGuard gd(x.device());
+  auto y = at::empty({a.M, glu ? a.N / 2 : a.N}, glu ? x.options() : x.options().dtype(at::kFloat));
+  if (glu) {
+    a.y = reinterpret_cast<unsigned short*>(y.data_ptr());
+    launch<st::EPI_NGLU>(a, fp8, 2);
+  } else {
+    a.yf = y.data_ptr<float>();
+    launch<st::EPI_HEAD>(a, fp8, plain_tiles(a, fp8));
+  }
+  return y;
+}
+
+// the q, k and v of nq + 2 nkv heads of 128 (bf16 [M, heads * 128]) of x . w^T / rms, q and k rotated, k and v in the cache as well
+at::Tensor stream_gemm_rope(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& wscale,
+                            const c10::optional<at::Tensor>& part, double eps, const at::Tensor& cos_t, const at::Tensor& sin_t,
+                            const at::Tensor& pos, const at::Tensor& slots, at::Tensor cache, int64_t nq, int64_t nkv) {
+  st::Args a{};
+  const bool fp8 = operands(a, x, w, wscale, c10::nullopt);
+  normed_by(a, x, part, eps);
+  check_beside(x, {cos_t, sin_t, pos, slots, cache});
+  SXE_CHECK(nq > 0 && nkv > 0 && a.N == (nq + 2 * nkv) * 128, "stream_gemm_rope: w rows = (nq + 2 nkv) * 128");
+  SXE_CHECK(cos_t.scalar_type() == at::kFloat && sin_t.scalar_type() == at::kFloat && cos_t.is_contiguous() && sin_t.is_contiguous() &&
+                cos_t.size(-1) == 64 && sin_t.sizes() == cos_t.sizes() && reinterpret_cast<uintptr_t>(cos_t.data_ptr()) % 16 == 0 &&
+                reinterpret_cast<uintptr_t>(sin_t.data_ptr()) % 16 == 0, "stream_gemm_rope: cos / sin fp32 [positions, 64]");
+  SXE_CHECK(pos.scalar_type() == at::kLong && slots.scalar_type() == at::kLong && pos.is_contiguous() && slots.is_contiguous() &&
+                pos.numel() == a.M && slots.numel() == a.M, "stream_gemm_rope: pos / slots int64 [M]");
+  SXE_CHECK(cache.scalar_type() == at::kBFloat16 && cache.dim() == 5 && cache.is_contiguous() && cache.size(1) == 2 && cache.size(2) == nkv &&
+                cache.size(4) == 128 && reinterpret_cast<uintptr_t>(cache.data_ptr()) % 8 == 0,
+            "stream_gemm_rope: cache bf16 [blocks, 2, nkv, bs, 128]");
+  c10::DeviceGuard gd(x.device());
+  auto y = at::empty({a.M, a.N}, x.options());
+  a.y = reinterpret_cast<unsigned short*>(y.data_ptr());
+  a.rcos = cos_t.data_ptr<float>();
+  a.rsin = sin_t.data_ptr<float>();
+  a.pos = pos.data_ptr<int64_t>();
+  a.slots = slots.data_ptr<int64_t>();
+  a.cache = reinterpret_cast<unsigned short*>(cache.data_ptr());
+  a.nq = nq;
+  a.nkv = nkv;
+  a.bs = cache.size(3);
+  launch<st::EPI_ROPE>(a, fp8, plain_tiles(a, fp8));
   return y;
 }
 
@@ -268,5 +540,14 @@ at::Tensor stream_gemm(const at::Tensor& x, const at::Tensor& w, const c10::opti
 
 TORCH_LIBRARY_FRAGMENT(sxe, m) {
   m.def("stream_gemm(Tensor x, Tensor w, Tensor? wscale, Tensor? bias, bool glu) -> Tensor");
+  m.def("stream_gemm_res(Tensor x, Tensor w, Tensor? wscale, Tensor? bias, Tensor res, Tensor gw) -> Tensor[]");
+  m.def("stream_gemm_normed(Tensor x, Tensor w, Tensor? wscale, Tensor? part, float eps, bool glu) -> Tensor");
+  m.def("stream_gemm_rope(Tensor x, Tensor w, Tensor? wscale, Tensor? part, float eps, Tensor cos, Tensor sin, Tensor pos, Tensor slots, "
+        "Tensor(a!) cache, int nq, int nkv) -> Tensor");
 }
-TORCH_LIBRARY_IMPL(sxe, CUDA, m) { m.impl("stream_gemm", &sxe::stream_gemm); }
+TORCH_LIBRARY_IMPL(sxe, CUDA, m) {
+  m.impl("stream_gemm", &sxe::stream_gemm);
+  m.impl("stream_gemm_res", &sxe::stream_gemm_res);
+  m.impl("stream_gemm_normed", &sxe::stream_gemm_normed);
+  m.impl("stream_gemm_rope", &sxe::stream_gemm_rope);
+}

@@ -42,6 +42,7 @@ class _StaticBatch:
         self.max_blocks = max_blocks
         self.max_kv_len = kv_bucket
         self.even_lengths = even
+        self.every_token = True  # the logits are those of every row, in order
         n64, n32 = 32 * S, 16 * S + 4 * S * max_blocks  # bytes: one copy brings both
         self.dev = torch.zeros(n64 + n32, dtype=torch.uint8, device=device)
         self.host = torch.zeros(n64 + n32, dtype=torch.uint8, pin_memory=True)

@@ -6,7 +6,8 @@ choices the reference makes through its registry (blocked KV rotary, blocked fla
 BLAS linear, cutlass MoE GEMM) replaced by this framework's gfx950 kernels:
 
   * RMSNorm with fused residual add (norm.hip), projections through hipBLASLt and, for few rows, the
-    decode kernels (skinny_gemm.hip, stream_gemm.hip),
+    decode kernels (skinny_gemm.hip, stream_gemm.hip); up to 32 tokens the products' epilogues hold the residual
+    sums, norms, RoPE and KV scatter (``_chain``), and a layer is its four products and the attention,
   * RoPE in place on the packed QKV (rope.hip), KV scatter into the blocked cache and paged
     attention (paged_attn.hip; sequences with many new tokens, with or without earlier ones, in one
     launch of the tile kernel, paged_prefill.hip; the longest prompts, flash_attn.hip),
@@ -32,6 +33,7 @@ import torch.nn.functional as F
 from ....ops import native
 from ....ops.activation import swiglu
 from ....ops.linear import Linear, STREAM_ROWS_SMALL, TILED_GLU_ROWS, glu_faster, glu_linear, glu_tiled, is_own_forward, linear
+from ....ops.linear import chain_faster, stream_glu, stream_head, stream_res, stream_rope, stream_weight
 from ....ops.norm import RMSNorm
 from ....ops.paged_attention import paged_attention_parts, paged_batch_attention, ragged_attention, rope_kv_cache_append
 from ....ops.rows import gather_last
@@ -270,6 +272,64 @@ class RaggedLlama:
                 return mid, h
         return swiglu(self._proj(mlp.gate_up_proj, a, li, "gu")), h
 
+    def _chain(self, T, batch, kv_cache, rope):
+        """Per layer the weights of its products, where all of them (up to 32 rows) run the streaming kernel with the residual sums, norms,
+        RoPE and the cache's append in their epilogues; None otherwise. MoE layers: of the first product alone."""
+        if not (0 < T <= STREAM_ROWS_SMALL and self.tps is None and self.device.type == "cuda" and self.head_dim == 128
+                and native.hip_available() and rope.cos.shape[-1] == 64 and rope.cos.dtype == torch.float32
+                and os.environ.get("SXE_DECODE_FUSE", "1") == "1"):
+            return None
+        small = self.qw is None or T <= 16  # quantized layers run more rows on the weight as it came
+
+        def weight(mod, li, key, columns=16):
+            if getattr(mod, "bias", None) is not None:
+                return None
+            w = self._wobj(mod, li, key) if small else self.qw[li][key].weight
+            return None if w is None else stream_weight(w, T, columns)
+        out = []
+        for li, layer in enumerate(self.model.layers):
+            kv, norms = kv_cache.layer(li), (layer.input_layernorm, layer.post_attention_layernorm)
+            mlp = getattr(layer, "mlp", None)
+            if (not kv.is_contiguous() or kv.dim() != 5 or kv.dtype != torch.bfloat16 or kv.shape[2] != self.nkv
+                    or any(not is_own_forward(n, RMSNorm) or n.weight.dtype != torch.bfloat16 for n in norms)):
+                return None
+            ws = [weight(layer.self_attn.qkv_proj, li, "qkv")]
+            if mlp is not None:
+                ws += [weight(layer.self_attn.o_proj, li, "o"), weight(mlp.gate_up_proj, li, "gu", 32), weight(mlp.down_proj, li, "down")]
+            if any(w is None for w in ws) or not chain_faster(T, ws) or ws[0][0].shape[0] != (self.nq + 2 * self.nkv) * 128:
+                return None
+            out.append(ws)
+        if not is_own_forward(self.model.norm, RMSNorm) or self.model.norm.weight.dtype != torch.bfloat16:
+            return None
+        return out
+
+    def _chained(self, batch, kv_cache, rope, x, chain):
+        """The layers and the head with ``_chain``'s weights: logits."""
+        model, T = self.model, batch.num_tokens
+        a = h = sums = None
+        for li, (layer, ws) in enumerate(zip(model.layers, chain)):
+            kv_layer, norm = kv_cache.layer(li), layer.input_layernorm
+            if a is None:
+                a, h = (norm(x), x) if h is None else norm(x, h)
+            qkv = stream_rope(a, ws[0], sums, norm.eps, rope, batch.positions, kv_layer, batch.slots, self.nq, self.nkv)
+            o = self._attention(qkv.view(T, self.nq + 2 * self.nkv, self.head_dim), kv_layer, batch).reshape(T, self.nq * self.head_dim)
+            norm = layer.post_attention_layernorm
+            if len(ws) == 1:
+                m, h = norm(self._proj(layer.self_attn.o_proj, o, li, "o"), h)
+                x, a, sums = self._moe(layer, m, li), None, None
+                continue
+            a, h, sums = stream_res(o, ws[1], h, norm.weight)
+            mid = stream_glu(a, ws[2], sums, norm.eps)
+            after = model.layers[li + 1].input_layernorm if li + 1 < len(chain) else model.norm
+            a, h, sums = stream_res(mid, ws[3], h, after.weight)
+        if a is not None and getattr(batch, "every_token", False):
+            w = model.lm_head.weight if self.qw is None else self._impl_weight(self.qhead)
+            wk = stream_weight(w, T, 4) if w is not None else None
+            if wk is not None:
+                return stream_head(a, wk, sums, model.norm.eps)
+        x = gather_last(x, batch.last_idx, h) if a is None else gather_last(h, batch.last_idx)
+        return self._head(model.norm(x))
+
     def _moe(self, layer, m, li):
         moe = layer.block_sparse_moe if hasattr(layer, "block_sparse_moe") else layer.moe
         if self.tps is not None:  # this rank's expert columns -> partial sums -> one all-reduce
@@ -331,6 +391,9 @@ class RaggedLlama:
                              f"({rope.max_pos} positions, max_position_embeddings)")
         T = batch.num_tokens
         x = self.embed_impl(batch.input_ids) if self.embed_impl is not None else model.embed_tokens(batch.input_ids)
+        chain = self._chain(T, batch, kv_cache, rope)
+        if chain is not None:
+            return self._chained(batch, kv_cache, rope, x, chain)
         res = None
         for li, layer in enumerate(model.layers):
             attn = layer.self_attn
@@ -377,6 +440,7 @@ class RaggedLlama:
             full = torch.empty(self.tp * part.shape[0], part.shape[1], dtype=part.dtype, device=part.device)
             dist.all_gather_into_tensor(full, part, group=self.tp_group)
             return full.view(self.tp, -1, part.shape[1]).permute(1, 0, 2).reshape(part.shape[0], -1)[:, :self.tps.vocab]
-        if self.qw is not None:
-            return self.qhead(h).float()
-        return linear(h, model.lm_head.weight).float()
+        return self._head(h)
+
+    def _head(self, h):
+        return (self.qhead(h) if self.qw is not None else linear(h, self.model.lm_head.weight)).float()

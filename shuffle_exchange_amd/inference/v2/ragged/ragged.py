@@ -242,6 +242,7 @@ class RaggedBatch:
         S = len(seqs)
         lens = [int(t.numel()) for t in tokens]
         T = sum(lens)
+        self.every_token = want is None and all(n == 1 for n in lens)  # last_idx is every row, in order
         if want is None:
             want = [(n - 1,) for n in lens]
         n_want = sum(len(x) for x in want)

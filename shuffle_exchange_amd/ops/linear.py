@@ -97,7 +97,7 @@ def _stream_faster(rows, N, K):
 
 def glu_faster(rows, weight):
     """Whether ``glu_linear`` beats the product and the activation's launch. e4m3: always (8 rows of 28672 x 4096 34 / 26 us with the
-    product of skinny_gemm.hip). bf16, four tiles a workgroup, us, with the library's product / here: 16 rows 16384 x 2048
+    product of skinny_gemm.hip). bf16, four tiles a workgroup (two, as now, take up to 5 % less), us, with the library's product / here: 16 rows 16384 x 2048
     20.7 / 17.4, 28672 x 4096 63 / 46, 36864 x 5120 80 / 76, but 57344 x 8192 170 / 183; 24 rows 10240 x 2560 17.9 / 15.9,
     16384 x 3072 24.4 / 23.3, 28672 x 4096 59 / 52, but 17920 x 2560 25.9 / 30.6, 27648 x 5120 54 / 63, 7168 x 4096 18.1 / 20.7."""
     if not isinstance(weight, torch.Tensor):
@@ -140,6 +140,60 @@ def glu_linear(x, weight):
     if not _streamable(x, w, None, 8 if sc is None else 16):
         return None
     return torch.ops.sxe.stream_gemm(x, w, sc, None, True)
+
+
+def stream_weight(weight, rows, columns=16):
+    """(w, scale) for the products of a decoder's layer that are chained without launches for its norms (``stream_res``, ``stream_glu``,
+    ``stream_rope``, ``stream_head``), or None: a bf16 weight, up to 32 rows, or an FP8Weight, up to 16; its rows a multiple of ``columns``."""
+    wk = _pro_weight(weight)
+    if wk is None or SKINNY_MAX_M <= 0:
+        return None
+    w, sc = wk
+    N, K = w.shape
+    if not 0 < rows <= (STREAM_ROWS_SMALL if sc is None else STREAM_ROWS) or N % columns or N == 0 or K == 0 or K % (8 if sc is None else 16):
+        return None
+    return (w, sc) if w.is_cuda and w.data_ptr() % 16 == 0 and native.plain(w) else None
+
+
+def chain_faster(rows, weights):
+    """Whether a layer's products (qkv, o, gate | up, down; of MoE layers the first) gain by having its norms, residual sums and RoPE in their
+    epilogues, three launches of ~4.7 us a layer, also where the library has the faster product. us a decode step of three layers (two from
+    5120 on) and the head, launches of their own (up to 4 rows the norms in prologues of skinny_gemm.hip) / so, 1, 8, 16 and 32 rows: hidden 2048,
+    ff 8192 184 / 173, 202 / 177, 208 / 188, 249 / 216; 3072, 8192 247 / 229, 265 / 234, 280 / 249, 324 / 297; 3584, 18944 386 / 345, 456 / 352,
+    472 / 374, 729 / 458; 4096, 11008 350 / 332, 374 / 341, 409 / 377, 540 / 509; 4096, 14336 362 / 340, 382 / 355, 402 / 379, 470 / 455; 6144,
+    16384, 16 and 32 rows 619 / 604, 688 / 659; 8192, 28672, 4 rows 868 / 756; e4m3 4096, 14336 248 / 254, 297 / 268, 339 / 301; 3072, 8192 179 / 180,
+    219 / 188, 245 / 212; 2048, 8192 140 / 136, 172 / 143; 5120, 13824, 1 and 8 rows 263 / 226, 275 / 254. So one row keeps the prologues where
+    they cost it least (with 1024 keys and more splits to merge 2048, 8192 of eight layers is 433 / 438), and from 17 rows on not 5120, 13824 with 40 kv heads (8 rows 382 / 347, 32 rows 483 / 513), whose last round of the
+    gate's workgroups is short."""
+    w, scale = weights[0]
+    if rows == 1:
+        return w.shape[1] > (2048 if scale is None else 4096)
+    if rows <= STREAM_ROWS or len(weights) == 1:
+        return True
+    N, K = weights[2][0].shape
+    return K <= 4096 or N * K > 1 << 28 or _full_rounds(N / 64) > 0.85
+
+
+def stream_res(x, wk, res, norm_weight):
+    """h = res + x . w^T and what the next product takes of rms_norm(h) * norm_weight, in ONE launch (stream_gemm.hip):
+    (bf16(h * norm_weight), h, sums of h^2 by tiles of 16 columns)."""
+    return torch.ops.sxe.stream_gemm_res(x, wk[0], wk[1], None, res, norm_weight)
+
+
+def stream_glu(x, wk, sums, eps):
+    """silu(gate) * up of the product of a normed input, x and ``sums`` of ``stream_res`` (None: x is normed)."""
+    return torch.ops.sxe.stream_gemm_normed(x, wk[0], wk[1], sums, float(eps), True)
+
+
+def stream_head(x, wk, sums, eps):
+    """The product of a normed input in fp32."""
+    return torch.ops.sxe.stream_gemm_normed(x, wk[0], wk[1], sums, float(eps), False)
+
+
+def stream_rope(x, wk, sums, eps, rope, positions, cache, slots, nq, nkv):
+    """q, k, v of a normed input [T, (nq + 2 nkv) * 128], q and k rotated, k and v in the paged cache as well."""
+    return torch.ops.sxe.stream_gemm_rope(x, wk[0], wk[1], sums, float(eps), rope.cos, rope.sin, positions.reshape(-1).contiguous().long(),
+                                          slots, cache, int(nq), int(nkv))
 
 
 # Many rows: csrc/kernels/gemm_tn.hip, us, library / here. The library's kernels fit whole tiles of 256 rows (8192 rows, 28672 x 4096

@@ -63,7 +63,7 @@ def _register_sxe_formulas():
         def _skinny8(x, wq, *a, out_shape=None, **kw):
             return 2 * x[0] * wq[0] * wq[1]
 
-        @register_flop_formula(ops.stream_gemm)
+        @register_flop_formula([ops.stream_gemm, ops.stream_gemm_res, ops.stream_gemm_normed, ops.stream_gemm_rope])
         def _stream(x, w, *a, out_shape=None, **kw):
             return 2 * x[0] * w[0] * w[1]
 

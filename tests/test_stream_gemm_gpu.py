@@ -94,3 +94,103 @@ def test_linear_routes_by_rows():
                 g, u = want.chunk(2, -1)
                 ref = torch.nn.functional.silu(g) * u
                 assert (mid.double() - ref).norm() < 3e-3 * ref.norm()
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 17, 32])
+@pytest.mark.parametrize("N,K", [(16, 16), (48, 1032 - 8), (6160, 2064), (4096, 4096)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_residual_and_what_a_normed_product_needs(M, N, K, fp8):
+    x, w, s, ref = _operands(M, N, K, fp8, M + N + K)
+    res = torch.randn(M, N + 12, device="cuda").bfloat16()[:, 4:N + 4]
+    gw = (1 + 0.3 * torch.randn(N, device="cuda")).bfloat16()
+    y, h, sums = torch.ops.sxe.stream_gemm_res(x, w, s, None, res, gw)
+    want = res.double() + x.double() @ ref.T
+    assert (h.double() - want).norm() < 1.01 * 2 ** -8 * want.norm()
+    assert torch.equal(y, (h.float() * gw.float()).bfloat16())
+    tiles, rows = sums.shape
+    assert N // tiles in (8, 16) and rows in (8, 16, 32) and rows >= M and not sums[:, M:].any()
+    squares = h.double().square().view(M, tiles, N // tiles).sum(-1)
+    assert (sums[:, :M].T.double() - squares).abs().max() <= 1e-6 * squares.max()
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 17, 32])
+@pytest.mark.parametrize("N,K,tiles", [(32, 16, 1), (96, 1024, 3), (6208, 2064, 129), (8192, 4096, 256), (16416, 4112, 600)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_products_behind_a_norm(M, N, K, tiles, fp8):
+    """The sums come from any number of tiles; what they say of the rows is up to who made them. From 64 MB on weights pass the caches."""
+    x, w, s, ref = _operands(M, N, K, fp8, M + N + K)
+    sums = torch.rand(tiles, 8 if M <= 8 else 16 if M <= 16 else 32, device="cuda") * 3
+    p = x.double() @ ref.T * (sums[:, :M].double().sum(0) / K + 1e-3).rsqrt()[:, None]
+    got = torch.ops.sxe.stream_gemm_normed(x, w, s, sums, 1e-3, False)
+    assert got.dtype == torch.float32 and (got.double() - p).norm() < 1e-5 * p.norm()
+    g, u = p.chunk(2, -1)
+    mid = torch.ops.sxe.stream_gemm_normed(x, w, s, sums, 1e-3, True)
+    want = torch.nn.functional.silu(g) * u
+    assert (mid.double() - want).norm() < 1.01 * 2 ** -8 * want.norm()
+    plain = torch.ops.sxe.stream_gemm_normed(x, w, s, None, 0.0, False)
+    assert torch.equal(plain.bfloat16(), torch.ops.sxe.stream_gemm(x, w, s, None, False))
+
+
+@pytest.mark.parametrize("M", [1, 9, 17, 32])
+@pytest.mark.parametrize("nq,nkv,K", [(1, 1, 16), (4, 2, 1024), (48, 8, 2064)])  # one and two tiles a workgroup
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("normed", [False, True])
+def test_rotated_heads_and_the_cache(M, nq, nkv, K, fp8, normed):
+    x, w, s, ref = _operands(M, (nq + 2 * nkv) * 128, K, fp8, M + nq + K)
+    sums = torch.rand(7, 8 if M <= 8 else 16 if M <= 16 else 32, device="cuda") if normed else None
+    a = torch.rand(50, 64, device="cuda") * 6.28
+    pos = torch.randint(0, 50, (M,), device="cuda")
+    slots = torch.randperm(5 * 16, device="cuda")[:M]
+    slots[::5] = -1
+    cache = torch.full((5, 2, nkv, 16, 128), 7.0, device="cuda").bfloat16()
+    got = torch.ops.sxe.stream_gemm_rope(x, w, s, sums, 1e-3, a.cos(), a.sin(), pos, slots, cache, nq, nkv)
+    p = x.double() @ ref.T
+    if normed:
+        p = p * (sums[:, :M].double().sum(0) / K + 1e-3).rsqrt()[:, None]
+    p = p.view(M, nq + 2 * nkv, 2, 64)
+    c, sn = a.cos().double()[pos][:, None], a.sin().double()[pos][:, None]
+    lo, hi = p.unbind(2)
+    want = torch.stack([lo * c - hi * sn, hi * c + lo * sn], 2)
+    want[:, nq + nkv:] = p[:, nq + nkv:]
+    want = want.view(M, nq + 2 * nkv, 128)
+    got = got.view(M, nq + 2 * nkv, 128)
+    assert (got.double() - want).norm() < 1.01 * 2 ** -8 * want.norm()
+    expect = torch.full_like(cache, 7.0)
+    for i, at in enumerate(slots.tolist()):
+        if at >= 0:
+            expect[at // 16, 0, :, at % 16], expect[at // 16, 1, :, at % 16] = got[i, nq:nq + nkv], got[i, nq + nkv:]
+    assert torch.equal(cache, expect)
+
+
+@pytest.mark.parametrize("quant", [None, "fp8"])
+@pytest.mark.parametrize("hidden,heads,kv", [(512, 4, 2), (2304, 18, 2)])  # half tiles and whole ones
+def test_layers_of_chained_products(hidden, heads, kv, quant, monkeypatch):
+    """Prompts, decode steps and a pass whose logits are not one a sequence, by either route over the same cache."""
+    from shuffle_exchange_amd.inference.v2 import RaggedInferenceEngineConfig, build_engine
+    from shuffle_exchange_amd.inference.v2.model_implementations.llama import RaggedLlama
+    from shuffle_exchange_amd.models import LlamaForCausalLM, llama_config
+    torch.manual_seed(1)
+    cfg = llama_config("llama-tiny", hidden_size=hidden, intermediate_size=1408, num_hidden_layers=2, num_attention_heads=heads,
+                       num_key_value_heads=kv, head_dim=128, vocab_size=1000)
+    model = LlamaForCausalLM(cfg).to("cuda", torch.bfloat16)
+    g = torch.Generator().manual_seed(2)
+    chained, runs = [], []
+    own = RaggedLlama._chain
+    for on in (True, False):
+        def chain(self, *args):
+            chained.append(on and own(self, *args) is not None)
+            return own(self, *args) if on else None
+        monkeypatch.setattr(RaggedLlama, "_chain", chain)
+        g.manual_seed(2)
+        e = build_engine(model, RaggedInferenceEngineConfig(kv_block_size=16, num_kv_blocks=200, weight_quant=quant))
+        out = [e.put([i], [torch.randint(0, 1000, (n,), generator=g)]) for i, n in enumerate((7, 31, 3))]
+        for uids in ([0, 1, 2], [1], [0, 2]):
+            for _ in range(2):
+                out.append(e.put(uids, [torch.randint(0, 1000, (1,), generator=g) for _ in uids]))
+        out.append(e.put([0, 1], [torch.randint(0, 1000, (n,), generator=g) for n in (5, 1)], want=[(1, 4, 0), ()]))
+        runs.append(out)
+    assert any(chained)
+    for a, b in zip(*runs):
+        assert a.dtype == b.dtype and a.shape == b.shape
+        # roundings to bf16 (2^-9 in the mean square) of a dozen tensors a layer, other ones by either route
+        assert (a - b).norm() < 0.02 * b.norm()
