@@ -48,6 +48,9 @@ struct Args {
   // RES: y = bf16(stream * gw)
   const unsigned short *res, *gw;
   int64_t ldr;
+  // RES of one row that attention has left in splits (null: x): unnormalised sums [splits, K] and (max, sum) [splits, K / dim, 2], log2
+  const float *po, *pml;
+  int splits, dim;
   unsigned short* h;  // [M, N], the new stream
   float* sums;        // [N / 16, mp]
   // ROPE: w's rows are nq + 2 nkv heads of 128
@@ -99,8 +102,7 @@ struct Piece {
   static constexpr int PIECE = FP8 ? 256 : 128, XL = FP8 ? 2 : 1;
   u32x4 w[NT][4], x[MB][XL][4];
   // wr, xr: the rows 4 (row / 4) + u of this lane's quad, at chunk 4 g + j
-  __device__ __forceinline__ void load(const char* const (&wr)[NT], int64_t ldw, const unsigned short* const (&xr)[MB][4], int k0, int K,
-                                       int c) {
+  __device__ __forceinline__ void load_w(const char* const (&wr)[NT], int64_t ldw, int k0, int K, int c) {
     const int kw = k0 + c * (FP8 ? 16 : 8);  // K is a multiple of 8 (16), so a lane's vector is in or out
     const bool win = kw < K;
 #pragma unroll
@@ -111,6 +113,8 @@ struct Piece {
         const auto* p = reinterpret_cast<const u32x4*>(wr[t] + u * ldw + (int64_t)kw * (FP8 ? 1 : 2));
         if (win) w[t][u] = ONCE ? __builtin_nontemporal_load(p) : *p;
       }
+  }
+  __device__ __forceinline__ void load_x(const unsigned short* const (&xr)[MB][4], int k0, int K, int c) {
 #pragma unroll
     for (int h = 0; h < XL; ++h) {
       const int kx = k0 + 8 * (FP8 ? 8 * (c >> 2) + 4 * h + (c & 3) : c);
@@ -124,11 +128,25 @@ struct Piece {
         }
     }
   }
+  // one row in LDS for all of them, as the exchange would leave it
+  __device__ __forceinline__ void row_x(const unsigned short* row, int k0, int K, int g) {
+#pragma unroll
+    for (int h = 0; h < XL; ++h)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int kx = k0 + 8 * (4 * (XL * g + h) + u);
+        x[0][h][u] = u32x4{0u, 0u, 0u, 0u};
+        if (kx < K) x[0][h][u] = *reinterpret_cast<const u32x4*>(row + kx);
+      }
+  }
+  template <bool ROW = false>
   __device__ __forceinline__ void multiply(f32x4 (&acc)[MB][NT], bool odd1, bool odd2) {
+    if constexpr (!ROW) {
 #pragma unroll
-    for (int m = 0; m < MB; ++m)
+      for (int m = 0; m < MB; ++m)
 #pragma unroll
-      for (int h = 0; h < XL; ++h) exchange(x[m][h], odd1, odd2);
+        for (int h = 0; h < XL; ++h) exchange(x[m][h], odd1, odd2);
+    }
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       exchange(w[t], odd1, odd2);
@@ -144,16 +162,62 @@ struct Piece {
   }
 };
 
+constexpr int MERGE_K = 2048;  // columns of a row that is merged on its way in
+
+// The row of attention's splits, sum_s 2^(M_s - M) o_s / sum_s 2^(M_s - M) L_s, in bf16 as a launch of its own would leave it. A split
+// without keys has a maximum of -inf and nothing behind it. Four columns a thread, the loads of eight splits at once.
+__device__ __forceinline__ void merge_row(const Args& a, unsigned short* row) {
+  constexpr int U = 8;
+  const int heads = a.K / a.dim;
+  for (int k = 4 * threadIdx.x; k < a.K; k += 4 * 64 * NW) {
+    float top = -INFINITY, den = 0.f;
+    f32x4 num = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < a.splits; s0 += U) {
+      float ms[U], ls[U];
+      f32x4 o[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t s = min(s0 + u, a.splits - 1), at = 2 * (s * heads + k / a.dim);
+        ms[u] = a.pml[at];
+        ls[u] = a.pml[at + 1];
+        o[u] = *reinterpret_cast<const f32x4*>(a.po + s * a.K + k);
+      }
+      float most = top;
+#pragma unroll
+      for (int u = 0; u < U; ++u) most = fmaxf(most, ms[u]);
+      const float r = top == -INFINITY ? 0.f : exp2f(top - most);
+      top = most;
+      den *= r;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) num[q] *= r;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (s0 + u >= a.splits || ms[u] == -INFINITY) continue;
+        const float f = exp2f(ms[u] - top);
+        den += f * ls[u];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) num[q] += f * o[u][q];
+      }
+    }
+    u16x4 v;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = f32_to_bf16(den > 0.f ? num[q] / den : 0.f);
+    *reinterpret_cast<u16x4*>(row + k) = v;
+  }
+}
+
 // HALF (up to 8 rows): a tile of 8 columns, each twice. The matrix core's rows 0 - 7 have one half of a piece's K, rows 8 - 15 the other one,
 // of W and of x alike, and the two blocks of the result that belong together are added: no lane loads what another one does, and there are
 // twice the workgroups, each with half the pieces one behind the other.
-template <bool FP8, int MB, int NT, int EPI, bool ONCE, bool HALF = false>
+template <bool FP8, int MB, int NT, int EPI, bool ONCE, bool HALF = false, bool MERGE = false>
 __global__ void __launch_bounds__(64 * NW, 2) stream_gemm_kernel(Args a) {
   static_assert(!HALF || (MB == 1 && NT == 1), "");
+  static_assert(!MERGE || (EPI == EPI_RES && HALF), "");
   constexpr bool GLU = EPI == EPI_GLU || EPI == EPI_NGLU, NORMED = EPI >= EPI_ROPE;
   constexpr int OT = GLU ? NT / 2 : NT;  // tiles of output columns
   constexpr int TC = HALF ? 8 : 16, PAIRS = TC * NT / 2;
   __shared__ f32x4 red[NW][NT][64];
+  __shared__ __attribute__((aligned(16))) unsigned short merged[MERGE ? MERGE_K : 8];
   __shared__ float squares[NORMED ? NW : 1][NORMED ? 32 : 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, g = lane >> 4;
   const int half = a.N / 2;
@@ -202,7 +266,8 @@ __global__ void __launch_bounds__(64 * NW, 2) stream_gemm_kernel(Args a) {
       }
     }
     P p;
-    p.load(wr, ldw, xr, k0, a.K, c);
+    p.load_w(wr, ldw, k0, a.K, c);
+    if constexpr (!MERGE) p.load_x(xr, k0, a.K, c);
     if (EPI == EPI_RES && wave < OT) {
       const int n = min(column(wave, fq), a.N - 4);
       gw = *reinterpret_cast<const u16x4*>(a.gw + n);
@@ -228,13 +293,20 @@ __global__ void __launch_bounds__(64 * NW, 2) stream_gemm_kernel(Args a) {
         if (lane < quads) *reinterpret_cast<f32x4*>(&squares[wave][4 * lane]) = s;
       }
     }
-    p.multiply(acc, odd1, odd2);
+    if constexpr (MERGE) {
+      merge_row(a, merged);
+      __syncthreads();
+      p.row_x(merged, k0, a.K, g);
+    }
+    p.template multiply<MERGE>(acc, odd1, odd2);
     k0 += NW * STEP;
   }
   for (; k0 - (HALF ? (l16 >> 3) * P::PIECE : 0) < a.K; k0 += NW * STEP) {
     P p;
-    p.load(wr, ldw, xr, k0, a.K, c);
-    p.multiply(acc, odd1, odd2);
+    p.load_w(wr, ldw, k0, a.K, c);
+    if constexpr (MERGE) p.row_x(merged, k0, a.K, g);
+    else p.load_x(xr, k0, a.K, c);
+    p.template multiply<MERGE>(acc, odd1, odd2);
   }
   // lane: columns 4 g .. + 3 of row l16 of every tile
   auto finish = [&](int m, int t) {
@@ -352,18 +424,17 @@ __global__ void __launch_bounds__(64 * NW, 2) stream_gemm_kernel(Args a) {
 }  // namespace st
 
 namespace {
-// the operands that all forms have: x [M, K] bf16, w [N, K] bf16, or e4m3 bytes with wscale fp32 [N]; -> whether w is e4m3
-bool operands(st::Args& a, const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& wscale,
-              const c10::optional<at::Tensor>& bias) {
-  check_beside(x, {w, wscale, bias});
+// w [N, K] bf16, or e4m3 bytes with wscale fp32 [N], for M rows of K; -> whether w is e4m3
+bool weights(st::Args& a, int64_t M, int64_t K, const at::Tensor& w, const c10::optional<at::Tensor>& wscale,
+             const c10::optional<at::Tensor>& bias) {
   const bool fp8 = wscale.has_value() && wscale->defined();
-  SXE_CHECK(x.scalar_type() == at::kBFloat16 && x.dim() == 2 && x.stride(1) == 1 && w.is_cuda() && w.dim() == 2 && w.stride(1) == 1 &&
-                x.size(1) == w.size(1) && (fp8 ? w.element_size() == 1 : w.scalar_type() == at::kBFloat16),
-            "stream_gemm: bf16 x [M, K], w [N, K] bf16 or e4m3 bytes");
-  const int64_t M = x.size(0), N = w.size(0), K = x.size(1), unit = fp8 ? 16 : 8;
+  SXE_CHECK(w.is_cuda() && w.dim() == 2 && w.stride(1) == 1 && w.size(1) == K && (fp8 ? w.element_size() == 1 : w.scalar_type() == at::kBFloat16),
+            "stream_gemm: w [N, K] bf16 or e4m3 bytes");
+  check_beside(w, {wscale, bias});
+  const int64_t N = w.size(0), unit = fp8 ? 16 : 8;
   SXE_CHECK(M >= 1 && M <= 32 && N > 0 && K > 0 && N < (1ll << 31) && K < (1ll << 31), "stream_gemm: 1 <= M <= 32");
-  SXE_CHECK(K % unit == 0 && w.stride(0) % unit == 0 && x.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
-                reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0, "stream_gemm: K and the rows must allow 16-byte loads");
+  SXE_CHECK(K % unit == 0 && w.stride(0) % unit == 0 && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0,
+            "stream_gemm: K and the rows must allow 16-byte loads");
   SXE_CHECK(N % 4 == 0, "stream_gemm: N a multiple of 4");
   if (fp8) {
     SXE_CHECK(wscale->scalar_type() == at::kFloat && wscale->is_contiguous() && wscale->numel() == N, "stream_gemm: wscale fp32 [N]");
@@ -373,8 +444,6 @@ bool operands(st::Args& a, const at::Tensor& x, const at::Tensor& w, const c10::
     SXE_CHECK(bias->scalar_type() == at::kBFloat16 && bias->is_contiguous() && bias->numel() == N, "stream_gemm: bias bf16 [N]");
     a.bias = reinterpret_cast<const unsigned short*>(bias->data_ptr());
   }
-  a.x = reinterpret_cast<const unsigned short*>(x.data_ptr());
-  a.ldx = x.stride(0);
   a.w = w.data_ptr();
   a.ldw = w.stride(0);
   a.M = M;
@@ -382,6 +451,17 @@ bool operands(st::Args& a, const at::Tensor& x, const at::Tensor& w, const c10::
   a.K = K;
   a.mp = M <= 8 ? 8 : M <= 16 ? 16 : 32;
   return fp8;
+}
+
+// x [M, K] bf16 and w
+bool operands(st::Args& a, const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& wscale,
+              const c10::optional<at::Tensor>& bias) {
+  check_beside(x, {w, wscale, bias});
+  SXE_CHECK(x.scalar_type() == at::kBFloat16 && x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0 &&
+                reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0, "stream_gemm: bf16 x [M, K] in rows that allow 16-byte loads");
+  a.x = reinterpret_cast<const unsigned short*>(x.data_ptr());
+  a.ldx = x.stride(0);
+  return weights(a, x.size(0), x.size(1), w, wscale, bias);
 }
 
 // the sums of squares that stream_gemm_res left for x's rows, or none: x is normed
@@ -461,28 +541,63 @@ at::Tensor stream_gemm(const at::Tensor& x, const at::Tensor& w, const c10::opti
   return y;
 }
 
-// h = res + x . w^T (+ bias), and what a product of rms_norm(h) * gw needs: -> [bf16(h * gw), h, sums of h^2 [N / 16, rows]]
-std::vector<at::Tensor> stream_gemm_res(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& wscale,
-                                        const c10::optional<at::Tensor>& bias, const at::Tensor& res, const at::Tensor& gw) {
-  st::Args a{};
-  const bool fp8 = operands(a, x, w, wscale, bias);
-  check_beside(x, {res, gw});
+// one row of attention's splits for x (part_ml given): [splits, 1, heads, dim] and (max, sum) [splits, 1, heads, 2], fp32; x is not read
+static void split_row(st::Args& a, const at::Tensor& part_o, const at::Tensor& part_ml) {
+  SXE_CHECK(part_o.scalar_type() == at::kFloat && part_o.dim() == 4 && part_o.is_contiguous() && part_ml.scalar_type() == at::kFloat &&
+                part_ml.dim() == 4 && part_ml.is_contiguous() && part_o.size(0) > 0 && part_o.size(1) == 1 && part_o.size(3) % 4 == 0 &&
+                part_ml.size(0) == part_o.size(0) && part_ml.size(1) == 1 && part_ml.size(2) == part_o.size(2) && part_ml.size(3) == 2 &&
+                reinterpret_cast<uintptr_t>(part_o.data_ptr()) % 16 == 0, "stream_gemm_res: splits fp32 [S, 1, heads, dim], [S, 1, heads, 2]");
+  a.po = part_o.data_ptr<float>();
+  a.pml = part_ml.data_ptr<float>();
+  a.splits = part_o.size(0);
+  a.dim = part_o.size(3);
+}
+
+// h = res + x . w^T (+ bias), and what a product of rms_norm(h) * gw needs: -> [bf16(h * gw), h, sums of h^2 [tiles of N, rows]]
+static std::vector<at::Tensor> residual(st::Args a, bool fp8, const at::Tensor& w, const at::Tensor& res, const at::Tensor& gw) {
+  check_beside(w, {res, gw});
   SXE_CHECK(a.N % 16 == 0, "stream_gemm_res: whole tiles of 16 columns");
   SXE_CHECK(res.scalar_type() == at::kBFloat16 && res.dim() == 2 && res.size(0) == a.M && res.size(1) == a.N && res.stride(1) == 1 &&
                 res.stride(0) % 4 == 0 && reinterpret_cast<uintptr_t>(res.data_ptr()) % 8 == 0, "stream_gemm_res: res bf16 [M, N]");
   SXE_CHECK(gw.scalar_type() == at::kBFloat16 && gw.is_contiguous() && gw.numel() == a.N && reinterpret_cast<uintptr_t>(gw.data_ptr()) % 8 == 0,
             "stream_gemm_res: gw bf16 [N]");
-  c10::DeviceGuard gd(x.device());
-  auto y = at::empty({a.M, a.N}, x.options()), h = at::empty({a.M, a.N}, x.options());
-  auto sums = at::empty({a.N / (halves(a) ? 8 : 16), a.mp}, x.options().dtype(at::kFloat));
+  c10::DeviceGuard gd(w.device());
+  auto y = at::empty({a.M, a.N}, res.options()), h = at::empty({a.M, a.N}, res.options());
+  auto sums = at::empty({a.N / (halves(a) ? 8 : 16), a.mp}, res.options().dtype(at::kFloat));
   a.y = reinterpret_cast<unsigned short*>(y.data_ptr());
   a.h = reinterpret_cast<unsigned short*>(h.data_ptr());
   a.sums = sums.data_ptr<float>();
   a.res = reinterpret_cast<const unsigned short*>(res.data_ptr());
   a.ldr = res.stride(0);
   a.gw = reinterpret_cast<const unsigned short*>(gw.data_ptr());
-  launch<st::EPI_RES>(a, fp8, plain_tiles(a, fp8));
+  if (a.po == nullptr) {
+    launch<st::EPI_RES>(a, fp8, plain_tiles(a, fp8));
+  } else {
+    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(a.N / 8), dim3(64 * st::NW), 0, cur_stream(), a); };
+    fp8 ? go(st::stream_gemm_kernel<true, 1, 1, st::EPI_RES, false, true, true>) : go(st::stream_gemm_kernel<false, 1, 1, st::EPI_RES, false, true, true>);
+    SXE_LAUNCH_CHECK();
+  }
   return {y, h, sums};
+}
+
+std::vector<at::Tensor> stream_gemm_res(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& wscale,
+                                        const c10::optional<at::Tensor>& bias, const at::Tensor& res, const at::Tensor& gw) {
+  st::Args a{};
+  const bool fp8 = operands(a, x, w, wscale, bias);
+  return residual(a, fp8, w, res, gw);
+}
+
+// the same of one row that attention has left in splits: the flash-decoding merge runs before the product's own loads arrive. Every workgroup
+// reads all splits, so small products only: a step of three layers of hidden 2048, ff 8192, 1000 / 3000 keys, us with a merge launch / so 173 /
+// 168, 175 / 172, e4m3 134 / 130, 142 / 140; but hidden 4096 342 / 342, 355 / 358, 12000 keys 394 / 418
+std::vector<at::Tensor> stream_gemm_res_splits(const at::Tensor& part_o, const at::Tensor& part_ml, const at::Tensor& w,
+                                               const c10::optional<at::Tensor>& wscale, const at::Tensor& res, const at::Tensor& gw) {
+  st::Args a{};
+  check_beside(w, {part_o, part_ml});
+  split_row(a, part_o, part_ml);
+  const bool fp8 = weights(a, 1, part_o.size(2) * part_o.size(3), w, wscale, c10::nullopt);
+  SXE_CHECK(a.K <= st::MERGE_K && halves(a), "stream_gemm_res_splits: w of up to 2048 x 2048");
+  return residual(a, fp8, w, res, gw);
 }
 
 // of x . w^T / rms (sums of stream_gemm_res; None: x is normed): silu(gate) * up in bf16 (glu), or the product in fp32
@@ -541,6 +656,7 @@ at::Tensor stream_gemm_rope(const at::Tensor& x, const at::Tensor& w, const c10:
 TORCH_LIBRARY_FRAGMENT(sxe, m) {
   m.def("stream_gemm(Tensor x, Tensor w, Tensor? wscale, Tensor? bias, bool glu) -> Tensor");
   m.def("stream_gemm_res(Tensor x, Tensor w, Tensor? wscale, Tensor? bias, Tensor res, Tensor gw) -> Tensor[]");
+  m.def("stream_gemm_res_splits(Tensor part_o, Tensor part_ml, Tensor w, Tensor? wscale, Tensor res, Tensor gw) -> Tensor[]");
   m.def("stream_gemm_normed(Tensor x, Tensor w, Tensor? wscale, Tensor? part, float eps, bool glu) -> Tensor");
   m.def("stream_gemm_rope(Tensor x, Tensor w, Tensor? wscale, Tensor? part, float eps, Tensor cos, Tensor sin, Tensor pos, Tensor slots, "
         "Tensor(a!) cache, int nq, int nkv) -> Tensor");
@@ -548,6 +664,7 @@ TORCH_LIBRARY_FRAGMENT(sxe, m) {
 TORCH_LIBRARY_IMPL(sxe, CUDA, m) {
   m.impl("stream_gemm", &sxe::stream_gemm);
   m.impl("stream_gemm_res", &sxe::stream_gemm_res);
+  m.impl("stream_gemm_res_splits", &sxe::stream_gemm_res_splits);
   m.impl("stream_gemm_normed", &sxe::stream_gemm_normed);
   m.impl("stream_gemm_rope", &sxe::stream_gemm_rope);
 }

@@ -33,7 +33,7 @@ import torch.nn.functional as F
 from ....ops import native
 from ....ops.activation import swiglu
 from ....ops.linear import Linear, STREAM_ROWS_SMALL, TILED_GLU_ROWS, glu_faster, glu_linear, glu_tiled, is_own_forward, linear
-from ....ops.linear import chain_faster, stream_glu, stream_head, stream_res, stream_rope, stream_weight
+from ....ops.linear import MERGE_COLUMNS, chain_faster, stream_glu, stream_head, stream_res, stream_res_splits, stream_rope, stream_weight
 from ....ops.norm import RMSNorm
 from ....ops.paged_attention import paged_attention_parts, paged_batch_attention, ragged_attention, rope_kv_cache_append
 from ....ops.rows import gather_last
@@ -312,13 +312,18 @@ class RaggedLlama:
             if a is None:
                 a, h = (norm(x), x) if h is None else norm(x, h)
             qkv = stream_rope(a, ws[0], sums, norm.eps, rope, batch.positions, kv_layer, batch.slots, self.nq, self.nkv)
-            o = self._attention(qkv.view(T, self.nq + 2 * self.nkv, self.head_dim), kv_layer, batch).reshape(T, self.nq * self.head_dim)
-            norm = layer.post_attention_layernorm
+            qkv, norm = qkv.view(T, self.nq + 2 * self.nkv, self.head_dim), layer.post_attention_layernorm
+            if T == 1 and len(ws) > 1 and max(ws[1][0].shape) <= MERGE_COLUMNS:  # the splits' merge in the o product's launch
+                o, parts = paged_attention_parts(qkv[:, :self.nq], kv_layer, batch.block_table, batch.q_start, batch.q_len, batch.kv_len,
+                                                 self.head_dim ** -0.5, batch.max_kv_len)
+            else:
+                o, parts = self._attention(qkv, kv_layer, batch), None
+            o = o.reshape(T, self.nq * self.head_dim) if parts is None else None
             if len(ws) == 1:
                 m, h = norm(self._proj(layer.self_attn.o_proj, o, li, "o"), h)
                 x, a, sums = self._moe(layer, m, li), None, None
                 continue
-            a, h, sums = stream_res(o, ws[1], h, norm.weight)
+            a, h, sums = stream_res(o, ws[1], h, norm.weight) if parts is None else stream_res_splits(parts, ws[1], h, norm.weight)
             mid = stream_glu(a, ws[2], sums, norm.eps)
             after = model.layers[li + 1].input_layernorm if li + 1 < len(chain) else model.norm
             a, h, sums = stream_res(mid, ws[3], h, after.weight)

@@ -159,15 +159,15 @@ def chain_faster(rows, weights):
     """Whether a layer's products (qkv, o, gate | up, down; of MoE layers the first) gain by having its norms, residual sums and RoPE in their
     epilogues, three launches of ~4.7 us a layer, also where the library has the faster product. us a decode step of three layers (two from
     5120 on) and the head, launches of their own (up to 4 rows the norms in prologues of skinny_gemm.hip) / so, 1, 8, 16 and 32 rows: hidden 2048,
-    ff 8192 184 / 173, 202 / 177, 208 / 188, 249 / 216; 3072, 8192 247 / 229, 265 / 234, 280 / 249, 324 / 297; 3584, 18944 386 / 345, 456 / 352,
+    ff 8192 184 / 168, 202 / 177, 208 / 188, 249 / 216; 3072, 8192 247 / 229, 265 / 234, 280 / 249, 324 / 297; 3584, 18944 386 / 345, 456 / 352,
     472 / 374, 729 / 458; 4096, 11008 350 / 332, 374 / 341, 409 / 377, 540 / 509; 4096, 14336 362 / 340, 382 / 355, 402 / 379, 470 / 455; 6144,
     16384, 16 and 32 rows 619 / 604, 688 / 659; 8192, 28672, 4 rows 868 / 756; e4m3 4096, 14336 248 / 254, 297 / 268, 339 / 301; 3072, 8192 179 / 180,
-    219 / 188, 245 / 212; 2048, 8192 140 / 136, 172 / 143; 5120, 13824, 1 and 8 rows 263 / 226, 275 / 254. So one row keeps the prologues where
-    they cost it least (with 1024 keys and more splits to merge 2048, 8192 of eight layers is 433 / 438), and from 17 rows on not 5120, 13824 with 40 kv heads (8 rows 382 / 347, 32 rows 483 / 513), whose last round of the
+    219 / 188, 245 / 212; 2048, 8192 138 / 128, 172 / 143; 5120, 13824, 1 and 8 rows 263 / 226, 275 / 254. So one row of e4m3 keeps the prologues where they cost it
+    least, and from 17 rows on not 5120, 13824 with 40 kv heads (8 rows 382 / 347, 32 rows 483 / 513), whose last round of the
     gate's workgroups is short."""
     w, scale = weights[0]
-    if rows == 1:
-        return w.shape[1] > (2048 if scale is None else 4096)
+    if rows == 1 and scale is not None:
+        return w.shape[1] <= 2048 or w.shape[1] > 4096
     if rows <= STREAM_ROWS or len(weights) == 1:
         return True
     N, K = weights[2][0].shape
@@ -178,6 +178,14 @@ def stream_res(x, wk, res, norm_weight):
     """h = res + x . w^T and what the next product takes of rms_norm(h) * norm_weight, in ONE launch (stream_gemm.hip):
     (bf16(h * norm_weight), h, sums of h^2 by tiles of 16 columns)."""
     return torch.ops.sxe.stream_gemm_res(x, wk[0], wk[1], None, res, norm_weight)
+
+
+MERGE_COLUMNS = 2048  # rows and columns of a weight that stream_gemm.hip merges the splits for in its own launch
+
+
+def stream_res_splits(parts, wk, res, norm_weight):
+    """``stream_res`` of one row that ``paged_attention_parts`` has left in splits, weights of up to MERGE_COLUMNS each way."""
+    return torch.ops.sxe.stream_gemm_res_splits(parts[0], parts[1], wk[0], wk[1], res, norm_weight)
 
 
 def stream_glu(x, wk, sums, eps):

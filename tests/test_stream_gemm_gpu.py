@@ -113,6 +113,26 @@ def test_residual_and_what_a_normed_product_needs(M, N, K, fp8):
     assert (sums[:, :M].T.double() - squares).abs().max() <= 1e-6 * squares.max()
 
 
+@pytest.mark.parametrize("N,heads,dim,splits", [(16, 1, 64, 1), (2048, 16, 128, 5), (2032, 9, 128, 8), (512, 16, 128, 17), (64, 3, 256, 9)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_residual_of_a_row_in_splits(N, heads, dim, splits, fp8):
+    from shuffle_exchange_amd.ops.paged_attention import merge_attention_parts
+    _, w, s, ref = _operands(1, N, heads * dim, fp8, N + splits)
+    po = torch.randn(splits, 1, heads, dim, device="cuda")
+    pml = torch.stack([torch.randn(splits, 1, heads, device="cuda") * 4, torch.rand(splits, 1, heads, device="cuda") + 0.5], -1)
+    if splits > 1:  # splits without keys: nothing is behind their maximum
+        pml[1::3, ..., 0], pml[1::3, ..., 1], po[1::3] = float("-inf"), float("nan"), float("nan")
+    res, gw = torch.randn(1, N, device="cuda").bfloat16(), (1 + 0.3 * torch.randn(N, device="cuda")).bfloat16()
+    got = torch.ops.sxe.stream_gemm_res_splits(po, pml, w, s, res, gw)
+    row = merge_attention_parts(po[pml[:, 0, 0, 0] > -1e30], pml[pml[:, 0, 0, 0] > -1e30], torch.float32).view(1, -1)
+    want = res.double() + row.double() @ ref.T
+    # the row's rounding to bf16 (2^-8 at most) on its way into the product, then that of the result
+    assert (got[1].double() - want).norm() < 1.01 * 2 ** -8 * (want.norm() + (want - res.double()).norm())
+    assert torch.equal(got[0], (got[1].float() * gw.float()).bfloat16())
+    squares = got[1].double().square().view(len(got[2]), -1).sum(-1)
+    assert (got[2][:, 0].double() - squares).abs().max() <= 1e-6 * squares.max() and not got[2][:, 1:].any()
+
+
 @pytest.mark.parametrize("M", [1, 8, 9, 17, 32])
 @pytest.mark.parametrize("N,K,tiles", [(32, 16, 1), (96, 1024, 3), (6208, 2064, 129), (8192, 4096, 256), (16416, 4112, 600)])
 @pytest.mark.parametrize("fp8", [False, True])
