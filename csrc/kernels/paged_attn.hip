@@ -433,7 +433,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const float* __restrict__ pa
   constexpr int TPR = D / 4, RPB = 256 / TPR;
   const int64_t sstride = T * nq, th = (int64_t)blockIdx.x * RPB + threadIdx.x / TPR;  // partial row * nq + h
   const int d = threadIdx.x % TPR * 4;
-  if (th >= sstride) return;
+  if (th >= sstride || part_ml[th * 2 + 1] < 0.f) return;  // a negative sum: no splits, the result is there (paged_prefill.hip)
   const int64_t pt = th / nq, t = rows ? rows[pt] : pt;  // rows: token row of every partial row
   const int h = th - pt * nq;
   float M = -INFINITY, L = 0.f;

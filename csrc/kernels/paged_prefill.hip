@@ -116,6 +116,21 @@ __global__ void __launch_bounds__(NW * 64, D >= 256 ? 1 : 2) prefill_kernel(Args
   const int G = a.nq / a.nkv, rows = nt * G;
   const int row = min(w * 32 + r, rows - 1), tok = row / G, head = kvh * G + row - tok * G, qpos = pos0 + tok;
   const bool wave_on = w * 32 < rows;
+  // keys that some row of the tile sees, in this split; starts are multiples of 64
+  int lo_key = a.window > 0 ? max(0, pos0 - a.window + 1) & ~(KT - 1) : 0, hi_key = min(kl, pos0 + nt);
+  // all of them in one split: its result is the tile's, and (max, sum) of split 0 says so (a sum is never negative)
+  const bool whole = a.splits == 1 || lo_key / a.keys_per_split == (hi_key - 1) / a.keys_per_split;
+  lo_key = max(lo_key, split * a.keys_per_split);
+  hi_key = min(hi_key, (split + 1) * a.keys_per_split);
+  const int n = hi_key > lo_key ? (hi_key - lo_key + KT - 1) / KT : 0;
+  auto partial = [&](int s, int first) { return ((int64_t)s * a.part_rows + first + tok) * a.nq + head; };
+  if (n == 0) {  // the merge reads nothing else of a split whose maximum is -inf
+    if (!whole && w * 32 + r < rows && hf == 0) {
+      a.part_ml[partial(split, part0) * 2] = -INFINITY;
+      a.part_ml[partial(split, part0) * 2 + 1] = 0.f;
+    }
+    return;
+  }
   const int pmin = pos0 + min(w * 32, rows - 1) / G, pmax = pos0 + min(w * 32 + 31, rows - 1) / G;
 
   bf16x8 qf[D / 16];
@@ -126,12 +141,6 @@ __global__ void __launch_bounds__(NW * 64, D >= 256 ? 1 : 2) prefill_kernel(Args
 #pragma unroll
   for (int t = 0; t < D / 32; ++t) o[t] = zero16();
   float m = -INFINITY, l = 0.f;
-
-  // keys that some row of the tile sees, in this split; starts are multiples of 64
-  int lo_key = a.window > 0 ? max(0, pos0 - a.window + 1) & ~(KT - 1) : 0, hi_key = min(kl, pos0 + nt);
-  lo_key = max(lo_key, split * a.keys_per_split);
-  hi_key = min(hi_key, (split + 1) * a.keys_per_split);
-  const int n = hi_key > lo_key ? (hi_key - lo_key + KT - 1) / KT : 0;
 
   const int* bt = a.block_table + (int64_t)seq * a.max_blocks;
   const int64_t head_stride = (int64_t)a.bs * D, half_stride = a.nkv * head_stride, block_stride = 2 * half_stride;
@@ -154,10 +163,8 @@ __global__ void __launch_bounds__(NW * 64, D >= 256 ? 1 : 2) prefill_kernel(Args
   };
   auto block_of = [&](int t) { return WHOLE ? bt[(lo_key + KT * min(t, n - 1)) / a.bs] : 0; };
   int blk = 0;
-  if (n > 0) {
-    load(lo_key, block_of(0), lds);
-    blk = block_of(1);
-  }
+  load(lo_key, block_of(0), lds);
+  blk = block_of(1);
   wait_loads();
   __syncthreads();
   LaneOffs<D> lo;
@@ -185,22 +192,25 @@ __global__ void __launch_bounds__(NW * 64, D >= 256 ? 1 : 2) prefill_kernel(Args
   }
   l += xor32(l);
   if (w * 32 + r >= rows) return;
-  if (a.splits == 1) {
+  int first = part0;
+  asm volatile("" : "+s"(first));  // the partials' rows are worked out here, not held from above
+  if (whole) {
+    if (a.splits > 1 && hf == 0) a.part_ml[partial(0, first) * 2 + 1] = -1.f;
     const float inv = l > 0.f ? 1.f / l : 0.f;
     unsigned short* op = a.out + (int64_t)(t0 + tok) * a.out_tok_stride + (int64_t)head * D + 4 * hf;
 #pragma unroll
     for (int dt = 0; dt < D / 32; ++dt) store_acc_t(o[dt], op + 32 * dt, inv);
   } else {
-    const int64_t idx = ((int64_t)split * a.part_rows + part0 + tok) * a.nq + head;
+    const int64_t mine = partial(split, first);
 #pragma unroll
     for (int dt = 0; dt < D / 32; ++dt)
 #pragma unroll
       for (int g = 0; g < 4; ++g)
-        *reinterpret_cast<f32x4*>(a.part_o + idx * D + 32 * dt + 8 * g + 4 * hf) =
+        *reinterpret_cast<f32x4*>(a.part_o + mine * D + 32 * dt + 8 * g + 4 * hf) =
             f32x4{o[dt][4 * g], o[dt][4 * g + 1], o[dt][4 * g + 2], o[dt][4 * g + 3]};
     if (hf == 0) {
-      a.part_ml[idx * 2] = m;
-      a.part_ml[idx * 2 + 1] = l;
+      a.part_ml[mine * 2] = m;
+      a.part_ml[mine * 2 + 1] = l;
     }
   }
 }

@@ -216,7 +216,8 @@ class DSStateManager:
 class AttentionLists:
     """int32 device lists of one attention over a ragged batch: ``tiles`` [n, 4] (sequence, first token row, tokens, row among
     the token rows that the tiles hold by sequence; None: none), ``tile_rows`` those rows (first row and count of each sequence until
-    ``RaggedBatch.tile_rows`` is asked for them), ``tile_keys`` the longest key range; ``seqs`` [m, 2] (sequence, row among
+    ``RaggedBatch.tile_rows`` is asked for them), ``tile_keys`` the longest key range, ``tile_sizes`` (keys, tokens) of all tiles on the
+    host, ``plans`` what has been made of them; ``seqs`` [m, 2] (sequence, row among
     ``seq_rows``), ``seq_rows``, ``seq_keys`` the same for the sequences outside the tiles (None: none), ``seq_even`` whether they
     are about as long as one another."""
     tiles: Optional[torch.Tensor]
@@ -226,6 +227,8 @@ class AttentionLists:
     seq_rows: Optional[torch.Tensor]
     seq_keys: int
     seq_even: bool
+    tile_sizes: tuple = ((), ())
+    plans: dict = field(default_factory=dict)
 
 
 class RaggedBatch:
@@ -362,7 +365,7 @@ class RaggedBatch:
                 self._tables[key] = AttentionLists(
                     d[:4 * nt].view(nt, 4) if nt else None, held, tiles[0][0] if nt else 0, d[4 * nt:4 * nt + 2 * ns].view(ns, 2) if ns else None,
                     d[4 * nt + 2 * ns:] if ns else None, max((self.host_kv_len[i] for i in flat[::2]), default=0),
-                    even_lengths([self.host_kv_len[i] for i in flat[::2]]))
+                    even_lengths([self.host_kv_len[i] for i in flat[::2]]), ([t[0] for t in tiles], [t[3] for t in tiles]))
             else:
                 self._tables[key] = None
         return self._tables[key]

@@ -10,6 +10,7 @@ import functools
 import math
 import os
 
+import numpy as np
 import torch
 
 from . import native
@@ -250,6 +251,33 @@ def choose_tile_splits(num_tiles, nkv, max_keys, target_wgs=None):
     return -(-max(max_keys, 1) // keys), keys
 
 
+# What a launch of the tile kernel takes, us, heads of 128: its longest piece, TILE_STEP for every 64 keys, or all of them together, TILE_FILL such
+# steps a us; and where tiles have more than one piece the merge, TILE_MERGE for every 16 pieces and 0.15 each, and the fp32 partials that go through
+# memory, a MB in half a us; no piece under 384 keys. Fitted to 450 times (106 batches of prompts, chunks and decodes, heads 32 / 8, 24 / 8, 16 / 4 and 32 / 32, pieces from 256 keys to all
+# of them): the piece that it names is 2 % slower than the best one on average, what ``choose_tile_splits`` names, with the decodes in a launch
+# of their own, 20 %. us, by the latter / by this: 1024 tokens alone 39.7 / 31.7, behind 2048 79 / 76; beside 16 sequences of 200 - 2500 keys 57 /
+# 44, 97 / 88; 64 of 300 - 4000 beside 512 tokens 113 / 93, 128 of 2000 beside 32 196 / 182. Heads of 64 and 256 have another balance: by this and in
+# one launch 1024 behind 2048 54 / 63, 128 of 2000 beside 32 218 / 361.
+TILE_STEP, TILE_FILL, TILE_MERGE = 1.6, 190, 5.0
+TILE_DIM = 128
+_PIECES = np.array([1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 32, 48, 64])
+
+
+def plan_tiles(keys, tokens, nq, nkv, dim):
+    """(splits, keys of a split) of a launch of tiles with these key ranges and tokens: equal pieces of the longest range; a tile has as many as
+    its own range reaches into, and no partials where that is one."""
+    keys, tokens = np.asarray(keys, dtype=np.int64), np.asarray(tokens, dtype=np.int64)
+    most, row = int(keys.max()), int(tokens.sum()) * nq * dim * 4
+    piece = -(-most // (64 * _PIECES[_PIECES <= max(1, -(-most // 384))])) * 64
+    piece = piece[((piece >= 384) | (piece >= most)) & (-(-most // piece) * row <= max(PA_SPLIT_BYTES, row))]
+    each = -(-keys // piece[:, None])  # pieces of every tile
+    partials = (np.where(each > 1, each, 0) * tokens).sum(1) * (nq * dim * 4 / 2 ** 21)
+    cost = (np.maximum(TILE_STEP * piece / 64, (-(-keys // 64)).sum() * nkv / TILE_FILL)
+            + np.where(piece < most, TILE_MERGE * -(-most // (16 * piece)) + 0.15 * -(-most // piece) + partials, 0.0))
+    best = int(piece[cost.argmin()])
+    return -(-most // best), best
+
+
 def _tileable(q, cache, scale):
     return (native.use_hip(q) and q.dtype == torch.bfloat16 and cache.dtype == torch.bfloat16 and q.shape[-1] in (64, 128, 256)
             and q.shape[1] % cache.shape[2] == 0 and q.shape[1] // cache.shape[2] <= TILE_ROWS and scale > 0
@@ -284,10 +312,21 @@ def _flash_prompts(q, kv, batch, window):
     return tuple(took)
 
 
+def _tile_plan(lists, nq, nkv, dim, window):
+    """All layers of a pass ask for the same."""
+    if window is not None or dim != TILE_DIM:
+        return choose_tile_splits(lists.tiles.shape[0], nkv, lists.tile_keys)
+    plan = lists.plans.get((nq, nkv, dim))
+    if plan is None:
+        plan = lists.plans[nq, nkv, dim] = plan_tiles(*lists.tile_sizes, nq, nkv, dim)
+    return plan
+
+
 def ragged_attention(q, cache, batch, scale, window=None, kv=None):
     """Causal attention of a ragged batch's new tokens q [T, nq, D] over their paged keys (the new ones among them).
-    Sequences with many new tokens -- prompts, and chunks of prompts behind earlier tokens -- run the tile kernel, the
-    others the decode kernel. ``kv`` [T, 2 nkv, D]: the new tokens' keys and values as they are in the cache, for the longest
+    Sequences with many new tokens -- prompts, and chunks of prompts behind earlier tokens -- run the tile kernel, and the others with them
+    (heads of 128; 16 sequences of 200 - 2500 keys beside 428 tokens behind 3072, us, in a launch of the decode kernel / so 78 / 56); other
+    heads, under a window, and where no sequence has as many, they run the decode kernel. ``kv`` [T, 2 nkv, D]: the new tokens' keys and values as they are in the cache, for the longest
     prompts."""
     nkv = cache.shape[2]
     if window is not None and batch.max_kv_len <= window:
@@ -296,6 +335,8 @@ def ragged_attention(q, cache, batch, scale, window=None, kv=None):
         return paged_batch_attention(q, cache, batch, scale, window)
     tile, least = TILE_ROWS // (q.shape[1] // nkv), -(-TILE_MIN_ROWS // (q.shape[1] // nkv))
     flash = _flash_prompts(q, kv, batch, window)
+    if window is None and q.shape[2] == TILE_DIM and any(n >= least and (i, n) not in flash for i, n in enumerate(batch.host_q_len)):
+        least = 1
     lists = batch.attention_lists(tile, least, flash)
     if lists is None and not flash:
         return paged_batch_attention(q, cache, batch, scale, window)
@@ -311,7 +352,7 @@ def ragged_attention(q, cache, batch, scale, window=None, kv=None):
     meta = (q, cache, batch.block_table, batch.q_start, batch.q_len, batch.kv_len)
     for x in (batch.attention_lists(tile, least, flash, True) if flash else None, lists):
         if x is not None and x.tiles is not None:
-            splits, keys = choose_tile_splits(x.tiles.shape[0], nkv, x.tile_keys)
+            splits, keys = _tile_plan(x, q.shape[1], nkv, q.shape[2], window)
             rows = batch.tile_rows(x) if splits > 1 else None
             torch.ops.sxe.paged_prefill(*meta, x.tiles, rows, float(scale), int(window or 0), splits, keys, out)
     if lists is not None and lists.seqs is not None:

@@ -48,6 +48,39 @@ def test_tile_splits_cover_the_keys():
                 assert k % 64 == 0 and n * k >= keys > (n - 1) * k
 
 
+@pytest.mark.parametrize("sizes", [[(1, 1)], [(64, 32)], [(65, 1)], [(257, 32), (33, 32)], [(100000, 32)] * 3 + [(1, 1)] * 9, [(4096, 32)] * 1000,
+                                   [(131072, 16)] * 2000])
+@pytest.mark.parametrize("nq,nkv", [(32, 8), (7, 7)])
+def test_tile_plan_covers_the_keys_and_bounds_its_partials(sizes, nq, nkv):
+    keys, tokens = zip(*sizes)
+    n, k = PA.plan_tiles(keys, tokens, nq, nkv, 128)
+    assert k % 64 == 0 and n * k >= max(keys) > (n - 1) * k
+    assert n == 1 or (k >= 384 and n * sum(tokens) * nq * 128 * 4 <= PA.PA_SPLIT_BYTES)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("seqs", [[(4000, 300), (700, 1), (31, 2), (5, 40)], [(0, 64), (63, 1), (64, 1), (300, 8)], [(0, 1), (0, 700)]])
+@pytest.mark.parametrize("keys", [64, 320, 1024, 4352])
+@pytest.mark.parametrize("nq,nkv,D,window", [(32, 8, 128, None), (12, 12, 128, None), (8, 4, 128, 100), (4, 4, 64, None), (8, 4, 256, 300)])
+def test_pieces_of_tiles(seqs, keys, nq, nkv, D, window):
+    """Tiles that lie in one piece, in several, in front of or behind the others' (windows): decodes and prompts in one launch."""
+    from shuffle_exchange_amd.ops import native
+    native.require_hip()
+    b, blocks = _batch(seqs, 64, "cuda", seed=3)
+    g = torch.Generator(device="cuda").manual_seed(4)
+    cache = torch.randn(blocks, 2, nkv, 64, D, device="cuda", generator=g).to(torch.bfloat16)
+    q = torch.randn(b.num_tokens, nq, D, device="cuda", generator=g).to(torch.bfloat16)
+    x = b.attention_lists(128 // (nq // nkv), 1)
+    splits = -(-x.tile_keys // keys)
+    out = torch.full_like(q, float("nan"))
+    torch.ops.sxe.paged_prefill(q, cache, b.block_table, b.q_start, b.q_len, b.kv_len, x.tiles, b.tile_rows(x) if splits > 1 else None,
+                                D ** -0.5, window or 0, splits, keys, out)
+    ref = PA.paged_attention_reference(q.float(), cache.float(), b.block_table, b.q_start, b.q_len, b.kv_len, D ** -0.5, window)
+    for i in range(b.num_seqs):  # p and the output are rounded to 8 bits each, as in test_ragged_attention
+        s, n = b.host_q_start[i], b.host_q_len[i]
+        assert ((out[s:s + n].float() - ref[s:s + n]).norm() / ref[s:s + n].norm()).item() < 8e-3, seqs[i]
+
+
 @pytest.mark.parametrize("rows,seqs,keys", [(8192, 1, 131072), (16984, 16, 16384), (32768, 64, 16384), (131072, 32, 4096), (256, 256, 131072),
                                             (64, 64, 8192), (1, 1, 131072), (0, 1, 1)])
 @pytest.mark.parametrize("nq,nkv,D", [(32, 8, 128), (64, 8, 128), (16, 1, 256), (7, 7, 64)])
@@ -132,6 +165,8 @@ def test_long_prompts(seqs, nq, nkv, monkeypatch):
     """The training forward for a prompt's first tokens beside the tile and decode kernels for the rest of the batch."""
     for name in ("FLASH_WHOLE", "FLASH_TAIL"):
         monkeypatch.setattr(PA, name, (128, 1))
+    from shuffle_exchange_amd.ops import native
+    native.require_hip()
     b, blocks = _batch(seqs, 64, "cuda", seed=3)
     g = torch.Generator(device="cuda").manual_seed(4)
     cache = torch.randn(blocks, 2, nkv, 64, 128, device="cuda", generator=g).to(torch.bfloat16)
