@@ -291,9 +291,45 @@ void paged_prefill(const at::Tensor& q, const at::Tensor& cache, const at::Tenso
   if (splits > 1) paged_merge(part_o, part_ml, *rows, out);
 }
 
+// (splits, keys of a split) of a launch of tiles with these key ranges (longest first) and tokens: equal pieces of the longest range, of which a
+// tile has as many as its own range reaches into, and no partials where that is one. What takes least by this account, in us: the longest
+// piece, 1.6 for every 64 keys, or all of them together, 190 such steps of a kv head a us; and where tiles have more than one piece the
+// merge, 5 for every 16 pieces and 0.15 each, and the fp32 partials through memory, a MB in half a us. No piece under 384 keys, and no more
+// partials than `bytes`. Fitted to 450 times of heads of 128 (106 batches of prompts, chunks and decodes, heads 32 / 8, 24 / 8, 16 / 4 and 32 / 32,
+// pieces from 256 keys to all of them): what it names is 2 % slower than the best piece on average; two workgroups a CU of equal key
+// ranges, with the decodes in a launch of their own, 20 %. us, by that rule / by this: 1024 tokens alone 39.7 / 31.7, behind 2048 79 / 76; beside
+// 16 sequences of 200 - 2500 keys 57 / 44, 97 / 88; 64 of 300 - 4000 beside 512 tokens 113 / 93, 128 of 2000 beside 32 196 / 182.
+std::tuple<int64_t, int64_t> paged_prefill_plan(at::IntArrayRef keys, at::IntArrayRef tokens, int64_t nq, int64_t nkv, int64_t dim, int64_t bytes) {
+  SXE_CHECK(!keys.empty() && keys.size() == tokens.size() && nq > 0 && nkv > 0 && dim > 0, "paged_prefill_plan: keys and tokens of every tile");
+  int64_t most = 1, all = 0, steps = 0;
+  for (size_t i = 0; i < keys.size(); ++i) {
+    SXE_CHECK(keys[i] > 0 && tokens[i] > 0, "paged_prefill_plan: tiles of no keys or tokens");
+    most = std::max(most, keys[i]);
+    all += tokens[i];
+    steps += (keys[i] + pp::KT - 1) / pp::KT;
+  }
+  const int64_t row = nq * dim * 4;
+  std::tuple<int64_t, int64_t> best;
+  double least = 1e30;
+  for (int64_t s : {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 32, 48, 64}) {
+    const int64_t piece = (most + s * pp::KT - 1) / (s * pp::KT) * pp::KT, splits = (most + piece - 1) / piece;
+    if (s > 1 && (piece < 384 || splits * all * row > bytes)) break;
+    double us = std::max(1.6 * piece / pp::KT, steps * nkv / 190.0);
+    if (splits > 1) {
+      int64_t held = 0;
+      for (size_t i = 0; i < keys.size(); ++i)
+        if (keys[i] > piece) held += (keys[i] + piece - 1) / piece * tokens[i];
+      us += 5.0 * ((splits + 15) / 16) + 0.15 * splits + (double)held * row / (1 << 21);
+    }
+    if (us < least) least = us, best = {splits, piece};
+  }
+  return best;
+}
+
 }  // namespace sxe
 
 TORCH_LIBRARY_FRAGMENT(sxe, m) {
+  m.def("paged_prefill_plan(int[] keys, int[] tokens, int nq, int nkv, int dim, int bytes) -> (int, int)", &sxe::paged_prefill_plan);
   m.def("paged_prefill(Tensor q, Tensor cache, Tensor block_table, Tensor q_start, Tensor q_len, Tensor kv_len, "
         "Tensor tiles, Tensor? rows, float scale, int window, int splits, int keys_per_split, Tensor(a!) out) -> ()");
 }

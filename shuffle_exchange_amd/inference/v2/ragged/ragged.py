@@ -215,7 +215,7 @@ class DSStateManager:
 @dataclass
 class AttentionLists:
     """int32 device lists of one attention over a ragged batch: ``tiles`` [n, 4] (sequence, first token row, tokens, row among
-    the token rows that the tiles hold by sequence; None: none), ``tile_rows`` those rows (first row and count of each sequence until
+    the token rows that the tiles hold by sequence; None: none), ``tile_rows`` those rows (first row and count of neighbouring sequences until
     ``RaggedBatch.tile_rows`` is asked for them), ``tile_keys`` the longest key range, ``tile_sizes`` (keys, tokens) of all tiles on the
     host, ``plans`` what has been made of them; ``seqs`` [m, 2] (sequence, row among
     ``seq_rows``), ``seq_rows``, ``seq_keys`` the same for the sequences outside the tiles (None: none), ``seq_even`` whether they
@@ -353,7 +353,10 @@ class RaggedBatch:
                 at = first.get(i, 0)
                 if n >= least or tails:
                     tiles += [(seen + min(j + tile, n), i, q + j, min(tile, n - j), a + j - at) for j in range(at, n, tile)]
-                    held.append((q + at, n - at))
+                    if held and sum(held[-1]) == q + at:
+                        held[-1] = (held[-1][0], held[-1][1] + n - at)
+                    else:
+                        held.append((q + at, n - at))
                     a += n - at
                 elif n:
                     flat += [i, len(rows)]
@@ -372,7 +375,10 @@ class RaggedBatch:
 
     def tile_rows(self, lists):
         """int32 device list of the token rows that ``lists.tiles`` hold, sequence by sequence."""
-        if isinstance(lists.tile_rows, list):
+        if isinstance(lists.tile_rows, list) and len(lists.tile_rows) == 1:
+            q, n = lists.tile_rows[0]
+            lists.tile_rows = torch.arange(q, q + n, dtype=torch.int32, device=self.slots.device)
+        elif isinstance(lists.tile_rows, list):
             lists.tile_rows = self._upload(torch.cat([torch.arange(q, q + n, dtype=torch.int32) for q, n in lists.tile_rows]), 1).view(-1)
         return lists.tile_rows
 

@@ -10,7 +10,6 @@ import functools
 import math
 import os
 
-import numpy as np
 import torch
 
 from . import native
@@ -251,31 +250,10 @@ def choose_tile_splits(num_tiles, nkv, max_keys, target_wgs=None):
     return -(-max(max_keys, 1) // keys), keys
 
 
-# What a launch of the tile kernel takes, us, heads of 128: its longest piece, TILE_STEP for every 64 keys, or all of them together, TILE_FILL such
-# steps a us; and where tiles have more than one piece the merge, TILE_MERGE for every 16 pieces and 0.15 each, and the fp32 partials that go through
-# memory, a MB in half a us; no piece under 384 keys. Fitted to 450 times (106 batches of prompts, chunks and decodes, heads 32 / 8, 24 / 8, 16 / 4 and 32 / 32, pieces from 256 keys to all
-# of them): the piece that it names is 2 % slower than the best one on average, what ``choose_tile_splits`` names, with the decodes in a launch
-# of their own, 20 %. us, by the latter / by this: 1024 tokens alone 39.7 / 31.7, behind 2048 79 / 76; beside 16 sequences of 200 - 2500 keys 57 /
-# 44, 97 / 88; 64 of 300 - 4000 beside 512 tokens 113 / 93, 128 of 2000 beside 32 196 / 182. Heads of 64 and 256 have another balance: by this and in
-# one launch 1024 behind 2048 54 / 63, 128 of 2000 beside 32 218 / 361.
-TILE_STEP, TILE_FILL, TILE_MERGE = 1.6, 190, 5.0
+# Heads that run all sequences of a batch in the tile kernel's launch, in pieces by ``paged_prefill_plan`` (csrc/kernels/paged_prefill.hip has the
+# figures). Heads of 64 and 256 have another balance: so, and by ``choose_tile_splits`` with the decodes in a launch of their own, 1024
+# tokens behind 2048 63 / 54 us, 128 decodes of 2000 keys beside 32 tokens 361 / 218.
 TILE_DIM = 128
-_PIECES = np.array([1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 32, 48, 64])
-
-
-def plan_tiles(keys, tokens, nq, nkv, dim):
-    """(splits, keys of a split) of a launch of tiles with these key ranges and tokens: equal pieces of the longest range; a tile has as many as
-    its own range reaches into, and no partials where that is one."""
-    keys, tokens = np.asarray(keys, dtype=np.int64), np.asarray(tokens, dtype=np.int64)
-    most, row = int(keys.max()), int(tokens.sum()) * nq * dim * 4
-    piece = -(-most // (64 * _PIECES[_PIECES <= max(1, -(-most // 384))])) * 64
-    piece = piece[((piece >= 384) | (piece >= most)) & (-(-most // piece) * row <= max(PA_SPLIT_BYTES, row))]
-    each = -(-keys // piece[:, None])  # pieces of every tile
-    partials = (np.where(each > 1, each, 0) * tokens).sum(1) * (nq * dim * 4 / 2 ** 21)
-    cost = (np.maximum(TILE_STEP * piece / 64, (-(-keys // 64)).sum() * nkv / TILE_FILL)
-            + np.where(piece < most, TILE_MERGE * -(-most // (16 * piece)) + 0.15 * -(-most // piece) + partials, 0.0))
-    best = int(piece[cost.argmin()])
-    return -(-most // best), best
 
 
 def _tileable(q, cache, scale):
@@ -318,7 +296,9 @@ def _tile_plan(lists, nq, nkv, dim, window):
         return choose_tile_splits(lists.tiles.shape[0], nkv, lists.tile_keys)
     plan = lists.plans.get((nq, nkv, dim))
     if plan is None:
-        plan = lists.plans[nq, nkv, dim] = plan_tiles(*lists.tile_sizes, nq, nkv, dim)
+        most = lists.tile_keys
+        plan = lists.plans[nq, nkv, dim] = ((1, -(-most // 64) * 64) if most <= 640 else  # no two pieces of 384 keys and more
+                                            torch.ops.sxe.paged_prefill_plan(*lists.tile_sizes, nq, nkv, dim, PA_SPLIT_BYTES))
     return plan
 
 
@@ -335,8 +315,10 @@ def ragged_attention(q, cache, batch, scale, window=None, kv=None):
         return paged_batch_attention(q, cache, batch, scale, window)
     tile, least = TILE_ROWS // (q.shape[1] // nkv), -(-TILE_MIN_ROWS // (q.shape[1] // nkv))
     flash = _flash_prompts(q, kv, batch, window)
-    if window is None and q.shape[2] == TILE_DIM and any(n >= least and (i, n) not in flash for i, n in enumerate(batch.host_q_len)):
-        least = 1
+    if window is None and q.shape[2] == TILE_DIM:
+        done = {i for i, _ in flash}
+        if (max(batch.host_q_len, default=0) >= least if not done else any(n >= least and i not in done for i, n in enumerate(batch.host_q_len))):
+            least = 1
     lists = batch.attention_lists(tile, least, flash)
     if lists is None and not flash:
         return paged_batch_attention(q, cache, batch, scale, window)

@@ -76,3 +76,26 @@ def test_even_and_uneven_lengths(monkeypatch):
             a, b = eg.put(live, toks), ee.put(live, toks)
             assert ((a - b).norm() / b.norm()).item() < 2e-2, live
     assert eg._decode_runner().num_graphs == 2 and eg._decode_runner().replays == 12
+
+
+@pytest.mark.parametrize("n", [9, 12, 13, 17, 25])
+def test_buckets_between_powers_of_two(n):
+    from shuffle_exchange_amd.inference.v2.decode_graphs import sequence_bucket
+    from shuffle_exchange_amd.models import LlamaForCausalLM, llama_config
+    assert [sequence_bucket(i) for i in (1, 3, 5, 8, 9, 12, 13, 17, 24, 25, 33, 49, 256)] == [1, 4, 8, 8, 12, 12, 16, 24, 24, 32, 64, 64, 256]
+    assert [sequence_bucket(i, True) for i in (3, 9, 24, 33, 48, 49, 192, 193)] == [4, 12, 24, 48, 48, 64, 192, 256]
+    torch.manual_seed(0)
+    cfg = llama_config("llama-tiny", hidden_size=512, intermediate_size=1024, num_attention_heads=4, num_key_value_heads=2,
+                       vocab_size=512, num_hidden_layers=2, max_position_embeddings=1024)
+    model = LlamaForCausalLM(cfg).to("cuda", torch.bfloat16).eval()
+    eg, ee = _engine(model, True), _engine(model, False)
+    g = torch.Generator().manual_seed(n)
+    uids = list(range(n))
+    for e in (eg, ee):
+        g.manual_seed(n)
+        e.put(uids, [torch.randint(0, 512, (3 + 5 * u,), generator=g) for u in uids])
+    for _ in range(4):
+        toks = [torch.randint(0, 512, (1,), generator=g) for _ in uids]
+        a, b = eg.put(uids, toks), ee.put(uids, toks)
+        assert a.shape == b.shape and ((a - b).norm() / b.norm()).item() < 2e-2
+    assert list(eg._decode_runner()._graphs)[0][0] == sequence_bucket(n)

@@ -52,8 +52,11 @@ def test_tile_splits_cover_the_keys():
                                    [(131072, 16)] * 2000])
 @pytest.mark.parametrize("nq,nkv", [(32, 8), (7, 7)])
 def test_tile_plan_covers_the_keys_and_bounds_its_partials(sizes, nq, nkv):
+    from shuffle_exchange_amd.ops import native
+    if not native.status()["hip"]:
+        pytest.skip("the HIP library is not built")
     keys, tokens = zip(*sizes)
-    n, k = PA.plan_tiles(keys, tokens, nq, nkv, 128)
+    n, k = torch.ops.sxe.paged_prefill_plan(keys, tokens, nq, nkv, 128, PA.PA_SPLIT_BYTES)
     assert k % 64 == 0 and n * k >= max(keys) > (n - 1) * k
     assert n == 1 or (k >= 384 and n * sum(tokens) * nq * 128 * 4 <= PA.PA_SPLIT_BYTES)
 
