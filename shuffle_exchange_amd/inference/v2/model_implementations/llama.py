@@ -123,6 +123,9 @@ class RaggedLlama:
         self.embed_impl = H.instantiate_embed(H.EmbedConfig(emb.shape[0], emb.shape[1], emb.dtype, dev), emb, pins) \
             if emb is not None else None
         self.moe_impl = None
+        # short passes wait for the host, those with experts for these: us a pass of two layers of 2048, experts of 8192 (0.8 GB), 2 prompts of 210
+        # and 564 tokens 704, with own short products 717; of 3072 (1.2 GB), 18 and 62 710, 718
+        self._host_bound = not self.is_moe
         if self.is_moe:
             l0 = model.layers[0]
             moe = (l0.block_sparse_moe if hasattr(l0, "block_sparse_moe") else l0.moe).deepspeed_moe
@@ -197,7 +200,7 @@ class RaggedLlama:
         # kernel); larger batches keep the module's bf16 weight on hipBLASLt
         if self.qw is not None and key in self.qw[li]:
             return self.qw[li][key](x)
-        return mod(x)
+        return linear(x, mod.weight, mod.bias, self._host_bound) if is_own_forward(mod, Linear) else mod(x)
 
     # decode (<= 4 tokens): RMSNorm folded into the QKV / gate_up GEMMs as their prologue, SwiGLU into gate_up's
     # epilogue (skinny_gemm.hip) -- three latency-bound launches fewer per layer

@@ -44,6 +44,8 @@ class _Gated(torch.autograd.Function):
 def gated_act(gu, act="silu"):
     a = ACT[act] if isinstance(act, str) else int(act)
     if native.use_hip(gu):
+        if not torch.is_grad_enabled() and native.plain(gu):
+            return torch.ops.sxe.gated_act_fwd(gu.contiguous(), a)
         return _Gated.apply(gu, a)
     g, u = gu.chunk(2, dim=-1)
     return (_act_ref(g.float(), a) * u.float()).to(gu.dtype)

@@ -280,6 +280,15 @@ def _narrow(rows, N, K):
 _capturing = torch.cuda.is_current_stream_capturing
 
 
+def _eager_own(rows, N, K):
+    """Products of eager serving passes of 33 to 768 rows: these wait for the host, whom a call of the library costs 14 us more; on the device own ones
+    take (us, library / here) at 2048 x 2048, 64 to 512 rows 12 / 14 - 13 / 24, 3072 x 2048 12 / 15 - 15 / 24, 4096 x 4096 15 / 19 - 29 / 31, 6144 x
+    4096 18 / 21 - 37 / 40, 16384 x 3072 26 / 32 - 53 / 51, beside 40 us and more of a layer's other kernels. So not where a graph is captured,
+    nor beyond NARROW_WORK, where the device is what a pass waits for. us a pass of two layers: prompts of 26 - 30 tokens, 1b 677 / 484, 136 and 140,
+    3b 652 / 568, 51 of 31 - 56, 8b 804 / 716; 256 tokens at a time beside 7 sequences, 8b 1550 / 1203."""
+    return STREAM_ROWS_SMALL < rows <= 768 and N >= 512 and K >= 512 and rows * N * K <= NARROW_WORK and not _capturing()
+
+
 def product(x, weight, bias=None):
     """``F.linear`` for the inside of autograd functions: no graph is built where it runs own kernels (``_tiled``)."""
     rows = x.numel() // max(1, x.shape[-1])
@@ -786,7 +795,8 @@ class _Linear(torch.autograd.Function):
         return dx, dw, db
 
 
-def linear(x, weight, bias=None):
+def linear(x, weight, bias=None, host_bound=False):
+    """``host_bound``: the calls around this one wait for the host, so short ones may take longer on the device (``_eager_own``)."""
     if not isinstance(weight, torch.Tensor):  # quantized inference weight (ops/fp_quantizer.FP8Weight)
         return weight.linear(x, bias)
     grad = torch.is_grad_enabled() and (weight.requires_grad or x.requires_grad or (bias is not None and bias.requires_grad))
@@ -796,7 +806,7 @@ def linear(x, weight, bias=None):
         n, K = x.numel(), x.shape[-1]
         few = n <= max(SKINNY_MAX_M, STREAM_ROWS_SMALL) * K
         # the sizes first: a call that stays with the library is host-bound at a few hundred rows, and what follows is 2 us
-        if ((few or (weight.dim() == 2 and _tiled_faster(n // K, *weight.shape)))
+        if ((few or (weight.dim() == 2 and (_tiled_faster(n // K, *weight.shape) or (host_bound and _eager_own(n // K, *weight.shape)))))
                 and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == torch.bfloat16)
                 and native.plain(x, weight, bias)):
             if few:
@@ -804,7 +814,7 @@ def linear(x, weight, bias=None):
                 if y is None:
                     y = _stream(x, weight, bias)
             else:
-                y = _tiled(x, weight, bias)
+                y = _tiled(x, weight, bias, True)
             if y is not None:
                 return y
     return F.linear(x, weight, bias)

@@ -22,7 +22,7 @@ HIP_LIB = os.environ.get("SXE_HIP_LIB") or os.path.join(_HERE, "_sxe_hip.so")  #
 CPU_LIB = os.path.join(_HERE, "_sxe_cpu.so")
 
 _lock = threading.Lock()
-_state = {"hip": None, "cpu": None, "hip_err": None, "cpu_err": None}
+_state = {"hip": None, "cpu": None, "hip_err": None, "cpu_err": None, "gpu": False}
 
 
 def _load(kind, path):
@@ -40,6 +40,8 @@ def _load(kind, path):
             return False
         try:
             torch.ops.load_library(path)
+            if kind == "hip":  # every operator asks for both: 3 us of the host a call where torch is asked for the GPU each time
+                _state["gpu"] = torch.cuda.is_available()
             _state[kind] = True
         except Exception as e:  # pragma: no cover - depends on the box
             _state[kind] = False
@@ -49,10 +51,12 @@ def _load(kind, path):
 
 def hip_available():
     """True when the HIP kernels can be used (extension loaded AND a GPU is present)."""
-    return torch.cuda.is_available() and _load("hip", HIP_LIB)
+    return _state["gpu"] or torch.cuda.is_available() and _load("hip", HIP_LIB)
 
 
 def require_hip():
+    if _state["gpu"]:  # loaded, beside a GPU
+        return torch.ops.sxe
     if not torch.cuda.is_available():
         raise RuntimeError("sxe: HIP kernels requested on a process without a GPU")
     if not _load("hip", HIP_LIB):

@@ -77,9 +77,19 @@ class _NormFn(torch.autograd.Function):
         return dx, (dx if ctx.has_res else None), dw, db, None, None
 
 
+def _no_graph(x, residual, weight, bias, eps, layernorm):
+    """The forward by itself: an autograd function costs the host 12 us a call, which is what eager serving passes wait for."""
+    shape = x.shape
+    y, _, _, h = torch.ops.sxe.norm_fwd(x.contiguous().view(-1, shape[-1]), residual.contiguous().view(-1, shape[-1]) if residual is not None else None,
+                                        weight, bias, float(eps), layernorm)
+    return y.view(shape) if residual is None else (y.view(shape), h.view(shape))
+
+
 def rms_norm(x, weight, eps=1e-6, residual=None):
     """Returns y (and the new residual h = x + residual when ``residual`` is given)."""
     if native.use_hip(x):
+        if not torch.is_grad_enabled() and native.plain(x, residual, weight):
+            return _no_graph(x, residual, weight, None, eps, False)
         y, h = _NormFn.apply(x, residual, weight, None, eps, False)
         return (y, h) if residual is not None else y
     h = x + residual if residual is not None else x
@@ -89,6 +99,8 @@ def rms_norm(x, weight, eps=1e-6, residual=None):
 
 def layer_norm(x, weight, bias=None, eps=1e-5, residual=None):
     if native.use_hip(x):
+        if not torch.is_grad_enabled() and native.plain(x, residual, weight, bias):
+            return _no_graph(x, residual, weight, bias, eps, True)
         y, h = _NormFn.apply(x, residual, weight, bias, eps, True)
         return (y, h) if residual is not None else y
     h = x + residual if residual is not None else x

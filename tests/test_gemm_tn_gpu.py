@@ -333,3 +333,45 @@ def test_gpt2_block_packed_attention():
     assert (y.double() - want).norm() <= 4e-3 * want.norm()  # roundings to 8 bits of the sums: 2^-9 each
     for a, b in zip(got, torch.autograd.grad(want, [xd, *P.values()], dy.double())):
         assert (a.double() - b).norm() <= 2e-2 * b.norm(), a.shape  # a chain of a dozen of them
+
+
+@pytest.mark.parametrize("M,N,K,taken", [(33, 512, 512, True), (768, 3072, 2048, True), (769, 3072, 2048, False), (32, 3072, 2048, False), (85, 28672, 4096, True),
+                                         (86, 28672, 4096, False), (300, 4096, 4096, True), (300, 4096, 448, False)])
+def test_short_products_of_eager_passes(M, N, K, taken, monkeypatch):
+    """Calls that wait for the host: own products from 33 rows on, with what these do not read, and what is captured, left to the library."""
+    from shuffle_exchange_amd.ops import linear as L
+    x, w, b = _operands(M, N, K)
+    seen = [None]
+    tiled = L._tiled
+    monkeypatch.setattr(L, "_tiled", lambda *a: seen.append(tiled(*a)) or seen[-1])
+    with torch.no_grad():
+        y = L.linear(x, w, b, True)
+        assert (seen[-1] is not None) == taken
+        _close(y, x.double() @ w.double().t() + b.double(), x, w, 2.0)
+        seen.append(None)
+        odd = torch.randn(M, K + 4, device="cuda").bfloat16()[:, :K]
+        assert torch.equal(L.linear(odd, w, None, True), F.linear(odd, w)) and seen[-1] is None
+        n = len(seen)
+        monkeypatch.setattr(L, "_capturing", lambda: True)
+        if M > 32:
+            assert torch.equal(L.linear(x, w, b, True), F.linear(x, w, b)) and len(seen) == n
+    assert L.linear(x.requires_grad_(), w, b, True).requires_grad
+
+
+@pytest.mark.parametrize("shape", [(5, 256), (2, 3, 1024), (1, 4128)])
+def test_norms_and_gates_without_a_graph(shape):
+    """The forward by itself and inside its autograd function: the same bits, for rows that lie apart, too."""
+    from shuffle_exchange_amd.ops.activation import gated_act
+    from shuffle_exchange_amd.ops.norm import layer_norm, rms_norm
+    H = shape[-1]
+    x = torch.randn(*shape[:-1], H + 8, device="cuda").bfloat16()[..., :H]
+    r = torch.randn(*shape, device="cuda").bfloat16()
+    w, b = torch.randn(H, device="cuda").bfloat16(), torch.randn(H, device="cuda").bfloat16()
+    calls = [lambda: rms_norm(x, w, 1e-5), lambda: rms_norm(x, w, 1e-5, r), lambda: layer_norm(x, w, b), lambda: layer_norm(x, w, None, 1e-6, r),
+             lambda: gated_act(x, "silu"), lambda: gated_act(x, "gelu")]
+    for f in calls:
+        with torch.no_grad():
+            a = f()
+        b_ = f()
+        for s, t in zip(*(v if isinstance(v, tuple) else (v,) for v in (a, b_))):
+            assert torch.equal(s, t) and s.shape == t.shape and s.dtype == t.dtype
