@@ -41,11 +41,24 @@ struct Args {
 
 // first row of an expert
 __device__ __forceinline__ int row_of(const Args& a, int e) { return a.offs != nullptr ? min(max(a.offs[e], 0), a.R) : e * a.C; }
-template <int BM>
-__device__ __forceinline__ int tiles_of(const Args& a, int e) {
-  if (e >= a.E) return 0;
-  const int lo = row_of(a, e), hi = row_of(a, e + 1);
-  return hi > lo ? (hi - lo + BM - 1) / BM : 0;
+__device__ __forceinline__ int rows_of(const Args& a, int e) { return e < a.E ? max(row_of(a, e + 1) - row_of(a, e), 0) : 0; }
+__device__ __forceinline__ int tiles_of(const Args& a, int e, int bm) { return (rows_of(a, e) + bm - 1) / bm; }
+
+// When tiles of `bm` rows end, in slabs of a tile of 256: rounds of `whole` ones over the CUs, then what is left of them with the experts' last
+// tiles, of more than 128 rows (`large`), of more than 64 or fewer. A slab of 192 rows takes 0.87 of one of 256, of 128
+// 0.65, of 64 0.5.
+constexpr float kClearly = 0.93f;
+__host__ __device__ inline float end_of(int bm, int whole, int large, int some, int few) {
+  const float w = bm == 256 ? 1.f : bm == 192 ? 0.87f : 0.65f, ws = some > 0 ? 0.65f : 0.5f;
+  const int small = some + few;
+  const int full = whole / kNumCUs, big = whole % kNumCUs + large, rounds = (big + kNumCUs - 1) / kNumCUs, free = rounds * kNumCUs - big;
+  const auto more = [](int n) { return (n + kNumCUs - 1) / kNumCUs; };
+  // the small ones on what the last round of large ones leaves free, a second time there if that is enough, else everywhere behind it
+  float tail = rounds * w;
+  if (rounds == 0) tail = more(small) * ws;
+  else if (small > 2 * free) tail += more(small - free) * ws;
+  else if (small > free) tail += 2 * ws > w ? 2 * ws - w : 0.f;
+  return full * w + tail;
 }
 
 // The tile of rows r0 .. r1 of an expert (T::BM of them at most, `used` of them with products), columns from n0 on
@@ -133,21 +146,46 @@ __device__ __forceinline__ void run_tile(const Args& a, int expert, int r0, int 
 }
 
 using T256 = Tile<2, 4, 8, 4, 2, 3, 2>;
+using T192 = Tile<2, 4, 6, 4, 2, 3, 2>;
 using T128 = Tile<2, 4, 4, 4, 3, 3, 2>;
 using T64 = Tile<2, 4, 2, 4, 3, 3, 2>;
 
 // An expert's last tile, of fewer rows, runs as one of 64 or 128 rows (as gemm_tn.hip): six prompts of 50 to 2000
 // tokens through two layers of 8 experts of 4096 x 14336, with the layers' other products, 4.48 / 4.44 ms
-template <typename T, bool GLU>
+// EITHER: tiles of 256 or of 192 rows, whichever end sooner with the rows that the experts have
+template <typename T, bool GLU, bool EITHER>
 __global__ void __launch_bounds__(T::NTHR, T::WAVES) tile_kernel(Args a) {
-  constexpr int BM = T::BM, HC = T::BN / 2;
+  constexpr int HC = T::BN / 2;
   const int lane = threadIdx.x & 63;
   // ---- block -> (expert, column block, row tile), row tiles fastest, consecutive ones on one XCD
   constexpr int CB = GLU ? HC : 2 * HC;
   const int tn = (a.cols + CB - 1) / CB;
+  int BM = T::BM;
+  if constexpr (EITHER) {
+    int n[8] = {};  // end_of's counts with tiles of 256 rows and of 192
+    for (int e0 = 0; e0 < a.E; e0 += 64) {
+      const int c = rows_of(a, e0 + lane);
+#pragma unroll
+      for (int f = 0; f < 2; ++f) {
+        const int bm = f ? 192 : 256, left = c % bm;
+        n[4 * f] += c / bm;
+        n[4 * f + 1] += left > 128;
+        n[4 * f + 2] += left > 64 && left <= 128;
+        n[4 * f + 3] += left > 0 && left <= 64;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) n[i] += __shfl_xor(n[i], o, 64);
+      n[i] *= tn;
+    }
+    if (end_of(192, n[4], n[5], n[6], n[7]) < kClearly * end_of(256, n[0], n[1], n[2], n[3])) BM = 192;
+    BM = __builtin_amdgcn_readfirstlane(BM);
+  }
   int total = 0;
   for (int e0 = 0; e0 < a.E; e0 += 64) {
-    int t = tiles_of<BM>(a, e0 + lane);
+    int t = tiles_of(a, e0 + lane, BM);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
     total += t;
@@ -160,7 +198,7 @@ __global__ void __launch_bounds__(T::NTHR, T::WAVES) tile_kernel(Args a) {
   {
     int before = 0;
     for (int e0 = 0; e0 < a.E; e0 += 64) {
-      const int t = tiles_of<BM>(a, e0 + lane);
+      const int t = tiles_of(a, e0 + lane, BM);
       int inc = t;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
@@ -189,14 +227,20 @@ __global__ void __launch_bounds__(T::NTHR, T::WAVES) tile_kernel(Args a) {
     clear_tile(a.y + (int64_t)r0 * a.cols + n0, a.cols, min(BM, r1 - r0), min(CB, a.cols - n0));
     return;
   }
-  static_assert(T64::LDS <= T::LDS && (BM <= 128 || T128::LDS <= T::LDS) && T64::NTHR == T::NTHR && T128::NTHR == T::NTHR);
-  if (used <= BM / 2) {
+  static_assert(T64::LDS <= T::LDS && (T::BM <= 128 || T128::LDS <= T::LDS) && T64::NTHR == T::NTHR && T128::NTHR == T::NTHR);
+  if (used <= (T::BM > 128 ? 128 : 64)) {
     const int there = min(BM, r1 - r0), small = used <= 64 ? T64::BM : T128::BM;
     if (there > small)  // rows that are not in use
       clear_tile(a.y + (int64_t)(r0 + small) * a.cols + n0, a.cols, there - small, min(CB, a.cols - n0));
-    if (used <= 64 || BM <= 128) run_tile<T64, GLU>(a, expert, r0, r1, n0, used);
+    if (used <= 64 || T::BM <= 128) run_tile<T64, GLU>(a, expert, r0, r1, n0, used);
     else run_tile<T128, GLU>(a, expert, r0, r1, n0, used);
     return;
+  }
+  if constexpr (EITHER) {
+    if (BM == 192) {
+      run_tile<T192, GLU>(a, expert, r0, r1, n0, used);
+      return;
+    }
   }
   run_tile<T, GLU>(a, expert, r0, r1, n0, used);
 }
@@ -228,20 +272,23 @@ static Args args(const at::Tensor& x, const at::Tensor& w, const at::Tensor& off
   return a;
 }
 
-template <typename T, bool GLU>
+template <typename T, bool GLU, bool EITHER>
 static void launch(const Args& a) {
   constexpr int CB = GLU ? T::BN / 2 : T::BN;
   // every expert may end in a part of a tile
-  const int64_t grid = ((int64_t)a.R / T::BM + std::min(a.E, a.R)) * ((a.cols + CB - 1) / CB);
+  const int64_t grid = ((int64_t)a.R / (EITHER ? 192 : T::BM) + std::min(a.E, a.R)) * ((a.cols + CB - 1) / CB);
   SXE_CHECK(grid < (1ll << 31), "expert tile product: too many tiles");
-  allow_lds<&tile_kernel<T, GLU>>(T::LDS);
-  hipLaunchKernelGGL((tile_kernel<T, GLU>), dim3((unsigned)grid), dim3(T::NTHR), T::LDS, cur_stream(), a);
+  allow_lds<&tile_kernel<T, GLU, EITHER>>(T::LDS);
+  hipLaunchKernelGGL((tile_kernel<T, GLU, EITHER>), dim3((unsigned)grid), dim3(T::NTHR), T::LDS, cur_stream(), a);
   SXE_LAUNCH_CHECK();
 }
 // 128 rows a tile where few column blocks make few rounds of workgroups over the CUs and theirs are the shorter ones (a round of 128 rows
 // takes 0.67 of one of 256). Products with h, us, 256 / 128: 4096 columns of 14336 k, 150 rows an expert of eight 271 / 233, 250
 // 318 / 382, 400 581 / 407, 800 661 / 768; 2048 of 8192, 250 170 / 118, 550 187 / 203. Many column blocks: 28672 of 4096 k, 50 rows
 // 379 / 364, 150 403 / 508, 800 1358 / 1481
+// 192 rows where as many for every expert would end clearly sooner in them; the kernel decides by the rows that they have (a prompt's lie near
+// the mean: 697 to 751 of eight experts). us, 128 or 256 / so: 4096 columns of 14336 k, 730 rows an expert of eight 645 / 576; 300 to 1500 rows an
+// expert, widths 2048, 3072 and 4096, evenly and unevenly filled, 1.03 of the speed on average, up to 1.2; but many column blocks, whose last round is one of many, and the workgroups that the grid has for 192: 28672 of 4096 k +1 % on average.
 template <bool GLU>
 static void launch(const Args& a) {
   const int64_t blocks = (a.cols + (GLU ? 127 : 255)) / (GLU ? 128 : 256);
@@ -249,8 +296,16 @@ static void launch(const Args& a) {
     const int64_t tiles = a.R < bm * a.E ? a.E : a.R / bm + a.E / 2;
     return (tiles * blocks + kNumCUs - 1) / kNumCUs;
   };
-  if (blocks <= 32 && 2 * rounds(128) <= 3 * rounds(256)) launch<T128, GLU>(a);
-  else launch<T256, GLU>(a);
+  auto even = [&](int bm) {  // all experts with as many rows
+    const int c = (a.R + a.E - 1) / a.E, left = c % bm, n = (int)std::min<int64_t>(a.E * blocks, 1 << 20);
+    return end_of(bm, c / bm * n, left > 128 ? n : 0, left > 64 && left <= 128 ? n : 0, left > 0 && left <= 64 ? n : 0);
+  };
+  const bool low = blocks <= 32 && 2 * rounds(128) <= 3 * rounds(256);
+  if constexpr (!GLU) {
+    if (a.offs != nullptr && blocks <= 32 && even(192) < kClearly * (low ? even(128) : even(256))) return launch<T256, GLU, true>(a);
+  }
+  if (low) launch<T128, GLU, false>(a);
+  else launch<T256, GLU, false>(a);
 }
 
 }  // namespace kt

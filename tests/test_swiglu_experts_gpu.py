@@ -74,6 +74,22 @@ def test_tile_kernels(T, E, k, K, I, N, skew):
         assert (y[r].double() - wy).norm() <= 3e-3 * wy.norm()
 
 
+@pytest.mark.parametrize("E,N,counts", [(8, 4096, [730] * 8), (8, 4096, [768, 767, 577, 640, 641, 705, 704, 769]), (8, 4096, [5840] + [0] * 7),
+                                        (8, 4096, [1, 64, 65, 128, 129, 192, 193, 5068]), (70, 1040, [300] * 69 + [299]), (70, 1040, [0, 600] * 35)])
+@pytest.mark.parametrize("K", [64, 160])
+def test_tiles_of_either_height(E, N, counts, K):
+    """Rows for which tiles of 192 may end sooner: the same sums whichever the kernel takes by the rows that the experts have."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    R = sum(counts)
+    h = torch.randn(R, K, generator=g, device="cuda").bfloat16()
+    w = (torch.randn(E, K, N, generator=g, device="cuda") * K ** -0.5).bfloat16()
+    offs = torch.tensor([0] + counts, device="cuda").cumsum(0).int()
+    y = torch.ops.sxe.expert_down_kn_tile(h, w, offs)
+    for e, (a, b) in enumerate(zip(offs.tolist(), offs.tolist()[1:])):
+        want = h[a:b].double() @ w[e].double()
+        assert (y[a:b].double() - want).norm() <= 3e-3 * want.norm()  # fp32 sums and one rounding of the result (2^-9)
+
+
 def _tile_activation(gate, up):
     """silu(gate) up of [I, 64] pairs that the products hold exactly, one term each."""
     offs, rows = torch.tensor([0, 64], device="cuda", dtype=torch.int32), torch.arange(64, device="cuda", dtype=torch.int32)
