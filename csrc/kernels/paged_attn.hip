@@ -7,7 +7,7 @@
 //  * cache layout per layer: [num_blocks, 2 (k|v), n_kv_heads, block_size, D] bf16 -- the keys of
 //    one (block, head) are one contiguous run, so a wave reading 64 consecutive keys streams
 //    64 x 256 B = 16 KB with no stride;
-//  * one workgroup (4 waves, 256 threads) per (sequence, kv head, KV split): all G = nq/nkv query
+//  * one workgroup (4 waves, 8 where a CU has only one) per (sequence, kv head, KV split): all G = nq/nkv query
 //    heads of the GQA group (x the sequence's new tokens) share every K/V byte loaded, so decode is
 //    pure HBM streaming at the GQA-reduced byte count;
 //  * both products on the matrix cores (v_mfma_f32_16x16x32_bf16), 16 query rows (token x head of
@@ -31,7 +31,6 @@
 namespace sxe {
 namespace pa {
 
-constexpr int kWaves = 4;
 constexpr float kLog2e = 1.4426950408889634f;
 
 template <int D>
@@ -152,23 +151,23 @@ constexpr int PR = 16;  // query rows per pass
 // sequences of 270 - 5300 keys (heads 32 / 8) 49 against 60 us, 32 of 3000 keys 78 against 82 us. 64 keys are the better form
 // where the workgroups make whole rounds of two a CU and a last round of three would be nearly empty (`wide`: the rule and its
 // figures are in ops/paged_attention.py).
-template <int D, int NT>
+template <int D, int NT, int W>
 struct PaGeo {
   static constexpr int KC = 16 * NT;           // keys per wave chunk
   static constexpr int KS = D / 32;            // k-steps of the Q K^T product
   static constexpr int DT = D / 16;            // 16-wide d tiles of O^T
   static constexpr int VIMG = KC * 2 * D;      // bytes of one wave's V image
-  static constexpr int MERGE = kWaves * PR * D * 4;
-  static constexpr int LDS = (kWaves * VIMG > MERGE ? kWaves * VIMG : MERGE);
+  static constexpr int MERGE = W * PR * D * 4;
+  static constexpr int LDS = (W * VIMG > MERGE ? W * VIMG : MERGE);
 };
 
-template <int D, int NT>
-__global__ __launch_bounds__(256, D == 256 ? 1 : D * NT > 256 ? 2 : 3) void paged_attn_kernel(Args a) {
-  using P = PaGeo<D, NT>;
+template <int D, int NT, int W = 4>
+__global__ __launch_bounds__(64 * W, W > 4 ? 2 : D == 256 ? 1 : D * NT > 256 ? 2 : 3) void paged_attn_kernel(Args a) {
+  using P = PaGeo<D, NT, W>;
   constexpr int KC = P::KC, KS = P::KS, DT = P::DT;
   extern __shared__ __attribute__((aligned(16))) char smem[];  // V images, then the wave-merge buffer
-  __shared__ int64_t koff_lds[kWaves][KC];
-  __shared__ float mrg_ml[kWaves][PR][2];
+  __shared__ int64_t koff_lds[W][KC];
+  __shared__ float mrg_ml[W][PR][2];
 
   const int item = blockIdx.x / a.nkv, kvh = blockIdx.x - item * a.nkv, seq = a.seqs ? a.seqs[2 * item] : item;
   const int split = blockIdx.y;
@@ -184,10 +183,10 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : D * NT > 256 ? 2 : 3) void page
   const int64_t half_stride = (int64_t)a.nkv * head_stride;  // k half -> v half
   const int64_t block_stride = 2 * half_stride;
   char* vimg = smem + wave * P::VIMG;
-  float* mrg_o = reinterpret_cast<float*>(smem);  // [kWaves][PR][D] after the key loop
+  float* mrg_o = reinterpret_cast<float*>(smem);  // [W][PR][D] after the key loop
   const int krow = kperm(i >> 2) + (i & 3);        // this lane's key row in a tile (A operand of Q K^T)
   if (a.lazy && k_begin >= kl) {  // a split behind the sequence's last key
-    for (int row = threadIdx.x; row < nrows_total; row += 256) {
+    for (int row = threadIdx.x; row < nrows_total; row += 64 * W) {
       const int tok = row / G, h = kvh * G + row - tok * G;
       const int64_t pidx = ((int64_t)split * a.T + (a.seqs ? a.seqs[2 * item + 1] : qs) + tok) * a.nq + h;
       a.part_ml[pidx * 2] = -INFINITY;
@@ -235,9 +234,9 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : D * NT > 256 ? 2 : 3) void page
       off = key - at * a.bs;
     };
     if (k_start + wave * KC < k_hi) find(k_start + wave * KC);
-    for (int kb = k_start + wave * KC; kb < k_hi; kb += kWaves * KC) {
+    for (int kb = k_start + wave * KC; kb < k_hi; kb += W * KC) {
       if (lane < KC) koff_lds[wave][lane] = (int64_t)blk * block_stride + kvh * head_stride + (int64_t)off * D;
-      if (kb + kWaves * KC < k_hi) find(kb + kWaves * KC);
+      if (kb + W * KC < k_hi) find(kb + W * KC);
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
       __builtin_amdgcn_wave_barrier();
       // ---- K fragments straight into the A operand: tile t, key row krow, d = 32 ks + 8 g ---------
@@ -341,14 +340,14 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : D * NT > 256 ? 2 : 3) void page
       }
     }
     __syncthreads();
-    for (int idx = threadIdx.x; idx < nrows * D; idx += 256) {
+    for (int idx = threadIdx.x; idx < nrows * D; idx += 64 * W) {
       const int r = idx / D, d = idx - r * D;
       float M = -INFINITY;
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) M = fmaxf(M, mrg_ml[w][r][0]);
+      for (int w = 0; w < W; ++w) M = fmaxf(M, mrg_ml[w][r][0]);
       float sum = 0.f, L = 0.f;
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) {
+      for (int w = 0; w < W; ++w) {
         const float mw = mrg_ml[w][r][0];
         const float f = (mw == -INFINITY) ? 0.f : exp2f(mw - M);
         sum += f * mrg_o[(w * PR + r) * D + d];
@@ -387,7 +386,7 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : D * NT > 256 ? 2 : 3) void page
     __threadfence();
     constexpr int U = 8;
     const int64_t sstride = (int64_t)a.T * a.nq;
-    for (int idx = threadIdx.x; idx < nrows_total * D; idx += 256) {
+    for (int idx = threadIdx.x; idx < nrows_total * D; idx += 64 * W) {
       const int r = idx / D, d = idx - r * D, tok = r / G, gh = r - tok * G;
       const int t = qs + tok, h = kvh * G + gh;
       const int64_t th = (int64_t)t * a.nq + h;
@@ -624,16 +623,23 @@ static at::Tensor paged_attention_impl(const at::Tensor& q, const at::Tensor& ca
   }
   dim3 grid(S * nkv, splits);
   SXE_CHECK(D == 128 || D == 64 || D == 256, "paged_attention: head_dim must be 64, 128 or 256");
-  auto launch = [&](auto d, auto nt) {
-    constexpr auto kern = &pa::paged_attn_kernel<decltype(d)::value, decltype(nt)::value>;
-    constexpr int lds = pa::PaGeo<decltype(d)::value, decltype(nt)::value>::LDS;
-    allow_lds<kern>(lds);  // with the static part up to 66 KB
-    hipLaunchKernelGGL(kern, grid, dim3(256), lds, cur_stream(), a);
+  auto launch = [&](auto d, auto nt, auto waves) {
+    constexpr int W = decltype(waves)::value;
+    constexpr auto kern = &pa::paged_attn_kernel<decltype(d)::value, decltype(nt)::value, W>;
+    constexpr int lds = pa::PaGeo<decltype(d)::value, decltype(nt)::value, W>::LDS;
+    allow_lds<kern>(lds);  // with the static part up to 67 KB
+    hipLaunchKernelGGL(kern, grid, dim3(64 * W), lds, cur_stream(), a);
   };
-  if (D == 128 && wide) launch(std::integral_constant<int, 128>{}, std::integral_constant<int, 4>{});
-  else if (D == 128) launch(std::integral_constant<int, 128>{}, std::integral_constant<int, 2>{});
-  else if (D == 256) launch(std::integral_constant<int, 256>{}, std::integral_constant<int, 2>{});
-  else launch(std::integral_constant<int, 64>{}, std::integral_constant<int, 4>{});
+  constexpr std::integral_constant<int, 2> n2{};
+  constexpr std::integral_constant<int, 4> n4{};
+  if (D == 128 && wide) launch(std::integral_constant<int, 128>{}, n4, n4);
+  // At most one workgroup a CU: eight waves walk a split's keys in half the rounds, each of 2 to 3 us from the table to the last product. A
+  // step of three layers, four / eight waves, us: hidden 2048, 1 sequence of 1000 keys (splits of 256) 174.4 / 171.0, 8 of 1000 189.5 / 184.0;
+  // 4096, 1 of 7000 378.9 / 374.4, 24 of 120 426.2 / 423.7. A split of up to 128 keys is one round of four waves.
+  else if (D == 128 && kps > 128 && (int64_t)S * nkv * splits <= 256) launch(std::integral_constant<int, 128>{}, n2, std::integral_constant<int, 8>{});
+  else if (D == 128) launch(std::integral_constant<int, 128>{}, n2, n4);
+  else if (D == 256) launch(std::integral_constant<int, 256>{}, n2, n4);
+  else launch(std::integral_constant<int, 64>{}, n4, n4);
   SXE_LAUNCH_CHECK();
   if (splits > 1 && parts != nullptr) {
     *parts = {part_o, part_ml};

@@ -82,7 +82,7 @@ def paged_attention_reference(q, cache, block_table, q_start, q_len, kv_len, sca
     return out
 
 
-# keys per split floor (see choose_splits): 256 = four 64-key wave chunks per split. Llama-3-8B decode,
+# keys per split floor (see choose_splits and _short_splits): 256 = four 64-key wave chunks per split. Llama-3-8B decode,
 # HIP graphs, fused merge: batch 1 ctx 1024 3.571 / 3.604 / 3.700 ms per token at 256 / 128 / 64,
 # ctx 4096 3.745 / 3.927 / 3.926; batch 8 and 32 within 1 % (profiles/r06/decode_split_floor_ab.log)
 PA_MIN_KEYS = int(os.environ.get("SXE_PA_MIN_KEYS", 256))
@@ -157,11 +157,30 @@ def choose_balanced_splits(num_seqs, nkv, max_kv_len, split_bytes, even=False, h
     return max(more, key=full)
 
 
+# Keys up to which few decoding sequences with heads of 128 have splits of half of PA_MIN_KEYS, as long as these are at most one workgroup a CU:
+# its four waves take 128 keys at a time. The same splits of 256 keys have the kernel's form of eight waves. A step of three layers, us, 256
+# keys in two rounds of four waves / in one of eight / splits of 128: hidden 2048, 1 sequence of 500 keys 175.0 / 172.1 / 168.0, 4 of 1000
+# 187.6 / 182.8 / 180.0; 3072, 2 of 1500 246.0 / 242.1 / 239.8; 4096, 1 of 1000 357.2 / 353.3 / 348.8; but with two workgroups a CU, hidden
+# 2048, 8 of 1500 191.9 / 189.3 / 191.7. 3000 keys, one sequence of hidden 2048 180.1 / 176.7 / 181.7, 4096 364.5 / 360.2 / 370.8.
+# Where two splits need the merge's launch and one does not (up to 256 keys), 120 keys cost 2 % more and 250 3 % less: as it was.
+PA_SHORT_KEYS = 2048
+PA_SHORT_WGS = 256
+
+
+def _short_splits(splits, num_seqs, nkv, max_kv_len, split_bytes, head_dim, merged=False):
+    """``merged``: the splits are read by the next product, with no launch for their merge."""
+    if head_dim != 128 or not (1 if merged else PA_MIN_KEYS) < max_kv_len <= PA_SHORT_KEYS:
+        return splits
+    want = min(PA_SHORT_WGS // max(1, num_seqs * nkv), math.ceil(max_kv_len / max(1, PA_MIN_KEYS // 2)))
+    return max(splits, min(want, PA_SPLIT_BYTES // max(1, split_bytes)))
+
+
 @functools.lru_cache(maxsize=4096)
 def _decode_plan(num_seqs, nkv, max_kv_len, split_bytes, even, head_dim, tuned):
     """(splits, two workgroups a CU) of a launch: all layers of a step ask for the same, a microsecond of the host each. ``tuned``: the
     settings that the choice reads."""
-    splits = choose_balanced_splits(num_seqs, nkv, max_kv_len, split_bytes, even, head_dim)
+    splits = _short_splits(choose_balanced_splits(num_seqs, nkv, max_kv_len, split_bytes, even, head_dim), num_seqs, nkv, max_kv_len,
+                           split_bytes, head_dim)
     return splits, splits == 1 and two_a_cu(num_seqs * nkv, head_dim)
 
 
@@ -171,7 +190,8 @@ def paged_attention_parts(q, cache, block_table, q_start, q_len, kv_len, scale, 
     partials [splits, T, nq, D] / [splits, T, nq, 2] for a consumer that merges them in its own
     prologue (``ops.linear.fused_merge_linear``: the o_proj skinny GEMM)."""
     if splits is None:
-        splits = choose_splits(block_table.shape[0], cache.shape[2], max_kv_len)
+        splits = _short_splits(choose_splits(block_table.shape[0], cache.shape[2], max_kv_len), block_table.shape[0], cache.shape[2],
+                               int(max_kv_len), 4 * q.numel(), q.shape[-1], True)
     out, po, pml = torch.ops.sxe.paged_attention_parts(q, cache, block_table, q_start, q_len, kv_len, float(scale),
                                                        int(max_kv_len), int(splits), 0)
     return (out, None) if po.numel() == 0 else (None, (po, pml))

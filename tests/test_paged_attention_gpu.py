@@ -156,3 +156,19 @@ def test_in_kernel_split_merge_matches_merge_launch(splits, monkeypatch):
         torch.cuda.synchronize()
         torch.testing.assert_close(out.float(), sep.float(), atol=1e-2, rtol=1e-2)
     assert int(PA._COUNTERS[q.device].abs().sum()) == 0
+
+
+@pytest.mark.parametrize("seqs,splits", [([(0, 129)], 1), ([(128, 1), (300, 1), (0, 1)], 1), ([(255, 1), (256, 1), (257, 2)], 2),
+                                         ([(1023, 1), (100, 1)], 4), ([(4000, 9), (2000, 40), (511, 1)], 7)])
+@pytest.mark.parametrize("nq,nkv,bs,window", [(32, 8, 64, 0), (7, 1, 48, 0), (8, 4, 16, 200)])
+def test_few_workgroups_of_eight_waves(seqs, splits, nq, nkv, bs, window):
+    """At most one workgroup a CU and more than 128 keys a split: the last round reaches any of the eight waves. Rounding of the
+    weights and of the result to bf16, 2^-9 each."""
+    from shuffle_exchange_amd.ops.paged_attention import kv_cache_append, paged_attention, paged_attention_reference
+    qkv, cache, bt, qs, ql, kl, slots, maxkv = _setup(seqs, nq, nkv, 128, bs, seed=5)
+    kv_cache_append(qkv, cache, slots, nq, nkv)
+    q, scale = qkv[:, :nq], 128 ** -0.5
+    assert len(seqs) * nkv * splits <= 256 and maxkv > 128 * splits
+    out = paged_attention(q, cache, bt, qs, ql, kl, scale, maxkv, splits, window=window or None)
+    ref = paged_attention_reference(q.float(), cache.float(), bt, qs, ql, kl, scale, window or None)
+    assert (out.float() - ref).norm() < 1.01 * 2 ** -8 * ref.norm()

@@ -269,3 +269,13 @@ def test_wide_chunks_match_reference(seqs, nkv, group, window):
     for y in got:  # bf16 weights and result: two roundings of 2^-9 on values that are averages of unit normals
         assert not y.isnan().any() and (y.float() - want.float()).norm() <= 2 ** -7 * want.float().norm()
     assert torch.equal(PA.paged_attention(q, cache, *meta, D ** -0.5, most, window=window, splits=1), got[0])
+
+
+def test_short_splits_of_few_workgroups():
+    """Splits of 128 keys are at most a workgroup a CU and stay within what partials may take; all else is as it was."""
+    assert PA._decode_plan(1, 8, 1024, 1 << 14, False, 128, None) == (8, False) == PA._decode_plan(1, 8, 1024, 1 << 14, True, 128, None)
+    for S in (1, 3, 8, 24, 33):
+        for keys in (100, 256, 257, 1000, 2048, 2049, 8192):
+            for nkv, dim, room in ((1, 128, 1 << 10), (8, 128, 1 << 14), (8, 128, 1 << 27), (8, 64, 1 << 14), (8, 256, 1 << 14)):
+                was, n = PA.choose_balanced_splits(S, nkv, keys, room, True, dim), PA._decode_plan(S, nkv, keys, room, True, dim, None)[0]
+                assert n == was or (dim == 128 and 256 < keys <= 2048 and was < n <= -(-keys // 128) and S * nkv * n <= 256 and n * room <= PA.PA_SPLIT_BYTES)
