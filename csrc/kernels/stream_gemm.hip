@@ -209,7 +209,7 @@ __device__ __forceinline__ void merge_row(const Args& a, unsigned short* row) {
 // HALF (up to 8 rows): a tile of 8 columns, each twice. The matrix core's rows 0 - 7 have one half of a piece's K, rows 8 - 15 the other one,
 // of W and of x alike, and the two blocks of the result that belong together are added: no lane loads what another one does, and there are
 // twice the workgroups, each with half the pieces one behind the other.
-template <bool FP8, int MB, int NT, int EPI, bool ONCE, bool HALF = false, bool MERGE = false>
+template <bool FP8, int MB, int NT, int EPI, bool ONCE, bool HALF = false, bool MERGE = false, int DEEP = 1>
 __global__ void __launch_bounds__(64 * NW, 2) stream_gemm_kernel(Args a) {
   static_assert(!HALF || (MB == 1 && NT == 1), "");
   static_assert(!MERGE || (EPI == EPI_RES && HALF), "");
@@ -247,10 +247,15 @@ __global__ void __launch_bounds__(64 * NW, 2) stream_gemm_kernel(Args a) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // (the next piece in flight behind this one's products halves the workgroups on a CU and gains nothing)
+  // DEEP 2: the next piece is in flight behind this one's products. It halves the workgroups on a CU: only where a launch has few
   using P = Piece<FP8, MB, NT, ONCE>;
   constexpr int STEP = HALF ? 2 * P::PIECE : P::PIECE;
   int k0 = wave * STEP + (HALF ? (l16 >> 3) * P::PIECE : 0);
+  P p[DEEP];
+  auto load = [&](P& q, int ahead) {  // the piece `ahead` of the one that is next
+    q.load_w(wr, ldw, k0 + ahead * NW * STEP, a.K, c);
+    if constexpr (!MERGE) q.load_x(xr, k0 + ahead * NW * STEP, a.K, c);
+  };
   // what the epilogue reads is on its way beside the first piece
   u16x4 res[MB], gw;
   f32x4 cs[MB], sn[MB];
@@ -279,9 +284,7 @@ __global__ void __launch_bounds__(64 * NW, 2) stream_gemm_kernel(Args a) {
         if (64 * NW * i + (int)threadIdx.x < pieces) sq[i] = reinterpret_cast<const f32x4*>(a.part)[64 * NW * i + threadIdx.x];
       }
     }
-    P p;
-    p.load_w(wr, ldw, k0, a.K, c);
-    if constexpr (!MERGE) p.load_x(xr, k0, a.K, c);
+    load(p[0], 0);
     if (EPI == EPI_RES && wave < OT) {
       const int n = min(column(wave, fq), a.N - 4);
       gw = *reinterpret_cast<const u16x4*>(a.gw + n);
@@ -309,17 +312,29 @@ __global__ void __launch_bounds__(64 * NW, 2) stream_gemm_kernel(Args a) {
     if constexpr (MERGE) {
       merge_row(a, merged);
       __syncthreads();
-      p.row_x(merged, k0, a.K, g);
     }
-    p.template multiply<MERGE>(acc, odd1, odd2);
-    k0 += NW * STEP;
   }
-  for (; k0 - (HALF ? (l16 >> 3) * P::PIECE : 0) < a.K; k0 += NW * STEP) {
-    P p;
-    p.load_w(wr, ldw, k0, a.K, c);
-    if constexpr (MERGE) p.row_x(merged, k0, a.K, g);
-    else p.load_x(xr, k0, a.K, c);
-    p.template multiply<MERGE>(acc, odd1, odd2);
+  auto multiply = [&](P& q) {
+    if constexpr (MERGE) q.row_x(merged, k0, a.K, g);
+    q.template multiply<MERGE>(acc, odd1, odd2);
+    k0 += NW * STEP;
+  };
+  if constexpr (DEEP == 1) {
+    if constexpr (EPI >= EPI_RES) multiply(p[0]);
+    while (k0 - (HALF ? (l16 >> 3) * P::PIECE : 0) < a.K) {
+      load(p[0], 0);
+      multiply(p[0]);
+    }
+  } else {
+    static_assert(DEEP == 2, "");
+    if constexpr (EPI < EPI_RES) load(p[0], 0);
+    for (int ku = wave * STEP; ku < a.K; ku += 2 * NW * STEP) {
+      load(p[1], 1);
+      multiply(p[0]);
+      if (ku + NW * STEP >= a.K) break;
+      load(p[0], 1);
+      multiply(p[1]);
+    }
   }
   // lane: columns 4 g .. + 3 of row l16 of every tile
   auto finish = [&](int m, int t) {
@@ -508,6 +523,14 @@ int plain_tiles(const st::Args& a, bool fp8) { return (a.N + 15) / 16 >= 384 && 
 // the head 189 / 180 us bf16, 148 / 142 e4m3; but 2560 columns (160 tiles) 230 / 236 and 180 / 187, 4096 (256) 367 / 380 and 266 / 284
 bool halves(const st::Args& a) { return a.M <= 8 && a.N <= 2048; }
 
+// A piece in flight behind the products of the one before, where a CU has one or two workgroups and a wave three or more pieces: bf16, us, so
+// off / on: 4096 x 4096 1 row 10.6 / 9.4, 8 rows 10.5 / 9.5, 3072 x 8192 14.8 / 13.9, 4096 x 14336 23.4 / 22.5, 8192 x 4096 14.6 / 14.0, QKV of
+// 6144 x 4096 14.9 / 14.5; but two pieces, 3072 x 2048 6.6 / 7.0; 16 rows and more, whose pieces are larger, 4096 x 14336 24.4 / 24.6, 5120 x
+// 3072 15.4 / 17.8, and e4m3 4096 x 14336 16.2 / 16.9. Three pieces in flight are slower than two everywhere.
+bool deep(const st::Args& a, bool fp8, int64_t workgroups) {
+  return !fp8 && a.M <= 8 && workgroups <= 512 && a.K > 2 * st::NW * 128 * (halves(a) ? 2 : 1);
+}
+
 template <int EPI>
 void launch(const st::Args& a, bool fp8, int nt) {
   if constexpr (EPI != st::EPI_GLU && EPI != st::EPI_NGLU) {
@@ -516,7 +539,8 @@ void launch(const st::Args& a, bool fp8, int nt) {
       auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(64 * st::NW), 0, cur_stream(), a); };
       by_rows(a, fp8, [&](auto, auto nontemporal) {
         constexpr bool ONCE = decltype(nontemporal)::value;
-        fp8 ? go(st::stream_gemm_kernel<true, 1, 1, EPI, ONCE, true>) : go(st::stream_gemm_kernel<false, 1, 1, EPI, ONCE, true>);
+        if (deep(a, fp8, grid.x)) go(st::stream_gemm_kernel<false, 1, 1, EPI, ONCE, true, false, 2>);
+        else fp8 ? go(st::stream_gemm_kernel<true, 1, 1, EPI, ONCE, true>) : go(st::stream_gemm_kernel<false, 1, 1, EPI, ONCE, true>);
       });
       return;
     }
@@ -531,6 +555,8 @@ void launch(const st::Args& a, bool fp8, int nt) {
       // a tile of gate and one of up; two of each leave a workgroup a CU, steps of three layers, us, two / one: 4096, 14336 1 row 358 / 340, 8
       // rows 372 / 355, 16 397 / 379, 32 467 / 455; 4096, 11008 32 rows 544 / 509; 3072, 8192 235 / 234, 300 / 297; 2048, 8192 180 / 177, 218 / 216
       fp8 ? go(st::stream_gemm_kernel<true, MB, 2, EPI, ONCE>) : go(st::stream_gemm_kernel<false, MB, 2, EPI, ONCE>);
+    } else if (MB == 1 && deep(a, fp8, grid.x)) {
+      nt == 2 ? go(st::stream_gemm_kernel<false, 1, 2, EPI, ONCE, false, false, 2>) : go(st::stream_gemm_kernel<false, 1, 1, EPI, ONCE, false, false, 2>);
     } else if (fp8) {
       nt == 2 ? go(st::stream_gemm_kernel<true, MB, 2, EPI, ONCE>) : go(st::stream_gemm_kernel<true, MB, 1, EPI, ONCE>);
     } else {

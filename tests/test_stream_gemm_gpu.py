@@ -38,6 +38,20 @@ def test_plain(M, N, K, fp8):
         assert (got.double() - want).norm() < 1.01 * 2 ** -8 * want.norm()
 
 
+@pytest.mark.parametrize("M", [1, 7, 8])
+@pytest.mark.parametrize("N", [80, 4112])  # half tiles and whole ones (multiples of 16: what stream_gemm_res takes)
+@pytest.mark.parametrize("K", [2048, 2056, 3072, 3080, 4096, 4104, 5000, 6152, 8200])
+def test_pieces_in_flight(M, N, K):
+    """Two at a time where a wave has three or more: any of the waves may have one more or one less than the others."""
+    x, w, _, ref = _operands(M, N, K, False, M + N + K)
+    want = x.double() @ ref.T
+    assert (torch.ops.sxe.stream_gemm(x, w, None, None, False).double() - want).norm() < 1.01 * 2 ** -8 * want.norm()
+    assert (torch.ops.sxe.stream_gemm_normed(x, w, None, None, 0.0, False).double() - want).norm() < 1e-5 * want.norm()
+    res, gw = torch.randn(M, N, device="cuda").bfloat16(), torch.ones(N, device="cuda").bfloat16()
+    want = want + res.double()
+    assert (torch.ops.sxe.stream_gemm_res(x, w, None, None, res, gw)[1].double() - want).norm() < 1.01 * 2 ** -8 * want.norm()
+
+
 def test_every_e4m3_value_is_exact():
     w = torch.arange(256, device="cuda", dtype=torch.uint8).view(16, 16)
     one = torch.ones(16, device="cuda")
