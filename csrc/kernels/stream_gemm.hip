@@ -97,27 +97,31 @@ __device__ __forceinline__ void exchange(u32x4 (&r)[4], bool odd1, bool odd2) {
 
 // A wave's operands of one piece of K: 256 bytes of every row of W (128 columns of bf16, 256 of e4m3) and the same columns of x.
 // After the exchange lane (row, g) holds chunk 4 g + c of 16 bytes of its row in register c.
-template <bool FP8, int MB, int NT, bool ONCE>
+// X8 (up to 8 rows): 256 columns, of which the matrix core's columns 0 - 7 have the one half of x and 8 - 15 the other one. A half of W goes to
+// sums of its own with the same registers of x, eight columns of which count: half the loads of x and half of its exchange.
+template <bool FP8, int MB, int NT, bool ONCE, bool X8 = false>
 struct Piece {
-  static constexpr int PIECE = FP8 ? 256 : 128, XL = FP8 ? 2 : 1;
-  u32x4 w[NT][4], x[MB][XL][4];
+  static constexpr int PIECE = FP8 || X8 ? 256 : 128, XL = FP8 && !X8 ? 2 : 1, WL = X8 && !FP8 ? 2 : 1;
+  u32x4 w[NT * WL][4], x[MB][XL][4];
   // wr, xr: the rows 4 (row / 4) + u of this lane's quad, at chunk 4 g + j
   __device__ __forceinline__ void load_w(const char* const (&wr)[NT], int64_t ldw, int k0, int K, int c) {
-    const int kw = k0 + c * (FP8 ? 16 : 8);  // K is a multiple of 8 (16), so a lane's vector is in or out
-    const bool win = kw < K;
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+    for (int t = 0; t < NT * WL; ++t) {
+      const int kw = k0 + 128 * (t % WL) + c * (FP8 ? 16 : 8);  // K is a multiple of 8 (16), so a lane's vector is in or out
+      const bool win = kw < K;
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         w[t][u] = u32x4{0u, 0u, 0u, 0u};
-        const auto* p = reinterpret_cast<const u32x4*>(wr[t] + u * ldw + (int64_t)kw * (FP8 ? 1 : 2));
+        const auto* p = reinterpret_cast<const u32x4*>(wr[t / WL] + u * ldw + (int64_t)kw * (FP8 ? 1 : 2));
         if (win) w[t][u] = ONCE ? __builtin_nontemporal_load(p) : *p;
       }
+    }
   }
   __device__ __forceinline__ void load_x(const unsigned short* const (&xr)[MB][4], int k0, int K, int c) {
 #pragma unroll
     for (int h = 0; h < XL; ++h) {
-      const int kx = k0 + 8 * (FP8 ? 8 * (c >> 2) + 4 * h + (c & 3) : c);
+      const int hx = X8 ? (threadIdx.x >> 3) & 1 : h;
+      const int kx = k0 + 8 * (FP8 ? 8 * (c >> 2) + 4 * hx + (c & 3) : X8 ? 16 * hx + c : c);
       const bool xin = kx < K;
 #pragma unroll
       for (int m = 0; m < MB; ++m)
@@ -140,7 +144,7 @@ struct Piece {
       }
   }
   template <bool ROW = false>
-  __device__ __forceinline__ void multiply(f32x4 (&acc)[MB][NT], bool odd1, bool odd2) {
+  __device__ __forceinline__ void multiply(f32x4 (&acc)[MB][NT * (X8 ? 2 : 1)], bool odd1, bool odd2) {
     if constexpr (!ROW) {
 #pragma unroll
       for (int m = 0; m < MB; ++m)
@@ -148,15 +152,16 @@ struct Piece {
         for (int h = 0; h < XL; ++h) exchange(x[m][h], odd1, odd2);
     }
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
+    for (int t = 0; t < NT * WL; ++t) {
       exchange(w[t], odd1, odd2);
 #pragma unroll
-      for (int f = 0; f < 4 * XL; ++f) {
+      for (int f = 0; f < (FP8 ? 8 : 4); ++f) {
         u32x4 a;
         if constexpr (FP8) a = widen(w[t][f >> 1][2 * (f & 1)], w[t][f >> 1][2 * (f & 1) + 1]);
         else a = w[t][f];
+        const int at = !X8 ? t : FP8 ? 2 * t + (f >> 2) : t;
 #pragma unroll
-        for (int m = 0; m < MB; ++m) acc[m][t] = mfma16(a, x[m][f >> 2][f & 3], acc[m][t]);
+        for (int m = 0; m < MB; ++m) acc[m][at] = mfma16(a, x[m][X8 ? 0 : f >> 2][f & 3], acc[m][at]);
       }
     }
   }
@@ -209,10 +214,11 @@ __device__ __forceinline__ void merge_row(const Args& a, unsigned short* row) {
 // HALF (up to 8 rows): a tile of 8 columns, each twice. The matrix core's rows 0 - 7 have one half of a piece's K, rows 8 - 15 the other one,
 // of W and of x alike, and the two blocks of the result that belong together are added: no lane loads what another one does, and there are
 // twice the workgroups, each with half the pieces one behind the other.
-template <bool FP8, int MB, int NT, int EPI, bool ONCE, bool HALF = false, bool MERGE = false, int DEEP = 1>
+template <bool FP8, int MB, int NT, int EPI, bool ONCE, bool HALF = false, bool MERGE = false, int DEEP = 1, bool X8 = false>
 __global__ void __launch_bounds__(64 * NW, 2) stream_gemm_kernel(Args a) {
   static_assert(!HALF || (MB == 1 && NT == 1), "");
   static_assert(!MERGE || (EPI == EPI_RES && HALF), "");
+  static_assert(!X8 || (MB == 1 && !HALF), "");
   constexpr bool GLU = EPI == EPI_GLU || EPI == EPI_NGLU, NORMED = EPI >= EPI_ROPE;
   constexpr int OT = GLU ? NT / 2 : NT;  // tiles of output columns
   constexpr int TC = HALF ? 8 : 16, PAIRS = TC * NT / 2;
@@ -239,16 +245,17 @@ __global__ void __launch_bounds__(64 * NW, 2) stream_gemm_kernel(Args a) {
 #pragma unroll
   for (int m = 0; m < MB; ++m)
 #pragma unroll
-    for (int u = 0; u < 4; ++u) xr[m][u] = a.x + (int64_t)min(16 * m + quad0 + u, a.M - 1) * a.ldx;
+    for (int u = 0; u < 4; ++u) xr[m][u] = a.x + (int64_t)min(16 * m + (X8 ? quad0 & 4 : quad0) + u, a.M - 1) * a.ldx;
   const bool odd1 = j & 1, odd2 = j & 2;
-  f32x4 acc[MB][NT];
+  constexpr int AL = X8 ? 2 : 1;
+  f32x4 acc[MB][NT * AL];
 #pragma unroll
   for (int m = 0; m < MB; ++m)
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < NT * AL; ++t) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // DEEP 2: the next piece is in flight behind this one's products. It halves the workgroups on a CU: only where a launch has few
-  using P = Piece<FP8, MB, NT, ONCE>;
+  using P = Piece<FP8, MB, NT, ONCE, X8>;
   constexpr int STEP = HALF ? 2 * P::PIECE : P::PIECE;
   int k0 = wave * STEP + (HALF ? (l16 >> 3) * P::PIECE : 0);
   P p[DEEP];
@@ -443,7 +450,13 @@ __global__ void __launch_bounds__(64 * NW, 2) stream_gemm_kernel(Args a) {
     if (16 * m >= a.M) break;
     if (m) __syncthreads();
 #pragma unroll
-    for (int t = 0; t < NT; ++t) red[wave][t][lane] = acc[m][t];
+    for (int t = 0; t < NT; ++t) {
+      if constexpr (X8) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[m][2 * t][q] += __shfl_xor(acc[m][2 * t + 1][q], 8, 64);
+      }
+      red[wave][t][lane] = acc[m][AL * t];
+    }
     __syncthreads();
     if (wave < OT) finish(m, wave);
   }
@@ -523,12 +536,20 @@ int plain_tiles(const st::Args& a, bool fp8) { return (a.N + 15) / 16 >= 384 && 
 // the head 189 / 180 us bf16, 148 / 142 e4m3; but 2560 columns (160 tiles) 230 / 236 and 180 / 187, 4096 (256) 367 / 380 and 266 / 284
 bool halves(const st::Args& a) { return a.M <= 8 && a.N <= 2048; }
 
-// A piece in flight behind the products of the one before, where a CU has one or two workgroups and a wave three or more pieces: bf16, us, so
-// off / on: 4096 x 4096 1 row 10.6 / 9.4, 8 rows 10.5 / 9.5, 3072 x 8192 14.8 / 13.9, 4096 x 14336 23.4 / 22.5, 8192 x 4096 14.6 / 14.0, QKV of
-// 6144 x 4096 14.9 / 14.5; but two pieces, 3072 x 2048 6.6 / 7.0; 16 rows and more, whose pieces are larger, 4096 x 14336 24.4 / 24.6, 5120 x
+// A piece in flight behind the products of the one before, where a CU has one workgroup (more: `x8`) and a wave three or more pieces: bf16, us,
+// so off / on: 4096 x 4096 1 row 10.6 / 9.4, 8 rows 10.5 / 9.5, 3072 x 8192 14.8 / 13.9, 4096 x 14336 23.4 / 22.5; but two pieces, 3072 x 2048
+// 6.6 / 7.0; 16 rows and more, whose pieces are larger, 4096 x 14336 24.4 / 24.6, 5120 x
 // 3072 15.4 / 17.8, and e4m3 4096 x 14336 16.2 / 16.9. Three pieces in flight are slower than two everywhere.
 bool deep(const st::Args& a, bool fp8, int64_t workgroups) {
-  return !fp8 && a.M <= 8 && workgroups <= 512 && a.K > 2 * st::NW * 128 * (halves(a) ? 2 : 1);
+  return !fp8 && a.M <= 8 && workgroups <= 256 && a.K > 2 * st::NW * 128 * (halves(a) ? 2 : 1);
+}
+
+// The two halves of x side by side (see Piece) in whole tiles of up to 8 rows. e4m3, 8 rows, us, so off / on: 4096 x 14336 17.5 / 15.4, 3072 x 8192
+// 10.7 / 9.7, 4096 x 4096 8.0 / 7.6, QKV of 6144 x 4096 10.4 / 9.9, gate and up of 28672 x 4096 27.5 / 26.3, 1 row 26.9 / 25.9. bf16 has twice the bytes
+// in a piece then, which takes turns with the other form: 8 rows, 1 or 2 pieces in flight as `deep` has it / so, 6144 x 4096 14.7 / 13.8, 8192 x
+// 4096 14.2 / 13.7, 3072 x 2048 6.8 / 6.5, but 4096 x 4096 9.4 / 10.0, 3072 x 8192 13.9 / 14.9, gate and up of 28672 x 4096 41.7 / 43.7
+bool x8(const st::Args& a, bool fp8, int64_t workgroups) {
+  return a.M <= 8 && (fp8 || (workgroups <= 512 && (workgroups > 256 || a.K <= 2 * st::NW * 128)));
 }
 
 template <int EPI>
@@ -554,9 +575,13 @@ void launch(const st::Args& a, bool fp8, int nt) {
     if constexpr (GLU) {
       // a tile of gate and one of up; two of each leave a workgroup a CU, steps of three layers, us, two / one: 4096, 14336 1 row 358 / 340, 8
       // rows 372 / 355, 16 397 / 379, 32 467 / 455; 4096, 11008 32 rows 544 / 509; 3072, 8192 235 / 234, 300 / 297; 2048, 8192 180 / 177, 218 / 216
-      fp8 ? go(st::stream_gemm_kernel<true, MB, 2, EPI, ONCE>) : go(st::stream_gemm_kernel<false, MB, 2, EPI, ONCE>);
+      if (MB == 1 && fp8 && x8(a, fp8, grid.x)) go(st::stream_gemm_kernel<true, 1, 2, EPI, ONCE, false, false, 1, true>);
+      else fp8 ? go(st::stream_gemm_kernel<true, MB, 2, EPI, ONCE>) : go(st::stream_gemm_kernel<false, MB, 2, EPI, ONCE>);
+    } else if (MB == 1 && x8(a, fp8, grid.x)) {
+      if (fp8) nt == 2 ? go(st::stream_gemm_kernel<true, 1, 2, EPI, ONCE, false, false, 1, true>) : go(st::stream_gemm_kernel<true, 1, 1, EPI, ONCE, false, false, 1, true>);
+      else go(st::stream_gemm_kernel<false, 1, 1, EPI, ONCE, false, false, 1, true>);
     } else if (MB == 1 && deep(a, fp8, grid.x)) {
-      nt == 2 ? go(st::stream_gemm_kernel<false, 1, 2, EPI, ONCE, false, false, 2>) : go(st::stream_gemm_kernel<false, 1, 1, EPI, ONCE, false, false, 2>);
+      go(st::stream_gemm_kernel<false, 1, 1, EPI, ONCE, false, false, 2>);
     } else if (fp8) {
       nt == 2 ? go(st::stream_gemm_kernel<true, MB, 2, EPI, ONCE>) : go(st::stream_gemm_kernel<true, MB, 1, EPI, ONCE>);
     } else {

@@ -161,13 +161,9 @@ def chain_faster(rows, weights):
     5120 on) and the head, launches of their own (up to 4 rows the norms in prologues of skinny_gemm.hip) / so, 1, 8, 16 and 32 rows: hidden 2048,
     ff 8192 184 / 168, 202 / 177, 208 / 188, 249 / 216; 3072, 8192 247 / 229, 265 / 234, 280 / 249, 324 / 297; 3584, 18944 386 / 345, 456 / 352,
     472 / 374, 729 / 458; 4096, 11008 350 / 332, 374 / 341, 409 / 377, 540 / 509; 4096, 14336 362 / 340, 382 / 355, 402 / 379, 470 / 455; 6144,
-    16384, 16 and 32 rows 619 / 604, 688 / 659; 8192, 28672, 4 rows 868 / 756; e4m3 4096, 14336 248 / 254, 297 / 268, 339 / 301; 3072, 8192 179 / 180,
-    219 / 188, 245 / 212; 2048, 8192 138 / 128, 172 / 143; 5120, 13824, 1 and 8 rows 263 / 226, 275 / 254. So one row of e4m3 keeps the prologues where they cost it
-    least, and from 17 rows on not 5120, 13824 with 40 kv heads (8 rows 382 / 347, 32 rows 483 / 513), whose last round of the
-    gate's workgroups is short."""
-    w, scale = weights[0]
-    if rows == 1 and scale is not None:
-        return w.shape[1] <= 2048 or w.shape[1] > 4096
+    16384, 16 and 32 rows 619 / 604, 688 / 659; 8192, 28672, 4 rows 868 / 756; e4m3 4096, 14336 265 / 252, 297 / 257, 339 / 301; 3072, 8192 187 / 178,
+    219 / 183, 245 / 212; 2048, 8192 138 / 128, 172 / 143; 5120, 13824, 1 and 8 rows 263 / 226, 275 / 254. From 17 rows on not 5120, 13824 with 40 kv
+    heads (8 rows 382 / 347, 32 rows 483 / 513), whose last round of the gate's workgroups is short."""
     if rows <= STREAM_ROWS or len(weights) == 1:
         return True
     N, K = weights[2][0].shape

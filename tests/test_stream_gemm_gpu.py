@@ -39,10 +39,10 @@ def test_plain(M, N, K, fp8):
 
 
 @pytest.mark.parametrize("M", [1, 7, 8])
-@pytest.mark.parametrize("N", [80, 4112])  # half tiles and whole ones (multiples of 16: what stream_gemm_res takes)
+@pytest.mark.parametrize("N", [80, 4096, 4112, 8208])  # half tiles, then whole ones: at most one workgroup a CU, two, more
 @pytest.mark.parametrize("K", [2048, 2056, 3072, 3080, 4096, 4104, 5000, 6152, 8200])
 def test_pieces_in_flight(M, N, K):
-    """Two at a time where a wave has three or more: any of the waves may have one more or one less than the others."""
+    """Two at a time, or pieces of twice the size: any of the waves may have one more or one less than the others."""
     x, w, _, ref = _operands(M, N, K, False, M + N + K)
     want = x.double() @ ref.T
     assert (torch.ops.sxe.stream_gemm(x, w, None, None, False).double() - want).norm() < 1.01 * 2 ** -8 * want.norm()
