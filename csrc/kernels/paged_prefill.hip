@@ -1,5 +1,5 @@
 // Attention of many new tokens of a sequence over its paged KV cache (gfx950): prompts, chunks of prompts behind
-// earlier tokens, any mixture of them in one launch. Decode-sized sequences run paged_attn.hip.
+// earlier tokens, any mixture of them in one launch. Decodes beside them share the launch, alone they run paged_attn.hip.
 //
 // Reference: inference/v2/kernels/ragged_ops/blocked_flash (an external flash-attn build over the blocked cache) with
 // its atom builder, inference/v2/kernels/ragged_ops/atom_builder.
@@ -17,7 +17,7 @@
 // The longest prompts run the training forward instead, 1.0 - 1.05 PFLOP/s where this reaches 0.9 - 0.95: the rule and its figures
 // are in ops/paged_attention.py.
 // Llama-8B heads (32 / 8, D 128), MI355X, a layer: a 3500-token prompt in chunks of 1024 beside 16 decodes took 2170 us a
-// chunk in the 16-row decode kernel (one read of the keys for every 4 tokens), 50 us here and 30 us for the decodes; 12
+// chunk in the 16-row decode kernel (one read of the keys for every 4 tokens), 92 us with the decodes in a launch of that and the merges of both, 78 us in one launch here; 12
 // fresh prompts of 20 - 3000 tokens took 630 us in one flash-attention launch a prompt with its padding copies, 172 us here.
 #include "sxe_common.h"
 #include "sxe_tile.h"

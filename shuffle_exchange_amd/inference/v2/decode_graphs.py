@@ -1,9 +1,9 @@
 """HIP-graph replay of decode steps for the ragged engine.
 
 A decode step of a dense model (every sequence adds ONE token) is launch-bound at serving batch
-sizes: Llama-3-8B issues ~10 kernels per layer (norm, QKV GEMM, RoPE, KV append, paged attention
-(+ split merge), O GEMM, norm, gate/up GEMM, SwiGLU, down GEMM), i.e. ~330 launches per token,
-while the HBM time of the step is ~2 ms. The reference captures CUDA graphs only in its v1 engine
+sizes: Llama-3-8B issues 6 kernels per layer up to 32 sequences (four products with norms, RoPE, KV append,
+residual sums and SwiGLU inside, paged attention, split merge) and ~10 beyond, i.e. 200 - 330 launches per
+token, while the HBM time of the step is ~2 ms. The reference captures CUDA graphs only in its v1 engine
 (inference/engine.py ``_create_cuda_graph``); here the v2 engine captures its decode steps:
 
 * graphs are keyed by (sequence bucket, KV-length bucket), powers of two (of sequences also 12 and 24, with experts 48, ..), and where the attention kernel splits the

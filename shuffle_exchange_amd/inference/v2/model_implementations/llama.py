@@ -280,7 +280,7 @@ class RaggedLlama:
         RoPE and the cache's append in their epilogues; None otherwise. MoE layers: of the first product alone."""
         if not (0 < T <= STREAM_ROWS_SMALL and self.tps is None and self.device.type == "cuda" and self.head_dim == 128
                 and native.hip_available() and rope.cos.shape[-1] == 64 and rope.cos.dtype == torch.float32
-                and os.environ.get("SXE_DECODE_FUSE", "1") == "1"):
+                and os.environ.get("SXE_DECODE_FUSE", "1") == "1" and os.environ.get("SXE_DECODE_FUSE_ATTN", "1") == "1"):
             return None
         small = self.qw is None or T <= 16  # quantized layers run more rows on the weight as it came
 
