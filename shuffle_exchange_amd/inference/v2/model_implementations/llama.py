@@ -36,7 +36,7 @@ from ....ops.linear import Linear, STREAM_ROWS_SMALL, TILED_GLU_ROWS, glu_faster
 from ....ops.linear import MERGE_COLUMNS, chain_faster, stream_glu, stream_head, stream_res, stream_res_splits, stream_rope, stream_weight
 from ....ops.norm import RMSNorm
 from ....ops.paged_attention import paged_attention_parts, paged_batch_attention, ragged_attention, rope_kv_cache_append
-from ....ops.rows import gather_last
+from ....ops.rows import embed_normed, gather_last
 
 
 class _TPShards:
@@ -306,10 +306,17 @@ class RaggedLlama:
             return None
         return out
 
-    def _chained(self, batch, kv_cache, rope, x, chain):
+    def _embed(self, ids):
+        return self.embed_impl(ids) if self.embed_impl is not None else self.model.embed_tokens(ids)
+
+    def _chained(self, batch, kv_cache, rope, chain):
         """The layers and the head with ``_chain``'s weights: logits."""
         model, T = self.model, batch.num_tokens
-        a = h = sums = None
+        from ..modules.implementations import RaggedEmbedding
+        own = type(self.embed_impl) is RaggedEmbedding
+        first = embed_normed(self.embed_impl.weight, batch.input_ids, model.layers[0].input_layernorm.weight) if own and chain else None
+        a, h, sums = first or (None, None, None)
+        x = self._embed(batch.input_ids) if first is None else h
         for li, (layer, ws) in enumerate(zip(model.layers, chain)):
             kv_layer, norm = kv_cache.layer(li), layer.input_layernorm
             if a is None:
@@ -398,10 +405,10 @@ class RaggedLlama:
             raise ValueError(f"sequence length {batch.max_kv_len} exceeds the model's RoPE table "
                              f"({rope.max_pos} positions, max_position_embeddings)")
         T = batch.num_tokens
-        x = self.embed_impl(batch.input_ids) if self.embed_impl is not None else model.embed_tokens(batch.input_ids)
         chain = self._chain(T, batch, kv_cache, rope)
         if chain is not None:
-            return self._chained(batch, kv_cache, rope, x, chain)
+            return self._chained(batch, kv_cache, rope, chain)
+        x = self._embed(batch.input_ids)
         res = None
         for li, layer in enumerate(model.layers):
             attn = layer.self_attn

@@ -46,6 +46,16 @@ def embed(weight, ids, offset=0):
     return gather_rows(weight, ids, offset)
 
 
+def embed_normed(weight, ids, norm_weight):
+    """(bf16(row * norm_weight), row, sums of squares) of up to 32 ids, as ``ops.linear.stream_res`` leaves them for the first norm and product
+    of a decoder, in one launch; None where the rows or the weight are not bf16 in whole 16 bytes on one device."""
+    if not (_hip_rows(weight) and weight.dtype == norm_weight.dtype == torch.bfloat16 and weight.device == norm_weight.device == ids.device
+            and norm_weight.is_contiguous() and norm_weight.data_ptr() % 16 == 0 and norm_weight.shape == weight.shape[1:]
+            and 0 < ids.numel() <= 32 and ids.dtype in (torch.int32, torch.int64)):
+        return None
+    return torch.ops.sxe.gather_rows_normed(weight, ids.reshape(-1).contiguous(), norm_weight)
+
+
 def gather_last(x, last, res=None):
     """x[last] (+ res[last]) for the final norm + LM head of a ragged batch."""
     return gather_rows(x, last, 0, res)

@@ -228,3 +228,21 @@ def test_layers_of_chained_products(hidden, heads, kv, quant, monkeypatch):
         assert a.dtype == b.dtype and a.shape == b.shape
         # roundings to bf16 (2^-9 in the mean square) of a dozen tensors a layer, other ones by either route
         assert (a - b).norm() < 0.02 * b.norm()
+
+
+@pytest.mark.parametrize("n", [1, 8, 9, 32])
+@pytest.mark.parametrize("K", [8, 1032, 2048, 4104])
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+def test_rows_of_the_embedding_with_their_squares(n, K, dtype):
+    from shuffle_exchange_amd.ops.rows import embed, embed_normed
+    g = torch.Generator(device="cuda").manual_seed(n + K)
+    w = torch.randn(50, K, generator=g, device="cuda").bfloat16()
+    gw = (1 + 0.3 * torch.randn(K, generator=g, device="cuda")).bfloat16()
+    ids = torch.randint(-3, 54, (n,), generator=g, device="cuda").to(dtype)  # ids outside read zeros
+    scaled, rows, sums = embed_normed(w, ids, gw)
+    assert torch.equal(rows, embed(w, ids)) and torch.equal(scaled, (rows.float() * gw.float()).bfloat16())
+    want = rows.double().square().sum(1)
+    assert sums.shape == (1, 8 if n <= 8 else 16 if n <= 16 else 32) and not sums[0, n:].any()
+    assert (sums[0, :n].double() - want).abs().max() <= 1e-6 * want.max()  # fp32 sums of exact squares, a tree of at most 25 steps
+    assert embed_normed(w.float(), ids, gw) is None and embed_normed(w, ids, gw.float()) is None and embed_normed(w[:, 4:], ids, gw[4:]) is None
+    assert embed_normed(w, ids.repeat(33), gw) is None
