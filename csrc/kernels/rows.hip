@@ -30,7 +30,7 @@ namespace rows {
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 // One workgroup a row. Bound by its launch: it takes the place of the gather and of the norm behind it, 4.5 + 3.5 us of a decode step
-// of one sequence of hidden 2048, with a launch of 5.
+// of one sequence of hidden 2048, with a launch of 3.6.
 template <typename I>
 __global__ void __launch_bounds__(256) gather_norm_kernel(const u32x4* __restrict__ src, const u32x4* __restrict__ gw, const I* __restrict__ idx,
                                                           u32x4* __restrict__ out, u32x4* __restrict__ scaled, float* __restrict__ sums, int N,
