@@ -289,12 +289,14 @@ class RaggedLlama:
                 return None
             w = self._wobj(mod, li, key) if small else self.qw[li][key].weight
             return None if w is None else stream_weight(w, T, columns)
+
+        def normed(n):  # four weights a load: one may lie anywhere in a buffer of many
+            return is_own_forward(n, RMSNorm) and n.weight.dtype == torch.bfloat16 and n.weight.data_ptr() % 8 == 0
         out = []
         for li, layer in enumerate(self.model.layers):
-            kv, norms = kv_cache.layer(li), (layer.input_layernorm, layer.post_attention_layernorm)
-            mlp = getattr(layer, "mlp", None)
+            kv, mlp = kv_cache.layer(li), getattr(layer, "mlp", None)
             if (not kv.is_contiguous() or kv.dim() != 5 or kv.dtype != torch.bfloat16 or kv.shape[2] != self.nkv
-                    or any(not is_own_forward(n, RMSNorm) or n.weight.dtype != torch.bfloat16 for n in norms)):
+                    or not normed(layer.input_layernorm) or not normed(layer.post_attention_layernorm)):
                 return None
             ws = [weight(layer.self_attn.qkv_proj, li, "qkv")]
             if mlp is not None:
@@ -302,9 +304,7 @@ class RaggedLlama:
             if any(w is None for w in ws) or not chain_faster(T, ws) or ws[0][0].shape[0] != (self.nq + 2 * self.nkv) * 128:
                 return None
             out.append(ws)
-        if not is_own_forward(self.model.norm, RMSNorm) or self.model.norm.weight.dtype != torch.bfloat16:
-            return None
-        return out
+        return out if normed(self.model.norm) else None
 
     def _embed(self, ids):
         return self.embed_impl(ids) if self.embed_impl is not None else self.model.embed_tokens(ids)

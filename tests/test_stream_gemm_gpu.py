@@ -230,6 +230,26 @@ def test_layers_of_chained_products(hidden, heads, kv, quant, monkeypatch):
         assert (a - b).norm() < 0.02 * b.norm()
 
 
+@pytest.mark.parametrize("which", ["layers.1.input_layernorm", "layers.0.post_attention_layernorm", "norm"])
+def test_norm_weights_anywhere_in_a_buffer(which):
+    """A parameter that starts between two loads of four of its values: the norm is a launch of its own again."""
+    from shuffle_exchange_amd.inference.v2 import RaggedInferenceEngineConfig, build_engine
+    from shuffle_exchange_amd.models import LlamaForCausalLM, llama_config
+    torch.manual_seed(3)
+    cfg = llama_config("llama-tiny", hidden_size=512, intermediate_size=1408, num_hidden_layers=2, num_attention_heads=4, num_key_value_heads=2,
+                       head_dim=128, vocab_size=1000)
+    model = LlamaForCausalLM(cfg).to("cuda", torch.bfloat16)
+    norm, runs = model.get_submodule(which), []
+    weight = (1 + 0.3 * torch.randn(516, device="cuda")).bfloat16()
+    for start in (0, 2):
+        norm.weight = torch.nn.Parameter(weight.roll(start)[start:start + 512])
+        assert norm.weight.data_ptr() % 8 == 2 * start
+        e, g = build_engine(model, RaggedInferenceEngineConfig(kv_block_size=16, num_kv_blocks=60)), torch.Generator().manual_seed(4)
+        runs.append([e.put(list(range(5)), [torch.randint(0, 1000, (n,), generator=g) for n in lens]) for lens in ((3, 1, 8, 2, 5), (1, 1, 1, 1, 1))])
+    for a, b in zip(*runs):  # roundings to bf16 (2^-9 in the mean square) of a dozen tensors a layer, other ones by either route
+        assert (a - b).norm() < 0.02 * b.norm()
+
+
 @pytest.mark.parametrize("n", [1, 8, 9, 32])
 @pytest.mark.parametrize("K", [8, 1032, 2048, 4104])
 @pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
