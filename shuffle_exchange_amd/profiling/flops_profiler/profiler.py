@@ -67,6 +67,10 @@ def _register_sxe_formulas():
         def _stream(x, w, *a, out_shape=None, **kw):
             return 2 * x[0] * w[0] * w[1]
 
+        @register_flop_formula(ops.stream_gemm_res_splits)
+        def _stream_splits(part_o, part_ml, w, *a, out_shape=None, **kw):  # one row, in splits
+            return 2 * w[0] * w[1]
+
         @register_flop_formula([ops.gemm_tn, ops.gemm_tn_into])
         def _tiled(x, w, *a, out_shape=None, **kw):  # x [.., K]
             return 2 * math.prod(x) * w[0]

@@ -106,3 +106,23 @@ def test_products_of_many_rows_and_experts_are_counted():
     c = torch.zeros(3, 128, 192, device="cuda")
     assert count(lambda: torch.ops.sxe.wgrad_gemm_(e, t(3, 40, 192), c, 1.0, False)) == 2 * 3 * 40 * 128 * 192
     assert count(lambda: torch.ops.sxe.wgrad_gemm2_(e, t(3, 40, 192), t(3, 24, 128), t(3, 24, 192), c, 1.0, False)) == 2 * 3 * 64 * 128 * 192
+
+
+@pytest.mark.gpu
+def test_chained_decode_products_are_counted():
+    """Every product of a decode step's layer, also the one that takes its row from attention's splits."""
+    from shuffle_exchange_amd.ops import native
+    from torch.utils.flop_counter import FlopCounterMode
+    from shuffle_exchange_amd.profiling.flops_profiler.profiler import _register_sxe_formulas
+    native.require_hip()
+    _register_sxe_formulas()
+
+    def t(*shape, dtype=torch.bfloat16):
+        return torch.randn(*shape, device="cuda", dtype=dtype)
+    w, gw = t(512, 256), t(512)
+    parts = t(3, 1, 2, 128, dtype=torch.float32), t(3, 1, 2, 2, dtype=torch.float32)
+    with FlopCounterMode(display=False) as fc:
+        torch.ops.sxe.stream_gemm_res_splits(*parts, w, None, t(1, 512), gw)
+        torch.ops.sxe.stream_gemm_res(t(3, 256), w, None, None, t(3, 512), gw)
+        torch.ops.sxe.stream_gemm_normed(t(3, 256), w, None, None, 1e-5, True)
+    assert fc.get_total_flops() == 2 * 512 * 256 * (1 + 3 + 3)
