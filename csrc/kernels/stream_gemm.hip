@@ -224,7 +224,7 @@ __global__ void __launch_bounds__(64 * NW, 2) stream_gemm_kernel(Args a) {
   constexpr int TC = HALF ? 8 : 16, PAIRS = TC * NT / 2;
   __shared__ f32x4 red[NW][NT][64];
   __shared__ __attribute__((aligned(16))) unsigned short merged[MERGE ? MERGE_K : 8];
-  __shared__ float squares[NORMED ? NW : 1][NORMED ? 32 : 1];
+  __shared__ __attribute__((aligned(16))) float squares[NORMED ? NW : 1][NORMED ? 32 : 1];  // written four at a time
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, g = lane >> 4;
   const int half = a.N / 2;
   const int j = lane & 3, quad0 = l16 & (TC - 4), c = 4 * g + j;
