@@ -425,14 +425,19 @@ __global__ __launch_bounds__(64 * W, W > 4 ? 2 : D == 256 ? 1 : D * NT > 256 ? 2
 // Combine the splits' fp32 partials: D / 4 threads a (token, head) row, 16 bytes a load, every load of a group of up to U
 // splits issued before the first use (a loop that consumes each partial before loading the next makes a chain of
 // dependent ~1 us memory round trips: 10 us at 16 splits). Splits without keys (maximum -inf) are not read.
-template <int D, int U>
+// MARKED: rows of which split 0 has a negative sum are there already (paged_prefill.hip). Asked for these alone: it is a load in front of all
+// others, 0.35 us of a decode step's call (8 sequences of 900 keys, heads 16 / 8, 10.69 / 10.31; 24 of 900, 32 / 8, 22.85 / 22.47).
+template <int D, int U, bool MARKED>
 __global__ __launch_bounds__(256) void merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                                     int splits, int64_t T, int nq, unsigned short* __restrict__ out,
                                                     int64_t out_tok_stride, const int* __restrict__ rows) {
   constexpr int TPR = D / 4, RPB = 256 / TPR;
   const int64_t sstride = T * nq, th = (int64_t)blockIdx.x * RPB + threadIdx.x / TPR;  // partial row * nq + h
   const int d = threadIdx.x % TPR * 4;
-  if (th >= sstride || part_ml[th * 2 + 1] < 0.f) return;  // a negative sum: no splits, the result is there (paged_prefill.hip)
+  if (th >= sstride) return;
+  if constexpr (MARKED) {
+    if (part_ml[th * 2 + 1] < 0.f) return;
+  }
   const int64_t pt = th / nq, t = rows ? rows[pt] : pt;  // rows: token row of every partial row
   const int h = th - pt * nq;
   float M = -INFINITY, L = 0.f;
@@ -537,6 +542,7 @@ void kv_cache_append(const at::Tensor& qkv, at::Tensor cache, const at::Tensor& 
 }
 
 // part_o [splits, R, nq, D], part_ml [splits, R, nq, 2] -> out [T, nq, D]; rows: token row of each of the R (null: itself)
+template <bool MARKED>
 static void launch_merge(const at::Tensor& part_o, const at::Tensor& part_ml, const int* rows, at::Tensor& out) {
   const int splits = part_o.size(0), R = part_o.size(1), nq = part_o.size(2), D = part_o.size(3);
   auto* op = reinterpret_cast<unsigned short*>(out.data_ptr());
@@ -545,14 +551,14 @@ static void launch_merge(const at::Tensor& part_o, const at::Tensor& part_ml, co
     hipLaunchKernelGGL(kern, dim3(((int64_t)R * nq + rpb - 1) / rpb), dim3(256), 0, cur_stream(), part_o.data_ptr<float>(),
                        part_ml.data_ptr<float>(), splits, (int64_t)R, nq, op, out.stride(0), rows);
   };
-  if (D == 128) launch(splits <= 4 ? pa::merge_kernel<128, 4> : pa::merge_kernel<128, 16>);
-  else if (D == 256) launch(splits <= 4 ? pa::merge_kernel<256, 4> : pa::merge_kernel<256, 16>);
-  else launch(splits <= 4 ? pa::merge_kernel<64, 4> : pa::merge_kernel<64, 16>);
+  if (D == 128) launch(splits <= 4 ? pa::merge_kernel<128, 4, MARKED> : pa::merge_kernel<128, 16, MARKED>);
+  else if (D == 256) launch(splits <= 4 ? pa::merge_kernel<256, 4, MARKED> : pa::merge_kernel<256, 16, MARKED>);
+  else launch(splits <= 4 ? pa::merge_kernel<64, 4, MARKED> : pa::merge_kernel<64, 16, MARKED>);
   SXE_LAUNCH_CHECK();
 }
 
 void paged_merge(const at::Tensor& part_o, const at::Tensor& part_ml, const at::Tensor& rows, at::Tensor& out) {
-  launch_merge(part_o, part_ml, rows.data_ptr<int>(), out);
+  launch_merge<true>(part_o, part_ml, rows.data_ptr<int>(), out);
 }
 
 // q: [T, nq, D] (token stride free); returns out [T, nq, D] bf16. parts != nullptr (and splits > 1):
@@ -645,7 +651,7 @@ static at::Tensor paged_attention_impl(const at::Tensor& q, const at::Tensor& ca
     *parts = {part_o, part_ml};
     return out;
   }
-  if (splits > 1 && a.counters == nullptr) launch_merge(part_o, part_ml, rows ? rows->data_ptr<int>() : nullptr, out);
+  if (splits > 1 && a.counters == nullptr) launch_merge<false>(part_o, part_ml, rows ? rows->data_ptr<int>() : nullptr, out);
   return out;
 }
 
