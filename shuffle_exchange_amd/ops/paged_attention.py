@@ -162,14 +162,15 @@ def choose_balanced_splits(num_seqs, nkv, max_kv_len, split_bytes, even=False, h
 # keys in two rounds of four waves / in one of eight / splits of 128: hidden 2048, 1 sequence of 500 keys 175.0 / 172.1 / 168.0, 4 of 1000
 # 187.6 / 182.8 / 180.0; 3072, 2 of 1500 246.0 / 242.1 / 239.8; 4096, 1 of 1000 357.2 / 353.3 / 348.8; but with two workgroups a CU, hidden
 # 2048, 8 of 1500 191.9 / 189.3 / 191.7. 3000 keys, one sequence of hidden 2048 180.1 / 176.7 / 181.7, 4096 364.5 / 360.2 / 370.8.
-# Where two splits need the merge's launch and one does not (up to 256 keys), 120 keys cost 2 % more and 250 3 % less: as it was.
+# Up to 256 keys one split stays one, with nothing to merge. One sequence, 1 / 2 splits of 128 keys, merged in the next product's launch: hidden
+# 2048, 64 keys 151 / 155, 250 keys 156 / 156, e4m3 113 / 118, 117 / 119; 4096 311 / 311, 316 / 316; o product of skinny_gemm.hip, 64 keys 171 / 174, e4m3
+# 125 / 131, hidden 4096 348 / 354, 236 / 240 (from 400 to 2000 keys there, splits of 256 / 128 keys, 360 / 356, 246 / 242).
 PA_SHORT_KEYS = 2048
 PA_SHORT_WGS = 256
 
 
-def _short_splits(splits, num_seqs, nkv, max_kv_len, split_bytes, head_dim, merged=False):
-    """``merged``: the splits are read by the next product, with no launch for their merge."""
-    if head_dim != 128 or not (1 if merged else PA_MIN_KEYS) < max_kv_len <= PA_SHORT_KEYS:
+def _short_splits(splits, num_seqs, nkv, max_kv_len, split_bytes, head_dim):
+    if head_dim != 128 or not PA_MIN_KEYS < max_kv_len <= PA_SHORT_KEYS:
         return splits
     want = min(PA_SHORT_WGS // max(1, num_seqs * nkv), math.ceil(max_kv_len / max(1, PA_MIN_KEYS // 2)))
     return max(splits, min(want, PA_SPLIT_BYTES // max(1, split_bytes)))
@@ -188,10 +189,10 @@ def paged_attention_parts(q, cache, block_table, q_start, q_len, kv_len, scale, 
     """``paged_attention`` without the split-merge launch (HIP only): returns ``(out, None)`` when the
     kernel ran one split per (sequence, kv head), else ``(None, (part_o, part_ml))`` -- fp32
     partials [splits, T, nq, D] / [splits, T, nq, 2] for a consumer that merges them in its own
-    prologue (``ops.linear.fused_merge_linear``: the o_proj skinny GEMM)."""
+    prologue (``ops.linear.fused_merge_linear``: the o_proj skinny GEMM; ``stream_res_splits``)."""
     if splits is None:
-        splits = _short_splits(choose_splits(block_table.shape[0], cache.shape[2], max_kv_len), block_table.shape[0], cache.shape[2],
-                               int(max_kv_len), 4 * q.numel(), q.shape[-1], True)
+        S, nkv = block_table.shape[0], cache.shape[2]
+        splits = _short_splits(choose_splits(S, nkv, max_kv_len), S, nkv, int(max_kv_len), 4 * q.numel(), q.shape[-1])
     out, po, pml = torch.ops.sxe.paged_attention_parts(q, cache, block_table, q_start, q_len, kv_len, float(scale),
                                                        int(max_kv_len), int(splits), 0)
     return (out, None) if po.numel() == 0 else (None, (po, pml))

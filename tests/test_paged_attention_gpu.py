@@ -125,6 +125,19 @@ def test_merge_attention_parts_matches_fused_kernel(splits):
     assert ((merged.float() - ref).norm() / ref.norm()).item() < 1e-2
 
 
+@pytest.mark.parametrize("keys,splits", [(100, 1), (200, 1), (256, 1), (300, 3), (1000, 8), (2048, 16), (3000, 12)])
+def test_splits_left_to_a_product(keys, splits):
+    """One up to 256 keys: there is nothing to merge then."""
+    from shuffle_exchange_amd.ops import paged_attention as PA
+    qkv, cache, bt, qs, ql, kl, slots, maxkv = _setup([(keys - 1, 1)], 32, 8, 128, 64)
+    args = (qkv[:, :32], cache, bt, qs, ql, kl, 128 ** -0.5)
+    ref = PA.paged_attention_reference(*(t.float() for t in args[:2]), *args[2:])
+    out, parts = PA.paged_attention_parts(*args, maxkv)
+    assert maxkv == keys and (1 if parts is None else len(parts[0])) == splits
+    got = PA.merge_attention_parts(*parts, torch.bfloat16) if out is None else out
+    assert ((got.float() - ref).norm() / ref.norm()).item() < 1e-2
+
+
 @pytest.mark.parametrize("splits", [2, 5, 16])
 def test_in_kernel_split_merge_matches_merge_launch(splits, monkeypatch):
     """Decode with the last split workgroup merging in-kernel (arrival counters) == the separate
