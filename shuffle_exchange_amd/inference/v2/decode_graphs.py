@@ -14,7 +14,7 @@ token, while the HBM time of the step is ~2 ms. The reference captures CUDA grap
 * padding sequences point at a reserved scratch KV block and state slot (q_len = kv_len = 1), so every
   row the graph computes is well defined and no real cache slot is touched;
 * the paged-attention grid is fixed per graph by the KV bucket (splits of at most 512 keys while their partials
-  are small, ops/paged_attention.choose_balanced_splits; workgroups past a sequence's length exit at once).
+  are small, ops/paged_attention.decode_plan; workgroups past a sequence's length exit at once).
 
 MoE models whose expert counts go through the host, sliding windows narrower than the KV bucket and modules whose
 weights are made anew for every generation (hybrid engine) run eagerly.
@@ -22,7 +22,7 @@ weights are made anew for every generation (hybrid engine) run eagerly.
 import numpy as np
 import torch
 
-from ...ops.paged_attention import choose_balanced_splits, even_lengths
+from ...ops.paged_attention import decode_plan, even_lengths
 
 MIN_KV_BUCKET = 256
 
@@ -111,8 +111,8 @@ class DecodeGraphRunner:
         matters = self._matters.get((S, kvb))
         if matters is None:
             nq, nkv, dim = (getattr(self.model, name, None) for name in ("nq", "nkv", "head_dim"))
-            splits = [choose_balanced_splits(S, nkv, kvb, 4 * S * nq * dim, even, dim) for even in (True, False)] if nq and nkv and dim else (1, 1)
-            matters = self._matters[S, kvb] = splits[0] != splits[1]
+            plans = [decode_plan(S, nkv, kvb, 4 * S * nq * dim, even, dim) for even in (True, False)] if nq and nkv and dim else (1, 1)
+            matters = self._matters[S, kvb] = plans[0] != plans[1]
         return matters and even_lengths([s.seen_tokens + 1 for s in seqs])
 
     # ------------------------------------------------------------------------------------- run

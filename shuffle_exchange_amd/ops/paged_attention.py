@@ -185,6 +185,11 @@ def _decode_plan(num_seqs, nkv, max_kv_len, split_bytes, even, head_dim, tuned):
     return splits, splits == 1 and two_a_cu(num_seqs * nkv, head_dim)
 
 
+def decode_plan(num_seqs, nkv, max_kv_len, split_bytes, even, head_dim):
+    """``_decode_plan`` by the settings as they are."""
+    return _decode_plan(num_seqs, nkv, max_kv_len, split_bytes, even, head_dim, (PA_TARGET_WGS, PA_MIN_KEYS))
+
+
 def paged_attention_parts(q, cache, block_table, q_start, q_len, kv_len, scale, max_kv_len, splits=None):
     """``paged_attention`` without the split-merge launch (HIP only): returns ``(out, None)`` when the
     kernel ran one split per (sequence, kv head), else ``(None, (part_o, part_ml))`` -- fp32
@@ -239,7 +244,7 @@ def paged_attention(q, cache, block_table, q_start, q_len, kv_len, scale, max_kv
     if native.use_hip(q) and q.shape[-1] in (64, 128, 256):
         S, nkv = block_table.shape[0], cache.shape[2]
         if splits is None:
-            splits, wide = _decode_plan(S, nkv, int(max_kv_len), 4 * q.numel(), even, q.shape[-1], (PA_TARGET_WGS, PA_MIN_KEYS))
+            splits, wide = decode_plan(S, nkv, int(max_kv_len), 4 * q.numel(), even, q.shape[-1])
         else:
             wide = splits == 1 and two_a_cu(S * nkv, q.shape[-1])
         cnt = (_split_counters(q.device, S * nkv)
@@ -360,8 +365,7 @@ def ragged_attention(q, cache, batch, scale, window=None, kv=None):
             torch.ops.sxe.paged_prefill(*meta, x.tiles, rows, float(scale), int(window or 0), splits, keys, out)
     if lists is not None and lists.seqs is not None:
         n, D = lists.seqs.shape[0], q.shape[2]
-        splits, wide = _decode_plan(n, nkv, lists.seq_keys, 4 * lists.seq_rows.numel() * q.shape[1] * D, lists.seq_even, D,
-                                    (PA_TARGET_WGS, PA_MIN_KEYS))
+        splits, wide = decode_plan(n, nkv, lists.seq_keys, 4 * lists.seq_rows.numel() * q.shape[1] * D, lists.seq_even, D)
         torch.ops.sxe.paged_attention_some(*meta, lists.seqs, lists.seq_rows, float(scale), int(lists.seq_keys), int(splits),
                                            int(window or 0), out, wide)
     return out

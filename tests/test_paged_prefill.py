@@ -279,3 +279,22 @@ def test_short_splits_of_few_workgroups():
             for nkv, dim, room in ((1, 128, 1 << 10), (8, 128, 1 << 14), (8, 128, 1 << 27), (8, 64, 1 << 14), (8, 256, 1 << 14)):
                 was, n = PA.choose_balanced_splits(S, nkv, keys, room, True, dim), PA._decode_plan(S, nkv, keys, room, True, dim, None)[0]
                 assert n == was or (dim == 128 and 256 < keys <= 2048 and was < n <= -(-keys // 128) and S * nkv * n <= 256 and n * room <= PA.PA_SPLIT_BYTES)
+
+
+@pytest.mark.parametrize("target", [512, 4])
+def test_graphs_by_lengths_only_where_the_splits_differ(target, monkeypatch):
+    """A decode graph of sequences of like lengths and one of any lengths are two where attention takes other splits for them, not else."""
+    from types import SimpleNamespace as N
+    from shuffle_exchange_amd.inference.v2.decode_graphs import DecodeGraphRunner
+    monkeypatch.setattr(PA, "PA_TARGET_WGS", target)  # few: chosen by the lengths, but for the short splits of few sequences
+    seen = set()
+    for nq, nkv, dim in ((32, 8, 128), (4, 2, 128), (12, 12, 64)):
+        r = DecodeGraphRunner.__new__(DecodeGraphRunner)
+        r.model, r._matters = N(nq=nq, nkv=nkv, head_dim=dim), {}
+        for S in (2, 4, 12, 24, 64, 128):
+            for kvb in (256, 512, 1024, 2048, 4096, 16384):
+                plans = [PA.decode_plan(S, nkv, kvb, 4 * S * nq * dim, even, dim) for even in (True, False)]
+                like, unlike = [N(seen_tokens=kvb - 1)] * S, [N(seen_tokens=kvb - 1)] + [N(seen_tokens=0)] * (2 * S)
+                assert r._even(S, kvb, like) == (plans[0] != plans[1]) and not r._even(S, kvb, unlike)
+                seen.add((dim, plans[0] != plans[1]))
+    assert seen == {(dim, differ) for dim in (64, 128) for differ in (False, True)}
