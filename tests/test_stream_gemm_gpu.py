@@ -24,6 +24,13 @@ def _operands(M, N, K, fp8, seed):
     return x, q.view(torch.uint8), s, q.double() * s.double()[:, None]
 
 
+def _rounding(values):
+    """Products of bf16 are exact in fp32; left are fp32 sums and the rounding of the result. It is at most 2^-8 of a value (just above a power
+    of two), which a result of a few values comes near; over many it is spread evenly, 2^-8 / sqrt(3) of the power of two below each, 1.7e-3
+    of normal values together and more where a few large ones are most of their norm."""
+    return 1.01 * 2 ** -8 if values.numel() < 256 else 3e-3
+
+
 @pytest.mark.parametrize("M", [1, 5, 15, 16, 17, 32])
 @pytest.mark.parametrize("N,K", [(4, 16), (20, 1024), (6144, 96), (6148, 4112), (128, 2064), (8192, 2048)])
 @pytest.mark.parametrize("fp8", [False, True])
@@ -33,9 +40,7 @@ def test_plain(M, N, K, fp8):
     for bias in (None, b):
         got = torch.ops.sxe.stream_gemm(x, w, s, bias, False)
         want = x.double() @ ref.T + (0 if bias is None else b.double())
-        # products of bf16 are exact in fp32; left are fp32 sums and the rounding of the result: at most 2^-8 of a value (just above a power
-        # of two), which a result of four values with a bias drawn anew each time comes near
-        assert (got.double() - want).norm() < 1.01 * 2 ** -8 * want.norm()
+        assert (got.double() - want).norm() < _rounding(want) * want.norm()
 
 
 @pytest.mark.parametrize("M", [1, 7, 8])
@@ -45,11 +50,11 @@ def test_pieces_in_flight(M, N, K):
     """Two at a time, or pieces of twice the size: any of the waves may have one more or one less than the others."""
     x, w, _, ref = _operands(M, N, K, False, M + N + K)
     want = x.double() @ ref.T
-    assert (torch.ops.sxe.stream_gemm(x, w, None, None, False).double() - want).norm() < 1.01 * 2 ** -8 * want.norm()
+    assert (torch.ops.sxe.stream_gemm(x, w, None, None, False).double() - want).norm() < _rounding(want) * want.norm()
     assert (torch.ops.sxe.stream_gemm_normed(x, w, None, None, 0.0, False).double() - want).norm() < 1e-5 * want.norm()
     res, gw = torch.randn(M, N, device="cuda").bfloat16(), torch.ones(N, device="cuda").bfloat16()
     want = want + res.double()
-    assert (torch.ops.sxe.stream_gemm_res(x, w, None, None, res, gw)[1].double() - want).norm() < 1.01 * 2 ** -8 * want.norm()
+    assert (torch.ops.sxe.stream_gemm_res(x, w, None, None, res, gw)[1].double() - want).norm() < _rounding(want) * want.norm()
 
 
 def test_every_e4m3_value_is_exact():
@@ -119,7 +124,7 @@ def test_residual_and_what_a_normed_product_needs(M, N, K, fp8):
     gw = (1 + 0.3 * torch.randn(N, device="cuda")).bfloat16()
     y, h, sums = torch.ops.sxe.stream_gemm_res(x, w, s, None, res, gw)
     want = res.double() + x.double() @ ref.T
-    assert (h.double() - want).norm() < 1.01 * 2 ** -8 * want.norm()
+    assert (h.double() - want).norm() < _rounding(want) * want.norm()
     assert torch.equal(y, (h.float() * gw.float()).bfloat16())
     tiles, rows = sums.shape
     assert N // tiles in (8, 16) and rows in (8, 16, 32) and rows >= M and not sums[:, M:].any()
@@ -141,7 +146,7 @@ def test_residual_of_a_row_in_splits(N, heads, dim, splits, fp8):
     row = merge_attention_parts(po[pml[:, 0, 0, 0] > -1e30], pml[pml[:, 0, 0, 0] > -1e30], torch.float32).view(1, -1)
     want = res.double() + row.double() @ ref.T
     # the row's rounding to bf16 (2^-8 at most) on its way into the product, then that of the result
-    assert (got[1].double() - want).norm() < 1.01 * 2 ** -8 * (want.norm() + (want - res.double()).norm())
+    assert (got[1].double() - want).norm() < _rounding(want) * (want.norm() + (want - res.double()).norm())
     assert torch.equal(got[0], (got[1].float() * gw.float()).bfloat16())
     squares = got[1].double().square().view(len(got[2]), -1).sum(-1)
     assert (got[2][:, 0].double() - squares).abs().max() <= 1e-6 * squares.max() and not got[2][:, 1:].any()
@@ -160,7 +165,7 @@ def test_products_behind_a_norm(M, N, K, tiles, fp8):
     g, u = p.chunk(2, -1)
     mid = torch.ops.sxe.stream_gemm_normed(x, w, s, sums, 1e-3, True)
     want = torch.nn.functional.silu(g) * u
-    assert (mid.double() - want).norm() < 1.01 * 2 ** -8 * want.norm()
+    assert (mid.double() - want).norm() < _rounding(want) * want.norm()
     plain = torch.ops.sxe.stream_gemm_normed(x, w, s, None, 0.0, False)
     assert torch.equal(plain.bfloat16(), torch.ops.sxe.stream_gemm(x, w, s, None, False))
 
@@ -188,7 +193,7 @@ def test_rotated_heads_and_the_cache(M, nq, nkv, K, fp8, normed):
     want[:, nq + nkv:] = p[:, nq + nkv:]
     want = want.view(M, nq + 2 * nkv, 128)
     got = got.view(M, nq + 2 * nkv, 128)
-    assert (got.double() - want).norm() < 1.01 * 2 ** -8 * want.norm()
+    assert (got.double() - want).norm() < _rounding(want) * want.norm()
     expect = torch.full_like(cache, 7.0)
     for i, at in enumerate(slots.tolist()):
         if at >= 0:
@@ -197,33 +202,52 @@ def test_rotated_heads_and_the_cache(M, nq, nkv, K, fp8, normed):
 
 
 @pytest.mark.parametrize("quant", [None, "fp8"])
-@pytest.mark.parametrize("hidden,heads,kv", [(512, 4, 2), (2304, 18, 2)])  # half tiles and whole ones
-def test_layers_of_chained_products(hidden, heads, kv, quant, monkeypatch):
-    """Prompts, decode steps and a pass whose logits are not one a sequence, by either route over the same cache."""
+@pytest.mark.parametrize("hidden,heads,kv,experts", [(512, 4, 2, 0), (2304, 18, 2, 0), (512, 4, 2, 2)])  # half tiles and whole ones
+def test_layers_of_chained_products(hidden, heads, kv, experts, quant, monkeypatch):
+    """Prompts, decode steps and a pass whose logits are not one a sequence, by either route over the same cache. With experts every token
+    has all of them, so that no near tie of the router goes another way."""
     from shuffle_exchange_amd.inference.v2 import RaggedInferenceEngineConfig, build_engine
-    from shuffle_exchange_amd.inference.v2.model_implementations.llama import RaggedLlama
-    from shuffle_exchange_amd.models import LlamaForCausalLM, llama_config
+    from shuffle_exchange_amd.inference.v2.model_implementations import llama as module
+    from shuffle_exchange_amd.models import LlamaForCausalLM, MixtralForCausalLM, llama_config, mixtral_config
     torch.manual_seed(1)
-    cfg = llama_config("llama-tiny", hidden_size=hidden, intermediate_size=1408, num_hidden_layers=2, num_attention_heads=heads,
-                       num_key_value_heads=kv, head_dim=128, vocab_size=1000)
-    model = LlamaForCausalLM(cfg).to("cuda", torch.bfloat16)
+    sizes = dict(hidden_size=hidden, intermediate_size=1408, num_hidden_layers=2, num_attention_heads=heads, num_key_value_heads=kv, head_dim=128,
+                 vocab_size=1000, max_position_embeddings=512)
+    model = (MixtralForCausalLM(mixtral_config("mixtral-tiny", num_local_experts=experts, num_experts_per_tok=experts, **sizes)) if experts
+             else LlamaForCausalLM(llama_config("llama-tiny", **sizes))).to("cuda", torch.bfloat16)
     g = torch.Generator().manual_seed(2)
-    chained, runs = [], []
-    own = RaggedLlama._chain
+    chained, runs, calls = [], [], {}
+    own = module.RaggedLlama._chain
+
+    def counted(name):
+        of = getattr(module, name)
+
+        def call(*args):
+            y = of(*args)
+            calls[name] = calls.get(name, 0) + (y is not None)
+            return y
+        monkeypatch.setattr(module, name, call)
+    for name in ("embed_normed", "stream_rope", "stream_res", "stream_res_splits", "stream_glu", "stream_head"):
+        counted(name)
     for on in (True, False):
         def chain(self, *args):
             chained.append(on and own(self, *args) is not None)
             return own(self, *args) if on else None
-        monkeypatch.setattr(RaggedLlama, "_chain", chain)
+        monkeypatch.setattr(module.RaggedLlama, "_chain", chain)
         g.manual_seed(2)
         e = build_engine(model, RaggedInferenceEngineConfig(kv_block_size=16, num_kv_blocks=200, weight_quant=quant))
-        out = [e.put([i], [torch.randint(0, 1000, (n,), generator=g)]) for i, n in enumerate((7, 31, 3))]
-        for uids in ([0, 1, 2], [1], [0, 2]):
+        out = [e.put([i], [torch.randint(0, 1000, (n,), generator=g)]) for i, n in enumerate((7, 31, 3, 300))]
+        for uids in ([0, 1, 2], [3], [0, 2]):
             for _ in range(2):
                 out.append(e.put(uids, [torch.randint(0, 1000, (1,), generator=g) for _ in uids]))
         out.append(e.put([0, 1], [torch.randint(0, 1000, (n,), generator=g) for n in (5, 1)], want=[(1, 4, 0), ()]))
         runs.append(out)
-    assert any(chained)
+    # three short prompts and one of 300 tokens, the steps' three graphs, each of a pass before its capture and the captured one, a mixed pass
+    assert chained == [True] * 3 + [False] + [True] * 7 + [False] * 11
+    splits = 4 if hidden <= 2048 and not experts else 0  # the graph of one sequence of 300 keys: two layers, twice
+    want = {"embed_normed": 10, "stream_rope": 20}
+    if not experts:  # else two launches of the norm a layer, and the head behind one
+        want.update(stream_res=40 - splits, stream_glu=20, stream_head=6, **({"stream_res_splits": splits} if splits else {}))
+    assert calls == want
     for a, b in zip(*runs):
         assert a.dtype == b.dtype and a.shape == b.shape
         # roundings to bf16 (2^-9 in the mean square) of a dozen tensors a layer, other ones by either route
