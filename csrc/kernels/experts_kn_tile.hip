@@ -283,7 +283,7 @@ static void launch(const Args& a) {
   SXE_LAUNCH_CHECK();
 }
 // 128 rows a tile where few column blocks make few rounds of workgroups over the CUs and theirs are the shorter ones (a round of 128 rows
-// takes 0.67 of one of 256). Products with h, us, 256 / 128: 4096 columns of 14336 k, 150 rows an expert of eight 271 / 233, 250
+// takes 0.65 of one of 256, as in `end_of`; the rule takes it for two thirds). Products with h, us, 256 / 128: 4096 columns of 14336 k, 150 rows an expert of eight 271 / 233, 250
 // 318 / 382, 400 581 / 407, 800 661 / 768; 2048 of 8192, 250 170 / 118, 550 187 / 203. Many column blocks: 28672 of 4096 k, 50 rows
 // 379 / 364, 150 403 / 508, 800 1358 / 1481
 // 192 rows where as many for every expert would end clearly sooner in them; the kernel decides by the rows that they have (a prompt's lie near

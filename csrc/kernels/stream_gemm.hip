@@ -26,7 +26,8 @@ constexpr int NW = 8;  // waves of a workgroup
 // launches of their own: EPI_RES adds the residual stream, EPI_ROPE rotates q and k and appends k and v to the paged cache, EPI_NGLU and
 // EPI_HEAD (fp32 result) are the other two products behind a norm. A norm between two products is split over both: the first one's
 // epilogue holds the new residual stream and leaves (stream x norm weight) in bf16 for the next product and its tiles' sums of squares; the
-// next one adds those up (rows x tiles, 32 KB at most, behind its first operand loads) and multiplies its sums by 1 / rms. The operand is
+// next one asks for those (rows x tiles of 4 bytes: 32 rows of hidden 4096 32 KB, of 8192 64) in front of its first operand loads, adds them up
+// behind these and multiplies its sums by 1 / rms. The operand is
 // rounded once, as a norm's result is; the product and the sum are no longer rounded before they meet the stream.
 // A launch costs a step ~4.7 us whatever it does: a layer of 4096 x 4096 / 28672 x 4096 has 6 of them, 9 before.
 enum Epi { EPI_PLAIN, EPI_GLU, EPI_RES, EPI_ROPE, EPI_NGLU, EPI_HEAD };
@@ -52,7 +53,7 @@ struct Args {
   const float *po, *pml;
   int splits, dim;
   unsigned short* h;  // [M, N], the new stream
-  float* sums;        // [N / 16, mp]
+  float* sums;        // [N / 16, mp]; half tiles: [N / 8, mp]
   // ROPE: w's rows are nq + 2 nkv heads of 128
   const float *rcos, *rsin;  // [positions, 64]
   const int64_t *pos, *slots;
@@ -617,7 +618,7 @@ static void split_row(st::Args& a, const at::Tensor& part_o, const at::Tensor& p
   a.dim = part_o.size(3);
 }
 
-// h = res + x . w^T (+ bias), and what a product of rms_norm(h) * gw needs: -> [bf16(h * gw), h, sums of h^2 [tiles of N, rows]]
+// h = res + x . w^T (+ bias), and what a product of rms_norm(h) * gw needs: -> [bf16(h * gw), h, sums of h^2 [tiles of 16 or 8 columns, rows]]
 static std::vector<at::Tensor> residual(st::Args a, bool fp8, const at::Tensor& w, const at::Tensor& res, const at::Tensor& gw) {
   check_beside(w, {res, gw});
   SXE_CHECK(a.N % 16 == 0, "stream_gemm_res: whole tiles of 16 columns");

@@ -38,7 +38,9 @@ def sequence_bucket(n, experts=False):
     """Rows of the graph that runs ``n`` sequences: powers of two and, from 8 on, what lies half way. Padding rows cost their part of the products
     and of attention's workgroups, and choose experts that no sequence needs; every bucket is captured by itself. us a step of two layers at the
     next power of two / here: 9 sequences of 8b 299 / 292, in e4m3 237 / 227, 17 379 / 366; of Mixtral 20 1427 / 1245, 33 1667 / 1313. Not from 33 on
-    without experts, whose products the library runs: 41 of 3b 299 / 308, 40 of 8b 444 / 461. (5 in e4m3 206, as 6 199.)"""
+    without experts, whose products the library runs: 41 of 3b 299 / 308, 40 of 8b 444 / 461. (5 in e4m3 206, as 6 199.) Other decoders, 9 and 24
+    sequences: RaggedDecoder, two layers of 8b 296 / 290, 381 / 374, of 3b 201 / 196, 263 / 257, of 1b 163.5 / 162.9, 191.9 / 192.1; eight layers of Tobinex 8b 1132
+    / 1107, 1454 / 1427, 1b 655 / 650, 771 / 746; of Bipotar 8b, with experts, 1514 / 1456, 1885 / 1748, 1b 664 / 642, 800 / 744."""
     p = _pow2_at_least(n)
     return p // 4 * 3 if 8 < p <= (256 if experts else 32) and n <= p // 4 * 3 else p
 

@@ -202,7 +202,8 @@ class RaggedLlama:
             return self.qw[li][key](x)
         return linear(x, mod.weight, mod.bias, self._host_bound) if is_own_forward(mod, Linear) else mod(x)
 
-    # decode (<= 4 tokens): RMSNorm folded into the QKV / gate_up GEMMs as their prologue, SwiGLU into gate_up's
+    # decode (<= 4 tokens) of a model that ``_chain`` does not cover, be it for one projection that is more than its product, one norm weight
+    # of another type or heads of another size: RMSNorm folded into the QKV / gate_up GEMMs as their prologue, SwiGLU into gate_up's
     # epilogue (skinny_gemm.hip) -- three latency-bound launches fewer per layer
     FUSE_MAX_T = 4
 
@@ -211,7 +212,7 @@ class RaggedLlama:
                 and os.environ.get("SXE_DECODE_FUSE", "1") == "1")
 
     def _attn_o(self, attn, qkv, kv_layer, batch, li, T):
-        """Attention + o_proj. One token: the KV-split merge runs inside the o_proj GEMM launch
+        """Attention + o_proj outside ``_chained``. One token: the KV-split merge runs inside the o_proj GEMM launch
         (paged_attention_parts + fused_merge_linear) -- one latency-bound launch fewer per layer. More tokens: every workgroup
         of that launch would read all of their partials; 4 sequences of 4000 keys, 4 layers of Llama-8B: 704 us a step so, 658
         with a merge launch (1 sequence: 548 / 547; 2: 602 / 581)."""

@@ -97,9 +97,11 @@ def _stream_faster(rows, N, K):
 
 def glu_faster(rows, weight):
     """Whether ``glu_linear`` beats the product and the activation's launch. e4m3: always (8 rows of 28672 x 4096 34 / 26 us with the
-    product of skinny_gemm.hip). bf16, four tiles a workgroup (two, as now, take up to 5 % less), us, with the library's product / here: 16 rows 16384 x 2048
-    20.7 / 17.4, 28672 x 4096 63 / 46, 36864 x 5120 80 / 76, but 57344 x 8192 170 / 183; 24 rows 10240 x 2560 17.9 / 15.9,
-    16384 x 3072 24.4 / 23.3, 28672 x 4096 59 / 52, but 17920 x 2560 25.9 / 30.6, 27648 x 5120 54 / 63, 7168 x 4096 18.1 / 20.7."""
+    product of skinny_gemm.hip). bf16, us, with the library's product / here: 8 rows 28672 x 4096 63 / 40; 16 rows 16384 x 2048 20.5 / 14.5, 28672 x
+    4096 68 / 42, 36864 x 5120 90 / 70; 24 rows 10240 x 2560 19.7 / 18.7, 16384 x 3072 24.9 / 21.9, 28672 x 4096 55 / 46; 32 rows 28672 x 4096 58 / 48;
+    but 24 rows 27648 x 5120 56 / 58. The line lies where four tiles a workgroup had it, and layers that chain their products do not ask; two
+    tiles are ahead behind it as well: 16 rows 57344 x 8192 194 / 154, 24 rows 17920 x 2560 26.6 / 24.3, 7168 x 4096 18.6 / 16.6, 32 rows 22016 x 4096
+    46 / 38."""
     if not isinstance(weight, torch.Tensor):
         return True
     N, K = weight.shape
@@ -163,7 +165,9 @@ def chain_faster(rows, weights):
     472 / 374, 729 / 458; 4096, 11008 350 / 332, 374 / 341, 409 / 377, 540 / 509; 4096, 14336 362 / 340, 382 / 355, 402 / 379, 470 / 455; 6144,
     16384, 16 and 32 rows 619 / 604, 688 / 659; 8192, 28672, 4 rows 868 / 756; e4m3 4096, 14336 265 / 252, 297 / 257, 339 / 301; 3072, 8192 187 / 178,
     219 / 183, 245 / 212; 2048, 8192 138 / 128, 172 / 143; 5120, 13824, 1 and 8 rows 263 / 226, 275 / 254. From 17 rows on not 5120, 13824 with 40 kv
-    heads (8 rows 382 / 347, 32 rows 483 / 513), whose last round of the gate's workgroups is short."""
+    heads (8 rows 382 / 347, 32 rows 483 / 513), whose last round of the gate's workgroups is short. One row again, behind 900 keys, on another card:
+    2048 177 / 154, 3072 241 / 217, 4096, 14336 356 / 322, e4m3 133 / 119, 172 / 161, 243 / 232; behind 64 keys 171 / 151, 234 / 205, 346 / 311, e4m3 124 /
+    114, 167 / 149, 234 / 220."""
     if rows <= STREAM_ROWS or len(weights) == 1:
         return True
     N, K = weights[2][0].shape
@@ -172,11 +176,15 @@ def chain_faster(rows, weights):
 
 def stream_res(x, wk, res, norm_weight):
     """h = res + x . w^T and what the next product takes of rms_norm(h) * norm_weight, in ONE launch (stream_gemm.hip):
-    (bf16(h * norm_weight), h, sums of h^2 by tiles of 16 columns)."""
+    (bf16(h * norm_weight), h, sums of h^2 by tiles of 16 columns, of 8 for up to 8 rows of up to 2048 columns)."""
     return torch.ops.sxe.stream_gemm_res(x, wk[0], wk[1], None, res, norm_weight)
 
 
-MERGE_COLUMNS = 2048  # rows and columns of a weight that stream_gemm.hip merges the splits for in its own launch
+# Rows and columns of a weight that stream_gemm.hip merges the splits for in its own launch, however many there are: one sequence, three layers of
+# hidden 2048, us a step with a launch for the merge / so: 4 kv heads 900 keys (8 splits) 163 / 157, 8000 (32) 180 / 172, 16000 (64) 204 / 197, 60000
+# (128, 1 MB of partials) 282 / 279, e4m3 126 / 119, 152 / 146, 173 / 169, 247 / 247; 16 kv heads 16000 257 / 249; hidden 1024, 2 kv heads, 60000 (256)
+# 248 / 240.
+MERGE_COLUMNS = 2048
 
 
 def stream_res_splits(parts, wk, res, norm_weight):
