@@ -6,8 +6,8 @@
 // not in the snapshot; kMax = 64 there too).
 //
 // What bounds it: with D = 32 the vector work of a score (exponent 8 clocks a wave's instruction, every other 4) beside two to four
-// products of it, and how little of the two the two or three waves of a SIMD overlap: at 1 x 128 x 384, 8 heads of 32, the vector units
-// are busy 70 % of the forward's time, 40 to 45 % of the backward's, the matrix cores 22 to 29 %. Structure:
+// products of it, and how little of the two the waves of a SIMD overlap: at 1 x 128 x 384, 8 heads of 32, the vector units are busy 69 % of the
+// forward's clocks, 53 % of dK-dV's and 34 % of dQ's (fewer than two waves a SIMD), the matrix cores 19, 29 and 16 %. Structure:
 //  * swapped products (S^T = K Q^T: one lane = one query's scores, lane-local softmax) on v_mfma_f32_32x32x16_bf16, the
 //    score accumulator reused as the B operand of O^T += V^T P^T; 128 queries (or keys) a workgroup, K / V (Q / dO) rows
 //    direct to LDS, two slots;
